@@ -31,6 +31,11 @@ __device__ __forceinline__ void deferred_run(char* lds, const DeferredJob& j, in
                                                   j.cols, GemmEpilogue<OutT>{nullptr, nullptr, 0}, j.rows,
                                                   (j.cols + kGemmBN - 1) / kGemmBN);
       break;
+    case kDeferSplitRows:
+      gemm_splitk_reduce_group<OutT, false, false>(static_cast<int64_t>(local_block) * 1024 + threadIdx.x, j.part,
+                                                   static_cast<const OutT*>(nullptr), out, j.slice, j.slice, j.groups,
+                                                   j.cols, GemmEpilogue<OutT>{nullptr, nullptr, 0});
+      break;
     case kDeferBiasRows:
       linear_bwd_db_block<OutT>(reinterpret_cast<float*>(lds) + sub * 256, tid, local_block * 4 + sub, j.part, out,
                                 j.groups, j.cols);

@@ -1,4 +1,7 @@
 // C ABI for the matmul family: operand classification, kernel choice, launches.
+#include <algorithm>
+
+#include "gemm_f32_direct.h"
 #include "gemm_impl.h"
 #include "mg_deferred.h"
 #include "mg_rows.h"
@@ -29,10 +32,25 @@ static GemmEpilogue<T> epilogue_of(const GemmArgs& g) {
 
 static bool mult4(int64_t v) { return (v & 3) == 0; }
 
-template <bool A_KC, bool B_KC>
-static int launch_f32_mfma(const GemmArgs& g, hipStream_t stream) {
-  const int tiles_m = static_cast<int>(ceil_div(g.M, kGemmBM));
-  const int tiles_n = static_cast<int>(ceil_div(g.N, kGemmBN));
+// Sums the (splits, batch, M, N) partial products of an fp32 product split along K.
+static int launch_f32_splitk_reduce(const GemmArgs& g, const float* partial, int splits, hipStream_t stream) {
+  const int64_t numel = g.batch * g.M * g.N;
+  const unsigned blocks = static_cast<unsigned>(ceil_div(numel, 1024));  // four outputs per thread
+  const float* bias = static_cast<const float*>(g.bias);
+  if (bias)
+    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<float, true>), dim3(blocks), dim3(256), 0, stream, partial, bias,
+                       static_cast<float*>(g.c), numel, numel, splits, static_cast<int>(g.N), epilogue_of<float>(g));
+  else
+    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<float, false>), dim3(blocks), dim3(256), 0, stream, partial, bias,
+                       static_cast<float*>(g.c), numel, numel, splits, static_cast<int>(g.N), epilogue_of<float>(g));
+  MG_LAUNCH_CHECK();
+  return MG_OK;
+}
+
+template <bool A_KC, bool B_KC, int TS>
+static int launch_f32_pipe(const GemmArgs& g, hipStream_t stream) {
+  const int tiles_m = static_cast<int>(ceil_div(g.M, TS));
+  const int tiles_n = static_cast<int>(ceil_div(g.N, TS));
   const int64_t blocks = static_cast<int64_t>(tiles_m) * tiles_n * g.batch;
   if (blocks > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
   const int64_t lda = A_KC ? g.sam : g.sak;
@@ -41,71 +59,148 @@ static int launch_f32_mfma(const GemmArgs& g, hipStream_t stream) {
   const float* b = static_cast<const float*>(g.b);
   const float* bias = static_cast<const float*>(g.bias);
   float* c = static_cast<float*>(g.c);
-  // Two workgroups are resident per CU; a larger problem is walked by that many workgroups.
-  int64_t grid = 2 * static_cast<int64_t>(device_info().cu_count) * env_int("MOGRAD_HIP_GEMM_F32_ROUNDS", 1);
+  const int M = static_cast<int>(g.M), N = static_cast<int>(g.N), K = static_cast<int>(g.K);
+  const int batches = static_cast<int>(g.batch);
+  // An output with fewer tiles than CUs (a 10-class head: 2048 x 10 from K = 4096 is 16
+  // tiles) is split along K so that the device is filled; the partial tiles are summed in a
+  // fixed order by the same reduction the 16-bit path uses.
+  const int64_t cus = device_info().cu_count;
+  int splits = 1;
+  if (blocks < cus && g.K >= 1024) {
+    splits = static_cast<int>(ceil_div(env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2) * cus, blocks));
+    const int max_splits = static_cast<int>(g.K / env_int("MOGRAD_HIP_GEMM_SPLITK_MIN_K", 256));
+    if (splits > max_splits) splits = max_splits;
+    if (splits > 64) splits = 64;
+  }
+  if (splits > 1) {
+    const int k_per_split = static_cast<int>(ceil_div(ceil_div(g.K, splits), kGemmBK) * kGemmBK);
+    splits = static_cast<int>(ceil_div(g.K, k_per_split));
+    const int64_t numel = g.batch * g.M * g.N;
+    Scratch partial;
+    MG_TRY(partial.take(static_cast<int64_t>(splits) * numel * static_cast<int64_t>(sizeof(float))));
+    const int64_t work = blocks * splits;
+    hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, false, true, TS>), dim3(static_cast<unsigned>(work)),
+                       dim3(kGemmThreads), 0, stream, a, b, bias, c, partial.as<float>(), M, N, K, lda, ldb, g.N, g.bsa,
+                       g.bsb, g.M * g.N, tiles_m, tiles_n, batches, k_per_split, static_cast<int>(work),
+                       GemmEpilogue<float>{nullptr, nullptr, 0});
+    MG_LAUNCH_CHECK();
+    return launch_f32_splitk_reduce(g, partial.as<float>(), splits, stream);
+  }
+  // The workgroups that are resident at once walk a larger problem.
+  int64_t grid = (TS == 128 ? 2 : 4) * cus * env_int("MOGRAD_HIP_GEMM_F32_ROUNDS", 1);
   if (grid > blocks || env_int("MOGRAD_HIP_GEMM_F32_ROUNDS", 1) == 0) grid = blocks;
-  // Tiles copied straight into LDS (gemm_f32_pipe_kernel, same results bit for bit) when K is a
-  // multiple of the 32-deep step; MOGRAD_HIP_GEMM_F32_PIPE=0 keeps the register-staged kernel.
-  if (g.K % kGemmBK == 0 && env_int("MOGRAD_HIP_GEMM_F32_PIPE", 1) != 0) {
-    const int M = static_cast<int>(g.M), N = static_cast<int>(g.N), K = static_cast<int>(g.K);
-    const int batches = static_cast<int>(g.batch);
-    // An output with fewer tiles than CUs (a 10-class head: 2048 x 10 from K = 4096 is 16
-    // tiles) is split along K so that the device is filled; the partial tiles are summed in a
-    // fixed order by the same reduction the 16-bit path uses.
-    const int64_t cus = device_info().cu_count;
-    int splits = 1;
-    if (blocks < cus && g.K >= 1024) {
-      splits = static_cast<int>(ceil_div(env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2) * cus, blocks));
-      const int max_splits = static_cast<int>(g.K / env_int("MOGRAD_HIP_GEMM_SPLITK_MIN_K", 256));
-      if (splits > max_splits) splits = max_splits;
-      if (splits > 64) splits = 64;
-    }
-    if (splits > 1) {
-      const int k_per_split = static_cast<int>(ceil_div(ceil_div(g.K, splits), kGemmBK) * kGemmBK);
-      splits = static_cast<int>(ceil_div(g.K, k_per_split));
-      const int64_t numel = g.batch * g.M * g.N;
-      Scratch partial;
-      MG_TRY(partial.take(static_cast<int64_t>(splits) * numel * static_cast<int64_t>(sizeof(float))));
-      const int64_t work = blocks * splits;
-      hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, false, true>), dim3(static_cast<unsigned>(work)),
-                         dim3(kGemmThreads), 0, stream, a, b, bias, c, partial.as<float>(), M, N, K, lda, ldb, g.N, g.bsa,
-                         g.bsb, g.M * g.N, tiles_m, tiles_n, batches, k_per_split, static_cast<int>(work),
-                         GemmEpilogue<float>{nullptr, nullptr, 0});
-      MG_LAUNCH_CHECK();
-      const unsigned rblocks = static_cast<unsigned>(ceil_div(numel, 1024));  // four outputs per thread
-      if (bias)
-        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<float, true>), dim3(rblocks), dim3(256), 0, stream,
-                           partial.as<float>(), bias, c, numel, numel, splits, N, epilogue_of<float>(g));
-      else
-        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<float, false>), dim3(rblocks), dim3(256), 0, stream,
-                           partial.as<float>(), bias, c, numel, numel, splits, N, epilogue_of<float>(g));
-      MG_LAUNCH_CHECK();
-      return MG_OK;
-    }
-    float* no_partial = nullptr;
-    if (bias)
-      hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, true, false>), dim3(static_cast<unsigned>(grid)),
-                         dim3(kGemmThreads), 0, stream, a, b, bias, c, no_partial, M, N, K, lda, ldb, g.N, g.bsa, g.bsb,
-                         g.M * g.N, tiles_m, tiles_n, batches, K, static_cast<int>(blocks), epilogue_of<float>(g));
-    else
-      hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, false, false>), dim3(static_cast<unsigned>(grid)),
-                         dim3(kGemmThreads), 0, stream, a, b, bias, c, no_partial, M, N, K, lda, ldb, g.N, g.bsa, g.bsb,
-                         g.M * g.N, tiles_m, tiles_n, batches, K, static_cast<int>(blocks), epilogue_of<float>(g));
+  float* no_partial = nullptr;
+  if (bias)
+    hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, true, false, TS>), dim3(static_cast<unsigned>(grid)),
+                       dim3(kGemmThreads), 0, stream, a, b, bias, c, no_partial, M, N, K, lda, ldb, g.N, g.bsa, g.bsb,
+                       g.M * g.N, tiles_m, tiles_n, batches, K, static_cast<int>(blocks), epilogue_of<float>(g));
+  else
+    hipLaunchKernelGGL((gemm_f32_pipe_kernel<A_KC, B_KC, false, false, TS>), dim3(static_cast<unsigned>(grid)),
+                       dim3(kGemmThreads), 0, stream, a, b, bias, c, no_partial, M, N, K, lda, ldb, g.N, g.bsa, g.bsb,
+                       g.M * g.N, tiles_m, tiles_n, batches, K, static_cast<int>(blocks), epilogue_of<float>(g));
+  MG_LAUNCH_CHECK();
+  return MG_OK;
+}
+
+// dst (batch, rows, cols_to) = src (batch, rows, cols) with zero columns appended: the image of an
+// operand that the copying kernels can read 16 bytes at a time.  cols_to is a whole number of
+// 16-byte chunks and dst aligned to them; src may lie anywhere.  One thread per chunk; up to three arrays
+// per launch.  Bound by its bytes, or by the launch for small arrays.
+template <typename T>
+struct PadJob {
+  const T* src;
+  T* dst;
+  int64_t ld, batch_stride, chunks;  // chunks: of the whole array
+  int rows, cols, cols_to;
+};
+template <typename T>
+struct PadJobs {
+  PadJob<T> job[3];
+  int block_end[3];
+};
+template <typename T>
+__global__ __launch_bounds__(256) void pad_columns_kernel(PadJobs<T> jobs) {
+  const int b = blockIdx.x;
+  const int which = b < jobs.block_end[0] ? 0 : b < jobs.block_end[1] ? 1 : 2;
+  const PadJob<T>& j = jobs.job[which];
+  const int64_t i = static_cast<int64_t>(b - (which ? jobs.block_end[which - 1] : 0)) * 256 + threadIdx.x;
+  if (i >= j.chunks) return;
+  constexpr int E = 16 / sizeof(T);
+  const int per_row = j.cols_to / E;
+  const int64_t row = i / per_row;
+  const int c0 = static_cast<int>(i - row * per_row) * E;
+  const T* src = j.src + row / j.rows * j.batch_stride + row % j.rows * j.ld + c0;
+  reinterpret_cast<uint4*>(j.dst)[i] = gemm_gather_chunk(src, j.cols - c0);
+}
+
+// Collects the operands of one product that need such an image and makes them in one launch.
+template <typename T>
+struct PadCopies {
+  PadJobs<T> jobs{};
+  Scratch mem[3];
+  int count = 0;
+  int64_t blocks = 0;
+  // The image of `src`, whose rows then lie `*ld` apart and batches `*batch_stride`.
+  int add(const void** src, int64_t batch, int64_t rows, int64_t cols, int64_t* ld, int64_t* batch_stride) {
+    constexpr int E = 16 / sizeof(T);
+    const int64_t to = ceil_div(cols, E) * E;
+    const int64_t images = *batch_stride == 0 ? 1 : batch;
+    MG_TRY(mem[count].take(images * rows * to * static_cast<int64_t>(sizeof(T))));
+    PadJob<T>& j = jobs.job[count];
+    j = PadJob<T>{static_cast<const T*>(*src), mem[count].template as<T>(), *ld, *batch_stride, images * rows * (to / E),
+                  static_cast<int>(rows), static_cast<int>(cols), static_cast<int>(to)};
+    blocks += ceil_div(j.chunks, 256);
+    for (int i = count; i < 3; ++i) jobs.block_end[i] = static_cast<int>(blocks);
+    ++count;
+    *src = j.dst;
+    *ld = to;
+    *batch_stride = images == 1 ? 0 : rows * to;
+    return MG_OK;
+  }
+  int launch(hipStream_t stream) {
+    if (count == 0 || blocks == 0) return MG_OK;
+    if (blocks > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: operand too large");
+    hipLaunchKernelGGL((pad_columns_kernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, jobs);
     MG_LAUNCH_CHECK();
     return MG_OK;
   }
-  if (bias)
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<A_KC, B_KC, true>), dim3(static_cast<unsigned>(grid)), dim3(kGemmThreads),
-                       0, stream, a, b, bias, c, static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K), lda,
-                       ldb, g.N, g.bsa, g.bsb, g.M * g.N, tiles_m, tiles_n, static_cast<int>(blocks),
-                       epilogue_of<float>(g));
-  else
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<A_KC, B_KC, false>), dim3(static_cast<unsigned>(grid)),
-                       dim3(kGemmThreads), 0, stream, a, b, bias, c, static_cast<int>(g.M), static_cast<int>(g.N),
-                       static_cast<int>(g.K), lda, ldb, g.N, g.bsa, g.bsb, g.M * g.N, tiles_m, tiles_n,
-                       static_cast<int>(blocks), epilogue_of<float>(g));
+};
+
+// Outputs of one tile column (or row) of 16 take gemm_f32_direct_kernel's 16 x 16 tiles, others its
+// 32 x 32 ones; four waves along k in either.
+static int f32_direct_tile(int64_t M, int64_t N) { return std::min(M, N) <= 16 ? 16 : 32; }
+
+template <bool A_KC, bool B_KC>
+static int launch_f32_direct(const GemmArgs& g, hipStream_t stream) {
+  const int tile = f32_direct_tile(g.M, g.N);
+  const int64_t tiles_m = ceil_div(g.M, tile), tiles_n = ceil_div(g.N, tile);
+  const int64_t blocks = tiles_m * tiles_n * g.batch;
+  // K ranges: enough for a workgroup per CU, each with at least 256 of K.
+  int splits = static_cast<int>(std::max<int64_t>(
+      1, std::min({ceil_div(device_info().cu_count, blocks), g.K / env_int("MOGRAD_HIP_GEMM_SPLITK_MIN_K", 256),
+                   static_cast<int64_t>(64)})));
+  const int k_per_split = static_cast<int>(ceil_div(ceil_div(g.K, splits), 64) * 64);
+  splits = static_cast<int>(ceil_div(g.K, k_per_split));
+  if (blocks * splits > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
+  Scratch partial;
+  if (splits > 1) MG_TRY(partial.take(splits * g.batch * g.M * g.N * static_cast<int64_t>(sizeof(float))));
+  const Gemm32Problem pr{static_cast<const float*>(g.a), static_cast<const float*>(g.b), static_cast<const float*>(g.bias),
+                         static_cast<float*>(g.c), partial.as<float>(), static_cast<int>(g.M), static_cast<int>(g.N),
+                         static_cast<int>(g.K), A_KC ? g.sam : g.sak, B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb, g.M * g.N,
+                         static_cast<int>(tiles_m), static_cast<int>(tiles_n), static_cast<int>(g.batch), k_per_split,
+                         splits, epilogue_of<float>(g)};
+  const dim3 grid(static_cast<unsigned>(blocks * splits));
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, pr); };
+  if (splits == 1) {
+    if (tile == 16) launch(gemm_f32_direct_kernel<A_KC, B_KC, 16, false>);
+    else launch(gemm_f32_direct_kernel<A_KC, B_KC, 32, false>);
+    MG_LAUNCH_CHECK();
+    return MG_OK;
+  }
+  if (tile == 16) launch(gemm_f32_direct_kernel<A_KC, B_KC, 16, true>);
+  else launch(gemm_f32_direct_kernel<A_KC, B_KC, 32, true>);
   MG_LAUNCH_CHECK();
-  return MG_OK;
+  return launch_f32_splitk_reduce(g, partial.as<float>(), splits, stream);
 }
 
 static bool mult8(int64_t v) { return (v & 7) == 0; }
@@ -152,41 +247,35 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
   const int M = static_cast<int>(g.M), N = static_cast<int>(g.N), K = static_cast<int>(g.K);
   const int64_t cus = device_info().cu_count;
   int splits = splitk_16bit_splits(blocks, g.K, env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2));
-  // Tiles copied straight into LDS (gemm_16bit_pipe_kernel) where that measured faster: an
-  // operand that is not k-contiguous is transposed by the LDS read instead of in registers
-  // (dX 15-25 %, dW 5-20 % faster at Linear-layer shapes, 20-30 % at 4096^3 and up), and long
-  // K loops gain from the single barrier per step.  Two k-contiguous operands: from 384 k per
-  // workgroup on (2-8 % faster at 16384 rows, 10-25 % at 256-2048 rows), and from 192 for
-  // outputs of at most two tiles per CU (8-15 %); shorter K loops, and 192-383 on larger outputs
-  // (3-8 % slower there), stay with the register-staged kernel, as does every shape the copy
-  // cannot take (MOGRAD_HIP_GEMM16_PIPE_MIN_K moves the 384).  The pair is k per step and copies
-  // of the tiles: (32, 2) runs four workgroups per CU, (64, 2) two.
-  // MOGRAD_HIP_GEMM16_PIPE = 0 | 322 | 642 | 2322 | 2642 overrides the choice (2xxx: 256 x 128 tiles).
+  // Tiles copied straight into LDS (gemm_16bit_pipe_kernel): an operand that is not k-contiguous is
+  // transposed by the LDS read instead of in registers, and a k-step costs one barrier.  64 k per
+  // step and two copies of the tiles measured fastest or equal at every layout and size swept, 64 to
+  // 16384 rows, 256 to 1536 columns, K 256 to 16384 (32 k per step 5-12 % slower below 16384 rows,
+  // the register-staged kernel 4-40 %).  What the copy cannot take (operands that do not lie on
+  // 16-byte chunks) is the register-staged kernel's, RAGGED.
+  // MOGRAD_HIP_GEMM16_PIPE = 0 | 322 | 642 | 2322 | 2642 overrides the choice: 0 the register-staged
+  // kernel, else k per step and copies of the tiles (2xxx: 256 x 128 tiles).
   int pipe = 0;
   if constexpr (!RAGGED) {
-    if (g.K % kG16BK == 0 && mult8(g.M) && mult8(g.N)) {
-      const int64_t k_wg = ceil_div(g.K, splits);  // the K range one workgroup walks
-      if (A_KC && B_KC) {
-        const int64_t min_k = env_int("MOGRAD_HIP_GEMM16_PIPE_MIN_K", 384);
-        pipe = k_wg >= min_k || (2 * k_wg >= min_k && blocks <= 2 * cus) ? 642 : 0;
-      }
-      else pipe = k_wg >= 4096 ? 642 : 322;
-      // Large products: 256 x 128 tiles (eight waves), a quarter fewer operand bytes per FLOP
-      // through L2, once they still give every CU two workgroups (4096^3: 3-11 % faster).
-      if (splits <= 1 && g.K >= 1024 && ceil_div(g.M, 256) * tiles_n * g.batch >= 2 * cus) pipe = 2322;
-      // Products with a 256 x 256 tile for every CU: four waves of 128 x 128 each, one workgroup
-      // per CU (gemm_16bit_big_kernel; 4642: 64 k per step and two copies of the tiles, 4324: 32 k
-      // and four; 4096^3 forward 147 -> 121 us, 8192^3 dW 1016 -> 887 us, bit-identical results).
-      if (splits <= 1 && g.K >= 1024 && ceil_div(g.M, kGemmBigT) * ceil_div(g.N, kGemmBigT) * g.batch >= cus) pipe = 4642;
-      pipe = static_cast<int>(env_int("MOGRAD_HIP_GEMM16_PIPE", pipe));
-    }
+    pipe = 642;
+    // Large products: 256 x 128 tiles (eight waves), a quarter fewer operand bytes per FLOP
+    // through L2, once they still give every CU two workgroups (4096^3: 3-11 % faster).
+    if (splits <= 1 && g.K >= 1024 && ceil_div(g.M, 256) * tiles_n * g.batch >= 2 * cus) pipe = 2322;
+    // Products with a 256 x 256 tile for every CU: four waves of 128 x 128 each, one workgroup
+    // per CU (gemm_16bit_big_kernel; 4642: 64 k per step and two copies of the tiles, 4324: 32 k
+    // and four; 4096^3 forward 147 -> 121 us, 8192^3 dW 1016 -> 887 us, bit-identical results).
+    // It takes whole k-steps only.
+    if (splits <= 1 && g.K >= 1024 && g.K % kG16BK == 0 &&
+        ceil_div(g.M, kGemmBigT) * ceil_div(g.N, kGemmBigT) * g.batch >= cus)
+      pipe = 4642;
+    pipe = static_cast<int>(env_int("MOGRAD_HIP_GEMM16_PIPE", pipe));
   }
-  if (splits <= 1 && pipe >= 4000) {
+  if (splits <= 1 && pipe >= 4000 && g.K % kG16BK == 0) {
     if constexpr (!RAGGED)
       return gemm16_big_launch(g.dtype, A_KC, B_KC, pipe, g.a, g.b, g.bias, g.c, g.batch, M, N, K, lda, ldb, g.bsa, g.bsb,
                                g.residual, g.relu_mask, g.relu, stream);
   }
-  if (pipe >= 4000) pipe = 322;
+  if (pipe >= 4000) pipe = 642;
 #define MG_GEMM16_LAUNCH(BIAS_, SPLIT_, GRID_, PARTIAL_, KPS_, NSPLIT_, EP_)                                                   \
   do {                                                                                                                 \
     auto launch = [&](auto kernel) {                                                                                   \
@@ -197,7 +286,7 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
       if (pipe == 322) { launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, BIAS_, SPLIT_, 32, 2>); break; }                 \
       if (pipe == 642) { launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, BIAS_, SPLIT_, 64, 2>); break; }                 \
     }                                                                                                                  \
-    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, BIAS_, SPLIT_, RAGGED>);                                              \
+    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, BIAS_, SPLIT_>);                                              \
   } while (0)
   if (splits <= 1 && (pipe == 2322 || pipe == 2642)) {
     // 256 x 128 tiles, eight waves: a quarter fewer operand bytes per FLOP through L2.
@@ -253,23 +342,92 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
   return MG_OK;
 }
 
+// fp32 products whose operands are each contiguous along one axis.
+//   tiles copied into LDS, 128 x 128 where every CU gets one ((4096, 1024) <- 1024: 74 us, 81 with
+//   64 x 64), else 64 x 64 down to one for every second CU ((2048, 768) <- 768: 31 us against 55 with
+//   128 x 128 and 42 straight from memory), fewer where a long reduction can be split as well;
+//   operands that do not lie on 16-byte chunks are copied to rows that do, which takes a tile
+//   per CU to pay ((1999, 1001) <- 767: 44 us against 59; (2587, 256) <- 256: 14 against 10);
+//   everything smaller straight from memory (gemm_f32_direct.h).
+// MOGRAD_HIP_GEMM_F32_TILE = 32 | 64 | 128 overrides the choice (32: straight from memory).
+static int dispatch_f32(const GemmArgs& g_in, hipStream_t stream, bool* handled) {
+  GemmArgs g = g_in;
+  const bool a_kc = g.sak == 1, b_kc = g.sbk == 1;
+  const int64_t cus = device_info().cu_count;
+  const int64_t blocks128 = ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch;
+  const int64_t blocks64 = ceil_div(g.M, 64) * ceil_div(g.N, 64) * g.batch;
+  // Next to no reduction and a large output (the dX of a 10-class head): neither the copies nor the
+  // fragments have anything to reuse, and the plain kernel's stores are the widest.
+  *handled = !(g.K < 32 && blocks64 >= cus);
+  if (!*handled) return MG_OK;
+  const bool a_wide = (a_kc ? mult4(g.sam) && mult4(g.K) : mult4(g.sak) && mult4(g.M)) && mult4(g.bsa) && aligned16(g.a);
+  const bool b_wide = (b_kc ? mult4(g.sbn) && mult4(g.K) : mult4(g.sbk) && mult4(g.N)) && mult4(g.bsb) && aligned16(g.b);
+  const bool use64 = a_wide && b_wide ? 2 * blocks64 >= cus || (8 * blocks64 >= cus && g.K >= 1024) : blocks64 >= cus;
+  const int tile = env_int("MOGRAD_HIP_GEMM_F32_TILE", blocks128 >= cus ? 128 : use64 ? 64 : 32);
+  if (tile == 32) {
+    if (a_kc && b_kc) return launch_f32_direct<true, true>(g, stream);
+    if (a_kc) return launch_f32_direct<true, false>(g, stream);
+    if (b_kc) return launch_f32_direct<false, true>(g, stream);
+    return launch_f32_direct<false, false>(g, stream);
+  }
+  PadCopies<float> pad;
+  if (!a_wide) {
+    if (a_kc) MG_TRY(pad.add(&g.a, g.batch, g.M, g.K, &g.sam, &g.bsa));
+    else MG_TRY(pad.add(&g.a, g.batch, g.K, g.M, &g.sak, &g.bsa));
+  }
+  if (!b_wide) {
+    if (b_kc) MG_TRY(pad.add(&g.b, g.batch, g.N, g.K, &g.sbn, &g.bsb));
+    else MG_TRY(pad.add(&g.b, g.batch, g.K, g.N, &g.sbk, &g.bsb));
+  }
+  MG_TRY(pad.launch(stream));
+#define MG_F32_PIPE(TS_)                                                       \
+  do {                                                                         \
+    if (a_kc && b_kc) return launch_f32_pipe<true, true, TS_>(g, stream);      \
+    if (a_kc) return launch_f32_pipe<true, false, TS_>(g, stream);             \
+    if (b_kc) return launch_f32_pipe<false, true, TS_>(g, stream);             \
+    return launch_f32_pipe<false, false, TS_>(g, stream);                      \
+  } while (0)
+  if (tile == 64) MG_F32_PIPE(64);
+  MG_F32_PIPE(128);
+#undef MG_F32_PIPE
+}
+
 template <typename T>
-static int dispatch_16bit(const GemmArgs& g, hipStream_t stream, bool* handled) {
+static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handled) {
   *handled = false;
+  GemmArgs g = g_in;
   if (g.K <= 0) return MG_OK;
   // Each operand must be contiguous along k or along its other axis.  When leading
-  // dimensions, extents and addresses are all multiples of 8 elements the tiles are staged
-  // with 16-byte loads; otherwise with element loads (the ragged variant).
+  // dimensions, extents and addresses are all multiples of 8 elements the tiles are copied
+  // straight into LDS; otherwise they are staged through registers (the ragged variant), or,
+  // where the product is long enough to pay for it, the operand is copied to rows that are.
   const bool a_kc = g.sak == 1;
   const bool a_mc = g.sam == 1;
   const bool b_kc = g.sbk == 1;
   const bool b_nc = g.sbn == 1;
-  const bool worth_it = g.M * g.N >= 64 * 64 || g.K >= 512;
-  if (!(worth_it && (a_kc || a_mc) && (b_kc || b_nc))) return MG_OK;
-  const bool a_wide = a_kc ? mult8(g.sam) && mult8(g.K) : mult8(g.sak) && mult8(g.M);
-  const bool b_wide = b_kc ? mult8(g.sbn) && mult8(g.K) : mult8(g.sbk) && mult8(g.N);
-  const bool wide = a_wide && b_wide && aligned16(g.a) && aligned16(g.b) && mult8(g.bsa) && mult8(g.bsb);
+  if (!((a_kc || a_mc) && (b_kc || b_nc))) return MG_OK;
+  const bool a_wide = (a_kc ? mult8(g.sam) && mult8(g.K) : mult8(g.sak) && mult8(g.M)) && aligned16(g.a) && mult8(g.bsa);
+  const bool b_wide = (b_kc ? mult8(g.sbn) && mult8(g.K) : mult8(g.sbk) && mult8(g.N)) && aligned16(g.b) && mult8(g.bsb);
   *handled = true;
+  bool wide = a_wide && b_wide;
+  PadCopies<T> pad;
+  // The copy costs a launch and two passes over the operand, the ragged variant its slower staging:
+  // two k-contiguous operands are as fast through it up to some 20 GFLOP ((2048, 1000) <- 1001:
+  // 19.9 us against 23.7; (4000, 4001) <- 1025: 68 against 66), the transposing layouts only at a
+  // few k-steps ((1999, 767) <- 1001: 51 against 28 us; (16384, 384) <- 65: 9 against 11).
+  const bool copy_pays = a_kc && b_kc ? 2.0 * g.batch * g.M * g.N * g.K >= 2e10 : g.K >= 128;
+  if (!wide && env_int("MOGRAD_HIP_GEMM16_PAD", copy_pays) != 0) {
+    if (!a_wide) {
+      if (a_kc) MG_TRY(pad.add(&g.a, g.batch, g.M, g.K, &g.sam, &g.bsa));
+      else MG_TRY(pad.add(&g.a, g.batch, g.K, g.M, &g.sak, &g.bsa));
+    }
+    if (!b_wide) {
+      if (b_kc) MG_TRY(pad.add(&g.b, g.batch, g.N, g.K, &g.sbn, &g.bsb));
+      else MG_TRY(pad.add(&g.b, g.batch, g.K, g.N, &g.sbk, &g.bsb));
+    }
+    MG_TRY(pad.launch(stream));
+    wide = true;
+  }
   if (wide) {
     if (a_kc && b_kc) return launch_16bit_mfma<T, true, true, false>(g, stream);
     if (a_kc) return launch_16bit_mfma<T, true, false, false>(g, stream);
@@ -312,42 +470,10 @@ int gemm_dispatch(const char* who, const GemmArgs& g_in, hipStream_t stream) {
   if (g.batch == 0 || g.M == 0 || g.N == 0) return MG_OK;
   if (!g.a || !g.b || !g.c) return fail(MG_ERR_INVALID, "%s: null pointer argument", who);
 
-  if (g_in.dtype == MG_F32 && g_in.K > 0) {
-    GemmArgs g = g_in;
-    // Which dimension of each operand is contiguous, and can it be read 16 bytes at a time?
-    bool a_kc = g.sak == 1 && mult4(g.sam) && mult4(g.K) && mult4(g.bsa) && aligned16(g.a);
-    const bool a_mc = g.sam == 1 && mult4(g.sak) && mult4(g.M) && mult4(g.bsa) && aligned16(g.a);
-    bool b_kc = g.sbk == 1 && mult4(g.sbn) && mult4(g.K) && mult4(g.bsb) && aligned16(g.b);
-    const bool b_nc = g.sbn == 1 && mult4(g.sbk) && mult4(g.N) && mult4(g.bsb) && aligned16(g.b);
-    // Tiny problems gain nothing from 128x128 tiles.
-    const bool worth_it = g.M * g.N >= 64 * 64 || g.K >= env_int("MOGRAD_HIP_GEMM_F32_MIN_K", 128);
-    // A thin operand that cannot be read 16 bytes at a time as it lies (the (K, 10) gradient
-    // of a 10-class head, read along its 10-wide rows for dW) is first copied k-contiguous:
-    // at most one tile of rows, so the copy is a small fraction of the other operand's bytes.
-    Scratch a_copy, b_copy;
-    const bool deep = g.K >= 512 && mult4(g.K);
-    if (deep && !(a_kc || a_mc) && g.M <= kGemmBM && (b_kc || b_nc || g.N <= kGemmBN)) {
-      MG_TRY(a_copy.take(g.batch * g.M * g.K * static_cast<int64_t>(sizeof(float))));
-      const int64_t shape[3] = {g.batch, g.M, g.K}, strides[3] = {g.bsa, g.sam, g.sak};
-      MG_TRY(mg_contiguous(g.a, a_copy.as<float>(), 3, shape, strides, MG_F32, stream));
-      g.a = a_copy.as<float>();
-      g.sam = g.K, g.sak = 1, g.bsa = g.M * g.K;
-      a_kc = true;
-    }
-    if (deep && !(b_kc || b_nc) && g.N <= kGemmBN && (a_kc || a_mc)) {
-      MG_TRY(b_copy.take(g.batch * g.N * g.K * static_cast<int64_t>(sizeof(float))));
-      const int64_t shape[3] = {g.batch, g.N, g.K}, strides[3] = {g.bsb, g.sbn, g.sbk};
-      MG_TRY(mg_contiguous(g.b, b_copy.as<float>(), 3, shape, strides, MG_F32, stream));
-      g.b = b_copy.as<float>();
-      g.sbn = g.K, g.sbk = 1, g.bsb = g.N * g.K;
-      b_kc = true;
-    }
-    if (worth_it && (a_kc || a_mc) && (b_kc || b_nc)) {
-      if (a_kc && b_kc) return launch_f32_mfma<true, true>(g, stream);
-      if (a_kc) return launch_f32_mfma<true, false>(g, stream);
-      if (b_kc) return launch_f32_mfma<false, true>(g, stream);
-      return launch_f32_mfma<false, false>(g, stream);
-    }
+  if (g.dtype == MG_F32 && g.K > 0 && (g.sak == 1 || g.sam == 1) && (g.sbk == 1 || g.sbn == 1)) {
+    bool handled = false;
+    const int rc = dispatch_f32(g_in, stream, &handled);
+    if (handled || rc != MG_OK) return rc;
   }
   if (g.dtype != MG_F32) {
     bool handled = false;
@@ -390,18 +516,17 @@ struct LinearBwdLayerNorm {
 };
 
 template <typename T>
-static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, void* dx, void* dw, int64_t M, int64_t N,
-                                 int64_t K, const void* relu_mask, bool dx_accumulate, hipStream_t stream, bool* done,
-                                 int64_t dw_rows = -1, void* db = nullptr, bool* db_done = nullptr,
-                                 const LinearBwdLayerNorm* ln = nullptr) {
+static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, void* dx, void* dw, void* db, int64_t M,
+                                 int64_t N, int64_t K, const void* relu_mask, bool dx_accumulate, hipStream_t stream,
+                                 bool* done, bool* db_done, const LinearBwdLayerNorm* ln) {
   *done = false;
-  if (db_done) *db_done = false;
-  if (dw_rows < 0) dw_rows = N;  // rows of dW to write: fewer than N when dY and W came zero-padded
+  *db_done = false;
   if (env_int("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", 1) == 0 || env_str("MOGRAD_HIP_GEMM16_PIPE")) return MG_OK;
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return MG_OK;
-  if (M % kG16BK || N % kG16BK || !mult8(K)) return MG_OK;
-  if (!aligned16(dy) || !aligned16(x) || !aligned16(w) || !aligned16(dx) || !aligned16(dw)) return MG_OK;
-  if (M * K < 64 * 64 || N * K < 64 * 64) return MG_OK;
+  // Widths that are no multiple of 8 (a 65-symbol vocabulary): rows of dY, or of X and W, start
+  // at odd addresses, which the copies into LDS cannot take.  Those arrays are first copied to
+  // rows of the next multiple of 8, zeros behind (`pads` below); dX, dW and db keep their shape.
+  const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || !aligned16(w);
   const int64_t cus = device_info().cu_count;
   // Input widths that are multiples of 384 take 128 x 384 output tiles (twelve waves, one
   // workgroup per CU): the three column tiles of a row block share one copy of the dY tile,
@@ -411,7 +536,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const bool wide = K % kGemmWideBN == 0 && ceil_div(M, kGemmBM) * (K / kGemmWideBN) < cus && N >= 768 &&
                     env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) != 0;
   if (ln && (!wide || K != kGemmWideBN || relu_mask || env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3 ||
-             !aligned16(ln->x) || !aligned16(ln->gamma)))
+             pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx)))
     return MG_OK;
   const int tiles_kk = static_cast<int>(ceil_div(K, wide ? kGemmWideBN : kGemmBN));
   // dW: must be split, each workgroup's rows short enough for the 32-k variant.
@@ -436,29 +561,39 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
     // the K ranges are half the partial tiles to write and sum (GPT step 3.06 -> 3.00 ms).
     splits = splitk_16bit_splits(w_tiles, M, env_int("MOGRAD_HIP_LINEAR_BWD_SPLIT_WG_PER_CU", 1));
   }
-  if (splits <= 1 || ceil_div(M, splits) >= 4096) return MG_OK;
-  const int k_per_split = splitk_16bit_range(M, &splits);
-  // Every K range of dW and the whole reduction of dX must be whole k-steps (of 32 or 64): the
-  // kernels drop a remainder.  Guaranteed by M % kG16BK == 0, N % kG16BK == 0 and ranges cut in
-  // units of kG16BK; checked here so that a change to either cannot lose rows silently.
-  if (k_per_split % kG16BK != 0 || M % kG16BK != 0 || N % kG16BK != 0) return MG_OK;
-  // dX: the 32-k variant.
-  if (N >= 4096 || (N >= 1024 && ceil_div(M, 256) * tiles_kk >= 2 * cus)) return MG_OK;
-  const int64_t n_dw = gemm_split_grid(w_tiles, splits, 1);
+  // Few rows (M < 1024): nothing is split, dW and db are the workgroups' own results
+  // (linear_bwd_short_16bit_kernel), unless their sums are deferred.
+  const bool split_sums = splits > 1 || deferred_current() != nullptr;
+  if (splits <= 1 && M >= 1024) return MG_OK;
+  if (ceil_div(M, splits) >= 4096) return MG_OK;
+  const int k_per_split = splits > 1 ? splitk_16bit_range(M, &splits) : static_cast<int>(M);
+  // dX, which is never split here: not a long reduction, and none that another split would serve better.
+  if (N >= 4096 || (N >= 1024 && (M < 1024 || ceil_div(M, 256) * tiles_kk >= 2 * cus))) return MG_OK;
+  const int64_t n_dw = split_sums ? gemm_split_grid(w_tiles, splits, 1) : w_tiles;
   if (n_dw + x_tiles > 0x7fffffffLL) return MG_OK;
+
+  int64_t ldy = N, ldx = K, ldw = K;
+  PadCopies<T> pads;
+  int64_t no_batch = 0;
+  if (pad_n) MG_TRY(pads.add(&dy, 1, M, N, &ldy, &no_batch));
+  if (pad_k) {
+    MG_TRY(pads.add(&x, 1, M, K, &ldx, &no_batch));
+    MG_TRY(pads.add(&w, 1, N, K, &ldw, &no_batch));
+  }
+  MG_TRY(pads.launch(stream));
 
   Scratch partial;
   const int64_t numel = N * K;
   const int64_t slice = gemm16_partial_floats(N, K, 1, 1);  // whole tiles per K range
-  MG_TRY(partial.take(static_cast<int64_t>(splits) * slice * static_cast<int64_t>(sizeof(float))));
+  if (split_sums) MG_TRY(partial.take(static_cast<int64_t>(splits) * slice * static_cast<int64_t>(sizeof(float))));
   const T* dyt = static_cast<const T*>(dy);
   const Gemm16Problem<T> pw{dyt, static_cast<const T*>(x), nullptr, static_cast<T*>(dw), partial.as<float>(),
                             static_cast<int>(N), static_cast<int>(K), static_cast<int>(M),
-                            N, K, K, 0, 0, numel, w_tiles_m, tiles_kk, k_per_split, splits, 1,
+                            ldy, ldx, K, 0, 0, numel, w_tiles_m, tiles_kk, k_per_split, splits, 1,
                             GemmEpilogue<T>{nullptr, nullptr, 0}};
   const Gemm16Problem<T> px{dyt, static_cast<const T*>(w), nullptr, static_cast<T*>(dx), nullptr,
                             static_cast<int>(M), static_cast<int>(K), static_cast<int>(N),
-                            N, K, K, 0, 0, M * K, x_tiles_m, tiles_kk, static_cast<int>(N), 1, 1,
+                            ldy, ldw, K, 0, 0, M * K, x_tiles_m, tiles_kk, static_cast<int>(N), 1, 1,
                             GemmEpilogue<T>{dx_accumulate ? static_cast<const T*>(dx) : nullptr,
                                             static_cast<const T*>(relu_mask), 0}};
   // The bias gradient rides along: the dW workgroups of the first tile column sum the dY
@@ -472,7 +607,17 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   pw2.partial_stream = deferred_current() != nullptr && env_int("MOGRAD_HIP_DEFER_NT_STORE", 1) != 0;
   Scratch db_part;
   int groups = 0;
-  if (db && dw_rows == N && env_int("MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH", 1) != 0) {
+  const bool db_here = db && env_int("MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH", 1) != 0;
+  if (!split_sums) {
+    if (db_here) pw2.colsum = static_cast<T*>(db);
+    hipLaunchKernelGGL((linear_bwd_short_16bit_kernel<T>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(kGemmThreads),
+                       0, stream, pw2, px, static_cast<int>(n_dw));
+    MG_LAUNCH_CHECK();
+    *db_done = db_here;
+    *done = true;
+    return MG_OK;
+  }
+  if (db_here) {
     groups = splits;
     MG_TRY(db_part.take(static_cast<int64_t>(groups) * N * static_cast<int64_t>(sizeof(float))));
     pw2.colsum_part = db_part.as<float>();
@@ -511,70 +656,96 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const int db_blocks = groups > 0 ? static_cast<int>(ceil_div(N, 64)) : 0;
   if (DeferredList* dl = deferred_current()) {
     // The sums of the K ranges are left to mg_finish_deferred (same code, same order).
-    dl->push(kDeferSplitK, partial.as<float>(), dw, slice, static_cast<int>(dw_rows), static_cast<int>(K), splits,
+    dl->push(kDeferSplitK, partial.as<float>(), dw, slice, static_cast<int>(N), static_cast<int>(K), splits,
              ceil_div(slice / 4, 1024));
     dl->hold(partial);
     if (groups > 0) {
       dl->push(kDeferBiasRows, db_part.as<float>(), db, 0, 0, static_cast<int>(N), groups, ceil_div(db_blocks, 4));
       dl->hold(db_part);
     }
-    if (db_done) *db_done = groups > 0;
+    *db_done = groups > 0;
     *done = true;
     return MG_OK;
   }
   hipLaunchKernelGGL((linear_bwd_finish_kernel<T>), dim3(static_cast<unsigned>(dw_blocks + db_blocks)), dim3(256), 0,
-                     stream, partial.as<float>(), static_cast<T*>(dw), static_cast<int>(dw_rows), slice, splits,
+                     stream, partial.as<float>(), static_cast<T*>(dw), static_cast<int>(N), slice, splits,
                      static_cast<int>(K), dw_blocks, db_part.as<float>(), static_cast<T*>(db), groups,
                      static_cast<int>(N));
   MG_LAUNCH_CHECK();
-  if (db_done) *db_done = groups > 0;
+  *db_done = groups > 0;
   *done = true;
   return MG_OK;
 }
 
-// dst (rows, cols_to) = src (rows, cols) with zero columns appended; cols_to is a multiple of 8
-// and dst 16-byte aligned.  One thread per 8 output columns.
-template <typename T>
-__global__ __launch_bounds__(256) void pad_columns_kernel(const T* __restrict__ src, T* __restrict__ dst, int64_t rows,
-                                                          int cols, int cols_to) {
-  const int chunks = cols_to / 8;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= rows * chunks) return;
-  const int64_t r = i / chunks;
-  const int c0 = static_cast<int>(i % chunks) * 8;
-  T v[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = c0 + e < cols ? src[r * cols + c0 + e] : from_float<T>(0.f);
-  *reinterpret_cast<uint4*>(dst + r * cols_to + c0) = *reinterpret_cast<const uint4*>(v);
-}
-
-// A layer whose width N is not a multiple of the k-step (a 65-symbol vocabulary) cannot take
-// the pipelined kernels as it lies: rows of dY start at odd addresses, and both products
-// would go to the element-staged kernel (3-4 % of the matrix cores busy).  Here dY gets
-// zero columns and W zero rows up to the next multiple of 64 (copies of M x N and N x K
-// elements, small beside X and dX), the padded layer goes through the common launch, and
-// only the first N rows of dW are written.  The padding adds exact zeros to every sum.
-template <typename T>
-static int linear_bwd_padded(const void* dy, const void* x, const void* w, void* dx, void* dw, int64_t M, int64_t N,
-                             int64_t K, const void* relu_mask, bool dx_accumulate, hipStream_t stream, bool* done) {
+// The same for an fp32 layer small enough for gemm_f32_direct_kernel's tiles: dX, dW and db in one
+// launch, dW split along the rows only when its tiles leave CUs idle and there are rows enough
+// (then a finishing launch follows, or the sum is deferred).  Up to 2 GFLOP for both products: below
+// that the launches saved and the filled device outweigh the direct kernel's lower rate.
+// MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH=0 switches it off.
+static int linear_bwd_f32_one_launch(const void* dy, const void* x, const void* w, void* dx, void* dw, void* db, int64_t M,
+                                     int64_t N, int64_t K, const void* relu_mask, bool dx_accumulate, hipStream_t stream,
+                                     bool* done, bool* db_done) {
   *done = false;
-  const int64_t n_to = ceil_div(N, kG16BK) * kG16BK;
-  if (N % kG16BK == 0 || n_to > 2 * N || M % kG16BK || !mult8(K) || M < 1024 || n_to * K > 0x7fffffffLL) return MG_OK;
-  if (env_int("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", 1) == 0 || env_str("MOGRAD_HIP_GEMM16_PIPE")) return MG_OK;
-  Scratch dy_pad, w_pad;
-  MG_TRY(dy_pad.take(M * n_to * static_cast<int64_t>(sizeof(T))));
-  MG_TRY(w_pad.take(n_to * K * static_cast<int64_t>(sizeof(T))));
-  // W: rows appended to a row-major array, i.e. one row of N * K elements padded to n_to * K
-  const int64_t w_chunks = n_to * K / 8, dy_chunks = M * (n_to / 8);
-  hipLaunchKernelGGL((pad_columns_kernel<T>), dim3(static_cast<unsigned>(ceil_div(w_chunks, 256))), dim3(256), 0, stream,
-                     static_cast<const T*>(w), w_pad.as<T>(), static_cast<int64_t>(1), static_cast<int>(N * K),
-                     static_cast<int>(n_to * K));
+  *db_done = false;
+  if (env_int("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", 1) == 0) return MG_OK;
+  if (M <= 0 || N <= 0 || K <= 0 || 4.0 * M * N * K > 1e6 * env_int("MOGRAD_HIP_LINEAR_BWD_F32_MFLOP", 2000)) return MG_OK;
+  if (M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return MG_OK;
+  constexpr int kTile = 32;
+  const int64_t tiles_m = ceil_div(M, kTile), tiles_n = ceil_div(N, kTile), tiles_k = ceil_div(K, kTile);
+  const int64_t x_blocks = tiles_m * tiles_k, w_blocks = tiles_n * tiles_k;
+  // a large dX with next to no reduction (a 10-class head): see dispatch_f32
+  if (N < 32 && x_blocks >= 4 * device_info().cu_count) return MG_OK;
+  int splits = static_cast<int>(
+      std::max<int64_t>(1, std::min({ceil_div(device_info().cu_count, w_blocks), M / 256, static_cast<int64_t>(64)})));
+  const int k_per_split = static_cast<int>(ceil_div(ceil_div(M, splits), 64) * 64);
+  splits = static_cast<int>(ceil_div(M, k_per_split));
+  const int64_t n_dw = w_blocks * splits;
+  if (n_dw + x_blocks > 0x7fffffffLL) return MG_OK;
+  const int64_t numel = N * K;
+  Scratch partial, db_part;
+  if (splits > 1) {
+    MG_TRY(partial.take(splits * numel * static_cast<int64_t>(sizeof(float))));
+    if (db) MG_TRY(db_part.take(splits * N * static_cast<int64_t>(sizeof(float))));
+  }
+  const float* dyf = static_cast<const float*>(dy);
+  Gemm32Problem pw{dyf, static_cast<const float*>(x), nullptr, static_cast<float*>(dw), partial.as<float>(),
+                   static_cast<int>(N), static_cast<int>(K), static_cast<int>(M), N, K, K, 0, 0, numel,
+                   static_cast<int>(tiles_n), static_cast<int>(tiles_k), 1, k_per_split, splits,
+                   GemmEpilogue<float>{nullptr, nullptr, 0}};
+  pw.colsum = !db ? nullptr : splits > 1 ? db_part.as<float>() : static_cast<float*>(db);
+  const Gemm32Problem px{dyf, static_cast<const float*>(w), nullptr, static_cast<float*>(dx), nullptr,
+                         static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), N, K, K, 0, 0, M * K,
+                         static_cast<int>(tiles_m), static_cast<int>(tiles_k), 1, static_cast<int>(N), 1,
+                         GemmEpilogue<float>{dx_accumulate ? static_cast<const float*>(dx) : nullptr,
+                                             static_cast<const float*>(relu_mask), 0}};
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_dw + x_blocks)), dim3(256), 0, stream, pw, px,
+                       static_cast<int>(n_dw));
+  };
+  if (splits > 1) launch(linear_bwd_f32_kernel<kTile, true>);
+  else launch(linear_bwd_f32_kernel<kTile, false>);
   MG_LAUNCH_CHECK();
-  hipLaunchKernelGGL((pad_columns_kernel<T>), dim3(static_cast<unsigned>(ceil_div(dy_chunks, 256))), dim3(256), 0, stream,
-                     static_cast<const T*>(dy), dy_pad.as<T>(), M, static_cast<int>(N), static_cast<int>(n_to));
+  *done = true;
+  *db_done = db != nullptr;
+  if (splits == 1) return MG_OK;
+  const int dw_blocks = static_cast<int>(ceil_div(numel, 1024));
+  const int db_blocks = db ? static_cast<int>(ceil_div(N, 64)) : 0;
+  if (DeferredList* dl = deferred_current()) {
+    dl->push(kDeferSplitRows, partial.as<float>(), dw, numel, static_cast<int>(N), static_cast<int>(K), splits,
+             ceil_div(ceil_div(numel, 4), 1024));
+    dl->hold(partial);
+    if (db) {
+      dl->push(kDeferBiasRows, db_part.as<float>(), db, 0, 0, static_cast<int>(N), splits, ceil_div(db_blocks, 4));
+      dl->hold(db_part);
+    }
+    return MG_OK;
+  }
+  hipLaunchKernelGGL((linear_bwd_finish_kernel<float, false>), dim3(static_cast<unsigned>(dw_blocks + db_blocks)), dim3(256),
+                     0, stream, partial.as<float>(), static_cast<float*>(dw), static_cast<int>(N), numel, splits,
+                     static_cast<int>(K), dw_blocks, db_part.as<float>(), static_cast<float*>(db), splits,
+                     static_cast<int>(N));
   MG_LAUNCH_CHECK();
-  return linear_bwd_one_launch<T>(dy_pad.as<T>(), x, w_pad.as<T>(), dx, dw, M, n_to, K, relu_mask, dx_accumulate, stream,
-                                  done, N);
+  return MG_OK;
 }
 
 // *done: dX and dW are on their way; *db_done: so is db (else the caller sums dY's columns).
@@ -583,24 +754,12 @@ int linear_bwd_products(const void* dy, const void* x, const void* w, void* dx, 
                         bool* db_done, const LinearBwdLayerNorm* ln = nullptr) {
   *done = false;
   *db_done = false;
-  if (ln) {  // only the one launch has the LayerNorm continuation
-    if (dtype == MG_BF16)
-      return linear_bwd_one_launch<bf16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done, -1, db,
-                                           db_done, ln);
-    if (dtype == MG_F16)
-      return linear_bwd_one_launch<f16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done, -1, db,
-                                          db_done, ln);
-    return MG_OK;
-  }
-  if (dtype == MG_BF16) {
-    MG_TRY(linear_bwd_one_launch<bf16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done, -1, db,
-                                         db_done));
-    if (!*done) MG_TRY(linear_bwd_padded<bf16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done));
-  } else if (dtype == MG_F16) {
-    MG_TRY(linear_bwd_one_launch<f16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done, -1, db,
-                                        db_done));
-    if (!*done) MG_TRY(linear_bwd_padded<f16_t>(dy, x, w, dx, dw, M, N, K, relu_mask, dx_accumulate, stream, done));
-  }
+  if (dtype == MG_BF16)
+    return linear_bwd_one_launch<bf16_t>(dy, x, w, dx, dw, db, M, N, K, relu_mask, dx_accumulate, stream, done, db_done, ln);
+  if (dtype == MG_F16)
+    return linear_bwd_one_launch<f16_t>(dy, x, w, dx, dw, db, M, N, K, relu_mask, dx_accumulate, stream, done, db_done, ln);
+  if (dtype == MG_F32 && !ln)
+    return linear_bwd_f32_one_launch(dy, x, w, dx, dw, db, M, N, K, relu_mask, dx_accumulate, stream, done, db_done);
   return MG_OK;
 }
 

@@ -7,11 +7,6 @@
 //              "n-contiguous"  B[k * ldb + n]   (a row-major (K,N) array)
 // so Y = X W^T is (k,k), dX = dY W is (k,n) and dW = dY^T X is (m,n), all without
 // materialising a transpose.  C is row-major (M,N) with leading dimension ldc.
-//
-// fp32 kernel: 128x128 output tile per 256-thread workgroup, four waves in a 2x2 grid,
-// each wave a 64x64 tile as 2x2 v_mfma_f32_32x32x2_f32 accumulators (64 registers).
-// A K-chunk of 32 is staged through LDS: global -> registers (prefetch of the next
-// chunk overlaps the MFMAs of the current one) -> LDS -> MFMA operands.
 #pragma once
 
 #include <type_traits>
@@ -28,7 +23,6 @@ constexpr int kGemmBM = 128;
 constexpr int kGemmBN = 128;
 constexpr int kGemmBK = 32;
 constexpr int kGemmThreads = 256;
-constexpr int kKcStride = kGemmBK + 4;  // floats per LDS row of a k-contiguous operand tile
 
 // Workgroup -> output tile.  Consecutive workgroup ids go to different XCDs (id % 8), each
 // with its own L2; ids are regrouped so that one XCD works on a compact block of tiles
@@ -92,158 +86,6 @@ __device__ __forceinline__ T gemm_finish(float v, const GemmEpilogue<T>& ep, int
   T out = from_float<T>(v);
   if (ep.residual) out = from_float<T>(to_float(out) + to_float(ep.residual[index]));
   return out;
-}
-
-// Registers holding one thread's share of a 128 x 32 (or 32 x 128) operand tile.
-struct GemmStage {
-  float4 v[4];
-};
-
-// Loads the tile of an operand whose "outer" index (m for A, n for B) starts at `o0` and
-// whose k index starts at `k0`.  KC: element (o, k) at base[o * ld + k]; else base[k * ld + o].
-template <bool KC>
-__device__ __forceinline__ void gemm_load_tile(const float* __restrict__ base, int64_t ld, int o0, int k0, int O, int K,
-                                               GemmStage& st) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = t + i * kGemmThreads;
-    if constexpr (KC) {
-      const int o = o0 + idx / 8;
-      const int k = k0 + (idx % 8) * 4;
-      const int oc = min(o, O - 1);  // rows past the edge are never stored
-      st.v[i] = k < K ? *reinterpret_cast<const float4*>(base + static_cast<int64_t>(oc) * ld + k)
-                      : make_float4(0.f, 0.f, 0.f, 0.f);
-    } else {
-      const int k = k0 + idx / 32;
-      const int o = o0 + (idx % 32) * 4;
-      st.v[i] = (k < K && o < O) ? *reinterpret_cast<const float4*>(base + static_cast<int64_t>(k) * ld + o)
-                                 : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  }
-}
-
-template <bool KC>
-__device__ __forceinline__ void gemm_store_tile(float* __restrict__ lds, const GemmStage& st) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = t + i * kGemmThreads;
-    if constexpr (KC) {
-      *reinterpret_cast<float4*>(lds + (idx / 8) * kKcStride + (idx % 8) * 4) = st.v[i];
-    } else {
-      *reinterpret_cast<float4*>(lds + (idx / 32) * kGemmBM + (idx % 32) * 4) = st.v[i];
-    }
-  }
-}
-
-// MFMA operand values of one 32-wide tile for one group of 8 k-values: lane (o = l % 32,
-// h = l / 32) takes k = g*8 + h*4 + j for j = 0..3, so MFMA j of the group multiplies
-// k in {g*8 + j, g*8 + 4 + j}: each k is used exactly once, in an order that lets a
-// k-contiguous operand be read with one 128-bit LDS load.
-template <bool KC>
-__device__ __forceinline__ void gemm_read_frag(const float* __restrict__ lds, int o_base, int g, float (&f)[4]) {
-  const int lane = threadIdx.x % kWave;
-  const int o = o_base + lane % 32;
-  const int k = g * 8 + (lane / 32) * 4;
-  if constexpr (KC) {
-    const float4 r = *reinterpret_cast<const float4*>(lds + o * kKcStride + k);
-    f[0] = r.x; f[1] = r.y; f[2] = r.z; f[3] = r.w;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f[j] = lds[(k + j) * kGemmBM + o];
-  }
-}
-
-template <bool A_KC, bool B_KC, bool HAS_BIAS>
-__global__ __launch_bounds__(kGemmThreads, 2) void gemm_f32_mfma_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias, float* __restrict__ C,
-    int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb, int64_t bsc, int tiles_m,
-    int tiles_n, int total_work, GemmEpilogue<float> ep_in) {
-  __shared__ __attribute__((aligned(16))) float lds_a[kGemmBM * kKcStride];
-  __shared__ __attribute__((aligned(16))) float lds_b[kGemmBN * kKcStride];
-
-  const int tiles = tiles_m * tiles_n;
-  const float* const A_in = A;
-  const float* const B_in = B;
-  float* const C_in = C;
-  // The grid holds at most the workgroups that are resident at once; each takes output tiles
-  // work, work + gridDim.x, ...  Workgroups that share operand slabs then start every tile
-  // together, which keeps their fetches of the shared rows close in time.
-  for (int work = blockIdx.x; work < total_work; work += gridDim.x) {
-  const int batch = work / tiles;
-  int tm, tn;
-  gemm_tile_of_block(work % tiles, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * kGemmBM;
-  const int n0 = tn * kGemmBN;
-  A = A_in + batch * bsa;
-  B = B_in + batch * bsb;
-  C = C_in + batch * bsc;
-  GemmEpilogue<float> ep = ep_in;
-  if (ep.residual) ep.residual += batch * bsc;
-  if (ep.relu_mask) ep.relu_mask += batch * bsc;
-
-  const int wave = threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  const int wm = (wave / 2) * 64;
-  const int wn = (wave % 2) * 64;
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  GemmStage sa, sb;
-  gemm_load_tile<A_KC>(A, lda, m0, 0, M, K, sa);
-  gemm_load_tile<B_KC>(B, ldb, n0, 0, N, K, sb);
-
-  for (int k0 = 0; k0 < K; k0 += kGemmBK) {
-    gemm_store_tile<A_KC>(lds_a, sa);
-    gemm_store_tile<B_KC>(lds_b, sb);
-    __syncthreads();
-    if (k0 + kGemmBK < K) {
-      gemm_load_tile<A_KC>(A, lda, m0, k0 + kGemmBK, M, K, sa);
-      gemm_load_tile<B_KC>(B, ldb, n0, k0 + kGemmBK, N, K, sb);
-    }
-#pragma unroll
-    for (int g = 0; g < kGemmBK / 8; ++g) {
-      float fa[2][4], fb[2][4];
-      gemm_read_frag<A_KC>(lds_a, wm, g, fa[0]);
-      gemm_read_frag<A_KC>(lds_a, wm + 32, g, fa[1]);
-      gemm_read_frag<B_KC>(lds_b, wn, g, fb[0]);
-      gemm_read_frag<B_KC>(lds_b, wn + 32, g, fb[1]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < 2; ++tj)
-            acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[ti][j], fb[tj][j], acc[ti][tj], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-
-  // Accumulator element r of a lane is row (r/4)*8 + (lane/32)*4 + r%4, column lane%32.
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const int col = n0 + wn + tj * 32 + lane % 32;
-      if (col >= N) continue;
-      const float bv = HAS_BIAS ? bias[col] : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + ti * 32 + (r / 4) * 8 + (lane / 32) * 4 + (r % 4);
-        if (row < M) {
-          const int64_t at = static_cast<int64_t>(row) * ldc + col;
-          C[at] = gemm_finish<float>(acc[ti][tj][r] + bv, ep, at);
-        }
-      }
-    }
-  }  // tiles of this workgroup
 }
 
 // ------------------------------------------------------------------------------------
@@ -386,10 +228,18 @@ struct Gemm16Stage {
 
 // KC: element (o, k) at base[o * ld + k].  4 chunks of 8 k-values per thread.
 // else: element (o, k) at base[k * ld + o].  2 tasks per thread, each two k rows x 8 o.
-// RAGGED: leading dimension, extents or base address are not multiples of 8 elements, so
-// each chunk is assembled from eight 2-byte loads with per-element bounds.
+// Leading dimension, extents and base address may be anything.  A whole
+// chunk is one 16-byte load, at whatever even address it lies (the memory pipeline takes
+// global accesses of any alignment); only the chunk over the edge is assembled from 2-byte
+// loads with per-element bounds.  (All chunks by 2-byte loads: (1999, 768) = dY (1999, 1001) W
+// took 105 us, against 24 us.)
+typedef uint32_t gemm_u4_any __attribute__((ext_vector_type(4), aligned(2)));
 template <typename T>
 __device__ __forceinline__ uint4 gemm16_gather8(const T* __restrict__ p, int valid) {
+  if (valid >= 8) {
+    const gemm_u4_any v = *reinterpret_cast<const gemm_u4_any*>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  }
   const uint16_t* q = reinterpret_cast<const uint16_t*>(p);
   uint32_t w[4];
 #pragma unroll
@@ -401,11 +251,22 @@ __device__ __forceinline__ uint4 gemm16_gather8(const T* __restrict__ p, int val
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <typename T, bool KC, bool RAGGED>
+// The 16-byte chunk at any address, `valid` elements of it and zeros behind.
+template <typename T>
+__device__ __forceinline__ uint4 gemm_gather_chunk(const T* __restrict__ p, int valid) {
+  if constexpr (sizeof(T) == 2) {
+    return gemm16_gather8(p, valid);
+  } else {
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(p);
+    return make_uint4(q[0], valid > 1 ? q[1] : 0u, valid > 2 ? q[2] : 0u, valid > 3 ? q[3] : 0u);
+  }
+}
+
+template <typename T, bool KC>
 __device__ __forceinline__ void gemm16_load(const T* __restrict__ base, int64_t ld, int o0, int k0, int O, int k_end,
                                             Gemm16Stage& st) {
   const int t = threadIdx.x;
-  if constexpr (RAGGED && KC) {
+  if constexpr (KC) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int idx = t + i * kGemmThreads;
@@ -413,7 +274,7 @@ __device__ __forceinline__ void gemm16_load(const T* __restrict__ base, int64_t 
       const int k = k0 + (idx % 8) * 8;
       st.v[i] = gemm16_gather8(base + static_cast<int64_t>(o) * ld + k, k_end - k);
     }
-  } else if constexpr (RAGGED) {
+  } else {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int idx = t + i * kGemmThreads;
@@ -422,30 +283,6 @@ __device__ __forceinline__ void gemm16_load(const T* __restrict__ base, int64_t 
       const int o = o0 + oc * 8;
       st.v[2 * i] = gemm16_gather8(base + static_cast<int64_t>(k) * ld + o, k < k_end ? O - o : 0);
       st.v[2 * i + 1] = gemm16_gather8(base + static_cast<int64_t>(k + 1) * ld + o, k + 1 < k_end ? O - o : 0);
-    }
-  } else if constexpr (KC) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = t + i * kGemmThreads;
-      const int o = min(o0 + idx / 8, O - 1);  // rows past the edge are never stored
-      const int k = k0 + (idx % 8) * 8;
-      st.v[i] = k < k_end ? *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(o) * ld + k)
-                          : make_uint4(0, 0, 0, 0);
-    }
-  } else {
-    // 16 consecutive lanes read the 256 contiguous bytes of one k row: whole cache lines.
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = t + i * kGemmThreads;
-      const int oc = idx % 16, kp = idx / 16;
-      const int k = k0 + 2 * kp;
-      const int o = o0 + oc * 8;
-      const bool o_ok = o < O;
-      st.v[2 * i] = (o_ok && k < k_end) ? *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(k) * ld + o)
-                                        : make_uint4(0, 0, 0, 0);
-      st.v[2 * i + 1] = (o_ok && k + 1 < k_end)
-                            ? *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(k + 1) * ld + o)
-                            : make_uint4(0, 0, 0, 0);
     }
   }
 }
@@ -488,11 +325,26 @@ __device__ __forceinline__ uint4 gemm16_frag(const uint16_t* __restrict__ lds, i
   return *reinterpret_cast<const uint4*>(lds + row * kG16Stride + g * 8);
 }
 
+// Eight consecutive elements from and to any even address.
+template <typename T>
+__device__ __forceinline__ void gemm16_load8(const T* p, float (&v)[8]) {
+  const gemm_u4_any r = *reinterpret_cast<const gemm_u4_any*>(p);
+  const uint32_t w[4] = {r[0], r[1], r[2], r[3]};
+  VecIO<T, 8>::unpack(w, v);
+}
+template <typename T>
+__device__ __forceinline__ void gemm16_store8(T* p, const float (&v)[8]) {
+  gemm_u4_any r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = gemm16_pack2<T>(v[2 * e], v[2 * e + 1]);
+  *reinterpret_cast<gemm_u4_any*>(p) = r;
+}
+
 // Output of one 128x128 tile from the four waves' accumulators (wave tile 64x64 at (wm, wn)).
 // The accumulators have lanes along n and registers along m, so a direct store writes
-// 2-byte elements.  When rows of C can be written 16 bytes at a time, each wave instead
-// transposes its tile through `mine`, 64 rows of kG16Stride elements of LDS that no wave
-// reads any more, and stores eight elements per lane.  SPLIT_K: fp32 partial tiles go to
+// 2-byte elements.  Each wave instead transposes its tile through `mine`, 64 rows of kG16Stride
+// elements of LDS that no wave reads any more, and stores eight elements per lane, at whatever
+// address the row starts (only the chunk over the right edge goes out in 2-byte elements).  SPLIT_K: fp32 partial tiles go to
 // partial[(split * batches + batch), M, N].
 template <typename T, bool HAS_BIAS, bool SPLIT_K>
 __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], uint16_t* __restrict__ mine,
@@ -533,8 +385,7 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
                                                           acc[ti][tj][4 * g + 2], acc[ti][tj][4 * g + 3]);
     return;
   } else {
-    const bool wide_out = (N % 8 == 0) && (ldc % 8 == 0) && (bsc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-    if (wide_out) {
+    {
       // An accumulator holds one column and, per group of four registers, four consecutive
       // rows.  Two lanes with neighbouring columns swap packed pairs of rows, so that the even
       // lane holds (own, neighbour) of the first row of a pair and the odd lane (neighbour,
@@ -585,6 +436,17 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
       const uint16_t* src = mine + rl0 * kG16Stride + ch * 8;
       const T* rbase = ep.residual;
       const T* mbase = ep.relu_mask;
+      if (col + 8 > N) {  // the chunk over the right edge, element by element
+        for (int i = 0; i < 8 && row0 + 8 * i < M; ++i)
+          for (int e = 0; col + e < N; ++e) {
+            const int64_t at = at0 + i * step + e;
+            float v = to_float(reinterpret_cast<const T*>(src + i * 8 * kG16Stride)[e]);
+            if (mbase) v = to_float(mbase[at]) > 0.f ? v : 0.f;
+            if (rbase) v += to_float(rbase[at]);
+            C[at] = from_float<T>(v);
+          }
+        return;
+      }
       if (!rbase && !mbase) {
         T* dst = C + at0;
         uint4 v[8];  // all eight LDS reads first: their latencies overlap
@@ -592,7 +454,10 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
         for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const uint4*>(src + i * 8 * kG16Stride);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          if (row0 + 8 * i < M) *reinterpret_cast<uint4*>(dst + i * step) = v[i];
+          if (row0 + 8 * i < M) {
+            const gemm_u4_any out = {v[i].x, v[i].y, v[i].z, v[i].w};
+            *reinterpret_cast<gemm_u4_any*>(dst + i * step) = out;
+          }
         return;
       }
 #pragma unroll
@@ -603,37 +468,20 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
         VecIO<T, 8>::load(reinterpret_cast<const T*>(src + i * 8 * kG16Stride), v);
         if (mbase) {
           float mk[8];
-          VecIO<T, 8>::load(mbase + at, mk);
+          gemm16_load8(mbase + at, mk);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = mk[e] > 0.f ? v[e] : 0.f;
         }
         if (rbase) {
           float rs[8];
-          VecIO<T, 8>::load(rbase + at, rs);
+          gemm16_load8(rbase + at, rs);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] += rs[e];
         }
-        VecIO<T, 8>::store(C + at, v);
+        gemm16_store8(C + at, v);
       }
-      return;
     }
   }
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const int col = n0 + wn + tj * 32 + lane % 32;
-      if (col >= N) continue;
-      const float bv = HAS_BIAS ? to_float(bias[col]) : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + ti * 32 + (r / 4) * 8 + (lane / 32) * 4 + (r % 4);
-        if (row < M) {
-          const int64_t at = batch * bsc + static_cast<int64_t>(row) * ldc + col;
-          C[at] = gemm_finish<T>(acc[ti][tj][r] + bv, ep, at);
-        }
-      }
-    }
 }
 
 // What a product's output tile needs to continue as a LayerNorm backward (see gemm16_ln_bwd_tile).
@@ -783,7 +631,7 @@ __device__ __forceinline__ void gemm16_ln_bwd_tile(const floatx16 (&acc)[2][2], 
   }
 }
 
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool RAGGED>
+template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
     const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ bias, T* __restrict__ C,
     float* __restrict__ partial, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb,
@@ -830,16 +678,16 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
     }
   }
   Gemm16Stage sa, sb;
-  gemm16_load<T, A_KC, RAGGED>(A, lda, m0, k_begin, M, k_end, sa);
-  gemm16_load<T, B_KC, RAGGED>(B, ldb, n0, k_begin, N, k_end, sb);
+  gemm16_load<T, A_KC>(A, lda, m0, k_begin, M, k_end, sa);
+  gemm16_load<T, B_KC>(B, ldb, n0, k_begin, N, k_end, sb);
 
   for (int k0 = k_begin; k0 < k_end; k0 += kG16BK) {
     gemm16_store<A_KC>(lds_a, sa);
     gemm16_store<B_KC>(lds_b, sb);
     __syncthreads();
     if (k0 + kG16BK < k_end) {
-      gemm16_load<T, A_KC, RAGGED>(A, lda, m0, k0 + kG16BK, M, k_end, sa);
-      gemm16_load<T, B_KC, RAGGED>(B, ldb, n0, k0 + kG16BK, N, k_end, sb);
+      gemm16_load<T, A_KC>(A, lda, m0, k0 + kG16BK, M, k_end, sa);
+      gemm16_load<T, B_KC>(B, ldb, n0, k0 + kG16BK, N, k_end, sb);
     }
 #pragma unroll
     for (int ks = 0; ks < kG16BK / 16; ++ks) {
@@ -949,6 +797,23 @@ __device__ __forceinline__ void gemm16_pipe_issue(const uint16_t* base, const in
   }
 }
 
+// The last, short step of a reduction that is no multiple of BK (`rem` k left, whole chunks of 8
+// for a k-contiguous operand): the same chunks through registers, zeros past the end, so nothing
+// beyond the operand is read and the step multiplies like any other.  The compiler waits for
+// these loads and with them for every older copy, once per tile.
+template <bool KC, int BK, int ROWS, int NW>
+__device__ __forceinline__ void gemm16_pipe_tail(const uint16_t* base, const int64_t* src, int rem, char* lds_step) {
+  constexpr int CPR = BK / 8, CPK = ROWS / 8;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+#pragma unroll
+  for (int i = 0; i < gemm16_pipe_requests(ROWS, BK, NW); ++i) {
+    const int slot = (i * NW + wave) * kWave + lane;
+    const int k = KC ? ((slot % CPR) ^ ((slot / CPR / (16 / CPR)) % CPR)) * 8 : slot / CPK;
+    const uint4 v = k < rem ? *reinterpret_cast<const uint4*>(base + src[i]) : make_uint4(0, 0, 0, 0);
+    *reinterpret_cast<uint4*>(lds_step + slot * 16) = v;
+  }
+}
+
 // MFMA operand fragment: row o_base + lane % 32, k = ks * 16 + (lane / 32) * 8 .. + 7.
 template <bool KC, int BK, int ROWS>
 __device__ __forceinline__ uint4 gemm16_pipe_frag(const char* __restrict__ lds_step, int o_base, int ks, int lane) {
@@ -1005,6 +870,7 @@ struct Gemm16Problem {
   // first tile column also sum their A tiles over k, i.e. dY over its rows, and leave one
   // partial row of the bias gradient per K range at colsum_part[split * M + m].
   float* colsum_part = nullptr;
+  T* colsum = nullptr;  // not split: the sums themselves
   // The partial tiles are read back much later (their sum is deferred to the end of a training
   // step): store them past the caches.
   bool partial_stream = false;
@@ -1016,7 +882,7 @@ struct Gemm16Problem {
 // gemm16_pipe_lds_bytes(BK, NSTAGE, TM, TN) bytes, aligned to 1024.  The output tile is
 // TM x TN, (TM / 64) x (TN / 64) waves with 64 x 64 each; pr.tiles_n counts tiles of TN columns.
 template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, int BK, int NSTAGE, int TM = 128,
-          int TN = kGemmBN, bool LN_BWD = false>
+          int TN = kGemmBN, bool LN_BWD = false, bool COLSUM = SPLIT_K>
 __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
   static_assert(NSTAGE >= 2 && NSTAGE <= 4 && (BK == 32 || BK == 64) && (TM == 128 || TM == 256), "stages");
   static_assert(TN % 128 == 0 && (!SPLIT_K || TM == 128), "partial tiles are 128 x 128");
@@ -1051,7 +917,8 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
   const int n0 = tn * TN;
   const int k_begin = SPLIT_K ? split * k_per_split : 0;
   const int k_end = SPLIT_K ? min(K, k_begin + k_per_split) : K;
-  const int steps = (k_end - k_begin) / BK;
+  const int full_steps = (k_end - k_begin) / BK, rem = (k_end - k_begin) % BK;
+  const int steps = full_steps + (rem > 0 ? 1 : 0);
   A += batch * bsa + (A_KC ? static_cast<int64_t>(k_begin) : k_begin * lda);
   B += batch * bsb + (B_KC ? static_cast<int64_t>(k_begin) : k_begin * ldb);
   const int64_t a_step = A_KC ? BK : BK * lda;
@@ -1075,8 +942,8 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
 
   // Column sums of the A tiles (see Gemm16Problem::colsum_part): a thread of the first four
   // waves takes one 16-byte chunk (8 of the tile's 128 m) of every 16th k-row.
-  constexpr bool CAN_COLSUM = SPLIT_K && !A_KC && TM == 128;
-  const bool colsum = CAN_COLSUM && pr.colsum_part != nullptr && tn == 0;
+  constexpr bool CAN_COLSUM = COLSUM && !A_KC && TM == 128;
+  const bool colsum = CAN_COLSUM && (SPLIT_K ? pr.colsum_part != nullptr : pr.colsum != nullptr) && tn == 0;
   const bool cs_thread = threadIdx.x < 256;
   const int cs_chunk = threadIdx.x % 16, cs_row = threadIdx.x / 16;
   float cs_acc[8];
@@ -1089,6 +956,11 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
   gemm16_pipe_sources<A_KC, BK, TM, NWA>(lda, m0, M, src_a);
   gemm16_pipe_sources<B_KC, BK, TN, NWB>(ldb, n0, N, src_b);
   auto request = [&](int step, int copy) {
+    if (step == full_steps) {
+      if (copies_a) gemm16_pipe_tail<A_KC, BK, TM, NWA>(a16 + step * a_step, src_a, rem, lds + copy * OP);
+      if (copies_b) gemm16_pipe_tail<B_KC, BK, TN, NWB>(b16 + step * b_step, src_b, rem, lds + copy * OP + OPA);
+      return;
+    }
     if (copies_a) gemm16_pipe_issue<NIA, NWA>(a16 + step * a_step, src_a, lds + copy * OP);
     if (copies_b) gemm16_pipe_issue<NIB, NWB>(b16 + step * b_step, src_b, lds + copy * OP + OPA);
   };
@@ -1115,7 +987,7 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
   int cur = 0, nxt = NSTAGE - 1;
   for (int it = 0; it < steps; ++it) {
     // all but the NSTAGE - 2 younger steps' requests
-    if (it + NSTAGE - 2 >= steps || NSTAGE == 2) MG_WAIT_VMCNT(0);
+    if (it + NSTAGE - 2 >= full_steps || NSTAGE == 2) MG_WAIT_VMCNT(0);
     else if (per_step == NIA + NIB) MG_WAIT_VMCNT((NIA + NIB) * (NSTAGE - 2));
     else if (per_step == NIB) MG_WAIT_VMCNT(NIB * (NSTAGE - 2));
     else if (per_step == NIA) MG_WAIT_VMCNT(NIA * (NSTAGE - 2));
@@ -1178,7 +1050,8 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sum += red[r * kPitch + threadIdx.x];
-        pr.colsum_part[static_cast<int64_t>(split) * M + m0 + threadIdx.x] = sum;
+        if constexpr (SPLIT_K) pr.colsum_part[static_cast<int64_t>(split) * M + m0 + threadIdx.x] = sum;
+        else pr.colsum[m0 + threadIdx.x] = from_float<T>(sum);
       }
       __syncthreads();
     }
@@ -1391,6 +1264,17 @@ __global__ __launch_bounds__(2 * TN, gemm16_pipe_occupancy(BK, NSTAGE, 128, TN))
   else gemm16_pipe_block<T, true, false, false, false, BK, NSTAGE, 128, TN>(lds, bid - n_dw, dx);
 }
 
+// The same launch for layers of few rows, whose dW is not split: dW and db are written by the
+// workgroups themselves and nothing follows (a small layer's backward is as long as its launches).
+template <typename T>
+__global__ __launch_bounds__(kGemmThreads, gemm16_pipe_occupancy(64, 2, 128)) void linear_bwd_short_16bit_kernel(
+    Gemm16Problem<T> dw, Gemm16Problem<T> dx, int n_dw) {
+  __shared__ __attribute__((aligned(1024))) char lds[gemm16_pipe_lds_bytes(64, 2, 128)];
+  const int bid = blockIdx.x;
+  if (bid < n_dw) gemm16_pipe_block<T, false, false, false, false, 64, 2, 128, 128, false, true>(lds, bid, dw);
+  else gemm16_pipe_block<T, true, false, false, false, 64, 2>(lds, bid - n_dw, dx);
+}
+
 // The same launch with the dX tiles (128 x 384: whole rows of a 384-wide layer input) continuing
 // as the backward of the LayerNorm that produced the layer's input (gemm16_ln_bwd_tile).
 template <typename T>
@@ -1404,31 +1288,34 @@ __global__ __launch_bounds__(2 * kGemmWideBN, 1) void linear_bwd_ln_16bit_kernel
 
 // ------------------------------------------------------------------------------------
 // fp32 product with the tiles copied global memory -> LDS by `global_load_lds_dwordx4`, two
-// copies of each 128 x 32 tile: the copy of k-step i + 1 runs under the MFMAs of step i with
-// one barrier per step and no registers or VALU work spent on staging.  Same tiles, same
-// wave layout, same k order inside a step as gemm_f32_mfma_kernel (MFMA j of k-group g
-// multiplies k in {g*8 + j, g*8 + 4 + j}), so the two kernels give identical bits.
-// Requires K % 32 == 0 on top of that kernel's alignment conditions.
+// copies of each TS x 32 tile: the copy of k-step i + 1 runs under the MFMAs of step i with
+// one barrier per step and no registers or VALU work spent on staging.  TS is 128 (wave tiles of
+// 64 x 64: 85-88 % of the matrix pipe at 2048 x 4096 x 4096) or, for outputs with too few such
+// tiles for the device, 64 (wave tiles of 32 x 32).  A product of K steps and a remainder ends on a short step whose tiles come
+// through registers, zeros behind (gemm32_pipe_tail).
 //
-// LDS image of one operand's step (16 KB):
-//   k-contiguous: [128 rows][8 chunks of 4 k], chunk c of row r at position c ^ (r/2 % 8)
+// MFMA j of k-group g multiplies k in {g*8 + j, g*8 + 4 + j}: lane (o = l % 32, h = l / 32) takes
+// k = g*8 + h*4 + j for j = 0..3, so a k-contiguous operand is read with one 128-bit LDS load.
+//
+// LDS image of one operand's step:
+//   k-contiguous: [TS rows][8 chunks of 4 k], chunk c of row r at position c ^ (r/2 % 8)
 //     (sixteen consecutive rows of a 128-bit fragment read hit sixteen bank groups);
-//   otherwise: [32 k][32 chunks of 4 rows], chunk c of k-row kk at position
+//   otherwise: [32 k][TS / 4 chunks of 4 rows], chunk c of k-row kk at position
 //     c ^ (8 * (kk/4 % 2)): the two halves of a wave read k and k + 4 of the same rows, 128
 //     bytes apart in the banks.
 // ------------------------------------------------------------------------------------
 
-template <bool KC>
-__device__ __forceinline__ void gemm32_pipe_sources(int64_t ld, int o0, int O, int64_t (&src)[4]) {
+template <bool KC, int TS>
+__device__ __forceinline__ void gemm32_pipe_sources(int64_t ld, int o0, int O, int64_t (&src)[TS / 32]) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < TS / 32; ++i) {
     const int slot = (i * 4 + wave) * kWave + lane;  // 16-byte position in the LDS image
     if constexpr (KC) {
       const int r = slot / 8, c = (slot % 8) ^ ((r / 2) % 8);
       src[i] = static_cast<int64_t>(min(o0 + r, O - 1)) * ld + c * 4;  // rows past the edge are never stored
     } else {
-      const int kk = slot / 32, c = (slot % 32) ^ (8 * ((kk / 4) % 2));
+      const int kk = slot / (TS / 4), c = (slot % (TS / 4)) ^ (8 * ((kk / 4) % 2));
       const int o = o0 + c * 4;
       src[i] = static_cast<int64_t>(kk) * ld + (o < O ? o : o0);
     }
@@ -1436,19 +1323,33 @@ __device__ __forceinline__ void gemm32_pipe_sources(int64_t ld, int o0, int O, i
 }
 
 // See gemm16_pipe_issue for why this is assembly.
+template <int NI>
 __device__ __forceinline__ void gemm32_pipe_issue(const float* base, const int64_t* src, char* lds_step) {
   using lds_ptr = __attribute__((address_space(3))) char*;
   const int wave = threadIdx.x / kWave;
   const unsigned dst = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)lds_step)) + wave * 1024;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const unsigned dst_i = __builtin_amdgcn_readfirstlane(dst + i * 4096);
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst_i), "v"(base + src[i]) : "memory");
   }
 }
 
-// MFMA operand values of one 32-wide tile for k-group g (see gemm_read_frag).
-template <bool KC>
+// The short last step (`rem` k left): see gemm16_pipe_tail.
+template <bool KC, int TS>
+__device__ __forceinline__ void gemm32_pipe_tail(const float* base, const int64_t* src, int rem, char* lds_step) {
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+#pragma unroll
+  for (int i = 0; i < TS / 32; ++i) {
+    const int slot = (i * 4 + wave) * kWave + lane;
+    const int k = KC ? ((slot % 8) ^ ((slot / 16) % 8)) * 4 : slot / (TS / 4);
+    const float4 v = k < rem ? *reinterpret_cast<const float4*>(base + src[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float4*>(lds_step + slot * 16) = v;
+  }
+}
+
+// MFMA operand values of one 32-wide tile for k-group g.
+template <bool KC, int TS>
 __device__ __forceinline__ void gemm32_pipe_frag(const char* __restrict__ lds_step, int o_base, int g, int lane,
                                                  float (&f)[4]) {
   const int o = o_base + lane % 32;
@@ -1458,42 +1359,47 @@ __device__ __forceinline__ void gemm32_pipe_frag(const char* __restrict__ lds_st
     f[0] = r.x; f[1] = r.y; f[2] = r.z; f[3] = r.w;
   } else {
     const int kk = g * 8 + (lane / 32) * 4;  // (kk / 4) % 2 == lane / 32 for all four k of this lane
-    const char* at = lds_step + kk * 512 + ((((o / 4) ^ (8 * (lane / 32))) * 16) + (o % 4) * 4);
+    const char* at = lds_step + kk * (TS * 4) + ((((o / 4) ^ (8 * (lane / 32))) * 16) + (o % 4) * 4);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const float*>(at + j * 512);
+    for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const float*>(at + j * (TS * 4));
   }
 }
 
 // SPLIT_K: a work item is (K range, batch, tile); the fp32 partial tiles go to
 // partial[(split * batches + batch), M, N] and gemm_splitk_reduce_kernel adds them up in a
 // fixed order (for outputs with too few tiles to fill the device, e.g. a 10-class head).
-template <bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
-__global__ __launch_bounds__(kGemmThreads, 2) void gemm_f32_pipe_kernel(
+template <bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, int TS>
+__global__ __launch_bounds__(kGemmThreads, TS == 128 ? 2 : 4) void gemm_f32_pipe_kernel(
     const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias, float* __restrict__ C,
     float* __restrict__ partial, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb,
     int64_t bsc, int tiles_m, int tiles_n, int batches, int k_per_split, int total_work, GemmEpilogue<float> ep_in) {
-  constexpr int OP = kGemmBM * kGemmBK * 4;  // bytes of one operand's step
+  constexpr int OP = TS * kGemmBK * 4;  // bytes of one operand's step
+  constexpr int NT = TS / 64;           // 32 x 32 tiles of a wave along either axis
+  constexpr int NI = TS / 32;           // copy requests per thread, operand and step
   __shared__ __attribute__((aligned(1024))) char lds[2][2][OP];
 
   const int tiles = tiles_m * tiles_n;
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
-  const int wm = (wave / 2) * 64;
-  const int wn = (wave % 2) * 64;
+  const int wm = (wave / 2) * (TS / 2);
+  const int wn = (wave % 2) * (TS / 2);
   const int64_t a_step = A_KC ? kGemmBK : kGemmBK * lda;
   const int64_t b_step = B_KC ? kGemmBK : kGemmBK * ldb;
   // The grid holds at most the workgroups that are resident at once; each takes output tiles
-  // work, work + gridDim.x, ... (see gemm_f32_mfma_kernel).
+  // work, work + gridDim.x, ...  Workgroups that share operand slabs then start every tile
+  // together, which keeps their fetches of the shared rows close in time.
   for (int work = blockIdx.x; work < total_work; work += gridDim.x) {
     const int split = SPLIT_K ? work / (tiles * batches) : 0;
     const int in_split = SPLIT_K ? work % (tiles * batches) : work;
     const int batch = in_split / tiles;
     int tm, tn;
     gemm_tile_of_block(in_split % tiles, tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * kGemmBM;
-    const int n0 = tn * kGemmBN;
+    const int m0 = tm * TS;
+    const int n0 = tn * TS;
     const int k_begin = SPLIT_K ? split * k_per_split : 0;
-    const int steps = (SPLIT_K ? min(K - k_begin, k_per_split) : K) / kGemmBK;
+    const int k_here = SPLIT_K ? min(K - k_begin, k_per_split) : K;
+    const int full_steps = k_here / kGemmBK, rem = k_here % kGemmBK;
+    const int steps = full_steps + (rem > 0 ? 1 : 0);
     const float* a = A + batch * bsa + (A_KC ? static_cast<int64_t>(k_begin) : k_begin * lda);
     const float* b = B + batch * bsb + (B_KC ? static_cast<int64_t>(k_begin) : k_begin * ldb);
     float* c = C + batch * bsc;
@@ -1501,19 +1407,27 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_f32_pipe_kernel(
     if (ep.residual) ep.residual += batch * bsc;
     if (ep.relu_mask) ep.relu_mask += batch * bsc;
 
-    floatx16 acc[2][2];
+    floatx16 acc[NT][NT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    int64_t src_a[4], src_b[4];
-    gemm32_pipe_sources<A_KC>(lda, m0, M, src_a);
-    gemm32_pipe_sources<B_KC>(ldb, n0, N, src_b);
-    gemm32_pipe_issue(a, src_a, lds[0][0]);
-    gemm32_pipe_issue(b, src_b, lds[0][1]);
+    int64_t src_a[NI], src_b[NI];
+    gemm32_pipe_sources<A_KC, TS>(lda, m0, M, src_a);
+    gemm32_pipe_sources<B_KC, TS>(ldb, n0, N, src_b);
+    auto request = [&](int step, int copy) {
+      if (step == full_steps) {
+        gemm32_pipe_tail<A_KC, TS>(a + step * a_step, src_a, rem, lds[copy][0]);
+        gemm32_pipe_tail<B_KC, TS>(b + step * b_step, src_b, rem, lds[copy][1]);
+        return;
+      }
+      gemm32_pipe_issue<NI>(a + step * a_step, src_a, lds[copy][0]);
+      gemm32_pipe_issue<NI>(b + step * b_step, src_b, lds[copy][1]);
+    };
+    request(0, 0);
     for (int it = 0; it < steps; ++it) {
       const int cur = it & 1;
       // This wave's copies of step `it` have landed; the barrier covers the other waves' and
@@ -1521,33 +1435,29 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_f32_pipe_kernel(
       // would be the same here, every copy being waited for, but costs a fence.)
       MG_WAIT_VMCNT(0);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (it + 1 < steps) {
-        gemm32_pipe_issue(a + (it + 1) * a_step, src_a, lds[cur ^ 1][0]);
-        gemm32_pipe_issue(b + (it + 1) * b_step, src_b, lds[cur ^ 1][1]);
-      }
+      if (it + 1 < steps) request(it + 1, cur ^ 1);
       const char* la = lds[cur][0];
       const char* lb = lds[cur][1];
       // The fragments of k-group g + 1 are requested before the products of group g.
-      float fa[2][2][4], fb[2][2][4];
-      gemm32_pipe_frag<A_KC>(la, wm, 0, lane, fa[0][0]);
-      gemm32_pipe_frag<A_KC>(la, wm + 32, 0, lane, fa[0][1]);
-      gemm32_pipe_frag<B_KC>(lb, wn, 0, lane, fb[0][0]);
-      gemm32_pipe_frag<B_KC>(lb, wn + 32, 0, lane, fb[0][1]);
+      float fa[2][NT][4], fb[2][NT][4];
+      auto frags = [&](int buf, int g) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          gemm32_pipe_frag<A_KC, TS>(la, wm + 32 * i, g, lane, fa[buf][i]);
+          gemm32_pipe_frag<B_KC, TS>(lb, wn + 32 * i, g, lane, fb[buf][i]);
+        }
+      };
+      frags(0, 0);
 #pragma unroll
       for (int g = 0; g < kGemmBK / 8; ++g) {
-        const int p = g % 2, n = p ^ 1;
-        if (g + 1 < kGemmBK / 8) {
-          gemm32_pipe_frag<A_KC>(la, wm, g + 1, lane, fa[n][0]);
-          gemm32_pipe_frag<A_KC>(la, wm + 32, g + 1, lane, fa[n][1]);
-          gemm32_pipe_frag<B_KC>(lb, wn, g + 1, lane, fb[n][0]);
-          gemm32_pipe_frag<B_KC>(lb, wn + 32, g + 1, lane, fb[n][1]);
-        }
+        const int p = g % 2;
+        if (g + 1 < kGemmBK / 8) frags(p ^ 1, g + 1);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int ti = 0; ti < 2; ++ti)
+          for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
-            for (int tj = 0; tj < 2; ++tj)
+            for (int tj = 0; tj < NT; ++tj)
               acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[p][ti][j], fb[p][tj][j], acc[ti][tj], 0, 0, 0);
       }
     }
@@ -1556,9 +1466,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_f32_pipe_kernel(
 
     // Accumulator element r of a lane is row (r/4)*8 + (lane/32)*4 + r%4, column lane%32.
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
+    for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
-      for (int tj = 0; tj < 2; ++tj) {
+      for (int tj = 0; tj < NT; ++tj) {
         const int col = n0 + wn + tj * 32 + lane % 32;
         if (col >= N) continue;
         const float bv = (HAS_BIAS && !SPLIT_K) ? bias[col] : 0.f;
@@ -1716,8 +1626,9 @@ __device__ __forceinline__ void linear_bwd_db_block(float* __restrict__ sums_, i
 // the K ranges of dW (gemm_splitk_reduce_block), the rest sum the `groups` partial rows of
 // the bias gradient that the launch left (one per K range), 64 columns per workgroup,
 // every fourth row per 64 threads, then (t0 + t1) + (t2 + t3).  Fixed order, no atomics.
-// dw_blocks = ceil(slice / 1024): a thread sums four consecutive values of a partial tile.
-template <typename T>
+// dw_blocks = ceil(slice / 1024): a thread sums four consecutive values of a partial tile (TILED) or
+// of a partial (dw_rows, K) matrix.
+template <typename T, bool TILED = true>
 __global__ __launch_bounds__(256) void linear_bwd_finish_kernel(const float* __restrict__ partial, T* __restrict__ dw,
                                                                 int dw_rows, int64_t slice, int splits, int K,
                                                                 int dw_blocks, const float* __restrict__ db_part,
@@ -1726,7 +1637,7 @@ __global__ __launch_bounds__(256) void linear_bwd_finish_kernel(const float* __r
   const int bid = blockIdx.x;
   if (bid < dw_blocks) {
     // dW is (dw_rows, K); the partial tiles cover the (N, K) product of the launch
-    gemm_splitk_reduce_group<T, false, true>(static_cast<int64_t>(bid) * 256 + threadIdx.x, partial,
+    gemm_splitk_reduce_group<T, false, TILED>(static_cast<int64_t>(bid) * 256 + threadIdx.x, partial,
                                              static_cast<const T*>(nullptr), dw, slice, slice, splits, K,
                                              GemmEpilogue<T>{nullptr, nullptr, 0}, dw_rows, (K + kGemmBN - 1) / kGemmBN);
     return;

@@ -22,6 +22,7 @@ namespace mg {
 
 enum DeferredKind : int {
   kDeferSplitK = 0,  // K ranges of a split dW, partial tiles in accumulator order
+  kDeferSplitRows,   // K ranges of a split dW, partial (rows, cols) matrices
   kDeferBiasRows,    // partial rows of a bias gradient
   kDeferSlab,        // (groups, cols) partials, slab form
   kDeferCw64,        // (groups, cols) partials, 64 / 32 / 16 columns per 256 threads
@@ -33,7 +34,7 @@ enum DeferredKind : int {
 struct DeferredJob {
   const float* part;
   void* out;
-  int64_t slice;  // kDeferSplitK: floats per K range
+  int64_t slice;  // kDeferSplitK, kDeferSplitRows: floats per K range
   int kind;
   int out_dtype;
   int rows;    // kDeferSplitK: rows of dW to write

@@ -1,0 +1,66 @@
+"""Products and Linear backwards whose sizes sit at the edges of the kernels' ranges: reductions
+that end on a short step, widths that are no multiple of a 16-byte chunk, outputs of a few tiles
+(fp32 straight from memory, 16 x 16 and 32 x 32), of 64 x 64 and of 128 x 128 tiles, and rows few enough
+that nothing is split.  All against float64 products of the rounded inputs."""
+import numpy as np
+import pytest
+
+from helpers import assert_close, normal
+
+pytestmark = pytest.mark.gpu
+
+from mograd_amd import BF16, F16, F32, AnyBuffer  # noqa: E402
+from mograd_amd.runtime import round_to_dtype  # noqa: E402
+
+RT = {F32: 1e-5, F16: 2e-3, BF16: 1.6e-2}
+SHAPES = [(1, 1, 1), (5, 3, 4), (64, 10, 256), (33, 17, 65), (130, 65, 100), (64, 256, 784), (333, 257, 129), (200, 136, 264),
+          (1000, 72, 88), (1023, 264, 8), (1025, 96, 384), (1999, 1001, 767), (2587, 256, 256), (1056, 1152, 384)]
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_linear_forward_and_backward(device, dtype, M, N, K):
+    lib, st, rt = device.lib, device.stream, RT[dtype]
+    x = np.maximum(round_to_dtype(normal(60, 0, (M, K)), dtype), 0)
+    w = round_to_dtype(normal(60, 1, (N, K), std=0.1), dtype)
+    b = round_to_dtype(normal(60, 2, (N,), std=0.1), dtype)
+    dy = round_to_dtype(normal(60, 3, (M, N), std=0.5), dtype)
+    prior = round_to_dtype(normal(60, 4, (M, K)), dtype)
+    bx, bw, bb, bdy = (AnyBuffer.from_numpy(device, a, dtype) for a in (x, w, b, dy))
+    dx = AnyBuffer.from_numpy(device, prior, dtype)
+    y, dw, db = (AnyBuffer.create(dtype, device, n) for n in (M * N, N * K, N))
+    P = lambda t: t.data_ptr()  # noqa: E731
+    lib.mg_matmul_bias_relu_bt(P(bx), P(bw), P(bb), P(y), 1, M, N, K, K, 1, K, 1, M * K, N * K, dtype, st)
+    lib.mg_linear_bwd_fused(P(bdy), P(bx), P(bw), P(dx), P(dw), P(db), M, N, K, 1, 1, dtype, st)
+    x, w, b, dy, prior = (a.astype(np.float64) for a in (x, w, b, dy, prior))
+    want = np.maximum(x @ w.T + b, 0)
+    assert_close(y.to_numpy((M, N)), want, rt, rt * max(np.abs(want).max(), 1e-3), "y")
+    want = dy @ w * (x > 0)
+    assert_close(dx.to_numpy((M, K)), prior + want, 2 * rt, 2 * rt * max(np.abs(want).max(), 1e-3), "dx")
+    want = dy.T @ x
+    assert_close(dw.to_numpy((N, K)), want, rt, rt * max(np.abs(want).max(), 1e-3), "dw")
+    want = dy.sum(axis=0)
+    assert_close(db.to_numpy(), want, rt, rt * max(np.abs(want).max(), 1e-3), "db")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("offset", [0, 1])  # elements that the operands start off a 16-byte boundary
+@pytest.mark.parametrize("M,N,K", [(96, 160, 133), (520, 390, 1026), (1500, 1300, 130)])
+def test_every_layout_batched(device, dtype, offset, M, N, K):
+    lib, st, rt, B = device.lib, device.stream, RT[dtype], 2
+    a = round_to_dtype(normal(61, 0, (B, M, K)), dtype)
+    b = round_to_dtype(normal(61, 1, (B, N, K), std=0.1), dtype)
+    want = a.astype(np.float64) @ b.astype(np.float64).transpose(0, 2, 1)
+
+    def up(t):
+        flat = AnyBuffer.from_numpy(device, np.concatenate([np.zeros(offset, np.float32), t.reshape(-1)]), dtype)
+        return AnyBuffer(flat.storage, dtype, t.size, offset)
+
+    for la in "km":
+        for lb in "kn":
+            ba = up(a if la == "k" else a.transpose(0, 2, 1))
+            bb = up(b if lb == "k" else b.transpose(0, 2, 1))
+            c = AnyBuffer.create(dtype, device, B * M * N)
+            lib.mg_matmul(ba.data_ptr(), bb.data_ptr(), c.data_ptr(), B, M, N, K, *((K, 1) if la == "k" else (1, M)),
+                          *((1, K) if lb == "k" else (N, 1)), M * K, N * K, dtype, st)
+            assert_close(c.to_numpy((B, M, N)), want, rt, rt * np.abs(want).max(), la + lb)
