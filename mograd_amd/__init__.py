@@ -2,11 +2,24 @@
 
 `mograd_amd.runtime` mirrors the reference's kernel-dispatch surface over the C ABI of
 libmograd_hip.so (declared in include/mograd_hip.h, built by `python -m mograd_amd.build`).
-Importing the package does not load the library; constructing a `Device` does, and raises
-if it is missing.
+Importing the package loads neither the library nor its host extension, so that the build can
+run from it; constructing a `Device` does, and raises if they are missing.
 """
-from ._lib import BF16, F16, F32, I32, I64, LibraryMissing, MogradError, load  # noqa: F401
-from .runtime import (GRAD_RULES, SCHEDULER_RULES, AnyBuffer, Device, Layout, Node, evaluate, evaluate_many,  # noqa: F401
-                      gradient, run)
+_FROM_LIB = ("BF16", "F16", "F32", "I32", "I64", "LibraryMissing", "MogradError", "load")
+_FROM_RUNTIME = ("GRAD_RULES", "SCHEDULER_RULES", "AnyBuffer", "Device", "Layout", "Node", "evaluate", "evaluate_many",
+                 "gradient", "run")
+__all__ = [*_FROM_LIB, *_FROM_RUNTIME]
 
 __version__ = "0.1"
+
+
+def __getattr__(name: str):
+    if name not in __all__:
+        raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+    from . import _lib, runtime
+
+    for n in _FROM_LIB:
+        globals()[n] = getattr(_lib, n)
+    for n in _FROM_RUNTIME:
+        globals()[n] = getattr(runtime, n)
+    return globals()[name]

@@ -1,4 +1,5 @@
-"""Builds libmograd_hip.so (gfx950) from mograd_amd/csrc/*.hip with hipcc.
+"""Builds libmograd_hip.so (gfx950) from mograd_amd/csrc/*.hip with hipcc, and the host extension
+_graph.so from mograd_amd/native/graph.cpp with g++.
 
 Usage: python -m mograd_amd.build [--force] [--jobs N]
 
@@ -12,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -20,6 +22,8 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 OBJ_DIR = CSRC / "build"
 LIB_PATH = PKG / "libmograd_hip.so"
+NATIVE_SRC = PKG / "native" / "graph.cpp"
+NATIVE_PATH = PKG / "_graph.so"
 
 ARCH = "gfx950"
 # -packed-fp32-ops is switched off: v_pk_*_f32 forms are not to be generated.
@@ -62,7 +66,22 @@ def _compile(hipcc: str, src: Path, obj: Path) -> tuple[Path, int, str]:
     return src, proc.returncode, err
 
 
+def build_native(force: bool = False, verbose: bool = True) -> Path:
+    """The CPython extension mograd_amd._graph (host code only)."""
+    newest = max(f.stat().st_mtime for f in (NATIVE_SRC, ROOT / "include" / "mograd_hip.h"))
+    if force or not NATIVE_PATH.exists() or NATIVE_PATH.stat().st_mtime < newest:
+        cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+               f"-I{sysconfig.get_paths()['include']}", f"-I{ROOT / 'include'}", str(NATIVE_SRC), "-o", str(NATIVE_PATH), "-ldl"]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"{NATIVE_SRC.name} failed:\n{proc.stderr}")
+        if verbose:
+            print(f"[mograd_amd.build] linked {NATIVE_PATH}", flush=True)
+    return NATIVE_PATH
+
+
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True) -> Path:
+    build_native(force, verbose)
     hipcc = _hipcc()
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))

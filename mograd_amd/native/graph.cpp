@@ -1,0 +1,1474 @@
+// The host path of mograd_amd in native code: the graph's vertices (Layout, Node), the pool buffers,
+// the calls into libmograd_hip, the rewriting pass and the evaluation of a graph.
+//
+// A small model's step is as long as its host work: a lazily built graph is some 260 nodes per
+// four transformer layers, each created, ordered, matched, rewritten and evaluated once, and each
+// kernel costs 2.3 us of the HIP runtime before anything of ours.  In Python the same path took
+// 3.1 ms for such a step on the box (of which 0.3 ms are the launches); see the figures at the
+// functions below.  What is not common (strided operands, ops a training step does not
+// contain) stays with the Python exec functions, which evaluate() calls where its own
+// forms do not apply.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+
+#include <dlfcn.h>
+
+#include <cstdint>
+#include <cstring>
+#include <tuple>
+#include <type_traits>
+#include <utility>
+#include <vector>
+
+#include "mograd_hip.h"
+
+namespace {
+
+// ------------------------------------------------------------------------------------------
+// References
+// ------------------------------------------------------------------------------------------
+
+struct Ref {  // owned reference
+  PyObject* p = nullptr;
+  Ref() = default;
+  explicit Ref(PyObject* o) : p(o) {}
+  Ref(Ref&& o) noexcept : p(o.p) { o.p = nullptr; }
+  Ref& operator=(Ref&& o) noexcept {
+    std::swap(p, o.p);
+    return *this;
+  }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  ~Ref() { Py_XDECREF(p); }
+  PyObject* release() {
+    PyObject* o = p;
+    p = nullptr;
+    return o;
+  }
+  explicit operator bool() const { return p != nullptr; }
+};
+
+PyObject* str_(const char* s) { return PyUnicode_InternFromString(s); }
+
+// Names used as attribute and dictionary keys.
+struct Names {
+  PyObject *index, *eps, *has_bias, *accumulate, *relu_mask, *scale, *is_causal, *stream, *pending, *func, *pat, *op_type,
+      *srcs, *subst, *uses, *origin, *consumers, *rules;
+} N;
+
+PyObject* g_mograd_error = nullptr;   // MogradError(status, message)
+PyObject* g_void_p = nullptr;         // ctypes.c_void_p
+PyTypeObject* g_buffer_type = nullptr;  // AnyBuffer
+PyObject* g_fallbacks = nullptr;      // name -> ctypes wrapper
+
+// ------------------------------------------------------------------------------------------
+// libmograd_hip
+// ------------------------------------------------------------------------------------------
+
+#define MG_FUNCTIONS(X)                                                                                                 \
+  X(mg_pool_free) X(mg_fill) X(mg_copy_device) X(mg_layer_norm_fwd) X(mg_layer_norm_fwd_stats) X(mg_layer_norm_bwd)       \
+  X(mg_layer_norm_bwd_stats) X(mg_layer_norm_bwd_stats_add) X(mg_cross_entropy) X(mg_cross_entropy_grad)                  \
+  X(mg_cross_entropy_ids) X(mg_cross_entropy_grad_ids) X(mg_cross_entropy_fused_ids) X(mg_cross_entropy_fused_ids_noalloc) \
+  X(mg_cross_entropy_fused) X(mg_matmul) X(mg_matmul_bt) X(mg_matmul_bias_bt) X(mg_linear_bwd) X(mg_matmul_bt_add)        \
+  X(mg_matmul_bias_relu_bt) X(mg_linear_bwd_fused) X(mg_sum_axis) X(mg_relu_grad) X(mg_softmax) X(mg_softmax_grad)        \
+  X(mg_argmax_axis) X(mg_adam_step) X(mg_sgd_step) X(mg_add) X(mg_relu) X(mg_cast) X(mg_gather) X(mg_scatter_add)         \
+  X(mg_finish_deferred) X(mg_linear_bwd_deferred) X(mg_layer_norm_bwd_stats_deferred) X(mg_linear_bwd_layer_norm_bwd)     \
+  X(mg_scatter_add_deferred) X(mg_flash_attn_fwd) X(mg_flash_attn_bwd) X(mg_flash_attn_fwd_bshd)                          \
+  X(mg_flash_attn_bwd_bshd) X(mg_flash_attn_fwd_packed) X(mg_flash_attn_bwd_packed)
+
+struct Lib {
+#define X(f) decltype(&::f) f = nullptr;
+  MG_FUNCTIONS(X)
+#undef X
+  decltype(&::mg_pool_alloc) pool_alloc = nullptr;
+  decltype(&::mg_last_error) last_error = nullptr;
+} L;
+
+// Sets MogradError(status, the library's message).
+void raise_status(int status) {
+  Ref e(PyObject_CallFunction(g_mograd_error, "is", status, L.last_error ? L.last_error() : ""));
+  if (e) PyErr_SetObject(g_mograd_error, e.p);
+}
+void raise_invalid(const char* message) {
+  Ref e(PyObject_CallFunction(g_mograd_error, "is", 1, message));
+  if (e) PyErr_SetObject(g_mograd_error, e.p);
+}
+
+// A call without the interpreter lock, as ctypes makes it.
+template <class F>
+int unlocked(F&& f) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS rc = f();
+  Py_END_ALLOW_THREADS return rc;
+}
+
+bool pointer_of(PyObject* o, void** out) {
+  if (o == Py_None) {
+    *out = nullptr;
+    return true;
+  }
+  if (PyLong_Check(o)) {
+    *out = PyLong_AsVoidPtr(o);
+    if (*out == nullptr && PyErr_Occurred()) return PyErr_Clear(), false;
+    return true;
+  }
+  if (reinterpret_cast<PyObject*>(Py_TYPE(o)) != g_void_p) return false;
+  Py_buffer view;
+  if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0) return PyErr_Clear(), false;
+  std::memcpy(out, view.buf, sizeof(void*));
+  PyBuffer_Release(&view);
+  return true;
+}
+
+template <class T>
+bool convert(PyObject* o, T* out) {
+  if constexpr (std::is_floating_point_v<T>) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) return PyErr_Clear(), false;
+    *out = static_cast<T>(v);
+    return true;
+  } else if constexpr (std::is_pointer_v<T>) {
+    void* p = nullptr;
+    if (!pointer_of(o, &p)) return false;
+    *out = static_cast<T>(p);
+    return true;
+  } else {
+    if (!PyLong_Check(o)) return false;
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) return PyErr_Clear(), false;
+    *out = static_cast<T>(v);
+    return static_cast<long long>(*out) == v;
+  }
+}
+
+template <class... A, size_t... I>
+bool convert_all(PyObject* const* args, std::tuple<A...>& t, std::index_sequence<I...>) {
+  return (convert(args[I], &std::get<I>(t)) && ...);
+}
+
+// lib.mg_xxx(...) from Python: anything the conversion above does not take goes to ctypes.
+template <class... A>
+PyObject* call_entry(const char* name, int (*fn)(A...), PyObject* const* args, Py_ssize_t n) {
+  std::tuple<A...> t;
+  if (fn && n == static_cast<Py_ssize_t>(sizeof...(A)) && convert_all(args, t, std::index_sequence_for<A...>{})) {
+    const int rc = unlocked([&] { return std::apply(fn, t); });
+    if (rc != 0) return raise_status(rc), nullptr;
+    return PyLong_FromLong(0);
+  }
+  PyObject* fallback = PyDict_GetItemString(g_fallbacks, name);
+  if (!fallback) return PyErr_Format(PyExc_RuntimeError, "%s is not available", name), nullptr;
+  return PyObject_Vectorcall(fallback, args, static_cast<size_t>(n), nullptr);
+}
+
+#define X(f)                                                                                        \
+  PyObject* py_##f(PyObject*, PyObject* const* args, Py_ssize_t n) { return call_entry(#f, L.f, args, n); }
+MG_FUNCTIONS(X)
+#undef X
+
+// ------------------------------------------------------------------------------------------
+// Layout: dims, strides (elements) and base offset; immutable
+// ------------------------------------------------------------------------------------------
+
+struct LayoutObj {
+  PyObject_HEAD PyObject* dims;  // tuples of int
+  PyObject* strides;
+  long long base_offset, numel;
+  bool contiguous;
+};
+PyTypeObject LayoutType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyObject* int_tuple(PyObject* seq) {  // a new tuple of ints from a tuple or list
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  PyObject* t = PyTuple_New(n);
+  if (!t) return nullptr;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* o = PySequence_Fast_GET_ITEM(seq, i);
+    PyObject* v = PyLong_CheckExact(o) ? (Py_INCREF(o), o) : PyNumber_Long(o);
+    if (!v) return Py_DECREF(t), nullptr;
+    PyTuple_SET_ITEM(t, i, v);
+  }
+  return t;
+}
+
+PyObject* row_major(PyObject* dims, long long* numel) {
+  const Py_ssize_t n = PyTuple_GET_SIZE(dims);
+  PyObject* t = PyTuple_New(n);
+  if (!t) return nullptr;
+  long long s = 1;
+  for (Py_ssize_t i = n - 1; i >= 0; --i) {
+    PyObject* v = PyLong_FromLongLong(s);
+    if (!v) return Py_DECREF(t), nullptr;
+    PyTuple_SET_ITEM(t, i, v);
+    s *= PyLong_AsLongLong(PyTuple_GET_ITEM(dims, i));
+  }
+  *numel = s;
+  if (PyErr_Occurred()) return Py_DECREF(t), nullptr;
+  return t;
+}
+
+// Takes over `dims`; `strides` null: row-major, else taken over.
+PyObject* layout_make(PyTypeObject* type, PyObject* dims, PyObject* strides, long long base) {
+  long long numel = 0;
+  Ref d(dims), s(strides), rm(dims ? row_major(dims, &numel) : nullptr);
+  if (!rm) return nullptr;
+  LayoutObj* o = reinterpret_cast<LayoutObj*>(type->tp_alloc(type, 0));
+  if (!o) return nullptr;
+  o->contiguous = !s || PyObject_RichCompareBool(s.p, rm.p, Py_EQ) == 1;
+  o->dims = d.release();
+  o->strides = s ? s.release() : rm.release();
+  o->base_offset = base;
+  o->numel = numel;
+  return reinterpret_cast<PyObject*>(o);
+}
+
+PyObject* layout_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
+  PyObject* strides = nullptr;
+  PyObject* base = nullptr;
+  if (kw) {
+    PyObject *k, *v;
+    Py_ssize_t pos = 0;
+    while (PyDict_Next(kw, &pos, &k, &v)) {
+      if (PyUnicode_CompareWithASCIIString(k, "strides") == 0) strides = v;
+      else if (PyUnicode_CompareWithASCIIString(k, "base_offset") == 0) base = v;
+      else return PyErr_Format(PyExc_TypeError, "Layout() got an unexpected keyword argument '%U'", k), nullptr;
+    }
+  }
+  PyObject* shape = args;
+  if (PyTuple_GET_SIZE(args) == 1) {
+    PyObject* only = PyTuple_GET_ITEM(args, 0);
+    if (PyTuple_Check(only) || PyList_Check(only)) shape = only;
+  }
+  Ref dims(int_tuple(shape));
+  if (!dims) return nullptr;
+  Ref st;
+  if (strides && strides != Py_None) {
+    Ref fast(PySequence_Fast(strides, "strides must be a sequence"));
+    if (!fast) return nullptr;
+    st = Ref(int_tuple(fast.p));
+    if (!st) return nullptr;
+    if (PyTuple_GET_SIZE(st.p) != PyTuple_GET_SIZE(dims.p)) {
+      PyErr_SetString(PyExc_ValueError, "strides rank differs from shape rank");
+      return nullptr;
+    }
+  }
+  long long b = 0;
+  if (base) {
+    Ref as_int(PyNumber_Long(base));
+    if (!as_int) return nullptr;
+    b = PyLong_AsLongLong(as_int.p);
+    if (b == -1 && PyErr_Occurred()) return nullptr;
+  }
+  return layout_make(type, dims.release(), st.release(), b);
+}
+
+void layout_dealloc(PyObject* self) {
+  LayoutObj* o = reinterpret_cast<LayoutObj*>(self);
+  Py_XDECREF(o->dims);
+  Py_XDECREF(o->strides);
+  Py_TYPE(self)->tp_free(self);  // (a Python subclass's own deallocator releases its type)
+}
+
+LayoutObj* as_layout(PyObject* o) { return reinterpret_cast<LayoutObj*>(o); }
+bool is_layout(PyObject* o) { return PyObject_TypeCheck(o, &LayoutType); }
+Py_ssize_t rank_of(const LayoutObj* l) { return PyTuple_GET_SIZE(l->dims); }
+long long dim_of(const LayoutObj* l, Py_ssize_t i) { return PyLong_AsLongLong(PyTuple_GET_ITEM(l->dims, i < 0 ? i + rank_of(l) : i)); }
+long long stride_of(const LayoutObj* l, Py_ssize_t i) {
+  return PyLong_AsLongLong(PyTuple_GET_ITEM(l->strides, i < 0 ? i + rank_of(l) : i));
+}
+
+PyObject* tuple_item(PyObject* tuple, PyObject* const* args, Py_ssize_t n, PyObject* kwnames, const char* who) {
+  PyObject* idx = nullptr;
+  if (n == 1 && !kwnames) idx = args[0];
+  else if (n == 0 && kwnames && PyTuple_GET_SIZE(kwnames) == 1 &&
+           PyUnicode_CompareWithASCIIString(PyTuple_GET_ITEM(kwnames, 0), "idx") == 0)
+    idx = args[0];
+  else if (n > 0 || kwnames) return PyErr_Format(PyExc_TypeError, "%s() takes one argument, idx", who), nullptr;
+  if (!idx || idx == Py_None) return Py_INCREF(tuple), tuple;
+  return PyObject_GetItem(tuple, idx);
+}
+PyObject* layout_shape(PyObject* self, PyObject* const* args, Py_ssize_t n, PyObject* kw) {
+  return tuple_item(as_layout(self)->dims, args, n, kw, "shape");
+}
+PyObject* layout_stride(PyObject* self, PyObject* const* args, Py_ssize_t n, PyObject* kw) {
+  return tuple_item(as_layout(self)->strides, args, n, kw, "stride");
+}
+PyObject* layout_rank(PyObject* self, PyObject*) { return PyLong_FromSsize_t(rank_of(as_layout(self))); }
+PyObject* layout_numel(PyObject* self, PyObject*) { return PyLong_FromLongLong(as_layout(self)->numel); }
+PyObject* layout_is_contiguous(PyObject* self, PyObject*) { return PyBool_FromLong(as_layout(self)->contiguous); }
+PyObject* layout_as_contiguous(PyObject* self, PyObject*) {
+  LayoutObj* l = as_layout(self);
+  if (l->contiguous && l->base_offset == 0) return Py_INCREF(self), self;  // immutable
+  Py_INCREF(l->dims);
+  return layout_make(Py_TYPE(self), l->dims, nullptr, 0);
+}
+PyObject* layout_richcompare(PyObject* a, PyObject* b, int op) {
+  if ((op != Py_EQ && op != Py_NE) || !is_layout(a) || !is_layout(b)) Py_RETURN_NOTIMPLEMENTED;
+  LayoutObj *x = as_layout(a), *y = as_layout(b);
+  bool same = a == b || (x->base_offset == y->base_offset && PyObject_RichCompareBool(x->dims, y->dims, Py_EQ) == 1 &&
+                         PyObject_RichCompareBool(x->strides, y->strides, Py_EQ) == 1);
+  return PyBool_FromLong(same == (op == Py_EQ));
+}
+Py_hash_t layout_hash(PyObject* self) {
+  LayoutObj* l = as_layout(self);
+  Ref t(Py_BuildValue("(OOL)", l->dims, l->strides, l->base_offset));
+  return t ? PyObject_Hash(t.p) : -1;
+}
+PyObject* layout_repr(PyObject* self) {
+  LayoutObj* l = as_layout(self);
+  return PyUnicode_FromFormat("Layout(dims=%R, strides=%R, base_offset=%lld)", l->dims, l->strides, l->base_offset);
+}
+PyMemberDef layout_members[] = {{"dims", T_OBJECT, offsetof(LayoutObj, dims), READONLY, nullptr},
+                                {"strides", T_OBJECT, offsetof(LayoutObj, strides), READONLY, nullptr},
+                                {"base_offset", T_LONGLONG, offsetof(LayoutObj, base_offset), READONLY, nullptr},
+                                {nullptr, 0, 0, 0, nullptr}};
+#define FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f))
+PyMethodDef layout_methods[] = {
+    {"rank", layout_rank, METH_NOARGS, nullptr},
+    {"shape", FAST(layout_shape), METH_FASTCALL | METH_KEYWORDS, nullptr},
+    {"stride", FAST(layout_stride), METH_FASTCALL | METH_KEYWORDS, nullptr},
+    {"numel", layout_numel, METH_NOARGS, nullptr},
+    {"is_contiguous", layout_is_contiguous, METH_NOARGS, nullptr},
+    {"as_contiguous", layout_as_contiguous, METH_NOARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+// ------------------------------------------------------------------------------------------
+// Node: a graph vertex; compared and hashed by identity
+// ------------------------------------------------------------------------------------------
+
+struct NodeObj {
+  PyObject_HEAD PyObject* op_type;
+  PyObject* node_layout;
+  PyObject* node_dtype;
+  PyObject* srcs;        // list
+  PyObject* node_attrs;  // dict
+  PyObject* bufs;        // list or None
+  uint64_t mark;         // the last walk that saw this node
+  uint32_t used;         // evaluate(): which outputs of a multi-output node are read
+};
+PyTypeObject NodeType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+uint64_t g_epoch = 0;
+
+NodeObj* as_node(PyObject* o) { return reinterpret_cast<NodeObj*>(o); }
+bool is_node(PyObject* o) { return PyObject_TypeCheck(o, &NodeType); }
+
+// Takes over srcs and attrs (null attrs: empty).
+PyObject* node_make(PyObject* op, PyObject* layout, PyObject* dtype, PyObject* srcs, PyObject* attrs, PyObject* bufs) {
+  Ref s(srcs), a(attrs ? attrs : PyDict_New());
+  if (!s || !a) return nullptr;
+  NodeObj* n = reinterpret_cast<NodeObj*>(NodeType.tp_alloc(&NodeType, 0));
+  if (!n) return nullptr;
+  Py_INCREF(op);
+  Py_INCREF(layout);
+  Py_INCREF(dtype);
+  Py_INCREF(bufs);
+  n->op_type = op, n->node_layout = layout, n->node_dtype = dtype, n->bufs = bufs;
+  n->srcs = s.release();
+  n->node_attrs = a.release();
+  n->mark = 0, n->used = 0;
+  return reinterpret_cast<PyObject*>(n);
+}
+
+PyObject* node_new(PyTypeObject*, PyObject* args, PyObject* kw) {
+  static const char* names[] = {"op_type", "node_layout", "node_dtype", "srcs", "node_attrs", "bufs", nullptr};
+  PyObject *op, *layout, *dtype, *srcs = nullptr, *attrs = nullptr, *bufs = Py_None;
+  if (!kw && PyTuple_GET_SIZE(args) >= 3 && PyTuple_GET_SIZE(args) <= 6) {
+    const Py_ssize_t n = PyTuple_GET_SIZE(args);
+    op = PyTuple_GET_ITEM(args, 0), layout = PyTuple_GET_ITEM(args, 1), dtype = PyTuple_GET_ITEM(args, 2);
+    if (n > 3) srcs = PyTuple_GET_ITEM(args, 3);
+    if (n > 4) attrs = PyTuple_GET_ITEM(args, 4);
+    if (n > 5) bufs = PyTuple_GET_ITEM(args, 5);
+  } else if (!PyArg_ParseTupleAndKeywords(args, kw, "OOO|OOO:Node", const_cast<char**>(names), &op, &layout, &dtype, &srcs,
+                                          &attrs, &bufs)) {
+    return nullptr;
+  }
+  if (srcs) Py_INCREF(srcs);
+  else if (!(srcs = PyList_New(0))) return nullptr;
+  Py_XINCREF(attrs);
+  return node_make(op, layout, dtype, srcs, attrs, bufs);
+}
+int node_traverse(PyObject* self, visitproc visit, void* arg) {
+  NodeObj* n = as_node(self);
+  Py_VISIT(n->op_type);
+  Py_VISIT(n->node_layout);
+  Py_VISIT(n->node_dtype);
+  Py_VISIT(n->srcs);
+  Py_VISIT(n->node_attrs);
+  Py_VISIT(n->bufs);
+  return 0;
+}
+int node_clear(PyObject* self) {
+  NodeObj* n = as_node(self);
+  Py_CLEAR(n->op_type);
+  Py_CLEAR(n->node_layout);
+  Py_CLEAR(n->node_dtype);
+  Py_CLEAR(n->srcs);
+  Py_CLEAR(n->node_attrs);
+  Py_CLEAR(n->bufs);
+  return 0;
+}
+void node_dealloc(PyObject* self) {
+  PyObject_GC_UnTrack(self);
+  Py_TRASHCAN_BEGIN(self, node_dealloc)  // a deep graph is freed without deep recursion
+      node_clear(self);
+  Py_TYPE(self)->tp_free(self);
+  Py_TRASHCAN_END
+}
+PyObject* node_layout(PyObject* self, PyObject*) {
+  PyObject* o = as_node(self)->node_layout;
+  return Py_INCREF(o), o;
+}
+PyObject* node_dtype(PyObject* self, PyObject*) {
+  PyObject* o = as_node(self)->node_dtype;
+  return Py_INCREF(o), o;
+}
+PyObject* node_attrs(PyObject* self, PyObject*) {
+  PyObject* o = as_node(self)->node_attrs;
+  return Py_INCREF(o), o;
+}
+PyObject* node_numel(PyObject* self, PyObject*) { return PyObject_CallMethod(as_node(self)->node_layout, "numel", nullptr); }
+PyObject* node_src(PyObject* self, PyObject* i) { return PyObject_GetItem(as_node(self)->srcs, i); }
+PyObject* node_shape(PyObject* self, PyObject* i) { return PyObject_CallMethod(as_node(self)->node_layout, "shape", "O", i); }
+PyObject* node_leaf(PyObject*, PyObject* args, PyObject* kw) {
+  static const char* names[] = {"layout", "dtype", "buf", nullptr};
+  PyObject *layout, *dtype = nullptr, *buf = Py_None;
+  if (!PyArg_ParseTupleAndKeywords(args, kw, "O|OO:leaf", const_cast<char**>(names), &layout, &dtype, &buf)) return nullptr;
+  static PyObject* kBuffer = str_("BUFFER");
+  static PyObject* kF32 = PyLong_FromLong(MG_F32);
+  Ref list;
+  if (buf != Py_None) {
+    list = Ref(PyList_New(1));
+    if (!list) return nullptr;
+    Py_INCREF(buf);
+    PyList_SET_ITEM(list.p, 0, buf);
+  }
+  return node_make(kBuffer, layout, dtype ? dtype : kF32, PyList_New(0), nullptr, list ? list.p : Py_None);
+}
+PyObject* node_repr(PyObject* self) {
+  NodeObj* n = as_node(self);
+  return PyUnicode_FromFormat("Node(op_type=%R, node_layout=%R, node_dtype=%R, %zd srcs, node_attrs=%R)", n->op_type,
+                              n->node_layout, n->node_dtype, PyObject_Size(n->srcs), n->node_attrs);
+}
+PyMemberDef node_members[] = {{"op_type", T_OBJECT, offsetof(NodeObj, op_type), 0, nullptr},
+                              {"node_layout", T_OBJECT, offsetof(NodeObj, node_layout), 0, nullptr},
+                              {"node_dtype", T_OBJECT, offsetof(NodeObj, node_dtype), 0, nullptr},
+                              {"srcs", T_OBJECT, offsetof(NodeObj, srcs), 0, nullptr},
+                              {"node_attrs", T_OBJECT, offsetof(NodeObj, node_attrs), 0, nullptr},
+                              {"bufs", T_OBJECT, offsetof(NodeObj, bufs), 0, nullptr},
+                              {nullptr, 0, 0, 0, nullptr}};
+PyMethodDef node_methods[] = {{"layout", node_layout, METH_NOARGS, nullptr},
+                              {"dtype", node_dtype, METH_NOARGS, nullptr},
+                              {"attrs", node_attrs, METH_NOARGS, nullptr},
+                              {"numel", node_numel, METH_NOARGS, nullptr},
+                              {"src", node_src, METH_O, nullptr},
+                              {"shape", node_shape, METH_O, nullptr},
+                              {"leaf", FAST(node_leaf), METH_VARARGS | METH_KEYWORDS | METH_STATIC, nullptr},
+                              {nullptr, nullptr, 0, nullptr}};
+
+bool node_ok(PyObject* o) {
+  if (is_node(o) && PyList_Check(as_node(o)->srcs)) return true;
+  PyErr_SetString(PyExc_TypeError, "a graph vertex is a Node with a list of Node sources");
+  return false;
+}
+
+// Sources before consumers, each node once, in the order of a depth-first walk over srcs.
+// Borrowed references: the graph keeps them.
+bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<NodeObj*>& order) {
+  const uint64_t epoch = ++g_epoch;
+  std::vector<std::pair<NodeObj*, Py_ssize_t>> stack;
+  for (Py_ssize_t r = 0; r < n_roots; ++r) {
+    if (!node_ok(roots[r])) return false;
+    if (as_node(roots[r])->mark == epoch) continue;
+    as_node(roots[r])->mark = epoch;
+    stack.emplace_back(as_node(roots[r]), 0);
+    while (!stack.empty()) {
+      NodeObj* n = stack.back().first;
+      const Py_ssize_t i = stack.back().second;
+      if (i < PyList_GET_SIZE(n->srcs)) {
+        stack.back().second = i + 1;
+        PyObject* c = PyList_GET_ITEM(n->srcs, i);
+        if (!node_ok(c)) return false;
+        if (as_node(c)->mark != epoch) {
+          as_node(c)->mark = epoch;
+          stack.emplace_back(as_node(c), 0);
+        }
+      } else {
+        order.push_back(n);
+        stack.pop_back();
+      }
+    }
+  }
+  return true;
+}
+
+PyObject* py_toposort(PyObject*, PyObject* root) {
+  std::vector<NodeObj*> order;
+  if (!toposort(&root, 1, order)) return nullptr;
+  PyObject* list = PyList_New(static_cast<Py_ssize_t>(order.size()));
+  if (!list) return nullptr;
+  for (size_t i = 0; i < order.size(); ++i) {
+    Py_INCREF(order[i]);
+    PyList_SET_ITEM(list, static_cast<Py_ssize_t>(i), reinterpret_cast<PyObject*>(order[i]));
+  }
+  return list;
+}
+
+// depends_on(node, target): whether `target` is `node` or feeds it.
+PyObject* py_depends_on(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 2 || !node_ok(args[0])) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "depends_on(node, target)");
+    return nullptr;
+  }
+  const uint64_t epoch = ++g_epoch;
+  std::vector<NodeObj*> stack{as_node(args[0])};
+  as_node(args[0])->mark = epoch;
+  while (!stack.empty()) {
+    NodeObj* v = stack.back();
+    stack.pop_back();
+    if (reinterpret_cast<PyObject*>(v) == args[1]) Py_RETURN_TRUE;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(v->srcs); ++i) {
+      PyObject* c = PyList_GET_ITEM(v->srcs, i);
+      if (!node_ok(c)) return nullptr;
+      if (as_node(c)->mark != epoch) {
+        as_node(c)->mark = epoch;
+        stack.push_back(as_node(c));
+      }
+    }
+  }
+  Py_RETURN_FALSE;
+}
+
+// ------------------------------------------------------------------------------------------
+// Storage and Buffer
+// ------------------------------------------------------------------------------------------
+
+struct StorageObj {  // one pooled allocation, returned to the pool with the last view of it
+  PyObject_HEAD PyObject* device;
+  unsigned long long ptr;
+  long long nbytes;
+};
+PyTypeObject StorageType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyObject* storage_make(PyObject* device, long long nbytes) {
+  void* p = nullptr;
+  const int rc = unlocked([&] { return L.pool_alloc(&p, nbytes); });
+  if (rc != 0) return raise_status(rc), nullptr;
+  StorageObj* s = PyObject_New(StorageObj, &StorageType);
+  if (!s) return nullptr;
+  Py_INCREF(device);
+  s->device = device;
+  s->ptr = reinterpret_cast<uintptr_t>(p);
+  s->nbytes = nbytes;
+  return reinterpret_cast<PyObject*>(s);
+}
+PyObject* storage_new(PyTypeObject*, PyObject* args, PyObject* kw) {
+  static const char* names[] = {"device", "nbytes", nullptr};
+  PyObject* device;
+  long long nbytes;
+  if (!PyArg_ParseTupleAndKeywords(args, kw, "OL:Storage", const_cast<char**>(names), &device, &nbytes)) return nullptr;
+  return storage_make(device, nbytes);
+}
+void storage_dealloc(PyObject* self) {
+  StorageObj* s = reinterpret_cast<StorageObj*>(self);
+  if (s->ptr) (void)L.mg_pool_free(reinterpret_cast<void*>(static_cast<uintptr_t>(s->ptr)));
+  Py_XDECREF(s->device);
+  PyObject_Free(self);
+}
+PyMemberDef storage_members[] = {{"device", T_OBJECT, offsetof(StorageObj, device), READONLY, nullptr},
+                                 {"ptr", T_ULONGLONG, offsetof(StorageObj, ptr), READONLY, nullptr},
+                                 {"nbytes", T_LONGLONG, offsetof(StorageObj, nbytes), READONLY, nullptr},
+                                 {nullptr, 0, 0, 0, nullptr}};
+
+struct BufferObj {  // a typed view of a storage
+  PyObject_HEAD PyObject* storage;
+  int dtype;
+  long long numel, offset_elems;
+};
+PyTypeObject BufferType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+int dtype_size(int dtype) {
+  switch (dtype) {
+    case MG_F32: case MG_I32: return 4;
+    case MG_F16: case MG_BF16: return 2;
+    case MG_I64: return 8;
+    default: return 0;
+  }
+}
+bool is_float(int dtype) { return dtype == MG_F32 || dtype == MG_F16 || dtype == MG_BF16; }
+BufferObj* as_buffer(PyObject* o) { return reinterpret_cast<BufferObj*>(o); }
+void* address(const BufferObj* b) {
+  return reinterpret_cast<void*>(static_cast<uintptr_t>(reinterpret_cast<StorageObj*>(b->storage)->ptr) +
+                                 static_cast<uintptr_t>(b->offset_elems * dtype_size(b->dtype)));
+}
+// Takes over `storage`.
+PyObject* buffer_make(PyTypeObject* type, PyObject* storage, int dtype, long long numel, long long offset) {
+  if (!storage) return nullptr;
+  BufferObj* b = reinterpret_cast<BufferObj*>(type->tp_alloc(type, 0));
+  if (!b) return Py_DECREF(storage), nullptr;
+  b->storage = storage;
+  b->dtype = dtype;
+  b->numel = numel;
+  b->offset_elems = offset;
+  return reinterpret_cast<PyObject*>(b);
+}
+PyObject* buffer_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
+  static const char* names[] = {"storage", "dtype", "numel", "offset_elems", nullptr};
+  PyObject* storage;
+  int dtype;
+  long long numel, offset = 0;
+  if (!PyArg_ParseTupleAndKeywords(args, kw, "O!iL|L:AnyBuffer", const_cast<char**>(names), &StorageType, &storage, &dtype,
+                                   &numel, &offset))
+    return nullptr;
+  Py_INCREF(storage);
+  return buffer_make(type, storage, dtype, numel, offset);
+}
+void buffer_dealloc(PyObject* self) {
+  Py_XDECREF(as_buffer(self)->storage);
+  Py_TYPE(self)->tp_free(self);  // (a Python subclass's own deallocator releases its type)
+}
+PyObject* buffer_data_ptr(PyObject* self, PyObject* const* args, Py_ssize_t n, PyObject* kw) {
+  bool with_offset = true;
+  if (n + (kw ? PyTuple_GET_SIZE(kw) : 0) > 0) {
+    const int t = PyObject_IsTrue(args[0]);
+    if (t < 0) return nullptr;
+    with_offset = t != 0;
+  }
+  BufferObj* b = as_buffer(self);
+  const unsigned long long at = with_offset ? reinterpret_cast<uintptr_t>(address(b))
+                                            : reinterpret_cast<StorageObj*>(b->storage)->ptr;
+  Ref v(PyLong_FromUnsignedLongLong(at));
+  return v ? PyObject_CallOneArg(g_void_p, v.p) : nullptr;
+}
+PyObject* buffer_view(PyObject* self, PyObject* layout) {
+  if (!is_layout(layout)) return PyErr_SetString(PyExc_TypeError, "view() takes a Layout"), nullptr;
+  BufferObj* b = as_buffer(self);
+  Py_INCREF(b->storage);
+  return buffer_make(Py_TYPE(self), b->storage, b->dtype, as_layout(layout)->numel, as_layout(layout)->base_offset);
+}
+PyObject* buffer_size_bytes(PyObject* self, PyObject*) {
+  return PyLong_FromLongLong(as_buffer(self)->numel * dtype_size(as_buffer(self)->dtype));
+}
+PyMemberDef buffer_members[] = {{"storage", T_OBJECT, offsetof(BufferObj, storage), READONLY, nullptr},
+                                {"dtype", T_INT, offsetof(BufferObj, dtype), READONLY, nullptr},
+                                {"numel", T_LONGLONG, offsetof(BufferObj, numel), READONLY, nullptr},
+                                {"offset_elems", T_LONGLONG, offsetof(BufferObj, offset_elems), READONLY, nullptr},
+                                {nullptr, 0, 0, 0, nullptr}};
+PyMethodDef buffer_methods[] = {{"data_ptr", FAST(buffer_data_ptr), METH_FASTCALL | METH_KEYWORDS, nullptr},
+                                {"view", buffer_view, METH_O, nullptr},
+                                {"size_bytes", buffer_size_bytes, METH_NOARGS, nullptr},
+                                {nullptr, nullptr, 0, nullptr}};
+
+// ------------------------------------------------------------------------------------------
+// Evaluation
+// ------------------------------------------------------------------------------------------
+
+// One node's execution: its operands, and what the library needs of the device.
+struct Exec {
+  NodeObj* n;
+  PyObject* device;
+  void* stream;
+  void* pending;  // the deferred list in use, or null
+  int dtype;
+  BufferObj* in[12];
+  LayoutObj* lay[12];  // of the sources
+  int count;
+
+  void* p(int i) const { return address(in[i]); }
+  // The first k operands are contiguous and start on the 16-byte boundary the flat kernels read from.
+  bool flat(int k) const {
+    if (count < k) return false;
+    for (int i = 0; i < k; ++i)
+      if (!lay[i]->contiguous || reinterpret_cast<uintptr_t>(p(i)) % 16 != 0) return false;
+    return true;
+  }
+  bool contiguous(int k) const {
+    if (count < k) return false;
+    for (int i = 0; i < k; ++i)
+      if (!lay[i]->contiguous) return false;
+    return true;
+  }
+  bool truth(PyObject* key, bool fallback) const {
+    PyObject* v = PyDict_GetItem(n->node_attrs, key);
+    return v ? PyObject_IsTrue(v) == 1 : fallback;
+  }
+  double number(PyObject* key) const {
+    PyObject* v = PyDict_GetItem(n->node_attrs, key);
+    return v ? PyFloat_AsDouble(v) : 0.0;
+  }
+  PyObject* buffer(int dt, long long numel) const {
+    return buffer_make(g_buffer_type, storage_make(device, numel * dtype_size(dt)), dt, numel, 0);
+  }
+};
+
+// New buffers for a node's results; release() hands them over as a list.
+struct Results {
+  Ref list;
+  std::vector<BufferObj*> b;
+  const Exec& x;
+  bool ok = true;
+  explicit Results(const Exec& e) : list(PyList_New(0)), x(e) {}
+  void add(int dt, long long numel) {
+    if (!ok || !list) return;
+    Ref o(x.buffer(dt, numel));
+    ok = o && PyList_Append(list.p, o.p) == 0;
+    if (ok) b.push_back(as_buffer(o.p));
+  }
+  void add_none() { ok = ok && list && PyList_Append(list.p, Py_None) == 0, b.push_back(nullptr); }
+  void* p(int i) const { return b[i] ? address(b[i]) : nullptr; }
+};
+
+struct GemmDims {
+  long long batch, M, N, K, lda0, lda1, ldb0, ldb1, bsa, bsb;
+};
+// A (.., M, K) by B (.., N, K); false: batch dimensions that do not collapse, left to the Python form.
+bool gemm_dims(const Exec& x, GemmDims* g) {
+  const LayoutObj *la = x.lay[0], *lb = x.lay[1], *lo = as_layout(x.n->node_layout);
+  for (const LayoutObj* l : {la, lb})
+    for (Py_ssize_t i = rank_of(l) - 4; i >= 0; --i)
+      if (stride_of(l, i) != dim_of(l, i + 1) * stride_of(l, i + 1)) return false;
+  if (rank_of(la) < 2 || rank_of(lb) < 2) return false;
+  g->N = dim_of(lo, -1);
+  g->M = dim_of(la, -2), g->K = dim_of(la, -1);
+  if (g->M == 0 || g->K == 0) return false;
+  g->lda0 = stride_of(la, -2), g->lda1 = stride_of(la, -1);
+  g->ldb0 = stride_of(lb, -2), g->ldb1 = stride_of(lb, -1);
+  g->batch = la->numel / (g->M * g->K);
+  g->bsa = rank_of(la) >= 3 ? stride_of(la, -3) : g->M * g->K;
+  g->bsb = rank_of(lb) >= 3 ? stride_of(lb, -3) : g->N * g->K;
+  return true;
+}
+
+// The result of an exec form: 1 done (`out` holds the list), 0 not its case, -1 an error is set.
+using Form = int (*)(const Exec&, PyObject** out);
+
+int finish(Results& r, int rc, PyObject** out) {
+  if (rc != 0) return raise_status(rc), -1;
+  *out = r.list.release();
+  return 1;
+}
+#define MG_RUN(call) finish(r, unlocked([&] { return call; }), out)
+
+long long out_numel(const Exec& x) { return as_layout(x.n->node_layout)->numel; }
+
+int run_matmul_bt(const Exec& x, PyObject** out) {
+  GemmDims g;
+  if (x.count < 2 || !gemm_dims(x, &g)) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_matmul_bt(x.p(0), x.p(1), r.p(0), g.batch, g.M, g.N, g.K, g.lda0, g.lda1, g.ldb0, g.ldb1, g.bsa,
+                               g.bsb, x.dtype, x.stream));
+}
+template <auto Lib::*FN, bool FLAT2>
+int run_matmul3(const Exec& x, PyObject** out) {
+  GemmDims g;
+  if (x.count < 3 || !gemm_dims(x, &g) || (FLAT2 && !x.lay[2]->contiguous)) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN((L.*FN)(x.p(0), x.p(1), x.p(2), r.p(0), g.batch, g.M, g.N, g.K, g.lda0, g.lda1, g.ldb0, g.ldb1, g.bsa,
+                        g.bsb, x.dtype, x.stream));
+}
+
+int run_linear_grad(const Exec& x, PyObject** out) {
+  const bool accumulate = x.truth(N.accumulate, false), relu = x.truth(N.relu_mask, false),
+             has_bias = x.truth(N.has_bias, true);
+  if (!x.contiguous(accumulate ? 4 : 3) || !is_float(x.dtype) || rank_of(x.lay[2]) != 2) return 0;
+  const long long n = dim_of(x.lay[2], 0), k = dim_of(x.lay[2], 1);
+  if (k == 0 || x.lay[0]->numel != x.lay[1]->numel / k * n) return 0;
+  const long long m = x.lay[1]->numel / k;
+  Results r(x);
+  // dX that nobody reads (the first layer's input is data) is not computed.
+  const bool want_dx = x.n->used & 1u;
+  if (want_dx) r.add(x.dtype, m * k);
+  else r.add_none();
+  r.add(x.dtype, n * k);
+  if (has_bias) r.add(x.dtype, n);
+  if (!r.ok) return -1;
+  void *dx = r.p(0), *dw = r.p(1), *db = has_bias ? r.p(2) : nullptr;
+  return MG_RUN([&]() -> int {
+    if (accumulate && dx)
+      if (int rc = L.mg_copy_device(dx, x.p(3), m * k * dtype_size(x.dtype), x.stream)) return rc;
+    if (x.pending)
+      return L.mg_linear_bwd_deferred(x.p(0), x.p(1), x.p(2), dx, dw, db, m, n, k, accumulate, relu, x.dtype, x.dtype,
+                                      x.pending, x.stream);
+    return L.mg_linear_bwd_fused(x.p(0), x.p(1), x.p(2), dx, dw, db, m, n, k, accumulate, relu, x.dtype, x.stream);
+  }());
+}
+
+int run_linear_ln_grad(const Exec& x, PyObject** out) {
+  const bool accumulate = x.truth(N.accumulate, false), has_bias = x.truth(N.has_bias, true);
+  if (!x.contiguous(accumulate ? 8 : 7) || !is_float(x.dtype) || rank_of(x.lay[2]) != 2) return 0;
+  const long long n = dim_of(x.lay[2], 0), k = dim_of(x.lay[2], 1);
+  if (k == 0) return 0;
+  const long long m = x.lay[1]->numel / k;
+  if (x.lay[0]->numel != m * n || x.lay[3]->numel != m * k) return 0;
+  Results r(x);
+  r.add(x.dtype, m * k);
+  r.add(x.dtype, k);
+  r.add(x.dtype, k);
+  r.add(x.dtype, n * k);
+  if (has_bias) r.add(x.dtype, n);
+  if (!r.ok) return -1;
+  return MG_RUN([&]() -> int {
+    if (accumulate)
+      if (int rc = L.mg_copy_device(r.p(0), x.p(7), m * k * dtype_size(x.dtype), x.stream)) return rc;
+    return L.mg_linear_bwd_layer_norm_bwd(x.p(0), x.p(1), x.p(2), x.p(3), x.p(4), static_cast<float*>(x.p(5)),
+                                          static_cast<float*>(x.p(6)), r.p(0), r.p(3), has_bias ? r.p(4) : nullptr, r.p(1),
+                                          r.p(2), m, n, k, accumulate, x.dtype, x.dtype, x.pending, x.stream);
+  }());
+}
+
+int run_layer_norm_stats(const Exec& x, PyObject** out) {
+  if (!x.contiguous(3) || !is_float(x.dtype)) return 0;
+  const long long cols = dim_of(x.lay[0], -1);
+  if (cols == 0) return 0;
+  const long long rows = x.lay[0]->numel / cols;
+  const float eps = static_cast<float>(x.number(N.eps));
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  r.add(MG_F32, rows);
+  r.add(MG_F32, rows);
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_layer_norm_fwd_stats(x.p(0), x.p(1), x.p(2), r.p(0), static_cast<float*>(r.p(1)),
+                                          static_cast<float*>(r.p(2)), rows, cols, eps, x.dtype, x.stream));
+}
+
+template <bool RESIDUAL>
+int run_layer_norm_stats_grad(const Exec& x, PyObject** out) {
+  if (!x.contiguous(RESIDUAL ? 6 : 5) || !is_float(x.dtype)) return 0;
+  const long long cols = dim_of(x.lay[1], -1);
+  if (cols == 0) return 0;
+  const long long rows = x.lay[1]->numel / cols;
+  Results r(x);
+  r.add(x.dtype, rows * cols);
+  r.add(x.dtype, x.lay[2]->numel);
+  r.add(x.dtype, x.lay[2]->numel);
+  if (!r.ok) return -1;
+  const float *mean = static_cast<float*>(x.p(3)), *rstd = static_cast<float*>(x.p(4));
+  void* res = RESIDUAL ? x.p(5) : nullptr;
+  return MG_RUN([&]() -> int {
+    if (x.pending)
+      return L.mg_layer_norm_bwd_stats_deferred(x.p(0), x.p(1), x.p(2), mean, rstd, res, r.p(0), r.p(1), r.p(2), rows, cols,
+                                                x.dtype, x.dtype, x.pending, x.stream);
+    if (RESIDUAL)
+      return L.mg_layer_norm_bwd_stats_add(x.p(0), x.p(1), x.p(2), mean, rstd, res, r.p(0), r.p(1), r.p(2), rows, cols,
+                                           x.dtype, x.stream);
+    return L.mg_layer_norm_bwd_stats(x.p(0), x.p(1), x.p(2), mean, rstd, r.p(0), r.p(1), r.p(2), rows, cols, x.dtype,
+                                     x.stream);
+  }());
+}
+
+int run_add(const Exec& x, PyObject** out) {
+  if (!x.flat(2)) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_add(x.p(0), x.p(1), r.p(0), out_numel(x), x.dtype, x.stream));
+}
+int run_relu(const Exec& x, PyObject** out) {
+  if (!x.flat(1)) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_relu(x.p(0), r.p(0), out_numel(x), x.dtype, x.stream));
+}
+int run_relu_grad(const Exec& x, PyObject** out) {
+  if (!x.flat(2)) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_relu_grad(x.p(0), x.p(1), r.p(0), out_numel(x), x.dtype, x.stream));
+}
+int run_gather(const Exec& x, PyObject** out) {
+  if (x.count < 2 || rank_of(x.lay[0]) != 2 || !x.lay[1]->contiguous) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_gather(x.p(0), x.p(1), r.p(0), x.lay[1]->numel, dim_of(x.lay[0], 0), dim_of(x.lay[0], 1),
+                            stride_of(x.lay[0], 0), stride_of(x.lay[0], 1), x.in[1]->dtype, x.dtype, x.stream));
+}
+int run_scatter_add(const Exec& x, PyObject** out) {
+  const LayoutObj* lo = as_layout(x.n->node_layout);
+  if (!x.contiguous(2) || rank_of(x.lay[1]) != rank_of(x.lay[0]) + 1) return 0;
+  Results r(x);
+  r.add(x.dtype, lo->numel);
+  if (!r.ok) return -1;
+  const long long n_idx = x.lay[0]->numel, rows = dim_of(lo, 0), row_size = dim_of(x.lay[1], -1);
+  return MG_RUN(x.pending ? L.mg_scatter_add_deferred(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0]->dtype, x.dtype,
+                                                      x.dtype, x.pending, x.stream)
+                          : L.mg_scatter_add(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0]->dtype, x.dtype, x.stream));
+}
+int run_attn_packed(const Exec& x, PyObject** out) {
+  const LayoutObj* q = x.lay[0];
+  if (x.count < 1 || !is_float(x.dtype) || rank_of(q) != 5 || dim_of(q, 2) != 3) return 0;
+  const long long B = dim_of(q, 0), S = dim_of(q, 1), H = dim_of(q, 3), D = dim_of(q, 4);
+  const float scale = static_cast<float>(x.number(N.scale));
+  const bool causal = x.truth(N.is_causal, false), bias = x.truth(N.has_bias, true);
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  r.add(MG_F32, B * H * S);
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_flash_attn_fwd_packed(x.p(0), x.count > 1 ? x.p(1) : nullptr, r.p(0), static_cast<float*>(r.p(1)), B, S,
+                                           H, D, scale, causal, bias, x.dtype, x.stream));
+}
+int run_attn_packed_grad(const Exec& x, PyObject** out) {
+  if (x.count < 4 || !is_float(x.dtype) || !x.lay[0]->contiguous || rank_of(x.lay[2]) != 5) return 0;
+  const LayoutObj* q = x.lay[2];
+  const long long B = dim_of(q, 0), S = dim_of(q, 1), H = dim_of(q, 3), D = dim_of(q, 4);
+  const float scale = static_cast<float>(x.number(N.scale));
+  const bool causal = x.truth(N.is_causal, false), bias = x.truth(N.has_bias, !causal);
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_flash_attn_bwd_packed(x.p(0), x.p(1), x.p(2), x.count > 4 ? x.p(4) : nullptr,
+                                           static_cast<float*>(x.p(3)), r.p(0), B, S, H, D, scale, causal, bias, x.dtype,
+                                           x.stream));
+}
+int run_ce_ids(const Exec& x, PyObject** out) {
+  if (!x.contiguous(2) || !is_float(x.dtype)) return 0;
+  const long long c = dim_of(x.lay[0], -1);
+  if (c == 0) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_cross_entropy_ids(x.p(0), x.p(1), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1]->dtype, x.stream));
+}
+int run_ce_grad_ids(const Exec& x, PyObject** out) {
+  if (!x.contiguous(2) || x.count < 3 || !is_float(x.dtype)) return 0;
+  const long long c = dim_of(x.lay[0], -1);
+  if (c == 0) return 0;
+  Results r(x);
+  r.add(x.dtype, out_numel(x));
+  if (!r.ok) return -1;
+  return MG_RUN(L.mg_cross_entropy_grad_ids(x.p(0), x.p(1), x.p(2), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1]->dtype,
+                                            x.stream));
+}
+int run_reshape(const Exec& x, PyObject** out) {
+  if (!x.contiguous(1)) return 0;
+  Ref list(PyList_New(1));
+  if (!list) return -1;
+  Py_INCREF(x.in[0]->storage);
+  PyObject* v = buffer_make(g_buffer_type, x.in[0]->storage, x.in[0]->dtype, out_numel(x), x.in[0]->offset_elems);
+  if (!v) return -1;
+  PyList_SET_ITEM(list.p, 0, v);
+  *out = list.release();
+  return 1;
+}
+
+PyObject* g_forms = nullptr;  // op type -> index into kForms
+const std::pair<const char*, Form> kForms[] = {
+    {"MATMUL_BT", run_matmul_bt},
+    {"MATMUL_BIAS_BT", run_matmul3<&Lib::mg_matmul_bias_bt, false>},
+    {"MATMUL_BIAS_RELU_BT", run_matmul3<&Lib::mg_matmul_bias_relu_bt, false>},
+    {"MATMUL_BT_ADD", run_matmul3<&Lib::mg_matmul_bt_add, true>},
+    {"LINEAR_GRAD", run_linear_grad},
+    {"LINEAR_LAYER_NORM_GRAD", run_linear_ln_grad},
+    {"LAYER_NORM_STATS", run_layer_norm_stats},
+    {"LAYER_NORM_STATS_GRAD", run_layer_norm_stats_grad<false>},
+    {"LAYER_NORM_STATS_GRAD_ADD", run_layer_norm_stats_grad<true>},
+    {"ADD", run_add},
+    {"RELU", run_relu},
+    {"RELU_GRAD", run_relu_grad},
+    {"GATHER", run_gather},
+    {"SCATTER_ADD", run_scatter_add},
+    {"FLASH_ATTN_PACKED", run_attn_packed},
+    {"FLASH_ATTN_PACKED_GRAD", run_attn_packed_grad},
+    {"CROSS_ENTROPY_IDS", run_ce_ids},
+    {"CROSS_ENTROPY_IDS_GRAD", run_ce_grad_ids},
+    {"RESHAPE", run_reshape},
+};
+
+struct Evaluation {
+  PyObject* device;
+  PyObject* run;  // runtime.run(node, inputs, device): the Python exec function of a node
+  void* stream = nullptr;
+  void* pending = nullptr;
+  PyObject *kBuffer, *kGetTuple;
+
+  bool op_is(const NodeObj* n, PyObject* name) const {
+    return n->op_type == name || PyUnicode_Compare(n->op_type, name) == 0;
+  }
+  static bool have(const NodeObj* n) { return n->bufs != Py_None; }
+  // Result i of an evaluated node (borrowed); one that was left out when the node first ran,
+  // because nobody read it then, is made now.
+  PyObject* result(NodeObj* s, Py_ssize_t i) {
+    if (!PyList_Check(s->bufs) || i < 0 || i >= PyList_GET_SIZE(s->bufs))
+      return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), nullptr;
+    if (PyList_GET_ITEM(s->bufs, i) == Py_None) {
+      s->used = ~0u;
+      if (!execute(s)) return nullptr;
+    }
+    return PyList_GET_ITEM(s->bufs, i);
+  }
+  bool set(NodeObj* n, PyObject* list) {  // takes over `list`
+    if (!list) return false;
+    Py_SETREF(n->bufs, list);
+    return true;
+  }
+
+  bool execute(NodeObj* n) {
+    const Py_ssize_t count = PyList_GET_SIZE(n->srcs);
+    PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
+    if (idx && count <= 12 && is_layout(n->node_layout) && PyLong_Check(n->node_dtype)) {
+      Exec x;
+      x.n = n, x.device = device, x.stream = stream, x.pending = pending;
+      x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
+      x.count = static_cast<int>(count);
+      bool plain = true;
+      for (int i = 0; i < x.count && plain; ++i) {
+        NodeObj* s = as_node(PyList_GET_ITEM(n->srcs, i));
+        PyObject* b = result(s, 0);
+        if (!b) return false;
+        plain = PyObject_TypeCheck(b, &BufferType) && is_layout(s->node_layout);
+        x.in[i] = as_buffer(b);
+        x.lay[i] = as_layout(s->node_layout);
+      }
+      if (plain) {
+        PyObject* out = nullptr;
+        const int rc = kForms[PyLong_AsLong(idx)].second(x, &out);
+        if (rc < 0) return false;
+        if (rc > 0) return set(n, out);
+      }
+    }
+    Ref inputs(PyList_New(count));
+    if (!inputs) return false;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      PyObject* b = result(as_node(PyList_GET_ITEM(n->srcs, i)), 0);
+      if (!b) return false;
+      Py_INCREF(b);
+      PyList_SET_ITEM(inputs.p, i, b);
+    }
+    return set(n, PyObject_CallFunctionObjArgs(run, n, inputs.p, device, nullptr));
+  }
+
+  // CROSS_ENTROPY_IDS[logits, ids] and the CROSS_ENTROPY_IDS_GRAD of the same operands in this walk: loss
+  // and dlogits in one pass over the logits, when the gradient's upstream is already there (it is the
+  // graph's root).  1 done, 0 not such a pair, -1 error.
+  std::vector<NodeObj*> ce_grads;
+  PyObject *kCeIds, *kCeIdsGrad;
+  int cross_entropy_pair(NodeObj* n) {
+    NodeObj* g = nullptr;
+    for (NodeObj* c : ce_grads)
+      if (!have(c) && PyList_GET_SIZE(c->srcs) == 3 && PyList_GET_SIZE(n->srcs) == 2 &&
+          PyList_GET_ITEM(c->srcs, 0) == PyList_GET_ITEM(n->srcs, 0) &&
+          PyList_GET_ITEM(c->srcs, 1) == PyList_GET_ITEM(n->srcs, 1) && have(as_node(PyList_GET_ITEM(c->srcs, 2))))
+        g = c;
+    if (!g || !is_layout(n->node_layout) || !is_layout(g->node_layout)) return 0;
+    BufferObj* b[3];
+    for (int i = 0; i < 3; ++i) {
+      NodeObj* s = as_node(PyList_GET_ITEM(g->srcs, i));
+      PyObject* r = result(s, 0);
+      if (!r) return -1;
+      if (!PyObject_TypeCheck(r, &BufferType) || !is_layout(s->node_layout) || !as_layout(s->node_layout)->contiguous) return 0;
+      b[i] = as_buffer(r);
+    }
+    const LayoutObj* logits = as_layout(as_node(PyList_GET_ITEM(g->srcs, 0))->node_layout);
+    const int dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
+    const long long c = rank_of(logits) ? dim_of(logits, -1) : 0;
+    if (c == 0 || !is_float(dtype) || static_cast<int>(PyLong_AsLong(g->node_dtype)) != dtype) return 0;
+    Exec x;
+    x.device = device, x.dtype = dtype;
+    Results loss(x), grad(x);
+    loss.add(dtype, as_layout(n->node_layout)->numel);
+    grad.add(dtype, as_layout(g->node_layout)->numel);
+    if (!loss.ok || !grad.ok) return -1;
+    const int rc = unlocked([&] {
+      return L.mg_cross_entropy_fused_ids(address(b[0]), address(b[1]), address(b[2]), loss.p(0), grad.p(0),
+                                          logits->numel / c, c, dtype, b[1]->dtype, stream);
+    });
+    if (rc != 0) return raise_status(rc), -1;
+    return set(n, loss.list.release()) && set(g, grad.list.release()) ? 1 : -1;
+  }
+
+  bool evaluate(NodeObj* n) {
+    if (have(n)) return true;
+    if (!ce_grads.empty() && op_is(n, kCeIds)) {
+      const int rc = cross_entropy_pair(n);
+      if (rc != 0) return rc > 0;
+    }
+    if (op_is(n, kBuffer)) return raise_invalid("evaluate: a leaf node without a buffer"), false;
+    if (!op_is(n, kGetTuple)) return execute(n);
+    if (PyList_GET_SIZE(n->srcs) != 1) return raise_invalid("GETTUPLE takes one source"), false;
+    NodeObj* s = as_node(PyList_GET_ITEM(n->srcs, 0));
+    PyObject* index = PyDict_GetItem(n->node_attrs, N.index);
+    const Py_ssize_t i = index ? PyLong_AsSsize_t(index) : 0;
+    if (i == -1 && PyErr_Occurred()) return false;
+    PyObject* b = result(s, i);
+    PyObject* list = b ? PyList_New(1) : nullptr;
+    if (!list) return false;
+    Py_INCREF(b);
+    PyList_SET_ITEM(list, 0, b);
+    return set(n, list);
+  }
+};
+
+// evaluate(nodes, device, run): gives every node of `nodes` and of their sources its buffers.
+// The sources of a multi-output node's results that nobody in this walk reads may be left out.
+PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 3) return PyErr_SetString(PyExc_TypeError, "evaluate(nodes, device, run)"), nullptr;
+  Ref nodes(PySequence_Fast(args[0], "evaluate: nodes must be a sequence"));
+  if (!nodes) return nullptr;
+  Evaluation e;
+  e.device = args[1], e.run = args[2];
+  static PyObject *kBuffer = str_("BUFFER"), *kGetTuple = str_("GETTUPLE");
+  e.kBuffer = kBuffer, e.kGetTuple = kGetTuple;
+  static PyObject *kCeIds = str_("CROSS_ENTROPY_IDS"), *kCeIdsGrad = str_("CROSS_ENTROPY_IDS_GRAD");
+  e.kCeIds = kCeIds, e.kCeIdsGrad = kCeIdsGrad;
+  Ref stream(PyObject_GetAttr(e.device, N.stream)), pending(PyObject_GetAttr(e.device, N.pending));
+  if (!stream || !pending) return nullptr;
+  if (!pointer_of(stream.p, &e.stream) || !pointer_of(pending.p, &e.pending))
+    return PyErr_SetString(PyExc_TypeError, "evaluate: the device's stream is not a pointer"), nullptr;
+  std::vector<NodeObj*> order;
+  if (!toposort(PySequence_Fast_ITEMS(nodes.p), PySequence_Fast_GET_SIZE(nodes.p), order)) return nullptr;
+  for (NodeObj* v : order) {
+    v->used = 0;
+    if (e.op_is(v, kCeIdsGrad)) e.ce_grads.push_back(v);
+  }
+  for (NodeObj* v : order) {
+    const bool get = e.op_is(v, kGetTuple);
+    const Py_ssize_t srcs = PyList_GET_SIZE(v->srcs);
+    for (Py_ssize_t i = 0; i < srcs; ++i) {
+      uint32_t bit = 1u;  // a node read directly gives its first result
+      if (get) {
+        PyObject* index = PyDict_GetItem(v->node_attrs, N.index);
+        const long at = index ? PyLong_AsLong(index) : 0;
+        bit = at >= 0 && at < 31 ? 1u << at : ~0u;
+      }
+      as_node(PyList_GET_ITEM(v->srcs, i))->used |= bit;
+    }
+  }
+  for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(nodes.p); ++i)
+    as_node(PySequence_Fast_GET_ITEM(nodes.p, i))->used = ~0u;
+  for (NodeObj* v : order)
+    if (!e.evaluate(v)) return nullptr;
+  Py_RETURN_NONE;
+}
+
+// ------------------------------------------------------------------------------------------
+// The rewriting pass (mograd_amd/rewrites.py says what it does; this is its loop)
+// ------------------------------------------------------------------------------------------
+
+bool op_names_equal(PyObject* a, PyObject* b) { return a == b || PyUnicode_Compare(a, b) == 0; }
+
+// Pat.matches
+int pat_matches(PyObject* pat, NodeObj* n) {
+  Ref op(PyObject_GetAttr(pat, N.op_type)), srcs(PyObject_GetAttr(pat, N.srcs));
+  if (!op || !srcs) return -1;
+  if (op.p != Py_None && !op_names_equal(op.p, n->op_type)) return 0;
+  Ref fast(PySequence_Fast(srcs.p, "Pat.srcs"));
+  if (!fast) return -1;
+  const Py_ssize_t k = PySequence_Fast_GET_SIZE(fast.p);
+  if (k > PyList_GET_SIZE(n->srcs)) return 0;
+  for (Py_ssize_t i = 0; i < k; ++i) {
+    const int rc = pat_matches(PySequence_Fast_GET_ITEM(fast.p, i), as_node(PyList_GET_ITEM(n->srcs, i)));
+    if (rc <= 0) return rc;
+  }
+  return 1;
+}
+
+struct Pass {
+  PyObject* sim;
+  PyObject *subst, *uses, *origin, *consumers;  // the Simplifier's dictionaries (borrowed: it holds them)
+
+  // The node that `n` has become (borrowed).
+  PyObject* resolve(PyObject* n) const {
+    int seen = 0;
+    while (PyObject* to = PyDict_GetItem(subst, n)) {
+      n = to;
+      if (++seen > 64) return raise_invalid("Simplifier: substitutions cycled without converging"), nullptr;
+    }
+    return n;
+  }
+  int count(PyObject* n) const {
+    PyObject* c = PyDict_GetItem(uses, n);
+    return c ? static_cast<int>(PyLong_AsLong(c)) : 0;
+  }
+  bool set_count(PyObject* n, int c) const {
+    Ref v(PyLong_FromLong(c));
+    return v && PyDict_SetItem(uses, n, v.p) == 0;
+  }
+  bool set_origin(PyObject* made, PyObject* from) const {
+    PyObject* o = PyDict_GetItem(origin, from);
+    return PyDict_SetItem(origin, made, o ? o : from) == 0;
+  }
+  // A node like `n` over other sources (takes over `srcs`).
+  static PyObject* rebuilt(NodeObj* n, PyObject* srcs) {
+    PyObject* attrs = PyDict_Copy(n->node_attrs);
+    if (!attrs) return Py_DECREF(srcs), nullptr;
+    return node_make(n->op_type, n->node_layout, n->node_dtype, srcs, attrs, n->bufs);
+  }
+  // `node` with every source replaced by what it has become; a new reference.
+  PyObject* with_subst(PyObject* node) const {
+    NodeObj* n = as_node(node);
+    const Py_ssize_t k = PyList_GET_SIZE(n->srcs);
+    Ref fresh;
+    for (Py_ssize_t i = 0; i < k; ++i) {
+      PyObject* s = PyList_GET_ITEM(n->srcs, i);
+      PyObject* to = resolve(s);
+      if (!to) return nullptr;
+      if (to != s && !fresh) {
+        fresh = Ref(PyList_GetSlice(n->srcs, 0, k));
+        if (!fresh) return nullptr;
+      }
+      if (to != s) {
+        Py_INCREF(to);
+        PyList_SetItem(fresh.p, i, to);
+      }
+    }
+    if (!fresh) return Py_INCREF(node), node;
+    Ref out(rebuilt(n, fresh.release()));
+    if (!out || !set_count(out.p, count(node)) || !set_origin(out.p, node)) return nullptr;
+    return out.release();
+  }
+
+  // Every edge of the result follows the final substitution table.
+  PyObject* redirect(PyObject* roots) const {
+    Ref done(PyDict_New());
+    if (!done) return nullptr;
+    std::vector<std::pair<PyObject*, Py_ssize_t>> stack;
+    const Py_ssize_t n_roots = PySequence_Fast_GET_SIZE(roots);
+    for (Py_ssize_t i = n_roots - 1; i >= 0; --i) stack.emplace_back(PySequence_Fast_GET_ITEM(roots, i), 0);
+    while (!stack.empty()) {
+      PyObject* n = stack.back().first;
+      const Py_ssize_t i = stack.back().second;
+      PyObject* r = resolve(n);
+      if (!r) return nullptr;
+      if (PyObject* d = PyDict_GetItem(done.p, r)) {
+        stack.pop_back();
+        if (n != r && PyDict_SetItem(done.p, n, d) != 0) return nullptr;
+        continue;
+      }
+      NodeObj* v = as_node(r);
+      if (i < PyList_GET_SIZE(v->srcs)) {
+        stack.back().second = i + 1;
+        PyObject* c = PyList_GET_ITEM(v->srcs, i);
+        if (!PyDict_GetItem(done.p, c)) stack.emplace_back(c, 0);
+        continue;
+      }
+      stack.pop_back();
+      Ref fresh;
+      for (Py_ssize_t k = 0; k < PyList_GET_SIZE(v->srcs); ++k) {
+        PyObject* s = PyList_GET_ITEM(v->srcs, k);
+        PyObject* to = PyDict_GetItem(done.p, s);
+        if (to == s) continue;
+        if (!fresh) {
+          fresh = Ref(PyList_GetSlice(v->srcs, 0, PyList_GET_SIZE(v->srcs)));
+          if (!fresh) return nullptr;
+        }
+        Py_INCREF(to);
+        PyList_SetItem(fresh.p, k, to);
+      }
+      Ref out(fresh ? rebuilt(v, fresh.release()) : (Py_INCREF(r), r));
+      if (!out || PyDict_SetItem(done.p, r, out.p) != 0) return nullptr;
+      if (n != r && PyDict_SetItem(done.p, n, out.p) != 0) return nullptr;
+    }
+    PyObject* list = PyList_New(n_roots);
+    for (Py_ssize_t i = 0; list && i < n_roots; ++i) {
+      PyObject* d = PyDict_GetItem(done.p, PySequence_Fast_GET_ITEM(roots, i));
+      Py_INCREF(d);
+      PyList_SET_ITEM(list, i, d);
+    }
+    return list;
+  }
+};
+
+// simplify(sim, roots): Simplifier.run_many.
+PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  if (n_args != 2) return PyErr_SetString(PyExc_TypeError, "simplify(sim, roots)"), nullptr;
+  PyObject* sim = args[0];
+  Ref roots(PySequence_Fast(args[1], "Simplifier: roots must be a sequence"));
+  if (!roots) return nullptr;
+  std::vector<NodeObj*> topo;
+  if (!toposort(PySequence_Fast_ITEMS(roots.p), PySequence_Fast_GET_SIZE(roots.p), topo)) return nullptr;
+  Ref subst(PyDict_New()), uses(PyDict_New()), origin(PyDict_New()), consumers(PyDict_New());
+  if (!subst || !uses || !origin || !consumers || PyObject_SetAttr(sim, N.subst, subst.p) != 0 ||
+      PyObject_SetAttr(sim, N.uses, uses.p) != 0 || PyObject_SetAttr(sim, N.origin, origin.p) != 0 ||
+      PyObject_SetAttr(sim, N.consumers, consumers.p) != 0)
+    return nullptr;
+  Pass pass{sim, subst.p, uses.p, origin.p, consumers.p};
+  for (NodeObj* v : topo)
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(v->srcs); ++i) {
+      PyObject* s = PyList_GET_ITEM(v->srcs, i);
+      PyObject* list = PyDict_GetItem(consumers.p, s);
+      if (!list) {
+        Ref fresh(PyList_New(0));
+        if (!fresh || PyDict_SetItem(consumers.p, s, fresh.p) != 0) return nullptr;
+        list = PyDict_GetItem(consumers.p, s);
+      }
+      if (PyList_Append(list, reinterpret_cast<PyObject*>(v)) != 0) return nullptr;
+    }
+  {
+    PyObject *k, *v;
+    Py_ssize_t pos = 0;
+    while (PyDict_Next(consumers.p, &pos, &k, &v))
+      if (!pass.set_count(k, static_cast<int>(PyList_GET_SIZE(v)))) return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(roots.p); ++i) {  // a root is read by the caller
+    PyObject* r = PySequence_Fast_GET_ITEM(roots.p, i);
+    if (!pass.set_count(r, pass.count(r) + 1)) return nullptr;
+  }
+  Ref rules_attr(PyObject_GetAttr(sim, N.rules));
+  if (!rules_attr) return nullptr;
+  Ref rules(PySequence_Fast(rules_attr.p, "Simplifier.rules"));
+  if (!rules) return nullptr;
+  struct Compiled {
+    Ref pat, func, op;
+  };
+  std::vector<Compiled> compiled;
+  for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(rules.p); ++i) {
+    PyObject* r = PySequence_Fast_GET_ITEM(rules.p, i);
+    Compiled c;
+    c.pat = Ref(PyObject_GetAttr(r, N.pat));
+    c.func = Ref(PyObject_GetAttr(r, N.func));
+    if (!c.pat || !c.func) return nullptr;
+    c.op = Ref(PyObject_GetAttr(c.pat.p, N.op_type));
+    if (!c.op) return nullptr;
+    compiled.push_back(std::move(c));
+  }
+  for (NodeObj* v : topo) {
+    PyObject* node = reinterpret_cast<PyObject*>(v);
+    if (PyDict_GetItem(subst.p, node)) continue;  // a rule that ran on another node has already replaced this one
+    Ref now(pass.with_subst(node));
+    if (!now) return nullptr;
+    int round = 0;
+    for (; round < 64; ++round) {
+      bool progressed = false;
+      for (Compiled& c : compiled) {
+        if (c.op.p != Py_None && !op_names_equal(c.op.p, as_node(now.p)->op_type)) continue;
+        const int m = pat_matches(c.pat.p, as_node(now.p));
+        if (m < 0) return nullptr;
+        if (m == 0) continue;
+        Ref made(PyObject_CallFunctionObjArgs(c.func.p, now.p, sim, nullptr));
+        if (!made) return nullptr;
+        if (made.p == Py_None) continue;
+        if (!node_ok(made.p) || !pass.set_count(made.p, pass.count(now.p))) return nullptr;
+        if (!PyDict_GetItem(origin.p, made.p) && !pass.set_origin(made.p, now.p)) return nullptr;
+        now = Ref(pass.with_subst(made.p));
+        if (!now) return nullptr;
+        progressed = true;
+        break;
+      }
+      if (!progressed) break;
+    }
+    if (round == 64) return raise_invalid("Simplifier: rewrite rules cycled without converging"), nullptr;
+    if (now.p != node && PyDict_SetItem(subst.p, node, now.p) != 0) return nullptr;
+  }
+  return pass.redirect(roots.p);
+}
+
+// ------------------------------------------------------------------------------------------
+// Module
+// ------------------------------------------------------------------------------------------
+
+// bind(handle, MogradError, c_void_p, fallbacks): the library's functions, from its dlopen handle.
+PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4) return PyErr_SetString(PyExc_TypeError, "bind(handle, MogradError, c_void_p, fallbacks)"), nullptr;
+  void* handle = PyLong_AsVoidPtr(args[0]);
+  if (!handle && PyErr_Occurred()) return nullptr;
+#define X(f) L.f = reinterpret_cast<decltype(L.f)>(dlsym(handle, #f));
+  MG_FUNCTIONS(X)
+#undef X
+  L.pool_alloc = reinterpret_cast<decltype(L.pool_alloc)>(dlsym(handle, "mg_pool_alloc"));
+  L.last_error = reinterpret_cast<decltype(L.last_error)>(dlsym(handle, "mg_last_error"));
+  for (int i = 1; i < 4; ++i) Py_INCREF(args[i]);
+  Py_XSETREF(g_mograd_error, args[1]);
+  Py_XSETREF(g_void_p, args[2]);
+  Py_XSETREF(g_fallbacks, args[3]);
+  Py_RETURN_NONE;
+}
+PyObject* py_set_buffer_type(PyObject*, PyObject* type) {
+  if (!PyType_Check(type) || !PyType_IsSubtype(reinterpret_cast<PyTypeObject*>(type), &BufferType))
+    return PyErr_SetString(PyExc_TypeError, "a subclass of Buffer is wanted"), nullptr;
+  Py_INCREF(type);
+  Py_XSETREF(g_buffer_type, reinterpret_cast<PyTypeObject*>(type));
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {
+    {"toposort", py_toposort, METH_O, "Sources before consumers, each node once."},
+    {"depends_on", FAST(py_depends_on), METH_FASTCALL, "depends_on(node, target): whether target is node or feeds it."},
+    {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run)"},
+    {"simplify", FAST(py_simplify), METH_FASTCALL, "simplify(sim, roots)"},
+    {"bind", FAST(py_bind), METH_FASTCALL, "bind(handle, MogradError, c_void_p, fallbacks)"},
+    {"set_buffer_type", py_set_buffer_type, METH_O, "The type of the buffers that evaluate() makes."},
+    {nullptr, nullptr, 0, nullptr}};
+PyMethodDef library_methods[] = {
+#define X(f) {#f, FAST(py_##f), METH_FASTCALL, nullptr},
+    MG_FUNCTIONS(X)
+#undef X
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_graph", "Native host path of mograd_amd.", -1, module_methods, nullptr,
+                          nullptr, nullptr, nullptr};
+
+bool add_type(PyObject* m, PyTypeObject* t, const char* name) {
+  if (PyType_Ready(t) != 0) return false;
+  Py_INCREF(t);
+  return PyModule_AddObject(m, name, reinterpret_cast<PyObject*>(t)) == 0;
+}
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__graph() {
+  LayoutType.tp_name = "mograd_amd._graph.Layout";
+  LayoutType.tp_basicsize = sizeof(LayoutObj);
+  LayoutType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+  LayoutType.tp_new = layout_new;
+  LayoutType.tp_dealloc = layout_dealloc;
+  LayoutType.tp_members = layout_members;
+  LayoutType.tp_methods = layout_methods;
+  LayoutType.tp_richcompare = layout_richcompare;
+  LayoutType.tp_hash = layout_hash;
+  LayoutType.tp_repr = layout_repr;
+
+  NodeType.tp_name = "mograd_amd._graph.Node";
+  NodeType.tp_basicsize = sizeof(NodeObj);
+  NodeType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  NodeType.tp_doc =
+      "Just enough of an op node for the exec functions: its own layout and dtype, the layouts of its\n"
+      "sources, and its attributes (mograd/op.mojo:124-185).  `bufs` is what the reference keeps in op().buf\n"
+      "(mograd/scheduler.mojo:74-78): a leaf's buffer, or the results of an evaluated node.";
+  NodeType.tp_new = node_new;
+  NodeType.tp_dealloc = node_dealloc;
+  NodeType.tp_traverse = node_traverse;
+  NodeType.tp_clear = node_clear;
+  NodeType.tp_members = node_members;
+  NodeType.tp_methods = node_methods;
+  NodeType.tp_repr = node_repr;
+
+  StorageType.tp_name = "mograd_amd._graph.Storage";
+  StorageType.tp_basicsize = sizeof(StorageObj);
+  StorageType.tp_flags = Py_TPFLAGS_DEFAULT;
+  StorageType.tp_new = storage_new;
+  StorageType.tp_dealloc = storage_dealloc;
+  StorageType.tp_members = storage_members;
+
+  BufferType.tp_name = "mograd_amd._graph.Buffer";
+  BufferType.tp_basicsize = sizeof(BufferObj);
+  BufferType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+  BufferType.tp_new = buffer_new;
+  BufferType.tp_dealloc = buffer_dealloc;
+  BufferType.tp_members = buffer_members;
+  BufferType.tp_methods = buffer_methods;
+
+  N = {str_("index"), str_("eps"), str_("has_bias"), str_("accumulate"), str_("relu_mask"), str_("scale"), str_("is_causal"),
+       str_("stream"), str_("pending"), str_("func"), str_("pat"), str_("op_type"), str_("srcs"), str_("subst"), str_("uses"),
+       str_("origin"), str_("consumers"), str_("rules")};
+  PyObject* m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  if (!add_type(m, &LayoutType, "Layout") || !add_type(m, &NodeType, "Node") || !add_type(m, &StorageType, "Storage") ||
+      !add_type(m, &BufferType, "Buffer"))
+    return nullptr;
+  g_forms = PyDict_New();
+  for (size_t i = 0; i < sizeof(kForms) / sizeof(kForms[0]); ++i) {
+    Ref v(PyLong_FromSize_t(i)), k(str_(kForms[i].first));
+    if (!v || PyDict_SetItem(g_forms, k.p, v.p) != 0) return nullptr;
+  }
+  PyObject* lib = PyDict_New();
+  for (PyMethodDef* d = library_methods; lib && d->ml_name; ++d) {
+    Ref f(PyCFunction_New(d, nullptr));
+    if (!f || PyDict_SetItemString(lib, d->ml_name, f.p) != 0) return nullptr;
+  }
+  if (!lib || PyModule_AddObject(m, "library", lib) != 0) return nullptr;
+  return m;
+}

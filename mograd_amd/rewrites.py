@@ -29,7 +29,10 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Callable, Dict, List, Optional, Sequence
 
-from .runtime import Layout, MogradError, Node, _toposort
+from . import _graph
+from .runtime import Layout, MogradError, Node
+
+_depends_on = _graph.depends_on
 
 __all__ = ["Pat", "Rule", "Simplifier", "GPU_REWRITES"]
 
@@ -87,18 +90,7 @@ class Simplifier:
         """The consumers that `node` had in the graph as it was handed to the pass."""
         return self.consumers.get(self.origin.get(node, node), [])
 
-    # -- the pass ---------------------------------------------------------------------------
-    def _with_subst(self, node: Node) -> Node:
-        if not node.srcs:
-            return node
-        new_srcs = [self.resolve(s) for s in node.srcs]
-        if all(a is b for a, b in zip(new_srcs, node.srcs)):
-            return node
-        out = Node(node.op_type, node.node_layout, node.node_dtype, new_srcs, dict(node.node_attrs), node.bufs)
-        self.uses[out] = self.uses.get(node, 0)
-        self.origin[out] = self.origin.get(node, node)
-        return out
-
+    # -- the pass (native: _graph.simplify) -------------------------------------------------
     def resolve(self, node: Node) -> Node:
         seen = 0
         while node in self.subst:
@@ -109,65 +101,12 @@ class Simplifier:
         return node
 
     def run_many(self, roots: Sequence[Node]) -> List[Node]:
-        sink = Node("SINK", Layout(1), 0, list(roots))
-        topo = _toposort(sink)[:-1]
-        self.subst, self.uses, self.origin, self.consumers = {}, {}, {}, {}
-        for n in topo:
-            for s_ in n.srcs:
-                self.uses[s_] = self.uses.get(s_, 0) + 1
-                self.consumers.setdefault(s_, []).append(n)
-        for r in roots:  # a root is read by the caller
-            self.uses[r] = self.uses.get(r, 0) + 1
-        for node in topo:
-            if node in self.subst:  # a rule that ran on another node has already replaced this one
-                continue
-            node_r = self._with_subst(node)
-            for _ in range(64):
-                progressed = False
-                for rule in self.rules:
-                    if not rule.pat.matches(node_r):
-                        continue
-                    rewritten = rule.func(node_r, self)
-                    if rewritten is not None:
-                        self.uses[rewritten] = self.uses.get(node_r, 0)
-                        self.origin.setdefault(rewritten, self.origin.get(node_r, node_r))
-                        node_r = self._with_subst(rewritten)
-                        progressed = True
-                        break
-                if not progressed:
-                    break
-            else:
-                raise MogradError(1, "Simplifier: rewrite rules cycled without converging")
-            if node_r is not node:
-                self.subst[node] = node_r
-        return self._redirect(roots)
-
-    def _redirect(self, roots: Sequence[Node]) -> List[Node]:
-        """A rule may replace a node that earlier consumers already hold (the other selectors of a
-        multi-output producer that was refitted for one of them): rebuilds the result so that
-        every edge follows the final substitution table."""
-        done: Dict[Node, Node] = {}
-        stack = [(r, 0) for r in reversed(list(roots))]
-        while stack:
-            n, i = stack.pop()
-            r = self.resolve(n)
-            if r in done:
-                done[n] = done[r]
-                continue
-            if i < len(r.srcs):
-                stack.append((n, i + 1))
-                child = r.srcs[i]
-                if child not in done:
-                    stack.append((child, 0))
-                continue
-            new_srcs = [done[c] for c in r.srcs]
-            if all(a is b for a, b in zip(new_srcs, r.srcs)):
-                out = r
-            else:
-                out = Node(r.op_type, r.node_layout, r.node_dtype, new_srcs, dict(r.node_attrs), r.bufs)
-            done[r] = out
-            done[n] = out
-        return [done[r] for r in roots]
+        """Rewrites every node to a fixed point, sources first, by the first rule whose pattern
+        matches; a node whose sources were rewritten is rebuilt over what they became.  A rule may
+        replace a node that earlier consumers already hold (the other selectors of a multi-output
+        producer that was refitted for one of them), so at the end every edge is made to follow
+        the final substitution table."""
+        return _graph.simplify(self, roots)
 
     def run(self, root: Node) -> Node:
         return self.run_many([root])[0]
@@ -227,7 +166,7 @@ def fuse_add_into_linear_grad(node: Node, sim: Simplifier) -> Optional[Node]:
         lin = sel.src(0)
         if lin.attrs().get("accumulate") or not sim.single_use(sel) or not _same_shape(sel, other):
             continue
-        if other.dtype() != sel.dtype() or lin in _toposort(other):  # `other` must not depend on the product
+        if other.dtype() != sel.dtype() or _depends_on(other, lin):  # `other` must not depend on the product
             continue
         new = _refit(lin, "LINEAR_GRAD", list(lin.srcs) + [other], {**lin.attrs(), "accumulate": True}, sim)
         return Node("GETTUPLE", sel.node_layout, sel.node_dtype, [new], {"index": 0})
@@ -242,7 +181,7 @@ def fuse_add_into_layer_norm_grad(node: Node, sim: Simplifier) -> Optional[Node]
         ln = sel.src(0)
         if int(sel.attrs().get("index", -1)) != 0 or not sim.single_use(sel) or not _same_shape(sel, other):
             continue
-        if other.dtype() != sel.dtype() or ln in _toposort(other):
+        if other.dtype() != sel.dtype() or _depends_on(other, ln):
             continue
         new = _refit(ln, "LAYER_NORM_STATS_GRAD_ADD", list(ln.srcs) + [other], dict(ln.attrs()), sim)
         return Node("GETTUPLE", sel.node_layout, sel.node_dtype, [new], {"index": 0})
@@ -284,7 +223,7 @@ def fuse_add_into_linear_layer_norm_grad(node: Node, sim: Simplifier) -> Optiona
         fused = sel.src(0)
         if int(sel.attrs().get("index", -1)) != 0 or fused.attrs().get("accumulate") or not sim.single_use(sel):
             continue
-        if not _same_shape(sel, other) or other.dtype() != sel.dtype() or fused in _toposort(other):
+        if not _same_shape(sel, other) or other.dtype() != sel.dtype() or _depends_on(other, fused):
             continue
         new = _refit(fused, "LINEAR_LAYER_NORM_GRAD", list(fused.srcs) + [other], {**fused.attrs(), "accumulate": True}, sim)
         return Node("GETTUPLE", sel.node_layout, sel.node_dtype, [new], {"index": 0})

@@ -16,12 +16,11 @@ tests.  It contains no arithmetic: every result comes from the C ABI.
 from __future__ import annotations
 
 import ctypes as C
-from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
 
-from . import _lib
+from . import _graph, _lib
 from ._lib import BF16, F16, F32, I32, I64, MogradError
 
 __all__ = [
@@ -69,51 +68,13 @@ def round_to_dtype(a, dtype: int) -> np.ndarray:
 # --------------------------------------------------------------------------- #
 
 
-def _row_major(shape: Sequence[int]) -> Tuple[int, ...]:
-    strides = [1] * len(shape)
-    for i in range(len(shape) - 2, -1, -1):
-        strides[i] = strides[i + 1] * shape[i + 1]
-    return tuple(strides)
+class Layout(_graph.Layout):
+    """Shape, element strides and base offset (mograd/layout.mojo); immutable.
+    Layout(*shape, strides=None, base_offset=0): `dims`, `strides`, `base_offset`, rank(), shape(idx),
+    stride(idx), numel(), is_contiguous() (layout.mojo:210-212) and as_contiguous() (:238-240) are the
+    native base's."""
 
-
-@dataclass(frozen=True)
-class Layout:
-    """Shape, element strides and base offset (mograd/layout.mojo)."""
-
-    dims: Tuple[int, ...]
-    strides: Tuple[int, ...] = ()
-    base_offset: int = 0
-
-    def __init__(self, *shape, strides: Optional[Sequence[int]] = None, base_offset: int = 0):
-        if len(shape) == 1 and isinstance(shape[0], (tuple, list)):
-            shape = tuple(shape[0])
-        object.__setattr__(self, "dims", tuple(int(s) for s in shape))
-        st = _row_major(self.dims) if strides is None else tuple(int(s) for s in strides)
-        if len(st) != len(self.dims):
-            raise ValueError("strides rank differs from shape rank")
-        object.__setattr__(self, "strides", st)
-        object.__setattr__(self, "base_offset", int(base_offset))
-
-    def rank(self) -> int:
-        return len(self.dims)
-
-    def shape(self, idx: Optional[int] = None):
-        return self.dims if idx is None else self.dims[idx]
-
-    def stride(self, idx: Optional[int] = None):
-        return self.strides if idx is None else self.strides[idx]
-
-    def numel(self) -> int:
-        n = 1
-        for s in self.dims:
-            n *= s
-        return n
-
-    def is_contiguous(self) -> bool:  # layout.mojo:210-212
-        return self.strides == _row_major(self.dims)
-
-    def as_contiguous(self) -> "Layout":  # layout.mojo:238-240
-        return Layout(*self.dims)
+    __slots__ = ()
 
     def batch_dims_collapsible(self) -> bool:  # layout.mojo:214-236
         for i in range(self.rank() - 4, -1, -1):
@@ -208,35 +169,16 @@ class Device:
             pass
 
 
-class _Storage:
-    """One pooled allocation; returns to the free lists when the last view dies
-    (Storage, mograd/memory.mojo:199-239)."""
-
-    def __init__(self, device: Device, nbytes: int):
-        self.device = device
-        self.lib = device.lib
-        p = C.c_void_p()
-        self.lib.mg_pool_alloc(C.byref(p), nbytes)
-        self.ptr = p.value or 0
-        self.nbytes = nbytes
-
-    def __del__(self):
-        try:
-            if self.ptr:
-                self.lib.mg_pool_free(C.c_void_p(self.ptr))
-                self.ptr = 0
-        except Exception:
-            pass
+# One pooled allocation; returns to the free lists when the last view dies
+# (Storage, mograd/memory.mojo:199-239).
+_Storage = _graph.Storage
 
 
-class AnyBuffer:
-    """A typed device buffer (mograd/buffer.mojo:135-214).  `view` shares storage."""
+class AnyBuffer(_graph.Buffer):
+    """A typed device buffer (mograd/buffer.mojo:135-214): AnyBuffer(storage, dtype, numel, offset_elems=0).
+    `view(layout)` shares storage; data_ptr(with_offset=True) is the device address as a c_void_p."""
 
-    def __init__(self, storage: _Storage, dtype: int, numel: int, offset_elems: int = 0):
-        self.storage = storage
-        self.dtype = dtype
-        self.numel = numel
-        self.offset_elems = offset_elems
+    __slots__ = ()
 
     @staticmethod
     def supports(dtype: int) -> bool:
@@ -265,16 +207,6 @@ class AnyBuffer:
         device.lib.mg_copy_to_device(buf.data_ptr(), host.ctypes.data_as(C.c_void_p), host.nbytes, device.stream)
         return buf
 
-    def data_ptr(self, with_offset: bool = True) -> C.c_void_p:
-        off = self.offset_elems * _lib.DTYPE_SIZE[self.dtype] if with_offset else 0
-        return C.c_void_p(self.storage.ptr + off)
-
-    def size_bytes(self) -> int:
-        return self.numel * _lib.DTYPE_SIZE[self.dtype]
-
-    def view(self, layout: Layout) -> "AnyBuffer":
-        return AnyBuffer(self.storage, self.dtype, layout.numel(), layout.base_offset)
-
     def to_numpy(self, shape: Optional[Sequence[int]] = None) -> np.ndarray:
         """Synchronous download.  bfloat16 comes back as float32."""
         dev = self.storage.device
@@ -290,52 +222,18 @@ class AnyBuffer:
         return self.to_numpy().reshape(-1)[0].item()
 
 
+_graph.set_buffer_type(AnyBuffer)
+
+
 # --------------------------------------------------------------------------- #
 # Op nodes
 # --------------------------------------------------------------------------- #
 
 
-@dataclass(eq=False)
-class Node:
-    """Just enough of an op node for the exec functions: its own layout and dtype, the
-    layouts of its sources, and its attributes (mograd/op.mojo:124-185)."""
-
-    op_type: str
-    node_layout: Layout
-    node_dtype: int
-    srcs: List["Node"] = field(default_factory=list)
-    node_attrs: Dict[str, object] = field(default_factory=dict)
-    # What the reference keeps in op().buf (mograd/scheduler.mojo:74-78): a leaf's buffer, or
-    # the cached results of an evaluated node (several for a multi-output node).
-    bufs: Optional[List["AnyBuffer"]] = field(default=None, repr=False, compare=False)
-
-    def layout(self) -> Layout:
-        return self.node_layout
-
-    def dtype(self) -> int:
-        return self.node_dtype
-
-    def numel(self) -> int:
-        return self.node_layout.numel()
-
-    def src(self, i: int) -> "Node":
-        return self.srcs[i]
-
-    def attrs(self) -> Dict[str, object]:
-        return self.node_attrs
-
-    def shape(self, i: int) -> int:
-        return self.node_layout.shape(i)
-
-    @staticmethod
-    def leaf(layout: Layout, dtype: int = F32, buf: Optional["AnyBuffer"] = None) -> "Node":
-        return Node("BUFFER", layout, dtype, bufs=None if buf is None else [buf])
-
-    def __hash__(self) -> int:  # nodes are graph vertices: identity, like OpRef
-        return id(self)
-
-    def __eq__(self, other) -> bool:
-        return self is other
+# Node(op_type, node_layout, node_dtype, srcs=[], node_attrs={}, bufs=None): a graph vertex with layout(),
+# dtype(), numel(), src(i), attrs(), shape(i) and Node.leaf(layout, dtype, buf), compared and hashed by
+# identity like OpRef.
+Node = _graph.Node
 
 
 def _require_float(dtype: int, who: str) -> None:
@@ -1164,24 +1062,8 @@ GRAD_RULES = {
 }
 
 
-def _toposort(root: Node) -> List[Node]:
-    """Sources before consumers, each node once (GraphUtils.toposort); iterative, so that deep
-    training graphs do not run into the interpreter's recursion limit."""
-    order: List[Node] = []
-    seen = set()
-    stack = [(root, 0)]
-    seen.add(root)
-    while stack:
-        n, i = stack.pop()
-        if i < len(n.srcs):
-            stack.append((n, i + 1))
-            child = n.srcs[i]
-            if child not in seen:
-                seen.add(child)
-                stack.append((child, 0))
-        else:
-            order.append(n)
-    return order
+# Sources before consumers, each node once (GraphUtils.toposort).
+_toposort = _graph.toposort
 
 
 def gradient(root: Node, initial_grad: Node, targets: Sequence[Node]) -> List[Optional[Node]]:
@@ -1210,22 +1092,10 @@ def gradient(root: Node, initial_grad: Node, targets: Sequence[Node]) -> List[Op
 def evaluate(node: Node, device: Device) -> AnyBuffer:
     """Scheduler.run for one result (mograd/scheduler.mojo:40-80): evaluates the sources
     first, runs the node's rule once and keeps its buffers on the node; GETTUPLE selects an
-    output of a multi-output source."""
-    for n in _toposort(node):
-        _evaluate_node(n, device)
+    output of a multi-output source.  The walk is native, and so are the common forms of a
+    training step's ops; other ops and strided operands go through `run`."""
+    _graph.evaluate([node], device, run)
     return node.bufs[0]
-
-
-def _evaluate_node(n: Node, device: Device) -> None:
-    """One node whose sources have their buffers."""
-    if n.bufs is not None:
-        return
-    if n.op_type == "BUFFER":
-        raise MogradError(1, "evaluate: a leaf node without a buffer")
-    if n.op_type == "GETTUPLE":
-        n.bufs = [n.src(0).bufs[int(n.attrs()["index"])]]
-    else:
-        n.bufs = run(n, [s_.bufs[0] for s_ in n.srcs], device)
 
 
 def evaluate_many(nodes: Sequence[Node], device: Device, deferred_sums: bool = False) -> List[AnyBuffer]:
@@ -1233,15 +1103,12 @@ def evaluate_many(nodes: Sequence[Node], device: Device, deferred_sums: bool = F
     sub-graphs evaluated once.  With `deferred_sums` the second-stage sums of the parameter
     gradients (LINEAR_GRAD, LAYER_NORM_STATS_GRAD(_ADD), SCATTER_ADD) are left on one mg_deferred
     list and finished by a single launch after the walk: same bits, fewer launches."""
-    sink = Node("SINK", Layout(1), F32, list(nodes))
-    order = _toposort(sink)[:-1]
     if deferred_sums:
         pending = C.c_void_p()
         device.lib.mg_deferred_create(C.byref(pending))
         device.pending = pending
     try:
-        for n in order:
-            _evaluate_node(n, device)
+        _graph.evaluate(nodes, device, run)
         if deferred_sums:
             device.lib.mg_finish_deferred(device.pending, device.stream)
     finally:

@@ -284,9 +284,8 @@ class TinyTransformer:
 
         def param(name, shape=None):
             sl = self.slices[name]
-            shape = shape or sl.shape
-            numel = int(np.prod(shape))
-            leaf = Node.leaf(Layout(*shape), cd, AnyBuffer(self.work.storage, cd, numel, sl.offset))
+            layout = Layout(*(shape or sl.shape))
+            leaf = Node.leaf(layout, cd, AnyBuffer(self.work.storage, cd, layout.numel(), sl.offset))
             leaves[name] = leaf
             return leaf
 
