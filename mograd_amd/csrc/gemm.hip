@@ -1,6 +1,8 @@
 // C ABI for the matmul family: operand classification, kernel choice, launches.
 #include <algorithm>
+#include <cmath>
 
+#include "gemm_16bit_small.h"
 #include "gemm_f32_direct.h"
 #include "gemm_impl.h"
 #include "mg_deferred.h"
@@ -222,11 +224,78 @@ static int splitk_16bit_splits(int64_t blocks, int64_t K, int wg_per_cu) {
   if (splits > 64) splits = 64;
   return splits < 1 ? 1 : splits;
 }
+
+// Whether a 16-bit product is done faster with the 64 x 64 tiles of gemm_16bit_small.h than with
+// 128 x 128 ones in `splits128` K ranges, and with how many K ranges of its own (*splits).  Both
+// sides are estimated from what the kernels measured over 80 products of 64 to 16384 rows, 64 to
+// 3768 columns and K 64 to 16384 (within 20 % where either side is close): 3.6 us for a launch and
+// its ends, 0.24 us per step of 64 k of a 64 x 64 tile for each workgroup that a CU has to walk,
+// 0.5 us (0.35 of each where a CU has several) of a 128 x 128 tile; K ranges cost 2.6 us and
+// the partial tiles' way to memory and back at 3.5 TB/s.
+static bool small_16bit_tiles(int64_t M, int64_t N, int64_t K, int64_t batch, int splits128, int* splits) {
+  const double cus = device_info().cu_count;
+  const double steps = std::ceil(static_cast<double>(K) / kSmallBK);
+  auto partials = [](double tiles, int edge) { return 2.6 + tiles * edge * edge * 8.0 / 3.5e6; };
+  const double tiles64 = static_cast<double>(ceil_div(M, kSmallT) * ceil_div(N, kSmallT) * batch);
+  const double tiles128 = static_cast<double>(ceil_div(M, kGemmBM) * ceil_div(N, kGemmBN) * batch) * splits128;
+  const double t128 = 3.6 + steps / splits128 * std::max(0.5, 0.35 * tiles128 / cus) +
+                      (splits128 > 1 ? partials(tiles128, kGemmBM) : 0.0);
+  double best = 1e30;
+  for (int s = 1; s <= 16 && (s == 1 || (tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s) {
+    const double t = 3.6 + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) +
+                     (s > 1 ? partials(tiles64 * s, kSmallT) : 0.0);
+    if (t < best) best = t, *splits = s;
+  }
+  return best < t128;
+}
 // The K range of one workgroup, a multiple of the k-step, and the number of ranges that leaves.
 static int splitk_16bit_range(int64_t K, int* splits) {
   const int k_per_split = static_cast<int>(ceil_div(ceil_div(K, *splits), kG16BK) * kG16BK);
   *splits = static_cast<int>(ceil_div(K, k_per_split));
   return k_per_split;
+}
+
+// Sums the K ranges of a 16-bit product's partial tiles (gemm16_partial_floats) into C.
+template <typename T>
+static int launch_16bit_splitk_reduce(const GemmArgs& g, const float* partial, int splits, hipStream_t stream) {
+  const int64_t slice = gemm16_partial_floats(g.M, g.N, g.batch, 1);
+  if (slice / 1024 > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
+  const unsigned blocks = static_cast<unsigned>(slice / 1024);  // whole tiles: four outputs per thread
+  const T* bias = static_cast<const T*>(g.bias);
+  T* c = static_cast<T*>(g.c);
+  const int N = static_cast<int>(g.N), M = static_cast<int>(g.M), tiles_n = static_cast<int>(ceil_div(g.N, kGemmBN));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, partial, bias, c, slice, slice, splits, N,
+                       epilogue_of<T>(g), M, tiles_n);
+  };
+  if (bias) launch(gemm_splitk_reduce_kernel<T, true, true>);
+  else launch(gemm_splitk_reduce_kernel<T, false, true>);
+  MG_LAUNCH_CHECK();
+  return MG_OK;
+}
+
+template <typename T, bool A_KC, bool B_KC>
+static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream) {
+  const int64_t tiles_m = ceil_div(g.M, kSmallT), tiles_n = ceil_div(g.N, kSmallT), tiles = tiles_m * tiles_n;
+  const int k_per_split = splitk_16bit_range(g.K, &splits);
+  const int64_t grid = splits > 1 ? gemm_split_grid(tiles, splits, g.batch) : tiles * g.batch;
+  if (grid > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
+  Scratch partial;
+  if (splits > 1)
+    MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
+  const Gemm16Problem<T> pr{static_cast<const T*>(g.a), static_cast<const T*>(g.b), static_cast<const T*>(g.bias),
+                            static_cast<T*>(g.c), partial.as<float>(), static_cast<int>(g.M), static_cast<int>(g.N),
+                            static_cast<int>(g.K), A_KC ? g.sam : g.sak, B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb,
+                            g.M * g.N, static_cast<int>(tiles_m), static_cast<int>(tiles_n), k_per_split, splits,
+                            static_cast<int>(g.batch), epilogue_of<T>(g)};
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, pr);
+  };
+  if (splits > 1) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, true>);
+  else if (g.bias) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, true, false>);
+  else launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, false>);
+  MG_LAUNCH_CHECK();
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
 }
 
 // 16-bit MFMA path, optionally split along K when the output has too few tiles to fill
@@ -247,28 +316,36 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
   const int M = static_cast<int>(g.M), N = static_cast<int>(g.N), K = static_cast<int>(g.K);
   const int64_t cus = device_info().cu_count;
   int splits = splitk_16bit_splits(blocks, g.K, env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2));
-  // Tiles copied straight into LDS (gemm_16bit_pipe_kernel): an operand that is not k-contiguous is
+  // Outputs with few tiles: 64 x 64 ones (gemm_16bit_small.h).  Otherwise tiles copied straight into LDS (gemm_16bit_pipe_kernel): an operand that is not k-contiguous is
   // transposed by the LDS read instead of in registers, and a k-step costs one barrier.  64 k per
   // step and two copies of the tiles measured fastest or equal at every layout and size swept, 64 to
   // 16384 rows, 256 to 1536 columns, K 256 to 16384 (32 k per step 5-12 % slower below 16384 rows,
   // the register-staged kernel 4-40 %).  What the copy cannot take (operands that do not lie on
   // 16-byte chunks) is the register-staged kernel's, RAGGED.
-  // MOGRAD_HIP_GEMM16_PIPE = 0 | 322 | 642 | 2322 | 2642 overrides the choice: 0 the register-staged
-  // kernel, else k per step and copies of the tiles (2xxx: 256 x 128 tiles).
+  // MOGRAD_HIP_GEMM16_PIPE = 0 | 64 | 322 | 642 | 2322 | 2642 overrides the choice: 0 the register-staged
+  // kernel, 64 the 64 x 64 tiles, else k per step and copies of the tiles (2xxx: 256 x 128 tiles).
   int pipe = 0;
   if constexpr (!RAGGED) {
-    pipe = 642;
+    // (The K ranges are chosen with the tiles; a kernel that is asked for takes the same ones.)
+    int splits64 = 1;
+    const bool small = !env_str("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU") &&
+                       small_16bit_tiles(g.M, g.N, g.K, g.batch, splits, &splits64);
+    if (small) splits = splits64;
+    pipe = small ? 64 : 642;
     // Large products: 256 x 128 tiles (eight waves), a quarter fewer operand bytes per FLOP
     // through L2, once they still give every CU two workgroups (4096^3: 3-11 % faster).
-    if (splits <= 1 && g.K >= 1024 && ceil_div(g.M, 256) * tiles_n * g.batch >= 2 * cus) pipe = 2322;
+    if (!small && splits <= 1 && g.K >= 1024 && ceil_div(g.M, 256) * tiles_n * g.batch >= 2 * cus) pipe = 2322;
     // Products with a 256 x 256 tile for every CU: four waves of 128 x 128 each, one workgroup
     // per CU (gemm_16bit_big_kernel; 4642: 64 k per step and two copies of the tiles, 4324: 32 k
     // and four; 4096^3 forward 147 -> 121 us, 8192^3 dW 1016 -> 887 us, bit-identical results).
     // It takes whole k-steps only.
-    if (splits <= 1 && g.K >= 1024 && g.K % kG16BK == 0 &&
+    if (!small && splits <= 1 && g.K >= 1024 && g.K % kG16BK == 0 &&
         ceil_div(g.M, kGemmBigT) * ceil_div(g.N, kGemmBigT) * g.batch >= cus)
       pipe = 4642;
     pipe = static_cast<int>(env_int("MOGRAD_HIP_GEMM16_PIPE", pipe));
+  }
+  if constexpr (!RAGGED) {
+    if (pipe == 64) return launch_16bit_small<T, A_KC, B_KC>(g, splits, stream);
   }
   if (splits <= 1 && pipe >= 4000 && g.K % kG16BK == 0) {
     if constexpr (!RAGGED)
@@ -330,16 +407,7 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
   MG_GEMM16_LAUNCH(false, true, grid, partial.as<float>(), k_per_split, splits, (GemmEpilogue<T>{nullptr, nullptr, 0}));
 #undef MG_GEMM16_LAUNCH
   MG_LAUNCH_CHECK();
-  if (slice / 1024 > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
-  const unsigned rblocks = static_cast<unsigned>(slice / 1024);  // whole tiles: four outputs per thread
-  if (bias)
-    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<T, true, true>), dim3(rblocks), dim3(256), 0, stream,
-                       partial.as<float>(), bias, c, slice, slice, splits, N, epilogue_of<T>(g), M, tiles_n);
-  else
-    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<T, false, true>), dim3(rblocks), dim3(256), 0, stream,
-                       partial.as<float>(), bias, c, slice, slice, splits, N, epilogue_of<T>(g), M, tiles_n);
-  MG_LAUNCH_CHECK();
-  return MG_OK;
+  return launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream);
 }
 
 // fp32 products whose operands are each contiguous along one axis.
@@ -515,6 +583,55 @@ struct LinearBwdLayerNorm {
   void* dbeta;
 };
 
+// Input widths that are multiples of 384 can take 128 x 384 output tiles (twelve waves, one
+// workgroup per CU): the three column tiles of a row block share one copy of the dY tile,
+// a third fewer bytes from L2 per FLOP.  Taken when those tiles leave CUs free for dW's K ranges, so
+// that the whole launch is one workgroup per CU, and the layer is wide enough to pay for
+// the larger partial tiles.  MOGRAD_HIP_LINEAR_BWD_WIDE=0: 128 x 128 tiles.
+static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
+  return K % kGemmWideBN == 0 && ceil_div(M, kGemmBM) * (K / kGemmWideBN) < device_info().cu_count && N >= 768 &&
+         env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) != 0;
+}
+
+// Whether the backward of a 16-bit layer takes 64 x 64 tiles (gemm_16bit_small.h), and into how many K
+// ranges dW is then cut: the fewest that keep dW's walk along the rows well inside the rest;
+// more than one costs 3.6 us and the partial tiles' way to memory and back.
+// The larger tiles' lower LDS traffic wins once all steps together outweigh the tails and
+// padding that come with them (0.3 us per step of 64 k and CU against 0.9 us for four times the
+// output): (1024, 1024 <- 1024) 22.8 -> 11.3 us, (2587, 768 <- 256) 17.8 -> 12.7,
+// (9455, 4568 <- 64) 61 -> 37, but (3094, 1704 <- 776) 36 against 48 and (16384, 384 <- 384) 24
+// against 26.  The 128 x 384 tiles are one round of workgroups that walk the layer's outputs, 1.4 us
+// a step whatever the number of rows ((2048, 1152 <- 384) 32 us against 15, (2048, 3072 <- 768) 71
+// against 38, (8192, 1152 <- 384) 36 against 32); for 384 columns they can carry the LayerNorm
+// backward, which is 6 us as a launch of its own.
+// MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
+static bool small_linear_bwd(int64_t M, int64_t N, int64_t K, int* splits) {
+  const double cus = device_info().cu_count;
+  auto steps_per_cu = [&](int64_t tile) {  // of 64 k
+    return static_cast<double>(ceil_div(N, tile) * ceil_div(K, tile) * ceil_div(M, kSmallBK) +
+                               ceil_div(M, tile) * ceil_div(K, tile) * ceil_div(N, kSmallBK)) / cus;
+  };
+  const double steps_w = static_cast<double>(ceil_div(M, kSmallBK)), steps_x = static_cast<double>(ceil_div(N, kSmallBK));
+  const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
+  const double tiles_w = steps_x * tiles_k, tiles_x = steps_w * tiles_k;
+  const double load = steps_per_cu(kSmallT);
+  double best = 1e30;
+  for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
+    double chain = std::max(steps_w / s, steps_x);
+    if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + steps_x));  // two share a CU
+    const double t = 3.6 + 0.27 * std::max(1.5 * chain, load) + (s > 1 ? 3.6 + tiles_w * s * 0.0094 : 0.0);
+    if (t < best) best = t, *splits = s;
+  }
+  *splits = static_cast<int>(env_int("MOGRAD_HIP_LINEAR_BWD_SPLITS", *splits));
+  bool small;
+  if (wide_linear_bwd(M, N, K))
+    small = best + (K == kGemmWideBN ? 6.0 : 0.0) <= 10.0 + 1.4 * steps_x;
+  else  // (few rows: the larger tiles would take a launch for each product)
+    small = 0.3 * load <= (M < 1024 ? 9.0 : 4.0) + 0.9 * steps_per_cu(kGemmBM);
+  // (A choice of the larger tiles' form is also one for them.)
+  return env_int("MOGRAD_HIP_LINEAR_BWD_SMALL", small && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE")) != 0;
+}
+
 template <typename T>
 static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, void* dx, void* dw, void* db, int64_t M,
                                  int64_t N, int64_t K, const void* relu_mask, bool dx_accumulate, hipStream_t stream,
@@ -528,24 +645,21 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   // rows of the next multiple of 8, zeros behind (`pads` below); dX, dW and db keep their shape.
   const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || !aligned16(w);
   const int64_t cus = device_info().cu_count;
-  // Input widths that are multiples of 384 take 128 x 384 output tiles (twelve waves, one
-  // workgroup per CU): the three column tiles of a row block share one copy of the dY tile,
-  // a third fewer bytes from L2 per FLOP.  MOGRAD_HIP_LINEAR_BWD_WIDE=0: 128 x 128 tiles.
-  // Taken when those tiles leave CUs free for dW's K ranges, so that the whole launch is one
-  // workgroup per CU, and the layer is wide enough to pay for the larger partial tiles.
-  const bool wide = K % kGemmWideBN == 0 && ceil_div(M, kGemmBM) * (K / kGemmWideBN) < cus && N >= 768 &&
-                    env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) != 0;
+  int splits = 1;
+  const bool small = small_linear_bwd(M, N, K, &splits);
+  const bool wide = !small && wide_linear_bwd(M, N, K);
   if (ln && (!wide || K != kGemmWideBN || relu_mask || env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3 ||
              pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx)))
     return MG_OK;
-  const int tiles_kk = static_cast<int>(ceil_div(K, wide ? kGemmWideBN : kGemmBN));
+  const int tile = small ? kSmallT : kGemmBM;  // rows of an output tile
+  const int tiles_kk = static_cast<int>(ceil_div(K, small ? kSmallT : wide ? kGemmWideBN : kGemmBN));
   // dW: must be split, each workgroup's rows short enough for the 32-k variant.
-  const int w_tiles_m = static_cast<int>(ceil_div(N, kGemmBM));
+  const int w_tiles_m = static_cast<int>(ceil_div(N, tile));
   const int64_t w_tiles = static_cast<int64_t>(w_tiles_m) * tiles_kk;
-  const int x_tiles_m = static_cast<int>(ceil_div(M, kGemmBM));
+  const int x_tiles_m = static_cast<int>(ceil_div(M, tile));
   const int64_t x_tiles = static_cast<int64_t>(x_tiles_m) * tiles_kk;
-  int splits;
-  if (wide) {
+  if (small) {
+  } else if (wide) {
     // Every workgroup step is the same work (a 128 x 384 x 32 product), so the K ranges of dW
     // are cut to what a CU's share of all steps comes to: with fewer dX tiles than CUs the
     // ranges take the CUs that the tiles leave free, all in one round; otherwise the ranges
@@ -561,14 +675,12 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
     // the K ranges are half the partial tiles to write and sum (GPT step 3.06 -> 3.00 ms).
     splits = splitk_16bit_splits(w_tiles, M, env_int("MOGRAD_HIP_LINEAR_BWD_SPLIT_WG_PER_CU", 1));
   }
-  // Few rows (M < 1024): nothing is split, dW and db are the workgroups' own results
-  // (linear_bwd_short_16bit_kernel), unless their sums are deferred.
-  const bool split_sums = splits > 1 || deferred_current() != nullptr;
-  if (splits <= 1 && M >= 1024) return MG_OK;
+  const bool split_sums = splits > 1 || !small;
+  if (!small && splits <= 1) return MG_OK;
   if (ceil_div(M, splits) >= 4096) return MG_OK;
   const int k_per_split = splits > 1 ? splitk_16bit_range(M, &splits) : static_cast<int>(M);
   // dX, which is never split here: not a long reduction, and none that another split would serve better.
-  if (N >= 4096 || (N >= 1024 && (M < 1024 || ceil_div(M, 256) * tiles_kk >= 2 * cus))) return MG_OK;
+  if (!small && (N >= 4096 || (N >= 1024 && (M < 1024 || ceil_div(M, 256) * tiles_kk >= 2 * cus)))) return MG_OK;
   const int64_t n_dw = split_sums ? gemm_split_grid(w_tiles, splits, 1) : w_tiles;
   if (n_dw + x_tiles > 0x7fffffffLL) return MG_OK;
 
@@ -609,9 +721,16 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   int groups = 0;
   const bool db_here = db && env_int("MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH", 1) != 0;
   if (!split_sums) {
-    if (db_here) pw2.colsum = static_cast<T*>(db);
-    hipLaunchKernelGGL((linear_bwd_short_16bit_kernel<T>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(kGemmThreads),
-                       0, stream, pw2, px, static_cast<int>(n_dw));
+    // nothing to sum: where the gradients are wanted in fp32 they are written so here
+    DeferredList* dl = deferred_current();
+    if (dl && dl->out_dtype == MG_F32) {
+      pw2.c32 = static_cast<float*>(dl->write_here(dw));
+      if (db_here) pw2.colsum32 = static_cast<float*>(dl->write_here(db));
+    } else if (db_here) {
+      pw2.colsum = static_cast<T*>(db);
+    }
+    hipLaunchKernelGGL((linear_bwd_small_16bit_kernel<T, false>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
+                       dim3(kGemmThreads), 0, stream, pw2, px, static_cast<int>(n_dw));
     MG_LAUNCH_CHECK();
     *db_done = db_here;
     *done = true;
@@ -634,7 +753,10 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
                                    ln_part_g.as<float>(), ln_part_b.as<float>()};
     hipLaunchKernelGGL((linear_bwd_ln_16bit_kernel<T>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(2 * kGemmWideBN),
                        0, stream, pw2, px2, static_cast<int>(n_dw));
-  } else if (wide && env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3)  // 32 k per step, three copies: 3-4 % slower
+  } else if (small)
+    hipLaunchKernelGGL((linear_bwd_small_16bit_kernel<T, true>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
+                       dim3(kGemmThreads), 0, stream, pw2, px, static_cast<int>(n_dw));
+  else if (wide && env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3)  // 32 k per step, three copies: 3-4 % slower
     hipLaunchKernelGGL((linear_bwd_16bit_kernel<T, 3, kGemmWideBN>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
                        dim3(2 * kGemmWideBN), 0, stream, pw2, px, static_cast<int>(n_dw));
   else if (wide)  // 64 k per step, two copies (128 KB of LDS): half the barriers, whole cache lines of dY

@@ -742,7 +742,12 @@ typedef short gemm_i16x4 __attribute__((ext_vector_type(4)));
 // whichever 32 lanes the LDS serves together touch every bank once.  (With c ^ 2 * (kk % 4),
 // two sixteen-lane groups shared their bank groups: 43 % of the LDS cycles of the Linear
 // backward kernel were conflict cycles.)
-__device__ __forceinline__ constexpr int gemm16_tr_swizzle(int kk) { return 4 * (kk % 4) ^ 2 * ((kk / 8) % 2); }
+// With 64 rows a k-row is half a trip round the banks: the k-rows of one parity share a half, and
+// 4 * (kk / 2 % 2) keeps those of a group apart.
+template <int ROWS>
+__device__ __forceinline__ constexpr int gemm16_tr_swizzle(int kk) {
+  return (ROWS == 64 ? 4 * ((kk / 2) % 2) : 4 * (kk % 4)) ^ 2 * ((kk / 8) % 2);
+}
 
 // Copying one k-step of an operand of ROWS rows in a workgroup of NW waves: the waves that
 // take part (all of them, unless the step has fewer kilobytes than the workgroup has waves)
@@ -773,7 +778,7 @@ __device__ __forceinline__ void gemm16_pipe_sources(int64_t ld, int o0, int O,
       const int r = slot / CPR, c = (slot % CPR) ^ ((r / (16 / CPR)) % CPR);
       src[i] = static_cast<int64_t>(min(o0 + r, O - 1)) * ld + c * 8;  // rows past the edge are never stored
     } else {
-      const int kk = slot / CPK, c = (slot % CPK) ^ gemm16_tr_swizzle(kk);
+      const int kk = slot / CPK, c = (slot % CPK) ^ gemm16_tr_swizzle<ROWS>(kk);
       const int o = o0 + c * 8;
       src[i] = static_cast<int64_t>(kk) * ld + (o < O ? o : o0);
     }
@@ -826,7 +831,7 @@ __device__ __forceinline__ uint4 gemm16_pipe_frag(const char* __restrict__ lds_s
     const int o = o_base + ((lane / 16) % 2) * 16 + 4 * (lane % 4);  // first of the 4 rows this lane supplies
     const int kq = (lane % 16) / 4;                                 // its k-row within a group of 4
     const int kk = ks * 16 + (lane / 32) * 8 + kq;
-    const char* at = lds_step + kk * (ROWS * 2) + (((o / 8) ^ gemm16_tr_swizzle(kk)) * 16) + (o % 8) * 2;
+    const char* at = lds_step + kk * (ROWS * 2) + (((o / 8) ^ gemm16_tr_swizzle<ROWS>(kk)) * 16) + (o % 8) * 2;
     using lds_i16x4 = __attribute__((address_space(3))) gemm_i16x4;
     const gemm_i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         reinterpret_cast<lds_i16x4*>(reinterpret_cast<uintptr_t>(at)));
@@ -870,7 +875,10 @@ struct Gemm16Problem {
   // first tile column also sum their A tiles over k, i.e. dY over its rows, and leave one
   // partial row of the bias gradient per K range at colsum_part[split * M + m].
   float* colsum_part = nullptr;
-  T* colsum = nullptr;  // not split: the sums themselves
+  // Not split (64 x 64 tiles only): the sums themselves, or dW and the sums in fp32 instead of C and colsum.
+  T* colsum = nullptr;
+  float* c32 = nullptr;
+  float* colsum32 = nullptr;
   // The partial tiles are read back much later (their sum is deferred to the end of a training
   // step): store them past the caches.
   bool partial_stream = false;
@@ -882,7 +890,7 @@ struct Gemm16Problem {
 // gemm16_pipe_lds_bytes(BK, NSTAGE, TM, TN) bytes, aligned to 1024.  The output tile is
 // TM x TN, (TM / 64) x (TN / 64) waves with 64 x 64 each; pr.tiles_n counts tiles of TN columns.
 template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, int BK, int NSTAGE, int TM = 128,
-          int TN = kGemmBN, bool LN_BWD = false, bool COLSUM = SPLIT_K>
+          int TN = kGemmBN, bool LN_BWD = false>
 __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
   static_assert(NSTAGE >= 2 && NSTAGE <= 4 && (BK == 32 || BK == 64) && (TM == 128 || TM == 256), "stages");
   static_assert(TN % 128 == 0 && (!SPLIT_K || TM == 128), "partial tiles are 128 x 128");
@@ -942,8 +950,8 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
 
   // Column sums of the A tiles (see Gemm16Problem::colsum_part): a thread of the first four
   // waves takes one 16-byte chunk (8 of the tile's 128 m) of every 16th k-row.
-  constexpr bool CAN_COLSUM = COLSUM && !A_KC && TM == 128;
-  const bool colsum = CAN_COLSUM && (SPLIT_K ? pr.colsum_part != nullptr : pr.colsum != nullptr) && tn == 0;
+  constexpr bool CAN_COLSUM = SPLIT_K && !A_KC && TM == 128;
+  const bool colsum = CAN_COLSUM && pr.colsum_part != nullptr && tn == 0;
   const bool cs_thread = threadIdx.x < 256;
   const int cs_chunk = threadIdx.x % 16, cs_row = threadIdx.x / 16;
   float cs_acc[8];
@@ -1003,7 +1011,7 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
         for (int j = 0; j < BK / 16; ++j) {
           const int kk = cs_row + 16 * j;
           float v[8];
-          VecIO<T, 8>::load(reinterpret_cast<const T*>(la + kk * (TM * 2) + ((cs_chunk ^ gemm16_tr_swizzle(kk)) * 16)), v);
+          VecIO<T, 8>::load(reinterpret_cast<const T*>(la + kk * (TM * 2) + ((cs_chunk ^ gemm16_tr_swizzle<TM>(kk)) * 16)), v);
 #pragma unroll
           for (int e = 0; e < 8; ++e) cs_acc[e] += v[e];
         }
@@ -1050,8 +1058,7 @@ __device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sum += red[r * kPitch + threadIdx.x];
-        if constexpr (SPLIT_K) pr.colsum_part[static_cast<int64_t>(split) * M + m0 + threadIdx.x] = sum;
-        else pr.colsum[m0 + threadIdx.x] = from_float<T>(sum);
+        pr.colsum_part[static_cast<int64_t>(split) * M + m0 + threadIdx.x] = sum;
       }
       __syncthreads();
     }
@@ -1262,17 +1269,6 @@ __global__ __launch_bounds__(2 * TN, gemm16_pipe_occupancy(BK, NSTAGE, 128, TN))
   const int bid = blockIdx.x;
   if (bid < n_dw) gemm16_pipe_block<T, false, false, false, true, BK, NSTAGE, 128, TN>(lds, bid, dw);
   else gemm16_pipe_block<T, true, false, false, false, BK, NSTAGE, 128, TN>(lds, bid - n_dw, dx);
-}
-
-// The same launch for layers of few rows, whose dW is not split: dW and db are written by the
-// workgroups themselves and nothing follows (a small layer's backward is as long as its launches).
-template <typename T>
-__global__ __launch_bounds__(kGemmThreads, gemm16_pipe_occupancy(64, 2, 128)) void linear_bwd_short_16bit_kernel(
-    Gemm16Problem<T> dw, Gemm16Problem<T> dx, int n_dw) {
-  __shared__ __attribute__((aligned(1024))) char lds[gemm16_pipe_lds_bytes(64, 2, 128)];
-  const int bid = blockIdx.x;
-  if (bid < n_dw) gemm16_pipe_block<T, false, false, false, false, 64, 2, 128, 128, false, true>(lds, bid, dw);
-  else gemm16_pipe_block<T, true, false, false, false, 64, 2>(lds, bid - n_dw, dx);
 }
 
 // The same launch with the dX tiles (128 x 384: whole rows of a 384-wide layer input) continuing

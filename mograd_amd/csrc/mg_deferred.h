@@ -14,6 +14,7 @@
 // places that would launch a second stage ask deferred_current() and hand their work over.
 #pragma once
 
+#include <algorithm>
 #include <vector>
 
 #include "mg_internal.h"
@@ -50,6 +51,7 @@ struct DeferredList {
   // substitutions (from, to) of output pointers made for it (see DeferredScope).
   int out_dtype = MG_F32;
   std::vector<std::pair<void*, void*>> redirect;
+  std::vector<void*> written;  // real outputs that the call's kernels wrote themselves, in out_dtype
 
   void* target(void* out) const {
     for (const auto& r : redirect)
@@ -58,6 +60,11 @@ struct DeferredList {
   }
   void push(int kind, const float* part, void* out, int64_t slice, int rows, int cols, int groups, int64_t blocks) {
     jobs.push_back(DeferredJob{part, target(out), slice, kind, out_dtype, rows, cols, groups, static_cast<int>(blocks)});
+  }
+  // Where a kernel that can write `out` in out_dtype itself is to write it.
+  void* write_here(void* out) {
+    written.push_back(target(out));
+    return written.back();
   }
   // Takes over the pool block of `s`: it now lives until the list is finished.
   void hold(Scratch& s) {
@@ -84,11 +91,13 @@ class DeferredScope {
   DeferredScope(DeferredList* list, int dtype, int out_dtype) : list_(list), dtype_(dtype), out_dtype_(out_dtype) {
     list_->out_dtype = out_dtype;
     list_->redirect.clear();
+    list_->written.clear();
     deferred_set_current(list_);
   }
   ~DeferredScope() {
     deferred_set_current(nullptr);
     list_->redirect.clear();
+    list_->written.clear();
     for (auto& t : temps_) pool_release(t.tmp);
   }
   // The pointer to hand to the kernels in place of `out` (numel elements).
@@ -103,10 +112,10 @@ class DeferredScope {
     return MG_OK;
   }
   // After the entry point's work is enqueued: converts the substituted outputs that no
-  // deferred job took over.
+  // deferred job or kernel took over.
   int finish(hipStream_t stream) {
     for (const auto& t : temps_) {
-      bool deferred = false;
+      bool deferred = std::find(list_->written.begin(), list_->written.end(), t.real) != list_->written.end();
       for (size_t j = t.first_job; j < list_->jobs.size(); ++j) deferred |= list_->jobs[j].out == t.real;
       if (!deferred) MG_TRY(mg_cast(t.tmp, t.real, t.numel, dtype_, out_dtype_, stream));
     }

@@ -2,6 +2,8 @@
 that end on a short step, widths that are no multiple of a 16-byte chunk, outputs of a few tiles
 (fp32 straight from memory, 16 x 16 and 32 x 32), of 64 x 64 and of 128 x 128 tiles, and rows few enough
 that nothing is split.  All against float64 products of the rounded inputs."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,33 @@ def test_every_layout_batched(device, dtype, offset, M, N, K):
             lib.mg_matmul(ba.data_ptr(), bb.data_ptr(), c.data_ptr(), B, M, N, K, *((K, 1) if la == "k" else (1, M)),
                           *((1, K) if lb == "k" else (N, 1)), M * K, N * K, dtype, st)
             assert_close(c.to_numpy((B, M, N)), want, rt, rt * np.abs(want).max(), la + lb)
+
+
+# 16-bit 64 x 64 tiles: k steps of 64 around the four copies, one tile and many, K ranges, both gradient types
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 64, 192), (65, 72, 256), (262, 768, 768), (330, 64, 320), (72, 1032, 64),
+                                   (2000, 64, 128), (262, 768, 3072)])
+def test_tiles_of_64(device, dtype, M, N, K):
+    lib, st, rt = device.lib, device.stream, RT[dtype]
+    x = round_to_dtype(normal(62, 0, (M, K)), dtype)
+    w = round_to_dtype(normal(62, 1, (N, K), std=0.1), dtype)
+    dy = round_to_dtype(normal(62, 2, (M, N), std=0.5), dtype)
+    r = round_to_dtype(normal(62, 3, (M, N)), dtype)
+    bx, bw, bdy, br = (AnyBuffer.from_numpy(device, a, dtype) for a in (x, w, dy, r))
+    P = lambda t: t.data_ptr()  # noqa: E731
+    y = AnyBuffer.create(dtype, device, M * N)
+    lib.mg_matmul_bt_add(P(bx), P(bw), P(br), P(y), 1, M, N, K, K, 1, K, 1, M * K, N * K, dtype, st)
+    x, w, dy, r = (a.astype(np.float64) for a in (x, w, dy, r))
+    assert_close(y.to_numpy((M, N)), x @ w.T + r, rt, 2 * rt * np.abs(x @ w.T).max(), "y")
+    pending = C.c_void_p()
+    lib.mg_deferred_create(C.byref(pending))
+    for grad in (dtype, F32):
+        dx = AnyBuffer.create(dtype, device, M * K)
+        dw, db = AnyBuffer.create(grad, device, N * K, fill=3.0), AnyBuffer.create(grad, device, N, fill=3.0)
+        lib.mg_linear_bwd_deferred(P(bdy), P(bx), P(bw), P(dx), P(dw), P(db), M, N, K, 0, 0, dtype, grad, pending, st)
+        lib.mg_finish_deferred(pending, st)
+        g = rt if grad == dtype else 1e-5
+        for got, want, tol, name in ((dx.to_numpy((M, K)), dy @ w, rt, "dx"), (dw.to_numpy((N, K)), dy.T @ x, g, "dw"),
+                                     (db.to_numpy(), dy.sum(axis=0), g, "db")):
+            assert_close(got, want, tol, tol * np.abs(want).max(), f"{name} {grad}")
+    lib.mg_deferred_destroy(pending)
