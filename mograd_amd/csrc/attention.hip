@@ -1,7 +1,8 @@
 // C ABI for flash attention: argument checks, routing between the 16-bit MFMA kernels (16-bit
-// storage, head dimension up to 256), the fp32 MFMA kernels (head dimension up to 128) and the
-// general fp32 FMA kernels.
+// storage, head dimension up to 256), the fp32 MFMA kernels (up to 256, or 128 where rows do not lie
+// on 16-byte chunks) and the general fp32 FMA kernels.
 #include "attention_f32_mfma.h"
+#include "attention_f32_wave.h"
 #include "attention_generic.h"
 #include "attention_tiled.h"
 #include "mg_internal.h"
@@ -91,6 +92,83 @@ static void bwd_f32_mfma_launch(const void* d_o, const void* q, const void* k, c
 #undef MG_BWD_DP
 }
 
+// fp32 tensors whose rows lie on 16-byte chunks (attention_f32_wave.h), any sequence length.  Up to 64
+// columns and with 32-row tiles for every SIMD twice over the kernels of attention_f32_mfma.h are
+// the faster ones: a step is short then, and theirs reads a tile for four waves ((31, 512, 16 heads,
+// 64), causal: 915 us against 1140; (1, 4096, 4, 64), 512 tiles: 1490 against 690).  So they are on short
+// causal walks of more than 96 columns, which are all theirs ((16, 500, 12, 128): 824 against 1010).
+// MOGRAD_HIP_ATTN_F32_WAVE = 0 | 1 overrides the choice where either can be had.
+static int64_t attn_tiles32(const AttnDims& a) { return static_cast<int64_t>(a.B) * a.H * ceil_div(a.S, 32); }
+static bool attn_f32_wave_ok(const AttnDims& a, bool causal, const void* const* ptrs, int nptrs) {
+  if (a.D % 4 != 0 || a.D > kF32WaveMaxD || a.ld % 4 != 0) return false;
+  for (int i = 0; i < nptrs; ++i)
+    if (!aligned16(ptrs[i])) return false;
+  const bool tile_kernels = (a.D <= 64 || (causal && a.D > 96 && a.D <= 128 && a.S < 1024)) && a.S >= 64 &&
+                            attn_tiles32(a) >= 8 * device_info().cu_count;
+  // (a form of theirs that is asked for is had)
+  return env_int("MOGRAD_HIP_ATTN_F32_WAVE", !tile_kernels && !env_str("MOGRAD_HIP_ATTN_F32_MFMA")) != 0;
+}
+
+// Whether a wave gets 32 rows of its own or shares them with the workgroup's other three, whose partial
+// results cost 3 us to meet: its own once every SIMD has that many and the walks are equally long
+// ((32, 200, 12, 80): 98 + 284 us against 147 + 414; (16, 1024, 12, 96) causal: 665 + 1990 against
+// 554 + 1650).
+static bool f32_wave_own_tiles(const AttnDims& a, bool causal) {
+  return a.D > 64 && a.D <= 128 &&
+         env_int("MOGRAD_HIP_ATTN_F32_OWN", !causal && attn_tiles32(a) >= 4 * device_info().cu_count) != 0;
+}
+
+// f(DP, MODE, CAUSAL, HAS_BIAS) with the constants that the shape asks for.
+template <typename F>
+static void f32_wave_pick(const AttnDims& a, bool causal, bool has_bias, F f) {
+  auto modes = [&](auto dp, auto mode) {
+    if (causal) f(dp, mode, std::true_type{}, std::false_type{});
+    else if (has_bias) f(dp, mode, std::false_type{}, std::true_type{});
+    else f(dp, mode, std::false_type{}, std::false_type{});
+  };
+  const auto rows = std::integral_constant<F32WaveMode, kF32SplitRows>{};
+  auto wide = [&](auto mode) {
+    if (a.D <= 80) modes(std::integral_constant<int, 80>{}, mode);
+    else if (a.D <= 96) modes(std::integral_constant<int, 96>{}, mode);
+    else modes(std::integral_constant<int, 128>{}, mode);
+  };
+  if (a.D > 128) modes(std::integral_constant<int, 64>{}, std::integral_constant<F32WaveMode, kF32SplitColumns>{});
+  else if (a.D <= 32) modes(std::integral_constant<int, 32>{}, rows);
+  else if (a.D <= 64) modes(std::integral_constant<int, 64>{}, rows);
+  else if (f32_wave_own_tiles(a, causal)) wide(std::integral_constant<F32WaveMode, kF32OwnTiles>{});
+  else wide(rows);
+}
+
+static int fwd_f32_wave(const float* q, const float* k, const float* v, const float* mask, float* o, float* lse,
+                        const AttnDims& a, float scale, bool causal, bool has_bias, hipStream_t stream) {
+  const int tiles = static_cast<int>(ceil_div(a.S, 32));
+  const dim3 grid(static_cast<unsigned>(f32_wave_grid(static_cast<int64_t>(a.B) * a.H, tiles, f32_wave_own_tiles(a, causal))));
+  f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
+    hipLaunchKernelGGL((attn_fwd_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
+                       grid, dim3(256), 0, stream, q, k, v, mask, o, lse, a, scale, tiles);
+  });
+  MG_LAUNCH_CHECK();
+  return MG_OK;
+}
+
+static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const float* k, const float* v, const float* mask,
+                        const float* lse, float* dq, float* dk, float* dv, const AttnDims& a, float scale, bool causal,
+                        bool has_bias, hipStream_t stream) {
+  const int tiles = static_cast<int>(ceil_div(a.S, 32));
+  const int64_t heads = static_cast<int64_t>(a.B) * a.H;
+  const dim3 grid(static_cast<unsigned>(f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal))));
+  Scratch delta;
+  MG_TRY(delta.take(heads * a.S * static_cast<int64_t>(sizeof(float))));
+  f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
+    hipLaunchKernelGGL((attn_dq_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
+                       grid, dim3(256), 0, stream, d_o, o, q, k, v, mask, lse, delta.as<float>(), dq, a, scale, tiles);
+    hipLaunchKernelGGL((attn_dkdv_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
+                       grid, dim3(256), 0, stream, d_o, q, k, v, mask, lse, delta.as<float>(), dk, dv, a, scale, tiles);
+  });
+  MG_LAUNCH_CHECK();
+  return MG_OK;
+}
+
 template <typename T, int NT, int DL>
 static void fwd_tiled_launch(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse,
                              const AttnDims& a, float scale, bool causal, bool has_bias, hipStream_t stream) {
@@ -132,6 +210,12 @@ template <typename T>
 static int fwd_generic(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse, AttnDims a,
                        float scale, bool causal, bool has_bias, hipStream_t stream) {
   const int64_t rows = static_cast<int64_t>(a.B) * a.H * a.S;
+  if constexpr (sizeof(T) == 4) {
+    const void* ptrs[] = {q, k, v, o};
+    if (attn_f32_wave_ok(a, causal, ptrs, 4))
+      return fwd_f32_wave(static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
+                          static_cast<const T*>(mask), static_cast<T*>(o), lse, a, scale, causal, has_bias, stream);
+  }
   if (attn_f32_mfma_ok(a)) {
     fwd_f32_mfma_launch<T>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
     MG_LAUNCH_CHECK();
@@ -164,6 +248,13 @@ static int bwd_generic(const void* d_o, const void* o, const void* q, const void
                        const float* lse, void* dq, void* dk, void* dv, AttnDims a, float scale, bool causal,
                        bool has_bias, hipStream_t stream) {
   const int64_t rows = static_cast<int64_t>(a.B) * a.H * a.S;
+  if constexpr (sizeof(T) == 4) {
+    const void* ptrs[] = {d_o, o, q, k, v, dq, dk, dv};
+    if (attn_f32_wave_ok(a, causal, ptrs, 8))
+      return bwd_f32_wave(static_cast<const T*>(d_o), static_cast<const T*>(o), static_cast<const T*>(q),
+                          static_cast<const T*>(k), static_cast<const T*>(v), static_cast<const T*>(mask), lse,
+                          static_cast<T*>(dq), static_cast<T*>(dk), static_cast<T*>(dv), a, scale, causal, has_bias, stream);
+  }
   Scratch delta;
   MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
   const dim3 grid(static_cast<unsigned>(ceil_div(rows, 4)));

@@ -129,6 +129,22 @@ def test_f32_matrix_core_kernels(device, monkeypatch, name, causal, with_mask, B
         np.testing.assert_array_equal(a_, b_)
 
 
+@pytest.mark.parametrize("own", ["0", "1"])  # tiles of 32 rows shared by the four waves, or one each
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("B,H,S,D", [(1, 1, 1, 4), (2, 3, 20, 32), (1, 2, 33, 64), (1, 1, 129, 80), (2, 1, 160, 72),
+                                     (1, 3, 100, 96), (1, 1, 257, 128), (1, 2, 31, 100), (1, 1, 65, 256), (1, 2, 200, 132)])
+def test_f32_waves_on_their_own(device, monkeypatch, own, name, causal, with_mask, B, H, S, D):
+    # One row to several tiles per wave, columns that fill a kernel's width and that do not, and
+    # columns divided among the waves (more than 128).
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_F32_WAVE", "1")
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_F32_OWN", own)
+    q, k, v, do, m = _inputs(61, B, S, H, D, F32, with_mask)
+    ro, rl = O.sdpa_fwd(q, k, v, m, causal)
+    want = (ro, rl) + tuple(O.sdpa_bwd(q, k, v, do, m, causal))
+    for g, w, what in zip(_fwd_bwd(device, q, k, v, do, m, causal), want, ("o", "lse", "dq", "dk", "dv")):
+        assert _max_err(g, w) <= (1e-5 if D <= 128 else 2e-5), f"{what}: {_max_err(g, w)}"
+
+
 HALF_SHAPES = [(2, 2, 96, 64), (1, 3, 200, 64), (2, 1, 128, 128), (1, 2, 257, 32), (1, 1, 4, 8), (1, 2, 96, 256),
                (1, 2, 130, 72), (1, 1, 80, 512), (1, 2, 40, 192), (1, 2, 300, 256), (2, 1, 130, 200), (1, 1, 129, 136)]
 
