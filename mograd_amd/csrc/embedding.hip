@@ -45,47 +45,6 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ 
   }
 }
 
-// One wave per (destination row, column block, slab).  DIRECT writes the row itself (one
-// slab); otherwise fp32 partials (slab, row, col) go to scratch for the partials reduction.
-template <typename T, typename I, int VEC, bool DIRECT>
-__global__ __launch_bounds__(64) void scatter_rows_kernel(const I* __restrict__ indices, const T* __restrict__ values,
-                                                          float* __restrict__ part, T* __restrict__ dst, int64_t n_idx,
-                                                          int64_t num_rows, int64_t row_size, int64_t slab_len) {
-  const int lane = threadIdx.x;
-  const int64_t col = (static_cast<int64_t>(blockIdx.y) * 64 + lane) * VEC;
-  const int64_t row = blockIdx.x;
-  const int64_t slab = blockIdx.z;
-  const int64_t i0 = slab * slab_len;
-  const int64_t i1 = min(i0 + slab_len, n_idx);
-  const bool active = col < row_size;
-  float acc[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
-  for (int64_t base = i0; base < i1; base += 64) {
-    const int64_t mine = base + lane;
-    const bool hit = mine < i1 && static_cast<int64_t>(indices[mine]) == row;
-    uint64_t hits = __ballot(hit);
-    while (hits) {  // wave-uniform: ascending index order
-      const int bit = __ffsll(static_cast<long long>(hits)) - 1;
-      hits &= hits - 1;
-      if (active) {
-        float v[VEC];
-        VecIO<T, VEC>::load(values + (base + bit) * row_size + col, v);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] += v[e];
-      }
-    }
-  }
-  if (!active) return;
-  if constexpr (DIRECT) {
-    VecIO<T, VEC>::store(dst + row * row_size + col, acc);
-  } else {
-    float* p = part + (slab * num_rows + row) * row_size + col;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) p[e] = acc[e];
-  }
-}
-
 // VEC elements of a value row as loaded, unpacked to floats only when they are added: eight
 // of them wait in registers for the loads of a long run.
 template <typename T, int VEC>
@@ -116,6 +75,73 @@ struct PackedChunk {
     }
   }
 };
+
+// One wave per (destination row, column block, slab).  DIRECT writes the row itself (one
+// slab); otherwise fp32 partials (slab, row, col) go to scratch for the partials reduction.
+// 256 indices are compared at a time and the positions that hit listed in LDS, in order; their value
+// rows are then fetched sixteen at a time and added in that order.  (Fetched where each was found, a
+// row waited for the one before it: the most frequent of 65 symbols over 16384 tokens of text is
+// a fifth of them, 54 round trips a slab, 24 us; a toy's 17 symbols over 128 tokens 10 us.)
+template <typename T, typename I, int VEC, bool DIRECT>
+__global__ __launch_bounds__(64) void scatter_rows_kernel(const I* __restrict__ indices, const T* __restrict__ values,
+                                                          float* __restrict__ part, T* __restrict__ dst, int64_t n_idx,
+                                                          int64_t num_rows, int64_t row_size, int64_t slab_len) {
+  constexpr int kBlocks = 4, kFlight = 16;
+  __shared__ int list[kBlocks * 64];
+  const int lane = threadIdx.x;
+  const int64_t col = (static_cast<int64_t>(blockIdx.y) * 64 + lane) * VEC;
+  const int64_t row = blockIdx.x;
+  const int64_t slab = blockIdx.z;
+  const int64_t i0 = slab * slab_len;
+  const int64_t i1 = min(i0 + slab_len, n_idx);
+  const bool active = col < row_size;
+  const int64_t col_in = active ? col : 0;
+  float acc[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
+  for (int64_t base = i0; base < i1; base += kBlocks * 64) {
+    I index[kBlocks];
+#pragma unroll
+    for (int k = 0; k < kBlocks; ++k) {
+      const int64_t mine = base + k * 64 + lane;
+      index[k] = mine < i1 ? indices[mine] : static_cast<I>(-1);
+    }
+    int count = 0;
+#pragma unroll
+    for (int k = 0; k < kBlocks; ++k) {
+      const bool hit = static_cast<int64_t>(index[k]) == row;
+      const uint64_t hits = __ballot(hit);
+      if (hit) list[count + __popcll(hits & ((uint64_t{1} << lane) - 1))] = k * 64 + lane;
+      count += __popcll(hits);
+    }
+    __syncthreads();
+    for (int j = 0; j < count; j += kFlight) {  // wave-uniform: ascending index order
+      const int mine = list[min(j + lane % kFlight, count - 1)];
+      PackedChunk<T, VEC> q[kFlight];
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u)  // (past the end the last row again)
+        q[u].load(values + (base + __builtin_amdgcn_readlane(mine, u)) * row_size + col_in);
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u) {
+        if (j + u < count) {
+          float v[VEC];
+          q[u].unpack(v);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) acc[e] += v[e];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!active) return;
+  if constexpr (DIRECT) {
+    VecIO<T, VEC>::store(dst + row * row_size + col, acc);
+  } else {
+    float* p = part + (slab * num_rows + row) * row_size + col;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) p[e] = acc[e];
+  }
+}
 
 // ---- large tables, short index lists: one launch ------------------------------------------
 // A workgroup owns 4 * rows_per_wave consecutive destination rows and one block of 64 * VEC
@@ -604,9 +630,11 @@ static int gather_typed(const void* src, const void* indices, void* dst, int64_t
 template <typename T, typename I, int VEC>
 static int scatter_launch(const I* indices, const T* values, T* dst, int64_t n_idx, int64_t num_rows, int64_t row_size,
                           hipStream_t s) {
-  // Tables of a thousand rows and more: bucket first (MOGRAD_HIP_SCATTER_BUCKET_MIN_ROWS moves
-  // the threshold; (50304, 768) from 8192 rows took 5 ms by scanning).
-  if (num_rows >= env_int("MOGRAD_HIP_SCATTER_BUCKET_MIN_ROWS", 1024) && n_idx > 0 && n_idx < 0x7fffffffLL &&
+  // Tables of a thousand rows and more: bucket first, unless the scan is short ((1476, 128) from 3388
+  // rows: 56 us bucketed, 21 scanned; (50304, 768) from 8192 rows took 5 ms by scanning).
+  // MOGRAD_HIP_SCATTER_BUCKET_MIN_ROWS moves the threshold.
+  const bool long_scan = num_rows * n_idx > (int64_t{1} << 24) || env_str("MOGRAD_HIP_SCATTER_BUCKET_MIN_ROWS");
+  if (num_rows >= env_int("MOGRAD_HIP_SCATTER_BUCKET_MIN_ROWS", 1024) && long_scan && n_idx > 0 && n_idx < 0x7fffffffLL &&
       num_rows < 0x7fffffffLL) {
     // Short lists: every workgroup of a row range reads the whole list, up to 2^(the knob)
     // index reads in all (MOGRAD_HIP_SCATTER_RANGE_READS_LOG2; 0 switches the form off), and a
