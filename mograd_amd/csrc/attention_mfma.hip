@@ -276,26 +276,27 @@ __device__ __forceinline__ void store4(T* dst, const floatx16& acc, int g, float
 
 // Additive bias (B, H, S, S): in the forward and the dQ walk a lane keeps one query row and its
 // accumulator registers run over keys in groups of four consecutive ones, so the bias of a
-// group is one 8-byte load where the row allows it (S a multiple of 4, the tensor 8-byte
-// aligned, the group inside the row); the two lanes of a row then read whole 16-byte pieces
-// and, over a step's eight groups, exactly the row's 128 bytes.  (Element by element, 32
-// two-byte loads per lane and step, the forward ran at 0.7 TB/s of bias: 1.10 ms at B2 H12
-// S4096 against 0.17 ms without a bias.)
+// group inside the row is one 8-byte load, at whatever even address it lies; the two lanes of a row then
+// read whole 16-byte pieces and, over a step's eight groups, exactly the row's 128 bytes.
+// (Element by element, 32 two-byte loads per lane and step, the forward ran at 0.7 TB/s of bias:
+// 1.10 ms at B2 H12 S4096 against 0.17 ms without a bias; and with rows of 1061, which start on no
+// 8-byte boundary, forward and backward took 279 us at B19 H2 D64 against 180.)
 template <typename T>
 __device__ __forceinline__ float bias_at(const uint2& w, int j) {
   T h[4];
   __builtin_memcpy(h, &w, 8);
   return to_float(h[j]);
 }
-__device__ __forceinline__ bool bias_rows_vectorise(const void* mask, int S) {
-  return S % 4 == 0 && reinterpret_cast<uintptr_t>(mask) % 8 == 0;
-}
+typedef uint32_t bias_u2_any __attribute__((ext_vector_type(2), aligned(2)));
 // row[n .. n + 3] as four packed 16-bit values; `packed`: one 8-byte load, else element by element
 // with the index clamped to the row (the values past its end are never used).
 template <typename T>
 __device__ __forceinline__ uint2 bias_group(const T* __restrict__ row, int n, int S, bool packed) {
   static_assert(sizeof(T) == 2, "16-bit tensors");
-  if (packed) return *reinterpret_cast<const uint2*>(row + n);
+  if (packed) {
+    const bias_u2_any v = *reinterpret_cast<const bias_u2_any*>(row + n);
+    return make_uint2(v[0], v[1]);
+  }
   const uint16_t* raw = reinterpret_cast<const uint16_t*>(row);
   uint2 w;
   w.x = raw[min(n, S - 1)] | static_cast<uint32_t>(raw[min(n + 1, S - 1)]) << 16;
@@ -348,7 +349,6 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_fwd_mfma
   float m_run = -INFINITY, l_run = 0.f;
   const float c = scale * kAttnLog2e;
   const T* mrow = HAS_BIAS ? mask + ((static_cast<int64_t>(b) * a.H + h) * a.S + min(m, a.S - 1)) * a.S : nullptr;
-  const bool bias_vec = HAS_BIAS && bias_rows_vectorise(mask, a.S);
 
   const int n_end = CAUSAL ? min(a.S, qb * BM + BM) : a.S;
   TileStager<T, BN, DP> ks_stage, vs_stage;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_fwd_mfma
     // heads), else tile by tile where it is used.
     constexpr bool BIAS_EARLY = DP <= 64;
     uint2 bias_w[2][4];
-    const bool bias_packed = bias_vec && n0 + BN <= a.S;
+    const bool bias_packed = n0 + BN <= a.S;
     auto load_bias = [&](int nt) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) bias_w[nt][g] = bias_group<T>(mrow, n0 + nt * 32 + g * 8 + half * 4, a.S, bias_packed);
@@ -577,7 +577,6 @@ __device__ __forceinline__ void attn_dq_block(const int block, char* smem, const
     for (int dt = 0; dt < DT; ++dt) acc[mq][dt] = zero16();
   }
 
-  const bool bias_vec = HAS_BIAS && bias_rows_vectorise(mask, a.S);
   const int n_end = CAUSAL ? min(a.S, qb * BM + BM) : a.S;
   TileStager<T, BN, DP> ks_stage, vs_stage;
   ks_stage.begin(kbase, ld, 0);
@@ -598,7 +597,7 @@ __device__ __forceinline__ void attn_dq_block(const int block, char* smem, const
   constexpr bool BIAS_AHEAD = HAS_BIAS && DP <= 64;
   uint2 bias_cur[MQ][BN / 32][4], bias_nxt[MQ][BN / 32][4];
   auto load_bias_step = [&](int n0, uint2 (&dst)[MQ][BN / 32][4]) {
-    const bool packed = bias_vec && n0 + BN <= a.S;
+    const bool packed = n0 + BN <= a.S;
 #pragma unroll
     for (int mq = 0; mq < MQ; ++mq)
 #pragma unroll
@@ -649,7 +648,7 @@ __device__ __forceinline__ void attn_dq_block(const int block, char* smem, const
     for (int nt = 0; nt < BN / 32; ++nt) {
       floatx16 s[MQ], dp[MQ];
       uint2 bias_w[MQ][4];
-      const bool bias_packed = bias_vec && n0 + nt * 32 + 32 <= a.S;
+      const bool bias_packed = n0 + nt * 32 + 32 <= a.S;
       auto load_bias = [&](int mq) {
 #pragma unroll
         for (int g = 0; g < 4; ++g)
