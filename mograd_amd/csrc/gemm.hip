@@ -411,9 +411,12 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
 }
 
 // fp32 products whose operands are each contiguous along one axis.
-//   tiles copied into LDS, 128 x 128 where every CU gets one ((4096, 1024) <- 1024: 74 us, 81 with
-//   64 x 64), else 64 x 64 down to one for every second CU ((2048, 768) <- 768: 31 us against 55 with
-//   128 x 128 and 42 straight from memory), fewer where a long reduction can be split as well;
+//   tiles copied into LDS, 128 x 128 where every CU gets one and the last round of them is not so
+//   empty that 64 x 64 ones, 6 % slower in themselves, are done first ((8000, 600) <- 900, 315 large
+//   tiles: 126 us against 89; (1390, 3016) <- 576: 80 against 58; (4096, 1024) <- 1024 74 against 81);
+//   64 x 64 down to one for every second CU ((2048, 768) <- 768: 31 us against 55 with
+//   128 x 128 and 42 straight from memory), fewer where a long reduction can be split as well
+//   ((480, 160) <- 11200: 35 against 51);
 //   operands that do not lie on 16-byte chunks are copied to rows that do, which takes a tile
 //   per CU to pay ((1999, 1001) <- 767: 44 us against 59; (2587, 256) <- 256: 14 against 10);
 //   everything smaller straight from memory (gemm_f32_direct.h).
@@ -430,8 +433,12 @@ static int dispatch_f32(const GemmArgs& g_in, hipStream_t stream, bool* handled)
   if (!*handled) return MG_OK;
   const bool a_wide = (a_kc ? mult4(g.sam) && mult4(g.K) : mult4(g.sak) && mult4(g.M)) && mult4(g.bsa) && aligned16(g.a);
   const bool b_wide = (b_kc ? mult4(g.sbn) && mult4(g.K) : mult4(g.sbk) && mult4(g.N)) && mult4(g.bsb) && aligned16(g.b);
-  const bool use64 = a_wide && b_wide ? 2 * blocks64 >= cus || (8 * blocks64 >= cus && g.K >= 1024) : blocks64 >= cus;
-  const int tile = env_int("MOGRAD_HIP_GEMM_F32_TILE", blocks128 >= cus ? 128 : use64 ? 64 : 32);
+  const bool wide = a_wide && b_wide;
+  const bool use64 = wide ? 2 * blocks64 >= cus || (8 * blocks64 >= cus && g.K >= 1024) ||
+                                (g.K >= 4096 && 2.0 * g.batch * g.M * g.N * g.K >= 4e8)
+                          : blocks64 >= cus;
+  const bool use128 = blocks128 >= cus && 4.0 * ceil_div(blocks128, cus) <= 1.06 * ceil_div(blocks64, cus);
+  const int tile = env_int("MOGRAD_HIP_GEMM_F32_TILE", use128 ? 128 : use64 ? 64 : 32);
   if (tile == 32) {
     if (a_kc && b_kc) return launch_f32_direct<true, true>(g, stream);
     if (a_kc) return launch_f32_direct<true, false>(g, stream);
