@@ -306,12 +306,16 @@ __device__ __forceinline__ uint2 bias_group(const T* __restrict__ row, int n, in
 
 // ---- forward -----------------------------------------------------------------------------
 
-template <typename T, int DP, bool CAUSAL, bool HAS_BIAS>
+// DC: the columns that are multiplied, where they are fewer than the DP of the staged rows (heads of 80
+// and 96 columns in the 128-column kernels, of 32 in the 64-column ones; the rest of a row is
+// staged as zeros and left alone).  bf16 (8, 500, 8 heads, 96), causal:
+// 20 + 78 us forward + backward with 128 columns, 17 + 58 with 96; (30, 1616, 3, 32): 53 -> 45 forward.
+template <typename T, int DP, bool CAUSAL, bool HAS_BIAS, int DC>
 __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_fwd_mfma_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                         const T* __restrict__ v,
                                                                         const T* __restrict__ mask, T* __restrict__ o,
                                                                         float* __restrict__ lse, AttnDims a, float scale) {
-  constexpr int BM = 128, BN = 64, KS = DP / 16, DT = DP / 32;
+  constexpr int BM = 128, BN = 64, KS = DC / 16, DT = DC / 32;
   // Two copies of each staged tile: step i computes from copy i % 2 while the tile of step
   // i + 1 is written into the other, so one barrier per step suffices.
   __shared__ __attribute__((aligned(16))) char k_rows_s[2][BN * tile_row_bytes<DP>()];
@@ -511,14 +515,14 @@ constexpr int dq_lds_bytes() {
 // DSPLIT > 1: the workgroup produces only part DPART of the head dimension's DSPLIT equal
 // parts of dQ (the score products still run over the whole head), so that the accumulators of a
 // 256-wide head fit the register file; the parts are separate workgroups.
-template <typename T, int DP, int MQ, bool CAUSAL, bool HAS_BIAS, int DSPLIT = 1, int DPART = 0>
+template <typename T, int DP, int MQ, bool CAUSAL, bool HAS_BIAS, int DC = DP, int DSPLIT = 1, int DPART = 0>
 __device__ __forceinline__ void attn_dq_block(const int block, char* smem, const T* __restrict__ d_o,
                                               const T* __restrict__ q, const T* __restrict__ k,
                                               const T* __restrict__ v, const T* __restrict__ mask,
                                               const float* __restrict__ lse, const float* __restrict__ delta,
                                               T* __restrict__ dq, const AttnDims& a, float scale) {
-  constexpr int BM = 128 * MQ, BN = 64, KS = DP / 16, DT = DP / 32 / DSPLIT, DT0 = DPART * DT;
-  static_assert((DP / 32) % DSPLIT == 0 && DPART < DSPLIT, "parts of the head dimension");
+  constexpr int BM = 128 * MQ, BN = 64, KS = DC / 16, DT = DC / 32 / DSPLIT, DT0 = DPART * DT;
+  static_assert((DC / 32) % DSPLIT == 0 && DPART < DSPLIT, "parts of the head dimension");
   // Two copies of each staged tile (step i computes from copy i % 2 while the tile of step
   // i + 1 is written into the other: one barrier per step) for head dims up to 64.  Above,
   // one copy and two barriers per step: the two-copy schedule spills more there (68-108 bytes
@@ -744,7 +748,7 @@ constexpr int dkdv_long_step() { return DP <= 64 ? 128 : 64; }
 // The work of workgroup `block` of a dK/dV launch, BQ queries per step; `smem` holds
 // dkdv_lds_bytes<DP, BQ>() bytes.
 // DSPLIT, DPART: as for attn_dq_block, for dK and dV.
-template <typename T, int DP, int BQ, bool CAUSAL, bool HAS_BIAS, int DSPLIT = 1, int DPART = 0>
+template <typename T, int DP, int BQ, bool CAUSAL, bool HAS_BIAS, int DC = DP, int DSPLIT = 1, int DPART = 0>
 __device__ __forceinline__ void attn_dkdv_block(const int block, char* smem, const T* __restrict__ d_o,
                                                 const T* __restrict__ q, const T* __restrict__ k,
                                                 const T* __restrict__ v, const T* __restrict__ mask,
@@ -752,8 +756,8 @@ __device__ __forceinline__ void attn_dkdv_block(const int block, char* smem, con
                                                 T* __restrict__ dk, T* __restrict__ dv, const AttnDims& a,
                                                 float scale) {
   constexpr int BNK = 128;                 // keys per workgroup
-  constexpr int MT = BQ / 32, KS = DP / 16, DT = DP / 32 / DSPLIT, DT0 = DPART * DT;
-  static_assert((DP / 32) % DSPLIT == 0 && DPART < DSPLIT, "parts of the head dimension");
+  constexpr int MT = BQ / 32, KS = DC / 16, DT = DC / 32 / DSPLIT, DT0 = DPART * DT;
+  static_assert((DC / 32) % DSPLIT == 0 && DPART < DSPLIT, "parts of the head dimension");
   // Two copies of every staged tile: step i computes from copy i % 2 while the tile of step
   // i + 1 is written into the other, so one barrier per step suffices.
   constexpr int ROWS = BQ * tile_row_bytes<DP>();
@@ -1912,7 +1916,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
   }
 }
 
-template <typename T, int DP, int MQ, bool CAUSAL, bool HAS_BIAS>
+template <typename T, int DP, int MQ, bool CAUSAL, bool HAS_BIAS, int DC>
 __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_dq_mfma_kernel(const T* __restrict__ d_o, const T* __restrict__ q,
                                                                        const T* __restrict__ k, const T* __restrict__ v,
                                                                        const T* __restrict__ mask,
@@ -1921,14 +1925,14 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_dq_mfma_
                                                                        T* __restrict__ dq, AttnDims a, float scale) {
   __shared__ __attribute__((aligned(16))) char smem[dq_lds_bytes<DP>()];
   if constexpr (DP <= 128) {
-    attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS>(blockIdx.x, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
+    attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS, DC>(blockIdx.x, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
   } else {
     // wider heads: each half of the head dimension of a query block is a workgroup of its own
     const int block = blockIdx.x / kAttnWideSplit;
     if (blockIdx.x % kAttnWideSplit == 0)
-      attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS, kAttnWideSplit, 0>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
+      attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS, DC, kAttnWideSplit, 0>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
     else
-      attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS, kAttnWideSplit, 1>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
+      attn_dq_block<T, DP, MQ, CAUSAL, HAS_BIAS, DC, kAttnWideSplit, 1>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
   }
 }
 
@@ -1952,29 +1956,30 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_dkdv_pipe_kernel(
   attn_dkdv_pipe_block<T, DP, CAUSAL, kAttnStatDpp>(blockIdx.x, smem, d_o, q, k, v, nlse, ndelta, s_pad, dk, dv, a, scale);
 }
 
-template <typename T, int DP, bool CAUSAL, bool HAS_BIAS>
+template <typename T, int DP, bool CAUSAL, bool HAS_BIAS, int DC>
 __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_dkdv_mfma_kernel(
     const T* __restrict__ d_o, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const T* __restrict__ mask, const float* __restrict__ lse, const float* __restrict__ delta, T* __restrict__ dk,
     T* __restrict__ dv, AttnDims a, float scale) {
   __shared__ __attribute__((aligned(16))) char smem[dkdv_lds_bytes<DP, dkdv_long_step<DP>()>()];
   if constexpr (DP <= 128) {
-    attn_dkdv_block<T, DP, dkdv_long_step<DP>(), CAUSAL, HAS_BIAS>(blockIdx.x, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
+    attn_dkdv_block<T, DP, dkdv_long_step<DP>(), CAUSAL, HAS_BIAS, DC>(blockIdx.x, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
   } else {
     const int block = blockIdx.x / kAttnWideSplit;
     if (blockIdx.x % kAttnWideSplit == 0)
-      attn_dkdv_block<T, DP, 32, CAUSAL, HAS_BIAS, kAttnWideSplit, 0>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
+      attn_dkdv_block<T, DP, 32, CAUSAL, HAS_BIAS, DC, kAttnWideSplit, 0>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
     else
-      attn_dkdv_block<T, DP, 32, CAUSAL, HAS_BIAS, kAttnWideSplit, 1>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
+      attn_dkdv_block<T, DP, 32, CAUSAL, HAS_BIAS, DC, kAttnWideSplit, 1>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
   }
 }
 
-// Both walks in one launch (head dims up to 64, where the two have the same occupancy):
+// Both walks in one launch (head dims up to 64, where the two have the same occupancy, and up to 128
+// where there is a CU for every workgroup of either):
 // groups of eight consecutive workgroups alternate between dK/dV and dQ blocks, so every
 // XCD runs both kinds, and short sequences pay for one launch instead of two.  `blocks` is
 // the block count of each walk; the grid is 2 * round_up(blocks, 8) workgroups.
-template <typename T, int DP, bool CAUSAL, bool HAS_BIAS, bool PIPE>
-__global__ __launch_bounds__(kAttnThreads, 2) void attn_bwd_mfma_kernel(
+template <typename T, int DP, bool CAUSAL, bool HAS_BIAS, bool PIPE, int DC>
+__global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_bwd_mfma_kernel(
     const T* __restrict__ d_o, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const T* __restrict__ mask, const float* __restrict__ lse, const float* __restrict__ delta, T* __restrict__ dq,
     T* __restrict__ dk, T* __restrict__ dv, AttnDims a, float scale, int blocks, const float* __restrict__ nlse,
@@ -1988,12 +1993,12 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_bwd_mfma_kernel(
     if constexpr (PIPE)
       attn_dkdv_pipe_block<T, DP, CAUSAL, kAttnStatDpp>(block, smem, d_o, q, k, v, nlse, ndelta, s_pad, dk, dv, a, scale);
     else
-      attn_dkdv_block<T, DP, 64, CAUSAL, HAS_BIAS>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
+      attn_dkdv_block<T, DP, 64, CAUSAL, HAS_BIAS, DC>(block, smem, d_o, q, k, v, mask, lse, delta, dk, dv, a, scale);
   } else {
     if constexpr (PIPE)
       attn_dq_pipe_block<T, DP, CAUSAL>(block, smem, d_o, q, k, v, lse, delta, dq, a, scale);
     else
-      attn_dq_block<T, DP, 1, CAUSAL, HAS_BIAS>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
+      attn_dq_block<T, DP, 1, CAUSAL, HAS_BIAS, DC>(block, smem, d_o, q, k, v, mask, lse, delta, dq, a, scale);
   }
 }
 
@@ -2009,12 +2014,12 @@ bool attn_mfma_supported(int dtype, int64_t D, const void* const* ptrs, int nptr
   return true;
 }
 
-template <typename T, int DP>
+template <typename T, int DP, int DC = DP>
 static int fwd_typed(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse, AttnDims a,
                      float scale, bool causal, bool has_bias, hipStream_t stream) {
   const int64_t blocks = static_cast<int64_t>(a.B) * a.H * ceil_div(a.S, 128);
 #define MG_LAUNCH(C_, B_)                                                                                             \
-  hipLaunchKernelGGL((attn_fwd_mfma_kernel<T, DP, C_, B_>), dim3(static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, \
+  hipLaunchKernelGGL((attn_fwd_mfma_kernel<T, DP, C_, B_, DC>), dim3(static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, \
                      stream, static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),            \
                      static_cast<const T*>(mask), static_cast<T*>(o), lse, a, scale)
   if (causal) MG_LAUNCH(true, false);
@@ -2078,7 +2083,7 @@ static int launch_delta(const T* d_o, const T* o, float* delta, int64_t rows, co
   return MG_OK;
 }
 
-template <typename T, int DP>
+template <typename T, int DP, int DC = DP>
 static int bwd_typed(const void* d_o, const void* o, const void* q, const void* k, const void* v, const void* mask,
                      const float* lse, void* dq, void* dk, void* dv, AttnDims a, float scale, bool causal, bool has_bias,
                      hipStream_t stream) {
@@ -2125,7 +2130,10 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
   // from 1024 on, where the two walks compete for the same CU.  MOGRAD_HIP_ATTN_FUSED_BWD_MAX_S
   // overrides it; 0 always launches dK/dV and dQ separately.
   const int fused_max_s = env_int("MOGRAD_HIP_ATTN_FUSED_BWD_MAX_S", causal ? 2048 : 512);
-  const bool fused = DP <= 64 && a.S <= fused_max_s && 2 * (blocks + 7) < 0x7fffffffLL;
+  // Walks that leave half of the CUs free between them go side by side whatever their length ((29, 29,
+  // 3 heads, 96) 17.8 -> 11.6 us; (2, 1000, 4, 128) 96 -> 53; (1, 3000, 4, 64) 76 -> 47).
+  const bool side_by_side = DP <= 128 && fused_max_s > 0 && 2 * blocks <= device_info().cu_count;
+  const bool fused = side_by_side || (DP <= 64 && a.S <= fused_max_s && 2 * (blocks + 7) < 0x7fffffffLL);
   const T* d_o_ = static_cast<const T*>(d_o);
   const T* q_ = static_cast<const T*>(q);
   const T* k_ = static_cast<const T*>(k);
@@ -2138,19 +2146,19 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
   const dim3 grid_plain(static_cast<unsigned>(blocks * (DP > 128 ? kAttnWideSplit : 1)));
 #define MG_LAUNCH(C_, B_)                                                                                            \
   do {                                                                                                               \
-    if constexpr (DP <= 64) {                                                                                        \
+    if constexpr (DP <= 128) {                                                                                       \
       if (fused) {                                                                                                   \
         if (!B_ && pipe)                                                                                             \
-          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, !B_>), grid_fused, dim3(kAttnThreads), 0, stream,  \
+          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, (!B_ && DP <= 64), DC>), grid_fused, dim3(kAttnThreads), 0, stream,  \
                              d_o_, q_, k_, v_, mask_, lse, delta.as<float>(), dq_, dk_, dv_, a, scale,               \
                              static_cast<int>(blocks), ps.nlse, ps.ndelta, s_pad);                                   \
         else                                                                                                         \
-          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, false>), grid_fused, dim3(kAttnThreads), 0,        \
+          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, false, DC>), grid_fused, dim3(kAttnThreads), 0,        \
                              stream, d_o_, q_, k_, v_, mask_, lse, delta.as<float>(), dq_, dk_, dv_, a, scale,       \
                              static_cast<int>(blocks), ps.nlse, ps.ndelta, s_pad);                                   \
         break;                                                                                                       \
       }                                                                                                              \
-      if constexpr (!B_) {                                                                                           \
+      if constexpr (!B_ && DP <= 64) {                                                                                           \
         if (pipe) {                                                                                                  \
           hipLaunchKernelGGL((attn_dkdv_pipe_kernel<T, DP, C_>), grid, dim3(kAttnThreads), 0, stream, d_o_, q_, k_,  \
                              v_, ps.nlse, ps.ndelta, s_pad, dk_, dv_, a, scale);                                     \
@@ -2160,9 +2168,9 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
         }                                                                                                            \
       }                                                                                                              \
     }                                                                                                                \
-    hipLaunchKernelGGL((attn_dkdv_mfma_kernel<T, DP, C_, B_>), grid_plain, dim3(kAttnThreads), 0, stream, d_o_, q_,  \
+    hipLaunchKernelGGL((attn_dkdv_mfma_kernel<T, DP, C_, B_, DC>), grid_plain, dim3(kAttnThreads), 0, stream, d_o_, q_,  \
                        k_, v_, mask_, lse, delta.as<float>(), dk_, dv_, a, scale);                                   \
-    hipLaunchKernelGGL((attn_dq_mfma_kernel<T, DP, 1, C_, B_>), grid_plain, dim3(kAttnThreads), 0, stream, d_o_, q_, \
+    hipLaunchKernelGGL((attn_dq_mfma_kernel<T, DP, 1, C_, B_, DC>), grid_plain, dim3(kAttnThreads), 0, stream, d_o_, q_, \
                        k_, v_, mask_, lse, delta.as<float>(), dq_, a, scale);                                        \
   } while (0)
   if (causal) MG_LAUNCH(true, false);
@@ -2175,30 +2183,29 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
 
 int attn_fwd_mfma(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse, AttnDims a,
                   float scale, bool causal, bool has_bias, int dtype, hipStream_t stream) {
-  const bool small = a.D <= 64;
-  if (a.D > 128)
-    return dtype == MG_BF16 ? fwd_typed<bf16_t, 256>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream)
-                            : fwd_typed<f16_t, 256>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
-  if (dtype == MG_BF16)
-    return small ? fwd_typed<bf16_t, 64>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream)
-                 : fwd_typed<bf16_t, 128>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
-  return small ? fwd_typed<f16_t, 64>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream)
-               : fwd_typed<f16_t, 128>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+  auto run = [&](auto t) {
+    using T = decltype(t);
+    if (a.D <= 32) return fwd_typed<T, 64, 32>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+    if (a.D <= 64) return fwd_typed<T, 64>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+    if (a.D <= 96) return fwd_typed<T, 128, 96>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+    if (a.D <= 128) return fwd_typed<T, 128>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+    return fwd_typed<T, 256>(q, k, v, mask, o, lse, a, scale, causal, has_bias, stream);
+  };
+  return dtype == MG_BF16 ? run(bf16_t{}) : run(f16_t{});
 }
 
 int attn_bwd_mfma(const void* d_o, const void* o, const void* q, const void* k, const void* v, const void* mask,
                   const float* lse, void* dq, void* dk, void* dv, AttnDims a, float scale, bool causal, bool has_bias,
                   int dtype, hipStream_t stream) {
-  const bool small = a.D <= 64;
-  if (a.D > 128)
-    return dtype == MG_BF16
-               ? bwd_typed<bf16_t, 256>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream)
-               : bwd_typed<f16_t, 256>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
-  if (dtype == MG_BF16)
-    return small ? bwd_typed<bf16_t, 64>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream)
-                 : bwd_typed<bf16_t, 128>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
-  return small ? bwd_typed<f16_t, 64>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream)
-               : bwd_typed<f16_t, 128>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+  auto run = [&](auto t) {
+    using T = decltype(t);
+    if (a.D <= 32) return bwd_typed<T, 64, 32>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+    if (a.D <= 64) return bwd_typed<T, 64>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+    if (a.D <= 96) return bwd_typed<T, 128, 96>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+    if (a.D <= 128) return bwd_typed<T, 128>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+    return bwd_typed<T, 256>(d_o, o, q, k, v, mask, lse, dq, dk, dv, a, scale, causal, has_bias, stream);
+  };
+  return dtype == MG_BF16 ? run(bf16_t{}) : run(f16_t{});
 }
 
 }  // namespace mg
