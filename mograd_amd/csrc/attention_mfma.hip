@@ -2130,9 +2130,12 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
   // from 1024 on, where the two walks compete for the same CU.  MOGRAD_HIP_ATTN_FUSED_BWD_MAX_S
   // overrides it; 0 always launches dK/dV and dQ separately.
   const int fused_max_s = env_int("MOGRAD_HIP_ATTN_FUSED_BWD_MAX_S", causal ? 2048 : 512);
-  // Walks that leave half of the CUs free between them go side by side whatever their length ((29, 29,
-  // 3 heads, 96) 17.8 -> 11.6 us; (2, 1000, 4, 128) 96 -> 53; (1, 3000, 4, 64) 76 -> 47).
-  const bool side_by_side = DP <= 128 && fused_max_s > 0 && 2 * blocks <= device_info().cu_count;
+  // Walks with a CU for every workgroup go side by side whatever their length ((29, 29, 3 heads, 96)
+  // 17.8 -> 11.6 us; (2, 1000, 4, 128) 96 -> 53; (8, 1000, 4, 64) with bias 74 -> 58); above 64 columns,
+  // where a CU holds one of them, equally long ones only when both kinds have their CUs
+  // ((6, 1000, 4, 96), 192 + 192 workgroups: 80 us apart, 89 together).
+  const bool side_by_side = DP <= 128 && fused_max_s > 0 &&
+                            blocks * (DP > 64 && !causal ? 2 : 1) <= device_info().cu_count;
   const bool fused = side_by_side || (DP <= 64 && a.S <= fused_max_s && 2 * (blocks + 7) < 0x7fffffffLL);
   const T* d_o_ = static_cast<const T*>(d_o);
   const T* q_ = static_cast<const T*>(q);
