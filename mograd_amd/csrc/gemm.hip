@@ -612,20 +612,20 @@ static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
 // against 38, (8192, 1152 <- 384) 36 against 32); for 384 columns they can carry the LayerNorm
 // backward, which is 6 us as a launch of its own.
 // MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
-static bool small_linear_bwd(int64_t M, int64_t N, int64_t K, int* splits) {
+static bool small_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx, int* splits) {
   const double cus = device_info().cu_count;
   auto steps_per_cu = [&](int64_t tile) {  // of 64 k
     return static_cast<double>(ceil_div(N, tile) * ceil_div(K, tile) * ceil_div(M, kSmallBK) +
-                               ceil_div(M, tile) * ceil_div(K, tile) * ceil_div(N, kSmallBK)) / cus;
+                               (with_dx ? ceil_div(M, tile) * ceil_div(K, tile) * ceil_div(N, kSmallBK) : 0)) / cus;
   };
   const double steps_w = static_cast<double>(ceil_div(M, kSmallBK)), steps_x = static_cast<double>(ceil_div(N, kSmallBK));
   const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
-  const double tiles_w = steps_x * tiles_k, tiles_x = steps_w * tiles_k;
-  const double load = steps_per_cu(kSmallT);
+  const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0;
+  const double chain_x = with_dx ? steps_x : 0.0, load = steps_per_cu(kSmallT);
   double best = 1e30;
   for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
-    double chain = std::max(steps_w / s, steps_x);
-    if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + steps_x));  // two share a CU
+    double chain = std::max(steps_w / s, chain_x);
+    if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + chain_x));  // two share a CU
     const double t = 3.6 + 0.27 * std::max(1.5 * chain, load) + (s > 1 ? 3.6 + tiles_w * s * 0.0094 : 0.0);
     if (t < best) best = t, *splits = s;
   }
@@ -650,10 +650,11 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   // Widths that are no multiple of 8 (a 65-symbol vocabulary): rows of dY, or of X and W, start
   // at odd addresses, which the copies into LDS cannot take.  Those arrays are first copied to
   // rows of the next multiple of 8, zeros behind (`pads` below); dX, dW and db keep their shape.
-  const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || !aligned16(w);
+  const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || (dx && !aligned16(w));
   const int64_t cus = device_info().cu_count;
   int splits = 1;
-  const bool small = small_linear_bwd(M, N, K, &splits);
+  const bool small = small_linear_bwd(M, N, K, dx != nullptr, &splits);
+  if (!dx && !small) return MG_OK;
   const bool wide = !small && wide_linear_bwd(M, N, K);
   if (ln && (!wide || K != kGemmWideBN || relu_mask || env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3 ||
              pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx)))
@@ -664,7 +665,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const int w_tiles_m = static_cast<int>(ceil_div(N, tile));
   const int64_t w_tiles = static_cast<int64_t>(w_tiles_m) * tiles_kk;
   const int x_tiles_m = static_cast<int>(ceil_div(M, tile));
-  const int64_t x_tiles = static_cast<int64_t>(x_tiles_m) * tiles_kk;
+  const int64_t x_tiles = dx ? static_cast<int64_t>(x_tiles_m) * tiles_kk : 0;  // (a first layer's dX is not wanted)
   if (small) {
   } else if (wide) {
     // Every workgroup step is the same work (a 128 x 384 x 32 product), so the K ranges of dW
@@ -697,7 +698,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   if (pad_n) MG_TRY(pads.add(&dy, 1, M, N, &ldy, &no_batch));
   if (pad_k) {
     MG_TRY(pads.add(&x, 1, M, K, &ldx, &no_batch));
-    MG_TRY(pads.add(&w, 1, N, K, &ldw, &no_batch));
+    if (dx) MG_TRY(pads.add(&w, 1, N, K, &ldw, &no_batch));
   }
   MG_TRY(pads.launch(stream));
 
@@ -817,11 +818,11 @@ static int linear_bwd_f32_one_launch(const void* dy, const void* x, const void* 
   *done = false;
   *db_done = false;
   if (env_int("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", 1) == 0) return MG_OK;
-  if (M <= 0 || N <= 0 || K <= 0 || 4.0 * M * N * K > 1e6 * env_int("MOGRAD_HIP_LINEAR_BWD_F32_MFLOP", 2000)) return MG_OK;
+  if (M <= 0 || N <= 0 || K <= 0 || (dx ? 4.0 : 2.0) * M * N * K > 1e6 * env_int("MOGRAD_HIP_LINEAR_BWD_F32_MFLOP", 2000)) return MG_OK;
   if (M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return MG_OK;
   constexpr int kTile = 32;
   const int64_t tiles_m = ceil_div(M, kTile), tiles_n = ceil_div(N, kTile), tiles_k = ceil_div(K, kTile);
-  const int64_t x_blocks = tiles_m * tiles_k, w_blocks = tiles_n * tiles_k;
+  const int64_t x_blocks = dx ? tiles_m * tiles_k : 0, w_blocks = tiles_n * tiles_k;
   // a large dX with next to no reduction (a 10-class head): see dispatch_f32
   if (N < 32 && x_blocks >= 4 * device_info().cu_count) return MG_OK;
   int splits = static_cast<int>(
@@ -877,6 +878,7 @@ static int linear_bwd_f32_one_launch(const void* dy, const void* x, const void* 
   return MG_OK;
 }
 
+// dx may be null: the gradients of the weights alone.
 // *done: dX and dW are on their way; *db_done: so is db (else the caller sums dY's columns).
 int linear_bwd_products(const void* dy, const void* x, const void* w, void* dx, void* dw, void* db, int64_t M, int64_t N,
                         int64_t K, const void* relu_mask, bool dx_accumulate, int dtype, hipStream_t stream, bool* done,
@@ -941,7 +943,7 @@ static int linear_bwd_impl(const void* dy, const void* x, const void* w, void* d
                            int64_t N, int64_t K, bool dx_accumulate, bool x_is_relu_output, int dtype, mg_stream stream) {
   hipStream_t s = mg::to_stream(stream);
   if (x_is_relu_output && dx && !x) return mg::fail(MG_ERR_INVALID, "linear_bwd: x is needed as the relu mask");
-  if (dx && dw && dy && x && w) {
+  if (dw && dy && x && (w || !dx)) {
     bool done = false, db_done = false;
     MG_TRY(mg::linear_bwd_products(dy, x, w, dx, dw, db, M, N, K, x_is_relu_output ? x : nullptr, dx_accumulate, dtype,
                                    s, &done, &db_done));

@@ -1149,7 +1149,11 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // The rewriting pass (mograd_amd/rewrites.py says what it does; this is its loop)
 // ------------------------------------------------------------------------------------------
 
-bool op_names_equal(PyObject* a, PyObject* b) { return a == b || PyUnicode_Compare(a, b) == 0; }
+bool op_names_equal(PyObject* a, PyObject* b) {
+  if (a == b) return true;
+  if (PyUnicode_CHECK_INTERNED(a) && PyUnicode_CHECK_INTERNED(b)) return false;  // as names written in a program are
+  return PyUnicode_Compare(a, b) == 0;
+}
 
 // Pat.matches
 int pat_matches(PyObject* pat, NodeObj* n) {

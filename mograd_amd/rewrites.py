@@ -280,22 +280,24 @@ def fuse_attention_grad_layout(node: Node, sim: Simplifier) -> Optional[Node]:
     return _refit(node, "FLASH_ATTN_GRAD", [g] + list(node.srcs[1:]), {**node.attrs(), "layout": "bshd"}, sim)
 
 
+_ADD_RULES = [(f, f.__name__) for f in (fuse_matmul_add, fuse_add_into_layer_norm_grad, fuse_add_into_linear_layer_norm_grad,
+                                       fuse_add_into_linear_grad)]
+# Made once: building some thirty patterns took as long as matching them (a classifier's pass 22 -> 12 us).
+_GPU_REWRITES = (
+    Rule(Pat("RELU", [Pat("MATMUL_BIAS_BT")]), fuse_matmul_bias_relu, "fuse_matmul_bias_relu"),
+    Rule(Pat("RELU_GRAD", [Pat(), _get0(Pat("LINEAR_GRAD"))]), fuse_relu_grad_into_linear_grad,
+         "fuse_relu_grad_into_linear_grad"),
+    Rule(Pat("CONTIGUOUS", [Pat("TRANSPOSE", [_get0(Pat("FLASH_ATTN"))])]), fuse_attention_output_layout,
+         "fuse_attention_output_layout"),
+    Rule(Pat("FLASH_ATTN_GRAD"), fuse_attention_grad_layout, "fuse_attention_grad_layout"),
+    Rule(Pat("LAYER_NORM_STATS_GRAD", [_get0(Pat("LINEAR_GRAD"))]), fuse_linear_grad_into_layer_norm_grad,
+         "fuse_linear_grad_into_layer_norm_grad"),
+    Rule(Pat("LAYER_NORM_STATS_GRAD_ADD", [_get0(Pat("LINEAR_GRAD"))]), fuse_linear_grad_into_layer_norm_grad,
+         "fuse_linear_grad_into_layer_norm_grad"),
+    *(Rule(Pat("ADD"), func, name) for func, name in _ADD_RULES),
+)
+
+
 def GPU_REWRITES() -> List[Rule]:
     """The fusions of a transformer training step, in matching priority."""
-    get0 = lambda op: _get0(Pat(op))
-    return [
-        Rule(Pat("RELU", [Pat("MATMUL_BIAS_BT")]), fuse_matmul_bias_relu, "fuse_matmul_bias_relu"),
-        Rule(Pat("RELU_GRAD", [Pat(), get0("LINEAR_GRAD")]), fuse_relu_grad_into_linear_grad,
-             "fuse_relu_grad_into_linear_grad"),
-        Rule(Pat("CONTIGUOUS", [Pat("TRANSPOSE", [get0("FLASH_ATTN")])]), fuse_attention_output_layout,
-             "fuse_attention_output_layout"),
-        Rule(Pat("FLASH_ATTN_GRAD"), fuse_attention_grad_layout, "fuse_attention_grad_layout"),
-        Rule(Pat("LAYER_NORM_STATS_GRAD", [get0("LINEAR_GRAD")]), fuse_linear_grad_into_layer_norm_grad,
-             "fuse_linear_grad_into_layer_norm_grad"),
-        Rule(Pat("LAYER_NORM_STATS_GRAD_ADD", [get0("LINEAR_GRAD")]), fuse_linear_grad_into_layer_norm_grad,
-             "fuse_linear_grad_into_layer_norm_grad"),
-        Rule(Pat("ADD"), fuse_matmul_add, "fuse_matmul_add"),
-        Rule(Pat("ADD"), fuse_add_into_layer_norm_grad, "fuse_add_into_layer_norm_grad"),
-        Rule(Pat("ADD"), fuse_add_into_linear_layer_norm_grad, "fuse_add_into_linear_layer_norm_grad"),
-        Rule(Pat("ADD"), fuse_add_into_linear_grad, "fuse_add_into_linear_grad"),
-    ]
+    return list(_GPU_REWRITES)

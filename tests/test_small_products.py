@@ -96,3 +96,17 @@ def test_tiles_of_64(device, dtype, M, N, K):
                                      (db.to_numpy(), dy.sum(axis=0), g, "db")):
             assert_close(got, want, tol, tol * np.abs(want).max(), f"{name} {grad}")
     lib.mg_deferred_destroy(pending)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("M,N,K", [(3, 5, 7), (64, 256, 784), (700, 33, 40), (1040, 72, 200)])
+def test_weight_gradients_alone(device, dtype, M, N, K):
+    lib, st, rt = device.lib, device.stream, RT[dtype]
+    x = round_to_dtype(normal(63, 0, (M, K)), dtype)
+    dy = round_to_dtype(normal(63, 1, (M, N), std=0.5), dtype)
+    bx, bdy = AnyBuffer.from_numpy(device, x, dtype), AnyBuffer.from_numpy(device, dy, dtype)
+    dw, db = AnyBuffer.create(dtype, device, N * K), AnyBuffer.create(dtype, device, N)
+    lib.mg_linear_bwd_fused(bdy.data_ptr(), bx.data_ptr(), None, None, dw.data_ptr(), db.data_ptr(), M, N, K, 0, 0, dtype, st)
+    x, dy = x.astype(np.float64), dy.astype(np.float64)
+    assert_close(dw.to_numpy((N, K)), dy.T @ x, rt, rt * np.abs(dy.T @ x).max(), "dw")
+    assert_close(db.to_numpy(), dy.sum(axis=0), rt, rt * np.abs(dy.sum(axis=0)).max(), "db")
