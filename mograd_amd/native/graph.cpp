@@ -41,6 +41,10 @@ struct Ref {  // owned reference
   Ref(const Ref&) = delete;
   Ref& operator=(const Ref&) = delete;
   ~Ref() { Py_XDECREF(p); }
+  static Ref to(PyObject* o) {  // a further reference to `o`
+    Py_XINCREF(o);
+    return Ref(o);
+  }
   PyObject* release() {
     PyObject* o = p;
     p = nullptr;
@@ -344,7 +348,7 @@ struct NodeObj {
   PyObject* node_attrs;  // dict
   PyObject* bufs;        // list or None
   uint64_t mark;         // the last walk that saw this node
-  uint32_t used;         // evaluate(): which outputs of a multi-output node are read
+  uint32_t position;     // its place in that walk (between steps that keep the interpreter lock)
 };
 PyTypeObject NodeType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 uint64_t g_epoch = 0;
@@ -365,7 +369,7 @@ PyObject* node_make(PyObject* op, PyObject* layout, PyObject* dtype, PyObject* s
   n->op_type = op, n->node_layout = layout, n->node_dtype = dtype, n->bufs = bufs;
   n->srcs = s.release();
   n->node_attrs = a.release();
-  n->mark = 0, n->used = 0;
+  n->mark = 0, n->position = 0;
   return reinterpret_cast<PyObject*>(n);
 }
 
@@ -472,8 +476,7 @@ bool node_ok(PyObject* o) {
 }
 
 // Sources before consumers, each node once, in the order of a depth-first walk over srcs.
-// Borrowed references: the graph keeps them.
-bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<NodeObj*>& order) {
+bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<Ref>& order) {
   const uint64_t epoch = ++g_epoch;
   std::vector<std::pair<NodeObj*, Py_ssize_t>> stack;
   for (Py_ssize_t r = 0; r < n_roots; ++r) {
@@ -493,7 +496,7 @@ bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<NodeObj*>&
           stack.emplace_back(as_node(c), 0);
         }
       } else {
-        order.push_back(n);
+        order.push_back(Ref::to(reinterpret_cast<PyObject*>(n)));
         stack.pop_back();
       }
     }
@@ -502,14 +505,11 @@ bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<NodeObj*>&
 }
 
 PyObject* py_toposort(PyObject*, PyObject* root) {
-  std::vector<NodeObj*> order;
+  std::vector<Ref> order;
   if (!toposort(&root, 1, order)) return nullptr;
   PyObject* list = PyList_New(static_cast<Py_ssize_t>(order.size()));
   if (!list) return nullptr;
-  for (size_t i = 0; i < order.size(); ++i) {
-    Py_INCREF(order[i]);
-    PyList_SET_ITEM(list, static_cast<Py_ssize_t>(i), reinterpret_cast<PyObject*>(order[i]));
-  }
+  for (size_t i = 0; i < order.size(); ++i) PyList_SET_ITEM(list, static_cast<Py_ssize_t>(i), order[i].release());
   return list;
 }
 
@@ -662,18 +662,39 @@ PyMethodDef buffer_methods[] = {{"data_ptr", FAST(buffer_data_ptr), METH_FASTCAL
 // Evaluation
 // ------------------------------------------------------------------------------------------
 
-// One node's execution: its operands, and what the library needs of the device.
+// One node's execution: its operands, and what the library needs of the device.  The library is called
+// without the interpreter lock, and another thread may evaluate the same nodes meanwhile and
+// replace their buffers: the operands are held here, and their addresses taken, before the call.
 struct Exec {
-  NodeObj* n;
-  PyObject* device;
-  void* stream;
-  void* pending;  // the deferred list in use, or null
-  int dtype;
-  BufferObj* in[12];
-  LayoutObj* lay[12];  // of the sources
-  int count;
+  static constexpr int kMost = 12;  // operands
+  struct Operand {
+    Ref buffer, layout;
+    void* p = nullptr;
+    int dtype = 0;
+  };
+  Ref attrs, layout;  // the node's own
+  PyObject* device = nullptr;
+  void* stream = nullptr;
+  void* pending = nullptr;  // the deferred list in use, or null
+  int dtype = 0;
+  uint32_t used = ~0u;  // which results are read
+  Operand in[kMost];
+  LayoutObj* lay[kMost];  // of the sources
+  int count = 0;
 
-  void* p(int i) const { return address(in[i]); }
+  // Whether the next operand is one of the package's own buffers under one of its layouts (and taken).
+  bool add(Ref buffer, PyObject* layout_of) {
+    if (!PyObject_TypeCheck(buffer.p, &BufferType) || !is_layout(layout_of)) return false;
+    Operand& o = in[count];
+    o.p = address(as_buffer(buffer.p));
+    o.dtype = as_buffer(buffer.p)->dtype;
+    o.buffer = std::move(buffer);
+    o.layout = Ref::to(layout_of);
+    lay[count++] = as_layout(layout_of);
+    return true;
+  }
+  const LayoutObj* out() const { return as_layout(layout.p); }
+  void* p(int i) const { return in[i].p; }
   // The first k operands are contiguous and start on the 16-byte boundary the flat kernels read from.
   bool flat(int k) const {
     if (count < k) return false;
@@ -688,11 +709,11 @@ struct Exec {
     return true;
   }
   bool truth(PyObject* key, bool fallback) const {
-    PyObject* v = PyDict_GetItem(n->node_attrs, key);
+    PyObject* v = PyDict_GetItem(attrs.p, key);
     return v ? PyObject_IsTrue(v) == 1 : fallback;
   }
   double number(PyObject* key) const {
-    PyObject* v = PyDict_GetItem(n->node_attrs, key);
+    PyObject* v = PyDict_GetItem(attrs.p, key);
     return v ? PyFloat_AsDouble(v) : 0.0;
   }
   PyObject* buffer(int dt, long long numel) const {
@@ -703,7 +724,7 @@ struct Exec {
 // New buffers for a node's results; release() hands them over as a list.
 struct Results {
   Ref list;
-  std::vector<BufferObj*> b;
+  std::vector<void*> at;
   const Exec& x;
   bool ok = true;
   explicit Results(const Exec& e) : list(PyList_New(0)), x(e) {}
@@ -711,10 +732,10 @@ struct Results {
     if (!ok || !list) return;
     Ref o(x.buffer(dt, numel));
     ok = o && PyList_Append(list.p, o.p) == 0;
-    if (ok) b.push_back(as_buffer(o.p));
+    if (ok) at.push_back(address(as_buffer(o.p)));
   }
-  void add_none() { ok = ok && list && PyList_Append(list.p, Py_None) == 0, b.push_back(nullptr); }
-  void* p(int i) const { return b[i] ? address(b[i]) : nullptr; }
+  void add_none() { ok = ok && list && PyList_Append(list.p, Py_None) == 0, at.push_back(nullptr); }
+  void* p(int i) const { return at[i]; }
 };
 
 struct GemmDims {
@@ -722,7 +743,7 @@ struct GemmDims {
 };
 // A (.., M, K) by B (.., N, K); false: batch dimensions that do not collapse, left to the Python form.
 bool gemm_dims(const Exec& x, GemmDims* g) {
-  const LayoutObj *la = x.lay[0], *lb = x.lay[1], *lo = as_layout(x.n->node_layout);
+  const LayoutObj *la = x.lay[0], *lb = x.lay[1], *lo = x.out();
   for (const LayoutObj* l : {la, lb})
     for (Py_ssize_t i = rank_of(l) - 4; i >= 0; --i)
       if (stride_of(l, i) != dim_of(l, i + 1) * stride_of(l, i + 1)) return false;
@@ -748,7 +769,7 @@ int finish(Results& r, int rc, PyObject** out) {
 }
 #define MG_RUN(call) finish(r, unlocked([&] { return call; }), out)
 
-long long out_numel(const Exec& x) { return as_layout(x.n->node_layout)->numel; }
+long long out_numel(const Exec& x) { return x.out()->numel; }
 
 int run_matmul_bt(const Exec& x, PyObject** out) {
   GemmDims g;
@@ -779,7 +800,7 @@ int run_linear_grad(const Exec& x, PyObject** out) {
   const long long m = x.lay[1]->numel / k;
   Results r(x);
   // dX that nobody reads (the first layer's input is data) is not computed.
-  const bool want_dx = x.n->used & 1u;
+  const bool want_dx = x.used & 1u;
   if (want_dx) r.add(x.dtype, m * k);
   else r.add_none();
   r.add(x.dtype, n * k);
@@ -886,18 +907,18 @@ int run_gather(const Exec& x, PyObject** out) {
   r.add(x.dtype, out_numel(x));
   if (!r.ok) return -1;
   return MG_RUN(L.mg_gather(x.p(0), x.p(1), r.p(0), x.lay[1]->numel, dim_of(x.lay[0], 0), dim_of(x.lay[0], 1),
-                            stride_of(x.lay[0], 0), stride_of(x.lay[0], 1), x.in[1]->dtype, x.dtype, x.stream));
+                            stride_of(x.lay[0], 0), stride_of(x.lay[0], 1), x.in[1].dtype, x.dtype, x.stream));
 }
 int run_scatter_add(const Exec& x, PyObject** out) {
-  const LayoutObj* lo = as_layout(x.n->node_layout);
+  const LayoutObj* lo = x.out();
   if (!x.contiguous(2) || rank_of(x.lay[1]) != rank_of(x.lay[0]) + 1) return 0;
   Results r(x);
   r.add(x.dtype, lo->numel);
   if (!r.ok) return -1;
   const long long n_idx = x.lay[0]->numel, rows = dim_of(lo, 0), row_size = dim_of(x.lay[1], -1);
-  return MG_RUN(x.pending ? L.mg_scatter_add_deferred(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0]->dtype, x.dtype,
+  return MG_RUN(x.pending ? L.mg_scatter_add_deferred(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0].dtype, x.dtype,
                                                       x.dtype, x.pending, x.stream)
-                          : L.mg_scatter_add(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0]->dtype, x.dtype, x.stream));
+                          : L.mg_scatter_add(x.p(0), x.p(1), r.p(0), n_idx, rows, row_size, x.in[0].dtype, x.dtype, x.stream));
 }
 int run_attn_packed(const Exec& x, PyObject** out) {
   const LayoutObj* q = x.lay[0];
@@ -932,7 +953,7 @@ int run_ce_ids(const Exec& x, PyObject** out) {
   Results r(x);
   r.add(x.dtype, out_numel(x));
   if (!r.ok) return -1;
-  return MG_RUN(L.mg_cross_entropy_ids(x.p(0), x.p(1), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1]->dtype, x.stream));
+  return MG_RUN(L.mg_cross_entropy_ids(x.p(0), x.p(1), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1].dtype, x.stream));
 }
 int run_ce_grad_ids(const Exec& x, PyObject** out) {
   if (!x.contiguous(2) || x.count < 3 || !is_float(x.dtype)) return 0;
@@ -941,15 +962,16 @@ int run_ce_grad_ids(const Exec& x, PyObject** out) {
   Results r(x);
   r.add(x.dtype, out_numel(x));
   if (!r.ok) return -1;
-  return MG_RUN(L.mg_cross_entropy_grad_ids(x.p(0), x.p(1), x.p(2), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1]->dtype,
+  return MG_RUN(L.mg_cross_entropy_grad_ids(x.p(0), x.p(1), x.p(2), r.p(0), x.lay[0]->numel / c, c, x.dtype, x.in[1].dtype,
                                             x.stream));
 }
 int run_reshape(const Exec& x, PyObject** out) {
   if (!x.contiguous(1)) return 0;
   Ref list(PyList_New(1));
   if (!list) return -1;
-  Py_INCREF(x.in[0]->storage);
-  PyObject* v = buffer_make(g_buffer_type, x.in[0]->storage, x.in[0]->dtype, out_numel(x), x.in[0]->offset_elems);
+  const BufferObj* b = as_buffer(x.in[0].buffer.p);
+  Py_INCREF(b->storage);
+  PyObject* v = buffer_make(g_buffer_type, b->storage, b->dtype, out_numel(x), b->offset_elems);
   if (!v) return -1;
   PyList_SET_ITEM(list.p, 0, v);
   *out = list.release();
@@ -979,127 +1001,177 @@ const std::pair<const char*, Form> kForms[] = {
     {"RESHAPE", run_reshape},
 };
 
+// One evaluate() call: the nodes in order, and what the walk knows of each.  Nothing of a walk is kept on
+// the nodes, which other walks (other threads, or an exec function of this one) may visit meanwhile.
 struct Evaluation {
+  struct Vertex {
+    Ref node;
+    uint32_t first = 0, count = 0;  // its sources: positions in the walk, sources[first ...]
+    uint32_t used = 0;              // which results of a multi-output node are read
+  };
+  std::vector<Vertex> walk;
+  std::vector<uint32_t> sources;
+  std::vector<uint32_t> ce_grads;  // CROSS_ENTROPY_IDS_GRAD nodes
+
   PyObject* device;
   PyObject* run;  // runtime.run(node, inputs, device): the Python exec function of a node
   void* stream = nullptr;
   void* pending = nullptr;
-  PyObject *kBuffer, *kGetTuple;
+  PyObject *kBuffer, *kGetTuple, *kCeIds, *kCeIdsGrad;
 
-  bool op_is(const NodeObj* n, PyObject* name) const {
+  NodeObj* node(uint32_t at) const { return as_node(walk[at].node.p); }
+  uint32_t source(uint32_t at, uint32_t i) const { return sources[walk[at].first + i]; }
+  static bool op_is(const NodeObj* n, PyObject* name) {
     return n->op_type == name || PyUnicode_Compare(n->op_type, name) == 0;
   }
-  static bool have(const NodeObj* n) { return n->bufs != Py_None; }
-  // Result i of an evaluated node (borrowed); one that was left out when the node first ran,
-  // because nobody read it then, is made now.
-  PyObject* result(NodeObj* s, Py_ssize_t i) {
-    if (!PyList_Check(s->bufs) || i < 0 || i >= PyList_GET_SIZE(s->bufs))
-      return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), nullptr;
-    if (PyList_GET_ITEM(s->bufs, i) == Py_None) {
-      s->used = ~0u;
-      if (!execute(s)) return nullptr;
+  bool have(uint32_t at) const { return node(at)->bufs != Py_None; }
+
+  bool build(PyObject* const* roots, Py_ssize_t n_roots) {
+    std::vector<Ref> order;
+    if (!toposort(roots, n_roots, order)) return false;
+    walk.resize(order.size());
+    for (uint32_t i = 0; i < walk.size(); ++i) {
+      walk[i].node = std::move(order[i]);
+      node(i)->position = i;
     }
-    return PyList_GET_ITEM(s->bufs, i);
-  }
-  bool set(NodeObj* n, PyObject* list) {  // takes over `list`
-    if (!list) return false;
-    Py_SETREF(n->bufs, list);
+    for (uint32_t i = 0; i < walk.size(); ++i) {  // (no Python code since toposort: the positions are ours)
+      PyObject* srcs = node(i)->srcs;
+      walk[i].first = static_cast<uint32_t>(sources.size());
+      walk[i].count = static_cast<uint32_t>(PyList_GET_SIZE(srcs));
+      for (uint32_t k = 0; k < walk[i].count; ++k) {
+        const uint32_t at = as_node(PyList_GET_ITEM(srcs, k))->position;
+        if (at >= i) return raise_invalid("evaluate: the graph has a cycle"), false;
+        sources.push_back(at);
+      }
+    }
+    for (uint32_t i = 0; i < walk.size(); ++i) {
+      if (op_is(node(i), kCeIdsGrad)) ce_grads.push_back(i);
+      uint32_t bit = 1u;  // a node read directly gives its first result
+      if (op_is(node(i), kGetTuple)) {
+        PyObject* index = PyDict_GetItem(node(i)->node_attrs, N.index);
+        const long at = index ? PyLong_AsLong(index) : 0;
+        bit = at >= 0 && at < 31 ? 1u << at : ~0u;
+      }
+      for (uint32_t k = 0; k < walk[i].count; ++k) walk[source(i, k)].used |= bit;
+    }
+    for (Py_ssize_t i = 0; i < n_roots; ++i) walk[as_node(roots[i])->position].used = ~0u;
     return true;
   }
 
-  bool execute(NodeObj* n) {
-    const Py_ssize_t count = PyList_GET_SIZE(n->srcs);
+  // Result i of an evaluated node; one that was left out when the node first ran, because nobody
+  // read it then, is made now.
+  Ref result(uint32_t at, Py_ssize_t i) {
+    Ref list = Ref::to(node(at)->bufs);
+    if (!PyList_Check(list.p) || i < 0 || i >= PyList_GET_SIZE(list.p))
+      return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
+    if (PyList_GET_ITEM(list.p, i) == Py_None) {
+      walk[at].used = ~0u;
+      list = execute(at);
+      if (!list) return Ref();
+      if (!PyList_Check(list.p) || i >= PyList_GET_SIZE(list.p))
+        return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
+    }
+    return Ref::to(PyList_GET_ITEM(list.p, i));
+  }
+  static bool set(NodeObj* n, Ref list) {
+    if (!list) return false;
+    Py_SETREF(n->bufs, list.release());
+    return true;
+  }
+
+  // Runs a node whose sources have their results and gives it its own, which are returned as well.
+  Ref execute(uint32_t at) {
+    NodeObj* n = node(at);
+    const uint32_t count = walk[at].count;
     PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
-    if (idx && count <= 12 && is_layout(n->node_layout) && PyLong_Check(n->node_dtype)) {
+    if (idx && count <= Exec::kMost && is_layout(n->node_layout) && PyLong_Check(n->node_dtype)) {
       Exec x;
-      x.n = n, x.device = device, x.stream = stream, x.pending = pending;
+      x.attrs = Ref::to(n->node_attrs), x.layout = Ref::to(n->node_layout);
+      x.device = device, x.stream = stream, x.pending = pending, x.used = walk[at].used;
       x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
-      x.count = static_cast<int>(count);
       bool plain = true;
-      for (int i = 0; i < x.count && plain; ++i) {
-        NodeObj* s = as_node(PyList_GET_ITEM(n->srcs, i));
-        PyObject* b = result(s, 0);
-        if (!b) return false;
-        plain = PyObject_TypeCheck(b, &BufferType) && is_layout(s->node_layout);
-        x.in[i] = as_buffer(b);
-        x.lay[i] = as_layout(s->node_layout);
+      for (uint32_t i = 0; i < count && plain; ++i) {
+        Ref b = result(source(at, i), 0);
+        if (!b) return Ref();
+        plain = x.add(std::move(b), node(source(at, i))->node_layout);
       }
       if (plain) {
         PyObject* out = nullptr;
         const int rc = kForms[PyLong_AsLong(idx)].second(x, &out);
-        if (rc < 0) return false;
-        if (rc > 0) return set(n, out);
+        if (rc < 0) return Ref();
+        if (rc > 0) {
+          Ref list(out);
+          return set(n, Ref::to(out)) ? std::move(list) : Ref();
+        }
       }
     }
     Ref inputs(PyList_New(count));
-    if (!inputs) return false;
-    for (Py_ssize_t i = 0; i < count; ++i) {
-      PyObject* b = result(as_node(PyList_GET_ITEM(n->srcs, i)), 0);
-      if (!b) return false;
-      Py_INCREF(b);
-      PyList_SET_ITEM(inputs.p, i, b);
+    if (!inputs) return Ref();
+    for (uint32_t i = 0; i < count; ++i) {
+      Ref b = result(source(at, i), 0);
+      if (!b) return Ref();
+      PyList_SET_ITEM(inputs.p, i, b.release());
     }
-    return set(n, PyObject_CallFunctionObjArgs(run, n, inputs.p, device, nullptr));
+    Ref list(PyObject_CallFunctionObjArgs(run, n, inputs.p, device, nullptr));
+    if (list) set(n, Ref::to(list.p));
+    return list;
   }
 
   // CROSS_ENTROPY_IDS[logits, ids] and the CROSS_ENTROPY_IDS_GRAD of the same operands in this walk: loss
   // and dlogits in one pass over the logits, when the gradient's upstream is already there (it is the
   // graph's root).  1 done, 0 not such a pair, -1 error.
-  std::vector<NodeObj*> ce_grads;
-  PyObject *kCeIds, *kCeIdsGrad;
-  int cross_entropy_pair(NodeObj* n) {
-    NodeObj* g = nullptr;
-    for (NodeObj* c : ce_grads)
-      if (!have(c) && PyList_GET_SIZE(c->srcs) == 3 && PyList_GET_SIZE(n->srcs) == 2 &&
-          PyList_GET_ITEM(c->srcs, 0) == PyList_GET_ITEM(n->srcs, 0) &&
-          PyList_GET_ITEM(c->srcs, 1) == PyList_GET_ITEM(n->srcs, 1) && have(as_node(PyList_GET_ITEM(c->srcs, 2))))
-        g = c;
-    if (!g || !is_layout(n->node_layout) || !is_layout(g->node_layout)) return 0;
-    BufferObj* b[3];
-    for (int i = 0; i < 3; ++i) {
-      NodeObj* s = as_node(PyList_GET_ITEM(g->srcs, i));
-      PyObject* r = result(s, 0);
-      if (!r) return -1;
-      if (!PyObject_TypeCheck(r, &BufferType) || !is_layout(s->node_layout) || !as_layout(s->node_layout)->contiguous) return 0;
-      b[i] = as_buffer(r);
-    }
-    const LayoutObj* logits = as_layout(as_node(PyList_GET_ITEM(g->srcs, 0))->node_layout);
-    const int dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
-    const long long c = rank_of(logits) ? dim_of(logits, -1) : 0;
-    if (c == 0 || !is_float(dtype) || static_cast<int>(PyLong_AsLong(g->node_dtype)) != dtype) return 0;
+  int cross_entropy_pair(uint32_t at) {
+    if (walk[at].count != 2) return 0;
+    uint32_t pair = at;
+    for (uint32_t c : ce_grads)
+      if (!have(c) && walk[c].count == 3 && source(c, 0) == source(at, 0) && source(c, 1) == source(at, 1) &&
+          have(source(c, 2)))
+        pair = c;
+    NodeObj *n = node(at), *g = node(pair);
+    if (pair == at || !is_layout(n->node_layout) || !is_layout(g->node_layout)) return 0;
     Exec x;
-    x.device = device, x.dtype = dtype;
+    x.layout = Ref::to(n->node_layout);
+    Ref grad_layout = Ref::to(g->node_layout);
+    x.device = device, x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
+    if (static_cast<int>(PyLong_AsLong(g->node_dtype)) != x.dtype || !is_float(x.dtype)) return 0;
+    for (uint32_t i = 0; i < 3; ++i) {
+      Ref b = result(source(pair, i), 0);
+      if (!b) return -1;
+      if (!x.add(std::move(b), node(source(pair, i))->node_layout)) return 0;
+    }
+    if (!x.contiguous(3) || rank_of(x.lay[0]) == 0) return 0;
+    const long long c = dim_of(x.lay[0], -1);
+    if (c == 0) return 0;
     Results loss(x), grad(x);
-    loss.add(dtype, as_layout(n->node_layout)->numel);
-    grad.add(dtype, as_layout(g->node_layout)->numel);
+    loss.add(x.dtype, out_numel(x));
+    grad.add(x.dtype, as_layout(grad_layout.p)->numel);
     if (!loss.ok || !grad.ok) return -1;
     const int rc = unlocked([&] {
-      return L.mg_cross_entropy_fused_ids(address(b[0]), address(b[1]), address(b[2]), loss.p(0), grad.p(0),
-                                          logits->numel / c, c, dtype, b[1]->dtype, stream);
+      return L.mg_cross_entropy_fused_ids(x.p(0), x.p(1), x.p(2), loss.p(0), grad.p(0), x.lay[0]->numel / c, c, x.dtype,
+                                          x.in[1].dtype, stream);
     });
     if (rc != 0) return raise_status(rc), -1;
-    return set(n, loss.list.release()) && set(g, grad.list.release()) ? 1 : -1;
+    return set(n, std::move(loss.list)) && set(g, std::move(grad.list)) ? 1 : -1;
   }
 
-  bool evaluate(NodeObj* n) {
-    if (have(n)) return true;
+  bool evaluate(uint32_t at) {
+    if (have(at)) return true;
+    NodeObj* n = node(at);
     if (!ce_grads.empty() && op_is(n, kCeIds)) {
-      const int rc = cross_entropy_pair(n);
+      const int rc = cross_entropy_pair(at);
       if (rc != 0) return rc > 0;
     }
     if (op_is(n, kBuffer)) return raise_invalid("evaluate: a leaf node without a buffer"), false;
-    if (!op_is(n, kGetTuple)) return execute(n);
-    if (PyList_GET_SIZE(n->srcs) != 1) return raise_invalid("GETTUPLE takes one source"), false;
-    NodeObj* s = as_node(PyList_GET_ITEM(n->srcs, 0));
+    if (!op_is(n, kGetTuple)) return static_cast<bool>(execute(at));
+    if (walk[at].count != 1) return raise_invalid("GETTUPLE takes one source"), false;
     PyObject* index = PyDict_GetItem(n->node_attrs, N.index);
     const Py_ssize_t i = index ? PyLong_AsSsize_t(index) : 0;
     if (i == -1 && PyErr_Occurred()) return false;
-    PyObject* b = result(s, i);
-    PyObject* list = b ? PyList_New(1) : nullptr;
+    Ref b = result(source(at, 0), i);
+    Ref list(b ? PyList_New(1) : nullptr);
     if (!list) return false;
-    Py_INCREF(b);
-    PyList_SET_ITEM(list, 0, b);
-    return set(n, list);
+    PyList_SET_ITEM(list.p, 0, b.release());
+    return set(n, std::move(list));
   }
 };
 
@@ -1107,7 +1179,7 @@ struct Evaluation {
 // The sources of a multi-output node's results that nobody in this walk reads may be left out.
 PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 3) return PyErr_SetString(PyExc_TypeError, "evaluate(nodes, device, run)"), nullptr;
-  Ref nodes(PySequence_Fast(args[0], "evaluate: nodes must be a sequence"));
+  Ref nodes(PySequence_Tuple(args[0]));
   if (!nodes) return nullptr;
   Evaluation e;
   e.device = args[1], e.run = args[2];
@@ -1119,29 +1191,9 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!stream || !pending) return nullptr;
   if (!pointer_of(stream.p, &e.stream) || !pointer_of(pending.p, &e.pending))
     return PyErr_SetString(PyExc_TypeError, "evaluate: the device's stream is not a pointer"), nullptr;
-  std::vector<NodeObj*> order;
-  if (!toposort(PySequence_Fast_ITEMS(nodes.p), PySequence_Fast_GET_SIZE(nodes.p), order)) return nullptr;
-  for (NodeObj* v : order) {
-    v->used = 0;
-    if (e.op_is(v, kCeIdsGrad)) e.ce_grads.push_back(v);
-  }
-  for (NodeObj* v : order) {
-    const bool get = e.op_is(v, kGetTuple);
-    const Py_ssize_t srcs = PyList_GET_SIZE(v->srcs);
-    for (Py_ssize_t i = 0; i < srcs; ++i) {
-      uint32_t bit = 1u;  // a node read directly gives its first result
-      if (get) {
-        PyObject* index = PyDict_GetItem(v->node_attrs, N.index);
-        const long at = index ? PyLong_AsLong(index) : 0;
-        bit = at >= 0 && at < 31 ? 1u << at : ~0u;
-      }
-      as_node(PyList_GET_ITEM(v->srcs, i))->used |= bit;
-    }
-  }
-  for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(nodes.p); ++i)
-    as_node(PySequence_Fast_GET_ITEM(nodes.p, i))->used = ~0u;
-  for (NodeObj* v : order)
-    if (!e.evaluate(v)) return nullptr;
+  if (!e.build(PySequence_Fast_ITEMS(nodes.p), PySequence_Fast_GET_SIZE(nodes.p))) return nullptr;
+  for (uint32_t i = 0; i < e.walk.size(); ++i)
+    if (!e.evaluate(i)) return nullptr;
   Py_RETURN_NONE;
 }
 
@@ -1281,9 +1333,9 @@ struct Pass {
 PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (n_args != 2) return PyErr_SetString(PyExc_TypeError, "simplify(sim, roots)"), nullptr;
   PyObject* sim = args[0];
-  Ref roots(PySequence_Fast(args[1], "Simplifier: roots must be a sequence"));
+  Ref roots(PySequence_Tuple(args[1]));
   if (!roots) return nullptr;
-  std::vector<NodeObj*> topo;
+  std::vector<Ref> topo;
   if (!toposort(PySequence_Fast_ITEMS(roots.p), PySequence_Fast_GET_SIZE(roots.p), topo)) return nullptr;
   Ref subst(PyDict_New()), uses(PyDict_New()), origin(PyDict_New()), consumers(PyDict_New());
   if (!subst || !uses || !origin || !consumers || PyObject_SetAttr(sim, N.subst, subst.p) != 0 ||
@@ -1291,16 +1343,16 @@ PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       PyObject_SetAttr(sim, N.consumers, consumers.p) != 0)
     return nullptr;
   Pass pass{sim, subst.p, uses.p, origin.p, consumers.p};
-  for (NodeObj* v : topo)
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(v->srcs); ++i) {
-      PyObject* s = PyList_GET_ITEM(v->srcs, i);
+  for (const Ref& v : topo)
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(as_node(v.p)->srcs); ++i) {
+      PyObject* s = PyList_GET_ITEM(as_node(v.p)->srcs, i);
       PyObject* list = PyDict_GetItem(consumers.p, s);
       if (!list) {
         Ref fresh(PyList_New(0));
         if (!fresh || PyDict_SetItem(consumers.p, s, fresh.p) != 0) return nullptr;
         list = PyDict_GetItem(consumers.p, s);
       }
-      if (PyList_Append(list, reinterpret_cast<PyObject*>(v)) != 0) return nullptr;
+      if (PyList_Append(list, v.p) != 0) return nullptr;
     }
   {
     PyObject *k, *v;
@@ -1330,8 +1382,8 @@ PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!c.op) return nullptr;
     compiled.push_back(std::move(c));
   }
-  for (NodeObj* v : topo) {
-    PyObject* node = reinterpret_cast<PyObject*>(v);
+  for (const Ref& v : topo) {
+    PyObject* node = v.p;
     if (PyDict_GetItem(subst.p, node)) continue;  // a rule that ran on another node has already replaced this one
     Ref now(pass.with_subst(node));
     if (!now) return nullptr;
