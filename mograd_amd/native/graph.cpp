@@ -677,7 +677,7 @@ struct Exec {
   void* stream = nullptr;
   void* pending = nullptr;  // the deferred list in use, or null
   int dtype = 0;
-  uint32_t used = ~0u;  // which results are read
+  uint32_t want = ~0u;  // bit i: result i is to be made (a form may make more)
   Operand in[kMost];
   LayoutObj* lay[kMost];  // of the sources
   int count = 0;
@@ -799,18 +799,17 @@ int run_linear_grad(const Exec& x, PyObject** out) {
   if (k == 0 || x.lay[0]->numel != x.lay[1]->numel / k * n) return 0;
   const long long m = x.lay[1]->numel / k;
   Results r(x);
-  // dX that nobody reads (the first layer's input is data) is not computed.
-  const bool want_dx = x.used & 1u;
-  if (want_dx) r.add(x.dtype, m * k);
-  else r.add_none();
-  r.add(x.dtype, n * k);
-  if (has_bias) r.add(x.dtype, n);
+  const long long size[3] = {m * k, n * k, n};
+  for (int i = 0; i < (has_bias ? 3 : 2); ++i) {
+    if (x.want >> i & 1u) r.add(x.dtype, size[i]);
+    else r.add_none();
+  }
   if (!r.ok) return -1;
   void *dx = r.p(0), *dw = r.p(1), *db = has_bias ? r.p(2) : nullptr;
   return MG_RUN([&]() -> int {
     if (accumulate && dx)
       if (int rc = L.mg_copy_device(dx, x.p(3), m * k * dtype_size(x.dtype), x.stream)) return rc;
-    if (x.pending)
+    if (x.pending && dw)
       return L.mg_linear_bwd_deferred(x.p(0), x.p(1), x.p(2), dx, dw, db, m, n, k, accumulate, relu, x.dtype, x.dtype,
                                       x.pending, x.stream);
     return L.mg_linear_bwd_fused(x.p(0), x.p(1), x.p(2), dx, dw, db, m, n, k, accumulate, relu, x.dtype, x.stream);
@@ -1017,7 +1016,7 @@ struct Evaluation {
   PyObject* run;  // runtime.run(node, inputs, device): the Python exec function of a node
   void* stream = nullptr;
   void* pending = nullptr;
-  PyObject *kBuffer, *kGetTuple, *kCeIds, *kCeIdsGrad;
+  PyObject *kBuffer, *kGetTuple, *kCeIds, *kCeIdsGrad, *kLinearGrad;
 
   NodeObj* node(uint32_t at) const { return as_node(walk[at].node.p); }
   uint32_t source(uint32_t at, uint32_t i) const { return sources[walk[at].first + i]; }
@@ -1034,6 +1033,7 @@ struct Evaluation {
       walk[i].node = std::move(order[i]);
       node(i)->position = i;
     }
+    std::vector<Py_ssize_t> readers(walk.size(), 0);
     for (uint32_t i = 0; i < walk.size(); ++i) {  // (no Python code since toposort: the positions are ours)
       PyObject* srcs = node(i)->srcs;
       walk[i].first = static_cast<uint32_t>(sources.size());
@@ -1042,6 +1042,7 @@ struct Evaluation {
         const uint32_t at = as_node(PyList_GET_ITEM(srcs, k))->position;
         if (at >= i) return raise_invalid("evaluate: the graph has a cycle"), false;
         sources.push_back(at);
+        ++readers[at];
       }
     }
     for (uint32_t i = 0; i < walk.size(); ++i) {
@@ -1055,22 +1056,38 @@ struct Evaluation {
       for (uint32_t k = 0; k < walk[i].count; ++k) walk[source(i, k)].used |= bit;
     }
     for (Py_ssize_t i = 0; i < n_roots; ++i) walk[as_node(roots[i])->position].used = ~0u;
+    // A layer's dX that nobody reads (the first layer's input is data) is not computed, unless something
+    // outside the walk holds the node too (a selector of dX that is kept for later): its result is
+    // that of the operands as they are now.
+    for (uint32_t i = 0; i < walk.size(); ++i)
+      if (!op_is(node(i), kLinearGrad) || Py_REFCNT(node(i)) > readers[i] + 1) walk[i].used |= 1u;
     return true;
   }
 
-  // Result i of an evaluated node; one that was left out when the node first ran, because nobody
-  // read it then, is made now.
+  // Whether an evaluated node's dX was left out.
+  bool lacks_dx(uint32_t at) const {
+    PyObject* list = node(at)->bufs;
+    return PyList_Check(list) && PyList_GET_SIZE(list) > 0 && PyList_GET_ITEM(list, 0) == Py_None && op_is(node(at), kLinearGrad);
+  }
+  // Makes it after all; the other results stay the ones they are.
+  Ref complete(uint32_t at) {
+    Ref old = Ref::to(node(at)->bufs), made = make(at, 1u), list;
+    if (!made) return Ref();
+    if (!PyList_Check(made.p) || PyList_GET_SIZE(made.p) != PyList_GET_SIZE(old.p)) list = std::move(made);
+    else list = Ref(PyList_GetSlice(old.p, 0, PyList_GET_SIZE(old.p)));
+    if (list && made) {
+      Ref dx = Ref::to(PyList_GET_ITEM(made.p, 0));
+      PyList_SetItem(list.p, 0, dx.release());
+    }
+    if (list) set(node(at), Ref::to(list.p));
+    return list;
+  }
+  // Result i of an evaluated node.
   Ref result(uint32_t at, Py_ssize_t i) {
-    Ref list = Ref::to(node(at)->bufs);
+    Ref list = i == 0 && lacks_dx(at) ? complete(at) : Ref::to(node(at)->bufs);
+    if (!list) return Ref();
     if (!PyList_Check(list.p) || i < 0 || i >= PyList_GET_SIZE(list.p))
       return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
-    if (PyList_GET_ITEM(list.p, i) == Py_None) {
-      walk[at].used = ~0u;
-      list = execute(at);
-      if (!list) return Ref();
-      if (!PyList_Check(list.p) || i >= PyList_GET_SIZE(list.p))
-        return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
-    }
     return Ref::to(PyList_GET_ITEM(list.p, i));
   }
   static bool set(NodeObj* n, Ref list) {
@@ -1079,15 +1096,15 @@ struct Evaluation {
     return true;
   }
 
-  // Runs a node whose sources have their results and gives it its own, which are returned as well.
-  Ref execute(uint32_t at) {
+  // The results of a node whose sources have theirs; without those that are neither wanted nor made anyway.
+  Ref make(uint32_t at, uint32_t want) {
     NodeObj* n = node(at);
     const uint32_t count = walk[at].count;
     PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
     if (idx && count <= Exec::kMost && is_layout(n->node_layout) && PyLong_Check(n->node_dtype)) {
       Exec x;
       x.attrs = Ref::to(n->node_attrs), x.layout = Ref::to(n->node_layout);
-      x.device = device, x.stream = stream, x.pending = pending, x.used = walk[at].used;
+      x.device = device, x.stream = stream, x.pending = pending, x.want = want;
       x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
       bool plain = true;
       for (uint32_t i = 0; i < count && plain; ++i) {
@@ -1099,10 +1116,7 @@ struct Evaluation {
         PyObject* out = nullptr;
         const int rc = kForms[PyLong_AsLong(idx)].second(x, &out);
         if (rc < 0) return Ref();
-        if (rc > 0) {
-          Ref list(out);
-          return set(n, Ref::to(out)) ? std::move(list) : Ref();
-        }
+        if (rc > 0) return Ref(out);
       }
     }
     Ref inputs(PyList_New(count));
@@ -1112,9 +1126,7 @@ struct Evaluation {
       if (!b) return Ref();
       PyList_SET_ITEM(inputs.p, i, b.release());
     }
-    Ref list(PyObject_CallFunctionObjArgs(run, n, inputs.p, device, nullptr));
-    if (list) set(n, Ref::to(list.p));
-    return list;
+    return Ref(PyObject_CallFunctionObjArgs(run, n, inputs.p, device, nullptr));
   }
 
   // CROSS_ENTROPY_IDS[logits, ids] and the CROSS_ENTROPY_IDS_GRAD of the same operands in this walk: loss
@@ -1155,14 +1167,14 @@ struct Evaluation {
   }
 
   bool evaluate(uint32_t at) {
-    if (have(at)) return true;
+    if (have(at)) return walk[at].used != ~0u || !lacks_dx(at) || complete(at);
     NodeObj* n = node(at);
     if (!ce_grads.empty() && op_is(n, kCeIds)) {
       const int rc = cross_entropy_pair(at);
       if (rc != 0) return rc > 0;
     }
     if (op_is(n, kBuffer)) return raise_invalid("evaluate: a leaf node without a buffer"), false;
-    if (!op_is(n, kGetTuple)) return static_cast<bool>(execute(at));
+    if (!op_is(n, kGetTuple)) return set(n, make(at, walk[at].used | ~1u));
     if (walk[at].count != 1) return raise_invalid("GETTUPLE takes one source"), false;
     PyObject* index = PyDict_GetItem(n->node_attrs, N.index);
     const Py_ssize_t i = index ? PyLong_AsSsize_t(index) : 0;
@@ -1176,7 +1188,6 @@ struct Evaluation {
 };
 
 // evaluate(nodes, device, run): gives every node of `nodes` and of their sources its buffers.
-// The sources of a multi-output node's results that nobody in this walk reads may be left out.
 PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 3) return PyErr_SetString(PyExc_TypeError, "evaluate(nodes, device, run)"), nullptr;
   Ref nodes(PySequence_Tuple(args[0]));
@@ -1187,6 +1198,8 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   e.kBuffer = kBuffer, e.kGetTuple = kGetTuple;
   static PyObject *kCeIds = str_("CROSS_ENTROPY_IDS"), *kCeIdsGrad = str_("CROSS_ENTROPY_IDS_GRAD");
   e.kCeIds = kCeIds, e.kCeIdsGrad = kCeIdsGrad;
+  static PyObject* kLinearGrad = str_("LINEAR_GRAD");
+  e.kLinearGrad = kLinearGrad;
   Ref stream(PyObject_GetAttr(e.device, N.stream)), pending(PyObject_GetAttr(e.device, N.pending));
   if (!stream || !pending) return nullptr;
   if (!pointer_of(stream.p, &e.stream) || !pointer_of(pending.p, &e.pending))

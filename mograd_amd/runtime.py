@@ -1093,7 +1093,11 @@ def evaluate(node: Node, device: Device) -> AnyBuffer:
     """Scheduler.run for one result (mograd/scheduler.mojo:40-80): evaluates the sources
     first, runs the node's rule once and keeps its buffers on the node; GETTUPLE selects an
     output of a multi-output source.  The walk is native, and so are the common forms of a
-    training step's ops; other ops and strided operands go through `run`."""
+    training step's ops; other ops and strided operands go through `run`.
+
+    The dX of a LINEAR_GRAD that nothing in the walk reads, and whose node nothing else holds, is
+    left out (None in its `bufs`); asked for after all, as a root or by a consumer, it is computed
+    then, and the node's other results stay the ones they are."""
     _graph.evaluate([node], device, run)
     return node.bufs[0]
 

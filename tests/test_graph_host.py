@@ -103,3 +103,42 @@ def test_what_a_walk_reads_of_a_node_is_the_walks_own(host, monkeypatch):
     del lin
     evaluate_many([Node("PROBE", Layout(2), F32, [host.leaf(2)]), dx, dw], host.device)
     assert host.log() == ["linear_bwd dx dw db"]
+
+
+def test_a_left_out_result_is_made_when_it_is_asked_for(host):
+    # evaluate_many([dW]) leaves out the dX that nobody holds; evaluating the LINEAR_GRAD itself
+    # afterwards gives dX, and dW and db stay the buffers they were.
+    lin, (_, dw, db) = linear_grad(host)
+    del _, lin
+    bw, bb = evaluate_many([dw, db], host.device)
+    assert host.log() == ["linear_bwd dw db"] and dw.src(0).bufs == [None, bw, bb]
+    got = evaluate(dw.src(0), host.device)
+    assert got.to_numpy((2, 4))[0, 0] == 1.0
+    assert host.log() == ["linear_bwd dw db", "linear_bwd dx"] and dw.src(0).bufs == [got, bw, bb]
+    assert evaluate(dw.src(0), host.device) is got and evaluate(dw, host.device) is bw
+    assert len(host.log()) == 2
+
+
+@pytest.mark.parametrize("how", ["selector", "operand", "root"])
+def test_a_left_out_result_reaches_every_reader(host, how):
+    lin, (_, dw, _) = linear_grad(host)
+    del _, lin
+    evaluate(dw, host.device)
+    lin = dw.src(0)
+    if how == "selector":
+        node = Node("GETTUPLE", Layout(2, 4), F32, [lin], {"index": 0})
+    elif how == "operand":
+        node = Node("RELU", Layout(2, 4), F32, [lin])
+    else:
+        node = lin
+    assert evaluate_many([dw, node], host.device)[1].to_numpy()[0] == 1.0
+    assert host.log()[:2] == ["linear_bwd dw db", "linear_bwd dx"]
+
+
+def test_a_result_that_is_still_held_is_not_left_out(host):
+    # Its selector is kept for later: dX is that of the weights as they are at the first evaluation.
+    _, (dx, dw, _) = linear_grad(host)
+    del _
+    evaluate(dw, host.device)
+    assert host.log() == ["linear_bwd dx dw db"]
+    assert evaluate(dx, host.device).to_numpy()[0] == 1.0 and len(host.log()) == 1
