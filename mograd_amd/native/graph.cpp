@@ -277,6 +277,7 @@ LayoutObj* as_layout(PyObject* o) { return reinterpret_cast<LayoutObj*>(o); }
 bool is_layout(PyObject* o) { return PyObject_TypeCheck(o, &LayoutType); }
 Py_ssize_t rank_of(const LayoutObj* l) { return PyTuple_GET_SIZE(l->dims); }
 long long dim_of(const LayoutObj* l, Py_ssize_t i) { return PyLong_AsLongLong(PyTuple_GET_ITEM(l->dims, i < 0 ? i + rank_of(l) : i)); }
+long long last_dim(const LayoutObj* l) { return rank_of(l) ? dim_of(l, -1) : 0; }
 long long stride_of(const LayoutObj* l, Py_ssize_t i) {
   return PyLong_AsLongLong(PyTuple_GET_ITEM(l->strides, i < 0 ? i + rank_of(l) : i));
 }
@@ -662,6 +663,14 @@ PyMethodDef buffer_methods[] = {{"data_ptr", FAST(buffer_data_ptr), METH_FASTCAL
 // Evaluation
 // ------------------------------------------------------------------------------------------
 
+// 1, 0, or -1 with an error (a name that is no string may compare as it likes).
+int op_names_equal(PyObject* a, PyObject* b) {
+  if (a == b) return 1;
+  if (!PyUnicode_CheckExact(a) || !PyUnicode_CheckExact(b)) return PyObject_RichCompareBool(a, b, Py_EQ);
+  if (PyUnicode_CHECK_INTERNED(a) && PyUnicode_CHECK_INTERNED(b)) return 0;  // as names written in a program are
+  return PyUnicode_Compare(a, b) == 0;
+}
+
 // One node's execution: its operands, and what the library needs of the device.  The library is called
 // without the interpreter lock, and another thread may evaluate the same nodes meanwhile and
 // replace their buffers: the operands are held here, and their addresses taken, before the call.
@@ -708,13 +717,22 @@ struct Exec {
       if (!lay[i]->contiguous) return false;
     return true;
   }
-  bool truth(PyObject* key, bool fallback) const {
+  // Attributes.  False where one is missing (without `fallback`) or no plain value: left to the Python form,
+  // which converts it or says what is wrong.
+  bool truth(PyObject* key, bool* out) const {
     PyObject* v = PyDict_GetItem(attrs.p, key);
-    return v ? PyObject_IsTrue(v) == 1 : fallback;
+    if (!v || !(PyBool_Check(v) || PyLong_CheckExact(v))) return false;
+    return *out = PyObject_IsTrue(v) == 1, true;
   }
-  double number(PyObject* key) const {
+  bool truth(PyObject* key, bool fallback, bool* out) const {
+    return PyDict_GetItem(attrs.p, key) ? truth(key, out) : (*out = fallback, true);
+  }
+  bool number(PyObject* key, float* out) const {
     PyObject* v = PyDict_GetItem(attrs.p, key);
-    return v ? PyFloat_AsDouble(v) : 0.0;
+    if (!v || !(PyFloat_CheckExact(v) || PyLong_CheckExact(v))) return false;
+    const double d = PyFloat_AsDouble(v);
+    if (d == -1.0 && PyErr_Occurred()) return PyErr_Clear(), false;
+    return *out = static_cast<float>(d), true;
   }
   PyObject* buffer(int dt, long long numel) const {
     return buffer_make(g_buffer_type, storage_make(device, numel * dtype_size(dt)), dt, numel, 0);
@@ -747,7 +765,7 @@ bool gemm_dims(const Exec& x, GemmDims* g) {
   for (const LayoutObj* l : {la, lb})
     for (Py_ssize_t i = rank_of(l) - 4; i >= 0; --i)
       if (stride_of(l, i) != dim_of(l, i + 1) * stride_of(l, i + 1)) return false;
-  if (rank_of(la) < 2 || rank_of(lb) < 2) return false;
+  if (rank_of(la) < 2 || rank_of(lb) < 2 || rank_of(lo) < 1) return false;
   g->N = dim_of(lo, -1);
   g->M = dim_of(la, -2), g->K = dim_of(la, -1);
   if (g->M == 0 || g->K == 0) return false;
@@ -792,8 +810,9 @@ int run_matmul3(const Exec& x, PyObject** out) {
 }
 
 int run_linear_grad(const Exec& x, PyObject** out) {
-  const bool accumulate = x.truth(N.accumulate, false), relu = x.truth(N.relu_mask, false),
-             has_bias = x.truth(N.has_bias, true);
+  bool accumulate, relu, has_bias;
+  if (!x.truth(N.accumulate, false, &accumulate) || !x.truth(N.relu_mask, false, &relu) || !x.truth(N.has_bias, true, &has_bias))
+    return 0;
   if (!x.contiguous(accumulate ? 4 : 3) || !is_float(x.dtype) || rank_of(x.lay[2]) != 2) return 0;
   const long long n = dim_of(x.lay[2], 0), k = dim_of(x.lay[2], 1);
   if (k == 0 || x.lay[0]->numel != x.lay[1]->numel / k * n) return 0;
@@ -817,7 +836,8 @@ int run_linear_grad(const Exec& x, PyObject** out) {
 }
 
 int run_linear_ln_grad(const Exec& x, PyObject** out) {
-  const bool accumulate = x.truth(N.accumulate, false), has_bias = x.truth(N.has_bias, true);
+  bool accumulate, has_bias;
+  if (!x.truth(N.accumulate, false, &accumulate) || !x.truth(N.has_bias, true, &has_bias)) return 0;
   if (!x.contiguous(accumulate ? 8 : 7) || !is_float(x.dtype) || rank_of(x.lay[2]) != 2) return 0;
   const long long n = dim_of(x.lay[2], 0), k = dim_of(x.lay[2], 1);
   if (k == 0) return 0;
@@ -840,11 +860,11 @@ int run_linear_ln_grad(const Exec& x, PyObject** out) {
 }
 
 int run_layer_norm_stats(const Exec& x, PyObject** out) {
-  if (!x.contiguous(3) || !is_float(x.dtype)) return 0;
-  const long long cols = dim_of(x.lay[0], -1);
+  float eps;
+  if (!x.contiguous(3) || !is_float(x.dtype) || !x.number(N.eps, &eps)) return 0;
+  const long long cols = last_dim(x.lay[0]);
   if (cols == 0) return 0;
   const long long rows = x.lay[0]->numel / cols;
-  const float eps = static_cast<float>(x.number(N.eps));
   Results r(x);
   r.add(x.dtype, out_numel(x));
   r.add(MG_F32, rows);
@@ -857,7 +877,7 @@ int run_layer_norm_stats(const Exec& x, PyObject** out) {
 template <bool RESIDUAL>
 int run_layer_norm_stats_grad(const Exec& x, PyObject** out) {
   if (!x.contiguous(RESIDUAL ? 6 : 5) || !is_float(x.dtype)) return 0;
-  const long long cols = dim_of(x.lay[1], -1);
+  const long long cols = last_dim(x.lay[1]);
   if (cols == 0) return 0;
   const long long rows = x.lay[1]->numel / cols;
   Results r(x);
@@ -910,7 +930,7 @@ int run_gather(const Exec& x, PyObject** out) {
 }
 int run_scatter_add(const Exec& x, PyObject** out) {
   const LayoutObj* lo = x.out();
-  if (!x.contiguous(2) || rank_of(x.lay[1]) != rank_of(x.lay[0]) + 1) return 0;
+  if (!x.contiguous(2) || rank_of(x.lay[1]) != rank_of(x.lay[0]) + 1 || rank_of(lo) < 1) return 0;
   Results r(x);
   r.add(x.dtype, lo->numel);
   if (!r.ok) return -1;
@@ -923,8 +943,9 @@ int run_attn_packed(const Exec& x, PyObject** out) {
   const LayoutObj* q = x.lay[0];
   if (x.count < 1 || !is_float(x.dtype) || rank_of(q) != 5 || dim_of(q, 2) != 3) return 0;
   const long long B = dim_of(q, 0), S = dim_of(q, 1), H = dim_of(q, 3), D = dim_of(q, 4);
-  const float scale = static_cast<float>(x.number(N.scale));
-  const bool causal = x.truth(N.is_causal, false), bias = x.truth(N.has_bias, true);
+  float scale;
+  bool causal, bias;
+  if (!x.number(N.scale, &scale) || !x.truth(N.is_causal, &causal) || !x.truth(N.has_bias, true, &bias)) return 0;
   Results r(x);
   r.add(x.dtype, out_numel(x));
   r.add(MG_F32, B * H * S);
@@ -936,8 +957,9 @@ int run_attn_packed_grad(const Exec& x, PyObject** out) {
   if (x.count < 4 || !is_float(x.dtype) || !x.lay[0]->contiguous || rank_of(x.lay[2]) != 5) return 0;
   const LayoutObj* q = x.lay[2];
   const long long B = dim_of(q, 0), S = dim_of(q, 1), H = dim_of(q, 3), D = dim_of(q, 4);
-  const float scale = static_cast<float>(x.number(N.scale));
-  const bool causal = x.truth(N.is_causal, false), bias = x.truth(N.has_bias, !causal);
+  float scale;
+  bool causal, bias;
+  if (!x.number(N.scale, &scale) || !x.truth(N.is_causal, &causal) || !x.truth(N.has_bias, !causal, &bias)) return 0;
   Results r(x);
   r.add(x.dtype, out_numel(x));
   if (!r.ok) return -1;
@@ -947,7 +969,7 @@ int run_attn_packed_grad(const Exec& x, PyObject** out) {
 }
 int run_ce_ids(const Exec& x, PyObject** out) {
   if (!x.contiguous(2) || !is_float(x.dtype)) return 0;
-  const long long c = dim_of(x.lay[0], -1);
+  const long long c = last_dim(x.lay[0]);
   if (c == 0) return 0;
   Results r(x);
   r.add(x.dtype, out_numel(x));
@@ -956,7 +978,7 @@ int run_ce_ids(const Exec& x, PyObject** out) {
 }
 int run_ce_grad_ids(const Exec& x, PyObject** out) {
   if (!x.contiguous(2) || x.count < 3 || !is_float(x.dtype)) return 0;
-  const long long c = dim_of(x.lay[0], -1);
+  const long long c = last_dim(x.lay[0]);
   if (c == 0) return 0;
   Results r(x);
   r.add(x.dtype, out_numel(x));
@@ -1016,14 +1038,27 @@ struct Evaluation {
   PyObject* run;  // runtime.run(node, inputs, device): the Python exec function of a node
   void* stream = nullptr;
   void* pending = nullptr;
+  bool native = true;  // whether the forms of this file may be used at all
   PyObject *kBuffer, *kGetTuple, *kCeIds, *kCeIdsGrad, *kLinearGrad;
 
   NodeObj* node(uint32_t at) const { return as_node(walk[at].node.p); }
   uint32_t source(uint32_t at, uint32_t i) const { return sources[walk[at].first + i]; }
   static bool op_is(const NodeObj* n, PyObject* name) {
-    return n->op_type == name || PyUnicode_Compare(n->op_type, name) == 0;
+    return n->op_type == name || (PyUnicode_Check(n->op_type) && PyUnicode_Compare(n->op_type, name) == 0);
   }
   bool have(uint32_t at) const { return node(at)->bufs != Py_None; }
+  static int dtype_of(const NodeObj* n) {  // -1: none of ours
+    int over = 0;
+    const long v = PyLong_Check(n->node_dtype) ? PyLong_AsLongAndOverflow(n->node_dtype, &over) : -1;
+    return over == 0 && v >= 0 && v <= MG_I64 ? static_cast<int>(v) : -1;
+  }
+  // GETTUPLE's `index`, read like attrs()["index"].
+  static bool index_of(const NodeObj* n, Py_ssize_t* out) {
+    Ref v(PyObject_GetItem(n->node_attrs, N.index)), as_int(v ? PyNumber_Long(v.p) : nullptr);
+    if (!as_int) return false;
+    *out = PyLong_AsSsize_t(as_int.p);
+    return *out != -1 || !PyErr_Occurred();
+  }
 
   bool build(PyObject* const* roots, Py_ssize_t n_roots) {
     std::vector<Ref> order;
@@ -1049,8 +1084,9 @@ struct Evaluation {
       if (op_is(node(i), kCeIdsGrad)) ce_grads.push_back(i);
       uint32_t bit = 1u;  // a node read directly gives its first result
       if (op_is(node(i), kGetTuple)) {
-        PyObject* index = PyDict_GetItem(node(i)->node_attrs, N.index);
-        const long at = index ? PyLong_AsLong(index) : 0;
+        PyObject* index = PyDict_Check(node(i)->node_attrs) ? PyDict_GetItem(node(i)->node_attrs, N.index) : nullptr;
+        int over = 0;
+        const long at = index && PyLong_Check(index) ? PyLong_AsLongAndOverflow(index, &over) : -1;
         bit = at >= 0 && at < 31 ? 1u << at : ~0u;
       }
       for (uint32_t k = 0; k < walk[i].count; ++k) walk[source(i, k)].used |= bit;
@@ -1101,11 +1137,13 @@ struct Evaluation {
     NodeObj* n = node(at);
     const uint32_t count = walk[at].count;
     PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
-    if (idx && count <= Exec::kMost && is_layout(n->node_layout) && PyLong_Check(n->node_dtype)) {
+    const int dtype = dtype_of(n);
+    if (idx && native && count <= Exec::kMost && is_layout(n->node_layout) && PyDict_CheckExact(n->node_attrs) &&
+        dtype_size(dtype) != 0) {
       Exec x;
       x.attrs = Ref::to(n->node_attrs), x.layout = Ref::to(n->node_layout);
       x.device = device, x.stream = stream, x.pending = pending, x.want = want;
-      x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
+      x.dtype = dtype;
       bool plain = true;
       for (uint32_t i = 0; i < count && plain; ++i) {
         Ref b = result(source(at, i), 0);
@@ -1144,15 +1182,15 @@ struct Evaluation {
     Exec x;
     x.layout = Ref::to(n->node_layout);
     Ref grad_layout = Ref::to(g->node_layout);
-    x.device = device, x.dtype = static_cast<int>(PyLong_AsLong(n->node_dtype));
-    if (static_cast<int>(PyLong_AsLong(g->node_dtype)) != x.dtype || !is_float(x.dtype)) return 0;
+    x.device = device, x.dtype = dtype_of(n);
+    if (!native || dtype_of(g) != x.dtype || !is_float(x.dtype)) return 0;
     for (uint32_t i = 0; i < 3; ++i) {
       Ref b = result(source(pair, i), 0);
       if (!b) return -1;
       if (!x.add(std::move(b), node(source(pair, i))->node_layout)) return 0;
     }
-    if (!x.contiguous(3) || rank_of(x.lay[0]) == 0) return 0;
-    const long long c = dim_of(x.lay[0], -1);
+    if (!x.contiguous(3)) return 0;
+    const long long c = last_dim(x.lay[0]);
     if (c == 0) return 0;
     Results loss(x), grad(x);
     loss.add(x.dtype, out_numel(x));
@@ -1176,9 +1214,8 @@ struct Evaluation {
     if (op_is(n, kBuffer)) return raise_invalid("evaluate: a leaf node without a buffer"), false;
     if (!op_is(n, kGetTuple)) return set(n, make(at, walk[at].used | ~1u));
     if (walk[at].count != 1) return raise_invalid("GETTUPLE takes one source"), false;
-    PyObject* index = PyDict_GetItem(n->node_attrs, N.index);
-    const Py_ssize_t i = index ? PyLong_AsSsize_t(index) : 0;
-    if (i == -1 && PyErr_Occurred()) return false;
+    Py_ssize_t i;
+    if (!index_of(n, &i)) return false;
     Ref b = result(source(at, 0), i);
     Ref list(b ? PyList_New(1) : nullptr);
     if (!list) return false;
@@ -1202,8 +1239,7 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   e.kLinearGrad = kLinearGrad;
   Ref stream(PyObject_GetAttr(e.device, N.stream)), pending(PyObject_GetAttr(e.device, N.pending));
   if (!stream || !pending) return nullptr;
-  if (!pointer_of(stream.p, &e.stream) || !pointer_of(pending.p, &e.pending))
-    return PyErr_SetString(PyExc_TypeError, "evaluate: the device's stream is not a pointer"), nullptr;
+  e.native = pointer_of(stream.p, &e.stream) && pointer_of(pending.p, &e.pending);
   if (!e.build(PySequence_Fast_ITEMS(nodes.p), PySequence_Fast_GET_SIZE(nodes.p))) return nullptr;
   for (uint32_t i = 0; i < e.walk.size(); ++i)
     if (!e.evaluate(i)) return nullptr;
@@ -1214,17 +1250,12 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // The rewriting pass (mograd_amd/rewrites.py says what it does; this is its loop)
 // ------------------------------------------------------------------------------------------
 
-bool op_names_equal(PyObject* a, PyObject* b) {
-  if (a == b) return true;
-  if (PyUnicode_CHECK_INTERNED(a) && PyUnicode_CHECK_INTERNED(b)) return false;  // as names written in a program are
-  return PyUnicode_Compare(a, b) == 0;
-}
-
 // Pat.matches
 int pat_matches(PyObject* pat, NodeObj* n) {
   Ref op(PyObject_GetAttr(pat, N.op_type)), srcs(PyObject_GetAttr(pat, N.srcs));
   if (!op || !srcs) return -1;
-  if (op.p != Py_None && !op_names_equal(op.p, n->op_type)) return 0;
+  const int same = op.p == Py_None ? 1 : op_names_equal(op.p, n->op_type);
+  if (same <= 0) return same;
   Ref fast(PySequence_Fast(srcs.p, "Pat.srcs"));
   if (!fast) return -1;
   const Py_ssize_t k = PySequence_Fast_GET_SIZE(fast.p);
@@ -1404,8 +1435,8 @@ PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     for (; round < 64; ++round) {
       bool progressed = false;
       for (Compiled& c : compiled) {
-        if (c.op.p != Py_None && !op_names_equal(c.op.p, as_node(now.p)->op_type)) continue;
-        const int m = pat_matches(c.pat.p, as_node(now.p));
+        int m = c.op.p == Py_None ? 1 : op_names_equal(c.op.p, as_node(now.p)->op_type);
+        if (m > 0) m = pat_matches(c.pat.p, as_node(now.p));
         if (m < 0) return nullptr;
         if (m == 0) continue;
         Ref made(PyObject_CallFunctionObjArgs(c.func.p, now.p, sim, nullptr));

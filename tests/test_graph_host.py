@@ -11,6 +11,7 @@ import pytest
 
 from mograd_amd import _lib
 from mograd_amd import runtime as R
+from mograd_amd.rewrites import GPU_REWRITES, Simplifier
 from mograd_amd.runtime import F32, AnyBuffer, Device, Layout, Node, evaluate, evaluate_many
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -142,3 +143,83 @@ def test_a_result_that_is_still_held_is_not_left_out(host):
     evaluate(dw, host.device)
     assert host.log() == ["linear_bwd dx dw db"]
     assert evaluate(dx, host.device).to_numpy()[0] == 1.0 and len(host.log()) == 1
+
+
+def packed_attention(host, grad=False, **attrs):
+    B, S, H, D = 1, 4, 2, 8
+    qkv = host.leaf(B, S, 3, H, D)
+    if not grad:
+        return Node("FLASH_ATTN_PACKED", Layout(B, S, H, D), F32, [qkv], attrs)
+    return Node("FLASH_ATTN_PACKED_GRAD", Layout(B, S, 3, H, D), F32,
+                [host.leaf(B, S, H, D), host.leaf(B, S, H, D), qkv, host.leaf(B, H, S)], attrs)
+
+
+def test_missing_attributes_are_errors(host):
+    x, g = host.leaf(2, 4), host.leaf(4)
+    norm = Node("LAYER_NORM_STATS", Layout(2, 4), F32, [x, g, g], {"eps": 1e-5})
+    cases = {
+        "scale": [packed_attention(host, is_causal=True), packed_attention(host, True, is_causal=True)],
+        "is_causal": [packed_attention(host, scale=0.5), packed_attention(host, True, scale=0.5)],
+        "eps": [Node("LAYER_NORM_STATS", Layout(2, 4), F32, [x, g, g])],
+        "index": [Node("GETTUPLE", Layout(2, 4), F32, [norm])],
+    }
+    for name, nodes in cases.items():
+        for node in nodes:
+            with pytest.raises(KeyError, match=name):
+                evaluate(node, host.device)
+            assert node.bufs is None
+    assert all(line.startswith("layer_norm_stats") for line in host.log())  # GETTUPLE's source alone ran
+
+
+def test_attributes_are_converted_as_the_python_forms_do(host):
+    evaluate(packed_attention(host, scale=np.float32(0.5), is_causal=np.bool_(True), has_bias=0), host.device)
+    evaluate(packed_attention(host, scale="0.25", is_causal=1, has_bias=[]), host.device)
+    assert host.log() == ["attn_packed 0.500000 1.000000 0.000000", "attn_packed 0.250000 1.000000 0.000000"]
+
+
+def test_operands_without_dimensions_are_errors(host):
+    s, ids = Node.leaf(Layout(), F32, host.leaf(1).bufs[0]), host.leaf(1, dtype=R.I32)
+    m, one = host.leaf(2, 2), host.leaf(1)
+    for op, srcs, attrs in (("CROSS_ENTROPY_IDS", [s, ids], {}), ("CROSS_ENTROPY_IDS_GRAD", [s, ids, one], {}),
+                            ("LAYER_NORM_STATS", [s, one, one], {"eps": 1e-5}),
+                            ("LAYER_NORM_STATS_GRAD", [s, s, one, one, one], {}), ("MATMUL_BT", [m, m], {}),
+                            ("SCATTER_ADD", [ids, host.leaf(1, 3)], {})):
+        with pytest.raises(IndexError):
+            evaluate(Node(op, Layout(), F32, srcs, attrs), host.device)
+    loss = Node("CROSS_ENTROPY_IDS", Layout(), F32, [s, ids])
+    with pytest.raises(IndexError):
+        evaluate_many([loss, Node("CROSS_ENTROPY_IDS_GRAD", Layout(), F32, [s, ids, one])], host.device)
+    assert host.log() == []
+
+
+def test_dtypes_and_ops_that_are_none_of_ours(host):
+    for dtype in (99, -1, 1 << 80):
+        with pytest.raises(R.MogradError, match="dtype"):
+            evaluate(Node("RELU", Layout(2), dtype, [host.leaf(2)]), host.device)
+    for op in (7, None, "NO_SUCH_OP"):
+        with pytest.raises(R.MogradError, match="no scheduler rule"):
+            evaluate(Node(op, Layout(2), F32, [host.leaf(2)]), host.device)
+        node = Node(op, Layout(2), F32, [host.leaf(2)])
+        assert Simplifier(GPU_REWRITES()).run(node) is node
+
+
+def test_a_loss_and_its_gradient_are_one_pass(host):
+    logits, ids, one = host.leaf(3, 5), host.leaf(3, dtype=R.I32, value=2), host.leaf(1)
+    loss = Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids])
+    grad = Node("CROSS_ENTROPY_IDS_GRAD", Layout(3, 5), F32, [logits, ids, one])
+    a, b = evaluate_many([loss, grad], host.device)
+    assert (a.item(), b.to_numpy()[0]) == (4.0, 5.0) and host.log() == ["ce_fused_ids 3.000000 5.000000"]
+    # not where the upstream comes from the walk, or another loss does
+    host.reset()
+    up = Node("RELU", Layout(1), F32, [host.leaf(1)])
+    loss = Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids])
+    evaluate_many([loss, Node("CROSS_ENTROPY_IDS_GRAD", Layout(3, 5), F32, [logits, ids, up])], host.device)
+    assert host.log() == ["ce_ids 3.000000 5.000000", "relu", "ce_grad_ids 3.000000 5.000000"]
+
+
+def test_sources_without_results_are_errors(host, monkeypatch):
+    with pytest.raises(R.MogradError, match="without a buffer"):
+        evaluate(Node("RELU", Layout(2), F32, [Node.leaf(Layout(2), F32)]), host.device)
+    monkeypatch.setitem(R.SCHEDULER_RULES, "EMPTY", lambda node, inputs, device: [])
+    with pytest.raises(IndexError):
+        evaluate(Node("RELU", Layout(2), F32, [Node("EMPTY", Layout(2), F32, [host.leaf(2)])]), host.device)
