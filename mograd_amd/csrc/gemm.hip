@@ -410,6 +410,8 @@ static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
   return launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream);
 }
 
+static bool generic_grid_fits(const GemmArgs& g) { return ceil_div(g.M, 64) <= 65535 && g.batch <= 65535; }
+
 // fp32 products whose operands are each contiguous along one axis.
 //   tiles copied into LDS, 128 x 128 where every CU gets one and the last round of them is not so
 //   empty that 64 x 64 ones, 6 % slower in themselves, are done first ((8000, 600) <- 900, 315 large
@@ -427,17 +429,21 @@ static int dispatch_f32(const GemmArgs& g_in, hipStream_t stream, bool* handled)
   const int64_t cus = device_info().cu_count;
   const int64_t blocks128 = ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch;
   const int64_t blocks64 = ceil_div(g.M, 64) * ceil_div(g.N, 64) * g.batch;
-  // Next to no reduction and a large output (the dX of a 10-class head): neither the copies nor the
-  // fragments have anything to reuse, and the plain kernel's stores are the widest.
-  *handled = !(g.K < 32 && blocks64 >= cus);
-  if (!*handled) return MG_OK;
   const bool a_wide = (a_kc ? mult4(g.sam) && mult4(g.K) : mult4(g.sak) && mult4(g.M)) && mult4(g.bsa) && aligned16(g.a);
   const bool b_wide = (b_kc ? mult4(g.sbn) && mult4(g.K) : mult4(g.sbk) && mult4(g.N)) && mult4(g.bsb) && aligned16(g.b);
   const bool wide = a_wide && b_wide;
+  // Next to no reduction and a large output (the dX of a 10-class head): neither the copies nor the
+  // fragments have anything to reuse, and the plain kernel's stores are the widest.  For one of its
+  // k-steps of 16 that holds whatever the alignment ((2048, 4096) <- 16: 13.0 us against 14.7 with 64 x 64
+  // tiles and 15.7 with 128 x 128; 8192 x 8192 68, 81, 90), for two only against operands that would have to be
+  // copied first (<- 20: 18.5, 14.9, 16.0; 94, 85, 91).  Its grid ends at 65535 batches.
+  const bool plain = g.K < 32 && blocks64 >= cus && (g.K <= kGenericBK || !wide) && generic_grid_fits(g);
+  *handled = !plain;
+  if (plain) return MG_OK;
   const bool use64 = wide ? 2 * blocks64 >= cus || (8 * blocks64 >= cus && g.K >= 1024) ||
                                 (g.K >= 4096 && 2.0 * g.batch * g.M * g.N * g.K >= 4e8)
                           : blocks64 >= cus;
-  const bool use128 = blocks128 >= cus && 4.0 * ceil_div(blocks128, cus) <= 1.06 * ceil_div(blocks64, cus);
+  const bool use128 = blocks128 >= cus && g.K >= 32 && 4.0 * ceil_div(blocks128, cus) <= 1.06 * ceil_div(blocks64, cus);
   const int tile = env_int("MOGRAD_HIP_GEMM_F32_TILE", use128 ? 128 : use64 ? 64 : 32);
   if (tile == 32) {
     if (a_kc && b_kc) return launch_f32_direct<true, true>(g, stream);
@@ -519,7 +525,7 @@ template <typename T>
 static int launch_generic(const GemmArgs& g, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(ceil_div(g.N, 64)), static_cast<unsigned>(ceil_div(g.M, 64)),
                   static_cast<unsigned>(g.batch));
-  if (grid.y > 65535u || grid.z > 65535u) return fail(MG_ERR_INVALID, "matmul: shape exceeds the generic kernel's grid");
+  if (!generic_grid_fits(g)) return fail(MG_ERR_INVALID, "matmul: shape exceeds the generic kernel's grid");
   const T* a = static_cast<const T*>(g.a);
   const T* b = static_cast<const T*>(g.b);
   const T* bias = static_cast<const T*>(g.bias);

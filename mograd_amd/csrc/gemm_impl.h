@@ -95,13 +95,15 @@ __device__ __forceinline__ T gemm_finish(float v, const GemmEpilogue<T>& ep, int
 //   A element (m, k) at A[m * sam + k * sak];  B element (k, n) at B[k * sbk + n * sbn].
 // ------------------------------------------------------------------------------------
 
+constexpr int kGenericBK = 16;  // k per step
+
 template <typename T, bool HAS_BIAS>
 __global__ __launch_bounds__(256) void gemm_generic_kernel(const T* __restrict__ A, const T* __restrict__ B,
                                                            const T* __restrict__ bias, T* __restrict__ C, int M, int N,
                                                            int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn,
                                                            int64_t ldc, int64_t bsa, int64_t bsb, int64_t bsc,
                                                            GemmEpilogue<T> ep) {
-  constexpr int TM = 64, TN = 64, TK = 16;
+  constexpr int TM = 64, TN = 64, TK = kGenericBK;
   __shared__ float as[TK][TM + 1];
   __shared__ float bs[TK][TN + 1];
   const int batch = blockIdx.z;

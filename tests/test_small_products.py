@@ -110,3 +110,23 @@ def test_weight_gradients_alone(device, dtype, M, N, K):
     x, dy = x.astype(np.float64), dy.astype(np.float64)
     assert_close(dw.to_numpy((N, K)), dy.T @ x, rt, rt * np.abs(dy.T @ x).max(), "dw")
     assert_close(db.to_numpy(), dy.sum(axis=0), rt, rt * np.abs(dy.sum(axis=0)).max(), "db")
+
+
+# fp32, a short reduction into a large output: the plain kernel up to its k-step of 16 and, for operands that
+# do not lie on 16-byte chunks, below 32; tiles elsewhere, and wherever the plain kernel's grid ends
+@pytest.mark.parametrize("B,M,N,K", [(1, 1024, 1024, 4), (1, 1024, 1028, 16), (1, 1028, 1024, 20), (1, 1024, 1024, 28),
+                                     (1, 1024, 1024, 17), (1, 1030, 1021, 31), (1, 4096, 4096, 24), (300, 64, 60, 20),
+                                     (65537, 8, 8, 16), (65537, 8, 8, 10), (65537, 8, 7, 20), (1, 4194305, 4, 16)])
+def test_short_reductions_into_large_outputs(device, B, M, N, K):
+    lib, st = device.lib, device.stream
+    a, b = normal(64, 0, (B, M, K)), normal(64, 1, (B, N, K))
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64).transpose(0, 2, 1))
+    for lb in "kn":
+        ba = AnyBuffer.from_numpy(device, a)
+        bb = AnyBuffer.from_numpy(device, b if lb == "k" else b.transpose(0, 2, 1))
+        c = AnyBuffer.create(F32, device, B * M * N)
+        lib.mg_matmul(ba.data_ptr(), bb.data_ptr(), c.data_ptr(), B, M, N, K, K, 1, *((1, K) if lb == "k" else (N, 1)),
+                      M * K, N * K, F32, st)
+        # K products and K - 1 sums, each rounded once: K 2^-24 of sum |a b| at most
+        bound = K * 2.0**-24 * np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64).transpose(0, 2, 1))
+        assert np.all(np.abs(c.to_numpy((B, M, N)) - want) <= bound), lb
