@@ -64,6 +64,7 @@ struct Names {
 PyObject* g_mograd_error = nullptr;   // MogradError(status, message)
 PyObject* g_void_p = nullptr;         // ctypes.c_void_p
 PyTypeObject* g_buffer_type = nullptr;  // AnyBuffer
+PyTypeObject* g_layout_type = nullptr;  // runtime.Layout
 PyObject* g_fallbacks = nullptr;      // name -> ctypes wrapper
 
 // ------------------------------------------------------------------------------------------
@@ -345,9 +346,11 @@ struct NodeObj {
   PyObject_HEAD PyObject* op_type;
   PyObject* node_layout;
   PyObject* node_dtype;
-  PyObject* srcs;        // list
-  PyObject* node_attrs;  // dict
-  PyObject* bufs;        // list or None
+  PyObject* srcs;        // a list or tuple, as a rule
+  PyObject* node_attrs;  // a dict, as a rule
+  PyObject* bufs;        // None, or a sequence of buffers
+  PyObject* dict;        // attributes that a program adds
+  PyObject* weakrefs;
   uint64_t mark;         // the last walk that saw this node
   uint32_t position;     // its place in that walk (between steps that keep the interpreter lock)
 };
@@ -357,24 +360,41 @@ uint64_t g_epoch = 0;
 NodeObj* as_node(PyObject* o) { return reinterpret_cast<NodeObj*>(o); }
 bool is_node(PyObject* o) { return PyObject_TypeCheck(o, &NodeType); }
 
-// Takes over srcs and attrs (null attrs: empty).
-PyObject* node_make(PyObject* op, PyObject* layout, PyObject* dtype, PyObject* srcs, PyObject* attrs, PyObject* bufs) {
-  Ref s(srcs), a(attrs ? attrs : PyDict_New());
-  if (!s || !a) return nullptr;
-  NodeObj* n = reinterpret_cast<NodeObj*>(NodeType.tp_alloc(&NodeType, 0));
+PyObject* new_ref(PyObject* o) { return Py_INCREF(o), o; }
+
+PyObject* node_new(PyTypeObject* type, PyObject*, PyObject*) {
+  NodeObj* n = reinterpret_cast<NodeObj*>(type->tp_alloc(type, 0));
   if (!n) return nullptr;
-  Py_INCREF(op);
-  Py_INCREF(layout);
-  Py_INCREF(dtype);
-  Py_INCREF(bufs);
-  n->op_type = op, n->node_layout = layout, n->node_dtype = dtype, n->bufs = bufs;
-  n->srcs = s.release();
-  n->node_attrs = a.release();
+  for (PyObject** field : {&n->op_type, &n->node_layout, &n->node_dtype, &n->srcs, &n->node_attrs, &n->bufs}) *field = new_ref(Py_None);
+  n->dict = n->weakrefs = nullptr;
   n->mark = 0, n->position = 0;
   return reinterpret_cast<PyObject*>(n);
 }
-
-PyObject* node_new(PyTypeObject*, PyObject* args, PyObject* kw) {
+// Sources as they are kept: a list or tuple itself, any other sequence as a list.
+PyObject* sources_of(PyObject* o) {
+  if (PyList_Check(o) || PyTuple_Check(o)) return new_ref(o);
+  PyObject* list = PySequence_List(o);
+  return list ? list : (PyErr_Clear(), new_ref(o));
+}
+// Takes over srcs and attrs (null: an empty list, an empty dict).
+bool node_fill(PyObject* self, PyObject* op, PyObject* layout, PyObject* dtype, PyObject* srcs, PyObject* attrs, PyObject* bufs) {
+  Ref s(srcs ? srcs : PyList_New(0)), a(attrs ? attrs : PyDict_New());
+  if (!s || !a) return false;
+  NodeObj* n = as_node(self);
+  Py_SETREF(n->op_type, new_ref(op));
+  Py_SETREF(n->node_layout, new_ref(layout));
+  Py_SETREF(n->node_dtype, new_ref(dtype));
+  Py_SETREF(n->srcs, s.release());
+  Py_SETREF(n->node_attrs, a.release());
+  Py_SETREF(n->bufs, new_ref(bufs));
+  return true;
+}
+PyObject* node_make(PyObject* op, PyObject* layout, PyObject* dtype, PyObject* srcs, PyObject* attrs, PyObject* bufs) {
+  Ref n(node_new(&NodeType, nullptr, nullptr));
+  if (!n) return Py_XDECREF(srcs), Py_XDECREF(attrs), nullptr;
+  return node_fill(n.p, op, layout, dtype, srcs, attrs, bufs) ? n.release() : nullptr;
+}
+int node_init(PyObject* self, PyObject* args, PyObject* kw) {
   static const char* names[] = {"op_type", "node_layout", "node_dtype", "srcs", "node_attrs", "bufs", nullptr};
   PyObject *op, *layout, *dtype, *srcs = nullptr, *attrs = nullptr, *bufs = Py_None;
   if (!kw && PyTuple_GET_SIZE(args) >= 3 && PyTuple_GET_SIZE(args) <= 6) {
@@ -385,39 +405,60 @@ PyObject* node_new(PyTypeObject*, PyObject* args, PyObject* kw) {
     if (n > 5) bufs = PyTuple_GET_ITEM(args, 5);
   } else if (!PyArg_ParseTupleAndKeywords(args, kw, "OOO|OOO:Node", const_cast<char**>(names), &op, &layout, &dtype, &srcs,
                                           &attrs, &bufs)) {
-    return nullptr;
+    return -1;
   }
-  if (srcs) Py_INCREF(srcs);
-  else if (!(srcs = PyList_New(0))) return nullptr;
   Py_XINCREF(attrs);
-  return node_make(op, layout, dtype, srcs, attrs, bufs);
+  return node_fill(self, op, layout, dtype, srcs ? sources_of(srcs) : nullptr, attrs, bufs) ? 0 : -1;
 }
 int node_traverse(PyObject* self, visitproc visit, void* arg) {
   NodeObj* n = as_node(self);
-  Py_VISIT(n->op_type);
-  Py_VISIT(n->node_layout);
-  Py_VISIT(n->node_dtype);
-  Py_VISIT(n->srcs);
-  Py_VISIT(n->node_attrs);
-  Py_VISIT(n->bufs);
+  for (PyObject* o : {n->op_type, n->node_layout, n->node_dtype, n->srcs, n->node_attrs, n->bufs, n->dict}) Py_VISIT(o);
   return 0;
 }
-int node_clear(PyObject* self) {
+int node_clear(PyObject* self) {  // (what a cycle can run through; the other fields go with the node)
   NodeObj* n = as_node(self);
-  Py_CLEAR(n->op_type);
-  Py_CLEAR(n->node_layout);
-  Py_CLEAR(n->node_dtype);
-  Py_CLEAR(n->srcs);
-  Py_CLEAR(n->node_attrs);
-  Py_CLEAR(n->bufs);
+  for (PyObject** field : {&n->srcs, &n->node_attrs, &n->bufs}) Py_SETREF(*field, new_ref(Py_None));
+  Py_CLEAR(n->dict);
   return 0;
 }
 void node_dealloc(PyObject* self) {
   PyObject_GC_UnTrack(self);
   Py_TRASHCAN_BEGIN(self, node_dealloc)  // a deep graph is freed without deep recursion
-      node_clear(self);
+  NodeObj* n = as_node(self);
+  if (n->weakrefs) PyObject_ClearWeakRefs(self);
+  for (PyObject** field : {&n->op_type, &n->node_layout, &n->node_dtype, &n->srcs, &n->node_attrs, &n->bufs, &n->dict})
+    Py_CLEAR(*field);
   Py_TYPE(self)->tp_free(self);
   Py_TRASHCAN_END
+}
+// copy, deepcopy, pickle: (fields, attributes) handed to a new node of the same type.
+PyObject* node_reduce(PyObject* self, PyObject*) {
+  NodeObj* n = as_node(self);
+  Ref copyreg(PyImport_ImportModule("copyreg")), make(copyreg ? PyObject_GetAttrString(copyreg.p, "__newobj__") : nullptr);
+  if (!make) return nullptr;
+  return Py_BuildValue("(O(O)((OOOOOO)O))", make.p, reinterpret_cast<PyObject*>(Py_TYPE(self)), n->op_type, n->node_layout,
+                       n->node_dtype, n->srcs, n->node_attrs, n->bufs, n->dict ? n->dict : Py_None);
+}
+PyObject* node_setstate(PyObject* self, PyObject* state) {
+  PyObject *op, *layout, *dtype, *srcs, *attrs, *bufs, *extra;
+  if (!PyArg_ParseTuple(state, "(OOOOOO)O:__setstate__", &op, &layout, &dtype, &srcs, &attrs, &bufs, &extra)) return nullptr;
+  if (!node_fill(self, op, layout, dtype, sources_of(srcs), new_ref(attrs), bufs)) return nullptr;
+  if (extra != Py_None) {
+    Ref dict(PyObject_GetAttrString(self, "__dict__"));
+    if (!dict || PyDict_Update(dict.p, extra) != 0) return nullptr;
+  }
+  Py_RETURN_NONE;
+}
+PyObject* node_get(PyObject* self, void* offset) {
+  return new_ref(*reinterpret_cast<PyObject**>(reinterpret_cast<char*>(self) + reinterpret_cast<uintptr_t>(offset)));
+}
+int node_set(PyObject* self, PyObject* value, void* offset) {
+  if (!value) return PyErr_SetString(PyExc_AttributeError, "a Node's own fields cannot be deleted"), -1;
+  PyObject** field = reinterpret_cast<PyObject**>(reinterpret_cast<char*>(self) + reinterpret_cast<uintptr_t>(offset));
+  PyObject* old = *field;
+  *field = field == &as_node(self)->srcs ? sources_of(value) : new_ref(value);
+  Py_DECREF(old);
+  return 0;
 }
 PyObject* node_layout(PyObject* self, PyObject*) {
   PyObject* o = as_node(self)->node_layout;
@@ -452,15 +493,13 @@ PyObject* node_leaf(PyObject*, PyObject* args, PyObject* kw) {
 PyObject* node_repr(PyObject* self) {
   NodeObj* n = as_node(self);
   return PyUnicode_FromFormat("Node(op_type=%R, node_layout=%R, node_dtype=%R, %zd srcs, node_attrs=%R)", n->op_type,
-                              n->node_layout, n->node_dtype, PyObject_Size(n->srcs), n->node_attrs);
+                              n->node_layout, n->node_dtype, PySequence_Size(n->srcs), n->node_attrs);
 }
-PyMemberDef node_members[] = {{"op_type", T_OBJECT, offsetof(NodeObj, op_type), 0, nullptr},
-                              {"node_layout", T_OBJECT, offsetof(NodeObj, node_layout), 0, nullptr},
-                              {"node_dtype", T_OBJECT, offsetof(NodeObj, node_dtype), 0, nullptr},
-                              {"srcs", T_OBJECT, offsetof(NodeObj, srcs), 0, nullptr},
-                              {"node_attrs", T_OBJECT, offsetof(NodeObj, node_attrs), 0, nullptr},
-                              {"bufs", T_OBJECT, offsetof(NodeObj, bufs), 0, nullptr},
-                              {nullptr, 0, 0, 0, nullptr}};
+#define FIELD(f) {#f, node_get, node_set, nullptr, reinterpret_cast<void*>(offsetof(NodeObj, f))}
+PyGetSetDef node_fields[] = {FIELD(op_type), FIELD(node_layout), FIELD(node_dtype), FIELD(srcs), FIELD(node_attrs), FIELD(bufs),
+                             {"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr},
+                             {nullptr, nullptr, nullptr, nullptr, nullptr}};
+#undef FIELD
 PyMethodDef node_methods[] = {{"layout", node_layout, METH_NOARGS, nullptr},
                               {"dtype", node_dtype, METH_NOARGS, nullptr},
                               {"attrs", node_attrs, METH_NOARGS, nullptr},
@@ -468,11 +507,16 @@ PyMethodDef node_methods[] = {{"layout", node_layout, METH_NOARGS, nullptr},
                               {"src", node_src, METH_O, nullptr},
                               {"shape", node_shape, METH_O, nullptr},
                               {"leaf", FAST(node_leaf), METH_VARARGS | METH_KEYWORDS | METH_STATIC, nullptr},
+                              {"__reduce__", node_reduce, METH_NOARGS, nullptr},
+                              {"__setstate__", node_setstate, METH_O, nullptr},
                               {nullptr, nullptr, 0, nullptr}};
 
+Py_ssize_t src_count(const NodeObj* n) { return PySequence_Fast_GET_SIZE(n->srcs); }
+PyObject* src_of(const NodeObj* n, Py_ssize_t i) { return PySequence_Fast_GET_ITEM(n->srcs, i); }
+
 bool node_ok(PyObject* o) {
-  if (is_node(o) && PyList_Check(as_node(o)->srcs)) return true;
-  PyErr_SetString(PyExc_TypeError, "a graph vertex is a Node with a list of Node sources");
+  if (is_node(o) && (PyList_Check(as_node(o)->srcs) || PyTuple_Check(as_node(o)->srcs))) return true;
+  PyErr_SetString(PyExc_TypeError, "a graph vertex is a Node with a sequence of Node sources");
   return false;
 }
 
@@ -488,9 +532,9 @@ bool toposort(PyObject* const* roots, Py_ssize_t n_roots, std::vector<Ref>& orde
     while (!stack.empty()) {
       NodeObj* n = stack.back().first;
       const Py_ssize_t i = stack.back().second;
-      if (i < PyList_GET_SIZE(n->srcs)) {
+      if (i < src_count(n)) {
         stack.back().second = i + 1;
-        PyObject* c = PyList_GET_ITEM(n->srcs, i);
+        PyObject* c = src_of(n, i);
         if (!node_ok(c)) return false;
         if (as_node(c)->mark != epoch) {
           as_node(c)->mark = epoch;
@@ -527,8 +571,8 @@ PyObject* py_depends_on(PyObject*, PyObject* const* args, Py_ssize_t n) {
     NodeObj* v = stack.back();
     stack.pop_back();
     if (reinterpret_cast<PyObject*>(v) == args[1]) Py_RETURN_TRUE;
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(v->srcs); ++i) {
-      PyObject* c = PyList_GET_ITEM(v->srcs, i);
+    for (Py_ssize_t i = 0; i < src_count(v); ++i) {
+      PyObject* c = src_of(v, i);
       if (!node_ok(c)) return nullptr;
       if (as_node(c)->mark != epoch) {
         as_node(c)->mark = epoch;
@@ -554,12 +598,13 @@ PyObject* storage_make(PyObject* device, long long nbytes) {
   void* p = nullptr;
   const int rc = unlocked([&] { return L.pool_alloc(&p, nbytes); });
   if (rc != 0) return raise_status(rc), nullptr;
-  StorageObj* s = PyObject_New(StorageObj, &StorageType);
-  if (!s) return nullptr;
+  StorageObj* s = PyObject_GC_New(StorageObj, &StorageType);
+  if (!s) return (void)L.mg_pool_free(p), nullptr;
   Py_INCREF(device);
   s->device = device;
   s->ptr = reinterpret_cast<uintptr_t>(p);
   s->nbytes = nbytes;
+  PyObject_GC_Track(s);
   return reinterpret_cast<PyObject*>(s);
 }
 PyObject* storage_new(PyTypeObject*, PyObject* args, PyObject* kw) {
@@ -571,9 +616,15 @@ PyObject* storage_new(PyTypeObject*, PyObject* args, PyObject* kw) {
 }
 void storage_dealloc(PyObject* self) {
   StorageObj* s = reinterpret_cast<StorageObj*>(self);
+  PyObject_GC_UnTrack(self);
   if (s->ptr) (void)L.mg_pool_free(reinterpret_cast<void*>(static_cast<uintptr_t>(s->ptr)));
   Py_XDECREF(s->device);
-  PyObject_Free(self);
+  PyObject_GC_Del(self);
+}
+// (No tp_clear here and for buffers: both are immutable in what a cycle can run through, the device is not.)
+int storage_traverse(PyObject* self, visitproc visit, void* arg) {
+  Py_VISIT(reinterpret_cast<StorageObj*>(self)->device);
+  return 0;
 }
 PyMemberDef storage_members[] = {{"device", T_OBJECT, offsetof(StorageObj, device), READONLY, nullptr},
                                  {"ptr", T_ULONGLONG, offsetof(StorageObj, ptr), READONLY, nullptr},
@@ -623,7 +674,12 @@ PyObject* buffer_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
   Py_INCREF(storage);
   return buffer_make(type, storage, dtype, numel, offset);
 }
+int buffer_traverse(PyObject* self, visitproc visit, void* arg) {
+  Py_VISIT(as_buffer(self)->storage);
+  return 0;
+}
 void buffer_dealloc(PyObject* self) {
+  PyObject_GC_UnTrack(self);
   Py_XDECREF(as_buffer(self)->storage);
   Py_TYPE(self)->tp_free(self);  // (a Python subclass's own deallocator releases its type)
 }
@@ -649,10 +705,17 @@ PyObject* buffer_view(PyObject* self, PyObject* layout) {
 PyObject* buffer_size_bytes(PyObject* self, PyObject*) {
   return PyLong_FromLongLong(as_buffer(self)->numel * dtype_size(as_buffer(self)->dtype));
 }
-PyMemberDef buffer_members[] = {{"storage", T_OBJECT, offsetof(BufferObj, storage), READONLY, nullptr},
-                                {"dtype", T_INT, offsetof(BufferObj, dtype), READONLY, nullptr},
-                                {"numel", T_LONGLONG, offsetof(BufferObj, numel), READONLY, nullptr},
-                                {"offset_elems", T_LONGLONG, offsetof(BufferObj, offset_elems), READONLY, nullptr},
+PyObject* buffer_get_storage(PyObject* self, void*) { return new_ref(as_buffer(self)->storage); }
+int buffer_set_storage(PyObject* self, PyObject* value, void*) {
+  if (!value || Py_TYPE(value) != &StorageType) return PyErr_SetString(PyExc_TypeError, "a buffer's storage is a Storage"), -1;
+  Py_SETREF(as_buffer(self)->storage, new_ref(value));
+  return 0;
+}
+PyGetSetDef buffer_fields[] = {{"storage", buffer_get_storage, buffer_set_storage, nullptr, nullptr},
+                               {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyMemberDef buffer_members[] = {{"dtype", T_INT, offsetof(BufferObj, dtype), 0, nullptr},
+                                {"numel", T_LONGLONG, offsetof(BufferObj, numel), 0, nullptr},
+                                {"offset_elems", T_LONGLONG, offsetof(BufferObj, offset_elems), 0, nullptr},
                                 {nullptr, 0, 0, 0, nullptr}};
 PyMethodDef buffer_methods[] = {{"data_ptr", FAST(buffer_data_ptr), METH_FASTCALL | METH_KEYWORDS, nullptr},
                                 {"view", buffer_view, METH_O, nullptr},
@@ -670,6 +733,13 @@ int op_names_equal(PyObject* a, PyObject* b) {
   if (PyUnicode_CHECK_INTERNED(a) && PyUnicode_CHECK_INTERNED(b)) return 0;  // as names written in a program are
   return PyUnicode_Compare(a, b) == 0;
 }
+
+int dtype_of(const NodeObj* n) {  // -1: none of ours
+  int over = 0;
+  const long v = PyLong_Check(n->node_dtype) ? PyLong_AsLongAndOverflow(n->node_dtype, &over) : -1;
+  return over == 0 && v >= 0 && v <= MG_I64 ? static_cast<int>(v) : -1;
+}
+bool plain_layout(PyObject* o) { return Py_TYPE(o) == g_layout_type || Py_TYPE(o) == &LayoutType; }
 
 // One node's execution: its operands, and what the library needs of the device.  The library is called
 // without the interpreter lock, and another thread may evaluate the same nodes meanwhile and
@@ -691,15 +761,16 @@ struct Exec {
   LayoutObj* lay[kMost];  // of the sources
   int count = 0;
 
-  // Whether the next operand is one of the package's own buffers under one of its layouts (and taken).
-  bool add(Ref buffer, PyObject* layout_of) {
-    if (!PyObject_TypeCheck(buffer.p, &BufferType) || !is_layout(layout_of)) return false;
+  // Whether the next operand, a result of `s`, is one of the package's own buffers under one of its layouts
+  // (and taken).  Types derived from these, whose methods may say something else, are the Python forms'.
+  bool add(Ref buffer, const NodeObj* s) {
+    if (Py_TYPE(s) != &NodeType || Py_TYPE(buffer.p) != g_buffer_type || !plain_layout(s->node_layout)) return false;
     Operand& o = in[count];
     o.p = address(as_buffer(buffer.p));
-    o.dtype = as_buffer(buffer.p)->dtype;
+    o.dtype = dtype_of(s);
     o.buffer = std::move(buffer);
-    o.layout = Ref::to(layout_of);
-    lay[count++] = as_layout(layout_of);
+    o.layout = Ref::to(s->node_layout);
+    lay[count++] = as_layout(s->node_layout);
     return true;
   }
   const LayoutObj* out() const { return as_layout(layout.p); }
@@ -1047,11 +1118,6 @@ struct Evaluation {
     return n->op_type == name || (PyUnicode_Check(n->op_type) && PyUnicode_Compare(n->op_type, name) == 0);
   }
   bool have(uint32_t at) const { return node(at)->bufs != Py_None; }
-  static int dtype_of(const NodeObj* n) {  // -1: none of ours
-    int over = 0;
-    const long v = PyLong_Check(n->node_dtype) ? PyLong_AsLongAndOverflow(n->node_dtype, &over) : -1;
-    return over == 0 && v >= 0 && v <= MG_I64 ? static_cast<int>(v) : -1;
-  }
   // GETTUPLE's `index`, read like attrs()["index"].
   static bool index_of(const NodeObj* n, Py_ssize_t* out) {
     Ref v(PyObject_GetItem(n->node_attrs, N.index)), as_int(v ? PyNumber_Long(v.p) : nullptr);
@@ -1070,11 +1136,10 @@ struct Evaluation {
     }
     std::vector<Py_ssize_t> readers(walk.size(), 0);
     for (uint32_t i = 0; i < walk.size(); ++i) {  // (no Python code since toposort: the positions are ours)
-      PyObject* srcs = node(i)->srcs;
       walk[i].first = static_cast<uint32_t>(sources.size());
-      walk[i].count = static_cast<uint32_t>(PyList_GET_SIZE(srcs));
+      walk[i].count = static_cast<uint32_t>(src_count(node(i)));
       for (uint32_t k = 0; k < walk[i].count; ++k) {
-        const uint32_t at = as_node(PyList_GET_ITEM(srcs, k))->position;
+        const uint32_t at = as_node(src_of(node(i), k))->position;
         if (at >= i) return raise_invalid("evaluate: the graph has a cycle"), false;
         sources.push_back(at);
         ++readers[at];
@@ -1120,11 +1185,16 @@ struct Evaluation {
   }
   // Result i of an evaluated node.
   Ref result(uint32_t at, Py_ssize_t i) {
-    Ref list = i == 0 && lacks_dx(at) ? complete(at) : Ref::to(node(at)->bufs);
+    const bool first = i == 0 || (i < 0 && PyList_Check(node(at)->bufs) && i == -PyList_GET_SIZE(node(at)->bufs));
+    Ref list = first && lacks_dx(at) ? complete(at) : Ref::to(node(at)->bufs);
     if (!list) return Ref();
-    if (!PyList_Check(list.p) || i < 0 || i >= PyList_GET_SIZE(list.p))
-      return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
-    return Ref::to(PyList_GET_ITEM(list.p, i));
+    if (!PyList_Check(list.p) && !PyTuple_Check(list.p)) {
+      Ref index(PyLong_FromSsize_t(i));
+      return index ? Ref(PyObject_GetItem(list.p, index.p)) : Ref();
+    }
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(list.p);
+    if (i < -n || i >= n) return PyErr_SetString(PyExc_IndexError, "evaluate: a source has no such result"), Ref();
+    return Ref::to(PySequence_Fast_GET_ITEM(list.p, i < 0 ? i + n : i));
   }
   static bool set(NodeObj* n, Ref list) {
     if (!list) return false;
@@ -1138,8 +1208,8 @@ struct Evaluation {
     const uint32_t count = walk[at].count;
     PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
     const int dtype = dtype_of(n);
-    if (idx && native && count <= Exec::kMost && is_layout(n->node_layout) && PyDict_CheckExact(n->node_attrs) &&
-        dtype_size(dtype) != 0) {
+    if (idx && native && count <= Exec::kMost && Py_TYPE(n) == &NodeType && plain_layout(n->node_layout) &&
+        PyDict_CheckExact(n->node_attrs) && dtype >= 0) {
       Exec x;
       x.attrs = Ref::to(n->node_attrs), x.layout = Ref::to(n->node_layout);
       x.device = device, x.stream = stream, x.pending = pending, x.want = want;
@@ -1148,7 +1218,7 @@ struct Evaluation {
       for (uint32_t i = 0; i < count && plain; ++i) {
         Ref b = result(source(at, i), 0);
         if (!b) return Ref();
-        plain = x.add(std::move(b), node(source(at, i))->node_layout);
+        plain = x.add(std::move(b), node(source(at, i)));
       }
       if (plain) {
         PyObject* out = nullptr;
@@ -1178,7 +1248,9 @@ struct Evaluation {
           have(source(c, 2)))
         pair = c;
     NodeObj *n = node(at), *g = node(pair);
-    if (pair == at || !is_layout(n->node_layout) || !is_layout(g->node_layout)) return 0;
+    if (pair == at || Py_TYPE(n) != &NodeType || Py_TYPE(g) != &NodeType || !plain_layout(n->node_layout) ||
+        !plain_layout(g->node_layout))
+      return 0;
     Exec x;
     x.layout = Ref::to(n->node_layout);
     Ref grad_layout = Ref::to(g->node_layout);
@@ -1187,7 +1259,7 @@ struct Evaluation {
     for (uint32_t i = 0; i < 3; ++i) {
       Ref b = result(source(pair, i), 0);
       if (!b) return -1;
-      if (!x.add(std::move(b), node(source(pair, i))->node_layout)) return 0;
+      if (!x.add(std::move(b), node(source(pair, i)))) return 0;
     }
     if (!x.contiguous(3)) return 0;
     const long long c = last_dim(x.lay[0]);
@@ -1213,7 +1285,7 @@ struct Evaluation {
     }
     if (op_is(n, kBuffer)) return raise_invalid("evaluate: a leaf node without a buffer"), false;
     if (!op_is(n, kGetTuple)) return set(n, make(at, walk[at].used | ~1u));
-    if (walk[at].count != 1) return raise_invalid("GETTUPLE takes one source"), false;
+    if (walk[at].count == 0) return PyErr_SetString(PyExc_IndexError, "GETTUPLE without a source"), false;
     Py_ssize_t i;
     if (!index_of(n, &i)) return false;
     Ref b = result(source(at, 0), i);
@@ -1259,9 +1331,11 @@ int pat_matches(PyObject* pat, NodeObj* n) {
   Ref fast(PySequence_Fast(srcs.p, "Pat.srcs"));
   if (!fast) return -1;
   const Py_ssize_t k = PySequence_Fast_GET_SIZE(fast.p);
-  if (k > PyList_GET_SIZE(n->srcs)) return 0;
+  if (k > src_count(n)) return 0;
   for (Py_ssize_t i = 0; i < k; ++i) {
-    const int rc = pat_matches(PySequence_Fast_GET_ITEM(fast.p, i), as_node(PyList_GET_ITEM(n->srcs, i)));
+    Ref s = i < src_count(n) ? Ref::to(src_of(n, i)) : Ref();  // (a pattern's op may compare by Python code)
+    if (!s || !node_ok(s.p)) return PyErr_Occurred() ? -1 : 0;
+    const int rc = pat_matches(PySequence_Fast_GET_ITEM(fast.p, i), as_node(s.p));
     if (rc <= 0) return rc;
   }
   return 1;
@@ -1294,21 +1368,21 @@ struct Pass {
   }
   // A node like `n` over other sources (takes over `srcs`).
   static PyObject* rebuilt(NodeObj* n, PyObject* srcs) {
-    PyObject* attrs = PyDict_Copy(n->node_attrs);
+    PyObject* attrs = PyDict_CheckExact(n->node_attrs) ? PyDict_Copy(n->node_attrs)
+                                                       : PyObject_CallOneArg(reinterpret_cast<PyObject*>(&PyDict_Type), n->node_attrs);
     if (!attrs) return Py_DECREF(srcs), nullptr;
     return node_make(n->op_type, n->node_layout, n->node_dtype, srcs, attrs, n->bufs);
   }
   // `node` with every source replaced by what it has become; a new reference.
   PyObject* with_subst(PyObject* node) const {
     NodeObj* n = as_node(node);
-    const Py_ssize_t k = PyList_GET_SIZE(n->srcs);
     Ref fresh;
-    for (Py_ssize_t i = 0; i < k; ++i) {
-      PyObject* s = PyList_GET_ITEM(n->srcs, i);
+    for (Py_ssize_t i = 0; i < src_count(n); ++i) {
+      PyObject* s = src_of(n, i);
       PyObject* to = resolve(s);
       if (!to) return nullptr;
       if (to != s && !fresh) {
-        fresh = Ref(PyList_GetSlice(n->srcs, 0, k));
+        fresh = Ref(PySequence_List(n->srcs));
         if (!fresh) return nullptr;
       }
       if (to != s) {
@@ -1340,20 +1414,21 @@ struct Pass {
         continue;
       }
       NodeObj* v = as_node(r);
-      if (i < PyList_GET_SIZE(v->srcs)) {
+      if (!node_ok(r)) return nullptr;
+      if (i < src_count(v)) {
         stack.back().second = i + 1;
-        PyObject* c = PyList_GET_ITEM(v->srcs, i);
+        PyObject* c = src_of(v, i);
         if (!PyDict_GetItem(done.p, c)) stack.emplace_back(c, 0);
         continue;
       }
       stack.pop_back();
       Ref fresh;
-      for (Py_ssize_t k = 0; k < PyList_GET_SIZE(v->srcs); ++k) {
-        PyObject* s = PyList_GET_ITEM(v->srcs, k);
+      for (Py_ssize_t k = 0; k < src_count(v); ++k) {
+        PyObject* s = src_of(v, k);
         PyObject* to = PyDict_GetItem(done.p, s);
         if (to == s) continue;
         if (!fresh) {
-          fresh = Ref(PyList_GetSlice(v->srcs, 0, PyList_GET_SIZE(v->srcs)));
+          fresh = Ref(PySequence_List(v->srcs));
           if (!fresh) return nullptr;
         }
         Py_INCREF(to);
@@ -1388,8 +1463,8 @@ PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return nullptr;
   Pass pass{sim, subst.p, uses.p, origin.p, consumers.p};
   for (const Ref& v : topo)
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(as_node(v.p)->srcs); ++i) {
-      PyObject* s = PyList_GET_ITEM(as_node(v.p)->srcs, i);
+    for (Py_ssize_t i = 0; i < src_count(as_node(v.p)); ++i) {
+      PyObject* s = src_of(as_node(v.p), i);
       PyObject* list = PyDict_GetItem(consumers.p, s);
       if (!list) {
         Ref fresh(PyList_New(0));
@@ -1477,11 +1552,15 @@ PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_XSETREF(g_fallbacks, args[3]);
   Py_RETURN_NONE;
 }
-PyObject* py_set_buffer_type(PyObject*, PyObject* type) {
-  if (!PyType_Check(type) || !PyType_IsSubtype(reinterpret_cast<PyTypeObject*>(type), &BufferType))
-    return PyErr_SetString(PyExc_TypeError, "a subclass of Buffer is wanted"), nullptr;
-  Py_INCREF(type);
-  Py_XSETREF(g_buffer_type, reinterpret_cast<PyTypeObject*>(type));
+// set_types(AnyBuffer, Layout): the package's own buffers and layouts.
+PyObject* py_set_types(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  auto derived = [&](int i, PyTypeObject* base) {
+    return PyType_Check(args[i]) && PyType_IsSubtype(reinterpret_cast<PyTypeObject*>(args[i]), base);
+  };
+  if (n != 2 || !derived(0, &BufferType) || !derived(1, &LayoutType))
+    return PyErr_SetString(PyExc_TypeError, "set_types(AnyBuffer, Layout)"), nullptr;
+  Py_XSETREF(g_buffer_type, reinterpret_cast<PyTypeObject*>(new_ref(args[0])));
+  Py_XSETREF(g_layout_type, reinterpret_cast<PyTypeObject*>(new_ref(args[1])));
   Py_RETURN_NONE;
 }
 
@@ -1491,7 +1570,7 @@ PyMethodDef module_methods[] = {
     {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run)"},
     {"simplify", FAST(py_simplify), METH_FASTCALL, "simplify(sim, roots)"},
     {"bind", FAST(py_bind), METH_FASTCALL, "bind(handle, MogradError, c_void_p, fallbacks)"},
-    {"set_buffer_type", py_set_buffer_type, METH_O, "The type of the buffers that evaluate() makes."},
+    {"set_types", FAST(py_set_types), METH_FASTCALL, "set_types(AnyBuffer, Layout)"},
     {nullptr, nullptr, 0, nullptr}};
 PyMethodDef library_methods[] = {
 #define X(f) {#f, FAST(py_##f), METH_FASTCALL, nullptr},
@@ -1523,29 +1602,35 @@ PyMODINIT_FUNC PyInit__graph() {
 
   NodeType.tp_name = "mograd_amd._graph.Node";
   NodeType.tp_basicsize = sizeof(NodeObj);
-  NodeType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  NodeType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC | Py_TPFLAGS_BASETYPE;
+  NodeType.tp_dictoffset = offsetof(NodeObj, dict);
+  NodeType.tp_weaklistoffset = offsetof(NodeObj, weakrefs);
   NodeType.tp_doc =
       "Just enough of an op node for the exec functions: its own layout and dtype, the layouts of its\n"
       "sources, and its attributes (mograd/op.mojo:124-185).  `bufs` is what the reference keeps in op().buf\n"
       "(mograd/scheduler.mojo:74-78): a leaf's buffer, or the results of an evaluated node.";
   NodeType.tp_new = node_new;
+  NodeType.tp_init = node_init;
   NodeType.tp_dealloc = node_dealloc;
   NodeType.tp_traverse = node_traverse;
   NodeType.tp_clear = node_clear;
-  NodeType.tp_members = node_members;
+  NodeType.tp_getset = node_fields;
   NodeType.tp_methods = node_methods;
   NodeType.tp_repr = node_repr;
 
   StorageType.tp_name = "mograd_amd._graph.Storage";
   StorageType.tp_basicsize = sizeof(StorageObj);
-  StorageType.tp_flags = Py_TPFLAGS_DEFAULT;
+  StorageType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  StorageType.tp_traverse = storage_traverse;
   StorageType.tp_new = storage_new;
   StorageType.tp_dealloc = storage_dealloc;
   StorageType.tp_members = storage_members;
 
   BufferType.tp_name = "mograd_amd._graph.Buffer";
   BufferType.tp_basicsize = sizeof(BufferObj);
-  BufferType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+  BufferType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
+  BufferType.tp_traverse = buffer_traverse;
+  BufferType.tp_getset = buffer_fields;
   BufferType.tp_new = buffer_new;
   BufferType.tp_dealloc = buffer_dealloc;
   BufferType.tp_members = buffer_members;

@@ -15,6 +15,7 @@ tests.  It contains no arithmetic: every result comes from the C ABI.
 """
 from __future__ import annotations
 
+import copyreg
 import ctypes as C
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -74,7 +75,11 @@ class Layout(_graph.Layout):
     stride(idx), numel(), is_contiguous() (layout.mojo:210-212) and as_contiguous() (:238-240) are the
     native base's."""
 
-    __slots__ = ()
+    __slots__ = ("__weakref__",)
+
+    def __reduce__(self):  # copy, pickle
+        kw = {"strides": self.strides, "base_offset": self.base_offset}
+        return copyreg.__newobj_ex__, (type(self), self.dims, kw), getattr(self, "__dict__", None)
 
     def batch_dims_collapsible(self) -> bool:  # layout.mojo:214-236
         for i in range(self.rank() - 4, -1, -1):
@@ -178,7 +183,8 @@ class AnyBuffer(_graph.Buffer):
     """A typed device buffer (mograd/buffer.mojo:135-214): AnyBuffer(storage, dtype, numel, offset_elems=0).
     `view(layout)` shares storage; data_ptr(with_offset=True) is the device address as a c_void_p."""
 
-    __slots__ = ()
+    def __reduce__(self):  # a copy shares the storage
+        return copyreg.__newobj__, (type(self), self.storage, self.dtype, self.numel, self.offset_elems), self.__dict__ or None
 
     @staticmethod
     def supports(dtype: int) -> bool:
@@ -222,7 +228,7 @@ class AnyBuffer(_graph.Buffer):
         return self.to_numpy().reshape(-1)[0].item()
 
 
-_graph.set_buffer_type(AnyBuffer)
+_graph.set_types(AnyBuffer, Layout)
 
 
 # --------------------------------------------------------------------------- #
@@ -232,7 +238,8 @@ _graph.set_buffer_type(AnyBuffer)
 
 # Node(op_type, node_layout, node_dtype, srcs=[], node_attrs={}, bufs=None): a graph vertex with layout(),
 # dtype(), numel(), src(i), attrs(), shape(i) and Node.leaf(layout, dtype, buf), compared and hashed by
-# identity like OpRef.
+# identity like OpRef.  An ordinary object otherwise: fields can be set and attributes added, it can be
+# derived from, copied, pickled and weakly referenced.
 Node = _graph.Node
 
 

@@ -143,8 +143,9 @@ int mg_flash_attn_bwd_packed(const void*, const void*, const void*, const void*,
                              int64_t, int64_t, float scale, int causal, int bias, int, mg_stream) {
   return note("attn_packed_bwd" + num(scale) + num(causal) + num(bias));
 }
-int mg_cross_entropy_ids(const void*, const void*, void* loss, int64_t rows, int64_t classes, int, int, mg_stream) {
-  return fill(loss, 4), note("ce_ids" + num(rows) + num(classes));
+int mg_cross_entropy_ids(const void*, const void*, void* loss, int64_t rows, int64_t classes, int, int id_dtype,
+                         mg_stream) {
+  return fill(loss, 4), note("ce_ids" + num(rows) + num(classes) + " dtype " + std::to_string(id_dtype));
 }
 int mg_cross_entropy_grad_ids(const void*, const void*, const void*, void* grad, int64_t rows, int64_t classes, int, int,
                               mg_stream) {

@@ -1,9 +1,13 @@
 """The native host path (mograd_amd/native/graph.cpp) without a GPU: the package over a library that
 records its calls (tests/host_cpp/stub_library.cpp)."""
+import collections
+import copy
 import ctypes as C
 import gc
+import pickle
 import subprocess
 import threading
+import weakref
 from pathlib import Path
 
 import numpy as np
@@ -214,7 +218,7 @@ def test_a_loss_and_its_gradient_are_one_pass(host):
     up = Node("RELU", Layout(1), F32, [host.leaf(1)])
     loss = Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids])
     evaluate_many([loss, Node("CROSS_ENTROPY_IDS_GRAD", Layout(3, 5), F32, [logits, ids, up])], host.device)
-    assert host.log() == ["ce_ids 3.000000 5.000000", "relu", "ce_grad_ids 3.000000 5.000000"]
+    assert host.log() == ["ce_ids 3.000000 5.000000 dtype 3", "relu", "ce_grad_ids 3.000000 5.000000"]
 
 
 def test_sources_without_results_are_errors(host, monkeypatch):
@@ -223,3 +227,114 @@ def test_sources_without_results_are_errors(host, monkeypatch):
     monkeypatch.setitem(R.SCHEDULER_RULES, "EMPTY", lambda node, inputs, device: [])
     with pytest.raises(IndexError):
         evaluate(Node("RELU", Layout(2), F32, [Node("EMPTY", Layout(2), F32, [host.leaf(2)])]), host.device)
+
+
+def test_sources_may_be_any_sequence(host):
+    leaf = host.leaf(4)
+    for make in (tuple, list, collections.deque):
+        mid = Node("ADD", Layout(4), F32, make([leaf, leaf]))
+        out = Node("RELU", Layout(4), F32, make([mid]))
+        assert R._toposort(out) == [leaf, mid, out]
+        assert Simplifier(GPU_REWRITES()).run(out) is out
+        (g,) = R.gradient(out, host.leaf(4), [leaf])
+        assert g.op_type == "ADD"
+        np.testing.assert_array_equal(evaluate(out, host.device).to_numpy(), np.full(4, 2.0))
+    for bad in (None, 3, [leaf, "x"]):
+        with pytest.raises(TypeError):
+            evaluate(Node("RELU", Layout(4), F32, bad), host.device)
+
+
+def test_a_rewritten_graph_over_tuples(host):
+    x, w, r = host.leaf(2, 4), host.leaf(3, 4), host.leaf(2, 3)
+    out = Node("ADD", Layout(2, 3), F32, (Node("MATMUL_BT", Layout(2, 3), F32, (x, w)), r))
+    top = Node("RELU", Layout(2, 3), F32, (out,))
+    new = Simplifier(GPU_REWRITES()).run(top)
+    assert new.src(0).op_type == "MATMUL_BT_ADD" and new.src(0).srcs == [x, w, r]
+
+
+def test_gettuple_counts_from_the_end(host):
+    lin, _ = linear_grad(host)
+    get = lambda i: Node("GETTUPLE", Layout(3), F32, [lin, lin], {"index": i})  # noqa: E731
+    got = [evaluate(get(i), host.device) for i in (-1, -2, -3, 2)]
+    assert got == [lin.bufs[2], lin.bufs[1], lin.bufs[0], lin.bufs[2]] and len(host.log()) == 1
+    for i in (3, -4):
+        with pytest.raises(IndexError):
+            evaluate(get(i), host.device)
+
+
+def test_results_may_be_any_sequence(host, monkeypatch):
+    buf = host.leaf(4).bufs[0]
+    monkeypatch.setitem(R.SCHEDULER_RULES, "PAIR", lambda node, inputs, device: (buf, inputs[0]))
+    pair = Node("PAIR", Layout(4), F32, [host.leaf(4)])
+    assert evaluate(Node("GETTUPLE", Layout(4), F32, [pair], {"index": -1}), host.device) is pair.src(0).bufs[0]
+    leaf = Node("BUFFER", Layout(4), F32, bufs=(buf,))
+    evaluate(Node("RELU", Layout(4), F32, [leaf]), host.device)
+
+
+def test_nodes_are_ordinary_objects(host):
+    class Tagged(Node):
+        def __init__(self, *args, tag="", **kw):
+            super().__init__(*args, **kw)
+            self.tag = tag
+
+        def layout(self):
+            return Layout(2, 2)
+
+    leaf = host.leaf(4)
+    node = Node("RELU", Layout(4), F32, [leaf], {"a": 1})
+    node.note = "kept"
+    assert weakref.ref(node)() is node and node.note == "kept" and vars(node) == {"note": "kept"}
+    with pytest.raises(AttributeError):
+        del node.srcs
+    tagged = Tagged("RELU", Layout(4), F32, [leaf], tag="t")
+    assert isinstance(tagged, Node) and tagged.tag == "t" and tagged in {tagged} and tagged != node
+    assert evaluate(tagged, host.device).numel == 4  # by the Python form: node.numel() is the node's own
+    for copied in (copy.copy(node), copy.copy(tagged)):
+        assert copied.srcs[0] is leaf and copied.op_type == "RELU"
+    assert copy.copy(node).note == "kept" and copy.copy(tagged).tag == "t" and type(copy.copy(tagged)) is Tagged
+    # a graph without results goes through deepcopy and pickle, shared nodes shared
+    shared = Node("RELU", Layout(4), F32, [Node.leaf(Layout(4), F32)])
+    add = Node("ADD", Layout(4), F32, [shared, shared], {"axis": 0})
+    add.note = 5
+    for proto in range(pickle.HIGHEST_PROTOCOL + 1):
+        for again in (copy.deepcopy(add), pickle.loads(pickle.dumps(add, proto))):
+            assert again is not add and again.srcs[0] is again.srcs[1] and again.srcs[0] is not shared
+            assert (again.layout(), again.attrs(), again.note, again.bufs) == (Layout(4), {"axis": 0}, 5, None)
+    ref = weakref.ref(add)
+    del add
+    assert ref() is None
+
+
+def test_layouts_are_copied_and_pickled():
+    for layout in (Layout(), Layout(3), Layout(2, 3, strides=[1, 2], base_offset=7), Layout((4, 5))):
+        for proto in range(pickle.HIGHEST_PROTOCOL + 1):
+            for again in (copy.copy(layout), copy.deepcopy(layout), pickle.loads(pickle.dumps(layout, proto))):
+                assert again == layout and hash(again) == hash(layout) and again.is_contiguous() == layout.is_contiguous()
+        assert weakref.ref(layout)() is layout
+
+
+def test_buffers_are_ordinary_objects(host):
+    buf = host.leaf(4).bufs[0]
+    buf.name = "b"
+    again = copy.copy(buf)
+    assert again.name == "b" and again.storage is buf.storage and weakref.ref(buf)() is buf
+    buf.numel = buf.offset_elems = 2
+    assert buf.to_numpy().shape == (2,) and buf.data_ptr().value == again.data_ptr().value + 8
+    buf.storage = host.leaf(8).bufs[0].storage
+    with pytest.raises(TypeError):
+        buf.storage = 3
+    # a device that keeps buffers of its own: both go when the last outside reference does
+    dev = Device()
+    dev.cache = AnyBuffer.create(F32, dev, 4)
+    gone = weakref.ref(dev)
+    del dev
+    gc.collect()
+    assert gone() is None
+
+
+def test_the_dtype_of_indices_is_the_nodes(host):
+    # as in the Python forms: a leaf declared float32 over int32 ids is what the library is told
+    logits, ids = host.leaf(3, 5), host.leaf(3, dtype=R.I32)
+    evaluate(Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, Node.leaf(Layout(3), F32, ids.bufs[0])]), host.device)
+    evaluate(Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids]), host.device)
+    assert host.log() == ["ce_ids 3.000000 5.000000 dtype 0", "ce_ids 3.000000 5.000000 dtype 3"]
