@@ -8,15 +8,16 @@ run from it; constructing a `Device` does, and raises if they are missing.
 _FROM_LIB = ("BF16", "F16", "F32", "I32", "I64", "LibraryMissing", "MogradError", "load")
 _FROM_RUNTIME = ("GRAD_RULES", "SCHEDULER_RULES", "AnyBuffer", "Device", "Layout", "Node", "evaluate", "evaluate_many",
                  "gradient", "run")
-__all__ = [*_FROM_LIB, *_FROM_RUNTIME]
+_MODULES = ("_lib", "runtime")
+__all__ = [*_FROM_LIB, *_FROM_RUNTIME, "runtime"]
 
 __version__ = "0.1"
 
 
 def __getattr__(name: str):
-    if name not in __all__:
+    if name not in __all__ and name not in _MODULES:
         raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
-    from . import _lib, runtime
+    from . import _lib, runtime  # (binds both names here as well)
 
     for n in _FROM_LIB:
         globals()[n] = getattr(_lib, n)

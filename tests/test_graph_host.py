@@ -6,6 +6,7 @@ import ctypes as C
 import gc
 import pickle
 import subprocess
+import sys
 import threading
 import weakref
 from pathlib import Path
@@ -338,3 +339,10 @@ def test_the_dtype_of_indices_is_the_nodes(host):
     evaluate(Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, Node.leaf(Layout(3), F32, ids.bufs[0])]), host.device)
     evaluate(Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids]), host.device)
     assert host.log() == ["ce_ids 3.000000 5.000000 dtype 0", "ce_ids 3.000000 5.000000 dtype 3"]
+
+
+@pytest.mark.parametrize("first", ["runtime", "_lib", "Node", "load"])
+def test_the_package_alone_gives_its_modules_and_names(first):
+    code = (f"import mograd_amd as m; m.{first}; m.runtime.Node is m.Node or 1 / 0; m._lib.load is m.load or 1 / 0\n"
+            "try:\n    m.no_such_name\nexcept AttributeError:\n    pass\nelse:\n    1 / 0")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT)
