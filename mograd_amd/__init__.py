@@ -17,10 +17,12 @@ __version__ = "0.1"
 def __getattr__(name: str):
     if name not in __all__ and name not in _MODULES:
         raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
-    from . import _lib, runtime  # (binds both names here as well)
+    # (not `from . import`, which asks this function for the modules before it imports them)
+    import importlib
 
+    _lib, runtime = (importlib.import_module(f"{__name__}.{m}") for m in _MODULES)
     for n in _FROM_LIB:
         globals()[n] = getattr(_lib, n)
     for n in _FROM_RUNTIME:
         globals()[n] = getattr(runtime, n)
-    return globals()[name]
+    return globals()[name]  # (importing the modules has bound their names too)
