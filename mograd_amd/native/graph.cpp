@@ -1092,6 +1092,12 @@ const std::pair<const char*, Form> kForms[] = {
     {"CROSS_ENTROPY_IDS_GRAD", run_ce_grad_ids},
     {"RESHAPE", run_reshape},
 };
+constexpr size_t kFormCount = sizeof(kForms) / sizeof(kForms[0]);
+
+// The package's own exec functions, and the run() that looks them up: a form stands in for its op's function
+// only while the rule table holds that one.
+PyObject* g_own_run = nullptr;
+PyObject* g_own_rules[kFormCount];
 
 // One evaluate() call: the nodes in order, and what the walk knows of each.  Nothing of a walk is kept on
 // the nodes, which other walks (other threads, or an exec function of this one) may visit meanwhile.
@@ -1106,7 +1112,8 @@ struct Evaluation {
   std::vector<uint32_t> ce_grads;  // CROSS_ENTROPY_IDS_GRAD nodes
 
   PyObject* device;
-  PyObject* run;  // runtime.run(node, inputs, device): the Python exec function of a node
+  PyObject* run;    // runtime.run(node, inputs, device): the Python exec function of a node
+  PyObject* rules;  // the table it looks in
   void* stream = nullptr;
   void* pending = nullptr;
   bool native = true;  // whether the forms of this file may be used at all
@@ -1202,13 +1209,19 @@ struct Evaluation {
     return true;
   }
 
+  // The index of the form for an op, or -1: there is none, or a program has put its own function in its place.
+  long form_of(PyObject* op) const {
+    PyObject* idx = native ? PyDict_GetItem(g_forms, op) : nullptr;
+    const long i = idx ? PyLong_AsLong(idx) : -1;
+    return i >= 0 && PyDict_GetItem(rules, op) == g_own_rules[i] ? i : -1;
+  }
   // The results of a node whose sources have theirs; without those that are neither wanted nor made anyway.
   Ref make(uint32_t at, uint32_t want) {
     NodeObj* n = node(at);
     const uint32_t count = walk[at].count;
-    PyObject* idx = PyDict_GetItem(g_forms, n->op_type);
+    const long form = form_of(n->op_type);
     const int dtype = dtype_of(n);
-    if (idx && native && count <= Exec::kMost && Py_TYPE(n) == &NodeType && plain_layout(n->node_layout) &&
+    if (form >= 0 && count <= Exec::kMost && Py_TYPE(n) == &NodeType && plain_layout(n->node_layout) &&
         PyDict_CheckExact(n->node_attrs) && dtype >= 0) {
       Exec x;
       x.attrs = Ref::to(n->node_attrs), x.layout = Ref::to(n->node_layout);
@@ -1222,7 +1235,7 @@ struct Evaluation {
       }
       if (plain) {
         PyObject* out = nullptr;
-        const int rc = kForms[PyLong_AsLong(idx)].second(x, &out);
+        const int rc = kForms[form].second(x, &out);
         if (rc < 0) return Ref();
         if (rc > 0) return Ref(out);
       }
@@ -1255,7 +1268,7 @@ struct Evaluation {
     x.layout = Ref::to(n->node_layout);
     Ref grad_layout = Ref::to(g->node_layout);
     x.device = device, x.dtype = dtype_of(n);
-    if (!native || dtype_of(g) != x.dtype || !is_float(x.dtype)) return 0;
+    if (form_of(kCeIds) < 0 || form_of(kCeIdsGrad) < 0 || dtype_of(g) != x.dtype || !is_float(x.dtype)) return 0;
     for (uint32_t i = 0; i < 3; ++i) {
       Ref b = result(source(pair, i), 0);
       if (!b) return -1;
@@ -1296,13 +1309,13 @@ struct Evaluation {
   }
 };
 
-// evaluate(nodes, device, run): gives every node of `nodes` and of their sources its buffers.
+// evaluate(nodes, device, run, rules): gives every node of `nodes` and of their sources its buffers.
 PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 3) return PyErr_SetString(PyExc_TypeError, "evaluate(nodes, device, run)"), nullptr;
+  if (n != 4) return PyErr_SetString(PyExc_TypeError, "evaluate(nodes, device, run, rules)"), nullptr;
   Ref nodes(PySequence_Tuple(args[0]));
   if (!nodes) return nullptr;
   Evaluation e;
-  e.device = args[1], e.run = args[2];
+  e.device = args[1], e.run = args[2], e.rules = args[3];
   static PyObject *kBuffer = str_("BUFFER"), *kGetTuple = str_("GETTUPLE");
   e.kBuffer = kBuffer, e.kGetTuple = kGetTuple;
   static PyObject *kCeIds = str_("CROSS_ENTROPY_IDS"), *kCeIdsGrad = str_("CROSS_ENTROPY_IDS_GRAD");
@@ -1311,7 +1324,7 @@ PyObject* py_evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   e.kLinearGrad = kLinearGrad;
   Ref stream(PyObject_GetAttr(e.device, N.stream)), pending(PyObject_GetAttr(e.device, N.pending));
   if (!stream || !pending) return nullptr;
-  e.native = pointer_of(stream.p, &e.stream) && pointer_of(pending.p, &e.pending);
+  e.native = e.run == g_own_run && PyDict_CheckExact(e.rules) && pointer_of(stream.p, &e.stream) && pointer_of(pending.p, &e.pending);
   if (!e.build(PySequence_Fast_ITEMS(nodes.p), PySequence_Fast_GET_SIZE(nodes.p))) return nullptr;
   for (uint32_t i = 0; i < e.walk.size(); ++i)
     if (!e.evaluate(i)) return nullptr;
@@ -1564,10 +1577,23 @@ PyObject* py_set_types(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// set_rules(run, rules): the package's own exec functions.
+PyObject* py_set_rules(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 2 || !PyDict_Check(args[1])) return PyErr_SetString(PyExc_TypeError, "set_rules(run, rules)"), nullptr;
+  Py_XSETREF(g_own_run, new_ref(args[0]));
+  for (size_t i = 0; i < kFormCount; ++i) {
+    PyObject* own = PyDict_GetItemString(args[1], kForms[i].first);
+    if (!own) return PyErr_Format(PyExc_KeyError, "%s", kForms[i].first), nullptr;
+    Py_XSETREF(g_own_rules[i], new_ref(own));
+  }
+  Py_RETURN_NONE;
+}
+
 PyMethodDef module_methods[] = {
     {"toposort", py_toposort, METH_O, "Sources before consumers, each node once."},
     {"depends_on", FAST(py_depends_on), METH_FASTCALL, "depends_on(node, target): whether target is node or feeds it."},
-    {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run)"},
+    {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run, rules)"},
+    {"set_rules", FAST(py_set_rules), METH_FASTCALL, "set_rules(run, rules): the package's own."},
     {"simplify", FAST(py_simplify), METH_FASTCALL, "simplify(sim, roots)"},
     {"bind", FAST(py_bind), METH_FASTCALL, "bind(handle, MogradError, c_void_p, fallbacks)"},
     {"set_types", FAST(py_set_types), METH_FASTCALL, "set_types(AnyBuffer, Layout)"},
@@ -1645,7 +1671,7 @@ PyMODINIT_FUNC PyInit__graph() {
       !add_type(m, &BufferType, "Buffer"))
     return nullptr;
   g_forms = PyDict_New();
-  for (size_t i = 0; i < sizeof(kForms) / sizeof(kForms[0]); ++i) {
+  for (size_t i = 0; i < kFormCount; ++i) {
     Ref v(PyLong_FromSize_t(i)), k(str_(kForms[i].first));
     if (!v || PyDict_SetItem(g_forms, k.p, v.p) != 0) return nullptr;
   }

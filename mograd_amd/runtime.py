@@ -861,12 +861,17 @@ SCHEDULER_RULES = {
 
 
 def run(node: Node, inputs: List[AnyBuffer], device: Device) -> List[AnyBuffer]:
-    """One scheduler step: first matching rule wins (pattern_matcher.mojo:74-80)."""
+    """One scheduler step: first matching rule wins (pattern_matcher.mojo:74-80).  evaluate() runs the
+    native form of an op instead, where it has one, as long as the table holds the op's function
+    from this module."""
     try:
         fn = SCHEDULER_RULES[node.op_type]
     except KeyError:
         raise MogradError(2, f"no scheduler rule for op {node.op_type} on the backward hot path") from None
     return fn(node, inputs, device)
+
+
+_graph.set_rules(run, SCHEDULER_RULES)
 
 
 # --------------------------------------------------------------------------- #
@@ -1105,7 +1110,7 @@ def evaluate(node: Node, device: Device) -> AnyBuffer:
     The dX of a LINEAR_GRAD that nothing in the walk reads, and whose node nothing else holds, is
     left out (None in its `bufs`); asked for after all, as a root or by a consumer, it is computed
     then, and the node's other results stay the ones they are."""
-    _graph.evaluate([node], device, run)
+    _graph.evaluate([node], device, run, SCHEDULER_RULES)
     return node.bufs[0]
 
 
@@ -1119,7 +1124,7 @@ def evaluate_many(nodes: Sequence[Node], device: Device, deferred_sums: bool = F
         device.lib.mg_deferred_create(C.byref(pending))
         device.pending = pending
     try:
-        _graph.evaluate(nodes, device, run)
+        _graph.evaluate(nodes, device, run, SCHEDULER_RULES)
         if deferred_sums:
             device.lib.mg_finish_deferred(device.pending, device.stream)
     finally:

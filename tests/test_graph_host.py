@@ -25,7 +25,7 @@ ROOT = Path(__file__).resolve().parent.parent
 @pytest.fixture(scope="module")
 def stub_path(tmp_path_factory):
     out = tmp_path_factory.mktemp("stub") / "libstub.so"
-    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", f"-I{ROOT / 'include'}",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-Wl,-Bsymbolic", f"-I{ROOT / 'include'}",
                     str(ROOT / "tests" / "host_cpp" / "stub_library.cpp"), "-o", str(out)], check=True)
     return out
 
@@ -346,3 +346,35 @@ def test_the_package_alone_gives_its_modules_and_names(first):
     code = (f"import mograd_amd as m; m.{first}; m.runtime.Node is m.Node or 1 / 0; m._lib.load is m.load or 1 / 0\n"
             "try:\n    m.no_such_name\nexcept AttributeError:\n    pass\nelse:\n    1 / 0")
     subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT)
+
+
+@pytest.mark.parametrize("op", ["RELU", "ADD", "CROSS_ENTROPY_IDS", "CROSS_ENTROPY_IDS_GRAD", "LINEAR_GRAD"])
+def test_a_replaced_rule_is_the_one_that_runs(host, monkeypatch, op):
+    seen, own = [], R.SCHEDULER_RULES[op]
+
+    def traced(node, inputs, device):
+        seen.append(node.op_type)
+        return own(node, inputs, device)
+
+    def graph():
+        logits, ids, leaf = host.leaf(3, 5), host.leaf(3, dtype=R.I32), host.leaf(4)
+        lin, (_, dw, _) = linear_grad(host)
+        return [Node("RELU", Layout(4), F32, [Node("ADD", Layout(4), F32, [leaf, leaf])]), dw,
+                Node("CROSS_ENTROPY_IDS", Layout(1), F32, [logits, ids]),
+                Node("CROSS_ENTROPY_IDS_GRAD", Layout(3, 5), F32, [logits, ids, host.leaf(1)])]
+
+    rules = dict(R.SCHEDULER_RULES)
+    monkeypatch.setattr(R, "SCHEDULER_RULES", rules)
+    rules[op] = traced
+    evaluate_many(graph(), host.device)
+    assert seen == [op]
+    del rules[op]
+    with pytest.raises(R.MogradError, match=f"no scheduler rule for op {op}"):
+        evaluate_many(graph(), host.device)
+
+
+def test_a_replaced_run_is_the_one_that_runs(host, monkeypatch):
+    seen, own = [], R.run
+    monkeypatch.setattr(R, "run", lambda node, inputs, device: (seen.append(node.op_type), own(node, inputs, device))[1])
+    evaluate(Node("RELU", Layout(4), F32, [host.leaf(4)]), host.device)
+    assert seen == ["RELU"]
