@@ -1461,6 +1461,44 @@ struct Pass {
   }
 };
 
+// A Rule or Pat like `o`, its own object down to the last pattern (a new reference).
+PyObject* rule_copy(PyObject* o) {
+  PyObject** from = _PyObject_GetDictPtr(o);
+  Ref made(Py_TYPE(o)->tp_alloc(Py_TYPE(o), 0));
+  PyObject** to = made ? _PyObject_GetDictPtr(made.p) : nullptr;
+  if (!from || !*from || !to || !(*to = PyDict_Copy(*from))) return nullptr;
+  if (PyObject* pat = PyDict_GetItem(*to, N.pat)) {
+    Ref fresh(rule_copy(pat));
+    if (!fresh || PyDict_SetItem(*to, N.pat, fresh.p) != 0) return nullptr;
+  }
+  PyObject* srcs = PyDict_GetItem(*to, N.srcs);
+  if (srcs && PyList_Check(srcs)) {
+    Ref list(PyList_GetSlice(srcs, 0, PyList_GET_SIZE(srcs)));
+    if (!list) return nullptr;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list.p); ++i) {
+      PyObject* fresh = rule_copy(PyList_GET_ITEM(list.p, i));
+      if (!fresh) return nullptr;
+      PyList_SetItem(list.p, i, fresh);
+    }
+    if (PyDict_SetItem(*to, N.srcs, list.p) != 0) return nullptr;
+  }
+  return made.release();
+}
+// copy_rules(rules): a list of new Rule objects over new patterns.
+PyObject* py_copy_rules(PyObject*, PyObject* rules) {
+  Ref list(PySequence_List(rules));
+  if (!list) return nullptr;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list.p); ++i) {
+    PyObject* fresh = rule_copy(PyList_GET_ITEM(list.p, i));
+    if (!fresh) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "copy_rules: not a Rule");
+      return nullptr;
+    }
+    PyList_SetItem(list.p, i, fresh);
+  }
+  return list.release();
+}
+
 // simplify(sim, roots): Simplifier.run_many.
 PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (n_args != 2) return PyErr_SetString(PyExc_TypeError, "simplify(sim, roots)"), nullptr;
@@ -1595,6 +1633,7 @@ PyMethodDef module_methods[] = {
     {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run, rules)"},
     {"set_rules", FAST(py_set_rules), METH_FASTCALL, "set_rules(run, rules): the package's own."},
     {"simplify", FAST(py_simplify), METH_FASTCALL, "simplify(sim, roots)"},
+    {"copy_rules", py_copy_rules, METH_O, "copy_rules(rules): new Rule objects over new patterns"},
     {"bind", FAST(py_bind), METH_FASTCALL, "bind(handle, MogradError, c_void_p, fallbacks)"},
     {"set_types", FAST(py_set_types), METH_FASTCALL, "set_types(AnyBuffer, Layout)"},
     {nullptr, nullptr, 0, nullptr}};

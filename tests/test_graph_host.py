@@ -378,3 +378,22 @@ def test_a_replaced_run_is_the_one_that_runs(host, monkeypatch):
     monkeypatch.setattr(R, "run", lambda node, inputs, device: (seen.append(node.op_type), own(node, inputs, device))[1])
     evaluate(Node("RELU", Layout(4), F32, [host.leaf(4)]), host.device)
     assert seen == ["RELU"]
+
+
+def test_rewrite_rules_belong_to_the_caller(host):
+    def flat(rules):
+        pats = [r.pat for r in rules]
+        for p in pats:
+            pats.extend(p.srcs)
+        return list(rules) + pats
+
+    first, second = GPU_REWRITES(), GPU_REWRITES()
+    assert first == second and [r.name for r in first] == [r.func.__name__ for r in first]
+    assert not {id(o) for o in flat(first)} & {id(o) for o in flat(second)}
+    for rule in first:
+        rule.func = lambda node, sim: None
+        rule.pat.op_type = "NO_SUCH_OP"
+    first[1].pat.srcs.clear()
+    assert GPU_REWRITES() == second
+    mm = Node("MATMUL_BIAS_BT", Layout(2, 3), F32, [host.leaf(2, 4), host.leaf(3, 4), host.leaf(3)])
+    assert Simplifier(GPU_REWRITES()).run(Node("RELU", Layout(2, 3), F32, [mm])).op_type == "MATMUL_BIAS_RELU_BT"
