@@ -1,5 +1,5 @@
 """Builds libmograd_hip.so (gfx950) from mograd_amd/csrc/*.hip with hipcc, and the host extension
-_graph.so from mograd_amd/native/graph.cpp with g++.
+_graph from mograd_amd/native/graph.cpp with g++.
 
 Usage: python -m mograd_amd.build [--force] [--jobs N]
 
@@ -23,7 +23,9 @@ CSRC = PKG / "csrc"
 OBJ_DIR = CSRC / "build"
 LIB_PATH = PKG / "libmograd_hip.so"
 NATIVE_SRC = PKG / "native" / "graph.cpp"
-NATIVE_PATH = PKG / "_graph.so"
+# Named for the interpreter it is compiled for (_graph.cpython-310-x86_64-linux-gnu.so): another Python
+# does not find it and asks for a build instead of loading it.
+NATIVE_PATH = PKG / f"_graph{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 ARCH = "gfx950"
 # -packed-fp32-ops is switched off: v_pk_*_f32 forms are not to be generated.
@@ -68,6 +70,7 @@ def _compile(hipcc: str, src: Path, obj: Path) -> tuple[Path, int, str]:
 
 def build_native(force: bool = False, verbose: bool = True) -> Path:
     """The CPython extension mograd_amd._graph (host code only)."""
+    (PKG / "_graph.so").unlink(missing_ok=True)  # the name it once had, which any Python would load
     newest = max(f.stat().st_mtime for f in (NATIVE_SRC, ROOT / "include" / "mograd_hip.h"))
     if force or not NATIVE_PATH.exists() or NATIVE_PATH.stat().st_mtime < newest:
         cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",

@@ -35,6 +35,14 @@ def test_binding_covers_the_header():
     assert declared == bound, f"header-only: {declared - bound}; binding-only: {bound - declared}"
 
 
+def test_host_extension_is_named_for_its_interpreter():
+    import sysconfig
+
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert "cpython" in suffix and Path(_lib._graph.__file__).name == "_graph" + suffix
+    assert not (ROOT / "mograd_amd" / "_graph.so").exists()
+
+
 def test_pure_host_entry_points():
     lib = mograd_amd.load()
     assert lib.mg_version().startswith(b"mograd_hip")
