@@ -542,8 +542,11 @@ static int launch_generic(const GemmArgs& g, hipStream_t stream) {
   return MG_OK;
 }
 
+// Rows of at most this many of an fp32 operand without a unit stride are copied k-contiguous.
+constexpr int64_t kThinRows = 128;
+
 int gemm_dispatch(const char* who, const GemmArgs& g_in, hipStream_t stream) {
-  const GemmArgs& g = g_in;
+  GemmArgs g = g_in;
   if (!is_float_dtype(g.dtype)) return fail(MG_ERR_INVALID, "%s: unsupported dtype %s", who, dtype_name(g.dtype));
   if (g.batch < 0 || g.M < 0 || g.N < 0 || g.K < 0 || g.M > 0x7fffffffLL || g.N > 0x7fffffffLL || g.K > 0x7fffffffLL)
     return fail(MG_ERR_INVALID, "%s: bad shape batch=%lld M=%lld N=%lld K=%lld", who, static_cast<long long>(g.batch),
@@ -551,9 +554,28 @@ int gemm_dispatch(const char* who, const GemmArgs& g_in, hipStream_t stream) {
   if (g.batch == 0 || g.M == 0 || g.N == 0) return MG_OK;
   if (!g.a || !g.b || !g.c) return fail(MG_ERR_INVALID, "%s: null pointer argument", who);
 
+  // A thin fp32 operand that is contiguous along neither axis (every second column of a table) would leave
+  // the whole product to the plain kernel, which walks a long K in few workgroups: it is copied first, a
+  // small fraction of the other operand's bytes.
+  Scratch a_copy, b_copy;
+  if (g.dtype == MG_F32 && g.K >= 512) {
+    const bool a_unit = g.sak == 1 || g.sam == 1, b_unit = g.sbk == 1 || g.sbn == 1;
+    const bool a_thin = g.M <= kThinRows, b_thin = g.N <= kThinRows;
+    auto copy = [&](Scratch& mem, const void** src, int64_t rows, int64_t* row_stride, int64_t* k_stride, int64_t* batch_stride) -> int {
+      const int64_t images = *batch_stride == 0 ? 1 : g.batch;
+      MG_TRY(mem.take(images * rows * g.K * static_cast<int64_t>(sizeof(float))));
+      const int64_t shape[3] = {images, rows, g.K}, strides[3] = {*batch_stride, *row_stride, *k_stride};
+      MG_TRY(mg_contiguous(*src, mem.as<float>(), 3, shape, strides, MG_F32, stream));
+      *src = mem.as<float>();
+      *row_stride = g.K, *k_stride = 1, *batch_stride = images == 1 ? 0 : rows * g.K;
+      return MG_OK;
+    };
+    if (!a_unit && a_thin && (b_unit || b_thin)) MG_TRY(copy(a_copy, &g.a, g.M, &g.sam, &g.sak, &g.bsa));
+    if (!b_unit && b_thin && (a_unit || a_thin)) MG_TRY(copy(b_copy, &g.b, g.N, &g.sbn, &g.sbk, &g.bsb));
+  }
   if (g.dtype == MG_F32 && g.K > 0 && (g.sak == 1 || g.sam == 1) && (g.sbk == 1 || g.sbn == 1)) {
     bool handled = false;
-    const int rc = dispatch_f32(g_in, stream, &handled);
+    const int rc = dispatch_f32(g, stream, &handled);
     if (handled || rc != MG_OK) return rc;
   }
   if (g.dtype != MG_F32) {

@@ -130,3 +130,29 @@ def test_short_reductions_into_large_outputs(device, B, M, N, K):
         # K products and K - 1 sums, each rounded once: K 2^-24 of sum |a b| at most
         bound = K * 2.0**-24 * np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64).transpose(0, 2, 1))
         assert np.all(np.abs(c.to_numpy((B, M, N)) - want) <= bound), lb
+
+
+# fp32 operands of at most 128 rows that are contiguous along neither axis, with a long K: copied to
+# k-contiguous rows, so that the product is bit for bit that of the copy
+@pytest.mark.parametrize("B,M,N,K,which", [(1, 10, 4096, 2048, "a"), (1, 1, 300, 512, "a"), (1, 256, 128, 1001, "b"),
+                                           (1, 96, 100, 1024, "ab"), (3, 128, 260, 520, "a"), (3, 200, 7, 640, "b"),
+                                           (1, 129, 64, 512, "a"), (1, 64, 300, 511, "a")])
+def test_thin_operands_without_a_unit_stride(device, B, M, N, K, which):
+    lib, st = device.lib, device.stream
+    a, b = normal(65, 0, (B, M, 2 * K)), normal(65, 1, (B, N, 2 * K))
+    ops = {"a": a, "b": b}
+    flat = {k: np.ascontiguousarray(t[..., ::2]) for k, t in ops.items()}
+
+    def product(strided):
+        buf = {k: AnyBuffer.from_numpy(device, ops[k] if k in strided else flat[k]) for k in "ab"}
+        ld = {k: (2 * K, 2, ops[k].shape[1] * 2 * K) if k in strided else (K, 1, ops[k].shape[1] * K) for k in "ab"}
+        c = AnyBuffer.create(F32, device, B * M * N)
+        lib.mg_matmul_bt(buf["a"].data_ptr(), buf["b"].data_ptr(), c.data_ptr(), B, M, N, K, *ld["a"][:2], *ld["b"][:2],
+                         ld["a"][2], ld["b"][2], F32, st)
+        return c.to_numpy((B, M, N))
+
+    got, x, y = product(which), flat["a"].astype(np.float64), flat["b"].astype(np.float64).transpose(0, 2, 1)
+    # K products and K - 1 sums, each rounded once: K 2^-24 of sum |a b| at most
+    assert np.all(np.abs(got - x @ y) <= K * 2.0**-24 * (np.abs(x) @ np.abs(y)))
+    if K >= 512 and all(ops[k].shape[1] <= 128 for k in which):
+        np.testing.assert_array_equal(got, product(""))
