@@ -16,7 +16,7 @@ import pytest
 
 from mograd_amd import _lib
 from mograd_amd import runtime as R
-from mograd_amd.rewrites import GPU_REWRITES, Simplifier
+from mograd_amd.rewrites import GPU_REWRITES, Pat, Rule, Simplifier
 from mograd_amd.runtime import F32, AnyBuffer, Device, Layout, Node, evaluate, evaluate_many
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -397,3 +397,15 @@ def test_rewrite_rules_belong_to_the_caller(host):
     assert GPU_REWRITES() == second
     mm = Node("MATMUL_BIAS_BT", Layout(2, 3), F32, [host.leaf(2, 4), host.leaf(3, 4), host.leaf(3)])
     assert Simplifier(GPU_REWRITES()).run(Node("RELU", Layout(2, 3), F32, [mm])).op_type == "MATMUL_BIAS_RELU_BT"
+
+
+def test_cycles_are_errors(host):
+    a = Node("RELU", Layout(4), F32, [host.leaf(4)])
+    b = Node("RELU", Layout(4), F32, [a])
+    a.srcs[0] = b
+    with pytest.raises(R.MogradError, match="cycle"):
+        evaluate(b, host.device)
+    flip = [Rule(Pat(x), lambda node, sim, y=y: Node(y, node.layout(), node.dtype(), node.srcs)) for x, y in ("AB", "BA")]
+    with pytest.raises(R.MogradError, match="cycled"):
+        Simplifier(flip).run(Node("A", Layout(4), F32, [host.leaf(4)]))
+    a.srcs.clear()

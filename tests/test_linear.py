@@ -419,28 +419,33 @@ def test_batched_projections_share_an_operand(device, dtype, rtol, M, d):
                                    (2048, 512, 1024),
                                    # 1024 output tiles: more than the resident workgroups, each walks two
                                    (4096, 4096, 64)])
-def test_f32_tile_staging_variants_agree(device, monkeypatch, M, N, K):
-    # fp32 products have a register-staged kernel and one whose tiles are copied straight into
-    # LDS (K a multiple of 32); same tiles and k order, so the results must be identical bits
-    # for the forward (k/k), dX (k/n) and dW (m/n) operand layouts, ragged tile edges included.
+def test_f32_tile_sizes_agree(device, monkeypatch, M, N, K):
+    # fp32 products have 128 x 128 and 64 x 64 output tiles that are copied into LDS, with the same k
+    # order, so that the results must be identical bits for the forward (k/k), dX (k/n) and dW (m/n) operand
+    # layouts, ragged tile edges included; and tiles straight from memory, whose waves share the
+    # reduction: another order of the sums.
     x = normal(59, 0, (M, K))
     w = normal(59, 1, (N, K), std=0.05)
     b = normal(59, 2, (N,), std=0.1)
     dy = normal(59, 3, (M, N), std=0.5)
-    # (an output of few tiles would be split along K, which changes the order of the sums:
-    # switched off for the bitwise comparison, on again for the comparison with the oracle)
+    # (an output of few tiles would be split along K, and differently for the two sizes, which changes the
+    # order of the sums: switched off for the bitwise comparison, on again for those with the oracle)
     monkeypatch.setenv("MOGRAD_HIP_GEMM_SPLITK_MIN_K", str(1 << 30))
-    monkeypatch.setenv("MOGRAD_HIP_GEMM_F32_PIPE", "0")
+    monkeypatch.setenv("MOGRAD_HIP_GEMM_F32_TILE", "128")
     base = _linear_all(device, x, w, b, dy)
-    monkeypatch.delenv("MOGRAD_HIP_GEMM_F32_PIPE")
-    got = _linear_all(device, x, w, b, dy)
-    for g, want, name in zip(got, base, ("y", "dx", "dw", "db")):
+    monkeypatch.setenv("MOGRAD_HIP_GEMM_F32_TILE", "64")
+    for g, want, name in zip(_linear_all(device, x, w, b, dy), base, ("y", "dx", "dw", "db")):
         np.testing.assert_array_equal(g, want, err_msg=name)
     monkeypatch.delenv("MOGRAD_HIP_GEMM_SPLITK_MIN_K")
-    got = _linear_all(device, x, w, b, dy)
-    assert_sum_close(got[0], O.matmul_bias_bt(x, w, b), np.abs(x) @ np.abs(w).T, what="y")
-    assert_sum_close(got[1], O.linear_grad_x(dy, w), np.abs(dy) @ np.abs(w), what="dx")
-    assert_sum_close(got[2], O.linear_grad_w(dy, x), np.abs(dy).T @ np.abs(x), what="dw")
+    for tile in ("32", "64", "128", None):
+        if tile:
+            monkeypatch.setenv("MOGRAD_HIP_GEMM_F32_TILE", tile)
+        else:
+            monkeypatch.delenv("MOGRAD_HIP_GEMM_F32_TILE")
+        got = _linear_all(device, x, w, b, dy)
+        assert_sum_close(got[0], O.matmul_bias_bt(x, w, b), np.abs(x) @ np.abs(w).T, what=f"y {tile}")
+        assert_sum_close(got[1], O.linear_grad_x(dy, w), np.abs(dy) @ np.abs(w), what=f"dx {tile}")
+        assert_sum_close(got[2], O.linear_grad_w(dy, x), np.abs(dy).T @ np.abs(x), what=f"dw {tile}")
 
 
 @pytest.mark.parametrize("M,N,K", [(8192, 2048, 1024), (4104, 4000, 1088), (2048, 8192, 2048)])

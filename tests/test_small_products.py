@@ -19,9 +19,8 @@ SHAPES = [(1, 1, 1), (5, 3, 4), (64, 10, 256), (33, 17, 65), (130, 65, 100), (64
           (1000, 72, 88), (1023, 264, 8), (1025, 96, 384), (1999, 1001, 767), (2587, 256, 256), (1056, 1152, 384)]
 
 
-@pytest.mark.parametrize("dtype", [F32, F16, BF16])
-@pytest.mark.parametrize("M,N,K", SHAPES)
-def test_linear_forward_and_backward(device, dtype, M, N, K):
+def check_linear(device, dtype, M, N, K):
+    """Forward (bias, ReLU) and the three gradients (ReLU mask, accumulating dX) of one layer."""
     lib, st, rt = device.lib, device.stream, RT[dtype]
     x = np.maximum(round_to_dtype(normal(60, 0, (M, K)), dtype), 0)
     w = round_to_dtype(normal(60, 1, (N, K), std=0.1), dtype)
@@ -43,6 +42,35 @@ def test_linear_forward_and_backward(device, dtype, M, N, K):
     assert_close(dw.to_numpy((N, K)), want, rt, rt * max(np.abs(want).max(), 1e-3), "dw")
     want = dy.sum(axis=0)
     assert_close(db.to_numpy(), want, rt, rt * max(np.abs(want).max(), 1e-3), "db")
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_linear_forward_and_backward(device, dtype, M, N, K):
+    check_linear(device, dtype, M, N, K)
+
+
+# Both sides of each choice that the dispatch makes by size, at sizes where it could go either way
+@pytest.mark.parametrize("dtype,knob,values,shapes", [
+    # fp32: tiles straight from memory, of 64 x 64, of 128 x 128, aligned and copied operands
+    (F32, "GEMM_F32_TILE", (32, 64, 128), [(300, 264, 200), (257, 129, 333), (70, 33, 1030)]),
+    # fp32 backward: one launch from memory (up to so many MFLOP), or a launch for each product
+    (F32, "LINEAR_BWD_F32_MFLOP", (0, 100000), [(300, 264, 200), (257, 129, 333), (1500, 10, 260)]),
+    # 16-bit operands off the 16-byte chunks: staged as they are, or copied first
+    (BF16, "GEMM16_PAD", (0, 1), [(300, 265, 200), (257, 129, 333), (1030, 130, 67)]),
+    (F16, "GEMM16_PAD", (0, 1), [(257, 129, 333)]),
+    # 16-bit forward on 64 x 64 and on 128 x 128 tiles
+    (BF16, "GEMM16_PIPE", (64, 642), [(300, 264, 200), (129, 72, 1024)]),
+    # 16-bit backward on 128-row tiles or 64 x 64 ones, and those with dW's rows in 1, 3 or 7 ranges
+    (BF16, "LINEAR_BWD_SMALL", (0, 1), [(2048, 264, 200), (1999, 129, 333), (2600, 776, 384)]),
+    (BF16, "LINEAR_BWD_SPLITS", (1, 3, 7), [(1030, 264, 200), (999, 129, 65)]),
+    (F16, "LINEAR_BWD_SPLITS", (1, 3), [(999, 129, 65)]),
+])
+def test_both_sides_of_a_choice(device, monkeypatch, dtype, knob, values, shapes):
+    for value in values:
+        monkeypatch.setenv("MOGRAD_HIP_" + knob, str(value))
+        for M, N, K in shapes:
+            check_linear(device, dtype, M, N, K)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
