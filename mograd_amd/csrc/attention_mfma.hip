@@ -306,9 +306,10 @@ __device__ __forceinline__ uint2 bias_group(const T* __restrict__ row, int n, in
 
 // ---- forward -----------------------------------------------------------------------------
 
-// DC: the columns that are multiplied, where they are fewer than the DP of the staged rows (heads of 80
-// and 96 columns in the 128-column kernels, of 32 in the 64-column ones; the rest of a row is
-// staged as zeros and left alone).  bf16 (8, 500, 8 heads, 96), causal:
+// DC: the columns that are multiplied, where they are fewer than the DP of the staged rows: 96 for heads
+// of 65 to 96 columns in the 128-column kernels, 32 for heads of up to 32 in the 64-column ones (80
+// columns are multiplied as 96; the rest of a row is staged as zeros and left alone).  The pipelined
+// backward walks multiply all 64.  bf16 (8, 500, 8 heads, 96), causal:
 // 20 + 78 us forward + backward with 128 columns, 17 + 58 with 96; (30, 1616, 3, 32): 53 -> 45 forward.
 template <typename T, int DP, bool CAUSAL, bool HAS_BIAS, int DC>
 __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_fwd_mfma_kernel(const T* __restrict__ q, const T* __restrict__ k,
@@ -2152,7 +2153,7 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
     if constexpr (DP <= 128) {                                                                                       \
       if (fused) {                                                                                                   \
         if (!B_ && pipe)                                                                                             \
-          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, (!B_ && DP <= 64), DC>), grid_fused, dim3(kAttnThreads), 0, stream,  \
+          hipLaunchKernelGGL((attn_bwd_mfma_kernel<T, DP, C_, B_, (!B_ && DP <= 64), (!B_ && DP <= 64 ? DP : DC)>), grid_fused, dim3(kAttnThreads), 0, stream,  \
                              d_o_, q_, k_, v_, mask_, lse, delta.as<float>(), dq_, dk_, dv_, a, scale,               \
                              static_cast<int>(blocks), ps.nlse, ps.ndelta, s_pad);                                   \
         else                                                                                                         \

@@ -9,9 +9,11 @@
 // s mod 4, and the four partial tiles meet in LDS in wave order.  With tiles of 16 or 32,
 // a 64 x 256 output is 64 (16) workgroups of four short loops, where a single
 // 128 x 128 tile walks its whole k range in one workgroup: what bounds such a product is the
-// latency of that walk.  Four sizes of it on one MI355X, 128 x 128 tiles -> this kernel:
-//   (64, 256) <- 784            68 -> 6.2 us      (2048, 4096) <- 10          18 -> 9.2 us
-//   (128, 64) <- 64             18 -> 4.1 us      (317, 568) <- 2400          33 -> 17 us
+// latency of that walk.  Three sizes of it on one MI355X, 128 x 128 tiles -> this kernel:
+//   (64, 256) <- 784            68 -> 6.2 us      (317, 568) <- 2400          33 -> 17 us
+//   (128, 64) <- 64             18 -> 4.1 us
+// Not for large outputs with a short reduction, which are bound by their stores ((2048, 4096) <- 16: 36 us
+// here, 13 with the plain kernel): dispatch_f32 sends none.
 #pragma once
 
 #include "gemm_impl.h"
