@@ -760,7 +760,7 @@ def bench_gpt(args, dev) -> dict:
                  "note": "gradient() + Simplifier(GPU_REWRITES()) + evaluate_many(deferred sums) over the model's node graph, "
                          "rebuilt every step (graph_kept: built once, evaluated every step); same kernels and bits as the "
                          "hand-sequenced step, whose time is `value`; the difference is host time of this Python mirror "
-                         "(one pool allocation and one ctypes call per node)"}
+                         "(graph building, gradient and rewrite rules, one pool allocation per result)"}
     flops = model.flops_per_step(B, T)
     tf = flops / (ms * 1e-3) / 1e12
     # The backward kernel that takes most of the step: linear_bwd_16bit_kernel (dX and dW of one
