@@ -1142,6 +1142,7 @@ struct Evaluation {
       node(i)->position = i;
     }
     std::vector<Py_ssize_t> readers(walk.size(), 0);
+    std::vector<uint32_t> at_root;
     for (uint32_t i = 0; i < walk.size(); ++i) {  // (no Python code since toposort: the positions are ours)
       walk[i].first = static_cast<uint32_t>(sources.size());
       walk[i].count = static_cast<uint32_t>(src_count(node(i)));
@@ -1152,6 +1153,8 @@ struct Evaluation {
         ++readers[at];
       }
     }
+    for (Py_ssize_t i = 0; i < n_roots; ++i) at_root.push_back(as_node(roots[i])->position);
+    // (Looking up an attribute may run Python code, after which the positions may be another walk's.)
     for (uint32_t i = 0; i < walk.size(); ++i) {
       if (op_is(node(i), kCeIdsGrad)) ce_grads.push_back(i);
       uint32_t bit = 1u;  // a node read directly gives its first result
@@ -1163,7 +1166,7 @@ struct Evaluation {
       }
       for (uint32_t k = 0; k < walk[i].count; ++k) walk[source(i, k)].used |= bit;
     }
-    for (Py_ssize_t i = 0; i < n_roots; ++i) walk[as_node(roots[i])->position].used = ~0u;
+    for (const uint32_t i : at_root) walk[i].used = ~0u;
     // A layer's dX that nobody reads (the first layer's input is data) is not computed, unless something
     // outside the walk holds the node too (a selector of dX that is kept for later): its result is
     // that of the operands as they are now.

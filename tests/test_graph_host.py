@@ -409,3 +409,24 @@ def test_cycles_are_errors(host):
     with pytest.raises(R.MogradError, match="cycled"):
         Simplifier(flip).run(Node("A", Layout(4), F32, [host.leaf(4)]))
     a.srcs.clear()
+
+
+def test_a_walk_keeps_its_places_when_an_attribute_lookup_walks_too(host):
+    # A key with the hash of "index" that compares by Python code evaluates another graph over the same
+    # nodes while the outer walk looks its attributes up.
+    lin, (_, dw, _) = linear_grad(host)
+    del _, lin
+    evaluate(dw, host.device)  # without dX
+    lin = dw.src(0)
+
+    class Key:
+        def __hash__(self):
+            return hash("index")
+
+        def __eq__(self, other):
+            evaluate_many([Node("RELU", Layout(4), F32, [host.leaf(4)]), dw], host.device)
+            return False
+
+    get = Node("GETTUPLE", Layout(3, 4), F32, [lin], {Key(): 0, "index": 1})
+    got = evaluate_many([get, lin], host.device)
+    assert got[0] is dw.bufs[0] and got[1].to_numpy()[0] == 1.0
