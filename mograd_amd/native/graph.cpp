@@ -16,6 +16,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <new>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -1630,12 +1631,23 @@ PyObject* py_set_rules(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// An entry whose containers may fail to grow: a MemoryError instead of an exception through the interpreter.
+template <auto F, class... A>
+PyObject* guarded(PyObject* self, A... args) {
+  try {
+    return F(self, args...);
+  } catch (const std::bad_alloc&) {
+    return PyErr_NoMemory();
+  }
+}
+using FastArgs = PyObject* const*;
+
 PyMethodDef module_methods[] = {
-    {"toposort", py_toposort, METH_O, "Sources before consumers, each node once."},
-    {"depends_on", FAST(py_depends_on), METH_FASTCALL, "depends_on(node, target): whether target is node or feeds it."},
-    {"evaluate", FAST(py_evaluate), METH_FASTCALL, "evaluate(nodes, device, run, rules)"},
+    {"toposort", guarded<py_toposort, PyObject*>, METH_O, "Sources before consumers, each node once."},
+    {"depends_on", FAST((guarded<py_depends_on, FastArgs, Py_ssize_t>)), METH_FASTCALL, "depends_on(node, target): whether target is node or feeds it."},
+    {"evaluate", FAST((guarded<py_evaluate, FastArgs, Py_ssize_t>)), METH_FASTCALL, "evaluate(nodes, device, run, rules)"},
     {"set_rules", FAST(py_set_rules), METH_FASTCALL, "set_rules(run, rules): the package's own."},
-    {"simplify", FAST(py_simplify), METH_FASTCALL, "simplify(sim, roots)"},
+    {"simplify", FAST((guarded<py_simplify, FastArgs, Py_ssize_t>)), METH_FASTCALL, "simplify(sim, roots)"},
     {"copy_rules", py_copy_rules, METH_O, "copy_rules(rules): new Rule objects over new patterns"},
     {"bind", FAST(py_bind), METH_FASTCALL, "bind(handle, MogradError, c_void_p, fallbacks)"},
     {"set_types", FAST(py_set_types), METH_FASTCALL, "set_types(AnyBuffer, Layout)"},
