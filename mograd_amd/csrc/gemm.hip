@@ -10,28 +10,6 @@
 
 namespace mg {
 
-// A x B with A element (m, k) at a[m * sam + k * sak] and B element (k, n) at
-// b[k * sbk + n * sbn]; C row-major (M, N).
-struct GemmArgs {
-  const void* a;
-  const void* b;
-  const void* bias;
-  void* c;
-  int64_t batch, M, N, K;
-  int64_t sam, sak, sbk, sbn;
-  int64_t bsa, bsb;
-  int dtype;
-  // Epilogue (see GemmEpilogue): all optional.
-  const void* residual = nullptr;
-  const void* relu_mask = nullptr;
-  int relu = 0;
-};
-
-template <typename T>
-static GemmEpilogue<T> epilogue_of(const GemmArgs& g) {
-  return GemmEpilogue<T>{static_cast<const T*>(g.residual), static_cast<const T*>(g.relu_mask), g.relu};
-}
-
 static bool mult4(int64_t v) { return (v & 3) == 0; }
 
 // Sums the (splits, batch, M, N) partial products of an fp32 product split along K.
@@ -145,7 +123,8 @@ struct PadCopies {
   // The image of `src`, whose rows then lie `*ld` apart and batches `*batch_stride`.
   int add(const void** src, int64_t batch, int64_t rows, int64_t cols, int64_t* ld, int64_t* batch_stride) {
     constexpr int E = 16 / sizeof(T);
-    const int64_t to = ceil_div(cols, E) * E;
+    // (long rows: whole cache lines, see deep_16bit_us)
+    const int64_t unit = sizeof(T) == 2 && cols >= 2048 ? 64 : E, to = ceil_div(cols, unit) * unit;
     const int64_t images = *batch_stride == 0 ? 1 : batch;
     MG_TRY(mem[count].take(images * rows * to * static_cast<int64_t>(sizeof(T))));
     PadJob<T>& j = jobs.job[count];
@@ -206,13 +185,6 @@ static int launch_f32_direct(const GemmArgs& g, hipStream_t stream) {
 }
 
 static bool mult8(int64_t v) { return (v & 7) == 0; }
-
-// gemm_big.hip: the 256 x 256-tile kernel for large 16-bit products (variant 4ksn: k per step,
-// copies of the tiles).
-int gemm16_big_launch(int dtype, bool a_kc, bool b_kc, int variant, const void* a, const void* b, const void* bias,
-                      void* c, int64_t batch, int M, int N, int K, int64_t lda, int64_t ldb, int64_t bsa, int64_t bsb,
-                      const void* residual, const void* relu_mask, int relu, hipStream_t stream);
-
 // Into how many K ranges a 16-bit product of `blocks` output tiles is split (1: not at all):
 // enough for `wg_per_cu` workgroups per CU, each with at least 256 of K.
 static int splitk_16bit_splits(int64_t blocks, int64_t K, int wg_per_cu) {
@@ -225,28 +197,57 @@ static int splitk_16bit_splits(int64_t blocks, int64_t K, int wg_per_cu) {
   return splits < 1 ? 1 : splits;
 }
 
-// Whether a 16-bit product is done faster with the 64 x 64 tiles of gemm_16bit_small.h than with
-// 128 x 128 ones in `splits128` K ranges, and with how many K ranges of its own (*splits).  Both
-// sides are estimated from what the kernels measured over 80 products of 64 to 16384 rows, 64 to
-// 3768 columns and K 64 to 16384 (within 20 % where either side is close): 3.6 us for a launch and
-// its ends, 0.24 us per step of 64 k of a 64 x 64 tile for each workgroup that a CU has to walk,
-// 0.5 us (0.35 of each where a CU has several) of a 128 x 128 tile; K ranges cost 2.6 us and
-// the partial tiles' way to memory and back at 3.5 TB/s.
-static bool small_16bit_tiles(int64_t M, int64_t N, int64_t K, int64_t batch, int splits128, int* splits) {
-  const double cus = device_info().cu_count;
-  const double steps = std::ceil(static_cast<double>(K) / kSmallBK);
-  auto partials = [](double tiles, int edge) { return 2.6 + tiles * edge * edge * 8.0 / 3.5e6; };
-  const double tiles64 = static_cast<double>(ceil_div(M, kSmallT) * ceil_div(N, kSmallT) * batch);
-  const double tiles128 = static_cast<double>(ceil_div(M, kGemmBM) * ceil_div(N, kGemmBN) * batch) * splits128;
-  const double t128 = 3.6 + steps / splits128 * std::max(0.5, 0.35 * tiles128 / cus) +
-                      (splits128 > 1 ? partials(tiles128, kGemmBM) : 0.0);
-  double best = 1e30;
-  for (int s = 1; s <= 16 && (s == 1 || (tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s) {
-    const double t = 3.6 + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) +
-                     (s > 1 ? partials(tiles64 * s, kSmallT) : 0.0);
-    if (t < best) best = t, *splits = s;
+// What a 16-bit product costs, in us, in workgroups of one kind of tile: `items` of them (K ranges included),
+// each `steps` k-steps of 64.  A CU holds two workgroups of 128-row tiles, whose steps take 0.85 us (128 x
+// 128) and 1.1 us (128 x 192) for the pair, 0.46 and 0.69 us where there is one; a 256 x 256 tile, alone
+// on its CU, 1.47 us (1.3 where CUs stay idle) and 1.5 us until its first MFMA.  `split_lines`: rows of a k-contiguous operand that do not start on
+// cache lines, so that every 128 bytes of a copy are two lines, long enough to matter ((13037, 680) <- 7288: 177 us with 128 x 192
+// tiles, 147 with 256 x 256 ones).  The launch, the last epilogue and writing the result, which the tiles of a round do
+// together, come on top.  (From 40 products of 2048 to 32768 rows, 64 to 8192 columns and K 64 to 7288, most within 10 %.)
+static double deep_16bit_us(Gemm16Tile tile, double items, double steps, bool split_lines) {
+  const double per_cu = std::ceil(items / device_info().cu_count);
+  if (tile == kTile256) return 4.0 + per_cu * ((items < 0.75 * device_info().cu_count ? 1.3 : 1.47) * steps + 1.5);
+  const double pairs = std::floor(per_cu / 2), odd = per_cu - 2 * pairs, f = split_lines ? 1.3 : 1.0;
+  return 3.6 + f * steps * (tile == kTile192 ? 1.1 * pairs + 0.69 * odd : 0.85 * pairs + 0.46 * odd);
+}
+static double partials_us(double values) { return 2.6 + values * 8.0 / 3.5e6; }
+
+// Which tiles a 16-bit product is done fastest with, and in how many K ranges.  kSmall: the 64 x 64 tiles of
+// gemm_16bit_small.h, whose estimate (3.4 us for a launch and its ends, 0.24 us per step for each
+// workgroup that a CU has to walk) comes from 80 products of 64 to 16384 rows, 64 to 3768 columns and K 64 to 16384.
+constexpr int kSmall = 4;
+struct Choice16 {
+  int tile;
+  int splits;
+  double us = 1e30;
+};
+static Choice16 choose_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, bool split_lines) {
+  const double cus = device_info().cu_count, steps = std::ceil(static_cast<double>(K) / kG16BK);
+  const double out = static_cast<double>(M) * N * batch * 2.0 / 5e6;  // (rows off the 16-byte chunks: 0.8 us more in the larger tiles)
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(64, K / env_int("MOGRAD_HIP_GEMM_SPLITK_MIN_K", 256)));
+  auto tiles_of = [&](int m, int n) { return static_cast<double>(ceil_div(M, m) * ceil_div(N, n) * batch); };
+  Choice16 best{kTile128, 1};
+  if (env_str("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU")) {
+    best.splits = splitk_16bit_splits(static_cast<int64_t>(tiles_of(kGemmBM, kGemmBN)), K,
+                                      env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2));
+    return best;
   }
-  return best < t128;
+  auto offer = [&](int tile, int splits, double us) {
+    if (us < best.us) best = Choice16{tile, splits, us};
+  };
+  for (int t = kTile128; t <= kTile256; ++t) {
+    const double tiles = tiles_of(kGemm16TileM[t], kGemm16TileN[t]);
+    for (int s = 1; s <= (t == kTile256 ? 1 : most); ++s) {
+      if (s > 1 && tiles * (s - 1) >= 2 * cus) break;
+      const double us = deep_16bit_us(static_cast<Gemm16Tile>(t), tiles * s, std::ceil(steps / s), split_lines);
+      offer(t, s, us + out + (N % 8 ? 0.8 : 0.0) + (s > 1 ? partials_us(tiles * s * kGemm16TileM[t] * kGemm16TileN[t]) : 0.0));
+    }
+  }
+  const double tiles64 = tiles_of(kSmallT, kSmallT);
+  for (int s = 1; s <= 16 && (s == 1 || (s <= most && tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s)
+    offer(kSmall, s, 3.4 + out + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) +
+                         (s > 1 ? partials_us(tiles64 * s * kSmallT * kSmallT) : 0.0));
+  return best;
 }
 // The K range of one workgroup, a multiple of the k-step, and the number of ranges that leaves.
 static int splitk_16bit_range(int64_t K, int* splits) {
@@ -298,116 +299,57 @@ static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream)
   return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
 }
 
-// 16-bit MFMA path, optionally split along K when the output has too few tiles to fill
-// the device (dW of a narrow layer: reduction over thousands of rows into a small matrix).
-template <typename T, bool A_KC, bool B_KC, bool RAGGED>
-static int launch_16bit_mfma(const GemmArgs& g, hipStream_t stream) {
-  const int tiles_m = static_cast<int>(ceil_div(g.M, kGemmBM));
-  const int tiles_n = static_cast<int>(ceil_div(g.N, kGemmBN));
+// Operands whose tiles cannot be copied straight into LDS (see dispatch_16bit): the register-staged kernel.
+template <typename T, bool A_KC, bool B_KC>
+static int launch_16bit_staged(const GemmArgs& g, int splits, hipStream_t stream) {
+  const int tiles_m = static_cast<int>(ceil_div(g.M, kGemmBM)), tiles_n = static_cast<int>(ceil_div(g.N, kGemmBN));
   const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
-  const int64_t blocks = tiles * g.batch;
-  if (blocks > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
-  const int64_t lda = A_KC ? g.sam : g.sak;
-  const int64_t ldb = B_KC ? g.sbn : g.sbk;
-  const T* a = static_cast<const T*>(g.a);
-  const T* b = static_cast<const T*>(g.b);
-  const T* bias = static_cast<const T*>(g.bias);
-  T* c = static_cast<T*>(g.c);
-  const int M = static_cast<int>(g.M), N = static_cast<int>(g.N), K = static_cast<int>(g.K);
-  const int64_t cus = device_info().cu_count;
-  int splits = splitk_16bit_splits(blocks, g.K, env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2));
-  // Outputs with few tiles: 64 x 64 ones (gemm_16bit_small.h).  Otherwise tiles copied straight into LDS (gemm_16bit_pipe_kernel): an operand that is not k-contiguous is
-  // transposed by the LDS read instead of in registers, and a k-step costs one barrier.  64 k per
-  // step and two copies of the tiles measured fastest or equal at every layout and size swept, 64 to
-  // 16384 rows, 256 to 1536 columns, K 256 to 16384 (32 k per step 5-12 % slower below 16384 rows,
-  // the register-staged kernel 4-40 %).  What the copy cannot take (operands that do not lie on
-  // 16-byte chunks) is the register-staged kernel's, RAGGED.
-  // MOGRAD_HIP_GEMM16_PIPE = 0 | 64 | 322 | 642 | 2322 | 2642 overrides the choice: 0 the register-staged
-  // kernel, 64 the 64 x 64 tiles, else k per step and copies of the tiles (2xxx: 256 x 128 tiles).
-  int pipe = 0;
-  if constexpr (!RAGGED) {
-    // (The K ranges are chosen with the tiles; a kernel that is asked for takes the same ones.)
-    int splits64 = 1;
-    const bool small = !env_str("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU") &&
-                       small_16bit_tiles(g.M, g.N, g.K, g.batch, splits, &splits64);
-    if (small) splits = splits64;
-    pipe = small ? 64 : 642;
-    // Large products: 256 x 128 tiles (eight waves), a quarter fewer operand bytes per FLOP
-    // through L2, once they still give every CU two workgroups (4096^3: 3-11 % faster).
-    if (!small && splits <= 1 && g.K >= 1024 && ceil_div(g.M, 256) * tiles_n * g.batch >= 2 * cus) pipe = 2322;
-    // Products with a 256 x 256 tile for every CU: four waves of 128 x 128 each, one workgroup
-    // per CU (gemm_16bit_big_kernel; 4642: 64 k per step and two copies of the tiles, 4324: 32 k
-    // and four; 4096^3 forward 147 -> 121 us, 8192^3 dW 1016 -> 887 us, bit-identical results).
-    // It takes whole k-steps only.
-    if (!small && splits <= 1 && g.K >= 1024 && g.K % kG16BK == 0 &&
-        ceil_div(g.M, kGemmBigT) * ceil_div(g.N, kGemmBigT) * g.batch >= cus)
-      pipe = 4642;
-    pipe = static_cast<int>(env_int("MOGRAD_HIP_GEMM16_PIPE", pipe));
-  }
-  if constexpr (!RAGGED) {
-    if (pipe == 64) return launch_16bit_small<T, A_KC, B_KC>(g, splits, stream);
-  }
-  if (splits <= 1 && pipe >= 4000 && g.K % kG16BK == 0) {
-    if constexpr (!RAGGED)
-      return gemm16_big_launch(g.dtype, A_KC, B_KC, pipe, g.a, g.b, g.bias, g.c, g.batch, M, N, K, lda, ldb, g.bsa, g.bsb,
-                               g.residual, g.relu_mask, g.relu, stream);
-  }
-  if (pipe >= 4000) pipe = 642;
-#define MG_GEMM16_LAUNCH(BIAS_, SPLIT_, GRID_, PARTIAL_, KPS_, NSPLIT_, EP_)                                                   \
-  do {                                                                                                                 \
-    auto launch = [&](auto kernel) {                                                                                   \
-      hipLaunchKernelGGL(kernel, GRID_, dim3(kGemmThreads), 0, stream, a, b, bias, c, PARTIAL_, M, N, K, lda, ldb, g.N,  \
-                         g.bsa, g.bsb, g.M * g.N, tiles_m, tiles_n, KPS_, NSPLIT_, static_cast<int>(g.batch), EP_);   \
-    };                                                                                                                 \
-    if constexpr (!RAGGED) {                                                                                           \
-      if (pipe == 322) { launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, BIAS_, SPLIT_, 32, 2>); break; }                 \
-      if (pipe == 642) { launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, BIAS_, SPLIT_, 64, 2>); break; }                 \
-    }                                                                                                                  \
-    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, BIAS_, SPLIT_>);                                              \
-  } while (0)
-  if (splits <= 1 && (pipe == 2322 || pipe == 2642)) {
-    // 256 x 128 tiles, eight waves: a quarter fewer operand bytes per FLOP through L2.
-    if constexpr (!RAGGED) {
-      const int tiles_m2 = static_cast<int>(ceil_div(g.M, 256));
-      const dim3 grid2(static_cast<unsigned>(static_cast<int64_t>(tiles_m2) * tiles_n * g.batch));
-      auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid2, dim3(512), 0, stream, a, b, bias, c, static_cast<float*>(nullptr), M, N, K, lda,
-                           ldb, g.N, g.bsa, g.bsb, g.M * g.N, tiles_m2, tiles_n, K, 1, static_cast<int>(g.batch),
-                           epilogue_of<T>(g));
-      };
-      if (pipe == 2322) {
-        if (bias) launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, true, false, 32, 2, 256>);
-        else launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, false, false, 32, 2, 256>);
-      } else {
-        if (bias) launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, true, false, 64, 2, 256>);
-        else launch(gemm_16bit_pipe_kernel<T, A_KC, B_KC, false, false, 64, 2, 256>);
-      }
-      MG_LAUNCH_CHECK();
-      return MG_OK;
-    }
-  }
-  if (pipe > 1000) pipe -= 2000;  // the split-K launch keeps 128 x 128 tiles
-  if (splits <= 1) {
-    const dim3 grid(static_cast<unsigned>(blocks));
-    float* no_partial = nullptr;
-    if (bias) MG_GEMM16_LAUNCH(true, false, grid, no_partial, K, 1, epilogue_of<T>(g));
-    else MG_GEMM16_LAUNCH(false, false, grid, no_partial, K, 1, epilogue_of<T>(g));
-    MG_LAUNCH_CHECK();
-    return MG_OK;
-  }
-  const int k_per_split = splitk_16bit_range(g.K, &splits);
-  // Partial tiles: whole 128 x 128 tiles in accumulator order (gemm16_partial_floats); the
-  // reduction maps them back onto the contiguous (batch, M, N) output.
+  const int k_per_split = splits > 1 ? splitk_16bit_range(g.K, &splits) : static_cast<int>(g.K);
+  const int64_t grid = splits > 1 ? gemm_split_grid(tiles, splits, g.batch) : tiles * g.batch;
+  if (grid > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
   Scratch partial;
-  const int64_t slice = gemm16_partial_floats(g.M, g.N, g.batch, 1);
-  MG_TRY(partial.take(static_cast<int64_t>(splits) * slice * static_cast<int64_t>(sizeof(float))));
-  const int64_t split_grid = gemm_split_grid(tiles, splits, g.batch);
-  if (split_grid > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
-  const dim3 grid(static_cast<unsigned>(split_grid));
-  MG_GEMM16_LAUNCH(false, true, grid, partial.as<float>(), k_per_split, splits, (GemmEpilogue<T>{nullptr, nullptr, 0}));
-#undef MG_GEMM16_LAUNCH
+  if (splits > 1)
+    MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
+  auto launch = [&](auto kernel, GemmEpilogue<T> ep) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kGemmThreads), 0, stream, static_cast<const T*>(g.a),
+                       static_cast<const T*>(g.b), static_cast<const T*>(g.bias), static_cast<T*>(g.c), partial.as<float>(),
+                       static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K), A_KC ? g.sam : g.sak,
+                       B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb, g.M * g.N, tiles_m, tiles_n, k_per_split, splits,
+                       static_cast<int>(g.batch), ep);
+  };
+  if (splits > 1) launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, true>, GemmEpilogue<T>{nullptr, nullptr, 0});
+  else if (g.bias) launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, true, false>, epilogue_of<T>(g));
+  else launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, false>, epilogue_of<T>(g));
   MG_LAUNCH_CHECK();
-  return launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream);
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
+}
+
+// 16-bit MFMA path, split along K where the output has too few tiles to fill the device (dW of a narrow
+// layer: reduction over thousands of rows into a small matrix).  `wide`: operands on 16-byte chunks.
+// MOGRAD_HIP_GEMM16_PIPE overrides the choice of tiles: 0 the register-staged kernel, 64 the 64 x 64 tiles,
+// 1 to 1999 the 128 x 128, 2xxx the 128 x 192, 4xxx the 256 x 256 ones.  (The K ranges are
+// chosen with the tiles; a kernel that is asked for takes the same ones.)
+template <typename T, bool A_KC, bool B_KC>
+static int launch_16bit(const GemmArgs& g, bool wide, hipStream_t stream) {
+  const int64_t tiles128 = ceil_div(g.M, kGemmBM) * ceil_div(g.N, kGemmBN) * g.batch;
+  const int64_t lda = A_KC ? g.sam : g.sak, ldb = B_KC ? g.sbn : g.sbk;
+  if (!wide)
+    return launch_16bit_staged<T, A_KC, B_KC>(
+        g, splitk_16bit_splits(tiles128, g.K, env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2)), stream);
+  Choice16 choice = choose_16bit(g.M, g.N, g.K, g.batch, g.K >= 1024 && ((A_KC && lda % 64 != 0) || (B_KC && ldb % 64 != 0)));
+  if (const int64_t pipe = env_int("MOGRAD_HIP_GEMM16_PIPE", -1); pipe >= 0) {
+    choice.tile = pipe == 0 ? -1 : pipe == 64 ? kSmall : pipe < 2000 ? kTile128 : pipe < 4000 ? kTile192 : kTile256;
+    if (choice.tile == kTile256 && choice.splits > 1) choice.tile = kTile128;
+  }
+  if (choice.tile == kSmall) return launch_16bit_small<T, A_KC, B_KC>(g, choice.splits, stream);
+  if (choice.tile < 0 || std::max(lda, ldb) > kGemmDeepMaxLd) return launch_16bit_staged<T, A_KC, B_KC>(g, choice.splits, stream);
+  int splits = choice.splits;
+  const int k_per_split = splits > 1 ? splitk_16bit_range(g.K, &splits) : static_cast<int>(g.K);
+  Scratch partial;  // whole 128 x 128 tiles in accumulator order; the reduction maps them back onto the output
+  if (splits > 1)
+    MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
+  MG_TRY(launch_16bit_deep<T>(g, static_cast<Gemm16Tile>(choice.tile), splits, k_per_split, partial.as<float>(), stream));
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
 }
 
 static bool generic_grid_fits(const GemmArgs& g) { return ceil_div(g.M, 64) <= 65535 && g.batch <= 65535; }
@@ -509,16 +451,10 @@ static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handle
     MG_TRY(pad.launch(stream));
     wide = true;
   }
-  if (wide) {
-    if (a_kc && b_kc) return launch_16bit_mfma<T, true, true, false>(g, stream);
-    if (a_kc) return launch_16bit_mfma<T, true, false, false>(g, stream);
-    if (b_kc) return launch_16bit_mfma<T, false, true, false>(g, stream);
-    return launch_16bit_mfma<T, false, false, false>(g, stream);
-  }
-  if (a_kc && b_kc) return launch_16bit_mfma<T, true, true, true>(g, stream);
-  if (a_kc) return launch_16bit_mfma<T, true, false, true>(g, stream);
-  if (b_kc) return launch_16bit_mfma<T, false, true, true>(g, stream);
-  return launch_16bit_mfma<T, false, false, true>(g, stream);
+  if (a_kc && b_kc) return launch_16bit<T, true, true>(g, wide, stream);
+  if (a_kc) return launch_16bit<T, true, false>(g, wide, stream);
+  if (b_kc) return launch_16bit<T, false, true>(g, wide, stream);
+  return launch_16bit<T, false, false>(g, wide, stream);
 }
 
 template <typename T>
@@ -598,16 +534,15 @@ int ln_bwd(const void* dy, const void* x, const void* gamma, const float* mean, 
            mg_stream stream);  // layer_norm.hip
 
 // dX (M,K) = dY (M,N) W (N,K) and dW (N,K) = dY^T X of a 16-bit Linear layer in one launch
-// (linear_bwd_16bit_kernel), for the shapes at which launch_16bit_mfma would give both the
-// pipelined kernel with 32 k per step and split dW along the rows.  dW comes out bit for bit
+// (linear_bwd_16bit_kernel), dW split along the rows.  dW comes out bit for bit
 // as from its own launch with the same number of K ranges, and so does dX unless its own launch would split it along N (fewer
 // dX tiles than CUs): here dX is never split, the dW workgroups fill the device.
 // *done = false: not such a shape, nothing launched.
 // MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH=0 switches it off (benchmarks, tests of the equivalence).
-// With `ln`, the launch's dX tiles continue as the backward of the LayerNorm whose output X is
-// (linear_bwd_ln_16bit_kernel): `dx` then receives that LayerNorm's input gradient (added to
+// With `ln`, the launch's dX tiles continue as the backward of the LayerNorm whose output X is:
+// `dx` then receives that LayerNorm's input gradient (added to
 // what it holds when dx_accumulate), dY W itself is not stored, and the LayerNorm's dgamma and
-// dbeta follow from one partial row per tile of 128 rows.  Only for the wide tiles of a
+// dbeta follow from one partial row per tile of 128 rows.  Only for the 128 x 384 tiles of a
 // 384-wide input (K == 384); otherwise *done stays false.
 struct LinearBwdLayerNorm {
   const void* x;       // the LayerNorm's input (M, K)
@@ -618,53 +553,71 @@ struct LinearBwdLayerNorm {
   void* dbeta;
 };
 
-// Input widths that are multiples of 384 can take 128 x 384 output tiles (twelve waves, one
-// workgroup per CU): the three column tiles of a row block share one copy of the dY tile,
-// a third fewer bytes from L2 per FLOP.  Taken when those tiles leave CUs free for dW's K ranges, so
-// that the whole launch is one workgroup per CU, and the layer is wide enough to pay for
-// the larger partial tiles.  MOGRAD_HIP_LINEAR_BWD_WIDE=0: 128 x 128 tiles.
+// Inputs of 384 columns can take 128 x 384 output tiles, which hold whole rows of dX (eight waves, one workgroup
+// per CU): taken for the LayerNorm backward that continues in them, when those tiles leave CUs free for dW's K ranges and
+// the layer is wide enough.  dW's K ranges are then those of that launch, with and without the LayerNorm.
+// MOGRAD_HIP_LINEAR_BWD_WIDE=0: as any other width, with the K ranges that dW has in a launch of its own.
 static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
-  return K % kGemmWideBN == 0 && ceil_div(M, kGemmBM) * (K / kGemmWideBN) < device_info().cu_count && N >= 768 &&
+  return K == kGemm16TileN[kTileWide] && ceil_div(M, kGemmBM) < device_info().cu_count && N >= 768 &&
          env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) != 0;
 }
 
-// Whether the backward of a 16-bit layer takes 64 x 64 tiles (gemm_16bit_small.h), and into how many K
-// ranges dW is then cut: the fewest that keep dW's walk along the rows well inside the rest;
-// more than one costs 3.6 us and the partial tiles' way to memory and back.
-// The larger tiles' lower LDS traffic wins once all steps together outweigh the tails and
-// padding that come with them (0.3 us per step of 64 k and CU against 0.9 us for four times the
-// output): (1024, 1024 <- 1024) 22.8 -> 11.3 us, (2587, 768 <- 256) 17.8 -> 12.7,
-// (9455, 4568 <- 64) 61 -> 37, but (3094, 1704 <- 776) 36 against 48 and (16384, 384 <- 384) 24
-// against 26.  The 128 x 384 tiles are one round of workgroups that walk the layer's outputs, 1.4 us
-// a step whatever the number of rows ((2048, 1152 <- 384) 32 us against 15, (2048, 3072 <- 768) 71
-// against 38, (8192, 1152 <- 384) 36 against 32); for 384 columns they can carry the LayerNorm
-// backward, which is 6 us as a launch of its own.
+// How the backward of a 16-bit layer goes out in one launch: with which tiles, and dW in how many K ranges.
+// Both products' k-steps (of 64) are dealt over the CUs; the longest chain of them in one workgroup is what a launch lasts at least.
+// For the 64 x 64 tiles of gemm_16bit_small.h: 3.1 us, 0.235 us per step; K ranges cost 3.1 us and 0.0082 us a
+// tile.  For the 128-row tiles as in deep_16bit_us, a chain's steps between the two figures there (it shares its
+// CU for a part of its life).  A range has at least 256 rows.  tile < 0: no such launch.
 // MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
-static bool small_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx, int* splits) {
+static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx) {
   const double cus = device_info().cu_count;
-  auto steps_per_cu = [&](int64_t tile) {  // of 64 k
-    return static_cast<double>(ceil_div(N, tile) * ceil_div(K, tile) * ceil_div(M, kSmallBK) +
-                               (with_dx ? ceil_div(M, tile) * ceil_div(K, tile) * ceil_div(N, kSmallBK) : 0)) / cus;
-  };
-  const double steps_w = static_cast<double>(ceil_div(M, kSmallBK)), steps_x = static_cast<double>(ceil_div(N, kSmallBK));
-  const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
-  const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0;
-  const double chain_x = with_dx ? steps_x : 0.0, load = steps_per_cu(kSmallT);
-  double best = 1e30;
-  for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
-    double chain = std::max(steps_w / s, chain_x);
-    if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + chain_x));  // two share a CU
-    const double t = 3.6 + 0.27 * std::max(1.5 * chain, load) + (s > 1 ? 3.6 + tiles_w * s * 0.0094 : 0.0);
-    if (t < best) best = t, *splits = s;
+  const double steps_w = static_cast<double>(ceil_div(M, kG16BK)), steps_x = static_cast<double>(ceil_div(N, kG16BK));
+  Choice16 small{kSmall, 1};
+  {
+    const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
+    const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0;
+    const double chain_x = with_dx ? steps_x : 0.0, load = (tiles_w * steps_w + tiles_x * steps_x) / cus;
+    for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
+      double chain = std::max(steps_w / s, chain_x);
+      if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + chain_x));  // two share a CU
+      if (tiles_w * s > 2 * cus) chain = std::max(chain, 0.67 * (tiles_w * steps_w / cus + 2 * chain_x));  // dX starts last
+      const double t = 3.1 + 0.235 * std::max(1.5 * chain, load) + (s > 1 ? 3.1 + tiles_w * s * 0.0082 : 0.0) +
+                       static_cast<double>(M) * K * 2.0 / 5e6;
+      if (t < small.us) small.us = t, small.splits = s;
+    }
+    small.splits = static_cast<int>(env_int("MOGRAD_HIP_LINEAR_BWD_SPLITS", small.splits));
   }
-  *splits = static_cast<int>(env_int("MOGRAD_HIP_LINEAR_BWD_SPLITS", *splits));
-  bool small;
-  if (wide_linear_bwd(M, N, K))
-    small = best + (K == kGemmWideBN ? 6.0 : 0.0) <= 10.0 + 1.4 * steps_x;
-  else  // (few rows: the larger tiles would take a launch for each product)
-    small = 0.3 * load <= (M < 1024 ? 9.0 : 4.0) + 0.9 * steps_per_cu(kGemmBM);
+  Choice16 deep{-1, 1};
+  const int most = static_cast<int>(std::min<int64_t>(64, M / 256));
+  auto offer = [&](Gemm16Tile t, int s) {
+    const double tiles_k = static_cast<double>(ceil_div(K, kGemm16TileN[t]));
+    const double tiles_w = static_cast<double>(ceil_div(N, kGemmBM)) * tiles_k * s, tiles_x = static_cast<double>(ceil_div(M, kGemmBM)) * tiles_k;
+    const double len = std::ceil(steps_w / s), pair = t == kTile192 ? 1.1 : t == kTileWide ? 2.2 : 0.85, one = t == kTile192 ? 0.69 : t == kTileWide ? 2.2 : 0.46;
+    const double slots = t == kTileWide ? cus : 2 * cus;
+    const double load = (tiles_w * len + tiles_x * steps_x) / slots * pair;
+    const double chain = std::max(len, steps_x) * 0.5 * (pair + one);
+    const double us = 3.6 + std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0) +
+                      static_cast<double>(M) * K * 2.0 / 5e6 + partials_us(tiles_w * kGemmBM * kGemm16TileN[t]);
+    if (us < deep.us) deep = Choice16{t, s, us};
+  };
+  if (!with_dx || ceil_div(N, kGemmBM) * ceil_div(K, kGemmBN) >= cus) {  // dW fills the device unsplit: a launch for each product
+  } else if (env_str("MOGRAD_HIP_LINEAR_BWD_WIDE") && env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) == 0) {
+    const Gemm16Tile t = K % 192 == 0 ? kTile192 : kTile128;
+    const int s = splitk_16bit_splits(ceil_div(N, kGemmBM) * ceil_div(K, kGemmBN), M, 1);
+    if (s > 1) offer(t, s);
+  } else if (wide_linear_bwd(M, N, K)) {
+    for (int s = 2; s <= most; ++s) offer(kTileWide, s);
+  } else {
+    const int64_t only = env_int("MOGRAD_HIP_LINEAR_BWD_TILE", 0);  // 128 | 192
+    for (int s = 2; s <= most; ++s) {
+      if (only != 192) offer(kTile128, s);
+      if (only != 128) offer(kTile192, s);
+    }
+  }
+  // (a launch of its own for each product; the LayerNorm's backward is 6 us as one)
+  if (deep.tile < 0) deep.us = choose_16bit(N, K, M, 1, false).us + (with_dx ? choose_16bit(M, K, N, 1, N >= 1024 && N % 64 != 0).us : 0.0);
+  const bool is_small = small.us + (deep.tile == kTileWide ? 6.0 : 0.0) <= deep.us;
   // (A choice of the larger tiles' form is also one for them.)
-  return env_int("MOGRAD_HIP_LINEAR_BWD_SMALL", small && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE")) != 0;
+  return env_int("MOGRAD_HIP_LINEAR_BWD_SMALL", is_small && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE")) != 0 ? small : deep;
 }
 
 template <typename T>
@@ -680,47 +633,26 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   // rows of the next multiple of 8, zeros behind (`pads` below); dX, dW and db keep their shape.
   const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || (dx && !aligned16(w));
   const int64_t cus = device_info().cu_count;
-  int splits = 1;
-  const bool small = small_linear_bwd(M, N, K, dx != nullptr, &splits);
-  if (!dx && !small) return MG_OK;
-  const bool wide = !small && wide_linear_bwd(M, N, K);
-  if (ln && (!wide || K != kGemmWideBN || relu_mask || env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3 ||
-             pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx)))
-    return MG_OK;
+  const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr);
+  if (choice.tile < 0) return MG_OK;
+  const bool small = choice.tile == kSmall, wide = choice.tile == kTileWide;
+  if (ln && (!wide || relu_mask || pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx))) return MG_OK;
+  // (without the LayerNorm the same K ranges in 128 x 192 tiles, two workgroups per CU)
+  const Gemm16Tile deep = wide && !ln ? kTile192 : static_cast<Gemm16Tile>(small ? kTile128 : choice.tile);
   const int tile = small ? kSmallT : kGemmBM;  // rows of an output tile
-  const int tiles_kk = static_cast<int>(ceil_div(K, small ? kSmallT : wide ? kGemmWideBN : kGemmBN));
-  // dW: must be split, each workgroup's rows short enough for the 32-k variant.
+  const int tiles_kk = static_cast<int>(ceil_div(K, small ? kSmallT : kGemm16TileN[deep]));
   const int w_tiles_m = static_cast<int>(ceil_div(N, tile));
   const int64_t w_tiles = static_cast<int64_t>(w_tiles_m) * tiles_kk;
   const int x_tiles_m = static_cast<int>(ceil_div(M, tile));
   const int64_t x_tiles = dx ? static_cast<int64_t>(x_tiles_m) * tiles_kk : 0;  // (a first layer's dX is not wanted)
-  if (small) {
-  } else if (wide) {
-    // Every workgroup step is the same work (a 128 x 384 x 32 product), so the K ranges of dW
-    // are cut to what a CU's share of all steps comes to: with fewer dX tiles than CUs the
-    // ranges take the CUs that the tiles leave free, all in one round; otherwise the ranges
-    // start first and the tiles fill in behind them.
-    const int64_t steps_w = M / kG16BK, steps_x = N / kG16BK;
-    const int64_t share = ceil_div(x_tiles * steps_x + w_tiles * steps_w, cus);
-    int64_t want = x_tiles < cus ? (cus - x_tiles) / w_tiles : 0;
-    if (want < 2) want = ceil_div(steps_w, share);
-    const int64_t most = std::min<int64_t>(64, M / 256);
-    splits = static_cast<int>(std::max<int64_t>(1, std::min(want, most)));
-  } else {
-    // One workgroup per CU is enough here: the dX tiles fill the rest of the device, and half
-    // the K ranges are half the partial tiles to write and sum (GPT step 3.06 -> 3.00 ms).
-    splits = splitk_16bit_splits(w_tiles, M, env_int("MOGRAD_HIP_LINEAR_BWD_SPLIT_WG_PER_CU", 1));
-  }
+  int splits = choice.splits;
   const bool split_sums = splits > 1 || !small;
-  if (!small && splits <= 1) return MG_OK;
-  if (ceil_div(M, splits) >= 4096) return MG_OK;
   const int k_per_split = splits > 1 ? splitk_16bit_range(M, &splits) : static_cast<int>(M);
-  // dX, which is never split here: not a long reduction, and none that another split would serve better.
-  if (!small && (N >= 4096 || (N >= 1024 && (M < 1024 || ceil_div(M, 256) * tiles_kk >= 2 * cus)))) return MG_OK;
   const int64_t n_dw = split_sums ? gemm_split_grid(w_tiles, splits, 1) : w_tiles;
   if (n_dw + x_tiles > 0x7fffffffLL) return MG_OK;
 
   int64_t ldy = N, ldx = K, ldw = K;
+  if (!small && std::max(N, K) + 8 > kGemmDeepMaxLd) return MG_OK;
   PadCopies<T> pads;
   int64_t no_batch = 0;
   if (pad_n) MG_TRY(pads.add(&dy, 1, M, N, &ldy, &no_batch));
@@ -777,9 +709,6 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
     MG_TRY(db_part.take(static_cast<int64_t>(groups) * N * static_cast<int64_t>(sizeof(float))));
     pw2.colsum_part = db_part.as<float>();
   }
-  // Three copies of the tiles (two k-steps in flight per workgroup, three workgroups per CU)
-  // measured 1 % faster on the GPT step than two copies and four workgroups; four copies no
-  // better than two.  MOGRAD_HIP_LINEAR_BWD_STAGES=2 selects two.
   Scratch ln_part_g, ln_part_b;
   if (ln) {
     MG_TRY(ln_part_g.take(static_cast<int64_t>(x_tiles_m) * K * static_cast<int64_t>(sizeof(float))));
@@ -787,24 +716,14 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
     Gemm16Problem<T> px2 = px;
     px2.ln = Gemm16LayerNormBwd<T>{static_cast<const T*>(ln->x), static_cast<const T*>(ln->gamma), ln->mean, ln->rstd,
                                    ln_part_g.as<float>(), ln_part_b.as<float>()};
-    hipLaunchKernelGGL((linear_bwd_ln_16bit_kernel<T>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(2 * kGemmWideBN),
-                       0, stream, pw2, px2, static_cast<int>(n_dw));
-  } else if (small)
+    MG_TRY(launch_linear_bwd_deep<T>(pw2, px2, kTileWide, n_dw, x_tiles, stream));
+  } else if (small) {
     hipLaunchKernelGGL((linear_bwd_small_16bit_kernel<T, true>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
                        dim3(kGemmThreads), 0, stream, pw2, px, static_cast<int>(n_dw));
-  else if (wide && env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 2) == 3)  // 32 k per step, three copies: 3-4 % slower
-    hipLaunchKernelGGL((linear_bwd_16bit_kernel<T, 3, kGemmWideBN>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
-                       dim3(2 * kGemmWideBN), 0, stream, pw2, px, static_cast<int>(n_dw));
-  else if (wide)  // 64 k per step, two copies (128 KB of LDS): half the barriers, whole cache lines of dY
-    hipLaunchKernelGGL((linear_bwd_16bit_kernel<T, 2, kGemmWideBN, 64>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
-                       dim3(2 * kGemmWideBN), 0, stream, pw2, px, static_cast<int>(n_dw));
-  else if (env_int("MOGRAD_HIP_LINEAR_BWD_STAGES", 3) == 2)
-    hipLaunchKernelGGL((linear_bwd_16bit_kernel<T, 2>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(kGemmThreads), 0,
-                       stream, pw2, px, static_cast<int>(n_dw));
-  else
-    hipLaunchKernelGGL((linear_bwd_16bit_kernel<T, 3>), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(kGemmThreads), 0,
-                       stream, pw2, px, static_cast<int>(n_dw));
-  MG_LAUNCH_CHECK();
+    MG_LAUNCH_CHECK();
+  } else {
+    MG_TRY(launch_linear_bwd_deep<T>(pw2, px, deep, n_dw, x_tiles, stream));
+  }
   if (ln) {  // the tiles' partial rows of dgamma / dbeta: summed now, or left on the deferred list
     reduce_partials_or_defer<T>(ln_part_g, static_cast<T*>(ln->dgamma), &ln_part_b, static_cast<T*>(ln->dbeta), x_tiles_m,
                                 K, static_cast<int>(cus), stream);

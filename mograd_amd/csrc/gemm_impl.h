@@ -79,6 +79,28 @@ struct GemmEpilogue {
   int relu;
 };
 
+// A x B with A element (m, k) at a[m * sam + k * sak] and B element (k, n) at
+// b[k * sbk + n * sbn]; C row-major (M, N).
+struct GemmArgs {
+  const void* a;
+  const void* b;
+  const void* bias;
+  void* c;
+  int64_t batch, M, N, K;
+  int64_t sam, sak, sbk, sbn;
+  int64_t bsa, bsb;
+  int dtype;
+  // Epilogue (see GemmEpilogue): all optional.
+  const void* residual = nullptr;
+  const void* relu_mask = nullptr;
+  int relu = 0;
+};
+
+template <typename T>
+inline GemmEpilogue<T> epilogue_of(const GemmArgs& g) {
+  return GemmEpilogue<T>{static_cast<const T*>(g.residual), static_cast<const T*>(g.relu_mask), g.relu};
+}
+
 template <typename T>
 __device__ __forceinline__ T gemm_finish(float v, const GemmEpilogue<T>& ep, int64_t index) {
   if (ep.relu) v = v > 0.f ? v : 0.f;
@@ -219,7 +241,6 @@ constexpr int kG16Stride = kG16BK + 8;  // elements per LDS row: 144 bytes, 16-b
 // of the tile.  Tiles are stored whole; rows and columns past the matrix hold whatever the
 // clamped operand rows produced and are dropped by the reduction.
 constexpr int kG16PartialTile = kGemmBM * kGemmBN;
-constexpr int kGemmWideBN = 384;  // columns of the wide tile of linear_bwd_16bit_kernel
 inline int64_t gemm16_partial_floats(int64_t M, int64_t N, int64_t batches, int64_t splits) {
   return splits * batches * ((M + kGemmBM - 1) / kGemmBM) * ((N + kGemmBN - 1) / kGemmBN) * kG16PartialTile;
 }
@@ -486,7 +507,7 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
   }
 }
 
-// What a product's output tile needs to continue as a LayerNorm backward (see gemm16_ln_bwd_tile).
+// What a product's output tile needs to continue as a LayerNorm backward (see gemm16_deep_ln_bwd).
 template <typename T>
 struct Gemm16LayerNormBwd {
   const T* x = nullptr;         // the LayerNorm's input, laid out like the product's output
@@ -496,142 +517,6 @@ struct Gemm16LayerNormBwd {
   float* part_g = nullptr;      // (row tiles, cols) partial column sums of dy * xhat and of dy
   float* part_b = nullptr;
 };
-
-// Output of a 128 x (64 WN) tile whose rows are whole rows of the result (N = 64 WN), when the
-// result dY is only wanted as the upstream of a LayerNorm backward: the tile is staged in LDS
-// as the rounded 16-bit values a store would have written, and the workgroup then computes,
-// from LDS and the matching rows of the LayerNorm's input x,
-//   dx = rstd (dY gamma - mean_n(dY gamma) - xhat mean_n(dY gamma xhat)),  xhat = (x - mean) rstd,
-// written to C as round(dx) (+ the residual, as the separate kernels give it), and the tile's
-// column sums of dY xhat and dY as one row of part_g / part_b.  dY itself never reaches memory.
-// A lane owns 8 columns of rows rl0 + 8 i of its wave's 64 x 64 tile (the layout of the plain
-// store); a row's sums go over the 8 lanes of its 64 columns by DPP and over the WN waves that
-// share the row through LDS, in a fixed order, and the column sums over the 8 row lanes by
-// shuffles and over the two row waves through LDS.  `free_lds` is LDS behind the waves' strips:
-// 128 * WN * 8 bytes for the row sums and 2 * 64 * WN * 8 for the column sums.
-template <typename T, int WN>
-__device__ __forceinline__ void gemm16_ln_bwd_tile(const floatx16 (&acc)[2][2], uint16_t* __restrict__ mine,
-                                                   float* __restrict__ free_lds, T* C, int M, int64_t ldc, int tile_m,
-                                                   int m0, int wm, int wn, int lane, const T* residual,
-                                                   const Gemm16LayerNormBwd<T>& ln) {  // residual may be C itself
-  constexpr int COLS = 64 * WN;
-  {  // the staging of gemm16_write_tile (no bias, no ReLU)
-    const int odd = lane & 1;
-    const uint32_t select = odd ? 0x03020706u : 0x05040100u;
-    uint32_t* const base32 = reinterpret_cast<uint32_t*>(mine + ((lane / 32) * 4 + odd) * kG16Stride + (lane % 32 - odd));
-#pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-      for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-        for (int rp = 0; rp < 8; ++rp) {
-          const uint32_t w = gemm16_pack2<T>(acc[ti][tj][2 * rp], acc[ti][tj][2 * rp + 1]);
-          const uint32_t y = __builtin_amdgcn_update_dpp(w, w, kDppQuadXor1, 0xf, 0xf, false);
-          const int rl = ti * 32 + (rp / 2) * 8 + (rp % 2) * 2;
-          base32[(rl * kG16Stride + tj * 32) / 2] = __builtin_amdgcn_perm(y, w, select);
-        }
-  }
-  float2* row_sums = reinterpret_cast<float2*>(free_lds);               // [128][WN]
-  float* col_sums = free_lds + 128 * WN * 2;                             // [2 row waves][which][COLS]
-  const int rl0 = lane / 8, ch = lane % 8;
-  const int col = wn + ch * 8;
-  const uint16_t* src = mine + rl0 * kG16Stride + ch * 8;
-  float gam[8];
-  VecIO<T, 8>::load(ln.gamma + col, gam);
-  uint4 xraw[8], rraw[8];
-  float mu[8], rs[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = min(m0 + wm + rl0 + 8 * i, M - 1);  // rows past the end: computed, never stored or summed
-    const int64_t at = static_cast<int64_t>(row) * ldc + col;
-    xraw[i] = *reinterpret_cast<const uint4*>(ln.x + at);
-    rraw[i] = residual ? *reinterpret_cast<const uint4*>(residual + at) : make_uint4(0, 0, 0, 0);
-    mu[i] = ln.mean[row];
-    rs[i] = ln.rstd[row];
-  }
-  __syncthreads();  // the strips are complete
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float dy[8], xv[8];
-    VecIO<T, 8>::load(reinterpret_cast<const T*>(src + i * 8 * kG16Stride), dy);
-    VecIO<T, 8>::load(reinterpret_cast<const T*>(&xraw[i]), xv);
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float xhat = (xv[e] - mu[i]) * rs[i];
-      const float dyg = dy[e] * gam[e];
-      s0 += dyg;
-      s1 += dyg * xhat;
-    }
-    s0 += dpp_move<kDppQuadXor1>(s0);
-    s1 += dpp_move<kDppQuadXor1>(s1);
-    s0 += dpp_move<kDppQuadXor2>(s0);
-    s1 += dpp_move<kDppQuadXor2>(s1);
-    s0 += dpp_move<kDppRowHalfMirror>(s0);
-    s1 += dpp_move<kDppRowHalfMirror>(s1);
-    if (ch == 0) row_sums[(wm + rl0 + 8 * i) * WN + wn / 64] = make_float2(s0, s1);
-  }
-  __syncthreads();
-  const float inv_n = 1.0f / static_cast<float>(COLS);
-  float acc_g[8], acc_b[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) acc_g[e] = acc_b[e] = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = m0 + wm + rl0 + 8 * i;
-    float c1 = 0.f, c2 = 0.f;
-#pragma unroll
-    for (int w = 0; w < WN; ++w) {
-      const float2 p = row_sums[(wm + rl0 + 8 * i) * WN + w];
-      c1 += p.x;
-      c2 += p.y;
-    }
-    c1 *= inv_n;
-    c2 *= inv_n;
-    float dy[8], xv[8], rv[8], out[8];
-    VecIO<T, 8>::load(reinterpret_cast<const T*>(src + i * 8 * kG16Stride), dy);
-    VecIO<T, 8>::load(reinterpret_cast<const T*>(&xraw[i]), xv);
-    VecIO<T, 8>::load(reinterpret_cast<const T*>(&rraw[i]), rv);
-    const bool ok = row < M;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float xhat = (xv[e] - mu[i]) * rs[i];
-      const float d = ok ? dy[e] : 0.f;
-      out[e] = rs[i] * (d * gam[e] - c1 - xhat * c2);
-      acc_g[e] += d * xhat;
-      acc_b[e] += d;
-    }
-    if (residual) {
-      // round(gradient) + residual: a plain addition, as the separate add performs it
-#pragma clang fp contract(off)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = to_float(from_float<T>(out[e])) + rv[e];
-    }
-    if (ok) VecIO<T, 8>::store(C + static_cast<int64_t>(row) * ldc + col, out);
-  }
-  // column sums over the wave's 64 rows: the 8 lanes with this lane's columns
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-#pragma unroll
-    for (int w = 8; w < kWave; w *= 2) {
-      acc_g[e] += __shfl_xor(acc_g[e], w);
-      acc_b[e] += __shfl_xor(acc_b[e], w);
-    }
-  }
-  if (rl0 == 0) {
-    float* mine_g = col_sums + (wm / 64) * 2 * COLS + col;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      mine_g[e] = acc_g[e];
-      mine_g[COLS + e] = acc_b[e];
-    }
-  }
-  __syncthreads();
-  for (int c = threadIdx.x; c < COLS; c += blockDim.x) {
-    ln.part_g[static_cast<int64_t>(tile_m) * COLS + c] = col_sums[c] + col_sums[2 * COLS + c];
-    ln.part_b[static_cast<int64_t>(tile_m) * COLS + c] = col_sums[COLS + c] + col_sums[3 * COLS + c];
-  }
-}
 
 template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
@@ -712,22 +597,19 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
 }
 
 // ------------------------------------------------------------------------------------
-// The same product with the tiles copied global memory -> LDS by the memory pipeline itself
-// (`global_load_lds_dwordx4`: every lane names a 16-byte source, the wave's 64 chunks land
-// back to back at an LDS address common to the wave), NSTAGE k-steps deep.  No registers
-// hold data in flight, so several steps' loads are outstanding while one step is multiplied:
-// what short-K products at a few hundred FLOP per byte need, being bound by memory latency
-// and not by the matrix cores.  Operands as above, all extents and strides multiples of 8
-// elements, K (and every K split) a multiple of 64.
+// Tiles copied global memory -> LDS by the memory pipeline itself (`global_load_lds_dwordx4`: every
+// lane names a 16-byte source, the wave's 64 chunks land back to back at an LDS address common to the
+// wave), several k-steps ahead: what the kernels of gemm_16bit_deep.h (output tiles of 128 x 128 to 256 x 256)
+// and gemm_16bit_small.h (64 x 64) share.  No registers hold data in flight.  Operands as above, all
+// extents and strides multiples of 8 elements, every K split a multiple of 64.
 //
-// LDS image of one operand's step, chosen per 16-byte chunk by which source chunk each lane
+// LDS image of one operand's step of 64 k, chosen per 16-byte chunk by which source chunk each lane
 // names (64 banks of four bytes; a 128-bit read is served 16 lanes per clock):
-//   k-contiguous, 64 k per step: [128 rows][8 chunks], chunk c of row r at position
-//     c ^ (r/2 % 8), with 32 k per step [128 rows][4 chunks] and c ^ (r/4 % 4): the sixteen
+//   k-contiguous: [rows][8 chunks], chunk c of row r at position c ^ (r/2 % 8): the sixteen
 //     consecutive rows of a fragment read then hit sixteen different 16-byte bank groups
 //     (timed on the device: 18.5-18.7 clocks per read with four waves reading, as for
 //     consecutive addresses; 32 with c ^ (r % 8));
-//   otherwise: [k][16 chunks of 8 rows], chunk c of k-row kk at position
+//   otherwise: [k][rows / 8 chunks], chunk c of k-row kk at position
 //     c ^ gemm16_tr_swizzle(kk), read with `ds_read_b64_tr_b16` (within 16 lanes, lane i supplies
 //     the four elements 4*i .. 4*i+3 of a 4 x 16 block and receives column i), which turns
 //     four k-rows of 16 consecutive rows into each lane's four consecutive k.
@@ -848,19 +730,6 @@ __device__ __forceinline__ uint4 gemm16_pipe_frag(const char* __restrict__ lds_s
 // 15:14, expcnt 6:4 and lgkmcnt 11:8 left at "no wait").
 #define MG_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0f70)
 
-// LDS of the pipelined kernel (TM = rows of the A tile: 128 with four waves, 256 with eight) and
-// the workgroups that fit a CU, by LDS (160 KB) and by the register file.
-constexpr int gemm16_pipe_lds_bytes(int bk, int nstage, int tm, int tn = 128) {
-  const int stages = nstage * (tm + tn) * bk * 2;
-  const int out = (tm / 64) * (tn / 64) * 64 * kG16Stride * 2;  // every wave transposes its output tile here
-  return stages > out ? stages : out;
-}
-constexpr int gemm16_pipe_occupancy(int bk, int nstage, int tm, int tn = 128) {
-  const int by_lds = 160 * 1024 / gemm16_pipe_lds_bytes(bk, nstage, tm, tn);
-  const int by_regs = 16 / ((tm / 64) * (tn / 64));  // four waves per SIMD at most
-  return by_lds < 1 ? 1 : (by_lds > by_regs ? by_regs : by_lds);
-}
-
 // One product's arguments, as the kernels below take them.
 template <typename T>
 struct Gemm16Problem {
@@ -884,405 +753,22 @@ struct Gemm16Problem {
   // The partial tiles are read back much later (their sum is deferred to the end of a training
   // step): store them past the caches.
   bool partial_stream = false;
-  // The output continues as a LayerNorm backward inside the launch (gemm16_pipe_block<.., LN_BWD>).
+  // The output continues as a LayerNorm backward inside the launch (gemm16_deep_ln_bwd).
   Gemm16LayerNormBwd<T> ln;
 };
 
-// The work of workgroup `bid` of a launch for one product; `lds` is the workgroup's
-// gemm16_pipe_lds_bytes(BK, NSTAGE, TM, TN) bytes, aligned to 1024.  The output tile is
-// TM x TN, (TM / 64) x (TN / 64) waves with 64 x 64 each; pr.tiles_n counts tiles of TN columns.
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, int BK, int NSTAGE, int TM = 128,
-          int TN = kGemmBN, bool LN_BWD = false>
-__device__ __forceinline__ void gemm16_pipe_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
-  static_assert(NSTAGE >= 2 && NSTAGE <= 4 && (BK == 32 || BK == 64) && (TM == 128 || TM == 256), "stages");
-  static_assert(TN % 128 == 0 && (!SPLIT_K || TM == 128), "partial tiles are 128 x 128");
-  // The host cuts K ranges and checks K in units of kG16BK: every range is then whole steps of BK.
-  static_assert(kG16BK % BK == 0, "K ranges are multiples of kG16BK, which must be whole steps");
-  constexpr int WN = TN / 64;                                 // waves side by side
-  constexpr int NW = (TM / 64) * WN;
-  constexpr int NWA = gemm16_pipe_waves(TM, BK, NW), NWB = gemm16_pipe_waves(TN, BK, NW);  // waves that copy A, B
-  constexpr int NIA = gemm16_pipe_requests(TM, BK, NW);       // copy requests per thread and step
-  constexpr int NIB = gemm16_pipe_requests(TN, BK, NW);
-  constexpr int OPA = TM * BK * 2, OPB = TN * BK * 2;         // bytes of an operand's step
-  constexpr int OP = OPA + OPB;
-  const T* __restrict__ A = pr.A;
-  const T* __restrict__ B = pr.B;
-  const T* __restrict__ bias = pr.bias;
-  T* __restrict__ C = pr.C;
-  float* __restrict__ partial = pr.partial;
-  const int M = pr.M, N = pr.N, K = pr.K;
-  const int64_t lda = pr.lda, ldb = pr.ldb, ldc = pr.ldc, bsa = pr.bsa, bsb = pr.bsb, bsc = pr.bsc;
-  const int tiles_m = pr.tiles_m, tiles_n = pr.tiles_n, k_per_split = pr.k_per_split, splits = pr.splits,
-            batches = pr.batches;
-  const GemmEpilogue<T> ep = pr.ep;
-
-  const int tiles = tiles_m * tiles_n;
-  int batch = bid / tiles, tile = bid % tiles, split = 0;
-  if constexpr (SPLIT_K) {
-    if (!gemm_split_work(bid, tiles, splits, batches, tile, split, batch)) return;
-  }
-  int tm, tn;
-  gemm_tile_of_block(tile, tiles_m, tiles_n, tm, tn, !SPLIT_K);
-  const int m0 = tm * TM;
-  const int n0 = tn * TN;
-  const int k_begin = SPLIT_K ? split * k_per_split : 0;
-  const int k_end = SPLIT_K ? min(K, k_begin + k_per_split) : K;
-  const int full_steps = (k_end - k_begin) / BK, rem = (k_end - k_begin) % BK;
-  const int steps = full_steps + (rem > 0 ? 1 : 0);
-  A += batch * bsa + (A_KC ? static_cast<int64_t>(k_begin) : k_begin * lda);
-  B += batch * bsb + (B_KC ? static_cast<int64_t>(k_begin) : k_begin * ldb);
-  const int64_t a_step = A_KC ? BK : BK * lda;
-  const int64_t b_step = B_KC ? BK : BK * ldb;
-
-  const int wave = threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  const int wm = (wave / WN) * 64;
-  const int wn = (wave % WN) * 64;
-  // Waves that copy fewer requests per step have fewer outstanding at the waits below.
-  const bool copies_a = NWA == NW || wave < NWA, copies_b = NWB == NW || wave < NWB;
-  const int per_step = (copies_a ? NIA : 0) + (copies_b ? NIB : 0);
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // Column sums of the A tiles (see Gemm16Problem::colsum_part): a thread of the first four
-  // waves takes one 16-byte chunk (8 of the tile's 128 m) of every 16th k-row.
-  constexpr bool CAN_COLSUM = SPLIT_K && !A_KC && TM == 128;
-  const bool colsum = CAN_COLSUM && pr.colsum_part != nullptr && tn == 0;
-  const bool cs_thread = threadIdx.x < 256;
-  const int cs_chunk = threadIdx.x % 16, cs_row = threadIdx.x / 16;
-  float cs_acc[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) cs_acc[e] = 0.f;
-
-  const uint16_t* a16 = reinterpret_cast<const uint16_t*>(A);
-  const uint16_t* b16 = reinterpret_cast<const uint16_t*>(B);
-  int64_t src_a[NIA], src_b[NIB];
-  gemm16_pipe_sources<A_KC, BK, TM, NWA>(lda, m0, M, src_a);
-  gemm16_pipe_sources<B_KC, BK, TN, NWB>(ldb, n0, N, src_b);
-  auto request = [&](int step, int copy) {
-    if (step == full_steps) {
-      if (copies_a) gemm16_pipe_tail<A_KC, BK, TM, NWA>(a16 + step * a_step, src_a, rem, lds + copy * OP);
-      if (copies_b) gemm16_pipe_tail<B_KC, BK, TN, NWB>(b16 + step * b_step, src_b, rem, lds + copy * OP + OPA);
-      return;
-    }
-    if (copies_a) gemm16_pipe_issue<NIA, NWA>(a16 + step * a_step, src_a, lds + copy * OP);
-    if (copies_b) gemm16_pipe_issue<NIB, NWB>(b16 + step * b_step, src_b, lds + copy * OP + OPA);
-  };
-
-  // The lane's two bias values are requested before the tiles and are in their registers when
-  // the first step's tiles are (the empty asm puts the compiler's wait here, where the first
-  // iteration waits anyway): fetched in the epilogue, every tile ended on an exposed load, 4-10 us
-  // of a 30-40 us product at 16384 rows.
-  float bias_v[2] = {0.f, 0.f};
-  if constexpr (HAS_BIAS && !SPLIT_K) {
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const int col = n0 + wn + tj * 32 + lane % 32;
-      bias_v[tj] = col < N ? to_float(bias[col]) : 0.f;
-    }
-  }
-  // Steps 0 .. NSTAGE-2 are requested up front; iteration `it` then waits for step `it`
-  // (its own NIA + NIB requests; the barrier covers the other waves'), requests step
-  // it + NSTAGE - 1 into the copy that step it - 1 was just multiplied from, and multiplies.
-#pragma unroll
-  for (int s = 0; s < NSTAGE - 1; ++s)
-    if (s < steps) request(s, s);
-  if constexpr (HAS_BIAS && !SPLIT_K) asm volatile("" : "+v"(bias_v[0]), "+v"(bias_v[1]));
-  int cur = 0, nxt = NSTAGE - 1;
-  for (int it = 0; it < steps; ++it) {
-    // all but the NSTAGE - 2 younger steps' requests
-    if (it + NSTAGE - 2 >= full_steps || NSTAGE == 2) MG_WAIT_VMCNT(0);
-    else if (per_step == NIA + NIB) MG_WAIT_VMCNT((NIA + NIB) * (NSTAGE - 2));
-    else if (per_step == NIB) MG_WAIT_VMCNT(NIB * (NSTAGE - 2));
-    else if (per_step == NIA) MG_WAIT_VMCNT(NIA * (NSTAGE - 2));
-    // A plain barrier: __syncthreads() carries a fence that waits for every outstanding
-    // copy into LDS, the younger steps' included.
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (it + NSTAGE - 1 < steps) request(it + NSTAGE - 1, nxt);
-    const char* la = lds + cur * OP;
-    const char* lb = la + OPA;
-    if constexpr (CAN_COLSUM) {
-      if (colsum && cs_thread) {
-#pragma unroll
-        for (int j = 0; j < BK / 16; ++j) {
-          const int kk = cs_row + 16 * j;
-          float v[8];
-          VecIO<T, 8>::load(reinterpret_cast<const T*>(la + kk * (TM * 2) + ((cs_chunk ^ gemm16_tr_swizzle<TM>(kk)) * 16)), v);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) cs_acc[e] += v[e];
-        }
-      }
-    }
-    // The fragments of k-slice ks + 1 are requested before the products of slice ks, so
-    // their LDS latency runs under four MFMAs.
-    uint4 fa[2][2], fb[2][2];
-    fa[0][0] = gemm16_pipe_frag<A_KC, BK, TM>(la, wm, 0, lane);
-    fa[0][1] = gemm16_pipe_frag<A_KC, BK, TM>(la, wm + 32, 0, lane);
-    fb[0][0] = gemm16_pipe_frag<B_KC, BK, TN>(lb, wn, 0, lane);
-    fb[0][1] = gemm16_pipe_frag<B_KC, BK, TN>(lb, wn + 32, 0, lane);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int c = ks % 2, n = c ^ 1;
-      if (ks + 1 < BK / 16) {
-        fa[n][0] = gemm16_pipe_frag<A_KC, BK, TM>(la, wm, ks + 1, lane);
-        fa[n][1] = gemm16_pipe_frag<A_KC, BK, TM>(la, wm + 32, ks + 1, lane);
-        fb[n][0] = gemm16_pipe_frag<B_KC, BK, TN>(lb, wn, ks + 1, lane);
-        fb[n][1] = gemm16_pipe_frag<B_KC, BK, TN>(lb, wn + 32, ks + 1, lane);
-      }
-      acc[0][0] = GemmMma16<T>::run(fa[c][0], fb[c][0], acc[0][0]);
-      acc[0][1] = GemmMma16<T>::run(fa[c][0], fb[c][1], acc[0][1]);
-      acc[1][0] = GemmMma16<T>::run(fa[c][1], fb[c][0], acc[1][0]);
-      acc[1][1] = GemmMma16<T>::run(fa[c][1], fb[c][1], acc[1][1]);
-    }
-    cur = cur + 1 == NSTAGE ? 0 : cur + 1;
-    nxt = nxt + 1 == NSTAGE ? 0 : nxt + 1;
-  }
-  __syncthreads();  // every wave is done with the staged tiles: their memory serves the output
-
-  if constexpr (CAN_COLSUM) {
-    if (colsum) {
-      // sixteen threads hold sums for the same 8 columns (k-rows 0, 16, ... / 1, 17, ... / ...):
-      // added in a fixed order through LDS, one thread per column
-      constexpr int kPitch = 128 + 4;
-      float* red = reinterpret_cast<float*>(lds);
-      if (cs_thread) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) red[cs_row * kPitch + cs_chunk * 8 + e] = cs_acc[e];
-      }
-      __syncthreads();
-      if (threadIdx.x < 128 && m0 + static_cast<int>(threadIdx.x) < M) {
-        float sum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sum += red[r * kPitch + threadIdx.x];
-        pr.colsum_part[static_cast<int64_t>(split) * M + m0 + threadIdx.x] = sum;
-      }
-      __syncthreads();
-    }
-  }
-
-  uint16_t* mine = reinterpret_cast<uint16_t*>(lds) + wave * 64 * kG16Stride;
-  if constexpr (LN_BWD) {
-    // whole rows per tile, and room behind the strips for the row and column sums
-    static_assert(!SPLIT_K && !HAS_BIAS && TM == 128, "the LayerNorm epilogue takes a plain 128-row tile");
-    static_assert(gemm16_pipe_lds_bytes(BK, NSTAGE, TM, TN) >= NW * 64 * kG16Stride * 2 + 128 * WN * 8 + 2 * 64 * WN * 8,
-                  "LDS behind the output strips");
-    float* free_lds = reinterpret_cast<float*>(lds + NW * 64 * kG16Stride * 2);
-    gemm16_ln_bwd_tile<T, WN>(acc, mine, free_lds, C + batch * bsc, M, ldc, tm, m0, wm, wn, lane, ep.residual, pr.ln);
-  } else {
-    gemm16_write_tile<T, HAS_BIAS, SPLIT_K>(acc, mine, bias, C, partial, M, N, ldc, bsc, batch,
-                                            split, SPLIT_K ? batches : 1,
-                                            m0, n0, wm, wn, lane, ep, pr.partial_stream,
-                                            HAS_BIAS && !SPLIT_K ? bias_v : nullptr);
-  }
-}
-
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, int BK, int NSTAGE, int TM = 128>
-__global__ __launch_bounds__(TM * 2, gemm16_pipe_occupancy(BK, NSTAGE, TM)) void gemm_16bit_pipe_kernel(
-    const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ bias, T* __restrict__ C,
-    float* __restrict__ partial, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb,
-    int64_t bsc, int tiles_m, int tiles_n, int k_per_split, int splits, int batches, GemmEpilogue<T> ep) {
-  __shared__ __attribute__((aligned(1024))) char lds[gemm16_pipe_lds_bytes(BK, NSTAGE, TM)];
-  const Gemm16Problem<T> pr{A, B, bias, C, partial, M, N, K, lda, ldb, ldc, bsa, bsb, bsc,
-                            tiles_m, tiles_n, k_per_split, splits, batches, ep};
-  gemm16_pipe_block<T, A_KC, B_KC, HAS_BIAS, SPLIT_K, BK, NSTAGE, TM>(lds, blockIdx.x, pr);
-}
-
-// ------------------------------------------------------------------------------------
-// Large products: 256 x 256 output tile per workgroup of four waves, one wave per SIMD, each
-// wave a 128 x 128 tile as 4 x 4 v_mfma_f32_32x32x16 accumulators (256 accumulator registers
-// of the 512 a lone wave may use).  A k-slice of 16 takes four A and four B fragments for
-// sixteen MFMAs, i.e. half a kilobyte of LDS reads per MFMA where the 64 x 64 wave tile of
-// the kernels above needs a whole one: with four SIMDs issuing MFMAs back to back those
-// kernels ask the LDS for exactly its 128 bytes per clock, this one for half of that, and a
-// 256 x 256 tile also halves the operand bytes a FLOP pulls through L2.  The price is one
-// workgroup per CU: no second wave hides a wait, so the fragments of slice ks + 1 are read
-// while slice ks is multiplied and the tiles are copied NSTAGE steps ahead.  Taken for
-// products with at least one such tile per CU; tiles, copy and LDS images are those of
-// gemm16_pipe_block, and so is the order of every sum (results are bit-identical).
-// 8192^3 bf16 forward / dX / dW: 1.26 / 1.11 / 1.02 ms with 256 x 128 tiles of 64 x 64 wave
-// tiles -> 1.06 / 0.95 / 0.89 ms; matrix pipe busy 64 % of the CU-busy cycles (44-49 % before).
-// With the copies compiled out the same loop takes 0.79 / 0.73 / 0.70 ms, with the MFMAs
-// compiled out 0.63-0.72 / 0.63 / 0.57-0.64 ms: the L2 -> LDS copy of 8.6 GB per launch is as
-// long as the arithmetic and the two do not overlap fully.
-// ------------------------------------------------------------------------------------
-constexpr int kGemmBigT = 256;
-constexpr int gemm16_big_lds_bytes(int bk, int nstage) {
-  const int stages = nstage * 2 * kGemmBigT * bk * 2;
-  const int out = 4 * 64 * kG16Stride * 2;
-  return stages > out ? stages : out;
-}
-
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, int BK, int NSTAGE>
-__global__ __launch_bounds__(256, 1) void gemm_16bit_big_kernel(
-    const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ bias, T* __restrict__ C, int M, int N, int K,
-    int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb, int64_t bsc, int tiles_m, int tiles_n,
-    GemmEpilogue<T> ep) {
-  static_assert(NSTAGE >= 2 && NSTAGE <= 4 && (BK == 32 || BK == 64), "stages");
-  constexpr int TT = kGemmBigT, NW = 4;
-  constexpr int NI = gemm16_pipe_requests(TT, BK, NW);  // copy requests per thread, operand and step
-  constexpr int OPB = TT * BK * 2;                      // bytes of an operand's step
-  constexpr int OP = 2 * OPB;
-  __shared__ __attribute__((aligned(1024))) char lds[gemm16_big_lds_bytes(BK, NSTAGE)];
-
-  const int tiles = tiles_m * tiles_n;
-  const int batch = blockIdx.x / tiles, tile = blockIdx.x % tiles;
-  int tm, tn;
-  gemm_tile_of_block(tile, tiles_m, tiles_n, tm, tn, true);
-  const int m0 = tm * TT, n0 = tn * TT;
-  const int steps = K / BK;
-  A += batch * bsa;
-  B += batch * bsb;
-  const int64_t a_step = A_KC ? BK : BK * lda;
-  const int64_t b_step = B_KC ? BK : BK * ldb;
-
-  const int wave = threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  const int wm = (wave / 2) * 128;
-  const int wn = (wave % 2) * 128;
-
-  floatx16 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const uint16_t* a16 = reinterpret_cast<const uint16_t*>(A);
-  const uint16_t* b16 = reinterpret_cast<const uint16_t*>(B);
-  int64_t src_a[NI], src_b[NI];
-  gemm16_pipe_sources<A_KC, BK, TT, NW>(lda, m0, M, src_a);
-  gemm16_pipe_sources<B_KC, BK, TT, NW>(ldb, n0, N, src_b);
-  auto request = [&](int step, int copy) {
-    gemm16_pipe_issue<NI, NW>(a16 + step * a_step, src_a, lds + copy * OP);
-    gemm16_pipe_issue<NI, NW>(b16 + step * b_step, src_b, lds + copy * OP + OPB);
-  };
-
-  // The k loop is one stream of 16-deep slices.  While the sixteen MFMAs of a slice run, the
-  // eight fragments of the next slice are read into the other half of `f` (the reads are dealt
-  // out between the MFMAs with sched_group_barrier: left to itself the compiler reads each
-  // fragment right before its use and waits for it).  Before the last slice of a step comes
-  // the step's one synchronisation: the data of the next step has arrived (all but the
-  // NSTAGE - 2 younger steps' copies), no wave reads the current step's tiles any more (their
-  // last fragments are in registers), so the copy of step it + NSTAGE may overwrite them.
-  constexpr int NS = BK / 16;
-  constexpr int RA = A_KC ? 1 : 2, RB = B_KC ? 1 : 2;  // LDS reads per fragment
-  uint4 f[2][8];
-  auto read_frags = [&](int buf, int step, int ks) {  // B first: every MFMA group needs all four
-    const char* la = lds + (step % NSTAGE) * OP;
-    const char* lb = la + OPB;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f[buf][4 + i] = gemm16_pipe_frag<B_KC, BK, TT>(lb, wn + 32 * i, ks, lane);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f[buf][i] = gemm16_pipe_frag<A_KC, BK, TT>(la, wm + 32 * i, ks, lane);
-  };
-  auto multiply = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = GemmMma16<T>::run(f[buf][i], f[buf][4 + j], acc[i][j]);
-  };
-  // Slice ks of step `it`.  MODE 0: steady state (a copy is requested at the step's
-  // synchronisation, the next step exists); 1: the product's last steps (nothing left to
-  // request, every copy is waited for); 2: the very last slice (nothing left to read either).
-  auto slice = [&](int it, int ks, auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    const int buf = ks % 2;
-    if (ks == NS - 1) {
-      if constexpr (MODE != 0 || NSTAGE == 2) MG_WAIT_VMCNT(0);
-      else MG_WAIT_VMCNT(2 * NI * (NSTAGE - 2));
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if constexpr (MODE == 0) request(it + NSTAGE, it % NSTAGE);
-      if constexpr (MODE != 2) read_frags(buf ^ 1, it + 1, 0);
-    } else {
-      read_frags(buf ^ 1, it, ks + 1);
-    }
-    multiply(buf);
-    if constexpr (MODE != 2) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {  // four groups of (4 MFMAs, a quarter of the reads)
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, RA + RB, 0);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  static_assert(NS % 2 == 0, "a step ends on the second fragment buffer");
-#pragma unroll
-  for (int s = 0; s < NSTAGE; ++s)
-    if (s < steps) request(s, s);
-  if (steps > NSTAGE - 1) MG_WAIT_VMCNT(2 * NI * (NSTAGE - 1));
-  else MG_WAIT_VMCNT(0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  read_frags(0, 0, 0);
-  // The loop body starts at a step's synchronisation (where nothing is outstanding anyway, so
-  // what the compiler assumes at a loop head costs nothing) and runs on through the first
-  // slices of the next step.
-#pragma unroll
-  for (int ks = 0; ks < NS - 1; ++ks) slice(0, ks, std::integral_constant<int, 0>{});
-  int it = 0;
-  for (; it < steps - NSTAGE; ++it) {
-    slice(it, NS - 1, std::integral_constant<int, 0>{});
-#pragma unroll
-    for (int ks = 0; ks < NS - 1; ++ks) slice(it + 1, ks, std::integral_constant<int, 0>{});
-  }
-  for (; it < steps - 1; ++it) {
-    slice(it, NS - 1, std::integral_constant<int, 1>{});
-#pragma unroll
-    for (int ks = 0; ks < NS - 1; ++ks) slice(it + 1, ks, std::integral_constant<int, 1>{});
-  }
-  slice(steps - 1, NS - 1, std::integral_constant<int, 2>{});
-  __syncthreads();  // every wave is done with the staged tiles: their memory serves the output
-
-  // The wave's 128 x 128 tile goes out as four 64 x 64 quadrants through its own strip of LDS.
-  uint16_t* mine = reinterpret_cast<uint16_t*>(lds) + wave * 64 * kG16Stride;
-#pragma unroll
-  for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-    for (int qj = 0; qj < 2; ++qj) {
-      floatx16 quad[2][2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) quad[i][j] = acc[2 * qi + i][2 * qj + j];
-      gemm16_write_tile<T, HAS_BIAS, false>(quad, mine, bias, C, nullptr, M, N, ldc, bsc, batch, 0, 1, m0, n0,
-                                            wm + 64 * qi, wn + 64 * qj, lane, ep);
-      __syncthreads();  // the strip is read out before the next quadrant is written into it
-    }
-}
-
-// Both products of a Linear layer's backward in one launch: workgroups [0, n_dw) take the
-// K ranges of dW = dY^T X (their partial tiles are summed by linear_bwd_finish_kernel
-// afterwards), the rest the tiles of dX = dY W.  The longer-running dW ranges start first
-// and the dX tiles fill the CUs as those drain, where two launches each end in a tail of
-// half-empty CUs (384 dX tiles on 256 CUs) and pay a launch apiece.  With
-// dw.colsum_part set, the dW workgroups of the first tile column also produce the bias
-// gradient's partial rows from the dY tiles they hold anyway.
-template <typename T, int NSTAGE = 2, int TN = kGemmBN, int BK = 32>
-__global__ __launch_bounds__(2 * TN, gemm16_pipe_occupancy(BK, NSTAGE, 128, TN)) void linear_bwd_16bit_kernel(
-    Gemm16Problem<T> dw, Gemm16Problem<T> dx, int n_dw) {
-  __shared__ __attribute__((aligned(1024))) char lds[gemm16_pipe_lds_bytes(BK, NSTAGE, 128, TN)];
-  const int bid = blockIdx.x;
-  if (bid < n_dw) gemm16_pipe_block<T, false, false, false, true, BK, NSTAGE, 128, TN>(lds, bid, dw);
-  else gemm16_pipe_block<T, true, false, false, false, BK, NSTAGE, 128, TN>(lds, bid - n_dw, dx);
-}
-
-// The same launch with the dX tiles (128 x 384: whole rows of a 384-wide layer input) continuing
-// as the backward of the LayerNorm that produced the layer's input (gemm16_ln_bwd_tile).
+// The output tiles of gemm_16bit_deep.h.
+enum Gemm16Tile { kTile128 = 0, kTile192 = 1, kTile256 = 2, kTileWide = 3 };  // 128 x 128, 128 x 192, 256 x 256, 128 x 384
+constexpr int kGemm16TileM[4] = {128, 128, 256, 128};
+constexpr int kGemm16TileN[4] = {128, 192, 256, 384};
+constexpr int64_t kGemmDeepMaxLd = 1 << 22;  // offsets within a tile are kept in 32 bits
+// One product of them (not kTileWide); partial: `splits` K ranges of k_per_split each, partial tiles (splits == 1: null).
 template <typename T>
-__global__ __launch_bounds__(2 * kGemmWideBN, 1) void linear_bwd_ln_16bit_kernel(Gemm16Problem<T> dw, Gemm16Problem<T> dx,
-                                                                                 int n_dw) {
-  __shared__ __attribute__((aligned(1024))) char lds[gemm16_pipe_lds_bytes(64, 2, 128, kGemmWideBN)];
-  const int bid = blockIdx.x;
-  if (bid < n_dw) gemm16_pipe_block<T, false, false, false, true, 64, 2, 128, kGemmWideBN>(lds, bid, dw);
-  else gemm16_pipe_block<T, true, false, false, false, 64, 2, 128, kGemmWideBN, true>(lds, bid - n_dw, dx);
-}
+int launch_16bit_deep(const GemmArgs& g, Gemm16Tile tile, int splits, int k_per_split, float* partial, hipStream_t stream);
+// dX and dW of a Linear layer (not kTile256), see linear_bwd_16bit_kernel; kTileWide: dX continues as px.ln says.
+template <typename T>
+int launch_linear_bwd_deep(const Gemm16Problem<T>& pw, const Gemm16Problem<T>& px, Gemm16Tile tile, int64_t n_dw,
+                           int64_t n_dx, hipStream_t stream);
 
 // ------------------------------------------------------------------------------------
 // fp32 product with the tiles copied global memory -> LDS by `global_load_lds_dwordx4`, two

@@ -197,6 +197,8 @@ constexpr int kDppQuadXor1 = 0xB1;      // quad_perm:[1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;      // quad_perm:[2,3,0,1]
 constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppRowMirror = 0x140;
+constexpr int kDppRowRor4 = 0x124;       // rotations within sixteen lanes
+constexpr int kDppRowRor8 = 0x128;
 constexpr int kSwizzleXor16 = 0x401F;   // ds_swizzle bit mode: and 0x1f, or 0, xor 0x10
 
 struct SumOp {
