@@ -1708,13 +1708,13 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
 
   const int nqb = (a.S + BM - 1) / BM;
   const int n_bh = a.B * a.H;
-  // Workgroups that are resident together share a CU with those a whole round (one per CU) before and behind
-  // them.  Causal: their work falls with their number, so every second round is handed out backwards
-  // (in groups of eight, one per XCD), which evens out what the CUs get.
+  // A CU's first workgroup is joined by the one a whole round (one per CU) behind it.  Causal: their work falls
+  // with their number, so the second round is handed out backwards (in groups of eight, one per XCD), which evens out
+  // what the CUs start on; what comes later goes where there is room.
   int block = blockIdx.x;
   if (CAUSAL) {
-    const int p = block / round, r = block % round;
-    if (p % 2 == 1 && (p + 1) * round <= static_cast<int>(gridDim.x)) block = p * round + (round / 8 - 1 - r / 8) * 8 + r % 8;
+    const int r = block - round;
+    if (r >= 0 && r < round && 2 * round <= static_cast<int>(gridDim.x)) block = round + (round / 8 - 1 - r / 8) * 8 + r % 8;
   }
   const int qb = CAUSAL ? nqb - 1 - block / n_bh : block / n_bh;  // heaviest query blocks first
   const int h = (block % n_bh) % a.H;
