@@ -100,7 +100,7 @@ static void bwd_f32_mfma_launch(const void* d_o, const void* q, const void* k, c
 // MOGRAD_HIP_ATTN_F32_WAVE = 0 | 1 overrides the choice where either can be had.
 static int64_t attn_tiles32(const AttnDims& a) { return static_cast<int64_t>(a.B) * a.H * ceil_div(a.S, 32); }
 static bool attn_f32_wave_ok(const AttnDims& a, bool causal, const void* const* ptrs, int nptrs) {
-  if (a.D % 4 != 0 || a.D > kF32WaveMaxD || a.ld % 4 != 0) return false;
+  if (a.D % 4 != 0 || a.D > kF32WaveMaxD || a.ld % 4 != 0 || a.ld >= 1 << 24) return false;  // (places in a tile: 32 bits)
   for (int i = 0; i < nptrs; ++i)
     if (!aligned16(ptrs[i])) return false;
   const bool tile_kernels = (a.D <= 64 || (causal && a.D > 96 && a.D <= 128 && a.S < 1024)) && a.S >= 64 &&

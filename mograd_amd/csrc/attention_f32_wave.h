@@ -12,11 +12,14 @@
 // third of the device, and a sequence of 32 is one wave's work.  80 and 96 columns have kernels of
 // their own instead of the 128-column one.
 //   fp32 forward + backward, one MI355X, before -> now:
-//     (3, 777, 8 heads, 80), bias        645 -> 412 us      (1, 1236, 6, 256), causal  3930 -> 541 us
-//     (1, 176, 10, 80), bias             164 ->  61 us      (2, 2048, 8, 128), causal  1440 -> 805 us
-//     (4, 32, 2, 32), causal              65 ->  19 us      (21, 79, 8, 32), causal      35 ->  29 us
-// The arithmetic is the matrix pipe's: 64 cycles per 32 x 32 x 2 product, two products per
-// column and step forward, seven over the two backward kernels.
+//     (3, 777, 8 heads, 80), bias        645 -> 387 us      (1, 1236, 6, 256), causal  3930 -> 513 us
+//     (1, 176, 10, 80), bias             164 ->  55 us      (2, 8 heads of 1500, 128)   816 -> 765 us (*)
+//     (4, 32, 2, 32), causal              65 ->  18 us      (21, 79, 8, 32), causal      35 ->  27 us
+// (*: before the addresses below).  The arithmetic is the matrix pipe's: 64 cycles per 32 x 32 x 2 product, two
+// products per column and step forward, seven over the two backward kernels.  What stands beside it on the one
+// wave of a SIMD is vector arithmetic, 1300 instructions a step at 80 columns until the copies took a scalar base
+// and a byte offset per lane, the bias' places were computed once, and exp2f became the one instruction:
+// 414 -> 387 us at 777 rows with bias, 260 -> 227 us at (2, 8 heads of 1024, 64) with bias.
 //
 // Layouts as in attention_f32_mfma.h: a score tile comes out with the workgroup's rows along the
 // lanes and the streamed rows along the registers, which is the operand of the products that
@@ -36,6 +39,10 @@
 namespace mg {
 
 constexpr int kF32WaveMaxD = 256;
+
+// v_exp_f32 alone: exp2f scales its argument around it so that results below 2^-126 come out as denormals, six
+// instructions for weights that 1 in a row's sum hides.
+__device__ __forceinline__ float f32_wave_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // What the four waves of a workgroup share: the streamed rows of one tile of 32, nothing (each has a
 // tile of its own), or the head columns of one tile.
@@ -65,24 +72,29 @@ template <int DP, F32WaveMode MODE, bool HAS_BIAS>
 constexpr int f32_wave_lds(int scores) {
   return 4 * f32_wave_bytes<DP, HAS_BIAS>() + (MODE == kF32SplitColumns ? 2 * 4 * scores * 4096 : 0);
 }
-// Workgroups per CU that the registers are budgeted for.
+// Workgroups per CU that the registers are budgeted for.  80 columns without a bias are 80 KB of LDS, two to a CU,
+// one's softmax beside the other's products: (3, 777, 8 heads, 80) 92 + 265 us -> 78 + 242, causal 50 + 154 ->
+// 40 + 139.  With a bias it is 96 KB; loading that straight to registers instead, to get under, is slower than
+// its copies (32 rows to a load: 96 columns 70 -> 77 us, 128 columns 76 -> 86), and dQ then spills.
 template <int DP, F32WaveMode MODE, bool HAS_BIAS>
 constexpr int f32_wave_occupancy(int results) {
-  return DP <= 32 || (DP <= 64 && MODE != kF32SplitColumns && !HAS_BIAS && results == 1) ? 2 : 1;
+  return DP <= 32 || (DP <= 80 && MODE != kF32SplitColumns && !HAS_BIAS && results == 1) ? 2 : 1;
 }
 
-// See gemm16_pipe_issue for why these are assembly.
-__device__ __forceinline__ void f32_wave_copy16(const float* src, unsigned dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(src)
-               : "memory");
+// See gemm16_deep_issue for why these are assembly.  `base` is the same for the wave; with a byte offset per lane
+// a copy costs no vector arithmetic (a 64-bit address per lane and copy was 3 instructions).
+__device__ __forceinline__ void f32_wave_copy16(const float* base, unsigned bytes, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(bytes), "s"(base) : "memory");
 }
-__device__ __forceinline__ void f32_wave_copy4(const float* src, unsigned dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(src)
-               : "memory");
+__device__ __forceinline__ void f32_wave_copy4(const float* base, unsigned bytes, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(bytes), "s"(base) : "memory");
+}
+__device__ __forceinline__ void f32_wave_copy4_at(const float* src, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(src) : "memory");
 }
 __device__ __forceinline__ unsigned f32_wave_lds_at(const char* p) {
   using lds_ptr = __attribute__((address_space(3))) const char*;
-  return static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)p));
+  return __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)p)));
 }
 // At most N of the wave's copies are outstanding, and none of its LDS reads.
 #define MG_F32_WAVE_WAIT(N)                                                        \
@@ -98,7 +110,7 @@ struct F32WaveTiles {
   const float* base;
   int64_t ld;
   int S, last_chunk;
-  int off[F32Wave<DP>::NI];  // the lane's place in a whole tile, in elements
+  unsigned off[F32Wave<DP>::NI];  // the lane's place in a whole tile, in bytes
   __device__ __forceinline__ void source(int i, int lane, int& row, int& c) const {
     using W = F32Wave<DP>;
     const int slot = i * 64 + lane;
@@ -115,15 +127,15 @@ struct F32WaveTiles {
     for (int i = 0; i < F32Wave<DP>::NI; ++i) {
       int row, c;
       source(i, lane, row, c);
-      off[i] = static_cast<int>(row * ld) + c * 4;
+      off[i] = static_cast<unsigned>(row * ld + c * 4) * 4;
     }
   }
   __device__ __forceinline__ void copy(int row0, const char* tile, int lane) const {
     const unsigned dst = f32_wave_lds_at(tile);
+    const float* p = base + row0 * ld;
     if (row0 + 32 <= S) {
-      const float* p = base + row0 * ld;
 #pragma unroll
-      for (int i = 0; i < F32Wave<DP>::NI; ++i) f32_wave_copy16(p + off[i], dst + i * 1024);
+      for (int i = 0; i < F32Wave<DP>::NI; ++i) f32_wave_copy16(p, off[i], dst + i * 1024);
       return;
     }
     asm volatile("" : "+v"(lane));  // computed here, once per walk, and not kept in registers throughout
@@ -131,23 +143,37 @@ struct F32WaveTiles {
     for (int i = 0; i < F32Wave<DP>::NI; ++i) {
       int row, c;
       source(i, lane, row, c);
-      f32_wave_copy16(base + min(row0 + row, S - 1) * ld + c * 4, dst + i * 1024);
+      f32_wave_copy16(p, static_cast<unsigned>(min(row, S - 1 - row0) * ld + c * 4) * 4, dst + i * 1024);
     }
   }
 };
 
 // The bias of queries i0 .. + 31 and keys j0 .. + 31, as a tile of 32 columns, in 4-byte copies (its rows
-// start anywhere).
-__device__ __forceinline__ void f32_wave_copy_bias(const float* mask, int i0, int j0, int S, const char* tile, int lane) {
-  const unsigned dst = f32_wave_lds_at(tile);
-  asm volatile("" : "+v"(lane));  // (not kept in registers)
+// start anywhere).  Copy i takes rows 2 i and 2 i + 1, whose chunks are permuted by i % 8: the lane's byte in a row
+// is (4 (lane % 32)) ^ 16 (i % 8).  A tile that reaches past the sequence has its places computed one by one.
+struct F32WaveBias {
+  unsigned off[8];
+  __device__ __forceinline__ void init(int S, int lane) {
+    static_assert(F32Wave<32>::X == 8, "rows 2 i and 2 i + 1 are permuted alike, eight ways");
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = 2 * i + lane / 32, p = lane % 32;
-    const int col = ((p / 4) ^ F32Wave<32>::swizzle(row)) * 4 + p % 4;
-    f32_wave_copy4(mask + static_cast<int64_t>(min(i0 + row, S - 1)) * S + min(j0 + col, S - 1), dst + i * 256);
+    for (int i = 0; i < 8; ++i) off[i] = static_cast<unsigned>(lane / 32 * S) * 4 + ((lane % 32 * 4) ^ (i * 16));
   }
-}
+  __device__ __forceinline__ void copy(const float* mask, int i0, int j0, int S, const char* tile, int lane) const {
+    const unsigned dst = f32_wave_lds_at(tile);
+    if (i0 + 32 <= S && j0 + 32 <= S) {
+      const float* p = mask + static_cast<int64_t>(i0) * S + j0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) f32_wave_copy4(p + 2 * i * static_cast<int64_t>(S), off[i % 8], dst + i * 256);
+      return;
+    }
+    asm volatile("" : "+v"(lane));  // (not kept in registers)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 2 * i + lane / 32, col = (lane % 32) ^ (i % 8 * 4);
+      f32_wave_copy4_at(mask + static_cast<int64_t>(min(i0 + row, S - 1)) * S + min(j0 + col, S - 1), dst + i * 256);
+    }
+  }
+};
 
 // tile * resident^T over the wave's columns (see f32_attn_scores).
 template <int DP>
@@ -332,8 +358,10 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     vt.copy(min(t, steps - 1) * 32, v_s, lane);
   };
   const float* mhead = HAS_BIAS ? mask + static_cast<int64_t>(bh) * a.S * a.S : nullptr;
+  F32WaveBias mt_copies;
+  if constexpr (HAS_BIAS) mt_copies.init(a.S, lane);
   auto copy_m = [&](int t) {
-    if constexpr (HAS_BIAS) f32_wave_copy_bias(mhead, r0, min(t, steps - 1) * 32, a.S, m_s, lane);
+    if constexpr (HAS_BIAS) mt_copies.copy(mhead, r0, min(t, steps - 1) * 32, a.S, m_s, lane);
   };
   float qr[DP / 2];
   f32_wave_resident<DP>(q + qkv_at(a, b, ic, h), row_ok && columns, col0, half, a.D, scale * kAttnLog2e, qr);
@@ -383,7 +411,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     // the sum and the result are relative to the same point).
     if (__any(m_tile > m + 8.0f)) {
       const float m_new = fmaxf(m, m_tile);
-      const float corr = m_new == -INFINITY ? 0.f : exp2f(m - m_new);
+      const float corr = m_new == -INFINITY ? 0.f : f32_wave_exp2(m - m_new);
       l *= corr;
 #pragma unroll
       for (int db = 0; db < W::NB; ++db)
@@ -394,7 +422,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     const float base = m == -INFINITY ? 0.f : m;  // (nothing visible to this row yet: its weights are zero)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[0][r] = exp2f(s[0][r] - base);
+      s[0][r] = f32_wave_exp2(s[0][r] - base);
       l += s[0][r];
     }
     MG_F32_WAVE_WAIT(NI + NM);
@@ -426,7 +454,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = ml[0][w][lane % 32];
-      f[w] = mw == -INFINITY ? 0.f : exp2f(mw - m);
+      f[w] = mw == -INFINITY ? 0.f : f32_wave_exp2(mw - m);
       l_row += f[w] * ml[1][w][lane % 32];
     }
     f32_wave_merge<DP>(lds, acc, f, orow, row_ok, 1.0f / l_row, a.D, wave, lane);
@@ -473,8 +501,10 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     vt.copy(min(t, steps - 1) * 32, v_s, lane);
   };
   const float* mhead = HAS_BIAS ? mask + static_cast<int64_t>(bh) * a.S * a.S : nullptr;
+  F32WaveBias mt_copies;
+  if constexpr (HAS_BIAS) mt_copies.init(a.S, lane);
   auto copy_m = [&](int t) {
-    if constexpr (HAS_BIAS) f32_wave_copy_bias(mhead, r0, min(t, steps - 1) * 32, a.S, m_s, lane);
+    if constexpr (HAS_BIAS) mt_copies.copy(mhead, r0, min(t, steps - 1) * 32, a.S, m_s, lane);
   };
   float qr[DP / 2], dor[DP / 2];
   float dl = 0.f;
@@ -534,7 +564,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
       float sv = s[0][r];
       if (HAS_BIAS) sv = fmaf(bias[r], kAttnLog2e, sv);
       const bool valid = j < a.S && (!CAUSAL || j <= i);
-      const float p = valid ? exp2f(sv - lse2) : 0.f;
+      const float p = valid ? f32_wave_exp2(sv - lse2) : 0.f;
       s[0][r] = p * (s[1][r] - dl);  // dS without the scale: K is unscaled, the scale goes on at the end
     }
     f32_wave_weighted<DP>(k_s, s[0], lane, acc);
@@ -588,11 +618,13 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) v
   auto copy_q = [&](int t) { qt.copy(min(t, steps - 1) * 32, q_s, lane); };
   auto copy_d = [&](int t) { dt.copy(min(t, steps - 1) * 32, do_s, lane); };
   const float* mhead = HAS_BIAS ? mask + static_cast<int64_t>(bh) * a.S * a.S : nullptr;
+  F32WaveBias mt_copies;
+  if constexpr (HAS_BIAS) mt_copies.init(a.S, lane);
   auto copy_m = [&](int t) {
     const int i0 = min(t, steps - 1) * 32, i = min(i0 + lane % 32, a.S - 1);
-    f32_wave_copy4(lse_h + i, f32_wave_lds_at(stats[wave][0]));
-    f32_wave_copy4(delta_h + i, f32_wave_lds_at(stats[wave][1]));
-    if constexpr (HAS_BIAS) f32_wave_copy_bias(mhead, i0, r0, a.S, m_s, lane);
+    f32_wave_copy4(lse_h, i * 4, f32_wave_lds_at(stats[wave][0]));
+    f32_wave_copy4(delta_h, i * 4, f32_wave_lds_at(stats[wave][1]));
+    if constexpr (HAS_BIAS) mt_copies.copy(mhead, i0, r0, a.S, m_s, lane);
   };
   float kr[DP / 2], vr[DP / 2];
   f32_wave_resident<DP>(k + qkv_at(a, b, jc, h), row_ok && columns, col0, half, a.D, scale * kAttnLog2e, kr);
@@ -629,7 +661,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) v
           sv = fmaf(mt[F32Wave<32>::place(rr + e, (lane % 32) / 4, 0) + lane % 4], kAttnLog2e, sv);
         }
         const bool valid = i < a.S && (!CAUSAL || j <= i);
-        const float p = valid ? exp2f(sv) : 0.f;
+        const float p = valid ? f32_wave_exp2(sv) : 0.f;
         s[0][r] = p;
         s[1][r] = p * (s[1][r] - dv4[e]);
       }
