@@ -568,7 +568,7 @@ static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
 // tile.  For the 128-row tiles as in deep_16bit_us, a chain's steps between the two figures there (it shares its
 // CU for a part of its life).  A range has at least 256 rows.  tile < 0: no such launch.
 // MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
-static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx) {
+static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx, bool with_db) {
   const double cus = device_info().cu_count;
   const double steps_w = static_cast<double>(ceil_div(M, kG16BK)), steps_x = static_cast<double>(ceil_div(N, kG16BK));
   Choice16 small{kSmall, 1};
@@ -613,8 +613,13 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx)
       if (only != 128) offer(kTile192, s);
     }
   }
-  // (a launch of its own for each product; the LayerNorm's backward is 6 us as one)
-  if (deep.tile < 0) deep.us = choose_16bit(N, K, M, 1, false).us + (with_dx ? choose_16bit(M, K, N, 1, N >= 1024 && N % 64 != 0).us : 0.0);
+  // (a launch of its own for each product, and 7 us of one or two more for the sum of dY's rows: (85, 2664 <- 632)
+  // 28 us with separate launches, 22 with one.  Off the 16-byte chunks dW is the register-staged kernel's, 5 us
+  // more: (114, 1771 <- 384) 20 us against 12.  The LayerNorm's backward is 6 us as one.)
+  if (deep.tile < 0) {
+    deep.us = choose_16bit(N, K, M, 1, false).us + (with_db ? 7.0 : 0.0) + (mult8(N) && mult8(K) ? 0.0 : 5.0);
+    if (with_dx) deep.us += choose_16bit(M, K, N, 1, N >= 1024 && N % 64 != 0).us;
+  }
   const bool is_small = small.us + (deep.tile == kTileWide ? 6.0 : 0.0) <= deep.us;
   // (A choice of the larger tiles' form is also one for them.)
   return env_int("MOGRAD_HIP_LINEAR_BWD_SMALL", is_small && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE")) != 0 ? small : deep;
@@ -633,7 +638,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   // rows of the next multiple of 8, zeros behind (`pads` below); dX, dW and db keep their shape.
   const bool pad_n = !mult8(N) || !aligned16(dy), pad_k = !mult8(K) || !aligned16(x) || (dx && !aligned16(w));
   const int64_t cus = device_info().cu_count;
-  const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr);
+  const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr, db != nullptr);
   if (choice.tile < 0) return MG_OK;
   const bool small = choice.tile == kSmall, wide = choice.tile == kTileWide;
   if (ln && (!wide || relu_mask || pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx))) return MG_OK;

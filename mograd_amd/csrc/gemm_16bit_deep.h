@@ -74,18 +74,14 @@ __device__ __forceinline__ void gemm16_deep_issue(const uint16_t* base, uint32_t
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
 }
 
-// An image of the last, short step (`rem` k left): through registers, zeros past the end (see gemm16_pipe_tail).
+// The same for request i of an image of the last, short step (`rem` k left), zeros past the end (see
+// gemm16_pipe_issue_short).
 template <bool KC, int ROWS, int NT>
-__device__ __forceinline__ void gemm16_deep_tail(const uint16_t* base, const uint32_t (&off)[ROWS * 8 / NT], int rem,
-                                                 char* image) {
-#pragma unroll
-  for (int i = 0; i < ROWS * 8 / NT; ++i) {
-    const int slot = i * NT + threadIdx.x;
-    const int k = KC ? ((slot % 8) ^ ((slot / 8 / 2) % 8)) * 8 : slot / (ROWS / 8);
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (k < rem) v = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) + off[i]);
-    *reinterpret_cast<uint4*>(image + slot * 16) = v;
-  }
+__device__ __forceinline__ void gemm16_deep_issue_short(const uint16_t* base, uint32_t off, int i, int rem, uint32_t dst) {
+  const int slot = i * NT + threadIdx.x;
+  const int k = KC ? ((slot % 8) ^ ((slot / 8 / 2) % 8)) * 8 : slot / (ROWS / 8);
+  const char* p = k < rem ? reinterpret_cast<const char*>(base) + off : reinterpret_cast<const char*>(kGemmZeros);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(p) : "memory");
 }
 
 // A wave's 64 x (32 BJ) values into its strip of LDS, rounded.  The accumulators have lanes along n and
@@ -378,13 +374,13 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
     if constexpr (IM == 2) gemm16_deep_issue(b16 + step * b_step, src_b0[i], dst);
     if constexpr (IM == 3) gemm16_deep_issue(b16 + step * b_step, src_b1[i], dst);
   };
-  auto tail = [&](auto image, int step, int copy, int left) {
+  auto request_short = [&](auto image, int i, int step, int copy, int left) {
     constexpr int IM = decltype(image)::value;
-    char* at = lds + copy * S::kStep + S::at(IM);
-    if constexpr (IM == 0) gemm16_deep_tail<A_KC, S::kRowsA, NT>(a16 + step * a_step, src_a0, left, at);
-    if constexpr (IM == 1) gemm16_deep_tail<A_KC, S::kRowsA, NT>(a16 + step * a_step, src_a1, left, at);
-    if constexpr (IM == 2) gemm16_deep_tail<B_KC, S::kRowsB0, NT>(b16 + step * b_step, src_b0, left, at);
-    if constexpr (IM == 3) gemm16_deep_tail<B_KC, S::kRowsB1, NT>(b16 + step * b_step, src_b1, left, at);
+    const uint32_t dst = lds_wave + copy * S::kStep + S::at(IM) + i * (NT * 16);
+    if constexpr (IM == 0) gemm16_deep_issue_short<A_KC, S::kRowsA, NT>(a16 + step * a_step, src_a0[i], i, left, dst);
+    if constexpr (IM == 1) gemm16_deep_issue_short<A_KC, S::kRowsA, NT>(a16 + step * a_step, src_a1[i], i, left, dst);
+    if constexpr (IM == 2) gemm16_deep_issue_short<B_KC, S::kRowsB0, NT>(b16 + step * b_step, src_b0[i], i, left, dst);
+    if constexpr (IM == 3) gemm16_deep_issue_short<B_KC, S::kRowsB1, NT>(b16 + step * b_step, src_b1[i], i, left, dst);
   };
 
   uint4 fa[2][AI][4], fb0[BJ0][4], fb1[BJ1][4];  // fragments [block of 32 rows][k-slice of 16]
@@ -410,8 +406,8 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
   constexpr auto blocks = [](int im) constexpr { return im < 2 ? AI : im == 2 ? BJ0 : im == 3 ? BJ1 : 0; };
   // One phase: half `ah` x part `bh`.  Meanwhile the fragments of `rd` are read from copy `rd_copy` (those of a
   // part that is being multiplied: each k-slice when it has been), and image `rq` of step `rq_step` is
-  // requested.  `sync` runs after the first k-slice.
-  auto phase = [&](auto ah, auto bh, auto rd, int rd_copy, auto rq, int rq_step, int rq_copy, auto sync) {
+  // requested (`is_short`: the last, short one).  `sync` runs after the first k-slice.
+  auto phase = [&](auto ah, auto bh, auto rd, int rd_copy, auto rq, int rq_step, int rq_copy, auto is_short, auto sync) {
     constexpr int AH = decltype(ah)::value, BH = decltype(bh)::value - 2;
     constexpr int RD = decltype(rd)::value, RQ = decltype(rq)::value;
     constexpr int NB = BH ? BJ1 : BJ0, KS = AI * NB, NM = 4 * KS;
@@ -445,16 +441,19 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
       if constexpr (NQ > 0) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
-          if (KS + (2 * q + 1) * (NM - KS) / (2 * NQ) == m) request(rq, q, rq_step, rq_copy);
+          if (KS + (2 * q + 1) * (NM - KS) / (2 * NQ) == m) {
+            if constexpr (decltype(is_short)::value) request_short(rq, q, rq_step, rq_copy, rem);
+            else request(rq, q, rq_step, rq_copy);
+          }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   // Step `it`, with LEFT more steps behind it.  LEFT == CP: so many at least, and step it + CP is requested (SHORT:
-  // it is the short one, written here).
+  // it is the short one).
   auto do_step = [&](int it, auto left, auto is_short) {
     constexpr int LEFT = decltype(left)::value;
-    constexpr bool SHORT = decltype(is_short)::value, STEADY = LEFT == CP && !SHORT;
+    constexpr bool STEADY = LEFT == CP;
     constexpr int YOUNGER = LEFT < CP - 1 ? LEFT : CP - 1;  // whole steps requested after this one
     const int copy = it % CP, next = (it + 1) % CP;
     auto s1 = [] {
@@ -474,7 +473,7 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
     using QB1 = std::conditional_t<STEADY, B1, None>;
     using NA = std::conditional_t<(LEFT > 0), A0, None>;
     using NB = std::conditional_t<(LEFT > 0), B0, None>;
-    phase(A0{}, B0{}, B1{}, copy, QA0{}, it + CP, copy, s1);
+    phase(A0{}, B0{}, B1{}, copy, QA0{}, it + CP, copy, is_short, s1);
     if constexpr (HAS_BIAS && !SPLIT_K && LEFT == 0) {  // arrives under the last three phases
 #pragma unroll
       for (int j = 0; j < BJ; ++j) {
@@ -482,18 +481,16 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
         bias_v[j] = col < N ? to_float(pr.bias[col]) : 0.f;
       }
     }
-    if constexpr (SHORT) tail(A0{}, it + CP, copy, rem), tail(B0{}, it + CP, copy, rem);
-    phase(A0{}, B1{}, A1{}, copy, QB0{}, it + CP, copy, no_sync);
-    phase(A1{}, B1{}, NA{}, next, QB1{}, it + CP, copy, s2);
-    if constexpr (SHORT) tail(B1{}, it + CP, copy, rem), tail(A1{}, it + CP, copy, rem);
-    phase(A1{}, B0{}, NB{}, next, QA1{}, it + CP, copy, no_sync);
-    if constexpr (SHORT) MG_WAIT_VMCNT(0);  // the next steps' counts of younger requests do not hold
+    phase(A0{}, B1{}, A1{}, copy, QB0{}, it + CP, copy, is_short, no_sync);
+    phase(A1{}, B1{}, NA{}, next, QB1{}, it + CP, copy, is_short, s2);
+    phase(A1{}, B0{}, NB{}, next, QA1{}, it + CP, copy, is_short, no_sync);
   };
   // Requested in the order in which the steps before would have done it.
   auto request_all = [&](auto image, int step) {
     constexpr int IM = decltype(image)::value;
     if (step >= full_steps) {
-      tail(image, step, step, step == full_steps ? rem : 0);
+#pragma unroll
+      for (int i = 0; i < S::requests(IM); ++i) request_short(image, i, step, step, step == full_steps ? rem : 0);
       return;
     }
 #pragma unroll
@@ -506,8 +503,7 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
     request_all(B1{}, s);
     request_all(A1{}, s);
   }
-  if (full_steps < CP) MG_WAIT_VMCNT(0);  // (the short step's waves have fewer requests outstanding)
-  else MG_WAIT_VMCNT(RB1 + RA + (CP - 1) * R);
+  MG_WAIT_VMCNT(RB1 + RA + (CP - 1) * R);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int n = 0; n < 4 * AI; ++n) read(A0{}, n, 0);

@@ -7,7 +7,7 @@
 // and four times the workgroups take both down.  The price is LDS traffic: a 32 x 32 wave tile reads
 // two fragments per MFMA where a 64 x 64 one reads one, so half the matrix rate is the most this
 // kernel can reach, and products that fill the device with 128 x 128 tiles keep those.
-// Copies, LDS images, partial tiles and the order of every sum are those of gemm16_pipe_block.
+// Copies, LDS images, partial tiles and the order of every sum are those of gemm16_deep_block.
 #pragma once
 
 #include "gemm_impl.h"
@@ -116,7 +116,7 @@ __device__ __forceinline__ void gemm16_small_write(const floatx16& acc, uint16_t
   }
 }
 
-// The work of workgroup `bid` of a launch for one product (see gemm16_pipe_block); pr.tiles_m and
+// The work of workgroup `bid` of a launch for one product (see gemm16_deep_block); pr.tiles_m and
 // pr.tiles_n count tiles of 64.
 template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM>
 __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
@@ -172,23 +172,17 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
   auto request = [&](int step, int copy) {
     char* at = lds + copy * 2 * OP;
     if (step == full_steps) {
-      gemm16_pipe_tail<A_KC, BK, TT, NW>(a16 + step * a_step, src_a, rem, at);
-      gemm16_pipe_tail<B_KC, BK, TT, NW>(b16 + step * b_step, src_b, rem, at + OP);
+      gemm16_pipe_issue_short<A_KC, BK, TT, NW>(a16 + step * a_step, src_a, rem, at);
+      gemm16_pipe_issue_short<B_KC, BK, TT, NW>(b16 + step * b_step, src_b, rem, at + OP);
       return;
     }
     gemm16_pipe_issue<NI, NW>(a16 + step * a_step, src_a, at);
     gemm16_pipe_issue<NI, NW>(b16 + step * b_step, src_b, at + OP);
   };
 
-  float bias_v = 0.f;  // requested ahead of the tiles, see gemm16_pipe_block
-  if constexpr (HAS_BIAS && !SPLIT_K) {
-    const int col = n0 + wn + lane % 32;
-    bias_v = col < N ? to_float(pr.bias[col]) : 0.f;
-  }
 #pragma unroll
   for (int s = 0; s < NSTAGE; ++s)
     if (s < steps) request(s, s);
-  if constexpr (HAS_BIAS && !SPLIT_K) asm volatile("" : "+v"(bias_v));
   // The fragments of step `it` + 1 are read while those of step `it` are multiplied, so a step's one
   // synchronisation says two things: step it + 1 has arrived, and every wave holds its fragments of
   // step it, whose copy then takes step it + NSTAGE.
@@ -235,14 +229,14 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
       MG_WAIT_VMCNT(2 * NI * (NSTAGE - 2));
       meet();
     } else {
-      arrive(min(full_steps - 2 - it, NSTAGE - 2));  // (a short step has waited for every older one)
+      arrive(min(steps - 2 - it, NSTAGE - 2));
     }
     if (it + NSTAGE < steps) request(it + NSTAGE, it % NSTAGE);
     read(buf ^ 1, it + 1);
     __builtin_amdgcn_sched_barrier(0);
     multiply(buf);
   };
-  arrive(min(full_steps - 1, NSTAGE - 1));
+  arrive(min(steps - 1, NSTAGE - 1));
   read(0, 0);
   // two turns at a time, so that the fragment buffers have fixed names
   int it = 0;
@@ -253,6 +247,11 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
   for (; it + 2 < steps; it += 2) {
     turn(0, it, std::false_type{});
     turn(1, it + 1, std::false_type{});
+  }
+  float bias_v = 0.f;  // under the last products: ahead of the tiles, the wait for it took in all their copies
+  if constexpr (HAS_BIAS && !SPLIT_K) {
+    const int col = n0 + wn + lane % 32;
+    bias_v = col < N ? to_float(pr.bias[col]) : 0.f;
   }
   if (it + 1 < steps) {
     turn(0, it, std::false_type{});

@@ -686,20 +686,25 @@ __device__ __forceinline__ void gemm16_pipe_issue(const uint16_t* base, const in
   }
 }
 
-// The last, short step of a reduction that is no multiple of BK (`rem` k left, whole chunks of 8
-// for a k-contiguous operand): the same chunks through registers, zeros past the end, so nothing
-// beyond the operand is read and the step multiplies like any other.  The compiler waits for
-// these loads and with them for every older copy, once per tile.
+// The last, short step of a reduction that is no multiple of BK (`rem` k left, whole chunks of 8 for a
+// k-contiguous operand): chunks past the end are copied from sixteen bytes of zeros, so nothing beyond the operand
+// is read, the step multiplies like any other, and a wave's requests number the same in every step.  (Through
+// registers the tail waited for every older copy as well: (39, 625 <- 920), forward + backward, 17.3 us against
+// 15.3.)
+__device__ const uint32_t kGemmZeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 template <bool KC, int BK, int ROWS, int NW>
-__device__ __forceinline__ void gemm16_pipe_tail(const uint16_t* base, const int64_t* src, int rem, char* lds_step) {
+__device__ __forceinline__ void gemm16_pipe_issue_short(const uint16_t* base, const int64_t* src, int rem, char* lds_step) {
+  using lds_ptr = __attribute__((address_space(3))) char*;
   constexpr int CPR = BK / 8, CPK = ROWS / 8;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const unsigned dst = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)lds_step)) + wave * 1024;
 #pragma unroll
   for (int i = 0; i < gemm16_pipe_requests(ROWS, BK, NW); ++i) {
     const int slot = (i * NW + wave) * kWave + lane;
     const int k = KC ? ((slot % CPR) ^ ((slot / CPR / (16 / CPR)) % CPR)) * 8 : slot / CPK;
-    const uint4 v = k < rem ? *reinterpret_cast<const uint4*>(base + src[i]) : make_uint4(0, 0, 0, 0);
-    *reinterpret_cast<uint4*>(lds_step + slot * 16) = v;
+    const uint16_t* p = k < rem ? base + src[i] : reinterpret_cast<const uint16_t*>(kGemmZeros);
+    const unsigned dst_i = __builtin_amdgcn_readfirstlane(dst + i * NW * 1024);
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst_i), "v"(p) : "memory");
   }
 }
 
