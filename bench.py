@@ -1073,9 +1073,9 @@ def bench_gemm16(args, dev) -> dict:
         "metric": "fwd+bwd step ms; per-bwd-kernel HBM GB/s or MFMA % of MI355X peak", "value": round(ms, 4), "unit": "ms",
         "n_gpus": 1, "steps": min(args.steps, 20), "warmup": min(args.warmup, 3), "ms_per_step": round(ms, 4),
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
-        "config": {"workload": "bf16 Linear 8192 -> 8192 on 8192 rows: forward, dX and dW products (gemm_16bit_big_kernel), "
+        "config": {"workload": "bf16 Linear 8192 -> 8192 on 8192 rows: forward, dX and dW products (gemm_16bit_deep_kernel), "
                                "N(0,1) activations and gradients; the same at 4096 in the kernel table"},
-        "roofline": {"bound": "mfma", "kernel": "gemm_16bit_big_kernel, " + dom["name"], "achieved": dom["achieved_TFLOPs"],
+        "roofline": {"bound": "mfma", "kernel": "gemm_16bit_deep_kernel, " + dom["name"], "achieved": dom["achieved_TFLOPs"],
                      "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": dom["frac_of_mfma_peak"], "traffic": None},
         "kernels": kernels,
     }
