@@ -12,14 +12,14 @@
 // third of the device, and a sequence of 32 is one wave's work.  80 and 96 columns have kernels of
 // their own instead of the 128-column one.
 //   fp32 forward + backward, one MI355X, before -> now:
-//     (3, 777, 8 heads, 80), bias        645 -> 387 us      (1, 1236, 6, 256), causal  3930 -> 513 us
-//     (1, 176, 10, 80), bias             164 ->  55 us      (2, 8 heads of 1500, 128)   816 -> 765 us (*)
+//     (3, 777, 8 heads, 80), bias        645 -> 389 us      (1, 1236, 6, 256), causal  3930 -> 513 us
+//     (1, 176, 10, 80), bias             164 ->  56 us      (2, 8 heads of 1500, 128)   816 -> 765 us (*)
 //     (4, 32, 2, 32), causal              65 ->  18 us      (21, 79, 8, 32), causal      35 ->  27 us
 // (*: before the addresses below).  The arithmetic is the matrix pipe's: 64 cycles per 32 x 32 x 2 product, two
 // products per column and step forward, seven over the two backward kernels.  What stands beside it on the one
 // wave of a SIMD is vector arithmetic, 1300 instructions a step at 80 columns until the copies took a scalar base
 // and a byte offset per lane, the bias' places were computed once, and exp2f became the one instruction:
-// 414 -> 387 us at 777 rows with bias, 260 -> 227 us at (2, 8 heads of 1024, 64) with bias.
+// 414 -> 389 us at 777 rows with bias, 260 -> 228 us at (2, 8 heads of 1024, 64) with bias.
 //
 // Layouts as in attention_f32_mfma.h: a score tile comes out with the workgroup's rows along the
 // lanes and the streamed rows along the registers, which is the operand of the products that

@@ -689,8 +689,8 @@ __device__ __forceinline__ void gemm16_pipe_issue(const uint16_t* base, const in
 // The last, short step of a reduction that is no multiple of BK (`rem` k left, whole chunks of 8 for a
 // k-contiguous operand): chunks past the end are copied from sixteen bytes of zeros, so nothing beyond the operand
 // is read, the step multiplies like any other, and a wave's requests number the same in every step.  (Through
-// registers the tail waited for every older copy as well: (39, 625 <- 920), forward + backward, 17.3 us against
-// 15.3.)
+// registers the tail waited for every older copy as well: (39, 625 <- 920), forward + backward, 16.7 us against
+// 15.6.)
 __device__ const uint32_t kGemmZeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 template <bool KC, int BK, int ROWS, int NW>
 __device__ __forceinline__ void gemm16_pipe_issue_short(const uint16_t* base, const int64_t* src, int rem, char* lds_step) {
