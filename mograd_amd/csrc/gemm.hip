@@ -208,7 +208,9 @@ static double deep_16bit_us(Gemm16Tile tile, double items, double steps, bool sp
   const double per_cu = std::ceil(items / device_info().cu_count);
   if (tile == kTile256) return 4.0 + per_cu * ((items < 0.75 * device_info().cu_count ? 1.3 : 1.47) * steps + 1.5);
   const double pairs = std::floor(per_cu / 2), odd = per_cu - 2 * pairs, f = split_lines ? 1.3 : 1.0;
-  return 3.6 + f * steps * (tile == kTile192 ? 1.1 * pairs + 0.69 * odd : 0.85 * pairs + 0.46 * odd);
+  if (tile == kTile128) return 3.6 + f * steps * (0.85 * pairs + 0.46 * odd);
+  // (alone on its CU a 128 x 192 tile's ends stand in the open: (8192, 384 <- 128) 6.3 us, 5.2 with 128 x 128)
+  return 3.6 + f * steps * (1.1 * pairs + 0.69 * odd) + (pairs == 0 ? 0.7 : 0.0);
 }
 static double partials_us(double values) { return 2.6 + values * 8.0 / 3.5e6; }
 
