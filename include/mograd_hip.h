@@ -443,10 +443,10 @@ int mg_sgd_step(void* w, const void* g, int64_t n, float lr, mg_stream stream);
 /* the same stream, which sums everything on the list in one launch and empties it.  The   */
 /* sums use the code of the immediate forms: with grad_dtype == dtype the results are      */
 /* bit-identical to them, with MG_F32 they are the same fp32 sums before rounding.  A      */
-/* shape whose immediate form has no second stage, or none that can be deferred, is        */
-/* computed at once (and converted if grad_dtype differs).  The list keeps the partial     */
-/* results' pool blocks until it is finished or destroyed.  One list serves one stream     */
-/* and one host thread at a time.                                                          */
+/* shape whose immediate form has no second stage is computed at once, dw and db in        */
+/* grad_dtype from the accumulators (a scatter_add without index slabs converts its        */
+/* result).  The list keeps the partial results' pool blocks until it is finished or       */
+/* destroyed.  One list serves one stream and one host thread at a time.                   */
 /* ------------------------------------------------------------------------------------ */
 
 typedef void* mg_deferred;

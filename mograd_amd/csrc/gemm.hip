@@ -258,11 +258,19 @@ static int splitk_16bit_range(int64_t K, int* splits) {
   return k_per_split;
 }
 
-// Sums the K ranges of a 16-bit product's partial tiles (gemm16_partial_floats) into C.
+// Sums the K ranges of a 16-bit product's partial tiles (gemm16_partial_floats) into C, or leaves that to
+// mg_finish_deferred (same code, same order).
 template <typename T>
-static int launch_16bit_splitk_reduce(const GemmArgs& g, const float* partial, int splits, hipStream_t stream) {
+static int launch_16bit_splitk_reduce(const GemmArgs& g, Scratch& partial_mem, int splits, hipStream_t stream) {
+  const float* const partial = partial_mem.as<float>();
   const int64_t slice = gemm16_partial_floats(g.M, g.N, g.batch, 1);
   if (slice / 1024 > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
+  if (g.deferred) {
+    DeferredList* dl = deferred_current();
+    dl->push(kDeferSplitK, partial, g.c, slice, static_cast<int>(g.M), static_cast<int>(g.N), splits, ceil_div(slice / 4, 1024));
+    dl->hold(partial_mem);
+    return MG_OK;
+  }
   const unsigned blocks = static_cast<unsigned>(slice / 1024);  // whole tiles: four outputs per thread
   const T* bias = static_cast<const T*>(g.bias);
   T* c = static_cast<T*>(g.c);
@@ -286,11 +294,12 @@ static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream)
   Scratch partial;
   if (splits > 1)
     MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
-  const Gemm16Problem<T> pr{static_cast<const T*>(g.a), static_cast<const T*>(g.b), static_cast<const T*>(g.bias),
-                            static_cast<T*>(g.c), partial.as<float>(), static_cast<int>(g.M), static_cast<int>(g.N),
-                            static_cast<int>(g.K), A_KC ? g.sam : g.sak, B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb,
-                            g.M * g.N, static_cast<int>(tiles_m), static_cast<int>(tiles_n), k_per_split, splits,
-                            static_cast<int>(g.batch), epilogue_of<T>(g)};
+  Gemm16Problem<T> pr{static_cast<const T*>(g.a), static_cast<const T*>(g.b), static_cast<const T*>(g.bias),
+                      static_cast<T*>(g.c), partial.as<float>(), static_cast<int>(g.M), static_cast<int>(g.N),
+                      static_cast<int>(g.K), A_KC ? g.sam : g.sak, B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb,
+                      g.M * g.N, static_cast<int>(tiles_m), static_cast<int>(tiles_n), k_per_split, splits,
+                      static_cast<int>(g.batch), epilogue_of<T>(g)};
+  gemm16_gradient(g, pr);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, pr);
   };
@@ -298,7 +307,7 @@ static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream)
   else if (g.bias) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, true, false>);
   else launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, false>);
   MG_LAUNCH_CHECK();
-  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial, splits, stream) : MG_OK;
 }
 
 // Operands whose tiles cannot be copied straight into LDS (see dispatch_16bit): the register-staged kernel.
@@ -312,18 +321,26 @@ static int launch_16bit_staged(const GemmArgs& g, int splits, hipStream_t stream
   Scratch partial;
   if (splits > 1)
     MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
-  auto launch = [&](auto kernel, GemmEpilogue<T> ep) {
+  auto launch = [&](auto kernel, GemmEpilogue<T> ep, auto* c) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kGemmThreads), 0, stream, static_cast<const T*>(g.a),
-                       static_cast<const T*>(g.b), static_cast<const T*>(g.bias), static_cast<T*>(g.c), partial.as<float>(),
+                       static_cast<const T*>(g.b), static_cast<const T*>(g.bias), c, partial.as<float>(),
                        static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K), A_KC ? g.sam : g.sak,
                        B_KC ? g.sbn : g.sbk, g.N, g.bsa, g.bsb, g.M * g.N, tiles_m, tiles_n, k_per_split, splits,
                        static_cast<int>(g.batch), ep);
   };
-  if (splits > 1) launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, true>, GemmEpilogue<T>{nullptr, nullptr, 0});
-  else if (g.bias) launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, true, false>, epilogue_of<T>(g));
-  else launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, false>, epilogue_of<T>(g));
+  T* const c = static_cast<T*>(g.c);
+  if (splits > 1) {
+    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, true>, GemmEpilogue<T>{nullptr, nullptr, 0}, c);
+  } else if (g.c_f32) {
+    if constexpr (!A_KC && !B_KC)
+      launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, false, float>, epilogue_of<T>(g), static_cast<float*>(g.c));
+  } else if (g.bias) {
+    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, true, false>, epilogue_of<T>(g), c);
+  } else {
+    launch(gemm_16bit_mfma_kernel<T, A_KC, B_KC, false, false>, epilogue_of<T>(g), c);
+  }
   MG_LAUNCH_CHECK();
-  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial, splits, stream) : MG_OK;
 }
 
 // 16-bit MFMA path, split along K where the output has too few tiles to fill the device (dW of a narrow
@@ -335,6 +352,7 @@ template <typename T, bool A_KC, bool B_KC>
 static int launch_16bit(const GemmArgs& g, bool wide, hipStream_t stream) {
   const int64_t tiles128 = ceil_div(g.M, kGemmBM) * ceil_div(g.N, kGemmBN) * g.batch;
   const int64_t lda = A_KC ? g.sam : g.sak, ldb = B_KC ? g.sbn : g.sbk;
+  if (g.c_f32 && (A_KC || B_KC)) return fail(MG_ERR_UNSUPPORTED, "matmul: no kernel for an fp32 result of this layout");
   if (!wide)
     return launch_16bit_staged<T, A_KC, B_KC>(
         g, splitk_16bit_splits(tiles128, g.K, env_int("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", 2)), stream);
@@ -351,7 +369,7 @@ static int launch_16bit(const GemmArgs& g, bool wide, hipStream_t stream) {
   if (splits > 1)
     MG_TRY(partial.take(gemm16_partial_floats(g.M, g.N, g.batch, splits) * static_cast<int64_t>(sizeof(float))));
   MG_TRY(launch_16bit_deep<T>(g, static_cast<Gemm16Tile>(choice.tile), splits, k_per_split, partial.as<float>(), stream));
-  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial.as<float>(), splits, stream) : MG_OK;
+  return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial, splits, stream) : MG_OK;
 }
 
 static bool generic_grid_fits(const GemmArgs& g) { return ceil_div(g.M, 64) <= 65535 && g.batch <= 65535; }
@@ -426,10 +444,11 @@ static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handle
   // dimensions, extents and addresses are all multiples of 8 elements the tiles are copied
   // straight into LDS; otherwise they are staged through registers (the ragged variant), or,
   // where the product is long enough to pay for it, the operand is copied to rows that are.
-  const bool a_kc = g.sak == 1;
   const bool a_mc = g.sam == 1;
-  const bool b_kc = g.sbk == 1;
   const bool b_nc = g.sbn == 1;
+  // (fp32 weight gradients have kernels for dW's own layout alone, also where a width of 1 makes it both)
+  const bool a_kc = g.sak == 1 && !(g.c_f32 && a_mc);
+  const bool b_kc = g.sbk == 1 && !(g.c_f32 && b_nc);
   if (!((a_kc || a_mc) && (b_kc || b_nc))) return MG_OK;
   const bool a_wide = (a_kc ? mult8(g.sam) && mult8(g.K) : mult8(g.sak) && mult8(g.M)) && aligned16(g.a) && mult8(g.bsa);
   const bool b_wide = (b_kc ? mult8(g.sbn) && mult8(g.K) : mult8(g.sbk) && mult8(g.N)) && aligned16(g.b) && mult8(g.bsb);
@@ -468,6 +487,15 @@ static int launch_generic(const GemmArgs& g, hipStream_t stream) {
   const T* b = static_cast<const T*>(g.b);
   const T* bias = static_cast<const T*>(g.bias);
   T* c = static_cast<T*>(g.c);
+  if constexpr (sizeof(T) == 2) {
+    if (g.c_f32) {
+      hipLaunchKernelGGL((gemm_generic_kernel<T, false, float>), grid, dim3(256), 0, stream, a, b, bias, static_cast<float*>(g.c),
+                         static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K), g.sam, g.sak, g.sbk, g.sbn, g.N,
+                         g.bsa, g.bsb, g.M * g.N, epilogue_of<T>(g));
+      MG_LAUNCH_CHECK();
+      return MG_OK;
+    }
+  }
   if (bias)
     hipLaunchKernelGGL((gemm_generic_kernel<T, true>), grid, dim3(256), 0, stream, a, b, bias, c, static_cast<int>(g.M),
                        static_cast<int>(g.N), static_cast<int>(g.K), g.sam, g.sak, g.sbk, g.sbn, g.N, g.bsa, g.bsb,
@@ -530,7 +558,7 @@ int gemm_dispatch(const char* who, const GemmArgs& g_in, hipStream_t stream) {
 }
 
 int colsum_dispatch(const void* a, void* dst, int64_t outer, int64_t reduce, int64_t inner, int dtype,
-                    hipStream_t stream);  // reduce.hip
+                    hipStream_t stream, bool dst_f32 = false);  // reduce.hip
 int ln_bwd(const void* dy, const void* x, const void* gamma, const float* mean, const float* rstd, const void* residual,
            void* dx, void* dgamma, void* dbeta, int64_t rows, int64_t cols, float eps, int dtype,
            mg_stream stream);  // layer_norm.hip
@@ -688,19 +716,16 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   // pass over dY: (16384, 1536 <- 384) with db 71 -> 60.5 us against dX, dW and a separate
   // mg_sum_axis.  MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH=0: the separate column sum.
   Gemm16Problem<T> pw2 = pw;
-  // Partial tiles whose sum is deferred are read back at the end of the training step: stored past
-  // the caches they do not evict the activations the next kernels read (GPT step 2.48 -> 2.43 ms
-  // on one box; MOGRAD_HIP_DEFER_NT_STORE=0 keeps ordinary stores).
-  pw2.partial_stream = deferred_current() != nullptr && env_int("MOGRAD_HIP_DEFER_NT_STORE", 1) != 0;
+  DeferredList* const dl = deferred_current();
+  pw2.partial_stream = dl != nullptr && env_int("MOGRAD_HIP_DEFER_NT_STORE", 1) != 0;  // see gemm16_gradient
   Scratch db_part;
   int groups = 0;
   const bool db_here = db && env_int("MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH", 1) != 0;
   if (!split_sums) {
     // nothing to sum: where the gradients are wanted in fp32 they are written so here
-    DeferredList* dl = deferred_current();
     if (dl && dl->out_dtype == MG_F32) {
-      pw2.c32 = static_cast<float*>(dl->write_here(dw));
-      if (db_here) pw2.colsum32 = static_cast<float*>(dl->write_here(db));
+      pw2.c32 = static_cast<float*>(dw);
+      if (db_here) pw2.colsum32 = static_cast<float*>(db);
     } else if (db_here) {
       pw2.colsum = static_cast<T*>(db);
     }
@@ -738,7 +763,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   }
   const int dw_blocks = static_cast<int>(slice / 1024);  // 256 threads, four consecutive partial values each
   const int db_blocks = groups > 0 ? static_cast<int>(ceil_div(N, 64)) : 0;
-  if (DeferredList* dl = deferred_current()) {
+  if (dl) {
     // The sums of the K ranges are left to mg_finish_deferred (same code, same order).
     dl->push(kDeferSplitK, partial.as<float>(), dw, slice, static_cast<int>(N), static_cast<int>(K), splits,
              ceil_div(slice / 4, 1024));
@@ -832,6 +857,17 @@ static int linear_bwd_f32_one_launch(const void* dy, const void* x, const void* 
   return MG_OK;
 }
 
+// Whether the `_deferred` entry point that runs on this thread wants fp32 gradients of 16-bit tensors.
+static bool gradients_in_f32(int dtype) {
+  const DeferredList* dl = deferred_current();
+  return dl && dl->out_dtype == MG_F32 && dtype != MG_F32;
+}
+
+// db (N) = the column sums of dY (M, N): in the tensors' type, or as the running `_deferred` entry point wants them.
+static int linear_bwd_bias(const void* dy, void* db, int64_t M, int64_t N, int dtype, hipStream_t stream) {
+  return colsum_dispatch(dy, db, 1, M, N, dtype, stream, gradients_in_f32(dtype));
+}
+
 // dx may be null: the gradients of the weights alone.
 // *done: dX and dW are on their way; *db_done: so is db (else the caller sums dY's columns).
 int linear_bwd_products(const void* dy, const void* x, const void* w, void* dx, void* dw, void* db, int64_t M, int64_t N,
@@ -902,7 +938,7 @@ static int linear_bwd_impl(const void* dy, const void* x, const void* w, void* d
     MG_TRY(mg::linear_bwd_products(dy, x, w, dx, dw, db, M, N, K, x_is_relu_output ? x : nullptr, dx_accumulate, dtype,
                                    s, &done, &db_done));
     if (done) {
-      if (db && !db_done) MG_TRY(mg::colsum_dispatch(dy, db, 1, M, N, dtype, s));
+      if (db && !db_done) MG_TRY(mg::linear_bwd_bias(dy, db, M, N, dtype, s));
       return MG_OK;
     }
   }
@@ -917,9 +953,11 @@ static int linear_bwd_impl(const void* dy, const void* x, const void* w, void* d
   }
   if (dw) {  // dW (N,K) = dY^T (N,M) x X (M,K): reduction over M, dY read as an m-contiguous left operand
     mg::GemmArgs g{dy, x, nullptr, dw, 1, N, K, M, 1, N, K, 1, 0, 0, dtype};
+    g.deferred = mg::deferred_current() != nullptr;
+    g.c_f32 = mg::gradients_in_f32(dtype);
     MG_TRY(mg::gemm_dispatch("linear_bwd(dw)", g, s));
   }
-  if (db) MG_TRY(mg::colsum_dispatch(dy, db, 1, M, N, dtype, s));
+  if (db) MG_TRY(mg::linear_bwd_bias(dy, db, M, N, dtype, s));
   return MG_OK;
 }
 
@@ -940,12 +978,9 @@ int mg_linear_bwd_deferred(const void* dy, const void* x, const void* w, void* d
     return mg::fail(MG_ERR_INVALID, "linear_bwd_deferred: unsupported dtype %s", mg::dtype_name(dtype));
   MG_TRY(mg::deferred_check("linear_bwd_deferred", list, dtype, grad_dtype));
   if (M < 0 || N < 0 || K < 0) return mg::fail(MG_ERR_INVALID, "linear_bwd_deferred: negative size");
+  // (every kernel of a Linear backward writes dW and db in the type that they are wanted in: no substitutes)
   mg::DeferredScope scope(static_cast<mg::DeferredList*>(list), dtype, grad_dtype);
-  void *dw_use, *db_use;
-  MG_TRY(scope.substitute(dw, N * K, &dw_use));
-  MG_TRY(scope.substitute(db, N, &db_use));
-  MG_TRY(linear_bwd_impl(dy, x, w, dx, dw_use, db_use, M, N, K, dx_accumulate != 0, x_is_relu_output != 0, dtype, stream));
-  return scope.finish(mg::to_stream(stream));
+  return linear_bwd_impl(dy, x, w, dx, dw, db, M, N, K, dx_accumulate != 0, x_is_relu_output != 0, dtype, stream);
 }
 
 int mg_linear_bwd_layer_norm_bwd(const void* dy, const void* x, const void* w, const void* ln_x, const void* gamma,
@@ -960,30 +995,28 @@ int mg_linear_bwd_layer_norm_bwd(const void* dy, const void* x, const void* w, c
   if (list) MG_TRY(mg::deferred_check(who, list, dtype, grad_dtype));
   else if (grad_dtype != dtype) return mg::fail(MG_ERR_INVALID, "%s: without a deferred list the gradients have the tensors' dtype", who);
   hipStream_t s = mg::to_stream(stream);
-  auto run = [&](void* dw_use, void* db_use, void* dg_use, void* dbt_use) -> int {
+  auto run = [&](void* dg_use, void* dbt_use) -> int {
     bool done = false, db_done = false;
     const mg::LinearBwdLayerNorm ln{ln_x, gamma, mean, rstd, dg_use, dbt_use};
-    MG_TRY(mg::linear_bwd_products(dy, x, w, dx, dw_use, db_use, M, N, K, nullptr, dx_accumulate != 0, dtype, s, &done,
+    MG_TRY(mg::linear_bwd_products(dy, x, w, dx, dw, db, M, N, K, nullptr, dx_accumulate != 0, dtype, s, &done,
                                    &db_done, &ln));
     if (done) {
-      if (db_use && !db_done) MG_TRY(mg::colsum_dispatch(dy, db_use, 1, M, N, dtype, s));
+      if (db && !db_done) MG_TRY(mg::linear_bwd_bias(dy, db, M, N, dtype, s));
       return MG_OK;
     }
     // Other shapes: dY W into a scratch tensor with the separate entry's kernels, then the LayerNorm backward.
     mg::Scratch dy_ln;
     MG_TRY(dy_ln.take(M * K * static_cast<int64_t>(mg::dtype_size(dtype))));
-    MG_TRY(linear_bwd_impl(dy, x, w, dy_ln.as<char>(), dw_use, db_use, M, N, K, false, false, dtype, stream));
+    MG_TRY(linear_bwd_impl(dy, x, w, dy_ln.as<char>(), dw, db, M, N, K, false, false, dtype, stream));
     return mg::ln_bwd(dy_ln.as<char>(), ln_x, gamma, mean, rstd, dx_accumulate ? dx : nullptr, dx, dg_use, dbt_use, M, K,
                       0.f, dtype, stream);
   };
-  if (!list) return run(dw, db, dgamma, dbeta);
+  if (!list) return run(dgamma, dbeta);
   mg::DeferredScope scope(static_cast<mg::DeferredList*>(list), dtype, grad_dtype);
-  void *dw_use, *db_use, *dg_use, *dbt_use;
-  MG_TRY(scope.substitute(dw, N * K, &dw_use));
-  MG_TRY(scope.substitute(db, N, &db_use));
+  void *dg_use, *dbt_use;
   MG_TRY(scope.substitute(dgamma, K, &dg_use));
   MG_TRY(scope.substitute(dbeta, K, &dbt_use));
-  MG_TRY(run(dw_use, db_use, dg_use, dbt_use));
+  MG_TRY(run(dg_use, dbt_use));
   return scope.finish(s);
 }
 

@@ -314,7 +314,9 @@ __device__ __forceinline__ void gemm16_deep_ln_bwd(const floatx16 (&acc)[2][S::B
 
 // The work of workgroup `bid` of a launch for one product; `lds` is S::kLds bytes, aligned to 1024.
 // pr.tiles_m, pr.tiles_n count tiles of S::kTM x S::kTN.  COLSUM: the sums of A over k as well (see Gemm16Problem).  LN_BWD: see gemm16_deep_ln_bwd.
-template <typename T, class S, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM = false, bool LN_BWD = false>
+// OUT_F32: the result goes to pr.c32.
+template <typename T, class S, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM = false, bool LN_BWD = false,
+          bool OUT_F32 = false>
 __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
   constexpr int AI = S::AI, BJ0 = S::BJ0, BJ1 = S::BJ1, BJ = S::BJ, WN = S::WN, NT = S::kThreads, CP = S::COPIES;
   const int M = pr.M, N = pr.N;
@@ -548,6 +550,14 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
         }
       }
   } else {
+    if constexpr (OUT_F32) {
+      static_assert(!HAS_BIAS && !LN_BWD, "a weight gradient");
+#pragma unroll
+      for (int i = 0; i < 2 * AI; ++i)
+#pragma unroll
+        for (int j = 0; j < BJ; ++j) gemm16_write_f32(acc[i][j], pr.c32, M, N, pr.ldc, row0 + 32 * i, col0 + 32 * j, lane);
+      return;
+    }
     __syncthreads();  // every wave is done with the staged tiles: their memory serves the output
     const int64_t at = batch * pr.bsc;
     if constexpr (LN_BWD) {
@@ -565,10 +575,10 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
   }
 }
 
-template <typename T, class S, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
+template <typename T, class S, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool OUT_F32 = false>
 __global__ __launch_bounds__(S::kThreads, S::kOccupancy * S::WN / 2) void gemm_16bit_deep_kernel(Gemm16Problem<T> pr) {
   __shared__ __attribute__((aligned(1024))) char lds[S::kLds];
-  gemm16_deep_block<T, S, A_KC, B_KC, HAS_BIAS, SPLIT_K>(lds, blockIdx.x, pr);
+  gemm16_deep_block<T, S, A_KC, B_KC, HAS_BIAS, SPLIT_K, false, false, OUT_F32>(lds, blockIdx.x, pr);
 }
 
 // Both products of a Linear layer's backward in one launch: workgroups [0, n_dw) take the K ranges of
@@ -599,11 +609,12 @@ int launch_16bit_deep(const GemmArgs& g, Gemm16Tile tile, int splits, int k_per_
   const int64_t tiles_m = ceil_div(g.M, kGemm16TileM[tile]), tiles_n = ceil_div(g.N, kGemm16TileN[tile]);
   const int64_t grid = splits > 1 ? gemm_split_grid(tiles_m * tiles_n, splits, g.batch) : tiles_m * tiles_n * g.batch;
   if (grid > 0x7fffffffLL) return fail(MG_ERR_INVALID, "matmul: too many output tiles");
-  const Gemm16Problem<T> pr{static_cast<const T*>(g.a), static_cast<const T*>(g.b), static_cast<const T*>(g.bias),
-                            static_cast<T*>(g.c), partial, static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K),
-                            a_kc ? g.sam : g.sak, b_kc ? g.sbn : g.sbk, g.N, g.bsa, g.bsb, g.M * g.N,
-                            static_cast<int>(tiles_m), static_cast<int>(tiles_n), k_per_split, splits,
-                            static_cast<int>(g.batch), epilogue_of<T>(g)};
+  Gemm16Problem<T> pr{static_cast<const T*>(g.a), static_cast<const T*>(g.b), static_cast<const T*>(g.bias),
+                      static_cast<T*>(g.c), partial, static_cast<int>(g.M), static_cast<int>(g.N), static_cast<int>(g.K),
+                      a_kc ? g.sam : g.sak, b_kc ? g.sbn : g.sbk, g.N, g.bsa, g.bsb, g.M * g.N,
+                      static_cast<int>(tiles_m), static_cast<int>(tiles_n), k_per_split, splits,
+                      static_cast<int>(g.batch), epilogue_of<T>(g)};
+  gemm16_gradient(g, pr);
   auto with = [&](auto shape, auto a_layout, auto b_layout) {
     using S = decltype(shape);
     constexpr bool AK = decltype(a_layout)::value, BK = decltype(b_layout)::value;
@@ -612,6 +623,9 @@ int launch_16bit_deep(const GemmArgs& g, Gemm16Tile tile, int splits, int k_per_
     };
     if constexpr (S::AI == 1) {
       if (splits > 1) return launch(gemm_16bit_deep_kernel<T, S, AK, BK, false, true>);
+    }
+    if constexpr (!AK && !BK) {
+      if (g.c_f32) return launch(gemm_16bit_deep_kernel<T, S, AK, BK, false, false, true>);
     }
     if (g.bias) launch(gemm_16bit_deep_kernel<T, S, AK, BK, true, false>);
     else launch(gemm_16bit_deep_kernel<T, S, AK, BK, false, false>);

@@ -21,7 +21,7 @@ constexpr int kSmallLdsBytes = kSmallStages * 2 * kSmallT * kSmallBK * 2;
 
 // Output of the 64 x 64 tile: see gemm16_write_tile.  Each wave stages its quadrant, then all 256
 // threads store 16 bytes of two rows each.
-template <typename T, bool HAS_BIAS, bool SPLIT_K, bool COLSUM>
+template <typename T, bool HAS_BIAS, bool SPLIT_K, bool MAY_F32>
 __device__ __forceinline__ void gemm16_small_write(const floatx16& acc, uint16_t* __restrict__ strip,
                                                    const Gemm16Problem<T>& pr, int batch, int split, int m0, int n0,
                                                    int wm, int wn, int lane, float bias_v) {
@@ -40,15 +40,9 @@ __device__ __forceinline__ void gemm16_small_write(const floatx16& acc, uint16_t
     }
     return;
   } else {
-    if constexpr (COLSUM) {
-      if (pr.c32) {  // dW of a layer whose gradients are kept in fp32: rows of 128 bytes per wave and store
-        const int col = n0 + wn + lane % 32;
-        if (col >= N) return;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = m0 + wm + (r / 4) * 8 + (lane / 32) * 4 + r % 4;
-          if (row < M) pr.c32[static_cast<int64_t>(row) * pr.ldc + col] = acc[r];
-        }
+    if constexpr (MAY_F32) {
+      if (pr.c32) {
+        gemm16_write_f32(acc, pr.c32, M, N, pr.ldc, m0 + wm, n0 + wn, lane);
         return;
       }
     }
@@ -117,8 +111,8 @@ __device__ __forceinline__ void gemm16_small_write(const floatx16& acc, uint16_t
 }
 
 // The work of workgroup `bid` of a launch for one product (see gemm16_deep_block); pr.tiles_m and
-// pr.tiles_n count tiles of 64.
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM>
+// pr.tiles_n count tiles of 64.  MAY_F32: pr.c32 is looked at.
+template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM, bool MAY_F32 = COLSUM>
 __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
   constexpr int TT = kSmallT, BK = kSmallBK, NSTAGE = kSmallStages, NW = 4;
   constexpr int NI = gemm16_pipe_requests(TT, BK, NW);  // copy requests per thread, operand and step
@@ -273,14 +267,15 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
       }
     }
   }
-  gemm16_small_write<T, HAS_BIAS, SPLIT_K, COLSUM>(acc, reinterpret_cast<uint16_t*>(lds), pr, batch, split, m0, n0, wm, wn, lane,
+  gemm16_small_write<T, HAS_BIAS, SPLIT_K, MAY_F32>(acc, reinterpret_cast<uint16_t*>(lds), pr, batch, split, m0, n0, wm, wn, lane,
                                            bias_v);
 }
 
 template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
 __global__ __launch_bounds__(256, 2) void gemm_16bit_small_kernel(Gemm16Problem<T> pr) {
   __shared__ __attribute__((aligned(1024))) char lds[kSmallLdsBytes];
-  gemm16_small_block<T, A_KC, B_KC, HAS_BIAS, SPLIT_K, false>(lds, blockIdx.x, pr);
+  // (dW = dY^T X is the layout that fp32 weight gradients come in)
+  gemm16_small_block<T, A_KC, B_KC, HAS_BIAS, SPLIT_K, false, !A_KC && !B_KC && !HAS_BIAS>(lds, blockIdx.x, pr);
 }
 
 // dX and dW (with db, the column sums of dY) of a Linear layer in one launch, see

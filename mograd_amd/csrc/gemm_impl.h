@@ -94,6 +94,10 @@ struct GemmArgs {
   const void* residual = nullptr;
   const void* relu_mask = nullptr;
   int relu = 0;
+  // A weight gradient (no epilogue, one batch) of a `_deferred` entry point: the sum of its K ranges may be left on the
+  // current list; c_f32: C is fp32 where A and B are 16-bit, written from the accumulators.
+  bool deferred = false;
+  bool c_f32 = false;
 };
 
 template <typename T>
@@ -119,9 +123,9 @@ __device__ __forceinline__ T gemm_finish(float v, const GemmEpilogue<T>& ep, int
 
 constexpr int kGenericBK = 16;  // k per step
 
-template <typename T, bool HAS_BIAS>
+template <typename T, bool HAS_BIAS, typename OutT = T>
 __global__ __launch_bounds__(256) void gemm_generic_kernel(const T* __restrict__ A, const T* __restrict__ B,
-                                                           const T* __restrict__ bias, T* __restrict__ C, int M, int N,
+                                                           const T* __restrict__ bias, OutT* __restrict__ C, int M, int N,
                                                            int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn,
                                                            int64_t ldc, int64_t bsa, int64_t bsb, int64_t bsc,
                                                            GemmEpilogue<T> ep) {
@@ -176,7 +180,8 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const T* __restrict__
       if (gm < M && gn < N) {
         const float bv = HAS_BIAS ? to_float(bias[gn]) : 0.f;
         const int64_t at = static_cast<int64_t>(gm) * ldc + gn;
-        C[at] = gemm_finish<T>(acc[i][j] + bv, ep, at);
+        if constexpr (std::is_same_v<OutT, T>) C[at] = gemm_finish<T>(acc[i][j] + bv, ep, at);
+        else C[at] = acc[i][j];  // (an fp32 weight gradient has neither bias nor epilogue)
       }
     }
 }
@@ -363,6 +368,18 @@ __device__ __forceinline__ void gemm16_store8(T* p, const float (&v)[8]) {
   *reinterpret_cast<gemm_u4_any*>(p) = r;
 }
 
+// A 32 x 32 accumulator block at (row0, col0) into an fp32 C, as it lies in the registers: every store is two runs of 128 bytes.
+__device__ __forceinline__ void gemm16_write_f32(const floatx16& acc, float* __restrict__ C, int M, int N, int64_t ldc, int row0,
+                                                 int col0, int lane) {
+  const int col = col0 + lane % 32;
+  if (col >= N) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int row = row0 + (r / 4) * 8 + (lane / 32) * 4 + r % 4;
+    if (row < M) C[static_cast<int64_t>(row) * ldc + col] = acc[r];
+  }
+}
+
 // Output of one 128x128 tile from the four waves' accumulators (wave tile 64x64 at (wm, wn)).
 // The accumulators have lanes along n and registers along m, so a direct store writes
 // 2-byte elements.  Each wave instead transposes its tile through `mine`, 64 rows of kG16Stride
@@ -518,9 +535,9 @@ struct Gemm16LayerNormBwd {
   float* part_b = nullptr;
 };
 
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
+template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, typename OutT = T>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
-    const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ bias, T* __restrict__ C,
+    const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ bias, OutT* __restrict__ C,
     float* __restrict__ partial, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t bsa, int64_t bsb,
     int64_t bsc, int tiles_m, int tiles_n, int k_per_split, int splits, int batches, GemmEpilogue<T> ep) {
   __shared__ __attribute__((aligned(16))) uint16_t lds_a[kGemmBM * kG16Stride];
@@ -590,10 +607,18 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
     __syncthreads();
   }
 
-  uint16_t* mine = (wave < 2 ? lds_a : lds_b) + (wave % 2) * 64 * kG16Stride;  // staging memory, idle now
-  gemm16_write_tile<T, HAS_BIAS, SPLIT_K>(acc, mine, bias, C, partial, M, N, ldc, bsc, batch,
-                                          split, SPLIT_K ? batches : 1,
-                                          m0, n0, wm, wn, lane, ep, false, HAS_BIAS && !SPLIT_K ? bias_v : nullptr);
+  if constexpr (!std::is_same_v<OutT, T>) {
+    static_assert(!SPLIT_K && !HAS_BIAS, "a whole weight gradient");
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) gemm16_write_f32(acc[i][j], C, M, N, ldc, m0 + wm + 32 * i, n0 + wn + 32 * j, lane);
+  } else {
+    uint16_t* mine = (wave < 2 ? lds_a : lds_b) + (wave % 2) * 64 * kG16Stride;  // staging memory, idle now
+    gemm16_write_tile<T, HAS_BIAS, SPLIT_K>(acc, mine, bias, C, partial, M, N, ldc, bsc, batch,
+                                            split, SPLIT_K ? batches : 1,
+                                            m0, n0, wm, wn, lane, ep, false, HAS_BIAS && !SPLIT_K ? bias_v : nullptr);
+  }
 }
 
 // ------------------------------------------------------------------------------------
@@ -751,16 +776,27 @@ struct Gemm16Problem {
   // first tile column also sum their A tiles over k, i.e. dY over its rows, and leave one
   // partial row of the bias gradient per K range at colsum_part[split * M + m].
   float* colsum_part = nullptr;
-  // Not split (64 x 64 tiles only): the sums themselves, or dW and the sums in fp32 instead of C and colsum.
+  // Not split (64 x 64 tiles only): the sums themselves, or in fp32.
   T* colsum = nullptr;
-  float* c32 = nullptr;
   float* colsum32 = nullptr;
+  // An fp32 C (not split), see GemmArgs::c_f32.
+  float* c32 = nullptr;
   // The partial tiles are read back much later (their sum is deferred to the end of a training
   // step): store them past the caches.
   bool partial_stream = false;
   // The output continues as a LayerNorm backward inside the launch (gemm16_deep_ln_bwd).
   Gemm16LayerNormBwd<T> ln;
 };
+
+// How a product's weight gradient is to be left (GemmArgs::deferred, c_f32).
+// Partial tiles whose sum is deferred are read back at the end of the training step: stored past
+// the caches they do not evict the activations the next kernels read (GPT step 2.48 -> 2.43 ms
+// on one box; MOGRAD_HIP_DEFER_NT_STORE=0 keeps ordinary stores).
+template <typename T>
+inline void gemm16_gradient(const GemmArgs& g, Gemm16Problem<T>& pr) {
+  pr.partial_stream = g.deferred && env_int("MOGRAD_HIP_DEFER_NT_STORE", 1) != 0;
+  if (g.c_f32) pr.c32 = static_cast<float*>(g.c);
+}
 
 // The output tiles of gemm_16bit_deep.h.
 enum Gemm16Tile { kTile128 = 0, kTile192 = 1, kTile256 = 2, kTileWide = 3 };  // 128 x 128, 128 x 192, 256 x 256, 128 x 384

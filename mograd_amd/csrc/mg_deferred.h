@@ -51,7 +51,6 @@ struct DeferredList {
   // substitutions (from, to) of output pointers made for it (see DeferredScope).
   int out_dtype = MG_F32;
   std::vector<std::pair<void*, void*>> redirect;
-  std::vector<void*> written;  // real outputs that the call's kernels wrote themselves, in out_dtype
 
   void* target(void* out) const {
     for (const auto& r : redirect)
@@ -60,11 +59,6 @@ struct DeferredList {
   }
   void push(int kind, const float* part, void* out, int64_t slice, int rows, int cols, int groups, int64_t blocks) {
     jobs.push_back(DeferredJob{part, target(out), slice, kind, out_dtype, rows, cols, groups, static_cast<int>(blocks)});
-  }
-  // Where a kernel that can write `out` in out_dtype itself is to write it.
-  void* write_here(void* out) {
-    written.push_back(target(out));
-    return written.back();
   }
   // Takes over the pool block of `s`: it now lives until the list is finished.
   void hold(Scratch& s) {
@@ -82,8 +76,8 @@ inline int64_t deferred_column_blocks(int variant, int64_t cols) {
 }
 
 // Makes `list` current for one entry point.  An output whose element type differs from the
-// tensors' (fp32 gradients of a 16-bit layer) is replaced by a scratch buffer of the tensors'
-// type for the duration: whatever part of the call defers its sum is redirected to write the
+// tensors' (fp32 gradients of 16-bit tensors) and that not every kernel behind the entry point can write
+// is replaced by a scratch buffer of the tensors' type for the duration: whatever part of the call defers its sum is redirected to write the
 // real output in `out_dtype`; outputs that the call produced at once are converted afterwards
 // (finish()).
 class DeferredScope {
@@ -91,13 +85,11 @@ class DeferredScope {
   DeferredScope(DeferredList* list, int dtype, int out_dtype) : list_(list), dtype_(dtype), out_dtype_(out_dtype) {
     list_->out_dtype = out_dtype;
     list_->redirect.clear();
-    list_->written.clear();
     deferred_set_current(list_);
   }
   ~DeferredScope() {
     deferred_set_current(nullptr);
     list_->redirect.clear();
-    list_->written.clear();
     for (auto& t : temps_) pool_release(t.tmp);
   }
   // The pointer to hand to the kernels in place of `out` (numel elements).
@@ -112,10 +104,10 @@ class DeferredScope {
     return MG_OK;
   }
   // After the entry point's work is enqueued: converts the substituted outputs that no
-  // deferred job or kernel took over.
+  // deferred job took over.
   int finish(hipStream_t stream) {
     for (const auto& t : temps_) {
-      bool deferred = std::find(list_->written.begin(), list_->written.end(), t.real) != list_->written.end();
+      bool deferred = false;
       for (size_t j = t.first_job; j < list_->jobs.size(); ++j) deferred |= list_->jobs[j].out == t.real;
       if (!deferred) MG_TRY(mg_cast(t.tmp, t.real, t.numel, dtype_, out_dtype_, stream));
     }

@@ -11,9 +11,9 @@ namespace mg {
 // the final value (one slab, one row lane); otherwise fp32 partials
 // (outer, slab * row_lanes + lane, inner) go to scratch and reduce_partials_cw_kernel finishes
 // in a fixed order.  No atomics.
-template <typename T, int VEC, bool DIRECT>
+template <typename T, int VEC, bool DIRECT, typename OutT = T>
 __global__ __launch_bounds__(256) void colsum_partial_kernel(const T* __restrict__ a, float* __restrict__ part,
-                                                             T* __restrict__ dst, int64_t reduce, int64_t inner,
+                                                             OutT* __restrict__ dst, int64_t reduce, int64_t inner,
                                                              int64_t rows_per_chunk, int tx_log2) {
   const int tx = 1 << tx_log2;
   const int ry = 256 >> tx_log2;
@@ -53,7 +53,12 @@ __global__ __launch_bounds__(256) void colsum_partial_kernel(const T* __restrict
 #pragma unroll
   for (int e = 0; e < VEC; ++e) out[e] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
   if constexpr (DIRECT) {
-    VecIO<T, VEC>::store(dst + o * inner + col, out);
+    if constexpr (std::is_same_v<OutT, T>) {
+      VecIO<T, VEC>::store(dst + o * inner + col, out);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) dst[o * inner + col + e] = from_float<OutT>(out[e]);
+    }
   } else {
     float* q = part + ((o * gridDim.y + chunk) * ry + ly) * inner + col;
 #pragma unroll
@@ -67,8 +72,8 @@ __global__ __launch_bounds__(256) void colsum_partial_kernel(const T* __restrict
 // thread sums every 128th row with eight loads in flight; the 128 row lanes are then added
 // through LDS in a fixed order and the result is stored directly: no partial sums in
 // memory, no second launch, no atomics.
-template <typename T, int VEC>
-__global__ __launch_bounds__(1024) void colsum_slab_kernel(const T* __restrict__ a, T* __restrict__ dst,
+template <typename T, int VEC, typename OutT>
+__global__ __launch_bounds__(1024) void colsum_slab_kernel(const T* __restrict__ a, OutT* __restrict__ dst,
                                                            int64_t reduce, int64_t inner) {
   constexpr int PIECES = 8;             // 16-byte pieces per slab row
   constexpr int LANES = 1024 / PIECES;  // row lanes
@@ -121,13 +126,13 @@ __global__ __launch_bounds__(1024) void colsum_slab_kernel(const T* __restrict__
     float t = 0.f;
 #pragma unroll
     for (int s = 0; s < SL; ++s) t += tile2[s][threadIdx.x];
-    if (c < inner) dst[o * inner + c] = from_float<T>(t);
+    if (c < inner) dst[o * inner + c] = from_float<OutT>(t);
   }
 }
 
 // Sum over the last axis (inner == 1): one wave per output element.
-template <typename T>
-__global__ __launch_bounds__(256) void rowsum_kernel(const T* __restrict__ a, T* __restrict__ dst, int64_t outer,
+template <typename T, typename OutT>
+__global__ __launch_bounds__(256) void rowsum_kernel(const T* __restrict__ a, OutT* __restrict__ dst, int64_t outer,
                                                      int64_t reduce) {
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
   if (row >= outer) return;  // wave-uniform
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const T* __restrict__ a, T*
   float acc = 0.f;
   for (int64_t c = lane; c < reduce; c += kWave) acc += to_float(a[row * reduce + c]);
   acc = wave_sum(acc);
-  if (lane == 0) dst[row] = from_float<T>(acc);
+  if (lane == 0) dst[row] = from_float<OutT>(acc);
 }
 
 template <typename T>
@@ -157,21 +162,23 @@ __global__ __launch_bounds__(256) void relu_grad_kernel(const T* __restrict__ ou
   }
 }
 
-template <typename T>
-static int colsum_typed(const T* a, T* dst, int64_t outer, int64_t reduce, int64_t inner, hipStream_t stream) {
+// OutT: T, or float for the bias gradient of a 16-bit layer whose gradients are kept in fp32.  Inside a `_deferred` entry
+// point the second stage is left on its list.
+template <typename T, typename OutT>
+static int colsum_typed(const T* a, OutT* dst, int64_t outer, int64_t reduce, int64_t inner, hipStream_t stream) {
   if (reduce == 0) {
     // zero fill by kernel, not hipMemsetAsync: safe to record into a HIP graph
-    const int dtype = sizeof(T) == 4 ? MG_F32 : MG_F16;  // all-zero bits are zero in every float type
+    const int dtype = sizeof(OutT) == 4 ? MG_F32 : MG_F16;  // all-zero bits are zero in every float type
     return mg_fill(dst, 0.0, outer * inner, dtype, stream);
   }
   if (inner == 1) {
-    hipLaunchKernelGGL((rowsum_kernel<T>), dim3(static_cast<unsigned>(ceil_div(outer, 4))), dim3(256), 0, stream, a, dst,
+    hipLaunchKernelGGL((rowsum_kernel<T, OutT>), dim3(static_cast<unsigned>(ceil_div(outer, 4))), dim3(256), 0, stream, a, dst,
                        outer, reduce);
     MG_LAUNCH_CHECK();
     return MG_OK;
   }
   constexpr int WIDE = WideVec<T>::value;
-  const bool wide = inner % WIDE == 0 && aligned16(a) && aligned16(dst);
+  const bool wide = inner % WIDE == 0 && aligned16(a) && (aligned16(dst) || !std::is_same_v<OutT, T>);
   const int vec = wide ? WIDE : 1;
   // Wide matrices take the one-launch kernel: always when there is a 128-byte column slab
   // for every CU; with slabs for half the CUs only up to 48 MiB of input (half the CUs
@@ -182,7 +189,7 @@ static int colsum_typed(const T* a, T* dst, int64_t outer, int64_t reduce, int64
   const bool slab_fits = slabs >= cus || (2 * slabs >= cus && outer * reduce * inner * static_cast<int64_t>(sizeof(T)) <=
                                                                    (int64_t{48} << 20));
   if (wide && outer <= 65535 && reduce >= 128 && slab_fits && env_int("MOGRAD_HIP_COLSUM_SLAB", 1) != 0) {
-    hipLaunchKernelGGL((colsum_slab_kernel<T, WIDE>),
+    hipLaunchKernelGGL((colsum_slab_kernel<T, WIDE, OutT>),
                        dim3(static_cast<unsigned>(ceil_div(inner, 8 * WIDE)), static_cast<unsigned>(outer)), dim3(1024),
                        0, stream, a, dst, reduce, inner);
     MG_LAUNCH_CHECK();
@@ -207,10 +214,10 @@ static int colsum_typed(const T* a, T* dst, int64_t outer, int64_t reduce, int64
   const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(chunks), static_cast<unsigned>(outer));
   if (chunks == 1 && ry == 1) {
     if (wide)
-      hipLaunchKernelGGL((colsum_partial_kernel<T, WIDE, true>), grid, dim3(256), 0, stream, a, nullptr, dst, reduce,
+      hipLaunchKernelGGL((colsum_partial_kernel<T, WIDE, true, OutT>), grid, dim3(256), 0, stream, a, nullptr, dst, reduce,
                          inner, rows_per_chunk, tx_log2);
     else
-      hipLaunchKernelGGL((colsum_partial_kernel<T, 1, true>), grid, dim3(256), 0, stream, a, nullptr, dst, reduce, inner,
+      hipLaunchKernelGGL((colsum_partial_kernel<T, 1, true, OutT>), grid, dim3(256), 0, stream, a, nullptr, dst, reduce, inner,
                          rows_per_chunk, tx_log2);
     MG_LAUNCH_CHECK();
     return MG_OK;
@@ -219,32 +226,44 @@ static int colsum_typed(const T* a, T* dst, int64_t outer, int64_t reduce, int64
   Scratch part;
   MG_TRY(part.take(outer * groups * inner * static_cast<int64_t>(sizeof(float))));
   if (wide)
-    hipLaunchKernelGGL((colsum_partial_kernel<T, WIDE, false>), grid, dim3(256), 0, stream, a, part.as<float>(), dst,
-                       reduce, inner, rows_per_chunk, tx_log2);
+    hipLaunchKernelGGL((colsum_partial_kernel<T, WIDE, false>), grid, dim3(256), 0, stream, a, part.as<float>(),
+                       static_cast<T*>(nullptr), reduce, inner, rows_per_chunk, tx_log2);
   else
-    hipLaunchKernelGGL((colsum_partial_kernel<T, 1, false>), grid, dim3(256), 0, stream, a, part.as<float>(), dst,
-                       reduce, inner, rows_per_chunk, tx_log2);
+    hipLaunchKernelGGL((colsum_partial_kernel<T, 1, false>), grid, dim3(256), 0, stream, a, part.as<float>(),
+                       static_cast<T*>(nullptr), reduce, inner, rows_per_chunk, tx_log2);
   MG_LAUNCH_CHECK();
+  if (outer == 1) {
+    reduce_partials_or_defer<OutT>(part, dst, nullptr, static_cast<OutT*>(nullptr), groups, inner, device_info().cu_count, stream);
+    MG_LAUNCH_CHECK();
+    return MG_OK;
+  }
   for (int64_t o = 0; o < outer; ++o) {
-    launch_reduce_partials<T>(part.as<float>() + o * groups * inner, dst + o * inner, nullptr, nullptr, groups, inner,
-                              device_info().cu_count, stream);
+    launch_reduce_partials<OutT>(part.as<float>() + o * groups * inner, dst + o * inner, nullptr, nullptr, groups, inner,
+                                 device_info().cu_count, stream);
     MG_LAUNCH_CHECK();
   }
   return MG_OK;
 }
 
 int colsum_dispatch(const void* a, void* dst, int64_t outer, int64_t reduce, int64_t inner, int dtype,
-                    hipStream_t stream) {
+                    hipStream_t stream, bool dst_f32) {
   if (!is_float_dtype(dtype)) return fail(MG_ERR_INVALID, "sum_axis: unsupported dtype %s", dtype_name(dtype));
   if (outer < 0 || reduce < 0 || inner < 0)
     return fail(MG_ERR_INVALID, "sum_axis: bad shape (%lld, %lld, %lld)", static_cast<long long>(outer),
                 static_cast<long long>(reduce), static_cast<long long>(inner));
   if (outer == 0 || inner == 0) return MG_OK;
   if (!dst || (reduce > 0 && !a)) return fail(MG_ERR_INVALID, "sum_axis: null pointer argument");
+  auto run = [&](auto type) -> int {
+    using T = decltype(type);
+    if constexpr (sizeof(T) == 2) {
+      if (dst_f32) return colsum_typed(static_cast<const T*>(a), static_cast<float*>(dst), outer, reduce, inner, stream);
+    }
+    return colsum_typed(static_cast<const T*>(a), static_cast<T*>(dst), outer, reduce, inner, stream);
+  };
   switch (dtype) {
-    case MG_F32: return colsum_typed(static_cast<const float*>(a), static_cast<float*>(dst), outer, reduce, inner, stream);
-    case MG_F16: return colsum_typed(static_cast<const f16_t*>(a), static_cast<f16_t*>(dst), outer, reduce, inner, stream);
-    default: return colsum_typed(static_cast<const bf16_t*>(a), static_cast<bf16_t*>(dst), outer, reduce, inner, stream);
+    case MG_F32: return run(float{});
+    case MG_F16: return run(f16_t{});
+    default: return run(bf16_t{});
   }
 }
 
@@ -267,7 +286,7 @@ static int relu_grad_typed(const void* out, const void* up, void* dst, int64_t n
 extern "C" {
 
 int mg_sum_axis(const void* a, void* dst, int64_t outer, int64_t reduce, int64_t inner, int dtype, mg_stream stream) {
-  return mg::colsum_dispatch(a, dst, outer, reduce, inner, dtype, mg::to_stream(stream));
+  return mg::colsum_dispatch(a, dst, outer, reduce, inner, dtype, mg::to_stream(stream), false);
 }
 
 int mg_relu_grad(const void* out, const void* upstream, void* dst, int64_t n, int dtype, mg_stream stream) {

@@ -71,6 +71,42 @@ def test_linear_bwd_deferred_matches_immediate(device, pending, dtype, M, N, K, 
             np.testing.assert_array_equal(got_db, db0.to_numpy(), err_msg=f"db, grad_dtype {grad_dtype}")
 
 
+# Layers of a few hundred rows, whose products may go out together or apart; large ones with whole and with split
+# dW tiles; widths off the 16-byte chunks, long and short; a width of 1, which gives an operand two unit strides; no rows.
+@pytest.mark.parametrize("dtype,M,N,K", [
+    (BF16, 200, 3072, 1024), (F16, 200, 3072, 1024), (BF16, 64, 4096, 1024), (BF16, 1000, 4608, 1536), (BF16, 16384, 4096, 1024),
+    (BF16, 4096, 8192, 4096), (BF16, 2048, 384, 384), (BF16, 2048, 3000, 2000), (F16, 114, 1771, 383), (BF16, 1999, 1001, 767),
+    (BF16, 5000, 1, 384), (BF16, 300, 384, 1), (BF16, 60, 1, 40), (BF16, 0, 24, 16)])
+@pytest.mark.parametrize("entry", ["linear", "layer_norm"])
+@pytest.mark.parametrize("one_launch", ["1", "0"])
+def test_fp32_gradients_of_16bit_layers_are_fp32_sums(device, pending, monkeypatch, dtype, M, N, K, entry, one_launch):
+    # dW and db in fp32 against float64 products of the 16-bit inputs.  fp32 accumulation of M terms of random sign: every
+    # partial sum rounds by 2^-24 of itself at most, sqrt(M) of them in quadrature, a factor 4 for luck.  Through bf16 the
+    # error is 1e-3, through fp16 1.4e-4, at any M here above 20 times that.
+    if entry == "layer_norm" and (M > 2048 or M == 0):
+        pytest.skip("the same kernels as below")
+    monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", one_launch)  # 0: a launch for each product
+    lib, st = device.lib, device.stream
+    x, dy = (_rounded(normal(75, i, (max(M, 1), n)), dtype) for i, n in ((0, K), (1, N)))
+    bx, bdy = (AnyBuffer.from_numpy(device, a, dtype) for a in (x, dy))
+    bw = AnyBuffer.from_numpy(device, _rounded(normal(75, 2, (N, K), std=0.05), dtype), dtype)
+    dx = AnyBuffer.create(dtype, device, max(M, 1) * K)
+    dw, db = AnyBuffer.create(F32, device, N * K, fill=7.0), AnyBuffer.create(F32, device, N, fill=7.0)
+    if entry == "linear":
+        lib.mg_linear_bwd_deferred(P(bdy), P(bx), P(bw), P(dx), P(dw), P(db), M, N, K, 0, 0, dtype, F32, pending.h, st)
+    else:
+        gamma = AnyBuffer.create(dtype, device, K, fill=1.0)
+        mean, rstd = AnyBuffer.create(F32, device, M, fill=0.0), AnyBuffer.create(F32, device, M, fill=1.0)
+        dg, dbeta = AnyBuffer.create(F32, device, K), AnyBuffer.create(F32, device, K)
+        lib.mg_linear_bwd_layer_norm_bwd(P(bdy), P(bx), P(bw), P(bx), P(gamma), P(mean), P(rstd), P(dx), P(dw), P(db), P(dg),
+                                         P(dbeta), M, N, K, 0, dtype, F32, pending.h, st)
+    lib.mg_finish_deferred(pending.h, st)
+    x64, dy64 = x[:M].astype(np.float64), dy[:M].astype(np.float64)
+    for name, got, want in (("dw", dw.to_numpy((N, K)), dy64.T @ x64), ("db", db.to_numpy(), dy64.sum(axis=0))):
+        error, size = np.linalg.norm(got - want), np.linalg.norm(want)
+        assert error <= 4 * 2.0 ** -24 * np.sqrt(M) * size, f"{name}: relative error {error / max(size, 1e-30):.2e}"
+
+
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows,cols,residual", [(16384, 384, True), (2048, 4096, False), (64, 384, True), (9, 1000, True),
                                                 (3, 40000, False)])
