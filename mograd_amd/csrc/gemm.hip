@@ -199,16 +199,19 @@ static int splitk_16bit_splits(int64_t blocks, int64_t K, int wg_per_cu) {
 
 // What a 16-bit product costs, in us, in workgroups of one kind of tile: `items` of them (K ranges included),
 // each `steps` k-steps of 64.  A CU holds two workgroups of 128-row tiles, whose steps take 0.85 us (128 x
-// 128) and 1.1 us (128 x 192) for the pair, 0.46 and 0.69 us where there is one; a 256 x 256 tile, alone
+// 128) and 1.1 us (128 x 192) for the pair, 0.46 and 0.69 us where there is one at the end; 0.52 us where no CU has more than one
+// 128 x 128 tile, whose steps then wait for weights that no cache holds ((700, 1536) <- 1536: 16.6 us, 12.9 with
+// 64 x 64 tiles; (512, 3072) <- 1024 13.2, 11.5; (4096, 384) <- 1536 17.1, 14.9); a 256 x 256 tile, alone
 // on its CU, 1.47 us (1.3 where CUs stay idle) and 1.5 us until its first MFMA.  `split_lines`: rows of a k-contiguous operand that do not start on
 // cache lines, so that every 128 bytes of a copy are two lines, long enough to matter ((13037, 680) <- 7288: 177 us with 128 x 192
 // tiles, 147 with 256 x 256 ones).  The launch, the last epilogue and writing the result, which the tiles of a round do
-// together, come on top.  (From 40 products of 2048 to 32768 rows, 64 to 8192 columns and K 64 to 7288, most within 10 %.)
+// together, come on top.  (From 40 products of 2048 to 32768 rows, 64 to 8192 columns and K 64 to 7288, most within 10 %; over 339
+// of 32 to 16384 rows with weights from memory the choice is 0.2 % slower than the best kind of tile of each, five of them more than 5 %.)
 static double deep_16bit_us(Gemm16Tile tile, double items, double steps, bool split_lines) {
   const double per_cu = std::ceil(items / device_info().cu_count);
   if (tile == kTile256) return 4.0 + per_cu * ((items < 0.75 * device_info().cu_count ? 1.3 : 1.47) * steps + 1.5);
   const double pairs = std::floor(per_cu / 2), odd = per_cu - 2 * pairs, f = split_lines ? 1.3 : 1.0;
-  if (tile == kTile128) return 3.6 + f * steps * (0.85 * pairs + 0.46 * odd);
+  if (tile == kTile128) return 3.6 + f * steps * (0.85 * pairs + (pairs == 0 ? 0.52 : 0.46) * odd);
   // (alone on its CU a 128 x 192 tile's ends stand in the open: (8192, 384 <- 128) 6.3 us, 5.2 with 128 x 128)
   return 3.6 + f * steps * (1.1 * pairs + 0.69 * odd) + (pairs == 0 ? 0.7 : 0.0);
 }
