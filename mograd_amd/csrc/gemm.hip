@@ -595,26 +595,39 @@ static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
          env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) != 0;
 }
 
-// How the backward of a 16-bit layer goes out in one launch: with which tiles, and dW in how many K ranges.
-// Both products' k-steps (of 64) are dealt over the CUs; the longest chain of them in one workgroup is what a launch lasts at least.
-// For the 64 x 64 tiles of gemm_16bit_small.h: 3.1 us, 0.235 us per step; K ranges cost 3.1 us and 0.0082 us a
-// tile.  For the 128-row tiles as in deep_16bit_us, a chain's steps between the two figures there (it shares its
-// CU for a part of its life).  A range has at least 256 rows.  tile < 0: no such launch.
-// MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
+// How the backward of a 16-bit layer goes out: in one launch, with which tiles and dW in how many K ranges, or in a
+// launch for each product (tile < 0).  The least of these estimates, in us, is taken:
+//   64 x 64 tiles (gemm_16bit_small.h): the longest chain of k-steps (of 64) in one workgroup, 0.24 us a step, dW's and
+//     dX's together by 0.75 where they share CUs, by 0.95 where dX's start when dW's end, dW's a seventh longer with db; the steps of all workgroups dealt over the
+//     CUs, 0.168 us each, a third more where rows do not start on cache lines; of the two the longer, and 0.36 of the
+//     other.  What is read and written at 4 TB/s; K ranges 3.5 us and 0.0058 us a tile.  (From 176 layers of 64 to 2048 rows and 384 to 6144 columns, as in transformer
+//     blocks of few tokens, and 156 of 32 to 16384 rows and any multiples of 8 up to 6144: fp32 gradients with
+//     deferred sums and 16-bit ones at once, with and without db, 1 to 8 K ranges; rms 7 %.)
+//   128-row tiles: chain and load as in deep_16bit_us, a chain's steps between the two figures there (it shares its
+//     CU for a part of its life).  128 x 384 tiles, which carry a LayerNorm's backward: 1.5 us a step, against a
+//     launch of its own for that (from 30 layers of 1024 to 32000 rows, 10 %).
+//   a launch for each product, and 7 us of one or two more for the sum of dY's rows.  Off the 16-byte chunks dW is the
+//     register-staged kernel's, 5 us more: (114, 1771 <- 384) 20 us against 12.
+// So (320, 3072 <- 768) with db is one launch, 19.4 us against 26.6, and (320, 1536 <- 6144) without three, 29.0 against
+// 33.2; the route taken is 0.5 to 0.9 % slower than the best one of each of the 176 layers, 0.9 to 1.7 % of the 156.  The
+// type of the gradients is not part of it: fp32 and 16-bit ones, deferred or not, come from the same sums.
+// A range has at least 256 rows (64 x 64 tiles: 128).  MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
 static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx, bool with_db) {
   const double cus = device_info().cu_count;
   const double steps_w = static_cast<double>(ceil_div(M, kG16BK)), steps_x = static_cast<double>(ceil_div(N, kG16BK));
+  const double x_mb = static_cast<double>(M) * K * 2.0 / 1e6, w_mb = static_cast<double>(N) * K * 2.0 / 1e6;
   Choice16 small{kSmall, 1};
   {
     const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
-    const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0;
-    const double chain_x = with_dx ? steps_x : 0.0, load = (tiles_w * steps_w + tiles_x * steps_x) / cus;
+    const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0, chain_x = with_dx ? steps_x : 0.0;
+    auto together = [&](double tiles) { return tiles > 2 * cus ? 0.95 : tiles > cus ? 0.75 : 0.0; };
+    const double step = N % 64 == 0 && K % 64 == 0 ? 0.168 : 0.222;
     for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
-      double chain = std::max(steps_w / s, chain_x);
-      if (tiles_w * s + tiles_x > cus) chain = std::max(chain, 0.75 * (steps_w / s + chain_x));  // two share a CU
-      if (tiles_w * s > 2 * cus) chain = std::max(chain, 0.67 * (tiles_w * steps_w / cus + 2 * chain_x));  // dX starts last
-      const double t = 3.1 + 0.235 * std::max(1.5 * chain, load) + (s > 1 ? 3.1 + tiles_w * s * 0.0082 : 0.0) +
-                       static_cast<double>(M) * K * 2.0 / 5e6;
+      const double len = std::ceil(steps_w / s), chain_w = with_db ? 1.14 * len : len;
+      const double chain = 0.24 * std::max({chain_w, chain_x, together(tiles_w * s + tiles_x) * (chain_w + chain_x)});
+      const double load = step * (tiles_w * s * len + tiles_x * steps_x) / cus;
+      const double t = 3.5 + std::max(chain, load) + 0.36 * std::min(chain, load) +
+                       0.25 * (with_dx ? x_mb + 2.5 * w_mb : 1.5 * w_mb) + (s > 1 ? 3.5 + tiles_w * s * 0.0058 : 0.0);
       if (t < small.us) small.us = t, small.splits = s;
     }
     small.splits = static_cast<int>(env_int("MOGRAD_HIP_LINEAR_BWD_SPLITS", small.splits));
@@ -624,36 +637,35 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx,
   auto offer = [&](Gemm16Tile t, int s) {
     const double tiles_k = static_cast<double>(ceil_div(K, kGemm16TileN[t]));
     const double tiles_w = static_cast<double>(ceil_div(N, kGemmBM)) * tiles_k * s, tiles_x = static_cast<double>(ceil_div(M, kGemmBM)) * tiles_k;
-    const double len = std::ceil(steps_w / s), pair = t == kTile192 ? 1.1 : t == kTileWide ? 2.2 : 0.85, one = t == kTile192 ? 0.69 : t == kTileWide ? 2.2 : 0.46;
+    const double len = std::ceil(steps_w / s), pair = t == kTile192 ? 1.1 : t == kTileWide ? 1.5 : 0.85, one = t == kTile192 ? 0.69 : t == kTileWide ? 1.5 : 0.46;
     const double slots = t == kTileWide ? cus : 2 * cus;
     const double load = (tiles_w * len + tiles_x * steps_x) / slots * pair;
     const double chain = std::max(len, steps_x) * 0.5 * (pair + one);
-    const double us = 3.6 + std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0) +
-                      static_cast<double>(M) * K * 2.0 / 5e6 + partials_us(tiles_w * kGemmBM * kGemm16TileN[t]);
+    const double us = (t == kTileWide ? 4.0 : 3.6) + std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0) +
+                      x_mb / 5.0 + partials_us(tiles_w * kGemmBM * kGemm16TileN[t]);
     if (us < deep.us) deep = Choice16{t, s, us};
   };
+  const bool wide = wide_linear_bwd(M, N, K);
+  const int64_t only = env_int("MOGRAD_HIP_LINEAR_BWD_TILE", 0);  // 128 | 192
   if (!with_dx || ceil_div(N, kGemmBM) * ceil_div(K, kGemmBN) >= cus) {  // dW fills the device unsplit: a launch for each product
   } else if (env_str("MOGRAD_HIP_LINEAR_BWD_WIDE") && env_int("MOGRAD_HIP_LINEAR_BWD_WIDE", 1) == 0) {
     const Gemm16Tile t = K % 192 == 0 ? kTile192 : kTile128;
     const int s = splitk_16bit_splits(ceil_div(N, kGemmBM) * ceil_div(K, kGemmBN), M, 1);
     if (s > 1) offer(t, s);
-  } else if (wide_linear_bwd(M, N, K)) {
+  } else if (wide) {
     for (int s = 2; s <= most; ++s) offer(kTileWide, s);
   } else {
-    const int64_t only = env_int("MOGRAD_HIP_LINEAR_BWD_TILE", 0);  // 128 | 192
     for (int s = 2; s <= most; ++s) {
       if (only != 192) offer(kTile128, s);
       if (only != 128) offer(kTile192, s);
     }
   }
-  // (a launch of its own for each product, and 7 us of one or two more for the sum of dY's rows: (85, 2664 <- 632)
-  // 28 us with separate launches, 22 with one.  Off the 16-byte chunks dW is the register-staged kernel's, 5 us
-  // more: (114, 1771 <- 384) 20 us against 12.  The LayerNorm's backward is 6 us as one.)
-  if (deep.tile < 0) {
-    deep.us = choose_16bit(N, K, M, 1, false).us + (with_db ? 7.0 : 0.0) + (mult8(N) && mult8(K) ? 0.0 : 5.0);
-    if (with_dx) deep.us += choose_16bit(M, K, N, 1, N >= 1024 && N % 64 != 0).us;
+  if (deep.tile < 0 || (!wide && only == 0 && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE"))) {
+    double apart = choose_16bit(N, K, M, 1, false).us + (with_db ? 7.0 : 0.0) + (mult8(N) && mult8(K) ? 0.0 : 5.0);
+    if (with_dx) apart += choose_16bit(M, K, N, 1, N >= 1024 && N % 64 != 0).us;
+    if (apart < deep.us) deep = Choice16{-1, 1, apart};
   }
-  const bool is_small = small.us + (deep.tile == kTileWide ? 6.0 : 0.0) <= deep.us;
+  const bool is_small = small.us + (deep.tile == kTileWide ? std::max(6.0, 3.0 + x_mb) : 0.0) <= deep.us;
   // (A choice of the larger tiles' form is also one for them.)
   return env_int("MOGRAD_HIP_LINEAR_BWD_SMALL", is_small && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE")) != 0 ? small : deep;
 }
