@@ -1788,7 +1788,8 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = zero16();
   uint4 kr[KS], vt[DT], pf[4];
-  float m_run = -INFINITY, l_run[2] = {0.f, 0.f};
+  // (A row whose first steps hold scores of -inf only, where a masked key leaves it nothing else, goes on from here.)
+  float m_run = -__FLT_MAX__, l_run[2] = {0.f, 0.f};
   typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
   using lds_u4 = __attribute__((address_space(3))) const uintx4*;
   using lds_i16x4 = __attribute__((address_space(3))) short4_t*;
@@ -1816,9 +1817,9 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
     const uintx4 x = *reinterpret_cast<lds_u4>(static_cast<uintptr_t>(ra[ks] + mt * 32 * tile_row_bytes<DP>()));
     kr[ks] = make_uint4(x[0], x[1], x[2], x[3]);
   };
-  auto a_piece = [&](auto PC, auto FRESH, int ks) {
+  auto a_piece = [&](auto PC, int ks) {
     constexpr int P = decltype(PC)::value;
-    s[P] = Mma<T>::run(kr[ks], qf[ks], decltype(FRESH)::value && ks == 0 ? zero16() : s[P]);
+    s[P] = Mma<T>::run(kr[ks], qf[ks], ks == 0 ? zero16() : s[P]);
   };
   // The transposed fragment of rows 16 hf of a step of V for one 32-column block, and the product it goes into.
   auto l2_piece = [&](int hf, int dt) {
@@ -1889,7 +1890,7 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
       if (decltype(NEXT)::value && cc >= 1) {  // (the first fragments are on their way)
 #pragma unroll
         for (int ks = (cc - 1) * KS / 7; ks < cc * KS / 7; ++ks) {
-          a_piece(P0{}, std::true_type{}, ks);
+          a_piece(P0{}, ks);
           l1_piece(ks, 1);
         }
       }
@@ -1908,7 +1909,7 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
     for (int cc = 0; cc < 8; ++cc) {
       if (decltype(NEXT)::value) {
 #pragma unroll
-        for (int ks = part(cc, KS); ks < part(cc + 1, KS); ++ks) a_piece(P1{}, std::true_type{}, ks);
+        for (int ks = part(cc, KS); ks < part(cc + 1, KS); ++ks) a_piece(P1{}, ks);
       }
       if (decltype(PREV)::value) {
 #pragma unroll
@@ -1938,25 +1939,25 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
   }
   advance_k(first_step % 2 * BUF);
   advance_v(first_step % 3 * BUF);
-  // The first step: accumulator r of tile t stands for key n0 + 32 t + acc_row(r).  Every row of the matrix has a
-  // key in it, so its maximum is finite.
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) l1_piece(ks, 0);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) a_piece(P0{}, ks);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) l1_piece(ks, 1);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) a_piece(P1{}, ks);
+  advance_k(first_step % 2 ? -BUF : BUF);
+  // The first step's mask: accumulator r of tile t stands for key n0 + 32 t + acc_row(r).  Selected after the products:
+  // a score that may not be seen leaves nothing behind, whatever it is.
   const int n0 = step_key0(first_step);
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = n0 + 32 * t + acc_row(r, lane);
-      s[t][r] = key < a.S && (!CAUSAL || key <= m) ? 0.f : -INFINITY;
+      s[t][r] = key < a.S && (!CAUSAL || key <= m) ? s[t][r] : -INFINITY;
     }
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) l1_piece(ks, 0);
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) a_piece(P0{}, No{}, ks);
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) l1_piece(ks, 1);
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) a_piece(P1{}, No{}, ks);
-  advance_k(first_step % 2 ? -BUF : BUF);
   int i = first_step;
   if (i + 1 < nsteps) {
     step(No{}, Yes{}, i);

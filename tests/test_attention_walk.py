@@ -48,3 +48,52 @@ def test_forward_walk(device, monkeypatch, pipe, dtype, half_ulp, S, D):
             bound = (1.05 * half_ulp + 1e-4) * (mass + np.abs(want_o)) + (2.0 ** -24 if dtype == F16 else 0.0)
             assert (err <= bound).all(), (causal, steep, float((err / bound).max()))
             assert np.abs(lse.to_numpy((B, H, S)) - want_lse).max() <= 1e-4, (causal, steep)
+
+
+# 256 and 257 tokens: narrow causal heads take either kernel there.
+@pytest.mark.parametrize("pipe", ["default", "1"])
+@pytest.mark.parametrize("dtype,half_ulp,later", [(BF16, 2.0 ** -8, "inf"), (BF16, 2.0 ** -8, "nan"), (BF16, 2.0 ** -8, "overflow"),
+                                                  (F16, 2.0 ** -11, "inf"), (F16, 2.0 ** -11, "nan")])
+@pytest.mark.parametrize("S,D", [(256, 64), (257, 64), (300, 96)])
+def test_a_later_key_that_is_not_finite_does_not_reach_earlier_rows(device, monkeypatch, pipe, dtype, half_ulp, later, S, D):
+    # Every row before key `at` sees finite scores only; its neighbours in a tile of 32 keys are among these rows.
+    if pipe != "default":
+        monkeypatch.setenv("MOGRAD_HIP_ATTN_FWD_PIPE", pipe)
+    B, H, scale, at = 1, 2, D ** -0.5, S - 30
+    q, k, v = (round_to_dtype(normal(98, i, (B, S, H, D)), dtype) for i in range(3))
+    if later == "overflow":  # finite numbers whose product is not: 2^100 against 2^100 there, against 0 elsewhere
+        q[..., 0], k[..., 0] = 2.0 ** 100, 0.0
+    k_bad = k.copy()
+    k_bad[:, at, :, 0] = {"inf": np.inf, "nan": np.nan, "overflow": 2.0 ** 100}[later]
+    bq, bk, bv = (AnyBuffer.from_numpy(device, t, dtype) for t in (q, k_bad, v))
+    o, lse = AnyBuffer.create(dtype, device, B * H * S * D), AnyBuffer.create(F32, device, B * H * S)
+    device.lib.mg_flash_attn_fwd(bq.data_ptr(), bk.data_ptr(), bv.data_ptr(), None, o.data_ptr(), lse.data_ptr(), B, S, H, D,
+                                 scale, 1, 0, dtype, device.stream)
+    want_o, want_lse, mass = reference(*(t[:, :at].astype(np.float64) for t in (q, k, v)), scale, True)
+    got = o.to_numpy((B, H, S, D))[:, :, :at]
+    bound = (1.05 * half_ulp + 1e-4) * (mass + np.abs(want_o)) + (2.0 ** -24 if dtype == F16 else 0.0)
+    assert (np.abs(got - want_o) <= bound).all()
+    assert np.abs(lse.to_numpy((B, H, S))[:, :, :at] - want_lse).max() <= 1e-4
+
+
+@pytest.mark.parametrize("S,D", [(257, 64), (300, 96)])
+def test_a_row_whose_last_step_has_no_finite_score(device, S, D):
+    # Row 64 of a causal problem sees one key of the step that its walk begins with, and its score is -inf: the rest of the
+    # row is as without that key.
+    B, H, scale = 1, 2, D ** -0.5
+    q, k, v = (round_to_dtype(normal(99, i, (B, S, H, D)), BF16) for i in range(3))
+    q[:, :, :, 0] = 1.0
+    k_bad = k.copy()
+    k_bad[:, 64, :, 0] = -np.inf
+    bq, bk, bv = (AnyBuffer.from_numpy(device, t, BF16) for t in (q, k_bad, v))
+    o, lse = AnyBuffer.create(BF16, device, B * H * S * D), AnyBuffer.create(F32, device, B * H * S)
+    device.lib.mg_flash_attn_fwd(bq.data_ptr(), bk.data_ptr(), bv.data_ptr(), None, o.data_ptr(), lse.data_ptr(), B, S, H, D,
+                                 scale, 1, 0, BF16, device.stream)
+    q64, k64, v64 = (t.astype(np.float64) for t in (q, k, v))
+    s = np.einsum("bhd,bnhd->bhn", q64[:, 64], k64[:, :64]) * scale
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("bhn,bnhd->bhd", p / p.sum(-1, keepdims=True), v64[:, :64])
+    mass = np.einsum("bhn,bnhd->bhd", p / p.sum(-1, keepdims=True), np.abs(v64[:, :64]))
+    assert (np.abs(o.to_numpy((B, H, S, D))[:, :, 64] - want) <= (1.05 * 2.0 ** -8 + 1e-4) * (mass + np.abs(want))).all()
+    want_lse = s.max(-1) + np.log(p.sum(-1))
+    assert np.abs(lse.to_numpy((B, H, S))[:, :, 64] - want_lse).max() <= 1e-4
