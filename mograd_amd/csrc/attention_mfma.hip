@@ -2332,6 +2332,10 @@ bool attn_mfma_supported(int dtype, int64_t D, const void* const* ptrs, int nptr
   return true;
 }
 
+// The pipelined walks reach the 64 rows of a step by 32-bit byte offsets; tensors with longer rows take the kernels
+// with 64-bit ones.  (O's rows are no longer than Q's.)
+static bool row_offsets_fit(const AttnDims& a) { return a.ld < 1 << 24; }
+
 template <typename T, int DP, int DC = DP>
 static int fwd_typed(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse, AttnDims a,
                      float scale, bool causal, bool has_bias, hipStream_t stream) {
@@ -2339,7 +2343,7 @@ static int fwd_typed(const void* q, const void* k, const void* v, const void* ma
   // Two query blocks or more: the pipelined walk (one block, two steps: B32 H16 S128 causal 8.8 us against 8.1; two of
   // narrow causal heads, two and four steps: B64 H6 S256 D64 16.1 against 15.7, B13 H4 S199 7.5 against 7.8).
   if constexpr (DP <= 128) {
-    if (!has_bias && scale > 0.f && env_int("MOGRAD_HIP_ATTN_FWD_PIPE", a.S > (causal && DP == 64 ? 256 : 128)) != 0) {
+    if (!has_bias && scale > 0.f && row_offsets_fit(a) && env_int("MOGRAD_HIP_ATTN_FWD_PIPE", a.S > (causal && DP == 64 ? 256 : 128)) != 0) {
       auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, stream, static_cast<const T*>(q),
                            static_cast<const T*>(k), static_cast<const T*>(v), static_cast<T*>(o), lse, a, scale,
@@ -2443,7 +2447,7 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
   }
   // The pipelined dK/dV walk (head dims up to 64, no bias) reads the row statistics negated
   // and padded per (batch, head) to a multiple of 64 rows; the delta kernel writes both forms.
-  const bool pipe = DP <= 64 && !has_bias && env_int("MOGRAD_HIP_ATTN_DKDV_PIPE", 1) != 0;
+  const bool pipe = DP <= 64 && !has_bias && row_offsets_fit(a) && env_int("MOGRAD_HIP_ATTN_DKDV_PIPE", 1) != 0;
   const int s_pad = static_cast<int>(ceil_div(a.S, 64) * 64);
   const int64_t padded = pipe ? static_cast<int64_t>(a.B) * a.H * s_pad : 0;
   Scratch delta;

@@ -97,3 +97,42 @@ def test_a_row_whose_last_step_has_no_finite_score(device, S, D):
     assert (np.abs(o.to_numpy((B, H, S, D))[:, :, 64] - want) <= (1.05 * 2.0 ** -8 + 1e-4) * (mass + np.abs(want))).all()
     want_lse = s.max(-1) + np.log(p.sum(-1))
     assert np.abs(lse.to_numpy((B, H, S))[:, :, 64] - want_lse).max() <= 1e-4
+
+
+def test_rows_too_long_for_32bit_offsets(device):
+    # Packed Q, K, V with 180000 heads: 69 MB from a token to the next, so that the last rows of a step of 64 lie more than
+    # 4 GiB behind its first.  Three heads hold numbers and are compared with the same heads on their own; 24 GB in all.
+    lib, st, S, H, D, dtype = device.lib, device.stream, 130, 180000, 64, BF16
+    heads, row = (0, H // 2 + 1, H - 1), D * 2
+    big = lambda n: AnyBuffer.create(dtype, device, n, fill=0.125)
+    place = lambda buf, token, h, n: buf.data_ptr().value + ((token * n) * H + h) * row  # (n: 3 for packed, 1 for O)
+    small_in = [AnyBuffer.from_numpy(device, normal(100, h, (S, 4, D)), dtype) for h in range(3)]  # Q, K, V and dO of a head
+    qkv, d_qkv, o, d_o = big(S * 3 * H * D), big(S * 3 * H * D), big(S * H * D), big(S * H * D)
+    lse = AnyBuffer.create(F32, device, H * S)
+    for h, t in zip(heads, small_in):
+        for s in range(S):
+            src = t.data_ptr().value + s * 4 * row
+            for j in range(3):
+                lib.mg_copy_device(place(qkv, s, 0, 3) + (j * H + h) * row, src + j * row, row, st)
+            lib.mg_copy_device(place(d_o, s, h, 1), src + 3 * row, row, st)
+    p = lambda b: b.data_ptr()
+    for causal in (0, 1):
+        lib.mg_flash_attn_fwd_packed(p(qkv), None, p(o), p(lse), 1, S, H, D, D ** -0.5, causal, 0, dtype, st)
+        lib.mg_flash_attn_bwd_packed(p(d_o), p(o), p(qkv), None, p(lse), p(d_qkv), 1, S, H, D, D ** -0.5, causal, 0, dtype, st)
+        for h, t in zip(heads, small_in):
+            t = t.to_numpy((S, 4, D))
+            one = [AnyBuffer.from_numpy(device, np.ascontiguousarray(a), dtype) for a in (t[:, :3], t[:, 3])]
+            o1, l1, g1 = (AnyBuffer.create(d, device, n) for d, n in ((dtype, S * D), (F32, S), (dtype, S * 3 * D)))
+            lib.mg_flash_attn_fwd_packed(p(one[0]), None, p(o1), p(l1), 1, S, 1, D, D ** -0.5, causal, 0, dtype, st)
+            lib.mg_flash_attn_bwd_packed(p(one[1]), p(o1), p(one[0]), None, p(l1), p(g1), 1, S, 1, D, D ** -0.5, causal, 0, dtype, st)
+            got_o, got_g = AnyBuffer.create(dtype, device, S * D), AnyBuffer.create(dtype, device, S * 3 * D)
+            for s in range(S):
+                lib.mg_copy_device(got_o.data_ptr().value + s * row, place(o, s, h, 1), row, st)
+                for j in range(3):
+                    lib.mg_copy_device(got_g.data_ptr().value + (s * 3 + j) * row, place(d_qkv, s, 0, 3) + (j * H + h) * row, row, st)
+            for name, got, want in (("o", got_o, o1), ("gradients", got_g, g1)):
+                a, b = got.to_numpy().astype(np.float64), want.to_numpy().astype(np.float64)
+                # two kernels that round a probability and a result each: 2^-8 of the largest numbers, over the norm
+                assert np.linalg.norm(a - b) <= 2.0 ** -7 * np.linalg.norm(b), (causal, h, name)
+    del qkv, d_qkv, o, d_o, lse
+    lib.mg_pool_empty_cache()
