@@ -19,7 +19,8 @@
 // products per column and step forward, seven over the two backward kernels.  What stands beside it on the one
 // wave of a SIMD is vector arithmetic, 1300 instructions a step at 80 columns until the copies took a scalar base
 // and a byte offset per lane, the bias' places were computed once, and exp2f became the one instruction:
-// 414 -> 389 us at 777 rows with bias, 260 -> 228 us at (2, 8 heads of 1024, 64) with bias.
+// 414 -> 389 us at 777 rows with bias, 260 -> 228 us at (2, 8 heads of 1024, 64) with bias; 1.5 and 2 % of that went
+// back to weights below 2^-126, see f32_wave_exp2.
 //
 // Layouts as in attention_f32_mfma.h: a score tile comes out with the workgroup's rows along the
 // lanes and the streamed rows along the registers, which is the operand of the products that
@@ -40,9 +41,29 @@ namespace mg {
 
 constexpr int kF32WaveMaxD = 256;
 
-// v_exp_f32 alone: exp2f scales its argument around it so that results below 2^-126 come out as denormals, six
-// instructions for weights that 1 in a row's sum hides.
-__device__ __forceinline__ float f32_wave_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// 2^x of a lane's sixteen weights, as exp2f gives them.  exp2f scales its argument around v_exp_f32 so that results below
+// 2^-126 come out as denormals, which show where a key's weights are all such (its dK, dV) or its V is all there is, and costs
+// six instructions a weight; here that is done only where a lane of the wave has such a weight (x in [-150, -126): what a
+// mask hides is far below), and v_exp_f32 alone gives the same bits elsewhere.  Forward 99.5 us against 103 with exp2f,
+// (2, 8 heads of 1500, 128) 189.5 against 199; the dK/dV walk, whose accumulators then move about, is faster with exp2f:
+// whole backward 285 us against 290 (281 where both walks flushed them), (2, 8 heads of 1024, 64), bias, 162 against 165.
+__device__ __forceinline__ void f32_wave_exp2(f32x16& x) {
+  float least = x[0];
+#pragma unroll
+  for (int r = 1; r < 16; ++r) least = fminf(least, x[r]);
+  if (__builtin_expect(__any(least < -126.0f), 0)) {
+    float off = INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) off = fminf(off, fabsf(x[r] + 138.0f));
+    if (__any(off <= 12.0f)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x[r] = exp2f(x[r]);
+      return;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(x[r]);
+}
 
 // What the four waves of a workgroup share: the streamed rows of one tile of 32, nothing (each has a
 // tile of its own), or the head columns of one tile.
@@ -411,7 +432,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     // the sum and the result are relative to the same point).
     if (__any(m_tile > m + 8.0f)) {
       const float m_new = fmaxf(m, m_tile);
-      const float corr = m_new == -INFINITY ? 0.f : f32_wave_exp2(m - m_new);
+      const float corr = m_new == -INFINITY ? 0.f : exp2f(m - m_new);
       l *= corr;
 #pragma unroll
       for (int db = 0; db < W::NB; ++db)
@@ -421,10 +442,10 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
     }
     const float base = m == -INFINITY ? 0.f : m;  // (nothing visible to this row yet: its weights are zero)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[0][r] = f32_wave_exp2(s[0][r] - base);
-      l += s[0][r];
-    }
+    for (int r = 0; r < 16; ++r) s[0][r] -= base;
+    f32_wave_exp2(s[0]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) l += s[0][r];
     MG_F32_WAVE_WAIT(NI + NM);
     f32_wave_weighted<DP>(v_s, s[0], lane, acc);
     MG_F32_WAVE_WAIT(NI + NM);
@@ -454,7 +475,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = ml[0][w][lane % 32];
-      f[w] = mw == -INFINITY ? 0.f : f32_wave_exp2(mw - m);
+      f[w] = mw == -INFINITY ? 0.f : exp2f(mw - m);
       l_row += f[w] * ml[1][w][lane % 32];
     }
     f32_wave_merge<DP>(lds, acc, f, orow, row_ok, 1.0f / l_row, a.D, wave, lane);
@@ -564,9 +585,11 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
       float sv = s[0][r];
       if (HAS_BIAS) sv = fmaf(bias[r], kAttnLog2e, sv);
       const bool valid = j < a.S && (!CAUSAL || j <= i);
-      const float p = valid ? f32_wave_exp2(sv - lse2) : 0.f;
-      s[0][r] = p * (s[1][r] - dl);  // dS without the scale: K is unscaled, the scale goes on at the end
+      s[0][r] = valid ? sv - lse2 : -INFINITY;
     }
+    f32_wave_exp2(s[0]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[0][r] *= s[1][r] - dl;  // dS without the scale: K is unscaled, the scale goes on at the end
     f32_wave_weighted<DP>(k_s, s[0], lane, acc);
     MG_F32_WAVE_WAIT(NI + NM);
     copy_k(t + stride);
@@ -661,7 +684,7 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) v
           sv = fmaf(mt[F32Wave<32>::place(rr + e, (lane % 32) / 4, 0) + lane % 4], kAttnLog2e, sv);
         }
         const bool valid = i < a.S && (!CAUSAL || j <= i);
-        const float p = valid ? f32_wave_exp2(sv) : 0.f;
+        const float p = valid ? exp2f(sv) : 0.f;
         s[0][r] = p;
         s[1][r] = p * (s[1][r] - dv4[e]);
       }

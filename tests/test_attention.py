@@ -145,6 +145,35 @@ def test_f32_waves_on_their_own(device, monkeypatch, own, name, causal, with_mas
         assert _max_err(g, w) <= (1e-5 if D <= 128 else 2e-5), f"{what}: {_max_err(g, w)}"
 
 
+@pytest.mark.parametrize("own", ["0", "1"])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("S,D", [(40, 32), (40, 64), (70, 80), (40, 128), (40, 256)])
+def test_f32_waves_keep_denormal_weights(device, monkeypatch, own, name, causal, with_mask, S, D):
+    # Key 0 lies 89 below the others for every query: its weights, e^-89 / S, are denormals (some 2^-134), and its V alone
+    # is not zero, so the output and every gradient stand on them.
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_F32_WAVE", "1")
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_F32_OWN", own)
+    q, k, v, do = (np.zeros((1, S, 1, D), np.float32) for _ in range(4))
+    do = do.reshape(1, 1, S, D)
+    q[..., 0] = math.sqrt(D)
+    k[:, 0, :, 0] = -45.0 if with_mask else -89.0
+    m = np.zeros((1, 1, S, S), np.float32) if with_mask else None
+    if with_mask:
+        m[..., 0] = -44.0
+    v[:, 0] = 1e6 * normal(62, 0, (D,))
+    do[:, :, 1:] = 1e3 * normal(62, 1, (S - 1, D))
+    want = (O.sdpa_fwd(q, k, v, m, causal)[0], *O.sdpa_bwd(q, k, v, do, m, causal))
+    o, _, *grads = _fwd_bwd(device, q, k, v, do, m, causal)
+    for got, w, what in zip((o, *grads), want, ("o", "dq", "dk", "dv")):
+        # a weight is a whole number of 2^-149, some 30000 of them: 2e-5; its exponent, some 134 with three roundings, 4e-5
+        if what == "o":  # (row 0 has one key alone where the walk is causal)
+            got, w = got[:, :, 1:], w[:, :, 1:]
+        if what == "dv":
+            got, w = got[:, 0], w[:, 0]
+        err = np.abs(got - w).max() / np.abs(w).max()
+        assert err <= 2e-4, f"{what}: {err}"
+
+
 HALF_SHAPES = [(2, 2, 96, 64), (1, 3, 200, 64), (2, 1, 128, 128), (1, 2, 257, 32), (1, 1, 4, 8), (1, 2, 96, 256),
                (1, 2, 130, 72), (1, 1, 80, 512), (1, 2, 40, 192), (1, 2, 300, 256), (2, 1, 130, 200), (1, 1, 129, 136)]
 
