@@ -207,9 +207,9 @@ static int splitk_16bit_splits(int64_t blocks, int64_t K, int wg_per_cu) {
 // tiles, 147 with 256 x 256 ones).  The launch, the last epilogue and writing the result, which the tiles of a round do
 // together, come on top.  (From 40 products of 2048 to 32768 rows, 64 to 8192 columns and K 64 to 7288, most within 10 %; over 339
 // of 32 to 16384 rows with weights from memory the choice is 0.2 % slower than the best kind of tile of each, five of them more than 5 %.)
-static double deep_16bit_us(Gemm16Tile tile, double items, double steps, bool split_lines) {
-  const double per_cu = std::ceil(items / device_info().cu_count);
-  if (tile == kTile256) return 4.0 + per_cu * ((items < 0.75 * device_info().cu_count ? 1.3 : 1.47) * steps + 1.5);
+static double deep_16bit_us(Gemm16Tile tile, double items, double steps, bool split_lines, double cus) {
+  const double per_cu = std::ceil(items / cus);
+  if (tile == kTile256) return 4.0 + per_cu * ((items < 0.75 * cus ? 1.3 : 1.47) * steps + 1.5);
   const double pairs = std::floor(per_cu / 2), odd = per_cu - 2 * pairs, f = split_lines ? 1.3 : 1.0;
   if (tile == kTile128) return 3.6 + f * steps * (0.85 * pairs + (pairs == 0 ? 0.52 : 0.46) * odd);
   // (alone on its CU a 128 x 192 tile's ends stand in the open: (8192, 384 <- 128) 6.3 us, 5.2 with 128 x 128)
@@ -226,6 +226,8 @@ struct Choice16 {
   int splits;
   double us = 1e30;
 };
+// (A search stops where the partial tiles alone, which grow with the ranges, cost more than the best form so far:
+// every call makes this choice, (512, 512) <- 65536 from 71 estimates.)
 static Choice16 choose_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, bool split_lines) {
   const double cus = device_info().cu_count, steps = std::ceil(static_cast<double>(K) / kG16BK);
   const double out = static_cast<double>(M) * N * batch * 2.0 / 5e6;  // (rows off the 16-byte chunks: 0.8 us more in the larger tiles)
@@ -243,15 +245,18 @@ static Choice16 choose_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, boo
   for (int t = kTile128; t <= kTile256; ++t) {
     const double tiles = tiles_of(kGemm16TileM[t], kGemm16TileN[t]);
     for (int s = 1; s <= (t == kTile256 ? 1 : most); ++s) {
-      if (s > 1 && tiles * (s - 1) >= 2 * cus) break;
-      const double us = deep_16bit_us(static_cast<Gemm16Tile>(t), tiles * s, std::ceil(steps / s), split_lines);
-      offer(t, s, us + out + (N % 8 ? 0.8 : 0.0) + (s > 1 ? partials_us(tiles * s * kGemm16TileM[t] * kGemm16TileN[t]) : 0.0));
+      const double sums = s > 1 ? partials_us(tiles * s * kGemm16TileM[t] * kGemm16TileN[t]) : 0.0;
+      if (s > 1 && (tiles * (s - 1) >= 2 * cus || sums >= best.us)) break;
+      const double us = deep_16bit_us(static_cast<Gemm16Tile>(t), tiles * s, std::ceil(steps / s), split_lines, cus);
+      offer(t, s, us + out + (N % 8 ? 0.8 : 0.0) + sums);
     }
   }
   const double tiles64 = tiles_of(kSmallT, kSmallT);
-  for (int s = 1; s <= 16 && (s == 1 || (s <= most && tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s)
-    offer(kSmall, s, 3.4 + out + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) +
-                         (s > 1 ? partials_us(tiles64 * s * kSmallT * kSmallT) : 0.0));
+  for (int s = 1; s <= 16 && (s == 1 || (s <= most && tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s) {
+    const double sums = s > 1 ? partials_us(tiles64 * s * kSmallT * kSmallT) : 0.0;
+    if (sums >= best.us) break;
+    offer(kSmall, s, 3.4 + out + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) + sums);
+  }
   return best;
 }
 // The K range of one workgroup, a multiple of the k-step, and the number of ranges that leaves.
@@ -623,6 +628,7 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx,
     auto together = [&](double tiles) { return tiles > 2 * cus ? 0.95 : tiles > cus ? 0.75 : 0.0; };
     const double step = N % 64 == 0 && K % 64 == 0 ? 0.168 : 0.222;
     for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
+      if (s > 1 && 7.0 + tiles_w * s * 0.0058 >= small.us) break;
       const double len = std::ceil(steps_w / s), chain_w = with_db ? 1.14 * len : len;
       const double chain = 0.24 * std::max({chain_w, chain_x, together(tiles_w * s + tiles_x) * (chain_w + chain_x)});
       const double load = step * (tiles_w * s * len + tiles_x * steps_x) / cus;
@@ -634,16 +640,18 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx,
   }
   Choice16 deep{-1, 1};
   const int most = static_cast<int>(std::min<int64_t>(64, M / 256));
-  auto offer = [&](Gemm16Tile t, int s) {
+  auto offer = [&](Gemm16Tile t, int s) {  // false: more ranges are not worth a look
     const double tiles_k = static_cast<double>(ceil_div(K, kGemm16TileN[t]));
     const double tiles_w = static_cast<double>(ceil_div(N, kGemmBM)) * tiles_k * s, tiles_x = static_cast<double>(ceil_div(M, kGemmBM)) * tiles_k;
     const double len = std::ceil(steps_w / s), pair = t == kTile192 ? 1.1 : t == kTileWide ? 1.5 : 0.85, one = t == kTile192 ? 0.69 : t == kTileWide ? 1.5 : 0.46;
-    const double slots = t == kTileWide ? cus : 2 * cus;
+    const double slots = t == kTileWide ? cus : 2 * cus, sums = partials_us(tiles_w * kGemmBM * kGemm16TileN[t]);
+    if (sums >= deep.us) return false;
     const double load = (tiles_w * len + tiles_x * steps_x) / slots * pair;
     const double chain = std::max(len, steps_x) * 0.5 * (pair + one);
     const double us = (t == kTileWide ? 4.0 : 3.6) + std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0) +
-                      x_mb / 5.0 + partials_us(tiles_w * kGemmBM * kGemm16TileN[t]);
+                      x_mb / 5.0 + sums;
     if (us < deep.us) deep = Choice16{t, s, us};
+    return true;
   };
   const bool wide = wide_linear_bwd(M, N, K);
   const int64_t only = env_int("MOGRAD_HIP_LINEAR_BWD_TILE", 0);  // 128 | 192
@@ -653,11 +661,12 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx,
     const int s = splitk_16bit_splits(ceil_div(N, kGemmBM) * ceil_div(K, kGemmBN), M, 1);
     if (s > 1) offer(t, s);
   } else if (wide) {
-    for (int s = 2; s <= most; ++s) offer(kTileWide, s);
+    for (int s = 2; s <= most && offer(kTileWide, s); ++s) {
+    }
   } else {
-    for (int s = 2; s <= most; ++s) {
-      if (only != 192) offer(kTile128, s);
-      if (only != 128) offer(kTile192, s);
+    for (int s = 2; s <= most && only != 192 && offer(kTile128, s); ++s) {
+    }
+    for (int s = 2; s <= most && only != 128 && offer(kTile192, s); ++s) {
     }
   }
   if (deep.tile < 0 || (!wide && only == 0 && !env_str("MOGRAD_HIP_LINEAR_BWD_WIDE"))) {
