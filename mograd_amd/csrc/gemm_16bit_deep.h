@@ -23,9 +23,9 @@ namespace mg {
 // the first phase and S2 in the third, behind a first k-slice of MFMAs: the data that is read until the next one
 // has arrived (younger requests stay outstanding), and no wave still reads what is requested until then.
 // ------------------------------------------------------------------------------------
-template <int AI_, int BJ0_, int BJ1_, int WN_ = 2, int COPIES_ = 2>
+template <int AI_, int BJ0_, int BJ1_, int WN_ = 2>
 struct Gemm16Deep {
-  static constexpr int AI = AI_, BJ0 = BJ0_, BJ1 = BJ1_, BJ = BJ0_ + BJ1_, WN = WN_, COPIES = COPIES_;
+  static constexpr int AI = AI_, BJ0 = BJ0_, BJ1 = BJ1_, BJ = BJ0_ + BJ1_, WN = WN_;
   static constexpr int kThreads = 2 * WN * 64;
   static constexpr int kWaveM = 64 * AI, kWaveN = 32 * BJ;
   static constexpr int kTM = 2 * kWaveM, kTN = WN * kWaveN;
@@ -40,7 +40,7 @@ struct Gemm16Deep {
   static constexpr int requests(int image) { return rows(image) * 8 / kThreads; }  // of 16 bytes, per thread and step
   static constexpr int kStripStride = kWaveN + 8;  // elements of a row of a wave's output strip (64 rows)
   static constexpr int kStrips = 2 * WN * 64 * kStripStride * 2;
-  static constexpr int kLds = COPIES * kStep > kStrips ? COPIES * kStep : kStrips;
+  static constexpr int kLds = 2 * kStep > kStrips ? 2 * kStep : kStrips;
   // Workgroups per CU: by LDS (160 KB) and by the register file (512 per lane and SIMD; fragments and
   // addresses next to the accumulators).
   static constexpr int kWavesPerSimd = AI * BJ <= 3 ? 2 : 1;
@@ -318,7 +318,7 @@ __device__ __forceinline__ void gemm16_deep_ln_bwd(const floatx16 (&acc)[2][S::B
 template <typename T, class S, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM = false, bool LN_BWD = false,
           bool OUT_F32 = false>
 __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
-  constexpr int AI = S::AI, BJ0 = S::BJ0, BJ1 = S::BJ1, BJ = S::BJ, WN = S::WN, NT = S::kThreads, CP = S::COPIES;
+  constexpr int AI = S::AI, BJ0 = S::BJ0, BJ1 = S::BJ1, BJ = S::BJ, WN = S::WN, NT = S::kThreads;
   const int M = pr.M, N = pr.N;
   const int64_t lda = pr.lda, ldb = pr.ldb;
   const int tiles = pr.tiles_m * pr.tiles_n;
@@ -336,7 +336,7 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
   const int k_end = SPLIT_K ? min(pr.K, k_begin + pr.k_per_split) : pr.K;
   // A reduction of fewer steps than there are copies ends on steps of zeros.
   const int full_steps = (k_end - k_begin) / S::kBK, rem = (k_end - k_begin) % S::kBK;
-  const int steps = max(CP, full_steps + (rem > 0 ? 1 : 0));
+  const int steps = max(2, full_steps + (rem > 0 ? 1 : 0));
   const int64_t a_step = A_KC ? S::kBK : S::kBK * lda;
   const int64_t b_step = B_KC ? S::kBK : S::kBK * ldb;
   const uint16_t* a16 = reinterpret_cast<const uint16_t*>(pr.A) + batch * pr.bsa + (A_KC ? m0 * lda + k_begin : m0 + k_begin * lda);
@@ -451,20 +451,20 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // Step `it`, with LEFT more steps behind it.  LEFT == CP: so many at least, and step it + CP is requested (SHORT:
+  // Step `it`, with LEFT more steps behind it.  LEFT == 2: so many at least, and step it + 2 is requested (SHORT:
   // it is the short one).
   auto do_step = [&](int it, auto left, auto is_short) {
     constexpr int LEFT = decltype(left)::value;
-    constexpr bool STEADY = LEFT == CP;
-    constexpr int YOUNGER = LEFT < CP - 1 ? LEFT : CP - 1;  // whole steps requested after this one
-    const int copy = it % CP, next = (it + 1) % CP;
+    constexpr bool STEADY = LEFT == 2;
+    constexpr int YOUNGER = LEFT < 1 ? LEFT : 1;  // whole steps requested after this one
+    const int copy = it % 2, next = (it + 1) % 2;
     auto s1 = [] {
       MG_WAIT_VMCNT(YOUNGER * R);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
     auto s2 = [] {
       if constexpr (LEFT > 0) {
-        MG_WAIT_VMCNT(RA + RB1 + (YOUNGER - 1) * R + (STEADY ? RA + RB0 : 0));
+        MG_WAIT_VMCNT(RA + RB1 + (STEADY ? RA + RB0 : 0));
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       }
     };
@@ -475,7 +475,7 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
     using QB1 = std::conditional_t<STEADY, B1, None>;
     using NA = std::conditional_t<(LEFT > 0), A0, None>;
     using NB = std::conditional_t<(LEFT > 0), B0, None>;
-    phase(A0{}, B0{}, B1{}, copy, QA0{}, it + CP, copy, is_short, s1);
+    phase(A0{}, B0{}, B1{}, copy, QA0{}, it + 2, copy, is_short, s1);
     if constexpr (HAS_BIAS && !SPLIT_K && LEFT == 0) {  // arrives under the last three phases
 #pragma unroll
       for (int j = 0; j < BJ; ++j) {
@@ -483,9 +483,9 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
         bias_v[j] = col < N ? to_float(pr.bias[col]) : 0.f;
       }
     }
-    phase(A0{}, B1{}, A1{}, copy, QB0{}, it + CP, copy, is_short, no_sync);
-    phase(A1{}, B1{}, NA{}, next, QB1{}, it + CP, copy, is_short, s2);
-    phase(A1{}, B0{}, NB{}, next, QA1{}, it + CP, copy, is_short, no_sync);
+    phase(A0{}, B1{}, A1{}, copy, QB0{}, it + 2, copy, is_short, no_sync);
+    phase(A1{}, B1{}, NA{}, next, QB1{}, it + 2, copy, is_short, s2);
+    phase(A1{}, B0{}, NB{}, next, QA1{}, it + 2, copy, is_short, no_sync);
   };
   // Requested in the order in which the steps before would have done it.
   auto request_all = [&](auto image, int step) {
@@ -499,13 +499,13 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
     for (int i = 0; i < S::requests(IM); ++i) request(image, i, step, step);
   };
 #pragma unroll
-  for (int s = 0; s < CP; ++s) {
+  for (int s = 0; s < 2; ++s) {
     request_all(A0{}, s);
     request_all(B0{}, s);
     request_all(B1{}, s);
     request_all(A1{}, s);
   }
-  MG_WAIT_VMCNT(RB1 + RA + (CP - 1) * R);
+  MG_WAIT_VMCNT(RB1 + RA + R);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int n = 0; n < 4 * AI; ++n) read(A0{}, n, 0);
@@ -513,10 +513,8 @@ __device__ __forceinline__ void gemm16_deep_block(char* lds, int bid, const Gemm
   for (int n = 0; n < 4 * BJ0; ++n) read(B0{}, n, 0);
   __builtin_amdgcn_sched_barrier(0);
   int it = 0;
-  for (; it + CP < full_steps; ++it) do_step(it, std::integral_constant<int, CP>{}, std::false_type{});
-  if (it < steps - CP) do_step(it, std::integral_constant<int, CP>{}, std::true_type{});
-  if constexpr (CP > 3) do_step(steps - 4, std::integral_constant<int, 3>{}, std::false_type{});
-  if constexpr (CP > 2) do_step(steps - 3, std::integral_constant<int, 2>{}, std::false_type{});
+  for (; it + 2 < full_steps; ++it) do_step(it, std::integral_constant<int, 2>{}, std::false_type{});
+  if (it < steps - 2) do_step(it, std::integral_constant<int, 2>{}, std::true_type{});
   do_step(steps - 2, std::integral_constant<int, 1>{}, std::false_type{});
   do_step(steps - 1, std::integral_constant<int, 0>{}, std::false_type{});
 

@@ -388,11 +388,10 @@ __device__ __forceinline__ void gemm16_write_f32(const floatx16& acc, float* __r
 // partial[(split * batches + batch), M, N].
 template <typename T, bool HAS_BIAS, bool SPLIT_K>
 __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], uint16_t* __restrict__ mine,
-                                                  const T* __restrict__ bias, T* __restrict__ C,
+                                                  const float (&bias_v)[2], T* __restrict__ C,
                                                   float* __restrict__ partial, int M, int N, int64_t ldc, int64_t bsc,
                                                   int batch, int split, int batches, int m0, int n0, int wm, int wn,
-                                                  int lane, const GemmEpilogue<T>& ep, bool partial_stream = false,
-                                                  const float* bias_early = nullptr) {
+                                                  int lane, const GemmEpilogue<T>& ep) {
   if constexpr (SPLIT_K) {
     // A K range's partial tile goes out as the accumulators lie in the registers: sixteen
     // unguarded 16-byte stores per thread, each a contiguous kilobyte of the wave
@@ -403,18 +402,6 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
                             static_cast<int64_t>(m0 / kGemmBM) * tiles_n + col0 / kGemmBN;
     float4* dst = reinterpret_cast<float4*>(partial) + tile_at * (kG16PartialTile / 4) +
                   ((wm / 64) * 2 + (col0 / 64) % 2) * 1024 + lane;
-    if (partial_stream) {
-#pragma unroll
-      for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-        for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const floatx4 v = {acc[ti][tj][4 * g], acc[ti][tj][4 * g + 1], acc[ti][tj][4 * g + 2], acc[ti][tj][4 * g + 3]};
-            __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(dst + ((ti * 2 + tj) * 4 + g) * 64));
-          }
-      return;
-    }
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
@@ -442,15 +429,10 @@ __device__ __forceinline__ void gemm16_write_tile(const floatx16 (&acc)[2][2], u
         for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
           for (int tj = 0; tj < 2; ++tj) {
-            float bv = 0.f;
-            if constexpr (HAS_BIAS) {
-              const int col = n0 + wn + tj * 32 + lane % 32;
-              bv = bias_early ? bias_early[tj] : (col < N ? to_float(bias[col]) : 0.f);
-            }
 #pragma unroll
             for (int rp = 0; rp < 8; ++rp) {  // rows 2 rp and 2 rp + 1 of the sixteen
               float f0 = acc[ti][tj][2 * rp], f1 = acc[ti][tj][2 * rp + 1];
-              if constexpr (HAS_BIAS) f0 += bv, f1 += bv;
+              if constexpr (HAS_BIAS) f0 += bias_v[tj], f1 += bias_v[tj];
               if constexpr (decltype(relu)::value) {
                 f0 = f0 > 0.f ? f0 : 0.f;
                 f1 = f1 > 0.f ? f1 : 0.f;
@@ -615,9 +597,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_16bit_mfma_kernel(
       for (int j = 0; j < 2; ++j) gemm16_write_f32(acc[i][j], C, M, N, ldc, m0 + wm + 32 * i, n0 + wn + 32 * j, lane);
   } else {
     uint16_t* mine = (wave < 2 ? lds_a : lds_b) + (wave % 2) * 64 * kG16Stride;  // staging memory, idle now
-    gemm16_write_tile<T, HAS_BIAS, SPLIT_K>(acc, mine, bias, C, partial, M, N, ldc, bsc, batch,
-                                            split, SPLIT_K ? batches : 1,
-                                            m0, n0, wm, wn, lane, ep, false, HAS_BIAS && !SPLIT_K ? bias_v : nullptr);
+    gemm16_write_tile<T, HAS_BIAS, SPLIT_K>(acc, mine, bias_v, C, partial, M, N, ldc, bsc, batch, split, SPLIT_K ? batches : 1,
+                                            m0, n0, wm, wn, lane, ep);
   }
 }
 
@@ -860,7 +841,7 @@ __device__ __forceinline__ void gemm32_pipe_issue(const float* base, const int64
   }
 }
 
-// The short last step (`rem` k left): see gemm16_pipe_tail.
+// The short last step (`rem` k left) comes through registers, zeros past the end.
 template <bool KC, int TS>
 __device__ __forceinline__ void gemm32_pipe_tail(const float* base, const int64_t* src, int rem, char* lds_step) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
