@@ -73,18 +73,21 @@ def test_linear_bwd_deferred_matches_immediate(device, pending, dtype, M, N, K, 
 
 # Layers of a few hundred rows, whose products may go out together or apart; large ones with whole and with split
 # dW tiles; widths off the 16-byte chunks, long and short; a width of 1, which gives an operand two unit strides; no rows.
-@pytest.mark.parametrize("dtype,M,N,K", [
+FP32_GRADIENT_CASES = [
     (BF16, 200, 3072, 1024), (F16, 200, 3072, 1024), (BF16, 64, 4096, 1024), (BF16, 1000, 4608, 1536), (BF16, 16384, 4096, 1024),
     (BF16, 4096, 8192, 4096), (BF16, 2048, 384, 384), (BF16, 2048, 3000, 2000), (F16, 114, 1771, 383), (BF16, 1999, 1001, 767),
-    (BF16, 5000, 1, 384), (BF16, 300, 384, 1), (BF16, 60, 1, 40), (BF16, 0, 24, 16)])
-@pytest.mark.parametrize("entry", ["linear", "layer_norm"])
+    (BF16, 5000, 1, 384), (BF16, 300, 384, 1), (BF16, 60, 1, 40), (BF16, 0, 24, 16)]
+# (the larger ones go through the same kernels from either entry)
+FP32_GRADIENT_CASES = ([("linear", *c) for c in FP32_GRADIENT_CASES] +
+                       [("layer_norm", *c) for c in FP32_GRADIENT_CASES if 0 < c[1] <= 2048])
+
+
+@pytest.mark.parametrize("entry,dtype,M,N,K", FP32_GRADIENT_CASES)
 @pytest.mark.parametrize("one_launch", ["1", "0"])
-def test_fp32_gradients_of_16bit_layers_are_fp32_sums(device, pending, monkeypatch, dtype, M, N, K, entry, one_launch):
+def test_fp32_gradients_of_16bit_layers_are_fp32_sums(device, pending, monkeypatch, entry, dtype, M, N, K, one_launch):
     # dW and db in fp32 against float64 products of the 16-bit inputs.  fp32 accumulation of M terms of random sign: every
     # partial sum rounds by 2^-24 of itself at most, sqrt(M) of them in quadrature, a factor 4 for luck.  Through bf16 the
     # error is 1e-3, through fp16 1.4e-4, at any M here above 20 times that.
-    if entry == "layer_norm" and (M > 2048 or M == 0):
-        pytest.skip("the same kernels as below")
     monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", one_launch)  # 0: a launch for each product
     lib, st = device.lib, device.stream
     x, dy = (_rounded(normal(75, i, (max(M, 1), n)), dtype) for i, n in ((0, K), (1, N)))

@@ -355,8 +355,8 @@ def test_half_precision_mfma_paths(device, dtype, rtol, M, N, K):
                                    (72, 1536, 64), (520, 264, 320)])
 def test_tile_staging_variants_agree(device, monkeypatch, dtype, rtol, M, N, K):
     # The 16-bit products have a register-staged kernel (0) and one whose tiles are copied
-    # straight into LDS, 32 or 64 k per step (322, 642), also with 256 x 128 output tiles
-    # (2322, 2642) or 256 x 256 tiles of 128 x 128 wave tiles (4324, 4642); the library picks by operand layout, K and size.  All accumulate each output element over k in the same order on the same MFMA,
+    # straight into LDS, with output tiles of 128 x 128 (128), 128 x 192 (2000) or 256 x 256 (4000; 128 x 128 where K is
+    # split); the library picks by layout, K and size.  All accumulate each output element over k in the same order on the same MFMA,
     # so forcing either must not change a bit, for every operand layout (forward k/k, dX
     # k/n, dW m/n, the last split along K for the tall shapes) and at ragged tile edges.
     x = round_to_dtype(normal(49, 0, (M, K)), dtype)
@@ -364,12 +364,12 @@ def test_tile_staging_variants_agree(device, monkeypatch, dtype, rtol, M, N, K):
     b = round_to_dtype(normal(49, 2, (N,), std=0.1), dtype)
     dy = round_to_dtype(normal(49, 3, (M, N), std=0.5), dtype)
     results = {}
-    for variant in ("0", "322", "642", "2322", "2642", "4324", "4642"):
+    for variant in ("0", "128", "2000", "4000"):
         monkeypatch.setenv("MOGRAD_HIP_GEMM16_PIPE", variant)
         results[variant] = _linear_all(device, x, w, b, dy, dtype)
     monkeypatch.delenv("MOGRAD_HIP_GEMM16_PIPE")
     results["auto"] = _linear_all(device, x, w, b, dy, dtype)
-    for variant in ("322", "642", "2322", "2642", "4324", "4642", "auto"):
+    for variant in ("128", "2000", "4000", "auto"):
         for got, base, name in zip(results[variant], results["0"], ("y", "dx", "dw", "db")):
             np.testing.assert_array_equal(got, base, err_msg=f"{name}, variant {variant}")
     y, dx, dw, _ = results["auto"]
@@ -476,7 +476,7 @@ def test_large_products_agree_with_the_register_staged_kernel(device, monkeypatc
     assert_close(auto[0][rows], want, 1.6e-2, 1.6e-2 * np.abs(want).max(), "y rows")
 
 
-@pytest.mark.parametrize("variant", ["0", "322", "642", "2322", "2642"])
+@pytest.mark.parametrize("variant", ["0", "128", "2000", "4000"])
 def test_batched_projections_tile_staging_variants(device, monkeypatch, variant):
     # The same two batched products (batch stride 0 on the shared operand; the second split
     # along K with the batch in the grid's z) through each 16-bit tile-staging variant.
@@ -577,8 +577,9 @@ def test_linear_bwd_one_launch_matches_two(device, monkeypatch, dtype, rtol, M, 
     results = {}
     # the common launch splits dW for one workgroup per CU; ask the separate launch for the same
     monkeypatch.setenv("MOGRAD_HIP_GEMM_SPLITK_WG_PER_CU", "1")
-    # Input widths that are multiples of 384 take 128 x 384 tiles in the common launch, with dW's
-    # K ranges cut differently: "wide" is compared within the tolerance, the 128 x 128 form bitwise.
+    # "wide": the tiles and K ranges of dW that the library picks (for 384 columns and layers 768 wide the ranges of the
+    # launch that carries a LayerNorm's backward in 128 x 384 tiles): dW is compared within the tolerance, and bitwise
+    # with the K ranges that it has in a launch of its own ("1").
     modes = ("0", "1", "wide") if K % 384 == 0 else ("0", "1")
     for mode in modes:
         monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_ONE_LAUNCH", "0" if mode == "0" else "1")
@@ -611,7 +612,7 @@ def test_linear_bwd_one_launch_matches_two(device, monkeypatch, dtype, rtol, M, 
             assert_close(got, want, rtol, rtol * np.abs(want).max(), f"{name} ({mode})")
         assert_close(res[3], prior + want_dx * (x > 0), 2 * rtol, 2 * rtol * np.abs(want_dx).max(), "dx masked+acc")
     if "wide" in results:
-        # same dX tiles' k order (one tile is three of the narrow ones side by side): bitwise
+        # the same k order of dX in any tile: bitwise
         if not dx_split_alone:
             np.testing.assert_array_equal(results["wide"][0], results["0"][0], err_msg="dx wide")
             np.testing.assert_array_equal(results["wide"][3], results["0"][3], err_msg="dx masked+acc wide")
@@ -650,24 +651,29 @@ def test_linear_bwd_ragged_width(device, monkeypatch, dtype, rtol, M, N, K):
         assert_close(results[mode][1], want_dw, rtol, rtol * np.abs(want_dw).max(), "dw " + mode)
 
 
-LN_CONT_SHAPES = [(4096, 1152, 384), (2048, 1536, 384), (2112, 768, 384), (16384, 1536, 384),  # one launch, whole rows
-                  (1024, 384, 384), (512, 96, 200), (2048, 832, 768)]                              # separate kernels
+LN_CONT_SHAPES = [(4096, 1152, 384), (2048, 1536, 384), (2112, 768, 384), (16384, 1536, 384),
+                  (1024, 384, 384), (512, 96, 200), (2048, 832, 768)]  # separate kernels
+# One launch whose tiles hold whole rows of dX: what the library picks for large layers only is asked for at these.
+LN_ONE_LAUNCH_SHAPES = [(4096, 1152, 384), (2048, 1536, 384), (2112, 768, 384), (2051, 1152, 384), (515, 768, 384)]
 
 
 # fp32 always takes the two separate entries: the largest shapes add nothing there
-LN_CONT_CASES = [(dt, *shape) for dt in (BF16, F16, F32) for shape in LN_CONT_SHAPES
+LN_CONT_CASES = [(dt, *shape, False) for dt in (BF16, F16, F32) for shape in LN_CONT_SHAPES
                  if dt != F32 or shape[0] * shape[1] * shape[2] <= 2048 * 1536 * 384]
+LN_CONT_CASES += [(dt, *shape, True) for dt in (BF16, F16) for shape in LN_ONE_LAUNCH_SHAPES]
 
 
 @pytest.mark.parametrize("deferred", [False, True])
-@pytest.mark.parametrize("dtype,M,N,K", LN_CONT_CASES)
-def test_linear_bwd_continues_as_layer_norm_bwd(device, dtype, M, N, K, deferred):
+@pytest.mark.parametrize("dtype,M,N,K,one_launch", LN_CONT_CASES)
+def test_linear_bwd_continues_as_layer_norm_bwd(device, monkeypatch, dtype, M, N, K, one_launch, deferred):
     # Y = LN(h) W^T + b: the layer's backward and the LayerNorm's in one entry.  For 16-bit layers
     # of 384 input columns the dX tiles hold whole rows and finish as the LayerNorm backward
-    # inside the launch ((2112, ..): the last tile is half empty); other shapes and fp32 run the
+    # inside the launch (2112, 2051 and 515 rows: the last tile has 64, 3 and 3); other shapes and fp32 run the
     # two separate entries on a scratch tensor.  Either way dW and db are the separate entry's
     # bits, and dh, dgamma and dbeta differ from the separate calls only by the order of their
     # fp32 sums; the oracle gets the same dY W rounded to the tensors' type.
+    if one_launch:
+        monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_SMALL", "0")
     lib, st = device.lib, device.stream
     h = round_to_dtype(normal(81, 0, (M, K), std=1.5) + 0.3, dtype)
     gamma = round_to_dtype(uniform(81, 1, (K,), 0.5, 1.5), dtype)
@@ -723,11 +729,14 @@ def test_linear_bwd_continues_as_layer_norm_bwd(device, dtype, M, N, K, deferred
         assert_close(dbt.to_numpy(), odb, rt, rt * np.abs(odb).max(), "dbeta")
 
 
-@pytest.mark.parametrize("M,N,K", [(2048, 1152, 384), (1024, 384, 384)])
-def test_linear_bwd_layer_norm_bwd_without_prior_and_bias(device, M, N, K):
+@pytest.mark.parametrize("M,N,K,one_launch", [(2048, 1152, 384, False), (1024, 384, 384, False), (2048, 1152, 384, True),
+                                              (2051, 768, 384, True)])
+def test_linear_bwd_layer_norm_bwd_without_prior_and_bias(device, monkeypatch, M, N, K, one_launch):
     # dx_accumulate = 0 (dh is written, whatever it held) and db = NULL, in the one launch and in
     # the separate-kernels form.
     dtype = BF16
+    if one_launch:
+        monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_SMALL", "0")
     lib, st = device.lib, device.stream
     h = round_to_dtype(normal(82, 0, (M, K), std=2.0), dtype)
     gamma = round_to_dtype(uniform(82, 1, (K,), 0.5, 1.5), dtype)
