@@ -602,38 +602,41 @@ static bool wide_linear_bwd(int64_t M, int64_t N, int64_t K) {
 
 // How the backward of a 16-bit layer goes out: in one launch, with which tiles and dW in how many K ranges, or in a
 // launch for each product (tile < 0).  The least of these estimates, in us, is taken:
-//   64 x 64 tiles (gemm_16bit_small.h): the longest chain of k-steps (of 64) in one workgroup, 0.24 us a step, dW's and
-//     dX's together by 0.75 where they share CUs, by 0.95 where dX's start when dW's end, dW's a seventh longer with db; the steps of all workgroups dealt over the
-//     CUs, 0.168 us each, a third more where rows do not start on cache lines; of the two the longer, and 0.36 of the
-//     other.  What is read and written at 4 TB/s; K ranges 3.5 us and 0.0058 us a tile.  (From 176 layers of 64 to 2048 rows and 384 to 6144 columns, as in transformer
-//     blocks of few tokens, and 156 of 32 to 16384 rows and any multiples of 8 up to 6144: fp32 gradients with
-//     deferred sums and 16-bit ones at once, with and without db, 1 to 8 K ranges; rms 7 %.)
+//   64 x 64 tiles (gemm_16bit_small.h): the longest chain of k-steps (of 64) in one workgroup, 0.217 us a step, dW's and
+//     dX's together by 0.68 where they share CUs, dW's a fifth longer with db; the steps of all workgroups dealt over the
+//     CUs, 0.192 us each, a sixth more where rows do not start on cache lines; of the two the longer, and a quarter of the
+//     other.  What is read and written of X and W; K ranges 1.6 us and 0.0096 us a tile.
 //   128-row tiles: chain and load as in deep_16bit_us, a chain's steps between the two figures there (it shares its
-//     CU for a part of its life).  128 x 384 tiles, which carry a LayerNorm's backward: 1.5 us a step, against a
-//     launch of its own for that (from 30 layers of 1024 to 32000 rows, 10 %).
+//     CU for a part of its life), by 0.84 in this launch, 1.02 where rows do not start on cache lines.  128 x 384 tiles,
+//     which carry a LayerNorm's backward: 1.5 us a step, against a launch of its own for that (from 30 layers of
+//     1024 to 32000 rows, 10 %).
 //   a launch for each product, and 7 us of one or two more for the sum of dY's rows.  Off the 16-byte chunks dW is the
 //     register-staged kernel's, 5 us more: (114, 1771 <- 384) 20 us against 12.
-// So (320, 3072 <- 768) with db is one launch, 19.4 us against 26.6, and (320, 1536 <- 6144) without three, 29.0 against
-// 33.2; the route taken is 0.5 to 0.9 % slower than the best one of each of the 176 layers, 0.9 to 1.7 % of the 156.  The
-// type of the gradients is not part of it: fp32 and 16-bit ones, deferred or not, come from the same sums.
+// Fitted to what the choice costs over 390 layers, each by every route and 1 to 32 K ranges, fp32 gradients with deferred
+// sums and 16-bit ones at once, caches warm and cold: a third of 64 to 16384 rows and any widths from 64 to 4608, a third as
+// in transformer blocks of 64 to 2048 tokens, a third of 2048 to 20000.  On 300 others the route taken is 1.6 to 2.4,
+// 0.2 to 1.4 and 2.7 to 3.0 % slower than each one's best.  So (320, 3072 <- 768) with db is one launch, 19.4 us
+// against 26.6, (320, 1536 <- 6144) without is two, 29.0 against 33.2, and (1999, 1001 <- 768) takes 64 x 64 tiles, 22.7
+// against 26.5.  The type of the gradients is not part of it: fp32 and 16-bit ones, deferred or not, come from the same sums.
 // A range has at least 256 rows (64 x 64 tiles: 128).  MOGRAD_HIP_LINEAR_BWD_SMALL = 0 | 1 and MOGRAD_HIP_LINEAR_BWD_SPLITS override the choice.
 static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx, bool with_db) {
   const double cus = device_info().cu_count;
   const double steps_w = static_cast<double>(ceil_div(M, kG16BK)), steps_x = static_cast<double>(ceil_div(N, kG16BK));
   const double x_mb = static_cast<double>(M) * K * 2.0 / 1e6, w_mb = static_cast<double>(N) * K * 2.0 / 1e6;
+  const bool on_lines = N % 64 == 0 && K % 64 == 0;  // rows that start on cache lines
   Choice16 small{kSmall, 1};
   {
     const double tiles_k = static_cast<double>(ceil_div(K, kSmallT));
     const double tiles_w = steps_x * tiles_k, tiles_x = with_dx ? steps_w * tiles_k : 0.0, chain_x = with_dx ? steps_x : 0.0;
-    auto together = [&](double tiles) { return tiles > 2 * cus ? 0.95 : tiles > cus ? 0.75 : 0.0; };
-    const double step = N % 64 == 0 && K % 64 == 0 ? 0.168 : 0.222;
+    const double step = on_lines ? 0.192 : 0.225;
     for (int s = 1; s <= 32 && (s == 1 || M >= 128 * s); ++s) {
-      if (s > 1 && 7.0 + tiles_w * s * 0.0058 >= small.us) break;
-      const double len = std::ceil(steps_w / s), chain_w = with_db ? 1.14 * len : len;
-      const double chain = 0.24 * std::max({chain_w, chain_x, together(tiles_w * s + tiles_x) * (chain_w + chain_x)});
+      if (s > 1 && 5.0 + tiles_w * s * 0.0096 >= small.us) break;
+      const double len = std::ceil(steps_w / s), chain_w = with_db ? 1.22 * len : len;
+      const double both = tiles_w * s + tiles_x > cus ? 0.68 * (chain_w + chain_x) : 0.0;
+      const double chain = 0.217 * std::max({chain_w, chain_x, both});
       const double load = step * (tiles_w * s * len + tiles_x * steps_x) / cus;
-      const double t = 3.5 + std::max(chain, load) + 0.36 * std::min(chain, load) +
-                       0.25 * (with_dx ? x_mb + 2.5 * w_mb : 1.5 * w_mb) + (s > 1 ? 3.5 + tiles_w * s * 0.0058 : 0.0);
+      const double t = 3.4 + std::max(chain, load) + 0.25 * std::min(chain, load) +
+                       (with_dx ? 0.38 * x_mb + 0.72 * w_mb : 0.43 * w_mb) + (s > 1 ? 1.6 + tiles_w * s * 0.0096 : 0.0);
       if (t < small.us) small.us = t, small.splits = s;
     }
     small.splits = static_cast<int>(env_int("MOGRAD_HIP_LINEAR_BWD_SPLITS", small.splits));
@@ -648,8 +651,8 @@ static Choice16 choose_linear_bwd(int64_t M, int64_t N, int64_t K, bool with_dx,
     if (sums >= deep.us) return false;
     const double load = (tiles_w * len + tiles_x * steps_x) / slots * pair;
     const double chain = std::max(len, steps_x) * 0.5 * (pair + one);
-    const double us = (t == kTileWide ? 4.0 : 3.6) + std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0) +
-                      x_mb / 5.0 + sums;
+    const double walk = std::max(load, chain) + (tiles_w + tiles_x > slots ? 0.5 * std::min(len, steps_x) * pair : 0.0);
+    const double us = (t == kTileWide ? 4.0 + walk : 4.4 + (on_lines ? 0.84 : 1.02) * walk) + x_mb / 5.0 + sums;
     if (us < deep.us) deep = Choice16{t, s, us};
     return true;
   };
