@@ -2367,8 +2367,8 @@ template <typename T, int DP, int DC = DP>
 static int fwd_typed(const void* q, const void* k, const void* v, const void* mask, void* o, float* lse, AttnDims a,
                      float scale, bool causal, bool has_bias, hipStream_t stream) {
   const int64_t blocks = static_cast<int64_t>(a.B) * a.H * ceil_div(a.S, 128);
-  // Two query blocks or more: the pipelined walk (one block, two steps: B32 H16 S128 causal 8.8 us against 8.1; two of
-  // narrow causal heads, two and four steps: B64 H6 S256 D64 16.1 against 15.7, B13 H4 S199 7.5 against 7.8).
+  // Two query blocks or more: the pipelined walk (one block, two steps: B32 H16 S128 causal 9.0 us against 8.3; two of
+  // narrow causal heads, two and four steps: B64 H6 S256 D64 15.1 against 14.4, B13 H4 S199 7.3 against 7.8).
   if constexpr (DP <= 128) {
     if (!has_bias && scale > 0.f && row_offsets_fit(a) && env_int("MOGRAD_HIP_ATTN_FWD_PIPE", a.S > (causal && DP == 64 ? 256 : 128)) != 0) {
       auto launch = [&](auto kernel) {
