@@ -156,14 +156,19 @@ static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const 
                         bool has_bias, hipStream_t stream) {
   const int tiles = static_cast<int>(ceil_div(a.S, 32));
   const int64_t heads = static_cast<int64_t>(a.B) * a.H;
-  const dim3 grid(static_cast<unsigned>(f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal))));
+  const int blocks = static_cast<int>(f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal)));
   Scratch delta;
-  MG_TRY(delta.take(heads * a.S * static_cast<int64_t>(sizeof(float))));
+  if (a.D > 96 && a.D <= 128) {
+    static_assert(f32_wave_delta_given<128>() && !f32_wave_delta_given<96>() && !f32_wave_delta_given<64>(), "who is handed delta");
+    const int64_t rows = heads * a.S;
+    MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
+    hipLaunchKernelGGL((attn_delta_kernel<float>), dim3(static_cast<unsigned>(ceil_div(rows, 4))), dim3(256), 0, stream, d_o, o,
+                       delta.as<float>(), rows, a.D, a.S, a.H, a.o_bshd);
+  }
   f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
-    hipLaunchKernelGGL((attn_dq_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
-                       grid, dim3(256), 0, stream, d_o, o, q, k, v, mask, lse, delta.as<float>(), dq, a, scale, tiles);
-    hipLaunchKernelGGL((attn_dkdv_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
-                       grid, dim3(256), 0, stream, d_o, q, k, v, mask, lse, delta.as<float>(), dk, dv, a, scale, tiles);
+    hipLaunchKernelGGL((attn_bwd_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
+                       dim3(2 * static_cast<unsigned>(blocks)), dim3(256), 0, stream, d_o, o, q, k, v, mask, lse,
+                       delta.as<float>(), dq, dk, dv, a, scale, tiles, blocks);
   });
   MG_LAUNCH_CHECK();
   return MG_OK;
