@@ -213,6 +213,48 @@ def test_long_ragged_sequence(device, causal, D):
         assert_attn_grad_close(got, want, what)
 
 
+@pytest.mark.parametrize("dtype,half_ulp", [(F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("B,H,S,D", [(1, 1, 1, 8), (2, 3, 16, 64), (1, 2, 33, 32), (1, 2, 58, 64), (1, 3, 128, 96), (1, 1, 129, 128),
+                                     (2, 1, 161, 80), (1, 2, 257, 24), (1, 1, 300, 72), (1, 1, 65, 128)])
+def test_workgroups_of_32_rows(device, monkeypatch, dtype, half_ulp, name, causal, with_mask, B, H, S, D):
+    # One row to several tiles per wave, waves without a tile, columns that fill a kernel's width and that do not.  A weight, a
+    # score gradient and a result are each rounded once: a sum over rounded factors is off by at most half a unit of its
+    # terms' magnitudes; what is computed in fp32 (scores of up to ten, their exponentials, sums) by 2^-18 of them.
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", "1")
+    q, k, v, do, m = _inputs(63, B, S, H, D, dtype, with_mask)
+    got = _fwd_bwd(device, q, k, v, do, m, causal, dtype=dtype)
+    q, k, v = (t.astype(np.float64).transpose(0, 2, 1, 3) for t in (q, k, v))
+    do = do.astype(np.float64)
+    turned = lambda t: t.transpose(0, 1, 3, 2)
+    scale = 1.0 / math.sqrt(D)
+    s = q @ turned(k) * scale + (0.0 if m is None else m.astype(np.float64))
+    if causal:
+        s = np.where(np.tril(np.ones((S, S), bool)), s, -np.inf)
+    top = s.max(-1, keepdims=True)
+    p = np.exp(s - top)
+    total = p.sum(-1, keepdims=True)
+    p /= total
+    # delta is formed from the O that was stored, as the backward's contract has it
+    ds = p * (do @ turned(v) - (do * got[0]).sum(-1, keepdims=True))
+    # the fp32 part of dS, P (dP - delta), cancels: its terms are at most these
+    terms = p * (np.abs(do) @ turned(np.abs(v)) + np.abs(do * got[0]).sum(-1, keepdims=True))
+    back = lambda t: t.transpose(0, 2, 1, 3)
+    want = {"o": (p @ v, p @ np.abs(v), p @ np.abs(v)), "lse": ((top + np.log(total))[..., 0], None, None),
+            "dq": tuple(back(x @ y * scale) for x, y in ((ds, k), (np.abs(ds), np.abs(k)), (terms, np.abs(k)))),
+            "dk": tuple(back(turned(x) @ y * scale) for x, y in ((ds, q), (np.abs(ds), np.abs(q)), (terms, np.abs(q)))),
+            "dv": tuple(back(turned(p) @ y) for y in (do, np.abs(do), np.abs(do)))}
+    # fp16: a weight, score gradient or result below 2^-14 is rounded to multiples of 2^-24; S of them times an operand
+    tiny = 2.0 ** -25 * (1 + S * max(np.abs(t).max() for t in (q, k, v, do))) if dtype == F16 else 0.0
+    for g, (what, (ref, rounded, exact)) in zip(got, want.items()):
+        err = np.abs(g.astype(np.float64) - ref)
+        if rounded is None:
+            assert err.max() <= 1e-5, what
+            continue
+        bound = 1.02 * half_ulp * (rounded + np.abs(ref)) + 2.0 ** -18 * exact + tiny
+        assert (err <= bound).all(), f"{what}: {float((err / np.maximum(bound, 1e-30)).max())}"
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_bf16_gradients_rtol(device, causal):
     # Parity bar for bf16 attention gradients: rtol 2e-2, with an absolute floor for entries that
