@@ -19,16 +19,17 @@ namespace mg {
 
 // Mean and rstd of the row held in `x` (shifted sums: the shift is the row's first
 // element, which keeps E[d^2] - E[d]^2 free of cancellation for rows with a large mean).
-template <typename T, int VEC, int TPR, int VPT, int WG>
-__device__ __forceinline__ void row_stats(const RowTile<T, VEC, TPR, VPT>& x, float shift, int t, int cols,
+template <typename T, int VEC, int TPR, int VPT, int WG, bool ANY>
+__device__ __forceinline__ void row_stats(const RowTile<T, VEC, TPR, VPT, ANY>& x, float shift, int t, int cols,
                                           float eps, float* slots, int& phase, float& mu, float& rstd) {
   float s[2] = {0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    if (RowTile<T, VEC, TPR, VPT>::col(i, t) < cols) {
+    const int c = RowTile<T, VEC, TPR, VPT, ANY>::col(i, t);
+    if (c < cols) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const float d = x.v[i][e] - shift;
+        const float d = !ANY || c + e < cols ? x.v[i][e] - shift : 0.f;
         s[0] += d;
         s[1] += d * d;
       }
@@ -46,7 +47,7 @@ __device__ __forceinline__ void row_stats(const RowTile<T, VEC, TPR, VPT>& x, fl
 // Forward
 // ------------------------------------------------------------------------------------
 
-template <typename T, int VEC, int TPR, int VPT, int WG>
+template <typename T, int VEC, int TPR, int VPT, int WG, bool ANY>
 __global__ __launch_bounds__(WG) void ln_fwd_rows_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                          const T* __restrict__ beta, T* __restrict__ y,
                                                          float* __restrict__ mean_out, float* __restrict__ rstd_out,
@@ -57,18 +58,18 @@ __global__ __launch_bounds__(WG) void ln_fwd_rows_kernel(const T* __restrict__ x
   row_thread<TPR, WG>(t, sub);
   int phase = 0;
 
-  RowTile<T, VEC, TPR, VPT> g, b;
+  RowTile<T, VEC, TPR, VPT, ANY> g, b;
   g.load(gamma, t, cols);
   b.load(beta, t, cols);
 
   for (int64_t row0 = static_cast<int64_t>(blockIdx.x) * RPW; row0 < rows; row0 += static_cast<int64_t>(gridDim.x) * RPW) {
     const int64_t row = row0 + sub;
     if (row >= rows) continue;  // uniform per row of 16 lanes (TPR == 16), per wave (64) or per workgroup (RPW == 1)
-    RowTile<T, VEC, TPR, VPT> xv;
+    RowTile<T, VEC, TPR, VPT, ANY> xv;
     xv.load(x + row * cols, t, cols);
     const float shift = to_float(x[row * cols]);
     float mu, rstd;
-    row_stats<T, VEC, TPR, VPT, WG>(xv, shift, t, cols, eps, slots, phase, mu, rstd);
+    row_stats<T, VEC, TPR, VPT, WG, ANY>(xv, shift, t, cols, eps, slots, phase, mu, rstd);
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(WG) void ln_fwd_stream_kernel(const T* __restrict__
 // Workgroup g owns rows [g*rows_per_group, (g+1)*rows_per_group).
 // ------------------------------------------------------------------------------------
 
-template <typename T, int VEC, int TPR, int VPT, int WG, bool HAS_STATS>
+template <typename T, int VEC, int TPR, int VPT, int WG, bool HAS_STATS, bool ANY>
 __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ dy, const T* __restrict__ x,
                                                          const T* __restrict__ gamma, const float* __restrict__ mean_in,
                                                          const float* __restrict__ rstd_in, const T* residual,
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
   row_thread<TPR, WG>(t, sub);
   int phase = 0;
 
-  RowTile<T, VEC, TPR, VPT> g, acc_g, acc_b;
+  RowTile<T, VEC, TPR, VPT, ANY> g, acc_g, acc_b;
   g.load(gamma, t, cols);
   acc_g.zero();
   acc_b.zero();
@@ -156,7 +157,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
   // rows sit side by side in a workgroup every one of them makes every trip of the loop; a
   // row slot past the end of the group works on zeros and touches no memory.
   constexpr bool LOCKSTEP = TPR > kWave && RPW > 1;
-  RowTile<T, VEC, TPR, VPT> xv, dyv, xn, dyn;
+  RowTile<T, VEC, TPR, VPT, ANY> xv, dyv, xn, dyn;
   int64_t row = r_begin + sub;
   // The row's scalars travel with its tile: the saved statistics, or the row's first element
   // (the shift of the one-pass sums), fetched a trip ahead like the tile itself.
@@ -220,10 +221,10 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
       float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
-        const bool in_row = RowTile<T, VEC, TPR, VPT>::col(i, t) < cols;
+        const int c = RowTile<T, VEC, TPR, VPT, ANY>::col(i, t);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const float d = in_row ? xv.v[i][e] - shift : 0.f;
+          const float d = RowTile<T, VEC, TPR, VPT, ANY>::in_row(c, e, cols) ? xv.v[i][e] - shift : 0.f;
           const float dyg = dyv.v[i][e] * g.v[i][e];
           xv.v[i][e] = d;
           s[0] += d;
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int c = RowTile<T, VEC, TPR, VPT>::col(i, t);
+      const int c = RowTile<T, VEC, TPR, VPT, ANY>::col(i, t);
       float out[VEC];
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
           // gradient gives.  `residual` may be `dx` itself (each element is read, then written,
           // by the same thread).
           float rs[VEC];
-          VecIO<T, VEC>::load(residual + row * cols + c, rs);
+          RowTile<T, VEC, TPR, VPT, ANY>::load_end(residual + row * cols + c, c, cols, rs);
           {
             // a plain addition, as the separate add kernel performs it: not to be contracted
             // with the multiplication that produced the gradient
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
             for (int e = 0; e < VEC; ++e) out[e] = to_float(from_float<T>(out[e])) + rs[e];
           }
         }
-        VecIO<T, VEC>::store_stream(dx + row * cols + c, out);
+        RowTile<T, VEC, TPR, VPT, ANY>::store_end_stream(dx + row * cols + c, c, cols, out);
       }
     }
     if constexpr (PREFETCH) {
@@ -289,10 +290,11 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
   if constexpr (RPW == 1) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int c = RowTile<T, VEC, TPR, VPT>::col(i, t);
+      const int c = RowTile<T, VEC, TPR, VPT, ANY>::col(i, t);
       if (c < cols) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
+          if (ANY && c + e >= cols) break;
           out_g[c + e] = acc_g.v[i][e];
           out_b[c + e] = acc_b.v[i][e];
         }
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(WG) void ln_bwd_rows_kernel(const T* __restrict__ d
     const bool writer = TPR >= kWave || threadIdx.x % kWave < TPR;
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
-      const RowTile<T, VEC, TPR, VPT>& acc = which == 0 ? acc_g : acc_b;
+      const RowTile<T, VEC, TPR, VPT, ANY>& acc = which == 0 ? acc_g : acc_b;
       float* out = which == 0 ? out_g : out_b;
       if (which == 1) __syncthreads();
       if (writer) {
@@ -425,6 +427,12 @@ template <typename T>
 struct LayerNormOps {
   static constexpr int WIDE = WideVec<T>::value;
 
+  // Rows that do not lie on 16-byte chunks are read and written in misaligned ones (RowTile's ANY): what they cost element by
+  // element was 317 / 64 loads of two bytes per lane and row, and rows past 4096 columns had no backward at all.  Forward +
+  // backward, us: (23721, 317) fp16 100 -> 33, fp32 66 -> 38; (9000, 4095) bf16 199 -> 97; (1000, 799) fp16 16.2 -> 15.8.
+  // Up to this many columns stay with an element per thread: of a row of a few chunks most of its sixteen lanes are idle.
+  static constexpr int kNarrow = 64;
+
   // How a row of `chunks` chunks is laid over threads.
   struct Shape {
     int tpr, vpt;
@@ -466,7 +474,7 @@ struct LayerNormOps {
     return true;
   }
 
-  template <int VEC, int TPR, int VPT>
+  template <int VEC, int TPR, int VPT, bool ANY>
   static int launch_fwd(const T* x, const T* gamma, const T* beta, T* y, float* mean, float* rstd, int64_t rows,
                         int64_t cols, float eps, hipStream_t stream) {
     constexpr int WG = TPR <= 64 ? 256 : TPR;
@@ -474,17 +482,18 @@ struct LayerNormOps {
     const int64_t want = ceil_div(rows, RPW);
     const int64_t cap = static_cast<int64_t>(device_info().cu_count) * env_int("MOGRAD_HIP_LN_FWD_WG_PER_CU", 4);
     const unsigned grid = static_cast<unsigned>(want < cap ? want : cap);
-    hipLaunchKernelGGL((ln_fwd_rows_kernel<T, VEC, TPR, VPT, WG>), dim3(grid), dim3(WG), 0, stream, x, gamma, beta, y,
+    hipLaunchKernelGGL((ln_fwd_rows_kernel<T, VEC, TPR, VPT, WG, ANY>), dim3(grid), dim3(WG), 0, stream, x, gamma, beta, y,
                        mean, rstd, rows, static_cast<int>(cols), eps);
     MG_LAUNCH_CHECK();
     return MG_OK;
   }
 
-  template <int VEC>
+  template <int VEC, bool ANY = false>
   static int dispatch_fwd(Shape s, const T* x, const T* gamma, const T* beta, T* y, float* mean, float* rstd,
                           int64_t rows, int64_t cols, float eps, hipStream_t stream) {
-#define MG_LN_FWD_CASE(TPR_, VPT_) \
-  if (s.tpr == TPR_ && s.vpt == VPT_) return launch_fwd<VEC, TPR_, VPT_>(x, gamma, beta, y, mean, rstd, rows, cols, eps, stream)
+#define MG_LN_FWD_CASE(TPR_, VPT_)             \
+  if constexpr (VEC > 1 || TPR_ * VPT_ <= 64) \
+  if (s.tpr == TPR_ && s.vpt == VPT_) return launch_fwd<VEC, TPR_, VPT_, ANY>(x, gamma, beta, y, mean, rstd, rows, cols, eps, stream)
     MG_LN_FWD_CASE(16, 1);
     MG_LN_FWD_CASE(16, 2);
     MG_LN_FWD_CASE(16, 3);
@@ -509,7 +518,9 @@ struct LayerNormOps {
     Shape s;
     if (can_vectorise(cols, {x, gamma, beta, y}) && pick_shape(cols / WIDE, &s))
       return dispatch_fwd<WIDE>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
-    if (pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
+    if (cols > kNarrow && pick_shape(ceil_div(cols, WIDE), &s))
+      return dispatch_fwd<WIDE, true>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
+    if (cols <= kNarrow && pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
     hipLaunchKernelGGL((ln_fwd_stream_kernel<T, 1024>), dim3(static_cast<unsigned>(rows)), dim3(1024), 0, stream, x,
                        gamma, beta, y, mean, rstd, rows, cols, eps);
     MG_LAUNCH_CHECK();
@@ -533,7 +544,7 @@ struct LayerNormOps {
   // workgroup.  One-wave rows (TPR = 64) of tall matrices use 1024 threads: sixteen rows in
   // flight per workgroup cover the load latency that four do not, and the number of partial
   // sums (one set per workgroup) stays the same.
-  template <int VEC, int TPR, int VPT, bool HAS_STATS, int WG_ = 0>
+  template <int VEC, int TPR, int VPT, bool HAS_STATS, bool ANY, int WG_ = 0>
   static int launch_bwd(const T* dy, const T* x, const T* gamma, const float* mean, const float* rstd,
                         const T* residual, T* dx, T* dgamma, T* dbeta, int64_t rows, int64_t cols, float eps,
                         hipStream_t stream) {
@@ -546,7 +557,7 @@ struct LayerNormOps {
       // workgroup (16 values: 2 % slower, 32 values: spills, 4x slower).
       // MOGRAD_HIP_LN_WIDE_PAIR=0 keeps single rows.
       if (rows >= 4 * static_cast<int64_t>(device_info().cu_count) && env_int("MOGRAD_HIP_LN_WIDE_PAIR", 1) != 0)
-        return launch_bwd<VEC, TPR, VPT, HAS_STATS, 1024>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows,
+        return launch_bwd<VEC, TPR, VPT, HAS_STATS, ANY, 1024>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows,
                                                           cols, eps, stream);
     }
     if constexpr (TPR <= 64 && WG_ == 0) {
@@ -555,7 +566,7 @@ struct LayerNormOps {
       constexpr int TALL_WG = VPT * VEC <= 8 ? 1024 : (VPT * VEC <= 16 ? 512 : 256);
       const int64_t tall = static_cast<int64_t>(device_info().cu_count) * env_int("MOGRAD_HIP_LN_TALL_ROWS_PER_CU", 16);
       if (rows >= tall && TALL_WG > 256)
-        return launch_bwd<VEC, TPR, VPT, HAS_STATS, TALL_WG>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta,
+        return launch_bwd<VEC, TPR, VPT, HAS_STATS, ANY, TALL_WG>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta,
                                                              rows, cols, eps, stream);
     }
     constexpr int WG = WG_ != 0 ? WG_ : (TPR <= 64 ? 256 : TPR);
@@ -574,7 +585,7 @@ struct LayerNormOps {
     Scratch part_g, part_b;
     MG_TRY(part_g.take(groups * cols * static_cast<int64_t>(sizeof(float))));
     MG_TRY(part_b.take(groups * cols * static_cast<int64_t>(sizeof(float))));
-    hipLaunchKernelGGL((ln_bwd_rows_kernel<T, VEC, TPR, VPT, WG, HAS_STATS>), dim3(static_cast<unsigned>(groups)),
+    hipLaunchKernelGGL((ln_bwd_rows_kernel<T, VEC, TPR, VPT, WG, HAS_STATS, ANY>), dim3(static_cast<unsigned>(groups)),
                        dim3(WG), 0, stream, dy, x, gamma, mean, rstd, residual, dx, part_g.as<float>(),
                        part_b.as<float>(), rows,
                        static_cast<int>(cols), eps, rows_per_group,
@@ -585,13 +596,14 @@ struct LayerNormOps {
     return MG_OK;
   }
 
-  template <int VEC, bool HAS_STATS>
+  template <int VEC, bool HAS_STATS, bool ANY = false>
   static int dispatch_bwd(Shape s, const T* dy, const T* x, const T* gamma, const float* mean, const float* rstd,
                           const T* residual, T* dx, T* dgamma, T* dbeta, int64_t rows, int64_t cols, float eps,
                           hipStream_t stream) {
-#define MG_LN_BWD_CASE(TPR_, VPT_)       \
+#define MG_LN_BWD_CASE(TPR_, VPT_)            \
+  if constexpr (VEC > 1 || TPR_ * VPT_ <= 64) \
   if (s.tpr == TPR_ && s.vpt == VPT_)    \
-  return launch_bwd<VEC, TPR_, VPT_, HAS_STATS>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, \
+  return launch_bwd<VEC, TPR_, VPT_, HAS_STATS, ANY>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, \
                                                 stream)
     MG_LN_BWD_CASE(16, 1);
     MG_LN_BWD_CASE(16, 2);
@@ -652,7 +664,10 @@ struct LayerNormOps {
     if (can_vectorise(cols, {dy, x, gamma, dx, residual}) && pick_shape_bwd(cols / WIDE, &s) && fits(s, WIDE))
       return dispatch_bwd<WIDE, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
                                            stream);
-    if (pick_shape_bwd(cols, &s) && fits(s, 1))
+    if (cols > kNarrow && pick_shape_bwd(ceil_div(cols, WIDE), &s) && fits(s, WIDE))
+      return dispatch_bwd<WIDE, HAS_STATS, true>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
+                                                 stream);
+    if (cols <= kNarrow && pick_shape_bwd(cols, &s))
       return dispatch_bwd<1, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, stream);
     if (residual == nullptr)
       return bwd_stream<HAS_STATS>(dy, x, gamma, mean, rstd, dx, dgamma, dbeta, rows, cols, eps, stream);

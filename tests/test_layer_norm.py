@@ -232,3 +232,59 @@ def test_errors(device):
         device.lib.mg_layer_norm_bwd(p, p, p, p, p, p, 4, 0, 1e-5, F32, device.stream)
     with pytest.raises(MogradError, match="null"):
         device.lib.mg_layer_norm_bwd(p, None, p, p, p, p, 4, 4, 1e-5, F32, device.stream)
+
+
+@pytest.mark.parametrize("dtype,half_ulp", [(F32, 2.0 ** -24), (F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
+@pytest.mark.parametrize("cols", [1, 63, 65, 66, 71, 130, 255, 317, 1025, 4101, 8191, 16383])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rows_off_the_16_byte_chunks(device, dtype, half_ulp, cols, offset):
+    # Rows whose last chunk is any part of one, from any element on, in every layout; the elements around the outputs stay
+    # as they are.  Sums of fp32 terms against float64 ones: 2^-20 of the terms' magnitudes, then one rounding.
+    rows = 37 if cols > 1000 else 5
+    x, dy, res = (round_to_dtype(normal(70, i, (rows, cols)) + 0.5, dtype) for i in range(3))
+    gamma, beta = (round_to_dtype(normal(70, 4 + i, (cols,)), dtype) for i in range(2))
+    guard = 16
+
+    def inside(a):
+        flat = np.full(a.size + offset + guard, 7.0, np.float32)
+        flat[offset:offset + a.size] = a.ravel()
+        return AnyBuffer.from_numpy(device, flat, dtype)
+
+    at = lambda buf: buf.data_ptr().value + offset * (4 if dtype == F32 else 2)
+    bx, bdy, bres, bg, bb = map(inside, (x, dy, res, gamma, beta))
+    by, bdx, bdg, bdb = (inside(np.full(n, 7.0)) for n in (x.size, x.size, cols, cols))
+    mean, rstd = AnyBuffer.create(F32, device, rows), AnyBuffer.create(F32, device, rows)
+    device.lib.mg_layer_norm_fwd_stats(at(bx), at(bg), at(bb), at(by), mean.data_ptr(), rstd.data_ptr(), rows, cols, 1e-5, dtype,
+                                       device.stream)
+    x64, dy64, g64 = (t.astype(np.float64) for t in (x, dy, gamma))
+    mu = x64.mean(-1, keepdims=True)
+    rs = 1.0 / np.sqrt(x64.var(-1, keepdims=True) + 1e-5)
+    xhat = (x64 - mu) * rs
+    dyg = dy64 * g64
+    c1, c2 = dyg.mean(-1, keepdims=True), (dyg * xhat).mean(-1, keepdims=True)
+    dx = rs * (dyg - c1 - xhat * c2)
+    spread = np.abs(xhat).max() + rs.max()
+    size = rs * (np.abs(dyg) + np.abs(dyg).mean(-1, keepdims=True) + np.abs(xhat) * np.abs(dyg * xhat).mean(-1, keepdims=True))
+
+    def check(buf, want, terms, what):
+        got = buf.to_numpy()
+        assert (got[:offset] == 7.0).all() and (got[offset + want.size:] == 7.0).all(), f"{what}: written outside"
+        err = np.abs(got[offset:offset + want.size].reshape(want.shape) - want)
+        bound = 1.02 * half_ulp * np.abs(want) + 2.0 ** -18 * spread * terms + 2.0 ** -24
+        assert (err <= bound).all(), f"{what}: {float((err / bound).max())}"
+
+    check(by, xhat * g64 + beta, np.abs(xhat * g64) + np.abs(beta) + 1.0, "y")
+    np.testing.assert_allclose(mean.to_numpy(), mu[:, 0], rtol=1e-5, atol=1e-5)
+    for stats in (False, True):
+        if stats:
+            device.lib.mg_layer_norm_bwd_stats(at(bdy), at(bx), at(bg), mean.data_ptr(), rstd.data_ptr(), at(bdx), at(bdg),
+                                               at(bdb), rows, cols, dtype, device.stream)
+        else:
+            device.lib.mg_layer_norm_bwd(at(bdy), at(bx), at(bg), at(bdx), at(bdg), at(bdb), rows, cols, 1e-5, dtype,
+                                         device.stream)
+        check(bdx, dx, size, "dx")
+        check(bdg, (dy64 * xhat).sum(0), np.abs(dy64 * xhat).sum(0) + rows, "dgamma")
+        check(bdb, dy64.sum(0), np.abs(dy64).sum(0), "dbeta")
+    device.lib.mg_layer_norm_bwd_stats_add(at(bdy), at(bx), at(bg), mean.data_ptr(), rstd.data_ptr(), at(bres), at(bdx), at(bdg),
+                                           at(bdb), rows, cols, dtype, device.stream)
+    check(bdx, dx + res, size + np.abs(res) + (2.0 ** 18 * half_ulp / spread) * np.abs(dx), "dx + residual")
