@@ -280,6 +280,10 @@ def fuse_attention_grad_layout(node: Node, sim: Simplifier) -> Optional[Node]:
     return _refit(node, "FLASH_ATTN_GRAD", [g] + list(node.srcs[1:]), {**node.attrs(), "layout": "bshd"}, sim)
 
 
+_graph.set_rewrites(Simplifier, {f.__name__: f for f in (
+    fuse_matmul_add, fuse_matmul_bias_relu, fuse_relu_grad_into_linear_grad, fuse_add_into_linear_grad, fuse_add_into_layer_norm_grad,
+    fuse_linear_grad_into_layer_norm_grad, fuse_add_into_linear_layer_norm_grad)})
+
 _ADD_RULES = [(f, f.__name__) for f in (fuse_matmul_add, fuse_add_into_layer_norm_grad, fuse_add_into_linear_layer_norm_grad,
                                        fuse_add_into_linear_grad)]
 # Made once and copied: constructing some thirty objects took as long as matching them (a classifier's pass

@@ -1074,6 +1074,8 @@ GRAD_RULES = {
 }
 
 
+_graph.set_gradients(GRAD_RULES, MogradError)
+
 # Sources before consumers, each node once (GraphUtils.toposort).
 _toposort = _graph.toposort
 
@@ -1082,23 +1084,9 @@ def gradient(root: Node, initial_grad: Node, targets: Sequence[Node]) -> List[Op
     """Grad.compute (mograd/grad.mojo:22-91): walks the graph from `root` in reverse
     topological order, applies the rule of each node to its accumulated upstream and adds the
     results to its sources' gradients (ADD nodes where two paths meet).  Returns the gradient
-    node of every target (None if no path reaches it)."""
-    grad_map: Dict[Node, Node] = {root: initial_grad}
-    for node in reversed(_toposort(root)):
-        upstream = grad_map.get(node)
-        if upstream is None or node.dtype() not in (F32, F16, BF16):
-            continue
-        rule = GRAD_RULES.get(node.op_type)
-        if rule is None:
-            if node.srcs:
-                raise MogradError(2, f"no gradient rule for op: {node.op_type}")
-            continue
-        for src, g in zip(node.srcs, rule(node, upstream)):
-            if g is None:
-                continue
-            prev = grad_map.get(src)
-            grad_map[src] = g if prev is None else Node("ADD", g.layout(), g.dtype(), [prev, g])
-    return [grad_map.get(t) for t in targets]
+    node of every target (None if no path reaches it).  The walk is native, and so are this package's
+    own rules for plain nodes; other rules and nodes go through the table's functions."""
+    return _graph.gradient(root, initial_grad, targets, GRAD_RULES)
 
 
 def evaluate(node: Node, device: Device) -> AnyBuffer:

@@ -430,3 +430,82 @@ def test_a_walk_keeps_its_places_when_an_attribute_lookup_walks_too(host):
     get = Node("GETTUPLE", Layout(3, 4), F32, [lin], {Key(): 0, "index": 1})
     got = evaluate_many([get, lin], host.device)
     assert got[0] is dw.bufs[0] and got[1].to_numpy()[0] == 1.0
+
+
+def structure(roots):
+    """What a graph is, whatever its nodes: each node's op, layout, dtype, attributes and sources by place."""
+    order, place = [], {}
+    for node in R._toposort(Node("SINK", Layout(1), F32, [r for r in roots if r is not None])):
+        place[node] = len(order)
+        order.append((node.op_type, node.layout().dims, node.layout().strides, node.layout().base_offset, node.dtype(),
+                      node.attrs(), type(node.srcs), [place[s] for s in node.srcs]))
+    return order, [None if r is None else place[r] for r in roots]
+
+
+def classifier(host, srcs=list, extra=None):
+    params = [host.leaf(4, 6), host.leaf(4), host.leaf(4), host.leaf(4), host.leaf(3, 4), host.leaf(3)]
+    w1, b1, gam, bet, w2, b2 = params
+    x = Node("RESHAPE", Layout(5, 6), F32, srcs([host.leaf(30)]))
+    h = Node("RELU", Layout(5, 4), F32, srcs([Node("MATMUL_BIAS_BT", Layout(5, 4), F32, srcs([x, w1, b1]))]))
+    ln = Node("LAYER_NORM_STATS", Layout(5, 4), F32, srcs([h, gam, bet]), {"eps": 1e-5})
+    y = Node("GETTUPLE", Layout(5, 4), F32, srcs([ln]), {"index": 0, **(extra or {})})
+    h2 = Node("ADD", Layout(5, 4), F32, srcs([Node("MATMUL_BT", Layout(5, 4), F32, srcs([y, host.leaf(4, 4)])), h]))
+    logits = Node("MATMUL_BIAS_BT", Layout(5, 3), F32, srcs([h2, w2, b2]))
+    loss = Node("CROSS_ENTROPY_IDS", Layout(1), F32, srcs([logits, host.leaf(5, dtype=R.I32)]))
+    return loss, params + [x, host.leaf(2)]
+
+
+def transformer(host, **_):
+    from mograd_amd.tiny_transformer import TinyTransformer
+
+    for name in ("mg_fill", "mg_deferred_create"):
+        setattr(host.device.lib, name, lambda *args: 0)  # (the stub has neither)
+    model = TinyTransformer(host.device, 11, 16, 32, 2, 2, compute_dtype=F32)
+    ids, labels = (AnyBuffer.from_numpy(host.device, np.zeros(6, np.int32)) for _ in range(2))
+    loss, leaves = model.graph(ids, labels, 2, 3)
+    return loss, list(leaves.values())
+
+
+@pytest.mark.parametrize("build", [
+    classifier, transformer,
+    lambda host: classifier(host, srcs=tuple),
+    lambda host: classifier(host, extra={"note": [1, 2]}),  # an attribute that only the Python rules look at
+    lambda host: classifier(host, extra={"index": np.int64(0)}),
+], ids=["classifier", "transformer", "tuples", "unusual", "numpy"])
+def test_native_rules_are_the_python_ones(host, monkeypatch, build):
+    def once(table, rules):
+        monkeypatch.setattr(R, "GRAD_RULES", table)
+        loss, targets = build(host)
+        grads = R.gradient(loss, host.leaf(1), targets)
+        plain = structure([loss] + grads)
+        sim = Simplifier(rules)
+        new = sim.run_many([loss] + [g for g in grads if g is not None])
+        return plain, structure(new), sorted(sim.uses.values())
+
+    table = dict(R.GRAD_RULES)
+    own = once(table, GPU_REWRITES())
+    calls = collections.Counter()
+
+    def counted(f):  # another function, which the native walk does not know
+        return lambda *args: (calls.update([f.__name__]), f(*args))[1]
+
+    python = once({op: counted(f) for op, f in table.items()}, [Rule(r.pat, counted(r.func), r.name) for r in GPU_REWRITES()])
+    assert own == python and calls["linear_grad"] and calls["fuse_matmul_add"]
+
+
+def test_a_replaced_gradient_rule_is_the_one_that_runs(host, monkeypatch):
+    x, w = host.leaf(4, 8), host.leaf(3, 8)
+    y = Node("MATMUL_BT", Layout(4, 3), F32, [x, w])
+    mark = host.leaf(4, 8)
+    monkeypatch.setitem(R.GRAD_RULES, "MATMUL_BT", lambda node, upstream: (mark,))  # shorter than the sources
+    assert R.gradient(y, host.leaf(4, 3), [x, w]) == [mark, None]
+
+    class Mine(Simplifier):
+        def single_use(self, node):
+            return False
+
+    relu = Node("RELU", Layout(4, 3), F32, [Node("MATMUL_BIAS_BT", Layout(4, 3), F32, [x, w, host.leaf(3)])])
+    assert Mine(GPU_REWRITES()).run(relu) is relu
+    sim = Simplifier(GPU_REWRITES())
+    sim.single_use = lambda node: False
+    assert sim.run(relu) is relu
