@@ -226,6 +226,19 @@ struct Choice16 {
   int splits;
   double us = 1e30;
 };
+static Choice16 small_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, double no_more_than = 1e30) {
+  const double cus = device_info().cu_count, steps = std::ceil(static_cast<double>(K) / kG16BK);
+  const double out = static_cast<double>(M) * N * batch * 2.0 / 5e6, tiles = static_cast<double>(ceil_div(M, kSmallT) * ceil_div(N, kSmallT) * batch);
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(64, K / env_int("MOGRAD_HIP_GEMM_SPLITK_MIN_K", 256)));
+  Choice16 best{kSmall, 1};
+  for (int s = 1; s <= 16 && (s == 1 || (s <= most && tiles * s <= 2 * cus && steps >= 4 * s)); ++s) {
+    const double sums = s > 1 ? partials_us(tiles * s * kSmallT * kSmallT) : 0.0;
+    if (sums >= std::min(best.us, no_more_than)) break;
+    const double us = 3.4 + out + std::ceil(steps / s) * 0.24 * std::ceil(tiles * s / cus) + sums;
+    if (us < best.us) best = Choice16{kSmall, s, us};
+  }
+  return best;
+}
 // (A search stops where the partial tiles alone, which grow with the ranges, cost more than the best form so far:
 // every call makes this choice, (512, 512) <- 65536 from 71 estimates.)
 static Choice16 choose_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, bool split_lines) {
@@ -251,13 +264,8 @@ static Choice16 choose_16bit(int64_t M, int64_t N, int64_t K, int64_t batch, boo
       offer(t, s, us + out + (N % 8 ? 0.8 : 0.0) + sums);
     }
   }
-  const double tiles64 = tiles_of(kSmallT, kSmallT);
-  for (int s = 1; s <= 16 && (s == 1 || (s <= most && tiles64 * s <= 2 * cus && steps >= 4 * s)); ++s) {
-    const double sums = s > 1 ? partials_us(tiles64 * s * kSmallT * kSmallT) : 0.0;
-    if (sums >= best.us) break;
-    offer(kSmall, s, 3.4 + out + std::ceil(steps / s) * 0.24 * std::ceil(tiles64 * s / cus) + sums);
-  }
-  return best;
+  const Choice16 small = small_16bit(M, N, K, batch, best.us);
+  return small.us < best.us ? small : best;
 }
 // The K range of one workgroup, a multiple of the k-step, and the number of ranges that leaves.
 static int splitk_16bit_range(int64_t K, int* splits) {
@@ -293,7 +301,8 @@ static int launch_16bit_splitk_reduce(const GemmArgs& g, Scratch& partial_mem, i
   return MG_OK;
 }
 
-template <typename T, bool A_KC, bool B_KC>
+// ANY: operands of any alignment, at least 8 elements along the axis that each is contiguous along.
+template <typename T, bool A_KC, bool B_KC, bool ANY = false>
 static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream) {
   const int64_t tiles_m = ceil_div(g.M, kSmallT), tiles_n = ceil_div(g.N, kSmallT), tiles = tiles_m * tiles_n;
   const int k_per_split = splitk_16bit_range(g.K, &splits);
@@ -311,9 +320,9 @@ static int launch_16bit_small(const GemmArgs& g, int splits, hipStream_t stream)
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, pr);
   };
-  if (splits > 1) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, true>);
-  else if (g.bias) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, true, false>);
-  else launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, false>);
+  if (splits > 1) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, true, ANY>);
+  else if (g.bias) launch(gemm_16bit_small_kernel<T, A_KC, B_KC, true, false, ANY>);
+  else launch(gemm_16bit_small_kernel<T, A_KC, B_KC, false, false, ANY>);
   MG_LAUNCH_CHECK();
   return splits > 1 ? launch_16bit_splitk_reduce<T>(g, partial, splits, stream) : MG_OK;
 }
@@ -468,6 +477,20 @@ static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handle
   // 19.9 us against 23.7; (4000, 4001) <- 1025: 68 against 66), the transposing layouts only at a
   // few k-steps ((1999, 767) <- 1001: 51 against 28 us; (16384, 384) <- 65: 9 against 11).
   const bool copy_pays = a_kc && b_kc ? 2.0 * g.batch * g.M * g.N * g.K >= 2e10 : g.K >= 128;
+  // 64 x 64 tiles that are staged through registers, whose steps take a third longer than copied ones, where they are done before
+  // either: us of the routes before | now, (2048, 1000 <- 1001) 20.7 | 15.1, (700, 701 <- 703) 21.0 | 8.5, (300, 3001 <- 517) 15.1 | 7.4,
+  // (5000, 333 <- 777) 21.1 | 12.9, (200, 8001 <- 1023) 28.4 | 15.6, (77, 164 <- 1681) 11.2 | 8.2.
+  const int64_t pipe = env_int("MOGRAD_HIP_GEMM16_PIPE", -1);
+  // (Of the transposing layouts short reductions stay with the ragged variant: (16, 4097 <- 4097) backward 44 | 54.)
+  if (!wide && (a_kc ? g.K : g.M) >= 8 && (b_kc ? g.K : g.N) >= 8 && ((a_kc && b_kc) || g.K >= 128) && !env_str("MOGRAD_HIP_GEMM16_PAD") && (pipe == -1 || pipe == 64)) {
+    const Choice16 small = small_16bit(g.M, g.N, g.K, g.batch);
+    if (pipe == 64 || 1.35 * small.us <= choose_16bit(g.M, g.N, g.K, g.batch, false).us + 7.0) {
+      if (a_kc && b_kc) return launch_16bit_small<T, true, true, true>(g, small.splits, stream);
+      if (a_kc) return launch_16bit_small<T, true, false, true>(g, small.splits, stream);
+      if (b_kc) return launch_16bit_small<T, false, true, true>(g, small.splits, stream);
+      return launch_16bit_small<T, false, false, true>(g, small.splits, stream);
+    }
+  }
   if (!wide && env_int("MOGRAD_HIP_GEMM16_PAD", copy_pays) != 0) {
     if (!a_wide) {
       if (a_kc) MG_TRY(pad.add(&g.a, g.batch, g.M, g.K, &g.sam, &g.bsa));
@@ -697,6 +720,10 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const int64_t cus = device_info().cu_count;
   const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr, db != nullptr);
   if (choice.tile < 0) return MG_OK;
+  // (64 x 64 tiles read arrays that are at least 8 wide from wherever they start, a step a third slower, which up to some 15 us
+  // costs less than the copies: (700, 701 <- 703) 16.8 us with them, 12.7; (1999, 1001 <- 768) 24.5, 25.2; (300, 3001 <- 517)
+  // 26.2, 31.0)
+  const bool any = choice.tile == kSmall && (pad_n || pad_k) && N >= 8 && K >= 8 && choice.us <= 15.0 && !env_str("MOGRAD_HIP_GEMM16_PAD");
   const bool small = choice.tile == kSmall, wide = choice.tile == kTileWide;
   if (ln && (!wide || relu_mask || pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx))) return MG_OK;
   // (without the LayerNorm the same K ranges in 128 x 192 tiles, two workgroups per CU)
@@ -717,8 +744,8 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   if (!small && std::max(N, K) + 8 > kGemmDeepMaxLd) return MG_OK;
   PadCopies<T> pads;
   int64_t no_batch = 0;
-  if (pad_n) MG_TRY(pads.add(&dy, 1, M, N, &ldy, &no_batch));
-  if (pad_k) {
+  if (pad_n && !any) MG_TRY(pads.add(&dy, 1, M, N, &ldy, &no_batch));
+  if (pad_k && !any) {
     MG_TRY(pads.add(&x, 1, M, K, &ldx, &no_batch));
     if (dx) MG_TRY(pads.add(&w, 1, N, K, &ldw, &no_batch));
   }
@@ -748,6 +775,10 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   Scratch db_part;
   int groups = 0;
   const bool db_here = db && env_int("MOGRAD_HIP_LINEAR_BWD_BIAS_IN_LAUNCH", 1) != 0;
+  auto launch_small = [&](auto aligned, auto ragged) {
+    hipLaunchKernelGGL((any ? ragged : aligned), dim3(static_cast<unsigned>(n_dw + x_tiles)), dim3(kGemmThreads), 0, stream, pw2, px,
+                       static_cast<int>(n_dw));
+  };
   if (!split_sums) {
     // nothing to sum: where the gradients are wanted in fp32 they are written so here
     if (dl && dl->out_dtype == MG_F32) {
@@ -756,8 +787,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
     } else if (db_here) {
       pw2.colsum = static_cast<T*>(db);
     }
-    hipLaunchKernelGGL((linear_bwd_small_16bit_kernel<T, false>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
-                       dim3(kGemmThreads), 0, stream, pw2, px, static_cast<int>(n_dw));
+    launch_small(linear_bwd_small_16bit_kernel<T, false, false>, linear_bwd_small_16bit_kernel<T, false, true>);
     MG_LAUNCH_CHECK();
     *db_done = db_here;
     *done = true;
@@ -777,8 +807,7 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
                                    ln_part_g.as<float>(), ln_part_b.as<float>()};
     MG_TRY(launch_linear_bwd_deep<T>(pw2, px2, kTileWide, n_dw, x_tiles, stream));
   } else if (small) {
-    hipLaunchKernelGGL((linear_bwd_small_16bit_kernel<T, true>), dim3(static_cast<unsigned>(n_dw + x_tiles)),
-                       dim3(kGemmThreads), 0, stream, pw2, px, static_cast<int>(n_dw));
+    launch_small(linear_bwd_small_16bit_kernel<T, true, false>, linear_bwd_small_16bit_kernel<T, true, true>);
     MG_LAUNCH_CHECK();
   } else {
     MG_TRY(launch_linear_bwd_deep<T>(pw2, px, deep, n_dw, x_tiles, stream));

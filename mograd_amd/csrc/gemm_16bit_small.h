@@ -110,9 +110,83 @@ __device__ __forceinline__ void gemm16_small_write(const floatx16& acc, uint16_t
   }
 }
 
+// What a thread carries of an operand that does not lie on 16-byte chunks: its chunks of a step, read from any address
+// (extents along the contiguous axis: at least 8).  A chunk that reaches past the end of its row is read as the sixteen
+// bytes that end it and moved down when it is put into LDS, so that no load stands under a condition and none is waited
+// for before its step (moved when they arrive, the tiles on an edge paid a memory latency per step: backward of
+// (1999, 1001 <- 768) 40 us).
+template <bool KC>
+struct SmallAnySource {
+  static constexpr int NW = 4, NI = gemm16_pipe_requests(kSmallT, kSmallBK, NW);
+  const uint16_t* base;
+  int64_t ld;
+  int o0, O, k_begin, K;
+  const uint16_t* row[NI];  // the chunks of the first step
+  __device__ __forceinline__ static void place(int i, int& line, int& chunk) {  // as gemm16_pipe_sources has them
+    const int slot = (i * NW + threadIdx.x / kWave) * kWave + threadIdx.x % kWave;
+    line = slot / 8;
+    chunk = (slot % 8) ^ (KC ? (line / 2) % 8 : gemm16_tr_swizzle<kSmallT>(line));
+  }
+  __device__ __forceinline__ void init(const uint16_t* base_, int64_t ld_, int o0_, int O_, int k_begin_, int K_) {
+    base = base_, ld = ld_, o0 = o0_, O = O_, k_begin = k_begin_, K = K_;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      int line, chunk;
+      place(i, line, chunk);
+      row[i] = KC ? base + static_cast<int64_t>(min(o0 + line, O - 1)) * ld + k_begin + chunk * 8
+                  : base + static_cast<int64_t>(k_begin + line) * ld + min(o0 + chunk * 8, O - 8);
+    }
+  }
+  __device__ __forceinline__ void fetch(int step, uint4 (&v)[NI]) const {
+    const int k0 = k_begin + step * kSmallBK;
+    int64_t back[NI] = {};  // in the last step: what a chunk past the end is moved back by
+    if (k0 + kSmallBK > K) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        int line, chunk;
+        place(i, line, chunk);
+        back[i] = KC ? max(k0 + chunk * 8 + 8 - K, 0) : max(k0 + line + 1 - K, 0) * ld;
+      }
+    }
+    const int64_t by = step * (KC ? static_cast<int64_t>(kSmallBK) : kSmallBK * ld);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const gemm_u4_any r = *reinterpret_cast<const gemm_u4_any*>(row[i] + by - back[i]);
+      v[i] = make_uint4(r[0], r[1], r[2], r[3]);
+    }
+  }
+  __device__ __forceinline__ void put(int step, uint4 (&v)[NI], char* lds_step) const {
+    const int k0 = k_begin + step * kSmallBK;
+    if (k0 + kSmallBK > K || (!KC && o0 + kSmallT > O)) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        int line, chunk;
+        place(i, line, chunk);
+        const int past = max((KC ? k0 : o0) + chunk * 8 + 8 - (KC ? K : O), 0);
+        const bool odd = past & 1, one = past & 2, two = past & 4, none = past >= 8 || (!KC && k0 + line >= K);
+        uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = odd ? w[j] >> 16 | (j < 3 ? w[j + 1] << 16 : 0u) : w[j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = one ? (j < 3 ? w[j + 1] : 0u) : w[j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = none ? 0u : two ? (j < 2 ? w[j + 2] : 0u) : w[j];
+        v[i] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      *reinterpret_cast<uint4*>(lds_step + ((i * NW + threadIdx.x / kWave) * kWave + threadIdx.x % kWave) * 16) = v[i];
+  }
+};
+
 // The work of workgroup `bid` of a launch for one product (see gemm16_deep_block); pr.tiles_m and
-// pr.tiles_n count tiles of 64.  MAY_F32: pr.c32 is looked at.
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM, bool MAY_F32 = COLSUM>
+// pr.tiles_n count tiles of 64.  MAY_F32: pr.c32 is looked at.  ANY: operands that do not lie on 16-byte chunks, which the
+// copies into LDS cannot take, come through registers, two steps of them under way and two in LDS.  Copied to rows that do
+// they cost a launch and a pass of 5 us, and the 128 x 128 kernel that stages them leaves CUs idle: (700, 701 <- 703) bf16
+// forward + backward 38.7 -> 20.6 us, (2048, 1000 <- 1001) forward 20.7 -> 15.1.  A step takes a third longer than a copied one,
+// misaligned chunks being two of the memory path's; more steps under way (four) measured the same.
+template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool COLSUM, bool MAY_F32 = COLSUM, bool ANY = false>
 __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gemm16Problem<T>& pr) {
   constexpr int TT = kSmallT, BK = kSmallBK, NSTAGE = kSmallStages, NW = 4;
   constexpr int NI = gemm16_pipe_requests(TT, BK, NW);  // copy requests per thread, operand and step
@@ -161,8 +235,25 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
   const uint16_t* a16 = reinterpret_cast<const uint16_t*>(A);
   const uint16_t* b16 = reinterpret_cast<const uint16_t*>(B);
   int64_t src_a[NI], src_b[NI];
-  gemm16_pipe_sources<A_KC, BK, TT, NW>(pr.lda, m0, M, src_a);
-  gemm16_pipe_sources<B_KC, BK, TT, NW>(pr.ldb, n0, N, src_b);
+  SmallAnySource<A_KC> any_a;
+  SmallAnySource<B_KC> any_b;
+  uint4 va[2][NI], vb[2][NI];  // ANY: the steps under way
+  if constexpr (ANY) {
+    any_a.init(reinterpret_cast<const uint16_t*>(pr.A + batch * pr.bsa), pr.lda, m0, M, k_begin, K);
+    any_b.init(reinterpret_cast<const uint16_t*>(pr.B + batch * pr.bsb), pr.ldb, n0, N, k_begin, K);
+  } else {
+    gemm16_pipe_sources<A_KC, BK, TT, NW>(pr.lda, m0, M, src_a);
+    gemm16_pipe_sources<B_KC, BK, TT, NW>(pr.ldb, n0, N, src_b);
+  }
+  auto fetch = [&](int set, int step) {
+    any_a.fetch(step, va[set]);
+    any_b.fetch(step, vb[set]);
+  };
+  auto put = [&](int set, int step) {
+    char* at = lds + step % NSTAGE * 2 * OP;
+    any_a.put(step, va[set], at);
+    any_b.put(step, vb[set], at + OP);
+  };
   auto request = [&](int step, int copy) {
     char* at = lds + copy * 2 * OP;
     if (step == full_steps) {
@@ -174,9 +265,20 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
     gemm16_pipe_issue<NI, NW>(b16 + step * b_step, src_b, at + OP);
   };
 
+  if constexpr (!ANY) {
 #pragma unroll
-  for (int s = 0; s < NSTAGE; ++s)
-    if (s < steps) request(s, s);
+    for (int s = 0; s < NSTAGE; ++s)
+      if (s < steps) request(s, s);
+  } else {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      if (s < steps) fetch(s, s);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if (s < steps) put(s, s);
+      if (s + 2 < steps) fetch(s, s + 2);
+    }
+  }
   // The fragments of step `it` + 1 are read while those of step `it` are multiplied, so a step's one
   // synchronisation says two things: step it + 1 has arrived, and every wave holds its fragments of
   // step it, whose copy then takes step it + NSTAGE.
@@ -219,22 +321,27 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
     }
   };
   auto turn = [&](int buf, int it, auto steady) {
-    if constexpr (decltype(steady)::value) {
+    if constexpr (ANY) {
+      meet();
+      if (it + 2 < steps) put(buf, it + 2);  // (its place was last read two steps ago)
+      if (it + 4 < steps) fetch(buf, it + 4);
+    } else if constexpr (decltype(steady)::value) {
       MG_WAIT_VMCNT(2 * NI * (NSTAGE - 2));
       meet();
     } else {
       arrive(min(steps - 2 - it, NSTAGE - 2));
     }
-    if (it + NSTAGE < steps) request(it + NSTAGE, it % NSTAGE);
+    if (!ANY && it + NSTAGE < steps) request(it + NSTAGE, it % NSTAGE);
     read(buf ^ 1, it + 1);
     __builtin_amdgcn_sched_barrier(0);
     multiply(buf);
   };
-  arrive(min(steps - 1, NSTAGE - 1));
+  if constexpr (ANY) meet();
+  else arrive(min(steps - 1, NSTAGE - 1));
   read(0, 0);
   // two turns at a time, so that the fragment buffers have fixed names
   int it = 0;
-  for (; it + NSTAGE < full_steps; it += 2) {
+  for (; !ANY && it + NSTAGE < full_steps; it += 2) {
     turn(0, it, std::true_type{});
     turn(1, it + 1, std::true_type{});
   }
@@ -271,22 +378,22 @@ __device__ __forceinline__ void gemm16_small_block(char* lds, int bid, const Gem
                                            bias_v);
 }
 
-template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K>
+template <typename T, bool A_KC, bool B_KC, bool HAS_BIAS, bool SPLIT_K, bool ANY>
 __global__ __launch_bounds__(256, 2) void gemm_16bit_small_kernel(Gemm16Problem<T> pr) {
   __shared__ __attribute__((aligned(1024))) char lds[kSmallLdsBytes];
   // (dW = dY^T X is the layout that fp32 weight gradients come in)
-  gemm16_small_block<T, A_KC, B_KC, HAS_BIAS, SPLIT_K, false, !A_KC && !B_KC && !HAS_BIAS>(lds, blockIdx.x, pr);
+  gemm16_small_block<T, A_KC, B_KC, HAS_BIAS, SPLIT_K, false, !A_KC && !B_KC && !HAS_BIAS, ANY>(lds, blockIdx.x, pr);
 }
 
 // dX and dW (with db, the column sums of dY) of a Linear layer in one launch, see
 // linear_bwd_16bit_kernel: workgroups [0, n_dw) take dW, the rest dX.
-template <typename T, bool SPLIT>
+template <typename T, bool SPLIT, bool ANY>
 __global__ __launch_bounds__(256, 2) void linear_bwd_small_16bit_kernel(Gemm16Problem<T> dw, Gemm16Problem<T> dx,
                                                                         int n_dw) {
   __shared__ __attribute__((aligned(1024))) char lds[kSmallLdsBytes];
   const int bid = blockIdx.x;
-  if (bid < n_dw) gemm16_small_block<T, false, false, false, SPLIT, true>(lds, bid, dw);
-  else gemm16_small_block<T, true, false, false, false, false>(lds, bid - n_dw, dx);
+  if (bid < n_dw) gemm16_small_block<T, false, false, false, SPLIT, true, true, ANY>(lds, bid, dw);
+  else gemm16_small_block<T, true, false, false, false, false, false, ANY>(lds, bid - n_dw, dx);
 }
 
 }  // namespace mg

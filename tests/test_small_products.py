@@ -96,6 +96,54 @@ def test_every_layout_batched(device, dtype, offset, M, N, K):
             assert_close(c.to_numpy((B, M, N)), want, rt, rt * np.abs(want).max(), la + lb)
 
 
+# 16-bit 64 x 64 tiles of operands off the 16-byte chunks: a reduction and edges that end anywhere in a chunk, every number of
+# steps under way, rows from any element on, K ranges
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("offset", [0, 1, 6])
+@pytest.mark.parametrize("M,N,K", [(8, 9, 8), (9, 64, 63), (65, 10, 65), (64, 71, 129), (70, 66, 193), (67, 130, 257), (33, 129, 321),
+                                   (129, 15, 391), (77, 65, 1681)])
+def test_tiles_of_64_off_the_chunks(device, monkeypatch, dtype, offset, M, N, K):
+    monkeypatch.setenv("MOGRAD_HIP_GEMM16_PIPE", "64")
+    lib, st, rt, B = device.lib, device.stream, RT[dtype], 2
+    a = round_to_dtype(normal(64, 0, (B, M, K)), dtype)
+    b = round_to_dtype(normal(64, 1, (B, N, K), std=0.1), dtype)
+    bias = round_to_dtype(normal(64, 2, (N,)), dtype)
+    want = a.astype(np.float64) @ b.astype(np.float64).transpose(0, 2, 1)
+
+    def up(t):  # (what lies around the operand is no number)
+        flat = np.full(t.size + offset + 16, np.nan, np.float32)
+        flat[offset:offset + t.size] = t.reshape(-1)
+        whole = AnyBuffer.from_numpy(device, flat, dtype)
+        return AnyBuffer(whole.storage, dtype, t.size, offset), whole
+
+    for la in "km":
+        for lb in "kn":
+            (ba, _a), (bb, _b) = up(a if la == "k" else a.transpose(0, 2, 1)), up(b if lb == "k" else b.transpose(0, 2, 1))
+            c = AnyBuffer.create(dtype, device, B * M * N)
+            lib.mg_matmul(ba.data_ptr(), bb.data_ptr(), c.data_ptr(), B, M, N, K, *((K, 1) if la == "k" else (1, M)),
+                          *((1, K) if lb == "k" else (N, 1)), M * K, N * K, dtype, st)
+            assert_close(c.to_numpy((B, M, N)), want, rt, rt * np.abs(want).max(), la + lb)
+    (ba, _a), (bb, _b), (bbias, _c) = up(a), up(b), up(bias)
+    c = AnyBuffer.create(dtype, device, B * M * N)
+    lib.mg_matmul_bias_bt(ba.data_ptr(), bb.data_ptr(), bbias.data_ptr(), c.data_ptr(), B, M, N, K, K, 1, K, 1, M * K, N * K,
+                          dtype, st)
+    assert_close(c.to_numpy((B, M, N)), want + bias, rt, rt * np.abs(want).max(), "bias")
+    # and one launch for a layer's three gradients
+    monkeypatch.delenv("MOGRAD_HIP_GEMM16_PIPE")
+    monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_SMALL", "1")
+    dy = round_to_dtype(normal(64, 3, (M, N), std=0.5), dtype)
+    (bdy, _d), (bx, _x), (bw, _w) = up(dy), up(a[0]), up(b[0])
+    for splits in ("1", "2"):
+        monkeypatch.setenv("MOGRAD_HIP_LINEAR_BWD_SPLITS", splits)
+        dx, dw, db = (AnyBuffer.create(dtype, device, n) for n in (M * K, N * K, N))
+        lib.mg_linear_bwd_fused(bdy.data_ptr(), bx.data_ptr(), bw.data_ptr(), dx.data_ptr(), dw.data_ptr(), db.data_ptr(), M, N, K,
+                                0, 0, dtype, st)
+        x64, w64, dy64 = (t.astype(np.float64) for t in (a[0], b[0], dy))
+        for got, ref, what in ((dx.to_numpy((M, K)), dy64 @ w64, "dx"), (dw.to_numpy((N, K)), dy64.T @ x64, "dw"),
+                               (db.to_numpy(), dy64.sum(0), "db")):
+            assert_close(got, ref, rt, rt * max(np.abs(ref).max(), 1e-3), f"{what}, {splits}")
+
+
 # 16-bit 64 x 64 tiles: k steps of 64 around the four copies, one tile and many, K ranges, both gradient types
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 64, 192), (65, 72, 256), (262, 768, 768), (330, 64, 320), (72, 1032, 64),
