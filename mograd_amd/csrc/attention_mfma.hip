@@ -273,18 +273,8 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 128 ? 2 : 1) void attn_fwd_mfma
     __builtin_amdgcn_s_setprio(0);
   }
 
-  if (m < a.S) {
-    const float inv = 1.0f / l_run;
-    T* orow = o + o_at(a, b, h, m);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dt * 32 + g * 8 + half * 4;
-        if (d < a.D) store4<T>(orow + d, acc_o[dt], g, inv);
-      }
-    if (half == 0) lse[(static_cast<int64_t>(b) * a.H + h) * a.S + m] = m_run * kAttnLn2 + logf(l_run);
-  }
+  store_tile<T>(o + o_at(a, b, h, m_wave), o_ld(a), a.S - m_wave, acc_o, 1.0f / l_run, a.D);
+  if (m < a.S && half == 0) lse[(static_cast<int64_t>(b) * a.H + h) * a.S + m] = m_run * kAttnLn2 + logf(l_run);
 }
 
 // ---- dQ ----------------------------------------------------------------------------------
@@ -520,16 +510,8 @@ __device__ __forceinline__ void attn_dq_block(const int block, char* smem, const
 
 #pragma unroll
   for (int mq = 0; mq < MQ; ++mq) {
-    if (m[mq] < a.S) {
-      T* out = dq + qkv_at(a, b, m[mq], h);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int d = (DT0 + dt) * 32 + g * 8 + half * 4;
-          if (d < a.D) store4<T>(out + d, acc[mq][dt], g, scale);
-        }
-    }
+    const int m0 = m_wave + mq * 32;
+    store_tile<T>(dq + qkv_at(a, b, m0, h) + DT0 * 32, a.ld, a.S - m0, acc[mq], scale, a.D - DT0 * 32);
   }
 }
 
@@ -732,19 +714,27 @@ __device__ __forceinline__ void attn_dkdv_block(const int block, char* smem, con
     }
   }
 
-  if (n < a.S) {
-    T* outk = dk + qkv_at(a, b, n, h);
-    T* outv = dv + qkv_at(a, b, n, h);
+  if constexpr (CAUSAL && DP > 128) {
+    // Eight bytes a lane: this walk takes every register there is, and with store_tile behind it spills 90 of them, not 40
+    // (a backward of B8 H8 S512 D256: 205 us against 175).
+    if (n < a.S) {
+      T* outk = dk + qkv_at(a, b, n, h);
+      T* outv = dv + qkv_at(a, b, n, h);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = (DT0 + dt) * 32 + g * 8 + half * 4;
-        if (d < a.D) {
-          store4<T>(outk + d, acc_k[dt], g, scale);
-          store4<T>(outv + d, acc_v[dt], g, 1.0f);
+        for (int g = 0; g < 4; ++g) {
+          const int d = (DT0 + dt) * 32 + g * 8 + half * 4;
+          if (d < a.D) {
+            store4<T>(outk + d, acc_k[dt], g, scale);
+            store4<T>(outv + d, acc_v[dt], g, 1.0f);
+          }
         }
-      }
+    }
+  } else {
+    const int64_t out = qkv_at(a, b, n_wave, h) + DT0 * 32;
+    store_tile<T>(dk + out, a.ld, a.S - n_wave, acc_k, scale, a.D - DT0 * 32);
+    store_tile<T>(dv + out, a.ld, a.S - n_wave, acc_v, 1.0f, a.D - DT0 * 32);
   }
 }
 
@@ -843,7 +833,8 @@ __device__ __forceinline__ void attn_dkdv_pipe_block(const int block, char* smem
   const int wave = threadIdx.x / kWave;
   const int half = lane / 32;
   const TileLane16<DP> at(lane);
-  const int n = kb * BNK + wave * 32 + lane % 32;
+  const int n_wave = kb * BNK + wave * 32;
+  const int n = n_wave + lane % 32;
   const int64_t bh = static_cast<int64_t>(b) * a.H + h;
 
   uint4 kf[KS], vf[KS];
@@ -1131,20 +1122,9 @@ __device__ __forceinline__ void attn_dkdv_pipe_block(const int block, char* smem
     iteration(P1{}, No{}, No{}, Fresh{}, g + 1);
   }
 
-  if (n < a.S) {
-    T* outk = dk + qkv_at(a, b, n, h);
-    T* outv = dv + qkv_at(a, b, n, h);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dt * 32 + g * 8 + half * 4;
-        if (d < a.D) {
-          store4<T>(outk + d, acc_k[dt], g, scale);
-          store4<T>(outv + d, acc_v[dt], g, 1.0f);
-        }
-      }
-  }
+  const int64_t out = qkv_at(a, b, n_wave, h);
+  store_tile<T>(dk + out, a.ld, a.S - n_wave, acc_k, scale, a.D);
+  store_tile<T>(dv + out, a.ld, a.S - n_wave, acc_v, 1.0f, a.D);
 }
 
 // ---- dQ: software-pipelined walk (head dim <= 64, no bias) -------------------------------
@@ -1411,16 +1391,7 @@ __device__ __forceinline__ void attn_dq_pipe_block(const int block, char* smem, 
     iteration(P1{}, No{}, No{}, Yes{}, g + 1);
   }
 
-  if (m < a.S) {
-    T* out = dq + qkv_at(a, b, m, h);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d = dt * 32 + g4 * 8 + half * 4;
-        if (d < a.D) store4<T>(out + d, acc[dt], g4, scale);
-      }
-  }
+  store_tile<T>(dq + qkv_at(a, b, m_wave, h), a.ld, a.S - m_wave, acc, scale, a.D);
 }
 
 // ---- forward: software-pipelined walk (head dim <= 128, no bias, scale > 0) ----------------
@@ -1698,18 +1669,8 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
 
   MG_ATTN_WAIT_VMCNT(0);  // (the last steps' copies have no reader, but the memory has a next owner)
   const float l_sum = sum_halves(l_run[0] + l_run[1]);
-  if (m < a.S) {
-    const float inv = 1.0f / l_sum;
-    T* orow = o + o_at(a, b, h, m);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d = dt * 32 + g4 * 8 + half * 4;
-        if (d < a.D) store4<T>(orow + d, acc[dt], g4, inv);
-      }
-    if (half == 0) lse[(static_cast<int64_t>(b) * a.H + h) * a.S + m] = m_run * kAttnLn2 + logf(l_sum);
-  }
+  store_tile<T>(o + o_at(a, b, h, m_wave), o_ld(a), a.S - m_wave, acc, 1.0f / l_sum, a.D);
+  if (m < a.S && half == 0) lse[(static_cast<int64_t>(b) * a.H + h) * a.S + m] = m_run * kAttnLn2 + logf(l_sum);
 }
 
 // ---- backward launches --------------------------------------------------------------------
@@ -1883,18 +1844,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
         }
       }
     }
-    if (n < a.S) {
-      T* outk = dk + qkv_at(a, b, n, h);
-      T* outv = dv + qkv_at(a, b, n, h);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int d = dt * 32 + g * 8 + half * 4;
-          store4<T>(outk + d, acc_k[dt], g, scale);
-          store4<T>(outv + d, acc_v[dt], g, 1.0f);
-        }
-    }
+    const int64_t out = qkv_at(a, b, n_wave, h);
+    store_tile<T>(dk + out, a.ld, a.S - n_wave, acc_k, scale, a.D);
+    store_tile<T>(dv + out, a.ld, a.S - n_wave, acc_v, 1.0f, a.D);
   }
 
   // ---- pass 2: dQ of queries 32 wave .. 32 wave + 31
@@ -1948,13 +1900,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
         for (int dt = 0; dt < DT; ++dt) acc[dt] = Mma<T>::run(kt[hf][dt], dsf, acc[dt]);
       }
     }
-    if (m < a.S) {
-      T* out = dq + qkv_at(a, b, m, h);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) store4<T>(out + dt * 32 + g * 8 + half * 4, acc[dt], g, scale);
-    }
+    store_tile<T>(dq + qkv_at(a, b, m_wave, h), a.ld, a.S - m_wave, acc, scale, a.D);
   }
 }
 

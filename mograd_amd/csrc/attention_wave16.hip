@@ -91,8 +91,8 @@ __device__ __forceinline__ bool attn_wave_item(int block, int heads, int tiles, 
 }
 static int attn_wave_blocks(int64_t heads, int64_t tiles) { return static_cast<int>(8 * ((heads * tiles + 7) / 8)); }
 
-// Adds up the waves' partial results, wave w's times f[w], and stores them times `scale`: wave w takes four columns of every
-// eight.  `lds` may hold anything; DT * 16 KB.
+// Adds up the waves' partial results, wave w's times f[w], and stores them times `scale`: a lane takes eight columns of its
+// row, 16 bytes, and its other half the next eight.  `lds` may hold anything; DT * 16 KB.
 template <typename T, int DT>
 __device__ __forceinline__ void attn_wave_merge(char* lds, const floatx16 (&acc)[DT], const float (&f)[4], T* row, bool row_ok,
                                                 float scale, int D, int wave, int lane) {
@@ -105,32 +105,23 @@ __device__ __forceinline__ void attn_wave_merge(char* lds, const floatx16 (&acc)
       x[((wave * DT + dt) * 4 + g) * 64 + lane] = make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
   __syncthreads();
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i = 0; i < (DT + 1) / 2; ++i) {
+    const int g = 8 * i + 2 * wave + lane / 32;
+    if (DT % 2 == 1 && i == DT / 2 && wave >= 2) break;  // past the last tile
+    uint32_t out[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float4 v = x[((w * DT + dt) * 4 + wave) * 64 + lane];
-      t.x = fmaf(v.x, f[w], t.x); t.y = fmaf(v.y, f[w], t.y); t.z = fmaf(v.z, f[w], t.z); t.w = fmaf(v.w, f[w], t.w);
+    for (int part = 0; part < 2; ++part) {
+      float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float4 v = x[(w * DT * 4 + g) * 64 + part * 32 + lane % 32];
+        t.x = fmaf(v.x, f[w], t.x); t.y = fmaf(v.y, f[w], t.y); t.z = fmaf(v.z, f[w], t.z); t.w = fmaf(v.w, f[w], t.w);
+      }
+      out[2 * part] = Mma<T>::pack2(t.x * scale, t.y * scale);
+      out[2 * part + 1] = Mma<T>::pack2(t.z * scale, t.w * scale);
     }
-    const int d = dt * 32 + wave * 8 + (lane / 32) * 4;
-    if (row_ok && d < D) {
-      uint2 w;
-      w.x = Mma<T>::pack2(t.x * scale, t.y * scale);
-      w.y = Mma<T>::pack2(t.z * scale, t.w * scale);
-      *reinterpret_cast<uint2*>(row + d) = w;
-    }
+    if (row_ok && g * 8 < D) *reinterpret_cast<uint4*>(row + g * 8) = make_uint4(out[0], out[1], out[2], out[3]);
   }
-}
-// The same where wave 0 alone has walked.
-template <typename T, int DT>
-__device__ __forceinline__ void attn_wave_store(const floatx16 (&acc)[DT], T* row, float scale, int D, int half) {
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d = dt * 32 + g * 8 + half * 4;
-      if (d < D) store4<T>(row + d, acc[dt], g, scale);
-    }
 }
 
 // sum of a[e] * b[e] over eight packed elements, added to `dot`.
@@ -252,9 +243,9 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_
   T* orow = o + o_at(a, b, h, mc);
   float* lrow = lse + static_cast<int64_t>(bh) * a.S + m;
   if (steps == 1) {
-    if (wave != 0 || !row_ok) return;
-    attn_wave_store<T, DT>(acc, orow, 1.0f / l_row, a.D, half);
-    if (half == 0) *lrow = m_run * kAttnLn2 + logf(l_row);
+    if (wave != 0) return;
+    store_tile<T>(o + o_at(a, b, h, r0), o_ld(a), a.S - r0, acc, 1.0f / l_row, a.D);
+    if (row_ok && half == 0) *lrow = m_run * kAttnLn2 + logf(l_row);
     return;
   }
   float(*ml)[4][32] = reinterpret_cast<float(*)[4][32]>(lds);  // [max, sum][wave][row]
@@ -375,7 +366,7 @@ __device__ __forceinline__ void attn_dq_wave_block(int block, char* lds, const T
   }
   T* row = dq + qkv_at(a, b, mc, h);
   if (steps == 1) {
-    if (wave == 0 && row_ok) attn_wave_store<T, DT>(acc, row, scale, a.D, half);
+    if (wave == 0) store_tile<T>(dq + qkv_at(a, b, r0, h), a.ld, a.S - r0, acc, scale, a.D);
     return;
   }
   const float f[4] = {1.f, 1.f, 1.f, 1.f};
@@ -509,9 +500,10 @@ __device__ __forceinline__ void attn_dkdv_wave_block(int block, char* lds, float
   T* krow = dk + qkv_at(a, b, nc, h);
   T* vrow = dv + qkv_at(a, b, nc, h);
   if (steps - (CAUSAL ? tile : 0) == 1) {
-    if (wave != 0 || !row_ok) return;
-    attn_wave_store<T, DT>(acc_k, krow, scale, a.D, half);
-    attn_wave_store<T, DT>(acc_v, vrow, 1.0f, a.D, half);
+    if (wave != 0) return;
+    const int64_t out = qkv_at(a, b, r0, h);
+    store_tile<T>(dk + out, a.ld, a.S - r0, acc_k, scale, a.D);
+    store_tile<T>(dv + out, a.ld, a.S - r0, acc_v, 1.0f, a.D);
     return;
   }
   const float f[4] = {1.f, 1.f, 1.f, 1.f};

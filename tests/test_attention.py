@@ -295,6 +295,35 @@ def test_whole_head_in_lds_backward(device, monkeypatch, dtype, rtol, causal, B,
         np.testing.assert_array_equal(a, b_)
 
 
+@pytest.mark.parametrize("dtype,tol", [(F16, 2e-3), (BF16, 1.6e-2)])
+@pytest.mark.parametrize("wave16", ["0", "1"])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("S,D", [(1, 8), (33, 24), (95, 40), (130, 64), (65, 72), (129, 104), (34, 128), (70, 136), (129, 256)])
+def test_results_end_with_their_rows(device, monkeypatch, dtype, tol, wave16, name, causal, with_mask, S, D):
+    # A lane stores eight columns after a swap with its other half: rows of an odd number of eights, last tiles cut off, and
+    # what lies behind the last row.
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", wave16)
+    lib, scale = device.lib, 1.0 / math.sqrt(D)
+    q, k, v, do, m = _inputs(64, 1, S, 1, D, dtype, with_mask)
+    bq, bk, bv, bdo = (AnyBuffer.from_numpy(device, t, dtype) for t in (q, k, v, do))
+    bm = AnyBuffer.from_numpy(device, m, dtype) if with_mask else None
+    mask = bm.data_ptr() if with_mask else None
+    out = {n: AnyBuffer.from_numpy(device, np.full(S * D + 64, 7.0, np.float32), dtype) for n in ("o", "dq", "dk", "dv")}
+    lse = AnyBuffer.from_numpy(device, np.full(S + 64, 7.0, np.float32), F32)
+    p = {n: t.data_ptr() for n, t in out.items()}
+    tail = (1, S, 1, D, scale, int(causal), int(with_mask), dtype, device.stream)
+    lib.mg_flash_attn_fwd(bq.data_ptr(), bk.data_ptr(), bv.data_ptr(), mask, p["o"], lse.data_ptr(), *tail)
+    lib.mg_flash_attn_bwd(bdo.data_ptr(), p["o"], bq.data_ptr(), bk.data_ptr(), bv.data_ptr(), mask, lse.data_ptr(), p["dq"], p["dk"],
+                          p["dv"], *tail)
+    for n, t in (*out.items(), ("lse", lse)):
+        assert (t.to_numpy()[-64:] == 7.0).all(), n
+    got = {n: t.to_numpy()[: S * D].reshape(1, S, 1, D) for n, t in out.items()}
+    assert _max_err(got["o"].transpose(0, 2, 1, 3), O.sdpa_fwd(q, k, v, m, causal)[0]) <= tol
+    for n, want in zip(("dq", "dk", "dv"), O.sdpa_bwd(q, k, v, do, m, causal)):
+        # (a single token has dq = dk = 0 exactly; the kernels leave the rounding of dP - delta)
+        assert_attn_grad_close(got[n], want, n, rtol=RTOL_BF16_ATTN * tol / 1.6e-2, floor=ATTN_BF16_FLOOR * tol / 1.6e-2, min_top=1e-2)
+
+
 def test_closed_forms(device):
     B, S, H, D = 1, 128, 1, 8
     z = np.zeros((B, S, H, D), np.float32)
