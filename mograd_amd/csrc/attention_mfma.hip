@@ -1680,30 +1680,32 @@ __global__ __launch_bounds__(kAttnThreads, DP == 64 ? 3 : 2) void attn_fwd_pipe_
 // after loading its resident operand and filling its ring, four workgroups per (batch, head)
 // each read Q, K, V and dO again, and delta needs a launch of its own.  But the four tensors
 // of one (batch, head) are then at most 4 x 256 x 128 bytes = 128 KB and fit one CU's LDS.
-// Here one workgroup of eight waves copies them in once (global_load_lds, the conflict-free
+// Here one workgroup of up to eight waves copies them in once (global_load_lds, the conflict-free
 // image of the pipelined walks), computes delta = rowsum(dO o O) itself, and after one barrier
 // every wave runs, straight from LDS, first the dK/dV products of its own 32 keys over the
 // query tiles and then the dQ products of its own 32 queries over the key tiles: the per-tile
 // arithmetic of attn_dkdv_block and attn_dq_block, with no streaming and no further barrier.
 // Causal: wave w meets 8 - w query tiles in the first pass and w + 1 key tiles in the second,
 // so the waves carry equal loads without waiting for each other between the passes.
+// RS: the rows that there is room for, 64, 128 or 256, and 32 to a wave.  A sequence takes the smallest that holds it, so that
+// two or four short heads share a CU, which with room for 256 had one of a few waves: B64 H12 S64, causal, 20.6 -> 12.5 us;
+// B128 H12 S32 26.7 -> 14.3; B100 H6 S100, causal, 26.1 -> 19.8.
 constexpr int kResidentS = 256;
-constexpr int kResidentTensor = kResidentS * 128;                        // bytes of one tensor's image
-constexpr int kResidentLds = 4 * kResidentTensor + 2 * kResidentS * 4;   // Q, K, V, dO, -lse, -delta
 
-template <typename T, bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
+template <typename T, bool CAUSAL, int RS>
+__global__ __launch_bounds__(2 * RS, 2) void attn_bwd_resident_kernel(
     const T* __restrict__ d_o, const T* __restrict__ o, const T* __restrict__ q, const T* __restrict__ k,
     const T* __restrict__ v, const float* __restrict__ lse, T* __restrict__ dq, T* __restrict__ dk, T* __restrict__ dv,
     AttnDims a, float scale) {
-  constexpr int DP = 64, KS = DP / 16, DT = DP / 32;
-  __shared__ __attribute__((aligned(1024))) char smem[kResidentLds];
+  constexpr int DP = 64, KS = DP / 16, DT = DP / 32, WAVES = RS / 32;
+  constexpr int TENSOR = RS * tile_row_bytes<DP>();  // bytes of one tensor's image
+  __shared__ __attribute__((aligned(1024))) char smem[4 * TENSOR + 2 * RS * 4];  // Q, K, V, dO, -lse, -delta
   const char* const q_rows = smem;
-  const char* const k_rows = smem + kResidentTensor;
-  const char* const v_rows = smem + 2 * kResidentTensor;
-  const char* const do_rows = smem + 3 * kResidentTensor;
-  float* const nlse_s = reinterpret_cast<float*>(smem + 4 * kResidentTensor);
-  float* const ndelta_s = nlse_s + kResidentS;
+  const char* const k_rows = smem + TENSOR;
+  const char* const v_rows = smem + 2 * TENSOR;
+  const char* const do_rows = smem + 3 * TENSOR;
+  float* const nlse_s = reinterpret_cast<float*>(smem + 4 * TENSOR);
+  float* const ndelta_s = nlse_s + RS;
 
   const int bh = blockIdx.x;
   const int b = bh / a.H, h = bh % a.H;
@@ -1713,7 +1715,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
   const int n_tiles = (a.S + 31) / 32;
 
   // ---- copies: wave instruction j of a tensor covers its rows 8j .. 8j+7 (1 KB); this wave
-  // issues j = wave, wave + 8, ...  Lane l writes chunk position l % 8 of row 8j + l / 8 and
+  // issues j = wave, wave + WAVES, ...  Lane l writes chunk position l % 8 of row 8j + l / 8 and
   // therefore names the source chunk (l % 8) ^ swz16(row), with row % 16 = 8 (wave % 2) + l / 8.
   // Rows past the end of the sequence (up to the end of its last 32-row tile) copy the last row.
   {
@@ -1728,12 +1730,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_resident_kernel(
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int jj = 0; jj < kResidentS / 64; ++jj) {
-        const int j = wave + 8 * jj;
+      for (int jj = 0; jj < 4; ++jj) {
+        const int j = wave + WAVES * jj;
         if (8 * j < n_tiles * 32) {
           const int row = min(8 * j + cp_row, a.S - 1);
           const unsigned off = row * (t == 3 ? do_pitch : qkv_pitch) + cp_col;
-          const unsigned dst = __builtin_amdgcn_readfirstlane(smem_base + t * kResidentTensor + j * 1024);
+          const unsigned dst = __builtin_amdgcn_readfirstlane(smem_base + t * TENSOR + j * 1024);
           asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(src[t]) : "memory");
         }
       }
@@ -2137,16 +2139,20 @@ static int bwd_typed(const void* d_o, const void* o, const void* q, const void* 
     if (a.D == 64 && a.S <= kResidentS && !has_bias && env_int("MOGRAD_HIP_ATTN_RESIDENT", 1) != 0 &&
         static_cast<int64_t>(a.S) * a.ld * 2 < 0x7fffffffLL) {
       const dim3 grid(static_cast<unsigned>(a.B * a.H));
-      if (causal)
-        hipLaunchKernelGGL((attn_bwd_resident_kernel<T, true>), grid, dim3(512), 0, stream, static_cast<const T*>(d_o),
-                           static_cast<const T*>(o), static_cast<const T*>(q), static_cast<const T*>(k),
-                           static_cast<const T*>(v), lse, static_cast<T*>(dq), static_cast<T*>(dk), static_cast<T*>(dv), a,
-                           scale);
-      else
-        hipLaunchKernelGGL((attn_bwd_resident_kernel<T, false>), grid, dim3(512), 0, stream, static_cast<const T*>(d_o),
-                           static_cast<const T*>(o), static_cast<const T*>(q), static_cast<const T*>(k),
-                           static_cast<const T*>(v), lse, static_cast<T*>(dq), static_cast<T*>(dk), static_cast<T*>(dv), a,
-                           scale);
+      auto launch = [&](auto rows, auto causal_walk) {
+        constexpr int RS = decltype(rows)::value;
+        hipLaunchKernelGGL((attn_bwd_resident_kernel<T, decltype(causal_walk)::value, RS>), grid, dim3(2 * RS), 0, stream,
+                           static_cast<const T*>(d_o), static_cast<const T*>(o), static_cast<const T*>(q),
+                           static_cast<const T*>(k), static_cast<const T*>(v), lse, static_cast<T*>(dq), static_cast<T*>(dk),
+                           static_cast<T*>(dv), a, scale);
+      };
+      auto launch_rows = [&](auto causal_walk) {
+        if (a.S <= 64) launch(std::integral_constant<int, 64>{}, causal_walk);
+        else if (a.S <= 128) launch(std::integral_constant<int, 128>{}, causal_walk);
+        else launch(std::integral_constant<int, kResidentS>{}, causal_walk);
+      };
+      if (causal) launch_rows(std::true_type{});
+      else launch_rows(std::false_type{});
       MG_LAUNCH_CHECK();
       return MG_OK;
     }

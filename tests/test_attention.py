@@ -213,16 +213,12 @@ def test_long_ragged_sequence(device, causal, D):
         assert_attn_grad_close(got, want, what)
 
 
-@pytest.mark.parametrize("dtype,half_ulp", [(F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
-@pytest.mark.parametrize("name,causal,with_mask", MODES)
-@pytest.mark.parametrize("B,H,S,D", [(1, 1, 1, 8), (2, 3, 16, 64), (1, 2, 33, 32), (1, 2, 58, 64), (1, 3, 128, 96), (1, 1, 129, 128),
-                                     (2, 1, 161, 80), (1, 2, 257, 24), (1, 1, 300, 72), (1, 1, 65, 128)])
-def test_workgroups_of_32_rows(device, monkeypatch, dtype, half_ulp, name, causal, with_mask, B, H, S, D):
-    # One row to several tiles per wave, waves without a tile, columns that fill a kernel's width and that do not.  A weight, a
-    # score gradient and a result are each rounded once: a sum over rounded factors is off by at most half a unit of its
-    # terms' magnitudes; what is computed in fp32 (scores of up to ten, their exponentials, sums) by 2^-18 of them.
-    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", "1")
-    q, k, v, do, m = _inputs(63, B, S, H, D, dtype, with_mask)
+def _assert_rounded_once(device, dtype, half_ulp, causal, with_mask, cfg, B, H, S, D, scaled=False):
+    # A weight, a score gradient and a result are each rounded once: a sum over rounded factors is off by at most half a unit of
+    # its terms' magnitudes; what is computed in fp32 (scores of up to ten, their exponentials, sums) by 2^-18 of them.  `scaled`:
+    # the backward rounds its scaled operand of the scores to 16 bits as well, so that a score is off by half a unit of its
+    # terms, a weight and a score gradient by as much of themselves.
+    q, k, v, do, m = _inputs(cfg, B, S, H, D, dtype, with_mask)
     got = _fwd_bwd(device, q, k, v, do, m, causal, dtype=dtype)
     q, k, v = (t.astype(np.float64).transpose(0, 2, 1, 3) for t in (q, k, v))
     do = do.astype(np.float64)
@@ -239,7 +235,10 @@ def test_workgroups_of_32_rows(device, monkeypatch, dtype, half_ulp, name, causa
     ds = p * (do @ turned(v) - (do * got[0]).sum(-1, keepdims=True))
     # the fp32 part of dS, P (dP - delta), cancels: its terms are at most these
     terms = p * (np.abs(do) @ turned(np.abs(v)) + np.abs(do * got[0]).sum(-1, keepdims=True))
+    score = half_ulp * scale * (np.abs(q) @ turned(np.abs(k))) if scaled else np.zeros_like(p)
     back = lambda t: t.transpose(0, 2, 1, 3)
+    by_score = {"dq": back((np.abs(ds) * score) @ np.abs(k) * scale), "dk": back(turned(np.abs(ds) * score) @ np.abs(q) * scale),
+                "dv": back(turned(p * score) @ np.abs(do))}
     want = {"o": (p @ v, p @ np.abs(v), p @ np.abs(v)), "lse": ((top + np.log(total))[..., 0], None, None),
             "dq": tuple(back(x @ y * scale) for x, y in ((ds, k), (np.abs(ds), np.abs(k)), (terms, np.abs(k)))),
             "dk": tuple(back(turned(x) @ y * scale) for x, y in ((ds, q), (np.abs(ds), np.abs(q)), (terms, np.abs(q)))),
@@ -251,8 +250,27 @@ def test_workgroups_of_32_rows(device, monkeypatch, dtype, half_ulp, name, causa
         if rounded is None:
             assert err.max() <= 1e-5, what
             continue
-        bound = 1.02 * half_ulp * (rounded + np.abs(ref)) + 2.0 ** -18 * exact + tiny
+        bound = 1.02 * half_ulp * (rounded + np.abs(ref)) + 2.0 ** -18 * exact + tiny + 1.02 * by_score.get(what, 0.0)
         assert (err <= bound).all(), f"{what}: {float((err / np.maximum(bound, 1e-30)).max())}"
+
+
+@pytest.mark.parametrize("dtype,half_ulp", [(F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("B,H,S,D", [(1, 1, 1, 8), (2, 3, 16, 64), (1, 2, 33, 32), (1, 2, 58, 64), (1, 3, 128, 96), (1, 1, 129, 128),
+                                     (2, 1, 161, 80), (1, 2, 257, 24), (1, 1, 300, 72), (1, 1, 65, 128)])
+def test_workgroups_of_32_rows(device, monkeypatch, dtype, half_ulp, name, causal, with_mask, B, H, S, D):
+    # One row to several tiles per wave, waves without a tile, columns that fill a kernel's width and that do not.
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", "1")
+    _assert_rounded_once(device, dtype, half_ulp, causal, with_mask, 63, B, H, S, D)
+
+
+@pytest.mark.parametrize("dtype,half_ulp", [(F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,H,S", [(5, 2, 2), (3, 2, 32), (1, 2, 63), (2, 3, 64), (3, 1, 65), (2, 2, 97), (1, 3, 127), (2, 1, 129)])
+def test_whole_heads_take_the_room_they_need(device, monkeypatch, dtype, half_ulp, causal, B, H, S):
+    # room for 64, 128 or 256 rows: either side of each, waves with rows and without
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_RESIDENT", "1")
+    _assert_rounded_once(device, dtype, half_ulp, causal, False, 65, B, H, S, 64, scaled=True)
 
 
 @pytest.mark.parametrize("causal", [True, False])
