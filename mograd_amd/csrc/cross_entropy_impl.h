@@ -23,6 +23,11 @@ constexpr float kLn2 = 0.6931471805599453f;
 
 __device__ __forceinline__ float fast_exp2(float v) { return __builtin_amdgcn_exp2f(v); }
 
+// Rows that do not lie on 16-byte chunks (ANY below) are read and written in misaligned ones, with -inf past a row's end: it
+// is no maximum and adds nothing to a sum of exponentials.
+template <typename T>
+constexpr uint32_t kMinusInfWord = sizeof(T) == 4 ? 0xff800000u : std::is_same<T, f16_t>::value ? 0xfc00fc00u : 0xff80ff80u;
+
 template <int TPR, int WG, int K>
 __device__ __forceinline__ void row_allreduce_max(float (&v)[K], float* slots, int& phase) {
   if constexpr (TPR == 16) {
@@ -50,12 +55,12 @@ __device__ __forceinline__ int64_t load_id(const void* ids, int64_t row, bool id
 //   upstream: one element of T, or nullptr for 1.
 // ------------------------------------------------------------------------------------
 
-template <typename T, int VEC, int TPR, int VPT, int WG, bool DENSE>
+template <typename T, int VEC, int TPR, int VPT, int WG, bool DENSE, bool ANY>
 __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void ce_rows_kernel(
     const T* __restrict__ logits, const void* __restrict__ labels, const T* __restrict__ upstream,
     float* __restrict__ rowloss, T* __restrict__ dlogits, int64_t N, int C, int id64) {
   constexpr int RPW = WG / TPR;
-  using Tile = RowTile<T, VEC, TPR, VPT>;
+  using Tile = RowTile<T, VEC, TPR, VPT, ANY>;
   __shared__ float slots[2 * (WG / kWave)];
   int t, sub;
   row_thread<TPR, WG>(t, sub);
@@ -70,9 +75,9 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
     if (row >= N) return;  // per 16-lane row, per wave or per workgroup (RPW == 1); no barrier follows for TPR <= 64
     const T* xr = logits + row * C;
     Tile x;
-    x.load(xr, t, C);
+    x.load(xr, t, C, kMinusInfWord<T>);
 
-    // Padding chunks hold zeros: mask them to -inf for the max and skip them in the sums.
+    // Absent chunks hold zeros: mask them to -inf for the max and skip them in the sums.
     const int nfull = Tile::full_chunks(C);
     float m[1] = {-INFINITY};
 #pragma unroll
@@ -115,13 +120,17 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
       for (int i = 0; i < VPT; ++i) {
         if (i < nfull || (i == nfull && Tile::col(i, t) < C)) {
           float y[VEC], out[VEC];
-          VecIO<T, VEC>::load(yr + i * (TPR * VEC) + lane_off, y);
+          const int c = Tile::col(i, t);
+          if (i < nfull) Tile::load_chunk(yr + i * (TPR * VEC) + lane_off, y);
+          else Tile::load_end(yr + i * (TPR * VEC) + lane_off, c, C, y);
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
-            acc[0] += (x.v[i][e] - shift) * y[e];
+            const float term = (x.v[i][e] - shift) * y[e];
+            acc[0] += !ANY || i < nfull || Tile::in_row(c, e, C) ? term : 0.f;
             out[e] = (fast_exp2(fmaf(x.v[i][e], kLog2e, -shift2)) - y[e]) * scale;
           }
-          VecIO<T, VEC>::store(out_row + i * (TPR * VEC) + lane_off, out);
+          if (i < nfull) Tile::store_chunk(out_row + i * (TPR * VEC) + lane_off, out);
+          else Tile::store_end(out_row + i * (TPR * VEC) + lane_off, c, C, out);
         }
       }
       if (rowloss != nullptr) {
@@ -176,6 +185,25 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
   }
 }
 
+// Eight 16-bit values out of four registers, word by word: seen as an array of eight, fp16 values were held one to a
+// register, and spilled ((8192, 50304) 610 us against 341).
+template <typename T>
+__device__ __forceinline__ void unpack_words(const uint4& r, float (&x)[8]) {
+  const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (std::is_same<T, f16_t>::value) {
+      typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+      const half2_t h = __builtin_bit_cast(half2_t, w[i]);
+      x[2 * i] = static_cast<float>(h[0]);
+      x[2 * i + 1] = static_cast<float>(h[1]);
+    } else {
+      x[2 * i] = __uint_as_float(w[i] << 16);
+      x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+  }
+}
+
 // Integer labels, 16-bit logits, rows of thousands of columns: the row stays in
 // registers as loaded (eight 16-bit values per 128-bit register quad) and is unpacked in each of
 // its three passes (maximum, sum of exponentials, gradient), so a thread holds VPT * 4 registers
@@ -183,7 +211,7 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
 // they were loaded into spill (656 bytes per lane at 50304 columns: 1.36 TB/s).  The second
 // exponential per element is free in a kernel that waits for memory.  The arithmetic per element
 // is that of ce_rows_kernel, so are the bits.  One row per workgroup.
-template <typename T, int TPR, int VPT>
+template <typename T, int TPR, int VPT, bool ANY>
 __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 ? 2 : 1)) void ce_rows_packed_kernel(
     const T* __restrict__ logits, const void* __restrict__ labels, const T* __restrict__ upstream,
     float* __restrict__ rowloss, T* __restrict__ dlogits, int64_t N, int C, int id64) {
@@ -198,24 +226,40 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
   const T* xr = logits + row * C;
   T* out_row = dlogits + row * C;
   const int nfull = (C / VEC) / TPR;  // chunk indices below it exist for every thread
-  const bool tail = (nfull * TPR + t) * VEC < C;  // this thread's chunk `nfull` exists
+  const int last = (nfull * TPR + t) * VEC;  // the column of this thread's chunk `nfull`,
+  const bool tail = last < C;                // if it exists
+  // On 16-byte chunks it is one like the others; else it may end with the row, and has registers and code of its own, which
+  // as a case of every one of VPT chunks took 25 more registers ((8192, 50257) bf16 391 us; in the aligned form the own
+  // registers cost 1.5 %).
+  auto here = [&](int i) { return i < nfull || (!ANY && i == nfull && tail); };
 
-  uint4 raw[VPT];
+  using Tile = RowTile<T, VEC, TPR, VPT, ANY>;
+  uint4 raw[VPT], end = make_uint4(0, 0, 0, 0);
+  if (ANY && tail) {
+    uint32_t w[4];
+    VecAny<T, VEC>::words_end(xr + last, max(last + VEC - C, 0), kMinusInfWord<T>, w);
+    end = make_uint4(w[0], w[1], w[2], w[3]);
+  }
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     raw[i] = make_uint4(0, 0, 0, 0);
-    if (i < nfull || (i == nfull && tail)) raw[i] = *reinterpret_cast<const uint4*>(xr + (i * TPR + t) * VEC);
-  }
-  float m[1] = {-INFINITY};
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    if (i < nfull || (i == nfull && tail)) {
-      float x[VEC];
-      VecIO<T, VEC>::load(reinterpret_cast<const T*>(&raw[i]), x);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) m[0] = fmaxf(m[0], x[e]);
+    if (here(i)) {
+      using Chunk = typename std::conditional<ANY, mg_u4_any, mg_u4>::type;
+      const Chunk w = *reinterpret_cast<const Chunk*>(xr + (i * TPR + t) * VEC);
+      raw[i] = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
+  float m[1] = {-INFINITY};
+  auto top = [&](const uint4& r) {
+    float x[VEC];
+    unpack_words<T>(r, x);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) m[0] = fmaxf(m[0], x[e]);
+  };
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+    if (here(i)) top(raw[i]);
+  if (ANY && tail) top(end);
   row_allreduce_max<TPR, TPR, 1>(m, slots, phase);
   const float m2 = m[0] * kLog2e;
   // Between the passes the packed registers are made opaque to the compiler, which would
@@ -223,30 +267,40 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
   auto forget = [&]() {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) asm volatile("" : "+v"(raw[i].x), "+v"(raw[i].y), "+v"(raw[i].z), "+v"(raw[i].w));
+    if constexpr (ANY) asm volatile("" : "+v"(end.x), "+v"(end.y), "+v"(end.z), "+v"(end.w));
   };
   forget();
   float s[1] = {0.f};
+  auto add = [&](const uint4& r) {
+    float x[VEC];
+    unpack_words<T>(r, x);
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    if (i < nfull || (i == nfull && tail)) {
-      float x[VEC];
-      VecIO<T, VEC>::load(reinterpret_cast<const T*>(&raw[i]), x);
+    for (int e = 0; e < VEC; ++e) s[0] += fast_exp2(fmaf(x[e], kLog2e, -m2));
+  };
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) s[0] += fast_exp2(fmaf(x[e], kLog2e, -m2));
-    }
-  }
+  for (int i = 0; i < VPT; ++i)
+    if (here(i)) add(raw[i]);
+  if (ANY && tail) add(end);
   row_allreduce_sum<TPR, TPR, 1>(s, slots, phase);
   const float k = scale / s[0];
   forget();
+  auto gradient = [&](const uint4& r, float (&x)[VEC]) {
+    unpack_words<T>(r, x);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[e] = fast_exp2(fmaf(x[e], kLog2e, -m2)) * k;
+  };
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    if (i < nfull || (i == nfull && tail)) {
+    if (here(i)) {
       float x[VEC];
-      VecIO<T, VEC>::load(reinterpret_cast<const T*>(&raw[i]), x);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) x[e] = fast_exp2(fmaf(x[e], kLog2e, -m2)) * k;
-      VecIO<T, VEC>::store(out_row + (i * TPR + t) * VEC, x);
+      gradient(raw[i], x);
+      Tile::store_chunk(out_row + (i * TPR + t) * VEC, x);
     }
+  }
+  if (ANY && tail) {
+    float x[VEC];
+    gradient(end, x);
+    Tile::store_end(out_row + last, last, C, x);
   }
   // the "- 1" at the label column: a scalar store by the thread that owns the column, after its
   // vector stores (same thread, same address: program order holds)
@@ -263,23 +317,33 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
 }
 
 // ------------------------------------------------------------------------------------
-// Streaming kernels: any C, any alignment.  One workgroup per row.
+// Streaming kernels: any C.  One workgroup per row.  ANY: at any address, C >= VEC.
 // ------------------------------------------------------------------------------------
+
+// The chunk at column c < C of a row at any address, `fill` past the row's end.
+template <typename T, int VEC>
+__device__ __forceinline__ void stream_load(const T* row, int64_t c, int64_t C, uint32_t fill, float (&v)[VEC]) {
+  uint32_t w[4];
+  VecAny<T, VEC>::words_end(row + c, static_cast<int>(max(c + VEC - C, int64_t{0})), fill, w);
+  VecAny<T, VEC>::unpack(w, v);
+}
 
 // Online (max, sum-exp) over the elements a thread visits, merged across the workgroup.  ONCE: the
 // row is not read again by this kernel, so its loads go past the caches.
-template <typename T, int VEC, int WG, bool ONCE = false>
+template <typename T, int VEC, int WG, bool ONCE = false, bool ANY = false>
 __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t C, float* slots, int& phase, float& m_out,
                                                float& s_out) {
   auto fetch = [](const T* p, float (&v)[VEC]) {
-    if constexpr (ONCE) VecIO<T, VEC>::load_stream(p, v);
+    if constexpr (ANY) VecAny<T, VEC>::load(p, v);
+    else if constexpr (ONCE) VecIO<T, VEC>::load_stream(p, v);
     else VecIO<T, VEC>::load(p, v);
   };
   float m = -INFINITY, s = 0.f;
   constexpr int U = 4;  // chunks in flight per thread: the loop is bound by memory-level parallelism
   const int64_t step = static_cast<int64_t>(WG) * VEC;
+  const int64_t whole = ANY ? C - C % VEC : C;  // where the last whole chunk ends
   int64_t c = static_cast<int64_t>(threadIdx.x) * VEC;
-  for (; c + (U - 1) * step < C; c += U * step) {
+  for (; c + (U - 1) * step < whole; c += U * step) {
     float v[U][VEC];
 #pragma unroll
     for (int u = 0; u < U; ++u) fetch(xr + c + u * step, v[u]);
@@ -300,7 +364,8 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
   }
   for (; c < C; c += step) {
     float v[VEC];
-    fetch(xr + c, v);
+    if constexpr (ANY) stream_load<T, VEC>(xr, c, C, kMinusInfWord<T>, v);
+    else fetch(xr + c, v);
     float cm = v[0];
 #pragma unroll
     for (int e = 1; e < VEC; ++e) cm = fmaxf(cm, v[e]);
@@ -329,7 +394,7 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
 // ONCE: the logits (and dense labels) are larger than the memory-side cache can hold, so they are
 // read past the caches (1.65 GB of logits: 266 -> 238 us, 6.9 TB/s; smaller tensors may still be
 // cached from the kernel that wrote them and keep the plain loads).
-template <typename T, int VEC, int WG, bool DENSE, bool ONCE = false>
+template <typename T, int VEC, int WG, bool DENSE, bool ONCE = false, bool ANY = false>
 __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__ logits, const void* __restrict__ labels,
                                                            float* __restrict__ rowloss, int64_t N, int64_t C, int id64) {
   __shared__ float slots[2 * 2 * (WG / kWave)];
@@ -345,7 +410,10 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
     float tm = -INFINITY, ts = 0.f;
     for (int64_t c = static_cast<int64_t>(threadIdx.x) * VEC; c < C; c += static_cast<int64_t>(WG) * VEC) {
       float v[VEC], y[VEC];
-      if constexpr (ONCE) {
+      if constexpr (ANY) {
+        stream_load<T, VEC>(xr, c, C, kMinusInfWord<T>, v);
+        stream_load<T, VEC>(yr, c, C, 0, y);
+      } else if constexpr (ONCE) {
         VecIO<T, VEC>::load_stream(xr + c, v);
         VecIO<T, VEC>::load_stream(yr + c, y);
       } else {
@@ -363,7 +431,7 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         ts += fast_exp2(fmaf(v[e], kLog2e, -m2));
-        dot[0] += v[e] * y[e];
+        dot[0] += !ANY || c + e < C ? v[e] * y[e] : 0.f;
         dot[1] += y[e];
       }
     }
@@ -377,7 +445,7 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
     s = red[0];
     if (threadIdx.x == 0) rowloss[row] = -(red[1] - (m + logf(s)) * red[2]) * inv_rows;
   } else {
-    stream_max_sum<T, VEC, WG, ONCE>(xr, C, slots, phase, m, s);
+    stream_max_sum<T, VEC, WG, ONCE, ANY>(xr, C, slots, phase, m, s);
     if (threadIdx.x == 0) {
       const int64_t id = load_id(labels, row, id64 != 0);
       rowloss[row] = (id < 0 || id >= C) ? NAN : -(to_float(xr[id]) - (m + logf(s))) * inv_rows;
@@ -386,7 +454,7 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
 }
 
 // Gradient (and optionally loss) for rows too wide for registers: two passes.
-template <typename T, int VEC, int WG, bool DENSE>
+template <typename T, int VEC, int WG, bool DENSE, bool ANY = false>
 __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict__ logits, const void* __restrict__ labels,
                                                             const T* __restrict__ upstream, float* __restrict__ rowloss,
                                                             T* __restrict__ dlogits, int64_t N, int64_t C, int id64) {
@@ -399,7 +467,7 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
   const float inv_rows = 1.0f / static_cast<float>(N);
   const float scale = (upstream != nullptr ? to_float(upstream[0]) : 1.0f) * inv_rows;
   float m, s;
-  stream_max_sum<T, VEC, WG>(xr, C, slots, phase, m, s);
+  stream_max_sum<T, VEC, WG, false, ANY>(xr, C, slots, phase, m, s);
   const float m2 = m * kLog2e;
   const float inv_sum = 1.0f / s;
   const float shift = m + logf(s);
@@ -407,12 +475,21 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
   float acc[1] = {0.f};
   constexpr int U = DENSE ? 1 : 4;  // integer labels: four chunks in flight per thread
   const int64_t step = static_cast<int64_t>(WG) * VEC;
+  const int64_t whole = ANY ? C - C % VEC : C;  // where the last whole chunk ends
   int64_t c0 = static_cast<int64_t>(threadIdx.x) * VEC;
+  auto put = [&](int64_t c, const float (&out)[VEC]) {
+    if constexpr (!ANY) VecIO<T, VEC>::store(out_row + c, out);
+    else if (c < whole) VecAny<T, VEC>::store(out_row + c, out);
+    else VecAny<T, VEC>::store_first(out_row + c, static_cast<int>(C - c), out);
+  };
   if constexpr (!DENSE) {
-    for (; c0 + (U - 1) * step < C; c0 += U * step) {
+    for (; c0 + (U - 1) * step < whole; c0 += U * step) {
       float v[U][VEC];
 #pragma unroll
-      for (int u = 0; u < U; ++u) VecIO<T, VEC>::load(xr + c0 + u * step, v[u]);
+      for (int u = 0; u < U; ++u) {
+        if constexpr (ANY) VecAny<T, VEC>::load(xr + c0 + u * step, v[u]);
+        else VecIO<T, VEC>::load(xr + c0 + u * step, v[u]);
+      }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t c = c0 + u * step;
@@ -426,19 +503,23 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
           }
           out[e] = p * scale;
         }
-        VecIO<T, VEC>::store(out_row + c, out);
+        put(c, out);
       }
     }
   }
   for (int64_t c = c0; c < C; c += step) {
     float v[VEC], out[VEC];
-    VecIO<T, VEC>::load(xr + c, v);
+    if constexpr (ANY) stream_load<T, VEC>(xr, c, C, kMinusInfWord<T>, v);
+    else VecIO<T, VEC>::load(xr + c, v);
     if constexpr (DENSE) {
+      const T* yr = static_cast<const T*>(labels) + row * C;
       float y[VEC];
-      VecIO<T, VEC>::load(static_cast<const T*>(labels) + row * C + c, y);
+      if constexpr (ANY) stream_load<T, VEC>(yr, c, C, 0, y);
+      else VecIO<T, VEC>::load(yr + c, y);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        acc[0] += (v[e] - shift) * y[e];
+        const float term = (v[e] - shift) * y[e];
+        acc[0] += !ANY || c + e < C ? term : 0.f;
         out[e] = (fast_exp2(fmaf(v[e], kLog2e, -m2)) * inv_sum - y[e]) * scale;
       }
     } else {
@@ -452,7 +533,7 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
         out[e] = p * scale;
       }
     }
-    VecIO<T, VEC>::store(out_row + c, out);
+    put(c, out);
   }
   if (rowloss != nullptr) {
     block_allreduce<SumOp, WG / kWave, 1>(acc, slots, phase);
@@ -537,28 +618,35 @@ struct CrossEntropyOps {
     int tpr, vpt;
   };
 
-  // Thread layout for a row of `chunks` chunks held in registers; false if too wide.
-  static bool pick_shape(int64_t chunks, bool wide, Shape* s) {
-    // Rows of up to 80 unaligned elements (a 65-symbol vocabulary): sixteen lanes per row, four
-    // rows per wave; one wave per row left most lanes idle and a latency per 130 bytes.
-    if (!wide && chunks <= 80 && env_int("MOGRAD_HIP_CE_NARROW", 1) != 0) *s = {16, 5};
+  // Rows of more chunks than these are streamed twice.  With dense labels, 32 chunks of two tensors a thread are more than
+  // registers hold well: (8192, 50304) bf16 683 us held | 475 streamed, fp32 1300 | 1000, (4096, 40000) bf16 288 | 195.
+  template <bool DENSE>
+  static constexpr int64_t kMostChunks = !DENSE ? 16384 : WIDE == 8 ? 4096 : 8192;
+
+  // Thread layout for a row of `chunks` chunks held in registers; false if too wide.  Up to 32 chunks: sixteen lanes per row,
+  // four rows per wave, as one wave per row left most lanes idle ((16384, 65) bf16 12.9 us | 9.4, (16384, 128) 12.5 | 9.5,
+  // (16384, 129) 13.5 | 10.3).
+  static bool pick_shape(int64_t chunks, Shape* s) {
+    const bool narrow = env_int("MOGRAD_HIP_CE_NARROW", 1) != 0;
+    if (narrow && chunks <= 16) *s = {16, 1};
+    else if (narrow && chunks <= 32) *s = {16, 2};
     else if (chunks <= 64) *s = {64, 1};
     else if (chunks <= 128) *s = {64, 2};
     else if (chunks <= 256) *s = {64, 4};
     else if (chunks <= 1024) *s = {256, 4};
     else if (chunks <= 2048) *s = {512, 4};
     else if (chunks <= 4096) *s = {512, 8};
-    else if (WIDE == 8 && wide && chunks <= 6400) *s = {256, 25};  // 16-bit rows up to 51200 columns: see below
+    else if (WIDE == 8 && chunks <= 6400) *s = {256, 25};  // 16-bit rows up to 51200 columns: see below
     else if (chunks <= 8192) *s = {512, 16};
-    else if (WIDE == 4 && wide && chunks <= 12800) *s = {256, 50};
-    else if (wide && chunks <= 16384) *s = {1024, 16};
+    else if (WIDE == 4 && chunks <= 12800) *s = {256, 50};
+    else if (chunks <= 16384) *s = {1024, 16};
     else return false;
     // Rows of about 50k columns (8193..12800 fp32 chunks, 4097..6400 16-bit chunks: 200
     // values per thread either way): 256 threads x 50 (fp32) or x 25 (16-bit) chunks by
     // default, which leaves room for two workgroups per CU so that one row's arithmetic
     // overlaps the other's memory traffic.  MOGRAD_HIP_CE_WIDE_ROW=512|1024 selects the
     // 512 x 25 or 1024 x 13 layout instead (tuning aid).
-    if (WIDE == 4 && wide && chunks > 8192 && chunks <= 12800) {
+    if (WIDE == 4 && chunks > 8192 && chunks <= 12800) {
       const int pick = env_int("MOGRAD_HIP_CE_WIDE_ROW", 256);
       if (pick == 512) *s = {512, 25};
       if (pick == 1024) *s = {1024, 13};
@@ -577,41 +665,58 @@ struct CrossEntropyOps {
     return static_cast<unsigned>(ceil_div(N, rpw));
   }
 
-  template <int VEC, int TPR, int VPT, bool DENSE>
+  template <int VEC, int TPR, int VPT, bool DENSE, bool ANY>
   static int launch_rows(const T* logits, const void* labels, const T* upstream, float* rowloss, T* dlogits, int64_t N,
                          int64_t C, int id64, hipStream_t stream) {
     constexpr int WG = TPR <= 64 ? 256 : TPR;
-    hipLaunchKernelGGL((ce_rows_kernel<T, VEC, TPR, VPT, WG, DENSE>), dim3(row_grid(N, WG / TPR)), dim3(WG), 0, stream,
+    hipLaunchKernelGGL((ce_rows_kernel<T, VEC, TPR, VPT, WG, DENSE, ANY>), dim3(row_grid(N, WG / TPR)), dim3(WG), 0, stream,
                        logits, labels, upstream, rowloss, dlogits, N, static_cast<int>(C), id64);
     MG_LAUNCH_CHECK();
     return MG_OK;
   }
 
-  template <int VEC, bool DENSE>
+  template <bool DENSE, bool ANY>
   static int dispatch_rows(Shape s, const T* logits, const void* labels, const T* upstream, float* rowloss, T* dlogits,
                            int64_t N, int64_t C, int id64, hipStream_t stream) {
 #define MG_CE_CASE(TPR_, VPT_)        \
   if (s.tpr == TPR_ && s.vpt == VPT_) \
-  return launch_rows<VEC, TPR_, VPT_, DENSE>(logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)
-    MG_CE_CASE(16, 5);
+  return launch_rows<WIDE, TPR_, VPT_, DENSE, ANY>(logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)
+    MG_CE_CASE(16, 1);
+    MG_CE_CASE(16, 2);
     MG_CE_CASE(64, 1);
     MG_CE_CASE(64, 2);
     MG_CE_CASE(64, 4);
     MG_CE_CASE(256, 4);
     MG_CE_CASE(512, 4);
     MG_CE_CASE(512, 8);
-    MG_CE_CASE(512, 16);
-    if constexpr (VEC == 8) {
-      MG_CE_CASE(256, 25);
-    }
-    if constexpr (VEC > 1) {
+    if constexpr (kMostChunks<DENSE> > 4096) MG_CE_CASE(512, 16);
+    if constexpr (!DENSE) MG_CE_CASE(1024, 16);
+    if constexpr (!DENSE && WIDE == 8) MG_CE_CASE(256, 25);
+    if constexpr (!DENSE && WIDE == 4) {
       MG_CE_CASE(256, 50);
       MG_CE_CASE(512, 25);
       MG_CE_CASE(1024, 13);
-      MG_CE_CASE(1024, 16);
     }
 #undef MG_CE_CASE
     return fail(MG_ERR_UNSUPPORTED, "cross_entropy: no kernel for row shape (%d, %d)", s.tpr, s.vpt);
+  }
+
+  // 16-bit rows of more than 512 chunks with integer labels.
+  template <bool ANY>
+  static void launch_packed(int64_t chunks, const T* logits, const void* labels, const T* upstream, float* rowloss, T* dlogits,
+                            int64_t N, int64_t C, int id64, hipStream_t stream) {
+    auto launch = [&](auto kernel, int tpr) {
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(N)), dim3(tpr), 0, stream, logits, labels, upstream, rowloss, dlogits,
+                         N, static_cast<int>(C), id64);
+    };
+    if constexpr (sizeof(T) == 2) {
+      if (chunks <= 1024) launch(ce_rows_packed_kernel<T, 256, 4, ANY>, 256);
+      else if (chunks <= 2048) launch(ce_rows_packed_kernel<T, 256, 8, ANY>, 256);
+      else if (chunks <= 4096) launch(ce_rows_packed_kernel<T, 256, 16, ANY>, 256);
+      else if (chunks <= 6400) launch(ce_rows_packed_kernel<T, 256, 25, ANY>, 256);
+      else if (chunks <= 12800) launch(ce_rows_packed_kernel<T, 512, 25, ANY>, 512);
+      else launch(ce_rows_packed_kernel<T, 1024, 16, ANY>, 1024);
+    }
   }
 
   static int finish_loss(const float* rowloss, T* loss, int64_t N, hipStream_t stream) {
@@ -639,6 +744,9 @@ struct CrossEntropyOps {
       rowloss = rowloss_buf.as<float>();
     }
     const bool wide = can_vectorise(C, {logits, DENSE ? labels : nullptr, dlogits});
+    // Rows off the 16-byte chunks, of one chunk and more: misaligned chunks instead of an element at a time ((8192, 50257) bf16
+    // 480 us | 361, fp32 779 | 620; (16384, 8191) bf16 288 | 114, 4099 148 | 53, 2001 62 | 30, 333 27 | 14; fp32 257 26 | 15).
+    const bool any = !wide && C >= WIDE;
     constexpr int SWG = 1024;
     if (dlogits == nullptr) {
       // larger than the 256 MB memory-side cache: read once, past the caches
@@ -649,6 +757,9 @@ struct CrossEntropyOps {
       else if (wide)
         hipLaunchKernelGGL((ce_fwd_stream_kernel<T, WIDE, SWG, DENSE>), dim3(static_cast<unsigned>(N)), dim3(SWG), 0,
                            stream, logits, labels, rowloss, N, C, id64);
+      else if (any)
+        hipLaunchKernelGGL((ce_fwd_stream_kernel<T, WIDE, 256, DENSE, false, true>), dim3(static_cast<unsigned>(N)), dim3(256),
+                           0, stream, logits, labels, rowloss, N, C, id64);
       else
         hipLaunchKernelGGL((ce_fwd_stream_kernel<T, 1, 256, DENSE>), dim3(static_cast<unsigned>(N)), dim3(256), 0,
                            stream, logits, labels, rowloss, N, C, id64);
@@ -656,48 +767,31 @@ struct CrossEntropyOps {
       return finish_loss(rowloss, loss, N, stream);
     }
     Shape s;
+    const int64_t chunks = ceil_div(C, WIDE);
     if constexpr (sizeof(T) == 2 && !DENSE) {
       // 16-bit rows of more than 512 chunks (4096 columns) with integer labels: the packed row
       // kernel ((8192, 50304) bf16 1220 -> 344 us, (16384, 16392) 415 -> 209 us, (65536, 4104)
       // 275 -> 205 us, (32768, 8192) 197 us either way).  MOGRAD_HIP_CE_PACKED=0: the fp32 tiles.
-      const int64_t chunks = C / WIDE;
-      if (wide && chunks > 512 && chunks <= 16384 && dlogits != nullptr && env_int("MOGRAD_HIP_CE_PACKED", 1) != 0) {
-        const unsigned grid = static_cast<unsigned>(N);
-        const int Ci = static_cast<int>(C);
-        if (chunks <= 1024)
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 256, 4>), dim3(grid), dim3(256), 0, stream, logits, labels, upstream,
-                             rowloss, dlogits, N, Ci, id64);
-        else if (chunks <= 2048)
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 256, 8>), dim3(grid), dim3(256), 0, stream, logits, labels, upstream,
-                             rowloss, dlogits, N, Ci, id64);
-        else if (chunks <= 4096)
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 256, 16>), dim3(grid), dim3(256), 0, stream, logits, labels, upstream,
-                             rowloss, dlogits, N, Ci, id64);
-        else if (chunks <= 6400)
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 256, 25>), dim3(grid), dim3(256), 0, stream, logits, labels, upstream,
-                             rowloss, dlogits, N, Ci, id64);
-        else if (chunks <= 12800)
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 512, 25>), dim3(grid), dim3(512), 0, stream, logits, labels, upstream,
-                             rowloss, dlogits, N, Ci, id64);
-        else
-          hipLaunchKernelGGL((ce_rows_packed_kernel<T, 1024, 16>), dim3(grid), dim3(1024), 0, stream, logits, labels,
-                             upstream, rowloss, dlogits, N, Ci, id64);
+      if ((wide || any) && chunks > 512 && chunks <= 16384 && env_int("MOGRAD_HIP_CE_PACKED", 1) != 0) {
+        if (wide) launch_packed<false>(chunks, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream);
+        else launch_packed<true>(chunks, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream);
         MG_LAUNCH_CHECK();
         if (loss != nullptr) return finish_loss(rowloss, loss, N, stream);
         return MG_OK;
       }
     }
-    if (wide && pick_shape(C / WIDE, true, &s)) {
-      MG_TRY((dispatch_rows<WIDE, DENSE>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
-    } else if (!wide && pick_shape(C, false, &s)) {
-      MG_TRY((dispatch_rows<1, DENSE>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
+    if (C < WIDE) {
+      MG_TRY((launch_rows<1, 16, 1, DENSE, false>(logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
+    } else if (chunks <= kMostChunks<DENSE> && pick_shape(chunks, &s)) {
+      if (wide) MG_TRY((dispatch_rows<DENSE, false>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
+      else MG_TRY((dispatch_rows<DENSE, true>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
     } else {
-      if (wide)
-        hipLaunchKernelGGL((ce_grad_stream_kernel<T, WIDE, SWG, DENSE>), dim3(static_cast<unsigned>(N)), dim3(SWG), 0,
-                           stream, logits, labels, upstream, rowloss, dlogits, N, C, id64);
-      else
-        hipLaunchKernelGGL((ce_grad_stream_kernel<T, 1, SWG, DENSE>), dim3(static_cast<unsigned>(N)), dim3(SWG), 0,
-                           stream, logits, labels, upstream, rowloss, dlogits, N, C, id64);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(N)), dim3(SWG), 0, stream, logits, labels, upstream, rowloss,
+                           dlogits, N, C, id64);
+      };
+      if (wide) launch(ce_grad_stream_kernel<T, WIDE, SWG, DENSE>);
+      else launch(ce_grad_stream_kernel<T, WIDE, SWG, DENSE, true>);
       MG_LAUNCH_CHECK();
     }
     if (loss != nullptr) return finish_loss(rowloss, loss, N, stream);

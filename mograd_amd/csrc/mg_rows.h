@@ -39,24 +39,34 @@ struct VecAny {
     const uint32_t w[4] = {r[0], r[1], r[2], r[3]};
     unpack(w, v);
   }
-  // The elements of the row from column c on, zeros past its end, with one load and no branch: the last sixteen bytes of
-  // the row where the chunk reaches past it, moved down.  (Element by element under conditions the row waited for each:
+  // The elements of the row from column c on, `fill` (words of it) past its end, with one load and no branch: the last sixteen
+  // bytes of the row where the chunk reaches past it, moved down.  (Element by element under conditions the row waited for each:
   // (100, 333) forward and backward 10.5 us against 13.0.)  Needs cols >= VEC.
-  static __device__ __forceinline__ void load_end(const T* p, int c, int cols, float (&v)[VEC]) {
-    const int past = max(c + VEC - cols, 0);  // elements of the chunk past the row
+  // `past`: how many elements of the chunk at `p` are past the row.
+  static __device__ __forceinline__ void words_end(const T* p, int past, uint32_t fill, uint32_t (&w)[4]) {
     const mg_u4_any r = *reinterpret_cast<const mg_u4_any*>(p - past);
-    uint32_t w[4] = {r[0], r[1], r[2], r[3]};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = r[i];
     const int words = past / PER_WORD;
     if constexpr (PER_WORD == 2) {
       const bool odd = past & 1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = odd ? w[i] >> 16 | (i < 3 ? w[i + 1] << 16 : 0u) : w[i];
+      for (int i = 0; i < 4; ++i) w[i] = odd ? w[i] >> 16 | (i < 3 ? w[i + 1] : fill) << 16 : w[i];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = words & 2 ? (i < 2 ? w[i + 2] : 0u) : w[i];
+    for (int i = 0; i < 4; ++i) w[i] = words & 2 ? (i < 2 ? w[i + 2] : fill) : w[i];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = words & 1 ? (i < 3 ? w[i + 1] : 0u) : w[i];
+    for (int i = 0; i < 4; ++i) w[i] = words & 1 ? (i < 3 ? w[i + 1] : fill) : w[i];
+  }
+  static __device__ __forceinline__ void load_end(const T* p, int c, int cols, uint32_t fill, float (&v)[VEC]) {
+    uint32_t w[4];
+    words_end(p, max(c + VEC - cols, 0), fill, w);
     unpack(w, v);
+  }
+  static __device__ __forceinline__ void store(T* p, const float (&v)[VEC]) {
+    uint32_t w[4];
+    pack(v, w);
+    *reinterpret_cast<mg_u4_any*>(p) = mg_u4_any{w[0], w[1], w[2], w[3]};
   }
   static __device__ __forceinline__ void store_stream(T* p, const float (&v)[VEC]) {
     uint32_t w[4];
@@ -106,10 +116,18 @@ struct RowTile {
     if constexpr (ANY) VecAny<T, VEC>::load(p, out);
     else VecIO<T, VEC>::load(p, out);
   }
-  // The chunk at `p`, column c of a row, zeros past the row's end.
-  static __device__ __forceinline__ void load_end(const T* p, int c, int cols, float (&out)[VEC]) {
-    if constexpr (ANY) VecAny<T, VEC>::load_end(p, c, cols, out);
+  // The chunk at `p`, column c of a row, `fill` past the row's end.
+  static __device__ __forceinline__ void load_end(const T* p, int c, int cols, float (&out)[VEC], uint32_t fill = 0) {
+    if constexpr (ANY) VecAny<T, VEC>::load_end(p, c, cols, fill, out);
     else VecIO<T, VEC>::load(p, out);
+  }
+  static __device__ __forceinline__ void store_chunk(T* p, const float (&out)[VEC]) {
+    if constexpr (ANY) VecAny<T, VEC>::store(p, out);
+    else VecIO<T, VEC>::store(p, out);
+  }
+  static __device__ __forceinline__ void store_end(T* p, int c, int cols, const float (&out)[VEC]) {
+    if (!ANY || c + VEC <= cols) store_chunk(p, out);
+    else if constexpr (ANY) VecAny<T, VEC>::store_first(p, cols % VEC, out);
   }
   static __device__ __forceinline__ void store_end_stream(T* p, int c, int cols, const float (&out)[VEC]) {
     if constexpr (!ANY) {
@@ -123,7 +141,8 @@ struct RowTile {
   // Whether element e of the chunk at column c is one of the row's.
   static __device__ __forceinline__ bool in_row(int c, int e, int cols) { return ANY ? c + e < cols : c < cols; }
 
-  __device__ __forceinline__ void load(const T* row_ptr, int t, int cols) {
+  // `fill`: the word that stands past the end of a row that ends inside a chunk (ANY); absent chunks are zeros.
+  __device__ __forceinline__ void load(const T* row_ptr, int t, int cols, uint32_t fill = 0) {
     const unsigned lane_off = static_cast<unsigned>(t) * VEC;
     const int nfull = full_chunks(cols);
 #pragma unroll
@@ -134,22 +153,18 @@ struct RowTile {
       } else {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[i][e] = 0.f;
-        if (i == nfull && col(i, t) < cols) load_end(chunk_base + lane_off, col(i, t), cols, v[i]);
+        if (i == nfull && col(i, t) < cols) load_end(chunk_base + lane_off, col(i, t), cols, v[i], fill);
       }
     }
   }
   __device__ __forceinline__ void store(T* row_ptr, int t, int cols) const {
-    static_assert(!ANY, "rows on 16-byte chunks");
     const unsigned lane_off = static_cast<unsigned>(t) * VEC;
     const int nfull = full_chunks(cols);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       T* chunk_base = row_ptr + i * (TPR * VEC);
-      if (i < nfull) {
-        VecIO<T, VEC>::store(chunk_base + lane_off, v[i]);
-      } else if (i == nfull && col(i, t) < cols) {
-        VecIO<T, VEC>::store(chunk_base + lane_off, v[i]);
-      }
+      if (i < nfull) store_chunk(chunk_base + lane_off, v[i]);
+      else if (i == nfull && col(i, t) < cols) store_end(chunk_base + lane_off, col(i, t), cols, v[i]);
     }
   }
   // The same with stores that bypass the caches (see VecIO::store_stream).

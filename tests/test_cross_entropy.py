@@ -245,6 +245,50 @@ def test_wide_16bit_rows_stay_packed(device, monkeypatch, dtype, rtol, N, Cc):
     assert got["1"][2] == got["0"][2]
 
 
+@pytest.mark.parametrize("dtype,half_ulp,size", [(F32, 2.0 ** -24, 4), (F16, 2.0 ** -11, 2), (BF16, 2.0 ** -8, 2)])
+@pytest.mark.parametrize("N,Cc,start", [(5, 3, 1), (6, 4, 1), (7, 8, 3), (5, 9, 0), (9, 31, 1), (5, 64, 1), (6, 65, 0), (5, 127, 0), (3, 129, 1),
+                                        (4, 257, 0), (3, 513, 1), (3, 1001, 0), (2, 2049, 1), (2, 4095, 0), (2, 4099, 3), (2, 8193, 0),
+                                        (2, 16386, 1), (2, 32769, 0), (2, 40002, 1), (1, 51207, 0), (2, 65539, 1), (1, 102403, 0),
+                                        (1, 131079, 1)])
+def test_rows_off_the_16_byte_chunks(device, dtype, half_ulp, size, N, Cc, start):
+    # Rows of any width at any element: every layout of a row's threads, a last chunk of one element, of all but one, whole.
+    # A result is rounded once; what is computed in fp32 (logits of up to ten, their exponentials, sums) is off by 2^-18 of its
+    # terms at most, fp16 below 2^-14 by 2^-25.
+    lib, st = device.lib, device.stream
+    x = round_to_dtype(normal(36, 0, (N, Cc), std=2.0), dtype)
+    ids = integers(36, 1, (N,), 0, Cc)
+    ids[0] = Cc - 1
+    dense = round_to_dtype(0.9 * O.one_hot(ids, Cc) + 0.1 / Cc, dtype)
+
+    def put(a, fill):  # `start` elements in, 64 behind
+        flat = np.full(a.size + start + 64, fill, np.float32)
+        flat[start : start + a.size] = a.reshape(-1)
+        return AnyBuffer.from_numpy(device, flat, dtype)
+
+    bx, by = put(x, 60000.0), put(dense, 7.0)
+    bi = AnyBuffer.from_numpy(device, ids.astype(np.int32), I32)
+    bu = AnyBuffer.from_numpy(device, np.array([2.0], np.float32), dtype)
+    at = lambda b: C.c_void_p(b.data_ptr().value + start * size)
+    e = np.exp(x.astype(np.float64) - x.max(-1, keepdims=True))
+    p = e / e.sum(-1, keepdims=True)
+    logp = np.log(p)
+    for y, ptr, call, loss_call, extra in ((O.one_hot(ids, Cc), bi.data_ptr(), lib.mg_cross_entropy_fused_ids, lib.mg_cross_entropy_ids, (I32,)),
+                                           (dense, at(by), lib.mg_cross_entropy_fused, lib.mg_cross_entropy, ())):
+        y = y.astype(np.float64)
+        loss, alone, out = AnyBuffer.create(dtype, device, 1), AnyBuffer.create(dtype, device, 1), put(np.zeros((N, Cc)), 7.0)
+        call(at(bx), ptr, bu.data_ptr(), loss.data_ptr(), at(out), N, Cc, dtype, *extra, st)
+        loss_call(at(bx), ptr, alone.data_ptr(), N, Cc, dtype, *extra, st)
+        want = -(y * logp).sum() / N
+        terms = (y * (np.abs(x) + np.abs(x - logp))).sum() / N
+        for got in (loss.item(), alone.item()):
+            assert abs(got - want) <= 1.02 * half_ulp * abs(want) + 2.0 ** -18 * terms
+        flat = out.to_numpy()
+        assert (flat[:start] == 7.0).all() and (flat[start + N * Cc :] == 7.0).all()
+        grad, scale = (p - y) * 2.0 / N, 2.0 / N
+        bound = 1.02 * half_ulp * np.abs(grad) + 2.0 ** -18 * (p + y) * scale + (2.0 ** -25 if dtype == F16 else 0.0)
+        assert (np.abs(flat[start : start + N * Cc].reshape(N, Cc) - grad) <= bound).all()
+
+
 def test_out_of_range_id_flags_loss(device):
     x = normal(34, 0, (4, 100))
     ids = np.array([0, 5, 100, 7], np.int32)
