@@ -597,12 +597,20 @@ __global__ __launch_bounds__(WG) void ce_strided_kernel(const T* __restrict__ lo
   }
 }
 
-// loss[0] = sum of the N per-row terms, one workgroup, fixed order (no atomics).
+// loss[0] = sum of the N per-row terms, one workgroup, fixed order (no atomics).  It waits for memory, so sixteen terms are in
+// flight to a thread (one after the other, 16384 rows took 5.7 us; so 4.7, of which a launch of one workgroup is half).
 template <typename T>
 __global__ __launch_bounds__(1024) void sum_rows_kernel(const float* __restrict__ rowloss, T* __restrict__ loss, int64_t N) {
   __shared__ float slots[2 * 16];
   float acc[1] = {0.f};
-  for (int64_t i = threadIdx.x; i < N; i += 1024) acc[0] += rowloss[i];
+  constexpr int U = 16;
+  for (int64_t i = threadIdx.x; i < N; i += U * 1024) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = i + u * 1024 < N ? rowloss[i + u * 1024] : 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[0] += v[u];
+  }
   block_allreduce<SumOp, 16, 1>(acc, slots, 0);
   if (threadIdx.x == 0) loss[0] = from_float<T>(acc[0]);
 }
