@@ -2024,6 +2024,9 @@ int attn_bwd_wave16(const void* d_o, const void* o, const void* q, const void* k
 //     loads the 128-row kernel waits for, twice as many where the walk is long: (8, 2000), 504 93.6 | 58.0, (72, 130), 360 14.4 | 16.7
 //   backward, 64: (3, 2000), 189 34.6 | 26.7; (11, 777), causal, 275 21.3 | 15.8; (7, 1200), 266 26.2 | 26.9; (14, 1200), causal, 532
 //     27.9 | 29.3; 32 columns: (24, 777), causal, 600 21.8 | 17.3, (36, 777), 900 30.4 | 32.4
+//   backward, two tiles a head, which the other kernels walk in one step (64 columns without a bias: hold whole): while both walks'
+//     workgroups have a CU each; D128, bias, (40, 36) 12.8 | 9.2, (84, 36) 13.3 | 16.8; full (84, 36) 11.8 | 15.0; D64 full (96, 64)
+//     6.8 | 7.2; one tile: D128 full (240, 32) 20.2 | 13.8
 //   backward, 80 and 128: (5, 1200), causal, 190 54.9 | 24.9; (24, 300), 240 21.1 | 18.9; (72, 80), 216 15.8 | 16.3; (48, 300), 480
 //     34.0 | 35.5; long causal walks to half as many again: (6, 2000), 378 88.6 | 54.5
 // MOGRAD_HIP_ATTN_WAVE16 = 0 | 1 overrides the choice where either can be had.
@@ -2041,6 +2044,7 @@ static bool attn_wave16_ok(const AttnDims& a, bool causal, bool has_bias, bool b
     return a.S > 64 && tiles <= (a.D <= 64 ? 2 : 1) * cus;
   }
   if (a.D <= 32) return 2 * tiles <= 5 * cus;
+  if (a.S > 32 && a.S <= 64) return 2 * tiles <= cus;
   return a.D > 64 && causal && a.S >= 1024 ? 2 * tiles <= 3 * cus : tiles <= cus;
 }
 
