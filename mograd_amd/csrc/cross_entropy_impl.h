@@ -604,10 +604,14 @@ __global__ __launch_bounds__(1024) void sum_rows_kernel(const float* __restrict_
   __shared__ float slots[2 * 16];
   float acc[1] = {0.f};
   constexpr int U = 16;
-  for (int64_t i = threadIdx.x; i < N; i += U * 1024) {
+  for (int64_t first = 0; first < N; first += U * 1024) {
     float v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = i + u * 1024 < N ? rowloss[i + u * 1024] : 0.f;
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = first + u * 1024 + threadIdx.x;
+      v[u] = 0.f;
+      if (first + u * 1024 < N && i < N) v[u] = rowloss[i];  // the first condition is the workgroup's: few rows branch past the rest
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) acc[0] += v[u];
   }
@@ -629,7 +633,7 @@ struct CrossEntropyOps {
   // Rows of more chunks than these are streamed twice.  With dense labels, 32 chunks of two tensors a thread are more than
   // registers hold well: (8192, 50304) bf16 683 us held | 475 streamed, fp32 1300 | 1000, (4096, 40000) bf16 288 | 195.
   template <bool DENSE>
-  static constexpr int64_t kMostChunks = !DENSE ? 16384 : WIDE == 8 ? 4096 : 8192;
+  static constexpr int64_t kMostChunks = !DENSE ? 16384 : 4096;
 
   // Thread layout for a row of `chunks` chunks held in registers; false if too wide.  Up to 32 chunks: sixteen lanes per row,
   // four rows per wave, as one wave per row left most lanes idle ((16384, 65) bf16 12.9 us | 9.4, (16384, 128) 12.5 | 9.5,
