@@ -484,7 +484,10 @@ static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handle
   // (Of the transposing layouts short reductions stay with the ragged variant: (16, 4097 <- 4097) backward 44 | 54.)
   if (!wide && (a_kc ? g.K : g.M) >= 8 && (b_kc ? g.K : g.N) >= 8 && ((a_kc && b_kc) || g.K >= 128) && !env_str("MOGRAD_HIP_GEMM16_PAD") && (pipe == -1 || pipe == 64)) {
     const Choice16 small = small_16bit(g.M, g.N, g.K, g.batch);
-    if (pipe == 64 || 1.35 * small.us <= choose_16bit(g.M, g.N, g.K, g.batch, false).us + 7.0) {
+    // (Up to three tiles to a CU: (700, 4400 <- 77) 8.8 | 8.3, 759 tiles; (1000, 4000 <- 141) 10.0 | 10.8, 1008; (966, 5920 <- 141)
+    // 12.5 | 15.8, 1488.)
+    const bool few = g.batch * ceil_div(g.M, 64) * ceil_div(g.N, 64) <= 3 * static_cast<int64_t>(device_info().cu_count);
+    if (pipe == 64 || (few && 1.35 * small.us <= choose_16bit(g.M, g.N, g.K, g.batch, false).us + 7.0)) {
       if (a_kc && b_kc) return launch_16bit_small<T, true, true, true>(g, small.splits, stream);
       if (a_kc) return launch_16bit_small<T, true, false, true>(g, small.splits, stream);
       if (b_kc) return launch_16bit_small<T, false, true, true>(g, small.splits, stream);
@@ -720,10 +723,15 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const int64_t cus = device_info().cu_count;
   const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr, db != nullptr);
   if (choice.tile < 0) return MG_OK;
-  // (64 x 64 tiles read arrays that are at least 8 wide from wherever they start, a step a third slower, which up to some 15 us
-  // costs less than the copies: (700, 701 <- 703) 16.8 us with them, 12.7; (1999, 1001 <- 768) 24.5, 25.2; (300, 3001 <- 517)
-  // 26.2, 31.0)
-  const bool any = choice.tile == kSmall && (pad_n || pad_k) && N >= 8 && K >= 8 && choice.us <= 15.0 && !env_str("MOGRAD_HIP_GEMM16_PAD");
+  // 64 x 64 tiles read arrays that are at least 8 wide from wherever they start.  That saves the copies, a launch of 2.4 us and
+  // their bytes, and makes a step of dX's walk over N 0.1 us longer, 0.2 where its last tile of columns is cut off: with the
+  // copies | without, (64, 1001 <- 192) 10.5 | 9.6, (64, 2601 <- 192) 16.4 | 18.1, (64, 1001 <- 200) 10.7 | 11.2, (64, 2601 <- 200)
+  // 16.5 | 22.1; (406, 1832 <- 83) 15.3 | 18.4, (675, 149 <- 2391) 18.4 | 14.0, (700, 701 <- 703) 16.8 | 12.7.  Longer products are
+  // faster with the copies ((1999, 1001 <- 768) 24.5 | 25.2; (300, 3001 <- 517) 26.2 | 31.0).
+  const double longer = !dx ? 0.0 : (K % 64 == 0 ? 0.1 : 0.2) * static_cast<double>(ceil_div(N, 64));
+  const double copied = (pad_n ? static_cast<double>(M) * N : 0.0) + (pad_k ? static_cast<double>(K) * (dx ? M + N : M) : 0.0);
+  const bool any = choice.tile == kSmall && (pad_n || pad_k) && N >= 8 && K >= 8 && choice.us <= 15.0 &&
+                   longer <= 2.4 + 4.0 * copied / 3.7e6 && !env_str("MOGRAD_HIP_GEMM16_PAD");
   const bool small = choice.tile == kSmall, wide = choice.tile == kTileWide;
   if (ln && (!wide || relu_mask || pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx))) return MG_OK;
   // (without the LayerNorm the same K ranges in 128 x 192 tiles, two workgroups per CU)
