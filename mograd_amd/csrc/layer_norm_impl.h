@@ -430,8 +430,16 @@ struct LayerNormOps {
   // Rows that do not lie on 16-byte chunks are read and written in misaligned ones (RowTile's ANY): what they cost element by
   // element was 317 / 64 loads of two bytes per lane and row, and rows past 4096 columns had no backward at all.  Forward +
   // backward, us: (23721, 317) fp16 100 -> 33, fp32 66 -> 38; (9000, 4095) bf16 199 -> 97; (1000, 799) fp16 16.2 -> 15.8.
-  // Up to this many columns stay with an element per thread: of a row of a few chunks most of its sixteen lanes are idle.
-  static constexpr int kNarrow = 64;
+  // Few rows stay with an element per thread, whose walk over a row is shorter where each has a workgroup to itself, and so do
+  // rows of up to 64 columns, of whose sixteen lanes most would be idle; us, by elements | in chunks: fp16 (193, 554) 11.0 | 13.1,
+  // (193, 1501) 13.0 | 16.9, (600, 2503) 22.1 | 25.2, (2000, 301) 15.5 | 16.7; (2000, 554) 18.8 | 18.2, (2000, 2503) 44.1 | 37.1; fp32
+  // (193, 777) 10.4 | 13.0, (2000, 301) 14.3 | 15.8, (2000, 777) 19.3 | 18.6.  (By elements there is no backward past 4096 columns.)
+  // MOGRAD_HIP_LN_CHUNKS = 0 | 1 overrides the choice where either can be had.
+  static bool in_chunks(int64_t rows, int64_t cols) {
+    if (cols > 4096) return true;
+    if (const char* const force = env_str("MOGRAD_HIP_LN_CHUNKS")) return force[0] != '0' && cols >= WIDE;
+    return cols > 64 && rows >= 1024 && rows * cols >= int64_t{1} << 20;
+  }
 
   // How a row of `chunks` chunks is laid over threads.
   struct Shape {
@@ -492,7 +500,7 @@ struct LayerNormOps {
   static int dispatch_fwd(Shape s, const T* x, const T* gamma, const T* beta, T* y, float* mean, float* rstd,
                           int64_t rows, int64_t cols, float eps, hipStream_t stream) {
 #define MG_LN_FWD_CASE(TPR_, VPT_)             \
-  if constexpr (VEC > 1 || TPR_ * VPT_ <= 64) \
+  if constexpr (VEC > 1 || TPR_ * VPT_ <= 4096) \
   if (s.tpr == TPR_ && s.vpt == VPT_) return launch_fwd<VEC, TPR_, VPT_, ANY>(x, gamma, beta, y, mean, rstd, rows, cols, eps, stream)
     MG_LN_FWD_CASE(16, 1);
     MG_LN_FWD_CASE(16, 2);
@@ -518,9 +526,9 @@ struct LayerNormOps {
     Shape s;
     if (can_vectorise(cols, {x, gamma, beta, y}) && pick_shape(cols / WIDE, &s))
       return dispatch_fwd<WIDE>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
-    if (cols > kNarrow && pick_shape(ceil_div(cols, WIDE), &s))
+    if (in_chunks(rows, cols) && pick_shape(ceil_div(cols, WIDE), &s))
       return dispatch_fwd<WIDE, true>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
-    if (cols <= kNarrow && pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
+    if (!in_chunks(rows, cols) && pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
     hipLaunchKernelGGL((ln_fwd_stream_kernel<T, 1024>), dim3(static_cast<unsigned>(rows)), dim3(1024), 0, stream, x,
                        gamma, beta, y, mean, rstd, rows, cols, eps);
     MG_LAUNCH_CHECK();
@@ -601,7 +609,6 @@ struct LayerNormOps {
                           const T* residual, T* dx, T* dgamma, T* dbeta, int64_t rows, int64_t cols, float eps,
                           hipStream_t stream) {
 #define MG_LN_BWD_CASE(TPR_, VPT_)            \
-  if constexpr (VEC > 1 || TPR_ * VPT_ <= 64) \
   if (s.tpr == TPR_ && s.vpt == VPT_)    \
   return launch_bwd<VEC, TPR_, VPT_, HAS_STATS, ANY>(dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, \
                                                 stream)
@@ -664,10 +671,10 @@ struct LayerNormOps {
     if (can_vectorise(cols, {dy, x, gamma, dx, residual}) && pick_shape_bwd(cols / WIDE, &s) && fits(s, WIDE))
       return dispatch_bwd<WIDE, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
                                            stream);
-    if (cols > kNarrow && pick_shape_bwd(ceil_div(cols, WIDE), &s) && fits(s, WIDE))
+    if (in_chunks(rows, cols) && pick_shape_bwd(ceil_div(cols, WIDE), &s) && fits(s, WIDE))
       return dispatch_bwd<WIDE, HAS_STATS, true>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
                                                  stream);
-    if (cols <= kNarrow && pick_shape_bwd(cols, &s))
+    if (!in_chunks(rows, cols) && pick_shape_bwd(cols, &s) && fits(s, 1))
       return dispatch_bwd<1, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, stream);
     if (residual == nullptr)
       return bwd_stream<HAS_STATS>(dy, x, gamma, mean, rstd, dx, dgamma, dbeta, rows, cols, eps, stream);

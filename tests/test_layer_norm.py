@@ -237,9 +237,11 @@ def test_errors(device):
 @pytest.mark.parametrize("dtype,half_ulp", [(F32, 2.0 ** -24), (F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
 @pytest.mark.parametrize("cols", [1, 63, 65, 66, 71, 130, 255, 317, 1025, 4101, 8191, 16383])
 @pytest.mark.parametrize("offset", [0, 1])
-def test_rows_off_the_16_byte_chunks(device, dtype, half_ulp, cols, offset):
+@pytest.mark.parametrize("chunks", ["1", "0"])
+def test_rows_off_the_16_byte_chunks(device, monkeypatch, dtype, half_ulp, cols, offset, chunks):
     # Rows whose last chunk is any part of one, from any element on, in every layout; the elements around the outputs stay
     # as they are.  Sums of fp32 terms against float64 ones: 2^-20 of the terms' magnitudes, then one rounding.
+    monkeypatch.setenv("MOGRAD_HIP_LN_CHUNKS", chunks)
     rows = 37 if cols > 1000 else 5
     x, dy, res = (round_to_dtype(normal(70, i, (rows, cols)) + 0.5, dtype) for i in range(3))
     gamma, beta = (round_to_dtype(normal(70, 4 + i, (cols,)), dtype) for i in range(2))
