@@ -68,19 +68,16 @@ __device__ __forceinline__ float dot_rows(const float (&a)[kAttnMaxDPerLane], co
 
 // The row statistics in the form the pipelined dK/dV walk copies straight into LDS: -lse in
 // log2 units and -delta, each (B*H, s_pad) with s_pad a multiple of 64 and the rows past S
-// holding -inf and 0 (probabilities of rows that do not exist vanish).  `idx` is the row's
-// index in (B,H,S) order; the thread that owns a sequence's last row writes its padding.
+// holding -inf and 0 (probabilities of rows that do not exist vanish).  The thread that owns a sequence's last row writes its
+// padding.
 struct AttnPaddedStats {
   const float* lse = nullptr;
   float* nlse = nullptr;    // null: not wanted
   float* ndelta = nullptr;
   int s_pad = 0;
 };
-__device__ __forceinline__ void write_padded_stats(const AttnPaddedStats& ps, int64_t idx, int S, float delta) {
-  if (ps.nlse == nullptr) return;
-  const int64_t bh = idx / S;
-  const int s = static_cast<int>(idx - bh * S);
-  ps.nlse[bh * ps.s_pad + s] = -ps.lse[idx] * kAttnLog2e;
+__device__ __forceinline__ void write_padded_stats(const AttnPaddedStats& ps, int64_t bh, int s, int S, float lse, float delta) {
+  ps.nlse[bh * ps.s_pad + s] = -lse * kAttnLog2e;
   ps.ndelta[bh * ps.s_pad + s] = -delta;
   if (s == S - 1)
     for (int t = S; t < ps.s_pad; ++t) {
@@ -103,7 +100,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const T* __restrict__ d
   if (lane == 0) {
     const int64_t idx = o_row_to_bhs(row, S, H, o_bshd);
     delta[idx] = acc;
-    write_padded_stats(ps, idx, S, acc);
+    if (ps.nlse != nullptr) write_padded_stats(ps, idx / S, static_cast<int>(idx % S), S, ps.lse[idx], acc);
   }
 }
 
