@@ -4,12 +4,13 @@
 // Layout in HBM: logits, dense labels and dlogits are row-major (N, C); integer labels
 // are (N) int32 or int64; per-row losses are (N) fp32 scratch; loss is one element of T.
 //
-// Gradient and fused kernels hold a whole row of logits in registers (chunks of VEC
-// elements dealt round-robin to the TPR threads that share the row), so the logits are
-// read from HBM once and dlogits written once.  The loss-only kernel streams the row
-// once with an online softmax and keeps nothing.
+// Gradient and fused kernels hold a row of logits in registers (chunks of VEC elements dealt
+// round-robin to the TPR threads that share the row), so the logits are read from HBM once
+// and dlogits written once; rows of more than kMostChunks chunks are streamed twice, the first time
+// with an online softmax.  The loss-only kernel streams the row once that way and keeps nothing.
 #pragma once
 
+#include <cfloat>
 #include <cstdlib>
 
 #include "mg_device.h"
@@ -328,6 +329,11 @@ __device__ __forceinline__ void stream_load(const T* row, int64_t c, int64_t C, 
   VecAny<T, VEC>::unpack(w, v);
 }
 
+// What an online sum of exponentials subtracts, in log2 units: the maximum so far, but no less than the least float, so that
+// classes masked with -inf or with the type's lowest value, where a thread has seen nothing else yet, add zeros (from minus
+// infinity they would be NaN, which no later maximum takes out of the sum).
+__device__ __forceinline__ float online_reference(float m) { return fmaxf(m * kLog2e, -FLT_MAX); }
+
 // Online (max, sum-exp) over the elements a thread visits, merged across the workgroup.  ONCE: the
 // row is not read again by this kernel, so its loads go past the caches.
 template <typename T, int VEC, int WG, bool ONCE = false, bool ANY = false>
@@ -356,7 +362,7 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);  // exp2(-inf) == 0 on the first chunk
       m = cm;
     }
-    const float m2 = m * kLog2e;
+    const float m2 = online_reference(m);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -373,7 +379,7 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);
       m = cm;
     }
-    const float m2 = m * kLog2e;
+    const float m2 = online_reference(m);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) s += fast_exp2(fmaf(v[e], kLog2e, -m2));
   }
@@ -427,7 +433,7 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
         ts *= fast_exp2((tm - cm) * kLog2e);
         tm = cm;
       }
-      const float m2 = tm * kLog2e;
+      const float m2 = online_reference(tm);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         ts += fast_exp2(fmaf(v[e], kLog2e, -m2));

@@ -289,6 +289,59 @@ def test_rows_off_the_16_byte_chunks(device, dtype, half_ulp, size, N, Cc, start
         assert (np.abs(flat[start : start + N * Cc].reshape(N, Cc) - grad) <= bound).all()
 
 
+@pytest.mark.parametrize("dtype,half_ulp,size,vec", [(F32, 2.0 ** -24, 4, 4), (F16, 2.0 ** -11, 2, 8), (BF16, 2.0 ** -8, 2, 8)])
+@pytest.mark.parametrize("mask", ["-inf", "lowest"])
+@pytest.mark.parametrize("seen", ["last quarter", "one", "every second group"])
+@pytest.mark.parametrize("Cc,start", [(9000, 0), (16384, 0), (20000, 0), (20001, 1), (40000, 0), (40000, 1), (70000, 0), (70001, 0), (140001, 1)])
+def test_masked_classes(device, dtype, half_ulp, size, vec, mask, seen, Cc, start):
+    # Classes at -inf or at the type's lowest value: whole groups of a thread's chunks, its first ones among them, in rows that
+    # are held and in rows that are streamed.  Bounds as above; a masked class has no weight.
+    lib, st, N = device.lib, device.stream, 2
+    x = round_to_dtype(normal(37, 0, (N, Cc), std=2.0), dtype)
+    cols = np.arange(Cc)
+    visible = {"last quarter": cols >= Cc - Cc // 4, "one": cols == Cc - 5, "every second group": cols // (1024 * vec) % 2 == 1}[seen]
+    if not visible.any():
+        visible[Cc // 2 :] = True
+    low = {F32: -np.finfo(np.float32).max, F16: -65504.0, BF16: -float(np.uint32(0x7F7F0000).view(np.float32))}[dtype]
+    x[:, ~visible] = -np.inf if mask == "-inf" else low
+    ids = np.flatnonzero(visible)[[0, -1]]
+    dense = round_to_dtype(0.9 * O.one_hot(ids, Cc) + 0.1 / Cc, dtype)
+
+    def put(a):
+        return AnyBuffer.from_numpy(device, np.concatenate([np.zeros(start, np.float32), a.reshape(-1).astype(np.float32)]), dtype)
+
+    bx, by, bi = put(x), put(dense), AnyBuffer.from_numpy(device, ids.astype(np.int32), I32)
+    bu = AnyBuffer.from_numpy(device, np.array([2.0], np.float32), dtype)
+    at = lambda b: C.c_void_p(b.data_ptr().value + start * size)
+    x = x.astype(np.float64)
+    top = x.max(-1, keepdims=True)
+    e = np.exp(x - top)
+    p = e / e.sum(-1, keepdims=True)
+    lse = top + np.log(e.sum(-1, keepdims=True))
+    logp = x - lse
+    for y, ptr, calls, extra in ((O.one_hot(ids, Cc), bi.data_ptr(), (lib.mg_cross_entropy_fused_ids, lib.mg_cross_entropy_grad_ids, lib.mg_cross_entropy_ids), (I32,)),
+                                 (dense, at(by), (lib.mg_cross_entropy_fused, lib.mg_cross_entropy_grad, lib.mg_cross_entropy), ())):
+        y = y.astype(np.float64)
+        fused, grad, alone = calls
+        loss, loss2, out, out2 = (AnyBuffer.create(dtype, device, 1), AnyBuffer.create(dtype, device, 1), put(np.zeros((N, Cc))), put(np.zeros((N, Cc))))
+        fused(at(bx), ptr, bu.data_ptr(), loss.data_ptr(), at(out), N, Cc, dtype, *extra, st)
+        grad(at(bx), ptr, bu.data_ptr(), at(out2), N, Cc, dtype, *extra, st)
+        alone(at(bx), ptr, loss2.data_ptr(), N, Cc, dtype, *extra, st)
+        of = y != 0.0
+        want = -(y[of] * logp[of]).sum() / N
+        # a thread adds up to Cc / 256 terms of one sign one behind the other, each addition off by 2^-24 of their sum
+        off = (2.0 ** -18 + 2.0 ** -24 * Cc / 256) * (y[of] * (np.abs(x[of]) + np.abs(lse).max())).sum() / N
+        for got in (loss.item(), loss2.item()):
+            if not np.isfinite(want) or abs(want) >= 65504.0 and dtype == F16:
+                assert got == np.inf
+            else:
+                assert abs(got - want) <= 1.02 * half_ulp * abs(want) + off, (got, want)
+        exact, scale = (p - y) * 2.0 / N, 2.0 / N
+        bound = 1.02 * half_ulp * np.abs(exact) + 2.0 ** -18 * (p + y) * scale + (2.0 ** -25 if dtype == F16 else 0.0)
+        for got in (out, out2):
+            assert (np.abs(got.to_numpy()[start:].reshape(N, Cc) - exact) <= bound).all()
+
+
 def test_out_of_range_id_flags_loss(device):
     x = normal(34, 0, (4, 100))
     ids = np.array([0, 5, 100, 7], np.int32)
