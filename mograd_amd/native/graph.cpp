@@ -1893,6 +1893,17 @@ const std::pair<const char*, RewriteForm> kRewriteForms[] = {
 };
 PyObject* g_own_rewrites = nullptr;       // the package's own function -> index into kRewriteForms
 PyObject* g_simplifier_type = nullptr;    // rewrites.Simplifier
+// The methods that the rules in Python call, as the package has them: a program may put others in their place on the class.
+struct SimplifierMethod {
+  const char* text;
+  PyObject *name = nullptr, *own = nullptr;
+} g_simplifier_methods[] = {{"single_use"}, {"replace"}, {"consumers_of"}, {"resolve"}};
+bool simplifier_methods_own() {
+  PyObject* const dict = reinterpret_cast<PyTypeObject*>(g_simplifier_type)->tp_dict;
+  for (const SimplifierMethod& m : g_simplifier_methods)
+    if (PyDict_GetItem(dict, m.name) != m.own) return false;
+  return true;
+}
 
 // name -> function of `given`, for every name of `forms`, as function -> place.
 template <class Table>
@@ -1922,6 +1933,13 @@ PyObject* py_set_rewrites(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return PyErr_SetString(PyExc_TypeError, "set_rewrites(Simplifier, functions)"), nullptr;
   PyObject* own = own_functions(kRewriteForms, args[1]);
   if (!own) return nullptr;
+  PyObject* const dict = reinterpret_cast<PyTypeObject*>(args[0])->tp_dict;
+  for (SimplifierMethod& m : g_simplifier_methods) {
+    if (!m.name) m.name = str_(m.text);
+    PyObject* const f = m.name ? PyDict_GetItem(dict, m.name) : nullptr;
+    if (!f) return Py_DECREF(own), PyErr_Format(PyExc_AttributeError, "Simplifier.%s", m.text), nullptr;
+    Py_XSETREF(m.own, new_ref(f));
+  }
   Py_XSETREF(g_own_rewrites, own);
   Py_XSETREF(g_simplifier_type, new_ref(args[0]));
   Py_RETURN_NONE;
@@ -2004,9 +2022,9 @@ PyObject* py_simplify(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (!rules_attr) return nullptr;
   Ref rules(PySequence_Fast(rules_attr.p, "Simplifier.rules"));
   if (!rules) return nullptr;
-  // The package's own rules where the pass is its own Simplifier, with no method of a program's own on it.
+  // The package's own rules where the pass is its own Simplifier, with no method of a program's own on it or on its class.
   PyObject** sim_dict = Py_TYPE(sim) == reinterpret_cast<PyTypeObject*>(g_simplifier_type) ? _PyObject_GetDictPtr(sim) : nullptr;
-  const bool own_pass = sim_dict && *sim_dict && PyDict_GET_SIZE(*sim_dict) == 5;
+  const bool own_pass = sim_dict && *sim_dict && PyDict_GET_SIZE(*sim_dict) == 5 && simplifier_methods_own();
   const Rewriting rewriting{pass};
   struct Compiled {
     Ref pat, func, op;

@@ -509,3 +509,21 @@ def test_a_replaced_gradient_rule_is_the_one_that_runs(host, monkeypatch):
     sim = Simplifier(GPU_REWRITES())
     sim.single_use = lambda node: False
     assert sim.run(relu) is relu
+
+
+@pytest.mark.parametrize("method", ["single_use", "replace", "consumers_of", "resolve"])
+def test_a_method_replaced_on_the_class_is_the_one_that_runs(host, monkeypatch, method):
+    def rewritten():
+        loss, targets = transformer(host)
+        grads = R.gradient(loss, host.leaf(1), targets)
+        return structure(Simplifier(GPU_REWRITES()).run_many([loss] + [g for g in grads if g is not None]))
+
+    own, calls, was = rewritten(), [], getattr(Simplifier, method)
+    with monkeypatch.context() as m:
+        m.setattr(Simplifier, method, lambda *args: (calls.append(args), was(*args))[1])
+        assert rewritten() == own and calls
+        if method == "single_use":
+            m.setattr(Simplifier, method, lambda self, node: False)
+            relu = Node("RELU", Layout(4, 3), F32, [Node("MATMUL_BIAS_BT", Layout(4, 3), F32, [host.leaf(4, 8), host.leaf(3, 8), host.leaf(3)])])
+            assert Simplifier(GPU_REWRITES()).run(relu) is relu
+    assert rewritten() == own
