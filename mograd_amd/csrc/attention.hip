@@ -151,12 +151,19 @@ static int fwd_f32_wave(const float* q, const float* k, const float* v, const fl
   return MG_OK;
 }
 
+// Whether a grid holds both walks of a backward of `blocks` workgroups each: one has fewer than 2^32 threads.  (Heads of 32
+// rows and fewer: 2^23 of them are 1.2 GB a tensor at 8 rows of 4 columns.)  MOGRAD_HIP_ATTN_F32_BWD_TOGETHER overrides it.
+constexpr bool f32_wave_together(int64_t blocks) { return 2 * blocks * 256 < int64_t{1} << 32; }
+static_assert(f32_wave_together((int64_t{1} << 23) - 1) && !f32_wave_together(int64_t{1} << 23) && !f32_wave_together(int64_t{1} << 31),
+              "grids of fewer than 2^32 threads");
+
 static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const float* k, const float* v, const float* mask,
                         const float* lse, float* dq, float* dk, float* dv, const AttnDims& a, float scale, bool causal,
                         bool has_bias, hipStream_t stream) {
   const int tiles = static_cast<int>(ceil_div(a.S, 32));
   const int64_t heads = static_cast<int64_t>(a.B) * a.H;
-  const int blocks = static_cast<int>(f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal)));
+  const int64_t blocks = f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal));
+  const bool together = env_int("MOGRAD_HIP_ATTN_F32_BWD_TOGETHER", f32_wave_together(blocks)) != 0;
   Scratch delta;
   if (a.D > 96 && a.D <= 128) {
     static_assert(f32_wave_delta_given<128>() && !f32_wave_delta_given<96>() && !f32_wave_delta_given<64>(), "who is handed delta");
@@ -166,9 +173,17 @@ static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const 
                        delta.as<float>(), rows, a.D, a.S, a.H, a.o_bshd);
   }
   f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
-    hipLaunchKernelGGL((attn_bwd_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
-                       dim3(2 * static_cast<unsigned>(blocks)), dim3(256), 0, stream, d_o, o, q, k, v, mask, lse,
-                       delta.as<float>(), dq, dk, dv, a, scale, tiles, blocks);
+    auto launch = [&](int64_t grid, int64_t dkdv_blocks) {
+      hipLaunchKernelGGL((attn_bwd_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
+                         dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, d_o, o, q, k, v, mask, lse,
+                         delta.as<float>(), dq, dk, dv, a, scale, tiles, static_cast<int>(dkdv_blocks));
+    };
+    if (together) {
+      launch(2 * blocks, blocks);
+    } else {
+      launch(blocks, blocks);
+      launch(blocks, 0);
+    }
   });
   MG_LAUNCH_CHECK();
   return MG_OK;

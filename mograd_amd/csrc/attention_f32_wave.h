@@ -868,7 +868,8 @@ __device__ __forceinline__ void attn_dkdv_f32_wave_block(
   }
 }
 
-// Both walks in one launch: workgroups [0, blocks) take dK and dV, whose steps are the longer ones, the rest dQ.
+// Both walks in one launch: workgroups [0, blocks) take dK and dV, whose steps are the longer ones, the rest dQ.  A grid of
+// `blocks` is dK and dV alone, one with `blocks` = 0 dQ.
 template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
 __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) void attn_bwd_f32_wave_kernel(
     const float* __restrict__ d_o, const float* __restrict__ o, const float* __restrict__ q, const float* __restrict__ k,
