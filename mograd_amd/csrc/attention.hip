@@ -169,7 +169,7 @@ static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const 
     static_assert(f32_wave_delta_given<128>() && !f32_wave_delta_given<96>() && !f32_wave_delta_given<64>(), "who is handed delta");
     const int64_t rows = heads * a.S;
     MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
-    hipLaunchKernelGGL((attn_delta_kernel<float>), dim3(static_cast<unsigned>(ceil_div(rows, 4))), dim3(256), 0, stream, d_o, o,
+    hipLaunchKernelGGL((attn_delta_kernel<float>), attn_delta_grid(rows), dim3(256), 0, stream, d_o, o,
                        delta.as<float>(), rows, a.D, a.S, a.H, a.o_bshd);
   }
   f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
@@ -277,10 +277,10 @@ static int bwd_generic(const void* d_o, const void* o, const void* q, const void
   }
   Scratch delta;
   MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
-  const dim3 grid(static_cast<unsigned>(ceil_div(rows, 4)));
-  hipLaunchKernelGGL((attn_delta_kernel<T>), grid, dim3(256), 0, stream, static_cast<const T*>(d_o),
+  hipLaunchKernelGGL((attn_delta_kernel<T>), attn_delta_grid(rows), dim3(256), 0, stream, static_cast<const T*>(d_o),
                      static_cast<const T*>(o), delta.as<float>(), rows, a.D, a.S, a.H, a.o_bshd);
   MG_LAUNCH_CHECK();
+  const dim3 grid(static_cast<unsigned>(ceil_div(rows, 4)));
   if (attn_f32_mfma_ok(a)) {
     bwd_f32_mfma_launch<T>(d_o, q, k, v, mask, lse, delta.as<float>(), dq, dk, dv, a, scale, causal, has_bias, stream);
     MG_LAUNCH_CHECK();

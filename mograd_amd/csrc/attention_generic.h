@@ -7,6 +7,8 @@
 // delta are (B, H, S) fp32, LSE in natural-log units.
 #pragma once
 
+#include <algorithm>
+
 #include "mg_device.h"
 #include "mg_internal.h"
 
@@ -86,22 +88,26 @@ __device__ __forceinline__ void write_padded_stats(const AttnPaddedStats& ps, in
     }
 }
 
-// delta[b,h,i] = sum_d dO[b,h,i,d] * O[b,h,i,d]
+// delta[b,h,i] = sum_d dO[b,h,i,d] * O[b,h,i,d], a wave to a row.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_delta_kernel(const T* __restrict__ d_o, const T* __restrict__ o,
                                                          float* __restrict__ delta, int64_t rows, int D, int S, int H,
                                                          int o_bshd, AttnPaddedStats ps = {}) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
-  if (row >= rows) return;
   const int lane = threadIdx.x % kWave;
-  float acc = 0.f;
-  for (int d = lane; d < D; d += kWave) acc = fmaf(to_float(d_o[row * D + d]), to_float(o[row * D + d]), acc);
-  acc = wave_sum(acc);
-  if (lane == 0) {
-    const int64_t idx = o_row_to_bhs(row, S, H, o_bshd);
-    delta[idx] = acc;
-    if (ps.nlse != nullptr) write_padded_stats(ps, idx / S, static_cast<int>(idx % S), S, ps.lse[idx], acc);
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave; row < rows; row += static_cast<int64_t>(gridDim.x) * 4) {
+    float acc = 0.f;
+    for (int d = lane; d < D; d += kWave) acc = fmaf(to_float(d_o[row * D + d]), to_float(o[row * D + d]), acc);
+    acc = wave_sum(acc);
+    if (lane == 0) {
+      const int64_t idx = o_row_to_bhs(row, S, H, o_bshd);
+      delta[idx] = acc;
+      if (ps.nlse != nullptr) write_padded_stats(ps, idx / S, static_cast<int>(idx % S), S, ps.lse[idx], acc);
+    }
   }
+}
+// Its workgroups: one for four rows, up to as many as a grid (of fewer than 2^32 threads) holds; past 2^26 rows each takes more.
+inline dim3 attn_delta_grid(int64_t rows) {
+  return dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(rows, 4), env_int("MOGRAD_HIP_ATTN_DELTA_MAX_BLOCKS", 1 << 23))));
 }
 
 // Forward: wave = one query row; online softmax in the exp2 domain.

@@ -2140,7 +2140,7 @@ static int launch_delta(const T* d_o, const T* o, float* delta, int64_t rows, co
     }
 #undef MG_DELTA
   } else {
-    hipLaunchKernelGGL((attn_delta_kernel<T>), dim3(static_cast<unsigned>(ceil_div(rows, 4))), dim3(256), 0, stream, d_o,
+    hipLaunchKernelGGL((attn_delta_kernel<T>), attn_delta_grid(rows), dim3(256), 0, stream, d_o,
                        o, delta, rows, D, a.S, a.H, a.o_bshd, ps);
   }
   MG_LAUNCH_CHECK();

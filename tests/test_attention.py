@@ -161,6 +161,18 @@ def test_f32_walks_together_and_apart(device, monkeypatch, name, causal, with_ma
         assert _max_err(two, want) <= (1e-5 if D <= 128 else 2e-5), what
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype,D", [(F32, 100), (F32, 7), (BF16, 72), (BF16, 40)])
+def test_delta_rows_past_the_grid(device, monkeypatch, dtype, D, causal):
+    # More rows than a grid of the delta kernel has waves (2^25 and more): with three workgroups, each takes several.
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", "0")
+    q, k, v, do, _ = _inputs(67, 2, 70, 3, D, dtype, False)
+    want = _fwd_bwd(device, q, k, v, do, None, causal, dtype=dtype)
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_DELTA_MAX_BLOCKS", "3")
+    for got, ref, what in zip(_fwd_bwd(device, q, k, v, do, None, causal, dtype=dtype), want, ("o", "lse", "dq", "dk", "dv")):
+        np.testing.assert_array_equal(got, ref, err_msg=what)
+
+
 @pytest.mark.parametrize("own", ["0", "1"])
 @pytest.mark.parametrize("name,causal,with_mask", MODES)
 @pytest.mark.parametrize("S,D", [(40, 32), (40, 64), (70, 80), (40, 128), (40, 256)])
