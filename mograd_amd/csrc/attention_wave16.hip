@@ -26,6 +26,12 @@ constexpr int attn_wave_lds() { return 4 * kAttnWaveSlots * 2 * attn_wave_tile<D
 __device__ __forceinline__ void attn_wave_copy16(const char* base, unsigned bytes, unsigned dst) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(bytes), "s"(base) : "memory");
 }
+// The same for the lanes of `mask` alone (a lane's bytes go to its own place, whichever lanes copy).  Every lane is here.
+__device__ __forceinline__ void attn_wave_copy16_of(uint64_t mask, const char* base, unsigned bytes, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(dst), "v"(bytes),
+               "s"(base), "s"(mask)
+               : "memory");
+}
 // All of the wave's copies, loads and LDS reads are done.
 __device__ __forceinline__ void attn_wave_settle() {
   asm volatile("" ::: "memory");
@@ -34,18 +40,21 @@ __device__ __forceinline__ void attn_wave_settle() {
 }
 
 // A tensor whose 32-row tiles a wave copies: the image of TileLane16, chunks past D copies of the row's first one (what they
-// give meets zeros or is not stored), rows past S copies of the last one.
-template <int DP>
+// give meets zeros or is not stored), rows past S copies of the last one.  KEPT: chunks past D are left as they are in LDS,
+// zeros (clear_tiles).  The forward's keys are: products of the query's zeros with a first chunk that is infinite are none.
+template <int DP, bool KEPT = false>
 struct WaveTiles16 {
   static constexpr int CH = DP / 8, ROWS = 64 / CH, NI = 32 / ROWS;  // chunks of a row, rows and copies per tile
   const char* base;
   unsigned pitch;
   int S, D;
   unsigned off[NI];
-  __device__ __forceinline__ void place(int i, int lane, int& row, unsigned& col) const {
+  uint64_t own[NI];  // the lanes whose chunk is one of the row's
+  __device__ __forceinline__ bool place(int i, int lane, int& row, unsigned& col) const {
     row = i * ROWS + lane / CH;
     const int c = (lane % CH) ^ tile_swz16<DP>(row);
     col = c * 8 < D ? c * 16 : 0;
+    return c * 8 < D;
   }
   __device__ __forceinline__ void init(const void* base_, int64_t ld, int S_, int D_, int lane) {
     base = static_cast<const char*>(base_);
@@ -56,16 +65,20 @@ struct WaveTiles16 {
     for (int i = 0; i < NI; ++i) {
       int row;
       unsigned col;
-      place(i, lane, row, col);
+      own[i] = __ballot(place(i, lane, row, col));
       off[i] = row * pitch + col;
     }
   }
   __device__ __forceinline__ void copy(int row0, const char* tile, int lane) const {
     const unsigned dst = __builtin_amdgcn_readfirstlane(lds_address(tile));
     const char* p = base + static_cast<int64_t>(row0) * pitch;
+    auto copy16 = [&](int i, unsigned from) {
+      if constexpr (KEPT) attn_wave_copy16_of(own[i], p, from, dst + i * 1024);
+      else attn_wave_copy16(p, from, dst + i * 1024);
+    };
     if (row0 + 32 <= S) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) attn_wave_copy16(p, off[i], dst + i * 1024);
+      for (int i = 0; i < NI; ++i) copy16(i, off[i]);
       return;
     }
     asm volatile("" : "+v"(lane));  // (computed here, not kept in registers)
@@ -74,8 +87,15 @@ struct WaveTiles16 {
       int row;
       unsigned col;
       place(i, lane, row, col);
-      attn_wave_copy16(p, min(row, S - 1 - row0) * pitch + col, dst + i * 1024);
+      copy16(i, min(row, S - 1 - row0) * pitch + col);
     }
+  }
+  // The tile at `tile` and the other slot's.
+  __device__ __forceinline__ void clear_tiles(char* tile, int lane) const {
+    for (int slot = 0; slot < kAttnWaveSlots; ++slot)
+      for (int i = 0; i < NI; ++i)
+        *reinterpret_cast<uint4*>(tile + slot * 2 * attn_wave_tile<DP>() + i * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 };
 
@@ -137,7 +157,10 @@ __device__ __forceinline__ float attn_wave_dot8(const uint4& a, const uint4& b, 
   return dot;
 }
 
-template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS>
+// CUT: D is less than the DC columns that are multiplied.  The masked copies and the cleared tiles cost such heads 1 to 3 % ((2, 4,
+// 600, 40), causal, 7.4 us | 7.6; (1, 8, 500, 80) 9.4 | 9.6), in one form for all also those that fill DC ((1, 6, 1200, 96), bias, 19.2 |
+// 19.8).
+template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS, bool CUT>
 __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ mask, T* __restrict__ o,
     float* __restrict__ lse, AttnDims a, float scale, int tiles) {
@@ -156,8 +179,10 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_
 
   uint4 qf[KS];
   request_row(q + qkv_at(a, b, mc, h), half, a.D, qf);
-  WaveTiles16<DP> kt, vt;
+  WaveTiles16<DP, CUT> kt;
+  WaveTiles16<DP> vt;
   kt.init(k + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
+  if constexpr (CUT) kt.clear_tiles(own, lane);
   vt.init(v + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
   const T* mrow = HAS_BIAS ? mask + (static_cast<int64_t>(bh) * a.S + mc) * a.S : nullptr;
   uint2 bias_next[4];
@@ -551,9 +576,13 @@ int attn_fwd_wave16(const void* q, const void* k, const void* v, const void* mas
   const dim3 grid(static_cast<unsigned>(attn_wave_blocks(static_cast<int64_t>(a.B) * a.H, tiles)));
   attn_wave_pick(dtype, a.D, causal, has_bias, [&](auto t, auto dp, auto dc, auto cz, auto hb) {
     using T = decltype(t);
-    hipLaunchKernelGGL((attn_fwd_wave_kernel<T, decltype(dp)::value, decltype(dc)::value, decltype(cz)::value, decltype(hb)::value>), grid,
-                       dim3(kAttnThreads), 0, stream, static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
-                       static_cast<const T*>(mask), static_cast<T*>(o), lse, a, scale, tiles);
+    auto launch = [&](auto cut) {
+      hipLaunchKernelGGL((attn_fwd_wave_kernel<T, decltype(dp)::value, decltype(dc)::value, decltype(cz)::value, decltype(hb)::value, decltype(cut)::value>),
+                         grid, dim3(kAttnThreads), 0, stream, static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
+                         static_cast<const T*>(mask), static_cast<T*>(o), lse, a, scale, tiles);
+    };
+    if (a.D < decltype(dc)::value) launch(std::true_type{});
+    else launch(std::false_type{});
   });
   MG_LAUNCH_CHECK();
   return MG_OK;
