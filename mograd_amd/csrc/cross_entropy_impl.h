@@ -24,6 +24,10 @@ constexpr float kLn2 = 0.6931471805599453f;
 
 __device__ __forceinline__ float fast_exp2(float v) { return __builtin_amdgcn_exp2f(v); }
 
+// What is taken off a row's logits before anything else: its largest one where that overflows in log2 units (a row of classes
+// that are all masked with the type's lowest value), or zero.  Such logits are the largest one or at least 2^103 below it.
+__device__ __forceinline__ float row_base(float m) { return fabsf(m) <= FLT_MAX && fabsf(m) > FLT_MAX / kLog2e ? m : 0.f; }
+
 // Rows that do not lie on 16-byte chunks (ANY below) are read and written in misaligned ones, with -inf past a row's end: it
 // is no maximum and adds nothing to a sum of exponentials.
 template <typename T>
@@ -93,6 +97,14 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
       }
     }
     row_allreduce_max<TPR, WG, 1>(m, slots, phase);
+    const float base = row_base(m[0]);
+    if (__builtin_expect(base != 0.f, 0)) {
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) x.v[i][e] -= base;
+      m[0] = 0.f;
+    }
     const float m2 = m[0] * kLog2e;
     T* out_row = dlogits + row * C;
 
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
       const bool id_ok = id >= 0 && id < C;
       const bool owner = id_ok && (static_cast<int>(id) / VEC) % TPR == t;
       if (owner) {
-        const float xl = to_float(xr[id]);
+        const float xl = to_float(xr[id]) - base;
         const float lp = xl - m[0] - logf(s[0]);  // log softmax at the label
         out_row[id] = from_float<T>((fast_exp2(fmaf(xl, kLog2e, -m2)) / s[0] - 1.0f) * scale);
         if (rowloss != nullptr) rowloss[row] = -lp * inv_rows;
@@ -185,6 +197,20 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
     }
   }
 }
+
+// exp(x - m), as 2^(x log2(e) - m log2(e)).  Where that overflows it is 2^(x - m), the same for such logits (see row_base), and
+// with m no less than the least float: classes masked with -inf or with the type's lowest value, where a thread has seen nothing
+// else yet, add finite terms to an online sum (from minus infinity they would be NaN, which no later maximum takes out of it).
+struct ExpReference {
+  float by, top;
+  __device__ __forceinline__ explicit ExpReference(float m) {
+    const float m2 = m * kLog2e;
+    const bool plain = fabsf(m2) <= FLT_MAX;
+    by = plain ? kLog2e : 1.f;
+    top = plain ? m2 : fmaxf(m, -FLT_MAX);
+  }
+  __device__ __forceinline__ float weight(float x) const { return fast_exp2(fmaf(x, by, -top)); }
+};
 
 // Eight 16-bit values out of four registers, word by word: seen as an array of eight, fp16 values were held one to a
 // register, and spilled ((8192, 50304) 610 us against 341).
@@ -262,7 +288,7 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
     if (here(i)) top(raw[i]);
   if (ANY && tail) top(end);
   row_allreduce_max<TPR, TPR, 1>(m, slots, phase);
-  const float m2 = m[0] * kLog2e;
+  const ExpReference ref(m[0]);
   // Between the passes the packed registers are made opaque to the compiler, which would
   // otherwise keep the unpacked values of one pass for the next.
   auto forget = [&]() {
@@ -276,7 +302,7 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
     float x[VEC];
     unpack_words<T>(r, x);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s[0] += fast_exp2(fmaf(x[e], kLog2e, -m2));
+    for (int e = 0; e < VEC; ++e) s[0] += ref.weight(x[e]);
   };
 #pragma unroll
   for (int i = 0; i < VPT; ++i)
@@ -288,7 +314,7 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
   auto gradient = [&](const uint4& r, float (&x)[VEC]) {
     unpack_words<T>(r, x);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) x[e] = fast_exp2(fmaf(x[e], kLog2e, -m2)) * k;
+    for (int e = 0; e < VEC; ++e) x[e] = ref.weight(x[e]) * k;
   };
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
@@ -310,7 +336,7 @@ __global__ __launch_bounds__(TPR, TPR <= 256 ? (VPT > 16 ? 3 : 4) : (TPR <= 512 
   if (id_ok && (static_cast<int>(id) / VEC) % TPR == t) {
     const float xl = to_float(xr[id]);
     const float lp = xl - m[0] - logf(s[0]);  // log softmax at the label
-    out_row[id] = from_float<T>((fast_exp2(fmaf(xl, kLog2e, -m2)) / s[0] - 1.0f) * scale);
+    out_row[id] = from_float<T>((ref.weight(xl) / s[0] - 1.0f) * scale);
     if (rowloss != nullptr) rowloss[row] = -lp * inv_rows;
   }
   // An id outside [0, C) selects no column: the row's loss term is flagged NaN.
@@ -328,11 +354,6 @@ __device__ __forceinline__ void stream_load(const T* row, int64_t c, int64_t C, 
   VecAny<T, VEC>::words_end(row + c, static_cast<int>(max(c + VEC - C, int64_t{0})), fill, w);
   VecAny<T, VEC>::unpack(w, v);
 }
-
-// What an online sum of exponentials subtracts, in log2 units: the maximum so far, but no less than the least float, so that
-// classes masked with -inf or with the type's lowest value, where a thread has seen nothing else yet, add zeros (from minus
-// infinity they would be NaN, which no later maximum takes out of the sum).
-__device__ __forceinline__ float online_reference(float m) { return fmaxf(m * kLog2e, -FLT_MAX); }
 
 // Online (max, sum-exp) over the elements a thread visits, merged across the workgroup.  ONCE: the
 // row is not read again by this kernel, so its loads go past the caches.
@@ -362,11 +383,11 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);  // exp2(-inf) == 0 on the first chunk
       m = cm;
     }
-    const float m2 = online_reference(m);
+    const ExpReference ref(m);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) s += fast_exp2(fmaf(v[u][e], kLog2e, -m2));
+      for (int e = 0; e < VEC; ++e) s += ref.weight(v[u][e]);
   }
   for (; c < C; c += step) {
     float v[VEC];
@@ -379,9 +400,9 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);
       m = cm;
     }
-    const float m2 = online_reference(m);
+    const ExpReference ref(m);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s += fast_exp2(fmaf(v[e], kLog2e, -m2));
+    for (int e = 0; e < VEC; ++e) s += ref.weight(v[e]);
   }
   float mm[1] = {m};
   block_allreduce<MaxOp, WG / kWave, 1>(mm, slots, phase);
@@ -433,10 +454,10 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
         ts *= fast_exp2((tm - cm) * kLog2e);
         tm = cm;
       }
-      const float m2 = online_reference(tm);
+      const ExpReference ref(tm);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        ts += fast_exp2(fmaf(v[e], kLog2e, -m2));
+        ts += ref.weight(v[e]);
         dot[0] += !ANY || c + e < C ? v[e] * y[e] : 0.f;
         dot[1] += y[e];
       }
@@ -449,12 +470,21 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
     block_allreduce<SumOp, WG / kWave, 3>(red, slots3, 0);
     m = mm[0];
     s = red[0];
+    const float base = row_base(m);
+    if (__builtin_expect(base != 0.f, 0)) {  // (the sums of label * x are as large as the type: once more, from the base)
+      float again[1] = {0.f};
+      for (int64_t c = threadIdx.x; c < C; c += WG) again[0] += (to_float(xr[c]) - base) * to_float(yr[c]);
+      block_allreduce<SumOp, WG / kWave, 1>(again, slots, 0);
+      red[1] = again[0];
+      m = 0.f;
+    }
     if (threadIdx.x == 0) rowloss[row] = -(red[1] - (m + logf(s)) * red[2]) * inv_rows;
   } else {
     stream_max_sum<T, VEC, WG, ONCE, ANY>(xr, C, slots, phase, m, s);
     if (threadIdx.x == 0) {
       const int64_t id = load_id(labels, row, id64 != 0);
-      rowloss[row] = (id < 0 || id >= C) ? NAN : -(to_float(xr[id]) - (m + logf(s))) * inv_rows;
+      const float base = row_base(m);
+      rowloss[row] = (id < 0 || id >= C) ? NAN : -((to_float(xr[id]) - base) - ((m - base) + logf(s))) * inv_rows;
     }
   }
 }
@@ -474,9 +504,17 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
   const float scale = (upstream != nullptr ? to_float(upstream[0]) : 1.0f) * inv_rows;
   float m, s;
   stream_max_sum<T, VEC, WG, false, ANY>(xr, C, slots, phase, m, s);
+  const float base = row_base(m);
+  m -= base;
   const float m2 = m * kLog2e;
   const float inv_sum = 1.0f / s;
   const float shift = m + logf(s);
+  auto rebase = [&](float (&v)[VEC]) {
+    if (__builtin_expect(base != 0.f, 0)) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] -= base;
+    }
+  };
   const int64_t id = DENSE ? 0 : load_id(labels, row, id64 != 0);
   float acc[1] = {0.f};
   constexpr int U = DENSE ? 1 : 4;  // integer labels: four chunks in flight per thread
@@ -500,6 +538,7 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
       for (int u = 0; u < U; ++u) {
         const int64_t c = c0 + u * step;
         float out[VEC];
+        rebase(v[u]);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           float p = fast_exp2(fmaf(v[u][e], kLog2e, -m2)) * inv_sum;
@@ -517,6 +556,7 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
     float v[VEC], out[VEC];
     if constexpr (ANY) stream_load<T, VEC>(xr, c, C, kMinusInfWord<T>, v);
     else VecIO<T, VEC>::load(xr + c, v);
+    rebase(v);
     if constexpr (DENSE) {
       const T* yr = static_cast<const T*>(labels) + row * C;
       float y[VEC];

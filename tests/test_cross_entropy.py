@@ -342,6 +342,53 @@ def test_masked_classes(device, dtype, half_ulp, size, vec, mask, seen, Cc, star
             assert (np.abs(got.to_numpy()[start:].reshape(N, Cc) - exact) <= bound).all()
 
 
+@pytest.mark.parametrize("dtype,half_ulp,size", [(F32, 2.0 ** -24, 4), (F16, 2.0 ** -11, 2), (BF16, 2.0 ** -8, 2)])
+@pytest.mark.parametrize("end", [-1.0, 1.0])
+@pytest.mark.parametrize("Cc,start", [(3, 0), (65, 0), (257, 1), (1001, 0), (4104, 0), (4105, 0), (16392, 0), (20001, 1), (40000, 0), (70001, 0), (140001, 0)])
+def test_a_row_of_the_types_last_values(device, dtype, half_ulp, size, end, Cc, start):
+    # A row whose classes are all at the type's lowest (or largest) value, whose multiples by log2(e) fp32 does not hold, next to
+    # ordinary ones: equally likely classes.  Bounds as above.
+    lib, st, N = device.lib, device.stream, 3
+    x = round_to_dtype(normal(38, 0, (N, Cc), std=2.0), dtype)
+    last = {F32: np.finfo(np.float32).max, F16: 65504.0, BF16: float(np.uint32(0x7F7F0000).view(np.float32))}[dtype]
+    x[1] = end * last
+    ids = np.array([0, Cc // 2, Cc - 1])
+    dense = round_to_dtype(0.9 * O.one_hot(ids, Cc) + 0.1 / Cc, dtype)
+
+    def put(a):
+        return AnyBuffer.from_numpy(device, np.concatenate([np.zeros(start, np.float32), a.reshape(-1).astype(np.float32)]), dtype)
+
+    bx, by, bi = put(x), put(dense), AnyBuffer.from_numpy(device, ids.astype(np.int32), I32)
+    bu = AnyBuffer.from_numpy(device, np.array([2.0], np.float32), dtype)
+    at = lambda b: C.c_void_p(b.data_ptr().value + start * size)
+    x = x.astype(np.float64)
+    x -= x.max(-1, keepdims=True)
+    e = np.exp(x)
+    p = e / e.sum(-1, keepdims=True)
+    logp = x - np.log(e.sum(-1, keepdims=True))
+    for y, ptr, calls, extra in ((O.one_hot(ids, Cc), bi.data_ptr(), (lib.mg_cross_entropy_fused_ids, lib.mg_cross_entropy_grad_ids, lib.mg_cross_entropy_ids), (I32,)),
+                                 (dense, at(by), (lib.mg_cross_entropy_fused, lib.mg_cross_entropy_grad, lib.mg_cross_entropy), ())):
+        y = y.astype(np.float64)
+        fused, grad, alone = calls
+        loss, loss2, out, out2 = (AnyBuffer.create(dtype, device, 1), AnyBuffer.create(dtype, device, 1), put(np.zeros((N, Cc))), put(np.zeros((N, Cc))))
+        fused(at(bx), ptr, bu.data_ptr(), loss.data_ptr(), at(out), N, Cc, dtype, *extra, st)
+        grad(at(bx), ptr, bu.data_ptr(), at(out2), N, Cc, dtype, *extra, st)
+        alone(at(bx), ptr, loss2.data_ptr(), N, Cc, dtype, *extra, st)
+        want = -(y * logp).sum() / N
+        # (fp16's last values are ordinary numbers, whose multiples of the labels and sum with log C fp32 rounds)
+        off = (2.0 ** -18 + 2.0 ** -24 * Cc / 256) * (y * (np.abs(logp) + 16.0)).sum() / N
+        if dtype == F16:
+            off += 2.0 ** -24 * (Cc / 256 + 32) * 65504.0 * y[1].sum() / N
+        for got in (loss.item(), loss2.item()):
+            assert abs(got - want) <= 1.02 * half_ulp * abs(want) + off, (got, want)
+        exact, scale = (p - y) * 2.0 / N, 2.0 / N
+        # (half an ulp of 65504 + log C and of its multiple by log2(e) are in the exponent)
+        rel = np.array([2.0 ** -18, 2.0 ** -9 + 2.0 ** -8 if dtype == F16 else 2.0 ** -18, 2.0 ** -18])[:, None]
+        bound = 1.02 * half_ulp * np.abs(exact) + rel * (p + y) * scale + (2.0 ** -25 if dtype == F16 else 0.0)
+        for got in (out, out2):
+            assert (np.abs(got.to_numpy()[start:].reshape(N, Cc) - exact) <= bound).all()
+
+
 def test_out_of_range_id_flags_loss(device):
     x = normal(34, 0, (4, 100))
     ids = np.array([0, 5, 100, 7], np.int32)
