@@ -41,7 +41,8 @@ __device__ __forceinline__ void attn_wave_settle() {
 
 // A tensor whose 32-row tiles a wave copies: the image of TileLane16, chunks past D copies of the row's first one (what they
 // give meets zeros or is not stored), rows past S copies of the last one.  KEPT: chunks past D are left as they are in LDS,
-// zeros (clear_tiles).  The forward's keys are: products of the query's zeros with a first chunk that is infinite are none.
+// zeros (clear_tiles).  K's are, in the forward and in dQ: a key whose first chunk is -inf has no weight, but products of the
+// query's zeros with that chunk would be NaN.
 template <int DP, bool KEPT = false>
 struct WaveTiles16 {
   static constexpr int CH = DP / 8, ROWS = 64 / CH, NI = 32 / ROWS;  // chunks of a row, rows and copies per tile
@@ -90,12 +91,12 @@ struct WaveTiles16 {
       copy16(i, min(row, S - 1 - row0) * pitch + col);
     }
   }
-  // The tile at `tile` and the other slot's.
+  // Zeros for chunks D / 8 .. DC / 8 - 1 of the tile at `tile` and of the other slot's, which the wave's first attn_wave_settle
+  // waits for.  (Clearing whole tiles was 7 % of a backward of 13 us.)
+  template <int DC>
   __device__ __forceinline__ void clear_tiles(char* tile, int lane) const {
-    for (int slot = 0; slot < kAttnWaveSlots; ++slot)
-      for (int i = 0; i < NI; ++i)
-        *reinterpret_cast<uint4*>(tile + slot * 2 * attn_wave_tile<DP>() + i * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    for (int c = D / 8; c < DC / 8; ++c)
+      *reinterpret_cast<uint4*>(tile + lane / 32 * 2 * attn_wave_tile<DP>() + tile16_chunk_at<DP>(lane % 32, c)) = make_uint4(0, 0, 0, 0);
   }
 };
 
@@ -157,9 +158,9 @@ __device__ __forceinline__ float attn_wave_dot8(const uint4& a, const uint4& b, 
   return dot;
 }
 
-// CUT: D is less than the DC columns that are multiplied.  The masked copies and the cleared tiles cost such heads 1 to 3 % ((2, 4,
-// 600, 40), causal, 7.4 us | 7.6; (1, 8, 500, 80) 9.4 | 9.6), in one form for all also those that fill DC ((1, 6, 1200, 96), bias, 19.2 |
-// 19.8).
+// CUT: D is less than the DC columns that are multiplied.  The masked copies and the cleared chunks cost such heads up to 3 % of the
+// forward ((1, 8, 500, 80) 9.2 us | 9.3; (1, 8, 1000, 40), bias, 12.7 | 13.0) and nothing of the backward; in one form for all they
+// cost those that fill DC as much ((1, 6, 1200, 96), bias, 19.2 | 19.8).
 template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS, bool CUT>
 __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ mask, T* __restrict__ o,
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_
   WaveTiles16<DP, CUT> kt;
   WaveTiles16<DP> vt;
   kt.init(k + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
-  if constexpr (CUT) kt.clear_tiles(own, lane);
+  if constexpr (CUT) kt.template clear_tiles<DC>(own, lane);
   vt.init(v + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
   const T* mrow = HAS_BIAS ? mask + (static_cast<int64_t>(bh) * a.S + mc) * a.S : nullptr;
   uint2 bias_next[4];
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 64 ? 2 : 1) void attn_fwd_wave_
 }
 
 // dQ of block `block`; `lds` holds attn_wave_lds<DP>() bytes.
-template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS>
+template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS, bool CUT>
 __device__ __forceinline__ void attn_dq_wave_block(int block, char* lds, const T* __restrict__ d_o, const T* __restrict__ o,
                                                    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                    const T* __restrict__ mask, const float* __restrict__ lse,
@@ -318,9 +319,11 @@ __device__ __forceinline__ void attn_dq_wave_block(int block, char* lds, const T
   request_row(o + o_at(a, b, h, mc), half, a.D, of);
   request_row(q + qkv_at(a, b, mc, h), half, a.D, qf);
   float lse2 = lse[static_cast<int64_t>(bh) * a.S + mc] * kAttnLog2e;
-  WaveTiles16<DP> kt, vt;
+  WaveTiles16<DP, CUT> kt;
+  WaveTiles16<DP> vt;
   kt.init(k + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
   vt.init(v + qkv_at(a, b, 0, h), a.ld, a.S, a.D, lane);
+  if constexpr (CUT) kt.template clear_tiles<DC>(own, lane);
   const T* mrow = HAS_BIAS ? mask + (static_cast<int64_t>(bh) * a.S + mc) * a.S : nullptr;
   uint2 bias_next[4];
   auto request = [&](int t, int slot) {
@@ -537,7 +540,7 @@ __device__ __forceinline__ void attn_dkdv_wave_block(int block, char* lds, float
 }
 
 // Both walks in one launch: workgroups [0, blocks) take dK and dV, whose steps are the longer ones, the rest dQ.
-template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS>
+template <typename T, int DP, int DC, bool CAUSAL, bool HAS_BIAS, bool CUT>
 __global__ __launch_bounds__(kAttnThreads, DP <= 64 && !(HAS_BIAS && DC > 32) ? 2 : 1) void attn_bwd_wave_kernel(
     const T* __restrict__ d_o, const T* __restrict__ o, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const T* __restrict__ mask, const float* __restrict__ lse, T* __restrict__ dq, T* __restrict__ dk, T* __restrict__ dv,
@@ -547,7 +550,7 @@ __global__ __launch_bounds__(kAttnThreads, DP <= 64 && !(HAS_BIAS && DC > 32) ? 
   if (static_cast<int>(blockIdx.x) < blocks)
     attn_dkdv_wave_block<T, DP, DC, CAUSAL, HAS_BIAS>(blockIdx.x, lds, stats, d_o, o, q, k, v, mask, lse, dk, dv, a, scale, tiles);
   else
-    attn_dq_wave_block<T, DP, DC, CAUSAL, HAS_BIAS>(blockIdx.x - blocks, lds, d_o, o, q, k, v, mask, lse, dq, a, scale, tiles);
+    attn_dq_wave_block<T, DP, DC, CAUSAL, HAS_BIAS, CUT>(blockIdx.x - blocks, lds, d_o, o, q, k, v, mask, lse, dq, a, scale, tiles);
 }
 
 // f(T, DP, DC, CAUSAL, HAS_BIAS) with the constants that the call asks for.
@@ -595,11 +598,15 @@ int attn_bwd_wave16(const void* d_o, const void* o, const void* q, const void* k
   const int blocks = attn_wave_blocks(static_cast<int64_t>(a.B) * a.H, tiles);
   attn_wave_pick(dtype, a.D, causal, has_bias, [&](auto t, auto dp, auto dc, auto cz, auto hb) {
     using T = decltype(t);
-    hipLaunchKernelGGL((attn_bwd_wave_kernel<T, decltype(dp)::value, decltype(dc)::value, decltype(cz)::value, decltype(hb)::value>),
-                       dim3(2 * static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, stream, static_cast<const T*>(d_o),
-                       static_cast<const T*>(o), static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
-                       static_cast<const T*>(mask), lse, static_cast<T*>(dq), static_cast<T*>(dk), static_cast<T*>(dv), a, scale,
-                       tiles, blocks);
+    auto launch = [&](auto cut) {
+      hipLaunchKernelGGL((attn_bwd_wave_kernel<T, decltype(dp)::value, decltype(dc)::value, decltype(cz)::value, decltype(hb)::value, decltype(cut)::value>),
+                         dim3(2 * static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, stream, static_cast<const T*>(d_o),
+                         static_cast<const T*>(o), static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
+                         static_cast<const T*>(mask), lse, static_cast<T*>(dq), static_cast<T*>(dk), static_cast<T*>(dv), a, scale,
+                         tiles, blocks);
+    };
+    if (a.D < decltype(dc)::value) launch(std::true_type{});
+    else launch(std::false_type{});
   });
   MG_LAUNCH_CHECK();
   return MG_OK;
