@@ -40,9 +40,10 @@ __device__ __forceinline__ void attn_wave_settle() {
 }
 
 // A tensor whose 32-row tiles a wave copies: the image of TileLane16, chunks past D copies of the row's first one (what they
-// give meets zeros or is not stored), rows past S copies of the last one.  KEPT: chunks past D are left as they are in LDS,
-// zeros (clear_tiles).  K's are, in the forward and in dQ: a key whose first chunk is -inf has no weight, but products of the
-// query's zeros with that chunk would be NaN.
+// give meets zeros or is not stored), rows past S zeros (their weights are zero, but a last row's copies with an
+// infinity, an overflowed gradient's, would make NaN of it).  KEPT: chunks past D are left as they are in LDS, zeros (clear_tiles).
+// K's are, in the forward and in dQ: a key whose first chunk is -inf has no weight, but products of the query's zeros with that
+// chunk would be NaN.  The wave's next attn_wave_settle waits for all of these.
 template <int DP, bool KEPT = false>
 struct WaveTiles16 {
   static constexpr int CH = DP / 8, ROWS = 64 / CH, NI = 32 / ROWS;  // chunks of a row, rows and copies per tile
@@ -51,12 +52,6 @@ struct WaveTiles16 {
   int S, D;
   unsigned off[NI];
   uint64_t own[NI];  // the lanes whose chunk is one of the row's
-  __device__ __forceinline__ bool place(int i, int lane, int& row, unsigned& col) const {
-    row = i * ROWS + lane / CH;
-    const int c = (lane % CH) ^ tile_swz16<DP>(row);
-    col = c * 8 < D ? c * 16 : 0;
-    return c * 8 < D;
-  }
   __device__ __forceinline__ void init(const void* base_, int64_t ld, int S_, int D_, int lane) {
     base = static_cast<const char*>(base_);
     pitch = static_cast<unsigned>(ld) * 2;
@@ -64,35 +59,35 @@ struct WaveTiles16 {
     D = D_;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      int row;
-      unsigned col;
-      own[i] = __ballot(place(i, lane, row, col));
-      off[i] = row * pitch + col;
+      const int row = i * ROWS + lane / CH, c = (lane % CH) ^ tile_swz16<DP>(row);
+      own[i] = __ballot(c * 8 < D);
+      off[i] = row * pitch + (c * 8 < D ? c * 16 : 0);
     }
   }
-  __device__ __forceinline__ void copy(int row0, const char* tile, int lane) const {
+  __device__ __forceinline__ void copy(int row0, char* tile, int lane) const {
     const unsigned dst = __builtin_amdgcn_readfirstlane(lds_address(tile));
     const char* p = base + static_cast<int64_t>(row0) * pitch;
-    auto copy16 = [&](int i, unsigned from) {
-      if constexpr (KEPT) attn_wave_copy16_of(own[i], p, from, dst + i * 1024);
-      else attn_wave_copy16(p, from, dst + i * 1024);
-    };
     if (row0 + 32 <= S) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) copy16(i, off[i]);
+      for (int i = 0; i < NI; ++i) {
+        if constexpr (KEPT) attn_wave_copy16_of(own[i], p, off[i], dst + i * 1024);
+        else attn_wave_copy16(p, off[i], dst + i * 1024);
+      }
       return;
     }
-    asm volatile("" : "+v"(lane));  // (computed here, not kept in registers)
+    // a copy is ROWS rows, CH lanes to a row
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      int row;
-      unsigned col;
-      place(i, lane, row, col);
-      copy16(i, min(row, S - 1 - row0) * pitch + col);
+      const int lanes = (S - row0 - i * ROWS) * CH;
+      if (lanes > 0) {
+        const uint64_t rows = lanes >= 64 ? ~uint64_t{0} : (uint64_t{1} << lanes) - 1;
+        attn_wave_copy16_of(KEPT ? rows & own[i] : rows, p, off[i], dst + i * 1024);
+      }
+      if (lane >= lanes) *reinterpret_cast<uint4*>(tile + i * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
     }
   }
-  // Zeros for chunks D / 8 .. DC / 8 - 1 of the tile at `tile` and of the other slot's, which the wave's first attn_wave_settle
-  // waits for.  (Clearing whole tiles was 7 % of a backward of 13 us.)
+  // Zeros for chunks D / 8 .. DC / 8 - 1 of the tile at `tile` and of the other slot's.  (Clearing whole tiles was 7 % of a backward
+  // of 13 us.)
   template <int DC>
   __device__ __forceinline__ void clear_tiles(char* tile, int lane) const {
     for (int c = D / 8; c < DC / 8; ++c)
@@ -467,7 +462,8 @@ __device__ __forceinline__ void attn_dkdv_wave_block(int block, char* lds, float
       dl = ks * 16 + half * 8 < a.D ? d : dl;
     }
     st[lane % 32] = -lse_next * kAttnLog2e;  // (both halves of the wave write the same)
-    st[32 + lane % 32] = sum_halves(dl);
+    dl = sum_halves(dl);
+    st[32 + lane % 32] = t * 32 + lane % 32 < a.S ? dl : 0.f;
     T bias_v[16];
     if constexpr (HAS_BIAS) {
 #pragma unroll

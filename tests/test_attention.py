@@ -328,6 +328,26 @@ def test_keys_of_minus_infinity_have_no_weight(device, monkeypatch, dtype, tol, 
         assert _max_err(got, want) <= tol * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("dtype,tol", [(F16, 2e-3), (BF16, 1.6e-2)])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
+@pytest.mark.parametrize("S,D", [(30, 8), (70, 64), (97, 72), (65, 128), (131, 96)])
+def test_a_last_row_with_an_infinity(device, monkeypatch, dtype, tol, name, causal, with_mask, S, D):
+    # An infinity in the last row of V or of dO, in a sequence that ends inside a tile: O's and dV's column is infinite, not NaN,
+    # and the other columns have nothing of it (the 32-row kernels; some of the 128-row ones have NaN).
+    monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", "1")
+    q, k, v, do, m = _inputs(69, 1, S, 2, D, dtype, with_mask)
+    ro, _ = O.sdpa_fwd(q, k, v, m, causal)
+    rdv = O.sdpa_bwd(q, k, v, do, m, causal)[2]
+    v2, do2 = v.copy(), do.copy()
+    v2[:, S - 1, :, 0] = -np.inf
+    do2[:, :, S - 1, 0] = np.inf
+    o = _fwd(device, q, k, v2, m, causal, 1.0 / math.sqrt(D), dtype)[0].to_numpy((1, 2, S, D))
+    seen = slice(S - 1, S) if causal else slice(0, S)  # (masked, it is zero times infinity)
+    assert np.all(np.isneginf(o[:, :, seen, 0])) and _max_err(o[..., 1:], ro[..., 1:]) <= tol
+    dv = _fwd_bwd(device, q, k, v, do2, m, causal, dtype=dtype)[4]
+    assert np.all(np.isposinf(dv[..., 0])) and _max_err(dv[..., 1:], rdv[..., 1:]) <= tol * max(1.0, np.abs(rdv).max())
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_bf16_gradients_rtol(device, causal):
     # Parity bar for bf16 attention gradients: rtol 2e-2, with an absolute floor for entries that
