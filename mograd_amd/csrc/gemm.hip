@@ -724,14 +724,19 @@ static int linear_bwd_one_launch(const void* dy, const void* x, const void* w, v
   const Choice16 choice = choose_linear_bwd(M, N, K, dx != nullptr, db != nullptr);
   if (choice.tile < 0) return MG_OK;
   // 64 x 64 tiles read arrays that are at least 8 wide from wherever they start.  That saves the copies, a launch of 2.4 us and
-  // their bytes, and makes a step of dX's walk over N 0.1 us longer, 0.2 where its last tile of columns is cut off: with the
-  // copies | without, (64, 1001 <- 192) 10.5 | 9.6, (64, 2601 <- 192) 16.4 | 18.1, (64, 1001 <- 200) 10.7 | 11.2, (64, 2601 <- 200)
-  // 16.5 | 22.1; (406, 1832 <- 83) 15.3 | 18.4, (675, 149 <- 2391) 18.4 | 14.0, (700, 701 <- 703) 16.8 | 12.7.  Longer products are
-  // faster with the copies ((1999, 1001 <- 768) 24.5 | 25.2; (300, 3001 <- 517) 26.2 | 31.0).
-  const double longer = !dx ? 0.0 : (K % 64 == 0 ? 0.1 : 0.2) * static_cast<double>(ceil_div(N, 64));
+  // their bytes, and makes the steps of the longer of the two walks longer: dX's over N by 0.1 us a step, 0.2 where its last tile
+  // of columns is cut off, dW's over M by 0.22, by 0.15 of what the copies of X and W leave of that.  With the copies | without,
+  // (64, 1001 <- 192) 9.7 | 8.8, (64, 2601 <- 192) 15.9 | 17.3, (64, 1001 <- 200) 10.0 | 10.3, (64, 2601 <- 200) 15.9 | 21.2;
+  // (406, 1832 <- 83) 14.0 | 17.0, (675, 149 <- 2391) 15.4 | 12.6, (700, 701 <- 703) 14.1 | 11.8; (2587, 101 <- 256) 12.7 | 11.1,
+  // (1481, 299 <- 1088) 16.1 | 19.2, (1344, 77 <- 2240) 13.8 | 16.2.  Longer products are faster with the copies ((1999, 1001 <- 768)
+  // 22.3 | 24.5; (300, 3001 <- 517) 24.9 | 30.4).  Over 3400 layers of 16 to 8192 rows and 16 to 4096 columns this takes 0.4 % more
+  // time than the better of the two for each, the copies always 20 %.  MOGRAD_HIP_LINEAR_BWD_ANY = 0 | 1 overrides it.
+  const double longer_x = !dx ? 0.0 : (K % 64 == 0 ? 0.1 : 0.2) * static_cast<double>(ceil_div(N, 64));
+  const double longer_w = (pad_k ? 0.15 : 0.22) * static_cast<double>(ceil_div(ceil_div(M, 64), std::max(choice.splits, 1)));
   const double copied = (pad_n ? static_cast<double>(M) * N : 0.0) + (pad_k ? static_cast<double>(K) * (dx ? M + N : M) : 0.0);
-  const bool any = choice.tile == kSmall && (pad_n || pad_k) && N >= 8 && K >= 8 && choice.us <= 15.0 &&
-                   longer <= 2.4 + 4.0 * copied / 3.7e6 && !env_str("MOGRAD_HIP_GEMM16_PAD");
+  const bool any_pays = choice.us <= 15.0 && std::max(longer_x, longer_w) <= 2.4 + 4.0 * copied / 3.7e6;
+  const bool any = choice.tile == kSmall && (pad_n || pad_k) && N >= 8 && K >= 8 && !env_str("MOGRAD_HIP_GEMM16_PAD") &&
+                   env_int("MOGRAD_HIP_LINEAR_BWD_ANY", any_pays) != 0;
   const bool small = choice.tile == kSmall, wide = choice.tile == kTileWide;
   if (ln && (!wide || relu_mask || pad_n || pad_k || !aligned16(ln->x) || !aligned16(ln->gamma) || !aligned16(dx))) return MG_OK;
   // (without the LayerNorm the same K ranges in 128 x 192 tiles, two workgroups per CU)

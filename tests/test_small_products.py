@@ -65,6 +65,9 @@ def test_linear_forward_and_backward(device, dtype, M, N, K):
     (BF16, "LINEAR_BWD_SMALL", (0, 1), [(2048, 264, 200), (1999, 129, 333), (2600, 776, 384)]),
     (BF16, "LINEAR_BWD_SPLITS", (1, 3, 7), [(1030, 264, 200), (999, 129, 65)]),
     (F16, "LINEAR_BWD_SPLITS", (1, 3), [(999, 129, 65)]),
+    # 16-bit backward of layers off the 16-byte chunks on 64 x 64 tiles: from copies or from where the arrays are
+    (BF16, "LINEAR_BWD_ANY", (0, 1), [(497, 45, 27), (1344, 77, 264), (1481, 299, 1088)]),
+    (F16, "LINEAR_BWD_ANY", (0, 1), [(1103, 152, 93)]),
 ])
 def test_both_sides_of_a_choice(device, monkeypatch, dtype, knob, values, shapes):
     for value in values:
