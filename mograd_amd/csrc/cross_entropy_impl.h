@@ -198,16 +198,14 @@ __global__ __launch_bounds__(WG, (TPR == 256 && VPT * VEC > 128) ? 2 : 1) void c
   }
 }
 
-// exp(x - m), as 2^(x log2(e) - m log2(e)).  Where that overflows it is 2^(x - m), the same for such logits (see row_base), and
-// with m no less than the least float: classes masked with -inf or with the type's lowest value, where a thread has seen nothing
-// else yet, add finite terms to an online sum (from minus infinity they would be NaN, which no later maximum takes out of it).
+// exp(x - m), as 2^(x log2(e) - m log2(e)), or where that overflows as 2^(x - m), the same for such logits (see row_base).
 struct ExpReference {
   float by, top;
   __device__ __forceinline__ explicit ExpReference(float m) {
     const float m2 = m * kLog2e;
     const bool plain = fabsf(m2) <= FLT_MAX;
     by = plain ? kLog2e : 1.f;
-    top = plain ? m2 : fmaxf(m, -FLT_MAX);
+    top = plain ? m2 : m;
   }
   __device__ __forceinline__ float weight(float x) const { return fast_exp2(fmaf(x, by, -top)); }
 };
@@ -355,11 +353,28 @@ __device__ __forceinline__ void stream_load(const T* row, int64_t c, int64_t C, 
   VecAny<T, VEC>::unpack(w, v);
 }
 
-// Online (max, sum-exp) over the elements a thread visits, merged across the workgroup.  ONCE: the
+// What an online sum of exponentials subtracts, in log2 units: the maximum so far, but no less than the least float, so that
+// classes masked with -inf or with the type's lowest value, where a thread has seen nothing else yet, add zeros (from minus
+// infinity they would be NaN, which no later maximum takes out of the sum).
+__device__ __forceinline__ float online_reference(float m) { return fmaxf(m * kLog2e, -FLT_MAX); }
+
+// A thread's share of the sum of exponentials (and of label * x) of a row from its base (see row_base), once more and an element at
+// a time.
+template <typename T, int WG, bool DENSE>
+__device__ __forceinline__ void rebased_sums(const T* xr, const T* yr, int64_t C, float base, float& sum, float& dot) {
+  sum = dot = 0.f;
+  for (int64_t c = threadIdx.x; c < C; c += WG) {
+    const float x = to_float(xr[c]) - base;
+    sum += fast_exp2(x * kLog2e);
+    if constexpr (DENSE) dot += x * to_float(yr[c]);
+  }
+}
+
+// Online (max, sum-exp) over the elements a thread visits, merged across the workgroup, the maximum less the row's base.  ONCE: the
 // row is not read again by this kernel, so its loads go past the caches.
 template <typename T, int VEC, int WG, bool ONCE = false, bool ANY = false>
 __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t C, float* slots, int& phase, float& m_out,
-                                               float& s_out) {
+                                               float& s_out, float& base_out) {
   auto fetch = [](const T* p, float (&v)[VEC]) {
     if constexpr (ANY) VecAny<T, VEC>::load(p, v);
     else if constexpr (ONCE) VecIO<T, VEC>::load_stream(p, v);
@@ -383,11 +398,11 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);  // exp2(-inf) == 0 on the first chunk
       m = cm;
     }
-    const ExpReference ref(m);
+    const float m2 = online_reference(m);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) s += ref.weight(v[u][e]);
+      for (int e = 0; e < VEC; ++e) s += fast_exp2(fmaf(v[u][e], kLog2e, -m2));
   }
   for (; c < C; c += step) {
     float v[VEC];
@@ -400,9 +415,9 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
       s *= fast_exp2((m - cm) * kLog2e);
       m = cm;
     }
-    const ExpReference ref(m);
+    const float m2 = online_reference(m);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s += ref.weight(v[e]);
+    for (int e = 0; e < VEC; ++e) s += fast_exp2(fmaf(v[e], kLog2e, -m2));
   }
   float mm[1] = {m};
   block_allreduce<MaxOp, WG / kWave, 1>(mm, slots, phase);
@@ -410,9 +425,12 @@ __device__ __forceinline__ void stream_max_sum(const T* __restrict__ xr, int64_t
   // Threads that saw nothing have m == -inf and s == 0; (m - mm) would be nan only if the
   // whole row were empty, which C > 0 excludes.
   float ss[1] = {m == -INFINITY ? 0.f : s * fast_exp2((m - mm[0]) * kLog2e)};
+  base_out = row_base(mm[0]);
+  float no_dot;
+  if (__builtin_expect(base_out != 0.f, 0)) rebased_sums<T, WG, false>(xr, nullptr, C, base_out, ss[0], no_dot);
   block_allreduce<SumOp, WG / kWave, 1>(ss, slots, phase);
   phase ^= 1;
-  m_out = mm[0];
+  m_out = mm[0] - base_out;
   s_out = ss[0];
 }
 
@@ -429,7 +447,7 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
   const int64_t row = blockIdx.x;
   if (row >= N) return;
   const T* xr = logits + row * C;
-  float m, s;
+  float m, s, base;
   const float inv_rows = 1.0f / static_cast<float>(N);
   if constexpr (DENSE) {
     const T* yr = static_cast<const T*>(labels) + row * C;
@@ -454,10 +472,10 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
         ts *= fast_exp2((tm - cm) * kLog2e);
         tm = cm;
       }
-      const ExpReference ref(tm);
+      const float m2 = online_reference(tm);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        ts += ref.weight(v[e]);
+        ts += fast_exp2(fmaf(v[e], kLog2e, -m2));
         dot[0] += !ANY || c + e < C ? v[e] * y[e] : 0.f;
         dot[1] += y[e];
       }
@@ -466,25 +484,18 @@ __global__ __launch_bounds__(WG) void ce_fwd_stream_kernel(const T* __restrict__
     block_allreduce<MaxOp, WG / kWave, 1>(mm, slots, phase);
     phase ^= 1;
     float red[3] = {tm == -INFINITY ? 0.f : ts * fast_exp2((tm - mm[0]) * kLog2e), dot[0], dot[1]};
+    base = row_base(mm[0]);
+    if (__builtin_expect(base != 0.f, 0)) rebased_sums<T, WG, true>(xr, yr, C, base, red[0], red[1]);
     __shared__ float slots3[2 * 3 * (WG / kWave)];
     block_allreduce<SumOp, WG / kWave, 3>(red, slots3, 0);
-    m = mm[0];
+    m = mm[0] - base;
     s = red[0];
-    const float base = row_base(m);
-    if (__builtin_expect(base != 0.f, 0)) {  // (the sums of label * x are as large as the type: once more, from the base)
-      float again[1] = {0.f};
-      for (int64_t c = threadIdx.x; c < C; c += WG) again[0] += (to_float(xr[c]) - base) * to_float(yr[c]);
-      block_allreduce<SumOp, WG / kWave, 1>(again, slots, 0);
-      red[1] = again[0];
-      m = 0.f;
-    }
     if (threadIdx.x == 0) rowloss[row] = -(red[1] - (m + logf(s)) * red[2]) * inv_rows;
   } else {
-    stream_max_sum<T, VEC, WG, ONCE, ANY>(xr, C, slots, phase, m, s);
+    stream_max_sum<T, VEC, WG, ONCE, ANY>(xr, C, slots, phase, m, s, base);
     if (threadIdx.x == 0) {
       const int64_t id = load_id(labels, row, id64 != 0);
-      const float base = row_base(m);
-      rowloss[row] = (id < 0 || id >= C) ? NAN : -((to_float(xr[id]) - base) - ((m - base) + logf(s))) * inv_rows;
+      rowloss[row] = (id < 0 || id >= C) ? NAN : -((to_float(xr[id]) - base) - (m + logf(s))) * inv_rows;
     }
   }
 }
@@ -502,25 +513,26 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
   T* out_row = dlogits + row * C;
   const float inv_rows = 1.0f / static_cast<float>(N);
   const float scale = (upstream != nullptr ? to_float(upstream[0]) : 1.0f) * inv_rows;
-  float m, s;
-  stream_max_sum<T, VEC, WG, false, ANY>(xr, C, slots, phase, m, s);
-  const float base = row_base(m);
-  m -= base;
+  float m, s, base;
+  stream_max_sum<T, VEC, WG, false, ANY>(xr, C, slots, phase, m, s, base);
   const float m2 = m * kLog2e;
   const float inv_sum = 1.0f / s;
   const float shift = m + logf(s);
-  auto rebase = [&](float (&v)[VEC]) {
-    if (__builtin_expect(base != 0.f, 0)) {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] -= base;
-    }
-  };
   const int64_t id = DENSE ? 0 : load_id(labels, row, id64 != 0);
   float acc[1] = {0.f};
   constexpr int U = DENSE ? 1 : 4;  // integer labels: four chunks in flight per thread
   const int64_t step = static_cast<int64_t>(WG) * VEC;
   const int64_t whole = ANY ? C - C % VEC : C;  // where the last whole chunk ends
   int64_t c0 = static_cast<int64_t>(threadIdx.x) * VEC;
+  if (__builtin_expect(base != 0.f, 0)) {
+    for (int64_t c = threadIdx.x; c < C; c += WG) {
+      const float x = to_float(xr[c]) - base;
+      const float y = DENSE ? to_float((static_cast<const T*>(labels) + row * C)[c]) : c == id ? 1.f : 0.f;
+      if (y != 0.f) acc[0] += (x - shift) * y;
+      out_row[c] = from_float<T>((fast_exp2(x * kLog2e) * inv_sum - y) * scale);
+    }
+    c0 = C;
+  }
   auto put = [&](int64_t c, const float (&out)[VEC]) {
     if constexpr (!ANY) VecIO<T, VEC>::store(out_row + c, out);
     else if (c < whole) VecAny<T, VEC>::store(out_row + c, out);
@@ -538,7 +550,6 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
       for (int u = 0; u < U; ++u) {
         const int64_t c = c0 + u * step;
         float out[VEC];
-        rebase(v[u]);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           float p = fast_exp2(fmaf(v[u][e], kLog2e, -m2)) * inv_sum;
@@ -556,7 +567,6 @@ __global__ __launch_bounds__(WG) void ce_grad_stream_kernel(const T* __restrict_
     float v[VEC], out[VEC];
     if constexpr (ANY) stream_load<T, VEC>(xr, c, C, kMinusInfWord<T>, v);
     else VecIO<T, VEC>::load(xr + c, v);
-    rebase(v);
     if constexpr (DENSE) {
       const T* yr = static_cast<const T*>(labels) + row * C;
       float y[VEC];
