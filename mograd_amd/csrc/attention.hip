@@ -1,6 +1,8 @@
 // C ABI for flash attention: argument checks, routing between the 16-bit MFMA kernels (16-bit
 // storage, head dimension up to 256), the fp32 MFMA kernels (up to 256, or 128 where rows do not lie
 // on 16-byte chunks) and the general fp32 FMA kernels.
+#include <cmath>
+
 #include "attention_f32_mfma.h"
 #include "attention_f32_wave.h"
 #include "attention_generic.h"
@@ -152,10 +154,29 @@ static int fwd_f32_wave(const float* q, const float* k, const float* v, const fl
 }
 
 // Whether a grid holds both walks of a backward of `blocks` workgroups each: one has fewer than 2^32 threads.  (Heads of 32
-// rows and fewer: 2^23 of them are 1.2 GB a tensor at 8 rows of 4 columns.)  MOGRAD_HIP_ATTN_F32_BWD_TOGETHER overrides it.
-constexpr bool f32_wave_together(int64_t blocks) { return 2 * blocks * 256 < int64_t{1} << 32; }
-static_assert(f32_wave_together((int64_t{1} << 23) - 1) && !f32_wave_together(int64_t{1} << 23) && !f32_wave_together(int64_t{1} << 31),
+// rows and fewer: 2^23 of them are 1.2 GB a tensor at 8 rows of 4 columns.)
+constexpr bool f32_wave_one_grid(int64_t blocks) { return 2 * blocks * 256 < int64_t{1} << 32; }
+static_assert(f32_wave_one_grid((int64_t{1} << 23) - 1) && !f32_wave_one_grid(int64_t{1} << 23) && !f32_wave_one_grid(int64_t{1} << 31),
               "grids of fewer than 2^32 threads");
+
+// Whether both walks of a backward go out together.  Together they fill each other's last rounds of workgroups; apart dQ has a
+// second workgroup per CU where its registers allow that (up to 64 columns, up to 80 without a bias) and delta is formed once.
+// So heads of 33 to 80 columns of equal walks go apart where a walk's last round is more than half full, or rounds are many, and
+// those of more than 128, whose waves all form delta's sum, from 0.6 rounds on.  us together | apart | start of it all, from 700
+// shapes: (13, 549, 5 heads, 64) 265 | 233, 4.6 rounds; (2, 1024, 8, 64), bias, 171 | 156, 2.0; (11, 653, 3, 64) 187 | 168, 2.7;
+// (22, 257, 15, 80), causal, 372 | 332, 11.6; (28, 64, 13, 80), causal, 67 | 60, 2.8; (11, 321, 6, 256) 404 | 378, 2.8; but
+// (3, 777, 8, 80), bias, 244 | 281, 2.3; 1.1 rounds of 64 columns 1.23 times as long apart, half a round 1.6 times; up to 32
+// columns never, 81 to 128 columns 0.97 to 1.3 times.  This choice takes 0.2 % more time than the better of the two for each,
+// together always 1.2 %, apart 11 %.  MOGRAD_HIP_ATTN_F32_BWD_TOGETHER = 0 | 1 overrides it.
+static bool f32_wave_together(const AttnDims& a, bool causal, bool has_bias, int64_t blocks) {
+  const int64_t tiles = ceil_div(a.S, 32);
+  const double rounds = static_cast<double>(blocks) / device_info().cu_count, idle = std::ceil(rounds) - rounds;
+  const bool dq_pairs = a.D > 32 && a.D <= (has_bias ? 64 : 80);
+  bool apart = false;
+  if (dq_pairs) apart = rounds > 4.0 || ((!causal || tiles <= 4) && rounds > 1.0 && idle < 0.48);
+  else if (a.D > 128) apart = !causal && (rounds > 4.0 || (tiles >= 8 && rounds > 0.6 && idle < 0.48));
+  return !apart && f32_wave_one_grid(blocks);
+}
 
 static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const float* k, const float* v, const float* mask,
                         const float* lse, float* dq, float* dk, float* dv, const AttnDims& a, float scale, bool causal,
@@ -163,26 +184,27 @@ static int bwd_f32_wave(const float* d_o, const float* o, const float* q, const 
   const int tiles = static_cast<int>(ceil_div(a.S, 32));
   const int64_t heads = static_cast<int64_t>(a.B) * a.H;
   const int64_t blocks = f32_wave_grid(heads, tiles, f32_wave_own_tiles(a, causal));
-  const bool together = env_int("MOGRAD_HIP_ATTN_F32_BWD_TOGETHER", f32_wave_together(blocks)) != 0;
+  const bool together = env_int("MOGRAD_HIP_ATTN_F32_BWD_TOGETHER", f32_wave_together(a, causal, has_bias, blocks)) != 0;
   Scratch delta;
-  if (a.D > 96 && a.D <= 128) {
-    static_assert(f32_wave_delta_given<128>() && !f32_wave_delta_given<96>() && !f32_wave_delta_given<64>(), "who is handed delta");
-    const int64_t rows = heads * a.S;
-    MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
-    hipLaunchKernelGGL((attn_delta_kernel<float>), attn_delta_grid(rows), dim3(256), 0, stream, d_o, o,
-                       delta.as<float>(), rows, a.D, a.S, a.H, a.o_bshd);
-  }
+  const int64_t rows = heads * a.S;
+  static_assert(f32_wave_delta_given<128>() && !f32_wave_delta_given<96>() && !f32_wave_delta_given<64>(), "who is handed delta");
+  if (!together || (a.D > 96 && a.D <= 128)) MG_TRY(delta.take(rows * static_cast<int64_t>(sizeof(float))));
   f32_wave_pick(a, causal, has_bias, [&](auto dp, auto mode, auto c, auto hb) {
-    auto launch = [&](int64_t grid, int64_t dkdv_blocks) {
-      hipLaunchKernelGGL((attn_bwd_f32_wave_kernel<decltype(dp)::value, decltype(mode)::value, decltype(c)::value, decltype(hb)::value>),
-                         dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, d_o, o, q, k, v, mask, lse,
-                         delta.as<float>(), dq, dk, dv, a, scale, tiles, static_cast<int>(dkdv_blocks));
-    };
+    constexpr int DP = decltype(dp)::value;
+    constexpr F32WaveMode MODE = decltype(mode)::value;
+    constexpr bool CAUSAL = decltype(c)::value, HAS_BIAS = decltype(hb)::value;
     if (together) {
-      launch(2 * blocks, blocks);
+      if (f32_wave_delta_given<DP>())
+        hipLaunchKernelGGL((attn_delta_kernel<float>), attn_delta_grid(rows), dim3(256), 0, stream, d_o, o, delta.as<float>(), rows, a.D,
+                           a.S, a.H, a.o_bshd);
+      hipLaunchKernelGGL((attn_bwd_f32_wave_kernel<DP, MODE, CAUSAL, HAS_BIAS>), dim3(static_cast<unsigned>(2 * blocks)), dim3(256), 0,
+                         stream, d_o, o, q, k, v, mask, lse, delta.as<float>(), dq, dk, dv, a, scale, tiles, static_cast<int>(blocks));
     } else {
-      launch(blocks, blocks);
-      launch(blocks, 0);
+      const dim3 grid(static_cast<unsigned>(blocks));
+      hipLaunchKernelGGL((attn_dq_f32_wave_kernel<DP, MODE, CAUSAL, HAS_BIAS>), grid, dim3(256), 0, stream, d_o, o, q, k, v, mask, lse,
+                         delta.as<float>(), dq, a, scale, tiles);
+      hipLaunchKernelGGL((attn_dkdv_f32_wave_kernel<DP, MODE, CAUSAL, HAS_BIAS>), grid, dim3(256), 0, stream, d_o, q, k, v, mask, lse,
+                         delta.as<float>(), dk, dv, a, scale, tiles);
     }
   });
   MG_LAUNCH_CHECK();

@@ -15,10 +15,9 @@
 //     (3, 777, 8 heads, 80), bias        645 -> 381 -> 336 us      (1, 1236, 6, 256), causal  3930 -> 520 -> 406 us
 //     (1, 500, 2 heads, 64), bias               66 ->  46 us       (2, 8 heads of 1500, 128)   816 -> 782 -> 777 us
 //     (4, 32, 2, 32), causal              65 ->  18 ->  12 us      (21, 79, 8, 32), causal      35 ->  28 ->  27 us
-// The backward is one launch: two walks of 600 workgroups end in two rounds of which a third is empty, five rounds
-// of both together in one, and a short sequence waits for one kernel instead of two.  (Walks of whole rounds have
-// nothing to gain by it and a little to lose, dQ's second workgroup per CU where it had one: (2, 8 heads of 1024, 64), bias,
-// 204 -> 211; (32, 200, 12, 80) 333 -> 340; dQ with a launch of its own there, 336, was not worth its kernels.)  The arithmetic is the matrix pipe's: 64 cycles per 32 x 32 x 2 product, two
+// Where the walks have little to gain from each other's company, each has a launch (f32_wave_together has the choice): two
+// walks of 600 workgroups end in two rounds of which a third is empty, five rounds of both together in one, and a short sequence
+// waits for one kernel instead of two, but walks of whole rounds lose dQ's second workgroup per CU.  The arithmetic is the matrix pipe's: 64 cycles per 32 x 32 x 2 product, two
 // products per column and step forward, seven over the two backward kernels.  What stands beside it on the one
 // wave of a SIMD is vector arithmetic, 1300 instructions a step at 80 columns until the copies took a scalar base
 // and a byte offset per lane, the bias' places were computed once, and exp2f became the one instruction:
@@ -588,12 +587,12 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) v
   }
 }
 
-// dQ.  `lds` holds f32_wave_lds<DP, MODE, HAS_BIAS>(2) bytes.
+// dQ, and where `delta` is not null the rows' delta.  `lds` holds f32_wave_lds<DP, MODE, HAS_BIAS>(2) bytes.
 template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
 __device__ __forceinline__ void attn_dq_f32_wave_block(
     int block, char* lds, const float* __restrict__ d_o, const float* __restrict__ o, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ mask, const float* __restrict__ lse,
-    float* __restrict__ dq, const AttnDims& a, float scale, int tiles) {
+    float* __restrict__ delta, float* __restrict__ dq, const AttnDims& a, float scale, int tiles) {
   using W = F32Wave<DP>;
   constexpr int NI = W::NI, NM = HAS_BIAS ? 16 : 0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (known to be one value per wave)
@@ -650,6 +649,7 @@ __device__ __forceinline__ void attn_dq_f32_wave_block(
     dl = (part[lane % 32] + part[32 + lane % 32]) + (part[64 + lane % 32] + part[96 + lane % 32]);
     __syncthreads();
   }
+  if (delta != nullptr && row_ok && (MODE == kF32OwnTiles || wave == 0) && half == 0) delta[static_cast<int64_t>(bh) * a.S + i] = dl;
 #pragma unroll
   for (int c = 0; c < DP / 2; ++c) asm volatile("" : "+v"(qr[c]), "+v"(dor[c]));  // their wait stands here
   asm volatile("" : "+v"(lse2));
@@ -717,7 +717,7 @@ __device__ __forceinline__ void attn_dq_f32_wave_block(
 // dK, dV: the workgroup's keys along the lanes, the streamed queries along the registers.  delta = rowsum(dO * O) of the
 // streamed rows is formed here as in dQ, from the dO tile that the products with V read anyway and O's rows in registers, so
 // that neither walk waits for the other (at 128 columns those registers are taken: `delta` has it, from a launch of its own).
-template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
+template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS, bool GIVEN>
 __device__ __forceinline__ void attn_dkdv_f32_wave_block(
     int block, char* lds, float (*stats)[4][64], const float* __restrict__ d_o, const float* __restrict__ o,
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ mask,
@@ -758,7 +758,6 @@ __device__ __forceinline__ void attn_dkdv_f32_wave_block(
     if constexpr (HAS_BIAS) mt_copies.copy(mhead, min(t, steps - 1) * 32, r0, a.S, m_s, lane);
   };
   // O's row (or its delta) and the LSE of streamed row lane % 32, requested a step ahead.
-  constexpr bool GIVEN = f32_wave_delta_given<DP>();
   const float* delta_h = delta + static_cast<int64_t>(bh) * a.S;
   float4 orow[DP / 8];
   float lse_i, dl_i;
@@ -835,7 +834,7 @@ __device__ __forceinline__ void attn_dkdv_f32_wave_block(
     for (int g = 0; g < 4; ++g) {
       const int rr = g * 8 + half * 4;
       float4 d4 = *reinterpret_cast<const float4*>(st + 32 + rr);
-      if constexpr (DSPLIT) {  // each wave has its columns' share
+      if constexpr (DSPLIT && !GIVEN) {  // each wave has its columns' share
         float4 w4[4];
 #pragma unroll
         for (int w = 0; w < 4; ++w) w4[w] = *reinterpret_cast<const float4*>(stats[t & 1][w] + 32 + rr);
@@ -868,8 +867,7 @@ __device__ __forceinline__ void attn_dkdv_f32_wave_block(
   }
 }
 
-// Both walks in one launch: workgroups [0, blocks) take dK and dV, whose steps are the longer ones, the rest dQ.  A grid of
-// `blocks` is dK and dV alone, one with `blocks` = 0 dQ.
+// Both walks in one launch: workgroups [0, blocks) take dK and dV, whose steps are the longer ones, the rest dQ.
 template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
 __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) void attn_bwd_f32_wave_kernel(
     const float* __restrict__ d_o, const float* __restrict__ o, const float* __restrict__ q, const float* __restrict__ k,
@@ -878,9 +876,29 @@ __global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) v
   __shared__ __attribute__((aligned(1024))) char lds[f32_wave_lds<DP, MODE, HAS_BIAS>(2)];
   __shared__ __attribute__((aligned(256))) float stats[MODE == kF32SplitColumns ? 2 : 1][4][64];
   if (static_cast<int>(blockIdx.x) < blocks)
-    attn_dkdv_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS>(blockIdx.x, lds, stats, d_o, o, q, k, v, mask, lse, delta, dk, dv, a, scale, tiles);
+    attn_dkdv_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS, f32_wave_delta_given<DP>()>(blockIdx.x, lds, stats, d_o, o, q, k, v, mask, lse, delta, dk, dv, a, scale, tiles);
   else
-    attn_dq_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS>(blockIdx.x - blocks, lds, d_o, o, q, k, v, mask, lse, dq, a, scale, tiles);
+    attn_dq_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS>(blockIdx.x - blocks, lds, d_o, o, q, k, v, mask, lse, nullptr, dq, a, scale, tiles);
+}
+
+// A launch for each walk: dQ, which leaves delta behind, and then dK and dV.
+template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
+__global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(1))) void attn_dq_f32_wave_kernel(
+    const float* __restrict__ d_o, const float* __restrict__ o, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, const float* __restrict__ mask, const float* __restrict__ lse, float* __restrict__ delta,
+    float* __restrict__ dq, AttnDims a, float scale, int tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[f32_wave_lds<DP, MODE, HAS_BIAS>(2)];
+  attn_dq_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS>(blockIdx.x, lds, d_o, o, q, k, v, mask, lse, delta, dq, a, scale, tiles);
+}
+template <int DP, F32WaveMode MODE, bool CAUSAL, bool HAS_BIAS>
+__global__ __launch_bounds__(256, (f32_wave_occupancy<DP, MODE, HAS_BIAS>(2))) void attn_dkdv_f32_wave_kernel(
+    const float* __restrict__ d_o, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    const float* __restrict__ mask, const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dk,
+    float* __restrict__ dv, AttnDims a, float scale, int tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[f32_wave_lds<DP, MODE, HAS_BIAS>(2)];
+  __shared__ __attribute__((aligned(256))) float stats[MODE == kF32SplitColumns ? 2 : 1][4][64];
+  attn_dkdv_f32_wave_block<DP, MODE, CAUSAL, HAS_BIAS, true>(blockIdx.x, lds, stats, d_o, nullptr, q, k, v, mask, lse, delta, dk, dv, a,
+                                                             scale, tiles);
 }
 
 }  // namespace mg
