@@ -162,7 +162,7 @@ static_assert(f32_wave_one_grid((int64_t{1} << 23) - 1) && !f32_wave_one_grid(in
 // Whether both walks of a backward go out together.  Together they fill each other's last rounds of workgroups; apart dQ has a
 // second workgroup per CU where its registers allow that (up to 64 columns, up to 80 without a bias) and delta is formed once.
 // So heads of 33 to 80 columns of equal walks go apart where a walk's last round is more than half full, or rounds are many, and
-// those of more than 128, whose waves all form delta's sum, from 0.6 rounds on.  us together | apart | start of it all, from 700
+// those of more than 128, whose waves all form delta's sum, from 0.6 rounds on.  us together | apart, from 700
 // shapes: (13, 549, 5 heads, 64) 265 | 233, 4.6 rounds; (2, 1024, 8, 64), bias, 171 | 156, 2.0; (11, 653, 3, 64) 187 | 168, 2.7;
 // (22, 257, 15, 80), causal, 372 | 332, 11.6; (28, 64, 13, 80), causal, 67 | 60, 2.8; (11, 321, 6, 256) 404 | 378, 2.8; but
 // (3, 777, 8, 80), bias, 244 | 281, 2.3; 1.1 rounds of 64 columns 1.23 times as long apart, half a round 1.6 times; up to 32

@@ -431,14 +431,32 @@ struct LayerNormOps {
   // element was 317 / 64 loads of two bytes per lane and row, and rows past 4096 columns had no backward at all.  Forward +
   // backward, us: (23721, 317) fp16 100 -> 33, fp32 66 -> 38; (9000, 4095) bf16 199 -> 97; (1000, 799) fp16 16.2 -> 15.8.
   // Few rows stay with an element per thread, whose walk over a row is shorter where each has a workgroup to itself, and so do
-  // rows of up to 64 columns, of whose sixteen lanes most would be idle; us, by elements | in chunks: fp16 (193, 554) 11.0 | 13.1,
-  // (193, 1501) 13.0 | 16.9, (600, 2503) 22.1 | 25.2, (2000, 301) 15.5 | 16.7; (2000, 554) 18.8 | 18.2, (2000, 2503) 44.1 | 37.1; fp32
-  // (193, 777) 10.4 | 13.0, (2000, 301) 14.3 | 15.8, (2000, 777) 19.3 | 18.6.  (By elements there is no backward past 4096 columns.)
+  // rows of up to 64 columns, of whose sixteen lanes most would be idle.  Between the two the better one changes with how many
+  // lanes and workgroups a row's chunks, or its elements, come to.  us by elements | in chunks, 16 bits: forward (1286, 1759)
+  // 5.7 | 7.2, (5225, 1862) 15.9 | 12.9; backward (1286, 1759) 15.3 | 21.4, (9480, 209) 12.7 | 16.2, (47891, 238) 44 | 31, (1041, 2555)
+  // 20.1 | 23.9; fp32: forward (45738, 198) 14.0 | 17.2, (4700, 355) 5.8 | 5.5; backward (2552, 1318) 18.0 | 20.7, given the statistics
+  // 15.9 | 20.2.  Over 1200 sizes of up to 4095 columns the choice takes 1 % (forward) and 2 % (backward) more time than the better
+  // of the two for each, always elements 21 to 26 %.  (By elements there is no backward past 4096 columns.)
   // MOGRAD_HIP_LN_CHUNKS = 0 | 1 overrides the choice where either can be had.
-  static bool in_chunks(int64_t rows, int64_t cols) {
+  enum Pass { kForward, kBackward, kBackwardOfStats };
+  static bool in_chunks(Pass pass, int64_t rows, int64_t cols) {
     if (cols > 4096) return true;
     if (const char* const force = env_str("MOGRAD_HIP_LN_CHUNKS")) return force[0] != '0' && cols >= WIDE;
-    return cols > 64 && rows >= 1024 && rows * cols >= int64_t{1} << 20;
+    if (cols <= 64 || rows < 1024 || rows * cols < int64_t{1} << 20) return false;
+    const int64_t chunks = ceil_div(cols, WIDE);
+    if (WIDE == 8) {
+      if (pass == kForward) {
+        if (chunks > 64 && chunks <= 128) return rows >= 2048;
+        return (chunks <= 32 || (chunks > 48 && chunks <= 64) || chunks > 256) || rows >= 4096;
+      }
+      if (chunks > 16 && chunks <= 32) return rows < 8192 || rows >= 24576;
+      return chunks <= 128 || rows >= (chunks <= 256 ? 4096 : 1536);
+    }
+    if (chunks <= 32) return true;
+    if (chunks <= 64) return pass == kForward && chunks <= 48 && rows >= 16384 && rows < 49152;
+    if (chunks <= 256) return rows >= (chunks <= 128 ? 4096 : 2048);
+    if (chunks > 512 || pass == kForward) return true;
+    return pass == kBackward && rows >= 3300 && rows < 22000;
   }
 
   // How a row of `chunks` chunks is laid over threads.
@@ -526,9 +544,10 @@ struct LayerNormOps {
     Shape s;
     if (can_vectorise(cols, {x, gamma, beta, y}) && pick_shape(cols / WIDE, &s))
       return dispatch_fwd<WIDE>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
-    if (in_chunks(rows, cols) && pick_shape(ceil_div(cols, WIDE), &s))
+    const bool chunks = in_chunks(kForward, rows, cols);
+    if (chunks && pick_shape(ceil_div(cols, WIDE), &s))
       return dispatch_fwd<WIDE, true>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
-    if (!in_chunks(rows, cols) && pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
+    if (!chunks && pick_shape(cols, &s)) return dispatch_fwd<1>(s, x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);
     hipLaunchKernelGGL((ln_fwd_stream_kernel<T, 1024>), dim3(static_cast<unsigned>(rows)), dim3(1024), 0, stream, x,
                        gamma, beta, y, mean, rstd, rows, cols, eps);
     MG_LAUNCH_CHECK();
@@ -671,10 +690,11 @@ struct LayerNormOps {
     if (can_vectorise(cols, {dy, x, gamma, dx, residual}) && pick_shape_bwd(cols / WIDE, &s) && fits(s, WIDE))
       return dispatch_bwd<WIDE, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
                                            stream);
-    if (in_chunks(rows, cols) && pick_shape_bwd(ceil_div(cols, WIDE), &s) && fits(s, WIDE))
+    const bool chunks = in_chunks(HAS_STATS ? kBackwardOfStats : kBackward, rows, cols);
+    if (chunks && pick_shape_bwd(ceil_div(cols, WIDE), &s) && fits(s, WIDE))
       return dispatch_bwd<WIDE, HAS_STATS, true>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps,
                                                  stream);
-    if (!in_chunks(rows, cols) && pick_shape_bwd(cols, &s) && fits(s, 1))
+    if (!chunks && pick_shape_bwd(cols, &s) && fits(s, 1))
       return dispatch_bwd<1, HAS_STATS>(s, dy, x, gamma, mean, rstd, residual, dx, dgamma, dbeta, rows, cols, eps, stream);
     if (residual == nullptr)
       return bwd_stream<HAS_STATS>(dy, x, gamma, mean, rstd, dx, dgamma, dbeta, rows, cols, eps, stream);
