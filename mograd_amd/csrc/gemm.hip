@@ -452,6 +452,23 @@ static int dispatch_f32(const GemmArgs& g_in, hipStream_t stream, bool* handled)
 #undef MG_F32_PIPE
 }
 
+// Two k-contiguous 16-bit operands off the 16-byte chunks, in us: in place in 64 x 64 tiles that are staged through registers
+// (0.43 us a step where a workgroup has its CU, 0.35 for each of several), and in the ragged variant's 128 x 128 ones.  From 1500
+// products of 16 to 32768 rows and up to 8192 columns and K, within a tenth for most.
+static double any_16bit_us(const GemmArgs& g, int splits, double cus) {
+  const double tiles = static_cast<double>(g.batch * ceil_div(g.M, kSmallT) * ceil_div(g.N, kSmallT)) * splits, rounds = std::ceil(tiles / cus);
+  return 3.4 + static_cast<double>(g.batch * g.M * g.N) / 2.5e6 + std::ceil(static_cast<double>(g.K) / kG16BK / splits) * (rounds == 1 ? 0.43 : 0.35 * rounds) +
+         (splits > 1 ? partials_us(tiles * kSmallT * kSmallT) : 0.0);
+}
+static double ragged_16bit_us(const GemmArgs& g, double cus) {
+  const int64_t tiles = g.batch * ceil_div(g.M, kGemmBM) * ceil_div(g.N, kGemmBN);
+  int splits = splitk_16bit_splits(tiles, g.K, 2);
+  const int k_per_split = splitk_16bit_range(g.K, &splits);
+  const double items = static_cast<double>(tiles) * splits, per_cu = std::ceil(items / cus), pairs = std::floor(per_cu / 2), odd = per_cu - 2 * pairs;
+  return 7.3 + static_cast<double>(g.batch * g.M * g.N) / 2.5e6 + k_per_split / kG16BK * (1.44 * pairs + (pairs == 0 ? 1.0 : 0.64) * odd) +
+         (splits > 1 ? items * kGemmBM * kGemmBN * 5.0 / 3.5e6 : 0.0);
+}
+
 template <typename T>
 static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handled) {
   *handled = false;
@@ -487,7 +504,10 @@ static int dispatch_16bit(const GemmArgs& g_in, hipStream_t stream, bool* handle
     // (Up to three tiles to a CU: (700, 4400 <- 77) 8.8 | 8.3, 759 tiles; (1000, 4000 <- 141) 10.0 | 10.8, 1008; (966, 5920 <- 141)
     // 12.5 | 15.8, 1488.)
     const bool few = g.batch * ceil_div(g.M, 64) * ceil_div(g.N, 64) <= 3 * static_cast<int64_t>(device_info().cu_count);
-    if (pipe == 64 || (few && 1.35 * small.us <= choose_16bit(g.M, g.N, g.K, g.batch, false).us + 7.0)) {
+    // (Long K in few tiles: the ragged variant's K ranges, (211, 2613 <- 4293) 23.7 | 33.9, (4430, 105 <- 3721) 23.0 | 30.2.)
+    const double cus = device_info().cu_count;
+    const bool ragged = a_kc && b_kc && !copy_pays && any_16bit_us(g, small.splits, cus) > ragged_16bit_us(g, cus);
+    if (pipe == 64 || (few && !ragged && 1.35 * small.us <= choose_16bit(g.M, g.N, g.K, g.batch, false).us + 7.0)) {
       if (a_kc && b_kc) return launch_16bit_small<T, true, true, true>(g, small.splits, stream);
       if (a_kc) return launch_16bit_small<T, true, false, true>(g, small.splits, stream);
       if (b_kc) return launch_16bit_small<T, false, true, true>(g, small.splits, stream);
