@@ -653,13 +653,13 @@ __global__ __launch_bounds__(WG) void ce_strided_kernel(const T* __restrict__ lo
   }
 }
 
-// loss[0] = sum of the N per-row terms, one workgroup, fixed order (no atomics).  It waits for memory, so sixteen terms are in
-// flight to a thread (one after the other, 16384 rows took 5.7 us; so 4.7, of which a launch of one workgroup is half).
-template <typename T>
+// loss[0] = sum of the N per-row terms, one workgroup, fixed order (no atomics).  It waits for memory, so U terms are in flight to
+// a thread: one after the other, 16384 rows took 5.7 us, with sixteen 4.7, of which a launch of one workgroup is half.  Up to 2048
+// rows the shorter code with one is faster, by 0.7 us at 300 and at 760.
+template <typename T, int U>
 __global__ __launch_bounds__(1024) void sum_rows_kernel(const float* __restrict__ rowloss, T* __restrict__ loss, int64_t N) {
   __shared__ float slots[2 * 16];
   float acc[1] = {0.f};
-  constexpr int U = 16;
   for (int64_t first = 0; first < N; first += U * 1024) {
     float v[U];
 #pragma unroll
@@ -788,7 +788,9 @@ struct CrossEntropyOps {
   }
 
   static int finish_loss(const float* rowloss, T* loss, int64_t N, hipStream_t stream) {
-    hipLaunchKernelGGL((sum_rows_kernel<T>), dim3(1), dim3(1024), 0, stream, rowloss, loss, N);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, stream, rowloss, loss, N); };
+    if (env_int("MOGRAD_HIP_CE_SUM_DEEP", N > 2048) != 0) launch(sum_rows_kernel<T, 16>);
+    else launch(sum_rows_kernel<T, 1>);
     MG_LAUNCH_CHECK();
     return MG_OK;
   }
@@ -825,7 +827,8 @@ struct CrossEntropyOps {
       else if (wide)
         hipLaunchKernelGGL((ce_fwd_stream_kernel<T, WIDE, SWG, DENSE>), dim3(static_cast<unsigned>(N)), dim3(SWG), 0,
                            stream, logits, labels, rowloss, N, C, id64);
-      else if (any)
+      // (rows of fewer elements than the workgroup has threads: one each; chunks were up to 23 % slower, (16239, 65) bf16 dense 12.8 us | 15.7)
+      else if (any && env_int("MOGRAD_HIP_CE_LOSS_CHUNKS", C >= 256) != 0)
         hipLaunchKernelGGL((ce_fwd_stream_kernel<T, WIDE, 256, DENSE, false, true>), dim3(static_cast<unsigned>(N)), dim3(256),
                            0, stream, logits, labels, rowloss, N, C, id64);
       else

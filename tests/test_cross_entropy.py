@@ -389,6 +389,24 @@ def test_a_row_of_the_types_last_values(device, dtype, half_ulp, size, end, Cc, 
             assert (np.abs(got.to_numpy()[start:].reshape(N, Cc) - exact) <= bound).all()
 
 
+@pytest.mark.parametrize("deep", ["0", "1"])
+@pytest.mark.parametrize("chunks", ["0", "1"])
+@pytest.mark.parametrize("N", [1, 1024, 1025, 2048, 2049, 16385, 40000])
+def test_sum_of_the_rows(device, monkeypatch, deep, chunks, N):
+    # One term after the other or sixteen at a time to a thread; rows off the 16-byte chunks by elements or in chunks.
+    monkeypatch.setenv("MOGRAD_HIP_CE_SUM_DEEP", deep)
+    monkeypatch.setenv("MOGRAD_HIP_CE_LOSS_CHUNKS", chunks)
+    lib, st, Cc = device.lib, device.stream, 7
+    x = normal(39, 0, (N, Cc), std=2.0)
+    ids = (np.arange(N) * 5) % Cc
+    bx, bi, loss = AnyBuffer.from_numpy(device, x, F32), AnyBuffer.from_numpy(device, ids.astype(np.int32), I32), AnyBuffer.create(F32, device, 1)
+    lib.mg_cross_entropy_ids(bx.data_ptr(), bi.data_ptr(), loss.data_ptr(), N, Cc, F32, I32, st)
+    x64 = x.astype(np.float64)
+    want = (np.log(np.exp(x64).sum(-1)) - x64[np.arange(N), ids]).mean()
+    # each term is off by 2^-20 of its size, their sum in 1024 shares by 2^-24 a term of a share
+    assert abs(loss.item() - want) <= (2.0 ** -20 + 2.0 ** -24 * (N / 1024 + 16)) * np.abs(x64).max()
+
+
 def test_out_of_range_id_flags_loss(device):
     x = normal(34, 0, (4, 100))
     ids = np.array([0, 5, 100, 7], np.int32)
