@@ -4,7 +4,7 @@
 //
 // What bounds few heads is not a rate but the walk of one workgroup: at (3, 1755, 2 heads, 64), causal, 84 workgroups of 128
 // queries walk up to 28 blocks of 64 keys one after the other, and the backward walks behind a launch of its own
-// that forms delta.  Here four times the workgroups walk an eighth as far each, no barrier stands in the walk (a wave's tiles are
+// that forms delta.  Here four times the workgroups walk a quarter as far each, no barrier stands in the walk (a wave's tiles are
 // copied into LDS of its own and waited for with its own counter), and both backward walks are one launch: dK/dV forms delta =
 // rowsum(dO * O) of its streamed rows from the dO fragments it multiplies anyway.  The price is that no wave's copy serves
 // another, four times the bytes from L2, so larger grids keep the kernels of attention_mfma.hip.

@@ -207,7 +207,10 @@ HALF_SHAPES = [(2, 2, 96, 64), (1, 3, 200, 64), (2, 1, 128, 128), (1, 2, 257, 32
 @pytest.mark.parametrize("dtype,budget_fwd,budget_bwd", [(F16, 2e-3, 8e-3), (BF16, 1.6e-2, 6.4e-2)])
 @pytest.mark.parametrize("name,causal,with_mask", MODES)
 @pytest.mark.parametrize("B,H,S,D", HALF_SHAPES)
-def test_half_error_budget(device, dtype, budget_fwd, budget_bwd, name, causal, with_mask, B, H, S, D):
+@pytest.mark.parametrize("wave16", [None, "0"])  # as few heads go, and the 128-row kernels, which larger grids take
+def test_half_error_budget(device, monkeypatch, dtype, budget_fwd, budget_bwd, name, causal, with_mask, B, H, S, D, wave16):
+    if wave16:
+        monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", wave16)
     # fp16: the reference's budget for its tensor-core backward is 8e-3 abs at S96
     # (tests/kernels/attention/mma.mojo:424); bf16 has 3 fewer mantissa bits: x8.
     q, k, v, do, m = _inputs(51, B, S, H, D, dtype, with_mask)
@@ -224,18 +227,22 @@ def test_half_error_budget(device, dtype, budget_fwd, budget_bwd, name, causal, 
         assert err <= budget_bwd * grow, f"{what}: {err}"
 
 
-@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("name,causal,with_mask", MODES)
 @pytest.mark.parametrize("D", [64, 128, 256])
-def test_long_ragged_sequence(device, causal, D):
-    # Past 1024 tokens the head-dim-64 backward launches its dK/dV and dQ walks separately
-    # (one launch below that); 1100 is not a multiple of any tile.  Head dims 128 and 256: the
-    # unpipelined walks, at 256 with the head dimension of the gradients split over two workgroups.
-    B, H, S = 1, 2, 1100
-    q, k, v, do, _ = _inputs(56, B, S, H, D, BF16, False)
-    o, lse, dq, dk, dv = _fwd_bwd(device, q, k, v, do, None, causal, dtype=BF16)
-    ro, rl = O.sdpa_fwd(q, k, v, None, causal)
+@pytest.mark.parametrize("wave16", [None, "0"])
+def test_long_ragged_sequence(device, monkeypatch, name, causal, with_mask, D, wave16):
+    # 1100 (with a bias 530) is not a multiple of any tile.  These few heads go to the 32-row workgroups up to 128 columns; kept
+    # from them, past 1024 tokens the head-dim-64 backward launches its dK/dV and dQ walks separately (one launch below that), and
+    # 128 columns, 256 and a bias take the unpipelined walks, 256 with the head dimension of the gradients split over two
+    # workgroups.
+    if wave16:
+        monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", wave16)
+    B, H, S = (2, 2, 530) if with_mask else (1, 2, 1100)
+    q, k, v, do, m = _inputs(56, B, S, H, D, BF16, with_mask)
+    o, lse, dq, dk, dv = _fwd_bwd(device, q, k, v, do, m, causal, dtype=BF16)
+    ro, rl = O.sdpa_fwd(q, k, v, m, causal)
     assert _max_err(o, ro) <= 1.6e-2 and _max_err(lse, rl) <= 1e-3 * max(1.0, float(np.abs(rl).max()))
-    for got, want, what in zip((dq, dk, dv), O.sdpa_bwd(q, k, v, do, None, causal), ("dq", "dk", "dv")):
+    for got, want, what in zip((dq, dk, dv), O.sdpa_bwd(q, k, v, do, m, causal), ("dq", "dk", "dv")):
         assert_attn_grad_close(got, want, what)
 
 
@@ -500,10 +507,22 @@ def test_errors(device):
         lib.mg_flash_attn_fwd(p, p, p, p, p, p, 1, 2, 1, 8, 1.0, 0, 0, R.int64, st)
 
 
-@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+# As these few heads go, and through the 128-row kernels' walks behind a launch for delta, whose rows of two a thread end
+# inside a thread's second one at 1200 rows of 64 columns and at 786 of 128.
+LAYOUT_ROUTES = [(F32, None), (F16, None), (BF16, None), (F16, "0"), (BF16, "0")]
+
+
+def _take_layout_route(monkeypatch, wave16):
+    if wave16:
+        monkeypatch.setenv("MOGRAD_HIP_ATTN_WAVE16", wave16)
+        monkeypatch.setenv("MOGRAD_HIP_ATTN_RESIDENT", "0")
+
+
+@pytest.mark.parametrize("dtype,wave16", LAYOUT_ROUTES)
 @pytest.mark.parametrize("name,causal,with_mask", MODES)
-@pytest.mark.parametrize("B,H,S,D", [(2, 3, 200, 64), (1, 2, 130, 72), (2, 2, 96, 128), (1, 1, 4, 8), (1, 2, 77, 40)])
-def test_bshd_output_forms_equal_the_standard_forms(device, dtype, name, causal, with_mask, B, H, S, D):
+@pytest.mark.parametrize("B,H,S,D", [(2, 3, 200, 64), (1, 2, 130, 72), (2, 2, 96, 128), (1, 1, 4, 8), (1, 2, 77, 40), (2, 3, 131, 128)])
+def test_bshd_output_forms_equal_the_standard_forms(device, monkeypatch, dtype, wave16, name, causal, with_mask, B, H, S, D):
+    _take_layout_route(monkeypatch, wave16)
     # O written and dO/O read as (B,S,H,D): bit for bit the standard entry points with the
     # (B,H,S,D) <-> (B,S,H,D) copies done on the host.  LSE stays (B,H,S).
     lib, st = device.lib, device.stream
@@ -530,10 +549,11 @@ def test_bshd_output_forms_equal_the_standard_forms(device, dtype, name, causal,
         np.testing.assert_array_equal(b.to_numpy(), a.to_numpy(), err_msg=what)
 
 
-@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("dtype,wave16", LAYOUT_ROUTES)
 @pytest.mark.parametrize("name,causal,with_mask", MODES)
-@pytest.mark.parametrize("B,H,S,D", [(2, 3, 200, 64), (1, 2, 130, 72), (2, 2, 96, 128), (1, 1, 4, 8), (1, 2, 77, 40)])
-def test_packed_qkv_forms_equal_the_separate_forms(device, dtype, name, causal, with_mask, B, H, S, D):
+@pytest.mark.parametrize("B,H,S,D", [(2, 3, 200, 64), (1, 2, 130, 72), (2, 2, 96, 128), (1, 1, 4, 8), (1, 2, 77, 40), (2, 3, 131, 128)])
+def test_packed_qkv_forms_equal_the_separate_forms(device, monkeypatch, dtype, wave16, name, causal, with_mask, B, H, S, D):
+    _take_layout_route(monkeypatch, wave16)
     # Q, K, V as slices of one (B,S,3,H,D) tensor and dQ, dK, dV written into one: bit for bit
     # the separate-tensor entry points (with O and dO in (B,S,H,D)).
     lib, st = device.lib, device.stream
