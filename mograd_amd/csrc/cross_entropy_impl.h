@@ -691,14 +691,18 @@ struct CrossEntropyOps {
   template <bool DENSE>
   static constexpr int64_t kMostChunks = !DENSE ? 16384 : 4096;
 
-  // Thread layout for a row of `chunks` chunks held in registers; false if too wide.  Up to 32 chunks: sixteen lanes per row,
-  // four rows per wave, as one wave per row left most lanes idle ((16384, 65) bf16 12.9 us | 9.4, (16384, 128) 12.5 | 9.5,
-  // (16384, 129) 13.5 | 10.3).
-  static bool pick_shape(int64_t chunks, Shape* s) {
-    const bool narrow = env_int("MOGRAD_HIP_CE_NARROW", 1) != 0;
+  // Thread layout for a row of `chunks` chunks held in registers; false if too wide.  Up to 16 chunks, and up to 32 where there are
+  // rows enough: sixteen lanes per row, four rows per wave, as one wave per row left most lanes idle ((16384, 65) bf16 12.9 us | 9.4,
+  // (16384, 128) 12.5 | 9.5, (16384, 129) 13.5 | 10.3; but (1905, 127) fp32, dense, 3.3 | 3.8).  Few rows of up to 256 chunks have a
+  // workgroup each, whose threads have one chunk, instead of a wave, whose lanes have four ((228, 924) fp32, dense, 3.8 us | 3.0;
+  // from 1100 rows of 128 chunks on, and 3600 of 256, waves are faster).
+  static bool pick_shape(int64_t chunks, int64_t rows, Shape* s) {
+    const bool narrow = env_int("MOGRAD_HIP_CE_NARROW", chunks <= 16 || rows >= 4096) != 0;
+    const bool few = env_int("MOGRAD_HIP_CE_FEW", chunks > 64 && rows < (chunks <= 128 ? 768 : 2048)) != 0;
     if (narrow && chunks <= 16) *s = {16, 1};
     else if (narrow && chunks <= 32) *s = {16, 2};
     else if (chunks <= 64) *s = {64, 1};
+    else if (few && chunks <= 256) *s = {256, 1};
     else if (chunks <= 128) *s = {64, 2};
     else if (chunks <= 256) *s = {64, 4};
     else if (chunks <= 1024) *s = {256, 4};
@@ -754,6 +758,7 @@ struct CrossEntropyOps {
     MG_CE_CASE(64, 1);
     MG_CE_CASE(64, 2);
     MG_CE_CASE(64, 4);
+    MG_CE_CASE(256, 1);
     MG_CE_CASE(256, 4);
     MG_CE_CASE(512, 4);
     MG_CE_CASE(512, 8);
@@ -851,9 +856,10 @@ struct CrossEntropyOps {
         return MG_OK;
       }
     }
-    if (C < WIDE) {
+    // (Up to 16 elements off the chunks: one to a lane; bf16, dense, (801, 13) 3.6 us in chunks | 3.0, (9159, 10) 3.8 | 3.4.)
+    if (C < WIDE || (any && C <= 16)) {
       MG_TRY((launch_rows<1, 16, 1, DENSE, false>(logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
-    } else if (chunks <= kMostChunks<DENSE> && pick_shape(chunks, &s)) {
+    } else if (chunks <= kMostChunks<DENSE> && pick_shape(chunks, N, &s)) {
       if (wide) MG_TRY((dispatch_rows<DENSE, false>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
       else MG_TRY((dispatch_rows<DENSE, true>(s, logits, labels, upstream, rowloss, dlogits, N, C, id64, stream)));
     } else {

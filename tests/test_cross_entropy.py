@@ -389,6 +389,33 @@ def test_a_row_of_the_types_last_values(device, dtype, half_ulp, size, end, Cc, 
             assert (np.abs(got.to_numpy()[start:].reshape(N, Cc) - exact) <= bound).all()
 
 
+@pytest.mark.parametrize("dtype,half_ulp", [(F32, 2.0 ** -24), (F16, 2.0 ** -11), (BF16, 2.0 ** -8)])
+@pytest.mark.parametrize("few,narrow", [("0", "0"), ("0", "1"), ("1", "1")])
+@pytest.mark.parametrize("N,Cc", [(1, 9), (5, 15), (6, 16), (7, 17), (9, 127), (4, 128), (3, 255), (5, 512), (3, 1021), (2, 1024), (3, 2041)])
+def test_layouts_of_few_and_of_many_rows(device, monkeypatch, dtype, half_ulp, few, narrow, N, Cc):
+    # A wave or a workgroup to a row of up to 256 chunks, sixteen lanes or a wave to one of up to 32.
+    monkeypatch.setenv("MOGRAD_HIP_CE_FEW", few)
+    monkeypatch.setenv("MOGRAD_HIP_CE_NARROW", narrow)
+    lib, st = device.lib, device.stream
+    x = round_to_dtype(normal(40, 0, (N, Cc), std=2.0), dtype)
+    ids = (np.arange(N) * 7 + Cc - 1) % Cc
+    dense = round_to_dtype(0.9 * O.one_hot(ids, Cc) + 0.1 / Cc, dtype)
+    bx, by, bi = AnyBuffer.from_numpy(device, x, dtype), AnyBuffer.from_numpy(device, dense, dtype), AnyBuffer.from_numpy(device, ids.astype(np.int32), I32)
+    bu = AnyBuffer.from_numpy(device, np.array([2.0], np.float32), dtype)
+    x = x.astype(np.float64)
+    p = np.exp(x - x.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    for y, labels, fused, extra in ((O.one_hot(ids, Cc), bi, lib.mg_cross_entropy_fused_ids, (I32,)), (dense, by, lib.mg_cross_entropy_fused, ())):
+        y = y.astype(np.float64)
+        loss, out = AnyBuffer.create(dtype, device, 1), AnyBuffer.create(dtype, device, N * Cc)
+        fused(bx.data_ptr(), labels.data_ptr(), bu.data_ptr(), loss.data_ptr(), out.data_ptr(), N, Cc, dtype, *extra, st)
+        want = -(y * np.log(p)).sum() / N
+        assert abs(loss.item() - want) <= (1.02 * half_ulp + 2.0 ** -18) * max(abs(want), 1.0)
+        exact = (p - y) * 2.0 / N
+        bound = 1.02 * half_ulp * np.abs(exact) + 2.0 ** -18 * (p + y) * 2.0 / N + (2.0 ** -25 if dtype == F16 else 0.0)
+        assert (np.abs(out.to_numpy((N, Cc)) - exact) <= bound).all()
+
+
 @pytest.mark.parametrize("deep", ["0", "1"])
 @pytest.mark.parametrize("chunks", ["0", "1"])
 @pytest.mark.parametrize("N", [1, 1024, 1025, 2048, 2049, 16385, 40000])
